@@ -239,12 +239,14 @@ void HcltCircuit::build_schedules() {
 
   std::vector<std::vector<int32_t>> ic(n_inner_), lc(n_inner_);
   std::vector<int32_t> par(n_inner_, -1), hin(n_inner_, 0);   // hin: longest chain of inner nodes below
+  std::vector<int32_t> below(n_inner_, 0);                    // inner nodes below (children come first in post-order)
+  const bool lean_k = K_ <= 32;                               // hidden sizes with lean walk kernels
   for (int n = 0; n < n_inner_; ++n) {
     const int v = var_of_inner_[n];
     if (parent_[v] >= 0) par[n] = inner_of_var_[parent_[v]];
     for (int c : children_[v]) {
       if (children_[c].empty()) lc[n].push_back(c);
-      else { ic[n].push_back(inner_of_var_[c]); hin[n] = std::max(hin[n], hin[inner_of_var_[c]] + 1); }
+      else { ic[n].push_back(inner_of_var_[c]); hin[n] = std::max(hin[n], hin[inner_of_var_[c]] + 1); below[n] += 1 + below[inner_of_var_[c]]; }
     }
   }
   std::vector<uint32_t> ext;
@@ -413,7 +415,7 @@ void HcltCircuit::build_schedules() {
   n_groups_ = (int)groups.size();
 
   // ---- forward -----------------------------------------------------------------------
-  auto schedule_forward = [&](int g0, int g1, std::vector<StepItem>& sched, std::vector<PreItem>& pre) {
+  auto schedule_forward = [&](int g0, int g1, std::vector<StepItem>& sched, std::vector<PreItem>& pre, bool reserve) {
     std::vector<int32_t> pending(n_inner_), slot(n_inner_, -1), free_slots;
     for (int s = trash_slot - 1; s >= 0; --s) free_slots.push_back(s);
     // max-heap: deeper first, then lower id (post-order).  In a forest the earlier tree goes first whatever the
@@ -423,9 +425,9 @@ void HcltCircuit::build_schedules() {
       if (tree_of_inner_[a] != tree_of_inner_[b]) return tree_of_inner_[a] > tree_of_inner_[b];
       return depth_of(a) != depth_of(b) ? depth_of(a) < depth_of(b) : a > b;
     };
-    // ... and a node without inner children, which fills a slot and frees none, only starts while more than a
-    // step's worth of slots is free (or nothing else can run)
-    const int producer_reserve = T_ > 1 ? kWalkWaves : 0;
+    // with `reserve` (always in a forest) a node without inner children, which fills a slot and frees none, only
+    // starts while more than a step's worth of slots is free (or nothing else can run)
+    const int producer_reserve = kWalkWaves;
     std::vector<int32_t> ready;
     for (int n = g0; n < g1; ++n) { pending[n] = (int)ic[n].size(); if (!pending[n]) ready.push_back(n); }
     std::make_heap(ready.begin(), ready.end(), cmp);
@@ -440,7 +442,7 @@ void HcltCircuit::build_schedules() {
         std::pop_heap(ready.begin(), ready.end(), cmp);
         const int n = ready.back();
         ready.pop_back();
-        if (T_ > 1) {
+        if (reserve) {
           if (par[n] >= 0) {
             if (slots_left <= (ic[n].empty() ? producer_reserve : 0)) { deferred.push_back(n); continue; }
             --slots_left;
@@ -452,8 +454,8 @@ void HcltCircuit::build_schedules() {
         step.push_back(n);
       }
       if (step.empty() && !deferred.empty()) {
-        // nothing fits: the first of the waiting nodes in heap order (a forest) / the last (one tree) goes anyway
-        const size_t pick = T_ > 1 ? 0 : deferred.size() - 1;
+        // nothing fits: the first of the waiting nodes in heap order / without a reserve the last one goes anyway
+        const size_t pick = reserve ? 0 : deferred.size() - 1;
         step.push_back(deferred[pick]);
         deferred.erase(deferred.begin() + (std::ptrdiff_t)pick);
       }
@@ -524,8 +526,23 @@ void HcltCircuit::build_schedules() {
     std::vector<std::vector<PreItem>> pre(n_groups_);
     n_fwd_steps_ = 0;
     for (int g = 0; g < n_groups_; ++g) {
-      schedule_forward(groups[g].first, groups[g].second, sched[g], pre[g]);
+      schedule_forward(groups[g].first, groups[g].second, sched[g], pre[g], forest_);
       n_fwd_steps_ = std::max(n_fwd_steps_, (int)sched[g].size() / kWalkWaves);
+    }
+    if (lean_k && !forest_ && fwd_spill_) {
+      // a single bushy tree whose waiting tiles overran the slots is scheduled again with a reserve (see kLeanStretch)
+      std::vector<StepItem> sched2;
+      std::vector<PreItem> pre2;
+      fwd_spill_ = false;
+      schedule_forward(0, n_inner_, sched2, pre2, true);
+      const int steps2 = (int)sched2.size() / kWalkWaves;
+      if (!fwd_spill_ && steps2 <= n_fwd_steps_ * kLeanStretch) {
+        n_fwd_steps_ = steps2;
+        sched[0].swap(sched2);
+        pre[0].swap(pre2);
+      } else {
+        fwd_spill_ = true;
+      }
     }
     std::vector<int32_t> lean_rows;
     fwd_lean_ = !fwd_spill_;
@@ -542,7 +559,7 @@ void HcltCircuit::build_schedules() {
   // Oldest-ready first (ties: longest chain below first): a parent's flow tile then leaves
   // its LDS slot a few steps after it was produced, so the number of live tiles stays near
   // the width of the tree instead of growing with every postponed short subtree.
-  auto schedule_backward = [&](int g0, int g1, std::vector<StepItem>& sched, std::vector<PreItem>& pre) {
+  auto schedule_backward = [&](int g0, int g1, std::vector<StepItem>& sched, std::vector<PreItem>& pre, bool counted) {
     std::vector<int32_t> remaining(n_inner_), slot(n_inner_, -1), ready_at(n_inner_, 0), free_slots;
     for (int s = trash_slot - 1; s >= 0; --s) free_slots.push_back(s);
     std::vector<int32_t> ready;
@@ -559,11 +576,15 @@ void HcltCircuit::build_schedules() {
       std::vector<int32_t> step, rest;
       int slots_left = (int)free_slots.size();
       for (int n : ready) {
-        // a forest also counts the ratio tiles of the lean walk while it schedules (one per inner child, from the
-        // parent's step to the end of the child's): a node only runs if its children's tiles fit, and a new tree
-        // only starts while half the slots are free, so that the trees under way can finish
+        // with `counted` the ratio tiles of the lean walk (one per inner child, from the parent's step to the end of
+        // the child's) are counted along: a node only runs if its children's tiles fit.  In a forest a new tree only
+        // starts while half the slots are free, so that the trees under way can finish; in a single tree a node that
+        // adds tiles (two inner children or more) leaves kBranchReserve slots to the chains, which hand on as many
+        // tiles as they take.
         const int need = (int)ic[n].size();
-        const bool ratio_ok = T_ == 1 || ratio_live + need <= (par[n] < 0 ? trash_slot / 2 : trash_slot);
+        const int limit = !counted ? n_inner_ + trash_slot
+                          : T_ > 1 ? (par[n] < 0 ? trash_slot / 2 : trash_slot) : trash_slot - (need > 1 ? kBranchReserve : 0);
+        const bool ratio_ok = ratio_live + need <= limit;
         if ((int)step.size() < kWalkWaves && (ic[n].empty() || slots_left > 0) && ratio_ok) {
           step.push_back(n);
           if (!ic[n].empty()) --slots_left;
@@ -574,8 +595,12 @@ void HcltCircuit::build_schedules() {
       }
       if (step.empty()) {
         if (rest.empty()) fail(PCM_ERR_SHAPE, "backward schedule stalled (tree is inconsistent)");
-        step.push_back(rest.front());
-        rest.erase(rest.begin());
+        // (a single tree: the node with the fewest nodes below it, whose tiles are gone again soonest)
+        const auto pick = T_ > 1 || !counted ? rest.begin()
+                                             : std::min_element(rest.begin(), rest.end(), [&](int a, int b) { return below[a] < below[b]; });
+        ratio_live += (int)ic[*pick].size();
+        step.push_back(*pick);
+        rest.erase(pick);
       }
       ready.swap(rest);
       for (int w = 0; w < kWalkWaves; ++w) {
@@ -611,12 +636,31 @@ void HcltCircuit::build_schedules() {
     std::vector<std::vector<PreItem>> pres(n_groups_);
     n_bwd_steps_ = 0;
     for (int g = 0; g < n_groups_; ++g) {
-      schedule_backward(groups[g].first, groups[g].second, scheds[g], pres[g]);
+      schedule_backward(groups[g].first, groups[g].second, scheds[g], pres[g], forest_);
       n_bwd_steps_ = std::max(n_bwd_steps_, (int)scheds[g].size() / kWalkWaves);
     }
     std::vector<int32_t> ratio_slot(n_inner_, -1);
     bool slots_ok = true;
     for (int g = 0; g < n_groups_ && slots_ok; ++g) slots_ok = assign_ratio_slots(scheds[g], ratio_slot);
+    if (lean_k && fwd_lean_ && !forest_ && !slots_ok) {
+      // a single tree whose ratio tiles overran the slots is scheduled again with the tiles counted
+      std::vector<StepItem> sched2;
+      std::vector<PreItem> pre2;
+      const bool spill = bwd_spill_;
+      bwd_spill_ = false;
+      schedule_backward(0, n_inner_, sched2, pre2, true);
+      std::vector<int32_t> ratio2(n_inner_, -1);
+      const int steps2 = (int)sched2.size() / kWalkWaves;
+      if (!bwd_spill_ && steps2 <= n_bwd_steps_ * kLeanStretch && assign_ratio_slots(sched2, ratio2)) {
+        slots_ok = true;
+        n_bwd_steps_ = steps2;
+        scheds[0].swap(sched2);
+        pres[0].swap(pre2);
+        ratio_slot.swap(ratio2);
+      } else {
+        bwd_spill_ = spill;
+      }
+    }
     std::vector<int32_t> lean_rows;
     bwd_lean_ = slots_ok;
     for (int g = 0; g < n_groups_; ++g) {
@@ -648,7 +692,7 @@ void HcltCircuit::build_schedules() {
         std::vector<std::vector<StepItem>> sched(gr.size());
         std::vector<std::vector<PreItem>> pre(gr.size());
         for (size_t g = 0; g < gr.size(); ++g) {
-          schedule_forward(gr[g].first, gr[g].second, sched[g], pre[g]);
+          schedule_forward(gr[g].first, gr[g].second, sched[g], pre[g], true);
           plan->n_fwd_steps = std::max(plan->n_fwd_steps, (int)sched[g].size() / kWalkWaves);
         }
         ok = !fwd_spill_;
@@ -664,7 +708,7 @@ void HcltCircuit::build_schedules() {
         std::vector<std::vector<StepItem>> sched(gr.size());
         std::vector<std::vector<PreItem>> pre(gr.size());
         for (size_t g = 0; g < gr.size(); ++g) {
-          schedule_backward(gr[g].first, gr[g].second, sched[g], pre[g]);
+          schedule_backward(gr[g].first, gr[g].second, sched[g], pre[g], true);
           plan->n_bwd_steps = std::max(plan->n_bwd_steps, (int)sched[g].size() / kWalkWaves);
         }
         ok = !bwd_spill_;

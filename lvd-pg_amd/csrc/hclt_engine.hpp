@@ -25,6 +25,13 @@ constexpr uint32_t kOpNone = 0x40000000u;    // absent operand: reads as zeros
 constexpr int kXSelShift = 28;               // leaf operand: which byte of the packed categories (2 bits)
 constexpr int kSlotShift = 22;               // LDS operand: (slot + 1) << kSlotShift | inner id
 constexpr int kItemRoot = 1, kItemHasInnerChild = 2, kItemOverflow = 4, kItemSpillOut = 8;
+// A single tree (K <= 32) whose tiles overrun the LDS slots under the plain greedy schedules is scheduled again with the
+// tiles counted, at up to kLeanStretch times the steps, before it goes to the general walk kernels: those take 1.45 times
+// as long per EM step (2.40 against 1.65 ms on a 3072-variable Chow-Liu tree at 4096 examples, which needed 80 ratio
+// tiles of the 78 that fit and needs no step more, 164, with the tiles counted).  A branching node leaves
+// kBranchReserve slots free to the chains; 0 / 16 / 24 gave 164 / 164 / 165 steps there.
+constexpr int kBranchReserve = 8;
+constexpr double kLeanStretch = 1.4;
 constexpr int kPre = 3;          // static operand tiles a wave requests one step ahead
 
 struct HcltNode {     // one non-leaf tree node, device-resident

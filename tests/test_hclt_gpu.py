@@ -92,6 +92,18 @@ def test_every_walk_kernel_family_is_exercised(gpu, oracle):
     assert bpc.size("walk_kernels") == 2
 
 
+@pytest.mark.parametrize("shape", ["random", "binary", "ternary"])
+def test_bushy_trees_keep_the_lean_walks(gpu, oracle, shape):
+    """Trees whose ratio tiles, scheduled without counting them, overran the LDS slots of K = 32 (78): the schedule
+    counts them, so these circuits walk on the lean kernels."""
+    n = {"random": 600, "binary": 511, "ternary": 364}[shape]
+    tree = {"random": lambda: oracle.random_tree(n, np.random.default_rng(2), 3),
+            "binary": lambda: [-1] + [(i - 1) // 2 for i in range(1, n)],
+            "ternary": lambda: [-1] + [(i - 1) // 3 for i in range(1, n)]}[shape]()
+    bpc = _compare_step(gpu, oracle, n, 32, 5, 19, seed=31, tree=list(tree))
+    assert bpc.size("walk_kernels") == 1
+
+
 def test_ragged_batch_and_example_ids(gpu, oracle):
     rng = np.random.default_rng(5)
     idx = rng.permutation(200)[:37].astype(np.int32)
