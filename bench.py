@@ -24,7 +24,7 @@ REQUESTED_NOTE = ("bytes the circuit asks for edge by edge: 8 per (node, example
                   "are served by L2 and the last-level cache, so frac is not a fraction of HBM traffic")
 # kernels the benchmark circuit runs (three children per node at most, K = 32: the lean set)
 PHASE_MASK = {"forward": 2, "backward": 4, "statistics": 8}   # pcm_set_timing: time that phase's kernel only
-KERNEL_NAMES = {"forward": "hclt_forward_lean_kernel<%d>", "backward": "hclt_backward_lean_kernel<%d, false>",
+KERNEL_NAMES = {"forward": "hclt_forward_lean_kernel<%d, 2>", "backward": "hclt_backward_lean_kernel<%d, false>",
                 "statistics": "hclt_stats_lean_kernel<%d>"}
 
 

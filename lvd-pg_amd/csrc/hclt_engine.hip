@@ -1289,7 +1289,19 @@ void HcltCircuit::update_parameters(const float* in, int64_t n) {
 
 // ---- batches ------------------------------------------------------------------------
 
+// the staged categories of a batch: all a scoring pass on the lean walk keeps of it
+void HcltCircuit::ensure_staged(int batch) {
+  const int ns = ceil_div(batch, kSlice);
+  if (ns <= cap_staged_) return;
+  d_xb_.alloc((size_t)V_ * ns * kSlice);
+  if (V_ > Vu_) d_xb_.zero(stream);   // the category of an auxiliary variable is always 0
+  d_xn_.alloc((size_t)(n_inner_ + 1) * ns * kSlice);
+  d_xn_.zero(stream);
+  cap_staged_ = ns;
+}
+
 void HcltCircuit::ensure_batch(int batch) {
+  ensure_staged(batch);
   const int ns = ceil_div(batch, kSlice);
   if (ns <= cap_slices_) return;
   const size_t tile = tile_floats(ns);
@@ -1299,9 +1311,6 @@ void HcltCircuit::ensure_batch(int batch) {
     d_wide_rs_.alloc((size_t)n_inner_ * tile);
     d_wide_es_.alloc((size_t)n_inner_ * tile);
     d_M_.alloc((size_t)(n_inner_ + 1) * ns * kSlice);
-    d_xb_.alloc((size_t)V_ * ns * kSlice);
-    d_xn_.alloc((size_t)(n_inner_ + 1) * ns * kSlice);
-    d_xn_.zero(stream);
     cap_slices_ = ns;
     return;
   }
@@ -1313,10 +1322,6 @@ void HcltCircuit::ensure_batch(int batch) {
     d_wide_es_.alloc((size_t)n_inner_ * tile);
   }
   d_M_.alloc((size_t)(n_inner_ + 1) * ns * kSlice);   // row maxima of the forward walk
-  d_xb_.alloc((size_t)V_ * ns * kSlice);
-  if (V_ > Vu_) d_xb_.zero(stream);   // the category of an auxiliary variable is always 0
-  d_xn_.alloc((size_t)(n_inner_ + 1) * ns * kSlice);
-  d_xn_.zero(stream);
   cap_slices_ = ns;
 }
 
@@ -1369,11 +1374,11 @@ BatchRef HcltCircuit::chunk_of(const BatchRef& b, int off, int chunk) {
   return part;
 }
 
-void HcltCircuit::stage_batch(const BatchRef& b) {
+void HcltCircuit::stage_batch(const BatchRef& b, bool tiles) {
   check_walks();
   if (!b.d_data) fail(PCM_ERR_ARG, "data pointer is null");
   if (b.batch < 1) fail(PCM_ERR_ARG, "batch must be positive, got %d", b.batch);
-  ensure_batch(b.batch);
+  if (tiles) ensure_batch(b.batch); else ensure_staged(b.batch);
   const int Bp = ceil_div(b.batch, kSlice) * kSlice;
   pcm_stage(b.d_data, b.stride_ex, b.stride_var, b.d_idx, b.batch, Bp, Vu_, C_, d_xb_.p, stream);   // (auxiliary rows stay 0)
   check_launch("stage_batch");
@@ -1391,27 +1396,34 @@ const HcltCircuit::LeanPlan* HcltCircuit::fine_plan(int nslices) const {
   return best;
 }
 
-void HcltCircuit::run_forward(const HcltDev& d, float* d_ll) {
+// the lean kernels address every array with 32-bit offsets from one descriptor
+bool HcltCircuit::lean_fits(int batch) const {
+  return lean_ && !force_general_walks_ && (size_t)(n_inner_ + 1) * tile_floats(ceil_div(batch, kSlice)) * 4 < ((size_t)1 << 31);
+}
+
+void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
   const size_t lds = (size_t)lds_slots_ * kSlice * K_ * sizeof(float);
   auto launch = [&](auto kernel) {
     PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices), dim3(kWalkWaves * 64), lds, d, d_fwd_fields_.p, fwd_stride_,
                      d_fwd_sched_.p, n_fwd_steps_, d_ll);
   };
-  // the lean kernels address every array with 32-bit offsets from one descriptor
-  const bool small = (size_t)(n_inner_ + 1) * d.tile_stride < ((size_t)1 << 31);
-  if (lean_ && small && !force_general_walks_) {
+  if (lean_fits(d.B)) {
     const size_t lean_lds = lds + kLeanFlagWords * 4;   // the slots' state words sit behind the slots
-    PCM_DISPATCH_LEAN_K(K_, {
-      PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&hclt_forward_lean_kernel<KK>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
+    auto launch_lean = [&](auto kernel) {
+      PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
       const LeanPlan* fp = fine_plan(d.nslices);
       if (fp)
-        PCM_LAUNCH_PHASE(0, hclt_forward_lean_kernel<KK>, dim3(d.nslices, fp->n_groups), dim3(kWalkWaves * 64), lean_lds, d,
-                         fp->fwd.p, fp->fwd_stride, fp->n_fwd_steps, d_ll, lds_slots_);
+        PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices, fp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, fp->fwd.p,
+                         fp->fwd_stride, fp->n_fwd_steps, d_ll, lds_slots_);
       else
-        PCM_LAUNCH_PHASE(0, hclt_forward_lean_kernel<KK>, dim3(d.nslices, n_groups_), dim3(kWalkWaves * 64), lean_lds, d,
-                         d_fwd_lean_.p, fwd_stride_, n_fwd_steps_, d_ll, lds_slots_);
+        PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices, n_groups_), dim3(kWalkWaves * 64), lean_lds, d, d_fwd_lean_.p, fwd_stride_,
+                         n_fwd_steps_, d_ll, lds_slots_);
+    };
+    PCM_DISPATCH_LEAN_K(K_, {
+      if (keep == kKeepAll) launch_lean(&hclt_forward_lean_kernel<KK, kKeepAll>);
+      else if (keep == kKeepRoots) launch_lean(&hclt_forward_lean_kernel<KK, kKeepRoots>);
+      else launch_lean(&hclt_forward_lean_kernel<KK, kKeepNone>);
     });
   } else {
     PCM_DISPATCH_K(K_, {
@@ -1428,8 +1440,7 @@ void HcltCircuit::run_backward(const HcltDev& d) {
     PCM_LAUNCH_PHASE(1, kernel, dim3(d.nslices), dim3(kWalkWaves * 64), lds, d, d_bwd_fields_.p, bwd_stride_,
                      d_bwd_sched_.p, n_bwd_steps_);
   };
-  const bool small = (size_t)(n_inner_ + 1) * d.tile_stride < ((size_t)1 << 31);
-  if (lean_ && small && !force_general_walks_) {
+  if (lean_fits(d.B)) {
     const size_t lean_lds = lds + kLeanFlagWords * 4;
     auto launch_lean = [&](auto kernel) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
@@ -1464,8 +1475,7 @@ void HcltCircuit::run_stats(const HcltDev& d, float rate) {
   const int limb = std::min(24, 32 - bits);
   if (limb < 12) fail(PCM_ERR_UNSUPPORTED, "batch of %d examples is too large for one call", d.B);
   const size_t hist = 2 * (size_t)C_ * (K_ + 1);                    // words per histogram (two limbs)
-  const bool small = (size_t)(n_inner_ + 1) * d.tile_stride < ((size_t)1 << 31);
-  if (lean_ && small && !force_general_walks_) {
+  if (lean_fits(d.B)) {
     // LDS: the histograms of a pass (or the parked edge-flow blocks, whichever is larger) | per-wave pads
     const size_t park = (size_t)kStatLeanWaves * K_ * K_;
     const size_t hw = std::max((size_t)stat_lean_hists_ * 2 * C_ * K_, park);
@@ -1511,15 +1521,17 @@ void HcltCircuit::loglikelihoods(const BatchRef& b, float* d_ll) {
     for (int off = 0; off < b.batch; off += chunk) loglikelihoods(chunk_of(b, off, chunk), d_ll + off);
     return;
   }
-  stage_batch(b);
+  // nobody reads a scoring pass's tiles: the lean walk keeps none (heads: the roots' only)
+  const bool lean = lean_fits(b.batch) && !wide_walk_;
+  stage_batch(b, !lean || H_ > 0);
   if (wide_walk_) return wide_forward(dev(b.batch), d_ll);
   if (H_ > 0) {   // per-head values [H][batch]
     const HcltDev d = dev(b.batch);
-    run_forward(d, nullptr);   // (the head kernel reads the root tiles and the row maxima)
+    run_forward(d, nullptr, kKeepRoots);   // (the head kernel reads the root tiles and the row maxima)
     heads_forward(d, nullptr, d_ll, nullptr);
     return;
   }
-  run_forward(dev(b.batch), d_ll);
+  run_forward(dev(b.batch), d_ll, kKeepNone);
 }
 
 // Soft evidence (src/regularization/reg_likelihood.jl:51-91, reg_flow.jl:50-82) runs on the layered

@@ -25,6 +25,7 @@ constexpr uint32_t kOpNone = 0x40000000u;    // absent operand: reads as zeros
 constexpr int kXSelShift = 28;               // leaf operand: which byte of the packed categories (2 bits)
 constexpr int kSlotShift = 22;               // LDS operand: (slot + 1) << kSlotShift | inner id
 constexpr int kItemRoot = 1, kItemHasInnerChild = 2, kItemOverflow = 4, kItemSpillOut = 8;
+enum { kKeepNone = 0, kKeepRoots, kKeepAll };   // what the lean forward walk leaves in memory (hclt_walk_lean.hip.hpp)
 // A single tree (K <= 32) whose tiles overrun the LDS slots under the plain greedy schedules is scheduled again with the
 // tiles counted, at up to kLeanStretch times the steps, before it goes to the general walk kernels: those take 1.45 times
 // as long per EM step (2.40 against 1.65 ms on a 3072-variable Chow-Liu tree at 4096 examples, which needed 80 ratio
@@ -334,7 +335,8 @@ class HcltCircuit : public pcm_circuit {
   DevBuf<float> d_part_;       // rows of partial sums (head statistics per slice, soft leaf counts per split)
   DevBuf<float> d_row_sum_;    // Adam from flows: per-sum-node / per-input-node flow totals
   DevBuf<int32_t> d_input_order_;   // i-th input node of the parameter vector -> v*K + j
-  int cap_slices_ = 0;
+  int cap_slices_ = 0;             // slices the tile arrays hold
+  int cap_staged_ = 0;             // ... the staged categories
   bool have_flows_ = false;
   // soft evidence on the block kernels (single head, K <= 64)
   bool soft_block_ok() const { return block_queries() && !wide_ && H_ == 0; }
@@ -372,10 +374,12 @@ class HcltCircuit : public pcm_circuit {
   void build_schedules();
   void build_param_order();
   void ensure_batch(int batch);
+  void ensure_staged(int batch);
   HcltDev dev(int batch) const;
-  void stage_batch(const BatchRef& b);
+  void stage_batch(const BatchRef& b, bool tiles = true);
   void rebuild_w();
-  void run_forward(const HcltDev& d, float* d_ll);
+  bool lean_fits(int batch) const;
+  void run_forward(const HcltDev& d, float* d_ll, int keep = kKeepAll);
   void run_backward(const HcltDev& d);
   void run_stats(const HcltDev& d, float rate);
   // wide block kernels

@@ -138,7 +138,13 @@ __device__ __forceinline__ void lean_post(unsigned* state, unsigned value) {
 // but the log-likelihood at the root.  Stored as one float32 it would cost every state of a 3000-variable circuit
 // (values near -14000) an absolute error of 1e-3, which is a relative error of 1e-3 on every flow; in two parts the
 // flows keep float32's relative accuracy at any depth.
-template <int K>
+//
+// kKeep: what the walk leaves in memory.  kKeepAll: every node's tile and row of maxima, for the passes behind it;
+// kKeepRoots: the maxima and the roots' tiles, what the head kernel of a multi-head circuit reads; kKeepNone: nothing
+// but the log-likelihoods: a scoring pass has nobody behind it, and value stores are 512 of a step's 1340 requests.
+// 10300 examples of 3072 variables (K = 32), which no longer need tile arrays and so go through 4096 at a time
+// whatever the caller's batch size: 3.93 ms in batches of 1000 -> 1.08 ms.
+template <int K, int kKeep>
 __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
     HcltDev d, const int32_t* __restrict__ fields, int stride, int n_steps, float* __restrict__ ll_out, int n_slots) {
   extern __shared__ float lds[];
@@ -151,7 +157,7 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
   const uint32_t vtile = (uint32_t)lane * 16, vleaf = (uint32_t)(lane >> 4) * 16, vx = (uint32_t)(lane & 15) * 4;
   const int bcol = slice * kSlice + (lane & 15);
   const uint32_t slice_bytes = (uint32_t)slice * (kSlice * K * 4);
-  const __amdgpu_buffer_rsrc_t rO =
+  const __amdgpu_buffer_rsrc_t rO =   // (kKeepNone: the arrays may not exist, and nothing is stored)
       make_rsrc(reinterpret_cast<const char*>(d.O) + slice_bytes, (uint32_t)(d.n_inner + 1) * d.tile_stride - slice_bytes);
   const __amdgpu_buffer_rsrc_t rW = make_rsrc(d.Wf, (uint32_t)d.n_inner * (K * K * 4));
   const __amdgpu_buffer_rsrc_t rL = make_rsrc(d.leaf, (uint32_t)d.V * d.leaf_stride);
@@ -190,6 +196,13 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
   float m_prev = 0.f;
   int mrow_prev = d.n_inner * xrow;
 
+  bool root_prev = false;
+  auto keep_prev = [&]() {
+    if (kKeep == kKeepAll || (kKeep == kKeepRoots && root_prev)) lean_tile_store<K, PCM_ST_O>(rO, vtile, store_prev, o_prev);
+    if (kKeep != kKeepNone)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, m_prev), rM, (int)vm, mrow_prev, kStreamStore);
+  };
+
   // the schedule is consumed in chunks of kLeanChunk steps (a chunk's registers also serve
   // the two steps of look-ahead past its end)
   auto step = [&](const int s, WTile<K>& w) {
@@ -199,8 +212,7 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
     if (a2 >= 0) tile_add<K>(z, P2);
     if (a3 >= 0) tile_add<K>(z, P3);
     // the previous step's value tile goes out now
-    lean_tile_store<K, PCM_ST_O>(rO, vtile, store_prev, o_prev);
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, m_prev), rM, (int)vm, mrow_prev, kStreamStore);
+    keep_prev();
     // (2) request the leaf rows of step s+1 and the categories of step s+2
     {
       // (the categories first: everything that later waits for a leaf row then covers them)
@@ -248,7 +260,8 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
       lds_tile_store<K>(lds, (int)so, lane, o);
       if (handed) lean_post(state + so, (2 * tn + 1) & 0xffu);
     }
-    if (lean_get(sc, kLFlags, s) & 1) ll = o.v[0][0];
+    root_prev = (lean_get(sc, kLFlags, s) & 1) != 0;
+    if (root_prev) ll = o.v[0][0];
   };
   // The schedule is consumed in chunks of kLeanChunk steps (a chunk's registers also serve the
   // two steps of look-ahead past its end), two steps per trip: the parameter blocks alternate
@@ -262,8 +275,7 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
       step(s + 1, wB);
     }
   }
-  lean_tile_store<K, PCM_ST_O>(rO, vtile, store_prev, o_prev);
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, m_prev), rM, (int)vm, mrow_prev, kStreamStore);
+  keep_prev();
   // log-likelihood of a single-root circuit: the root's (scaled) value plus the row maxima of all nodes, the
   // waves' sums added in wave order (a multi-head circuit's head kernel adds up the stored maxima per tree)
   if (!ll_out) return;

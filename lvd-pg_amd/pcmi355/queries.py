@@ -63,6 +63,11 @@ def loglikelihoods(bpc, data, batch_size=None, example_ids=None):
     if n == 0:                                  # no examples: an empty result, no launch
         return torch.empty((0, heads) if heads else (0,), dtype=torch.float32, device=data.device)
     batch_size = n if batch_size is None else batch_size
+    if n > batch_size and not heads and not _is_soft(data) and bpc.size("walk_kernels") == 1:
+        # the lean walk keeps nothing of a batch but its categories, and the library itself takes as many examples at a
+        # time as fill the device, which smaller batches would not (10300 examples of 3072 variables: 3.9 ms in batches
+        # of 1000, 1.1 ms this way)
+        batch_size = n
     out = torch.empty((max(heads, 1), n), dtype=torch.float32, device=data.device)
     for s in range(0, n, batch_size):
         b = min(batch_size, n - s)

@@ -104,6 +104,25 @@ def test_bushy_trees_keep_the_lean_walks(gpu, oracle, shape):
     assert bpc.size("walk_kernels") == 1
 
 
+@pytest.mark.parametrize("K,V", [(16, 9), (32, 40), (64, 6), (8, 5)])
+def test_scores_do_not_depend_on_the_batch_size(gpu, K, V):
+    """A scoring pass on the lean walk keeps no tiles and takes the examples in batches of its own; the other kernels
+    take the caller's.  A fresh handle, a larger batch after a smaller one, and the tiles of a flow pass in between."""
+    torch, P = gpu
+    from helpers import make_hclt, correlated_data, block_theta
+    parent, theta, leaf, _ = make_hclt(V, K, 7, 3)
+    d = torch.from_numpy(correlated_data(4500, V, 7, 4, parent)).cuda()
+    a, b = P.hclt_from_clt(parent, 7, K), P.hclt_from_clt(parent, 7, K)
+    for c in (a, b):
+        c.set_params(block_theta(parent, K, theta), leaf)
+    want = P.probs_flows_circuit(b, d)
+    few = P.loglikelihoods(a, d[:17].contiguous(), batch_size=5)
+    every = P.loglikelihoods(a, d, batch_size=1000)
+    assert torch.equal(few, want[:17]) and torch.equal(every, want)
+    assert torch.equal(P.probs_flows_circuit(a, d[:50].contiguous()), want[:50])
+    assert torch.equal(P.loglikelihoods(a, d, batch_size=4499), want)
+
+
 def test_ragged_batch_and_example_ids(gpu, oracle):
     rng = np.random.default_rng(5)
     idx = rng.permutation(200)[:37].astype(np.int32)
