@@ -229,9 +229,6 @@ class HcltCircuit : public pcm_circuit {
   int Vu_ = 0;                     // the caller's variables; V_ - Vu_ auxiliary ones behind them (forests only)
   void split_wide_nodes();
   std::vector<std::vector<int32_t>> uchildren_;   // the caller's tree (children of every variable) where nodes were split
-  // soft evidence on the block form reads evidence per variable of the stored tree; with auxiliary nodes in it
-  // that query takes the general form of the caller's circuit instead
-  bool block_queries() const { return block_ && V_ == Vu_; }
   bool forest_ = false;
   int T_ = 1;                      // trees (1 unless a forest)
   int n_groups_ = 1;               // groups of trees the walk kernels take side by side (blockIdx.y)
@@ -339,7 +336,9 @@ class HcltCircuit : public pcm_circuit {
   int cap_staged_ = 0;             // ... the staged categories
   bool have_flows_ = false;
   // soft evidence on the block kernels (single head, K <= 64)
-  bool soft_block_ok() const { return block_queries() && !wide_ && H_ == 0; }
+  // (the values of soft evidence are per variable of the stored tree: a tree whose nodes were split takes the general
+  // form of the caller's circuit instead)
+  bool soft_block_ok() const { return block_ && V_ == Vu_ && !wide_ && H_ == 0; }
   HcltDev soft_stage(const SoftRef& s);
   DevBuf<float> d_soft_lv_, d_soft_m_;   // value table [V][Bp][K] and largest evidence [V][Bp] of the batch
   DevBuf<int32_t> d_soft_gnode_;
@@ -358,7 +357,7 @@ class HcltCircuit : public pcm_circuit {
   SparseCircuit* general_structure();   // the same object without bringing its parameters up to date
   // KL recursion on the block form
   DevBuf<int32_t> d_kl_up_, d_kl_down_;   // chain steps (KlItem records) bottom-up / top-down
-  DevBuf<int32_t> d_blk2par_;             // entry of the [n_inner][K][K] blocks -> parameter (-1: no such edge), for the row queries
+  DevBuf<int32_t> d_blk2par_;             // entry of the [n_inner][K][K] blocks -> parameter, for the row queries (build_block_params)
   DevBuf<float> d_rows_scratch_, d_rows_pk1_, d_rows_pk2_, d_rows_pg1_, d_rows_pg2_;   // row queries: per-row arrays; re-laid-out matrices
   DevBuf<int32_t> d_kl_tabs_;             // parent of every inner node | h-giving node of every variable | input-node positions
   DevBuf<int32_t> d_kl_pos_;              // chain slot of every inner node: upward | downward
@@ -368,6 +367,7 @@ class HcltCircuit : public pcm_circuit {
   int kl_ring_slots_ = 0;                 // slots of the chains' LDS ring; 0: levels too wide, the ring is the whole chain in device memory
   HcltCircuit* same_tree(pcm_circuit* q);
   void build_kld_tables();
+  void build_block_params();
   void kld_device(HcltCircuit* q, bool with_down);
   void pull_from_general();
   void build_structure();

@@ -697,8 +697,15 @@ __global__ __launch_bounds__(256) void hclt_rows_leaf_kl_kernel(const float* __r
   }
 }
 
-// hclt_kld_base_kernel for (tree node, row): theta through blk2par (entry of the [n_inner][K][K] blocks -> parameter,
-// -1: an edge that is not there, the root's rows past the first)
+// What an entry of the [n_inner][K][K] blocks is in a parameter row: its position, kBlkNone for an edge that is not there
+// (the root's rows past the first, everything off the diagonal of an auxiliary node's block), kBlkOne for one of weight 1
+// that no parameter stands for (an auxiliary node's diagonal).  A tree whose nodes were split (split_wide_nodes) runs on
+// these kernels like any other: an identity block adds nothing to the KL recursion and hands a td or a gradient on.
+// (On the per-layer kernels of the general form, which such trees took before: KL and gradient of 16 rows of a 3072-variable
+// circuit 7.0 -> 3.05 ms, relaxed samples and their reverse pass of 100 rows of 768 variables at K = 16 4.4 -> 1.05 ms.)
+constexpr int kBlkNone = -1, kBlkOne = -2;
+
+// hclt_kld_base_kernel for (tree node, row): theta through blk2par
 template <int K>
 __global__ __launch_bounds__(256) void hclt_rows_base_kernel(const HcltNode* __restrict__ nodes,
                                                              const int32_t* __restrict__ child_leaf,
@@ -706,7 +713,7 @@ __global__ __launch_bounds__(256) void hclt_rows_base_kernel(const HcltNode* __r
                                                              const int32_t* __restrict__ blk2par,
                                                              const float* __restrict__ P1, const float* __restrict__ P2,
                                                              size_t n_par, const float* __restrict__ kl_leaf, size_t vk,
-                                                             float* __restrict__ ell, float* __restrict__ base,
+                                                             int n_vars, float* __restrict__ ell, float* __restrict__ base,
                                                              float* __restrict__ pu, float* __restrict__ pd, KlRowStrides rs) {
   // (kl_leaf null: the leaf terms are not known yet -- the gradient's downward chain runs before the one pass over the
   // leaf parameters -- and base gets the node's own part sum_j p (x - y) only; hclt_rows_soft_base2_kernel adds
@@ -725,7 +732,7 @@ __global__ __launch_bounds__(256) void hclt_rows_base_kernel(const HcltNode* __r
     float s = 0.f;
     if (kl_leaf) {
       kl_leaf += row * vk;
-      s = kl_leaf[(size_t)nd.var * K + t];
+      if (nd.var < n_vars) s = kl_leaf[(size_t)nd.var * K + t];   // (auxiliary variables have no leaves of their own)
       for (int q = 0; q < nd.lc_cnt; ++q) s += kl_leaf[(size_t)child_leaf[nd.lc_off + q] * K + t];
       ell[su * K + t] = s;
     }
@@ -735,7 +742,7 @@ __global__ __launch_bounds__(256) void hclt_rows_base_kernel(const HcltNode* __r
   const int j = t % K;
   for (int k = t / K; k < K; k += 256 / K) {
     const int idx = blk2par[((size_t)n * K + k) * K + j];
-    const float x = idx >= 0 ? p1[idx] : -INFINITY, y = idx >= 0 ? p2[idx] : 0.f;
+    const float x = idx >= 0 ? p1[idx] : idx == kBlkOne ? 0.f : -INFINITY, y = idx >= 0 ? p2[idx] : 0.f;
     const float p = expf(x);
     tile[k][j] = p;
     float term = p > 0.f ? p * (x - y + l[j]) : 0.f;
@@ -838,8 +845,18 @@ __global__ __launch_bounds__(256) void hclt_rows_leaf_kl_grad_kernel(const float
 template <int K>
 __global__ void hclt_rows_soft_base2_kernel(const HcltNode* __restrict__ nodes, const int32_t* __restrict__ child_leaf,
                                             const int32_t* __restrict__ pos, int n_inner, const float* __restrict__ leaf_grad,
-                                            size_t vk, const float* __restrict__ pd, float* __restrict__ ell,
+                                            size_t vk, int n_vars, const float* __restrict__ pd, float* __restrict__ ell,
                                             float* __restrict__ base, KlRowStrides rs, int add);
+
+void HcltCircuit::build_block_params() {
+  if (d_blk2par_.n) return;
+  std::vector<int32_t> b2p((size_t)n_inner_ * K_ * K_, kBlkNone);
+  for (size_t i = 0; i < sum_param_src_.size(); ++i) b2p[(size_t)sum_param_src_[i]] = (int32_t)i;
+  for (int nd = 0; nd < n_inner_; ++nd)
+    if (var_of_inner_[nd] >= Vu_)
+      for (int k = 0; k < K_; ++k) b2p[((size_t)nd * K_ + k) * K_ + k] = kBlkOne;
+  d_blk2par_.upload(b2p, stream);
+}
 
 // KL of every row (d_klds, may be null with gradients) and, with d_g1 / d_g2, its gradients in the layout of the inputs
 void HcltCircuit::kld_rows_block(const float* d_p1, const float* d_p2, int64_t sr, int64_t sp, int32_t rows, bool norm,
@@ -848,11 +865,7 @@ void HcltCircuit::kld_rows_block(const float* d_p1, const float* d_p2, int64_t s
   build_kld_tables();
   const int64_t ns = (int64_t)sum_param_src_.size();
   const int64_t n = size(0);
-  if (d_blk2par_.n == 0) {
-    std::vector<int32_t> b2p((size_t)n_inner_ * K_ * K_, -1);
-    for (int64_t i = 0; i < ns; ++i) b2p[(size_t)sum_param_src_[i]] = (int32_t)i;
-    d_blk2par_.upload(b2p, stream);
-  }
+  build_block_params();
   if (d_input_order_.n == 0) d_input_order_.upload(input_order_, stream);
   const float* p1 = rows_packed_in(d_p1, sr, sp, rows, n, d_rows_pk1_, stream);
   const float* p2 = rows_packed_in(d_p2, sr, sp, rows, n, d_rows_pk2_, stream);
@@ -917,7 +930,7 @@ void HcltCircuit::kld_rows_block(const float* d_p1, const float* d_p2, int64_t s
     auto base_pass = [&](const float* leaf_terms, float* up, float* down) {
       PCM_DISPATCH_K(K_, hipLaunchKernelGGL(hclt_rows_base_kernel<KK>, dim3(n_inner_, rc), dim3(256), 0, stream, d_nodes_.p,
                                             d_child_leaf_.p, d_kl_pos_.p, n_inner_, d_blk2par_.p, q1, q2, (size_t)n, leaf_terms,
-                                            vk, ell, base, up, down, rs));
+                                            vk, Vu_, ell, base, up, down, rs));
     };
     if (!with_down) {
       const dim3 lgrid(ceil_div(n_inputs, 16), rc);
@@ -945,7 +958,7 @@ void HcltCircuit::kld_rows_block(const float* d_p1, const float* d_p2, int64_t s
         hipLaunchKernelGGL(hclt_rows_leaf_kl_grad_kernel<false>, ggrid, dim3(256), 0, stream, q1, q2, (size_t)n, (size_t)ns, C_, K_,
                            n_inputs, L, d_input_order_.p, d_kl_tabs_.p + n_inner_, h, nk, vk, kl_leaf, o1, o2);
       PCM_DISPATCH_K(K_, hipLaunchKernelGGL(hclt_rows_soft_base2_kernel<KK>, dim3(n_inner_, rc), dim3(256), 0, stream, d_nodes_.p,
-                                            d_child_leaf_.p, d_kl_pos_.p, n_inner_, kl_leaf, vk, pd, ell, base, rs, 1));
+                                            d_child_leaf_.p, d_kl_pos_.p, n_inner_, kl_leaf, vk, Vu_, pd, ell, base, rs, 1));
       chain(0);
       hipLaunchKernelGGL(hclt_rows_edge_grad_kernel, dim3((unsigned)ceil_div(ns, 256), ceil_div(rc, kEdgeGradRows)), dim3(256), 0,
                          stream, ns, K_, d_sum_param_src_.p, d_kl_tabs_.p, q1, q2, (size_t)n, z, h, nk, rc, o1, o2);
@@ -984,6 +997,7 @@ __global__ __launch_bounds__(256) void hclt_rows_soft_base_kernel(const int32_t*
     const int idx = blk2par[((size_t)n * K + k) * K + j];
     float x = -INFINITY;
     if (idx >= 0) x = (p[idx] + (g ? g[idx] : 0.f)) * inv_t;
+    else if (idx == kBlkOne) x = 0.f;
     float m = x;
 #pragma unroll
     for (int o = K / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, K));
@@ -1071,7 +1085,7 @@ template <int K>
 __global__ __launch_bounds__(256) void hclt_rows_soft_base2_kernel(const HcltNode* __restrict__ nodes,
                                                                    const int32_t* __restrict__ child_leaf,
                                                                    const int32_t* __restrict__ pos, int n_inner,
-                                                                   const float* __restrict__ leaf_grad, size_t vk,
+                                                                   const float* __restrict__ leaf_grad, size_t vk, int n_vars,
                                                                    const float* __restrict__ pd, float* __restrict__ ell,
                                                                    float* __restrict__ base, KlRowStrides rs, int add) {
   __shared__ float l[K];
@@ -1083,7 +1097,7 @@ __global__ __launch_bounds__(256) void hclt_rows_soft_base2_kernel(const HcltNod
   ell += row * rs.vec;
   base += row * rs.vec;
   if (t < K) {
-    float s = leaf_grad[(size_t)nd.var * K + t];
+    float s = nd.var < n_vars ? leaf_grad[(size_t)nd.var * K + t] : 0.f;
     for (int q = 0; q < nd.lc_cnt; ++q) s += leaf_grad[(size_t)child_leaf[nd.lc_off + q] * K + t];
     l[t] = s;
     ell[su * K + t] = s;
@@ -1157,7 +1171,7 @@ __global__ __launch_bounds__(256) void hclt_rows_soft_leaf_kernel(const float* _
 
 void HcltCircuit::gumbel_sample_rows(const float* d_params, int64_t sr, int64_t sp, int32_t rows, const float* d_noise,
                                      float temperature, bool norm_params, float* d_out) {
-  if (!block_queries() || H_ > 0 || missing_)
+  if (!block_ || H_ > 0 || missing_)
     return general_structure()->gumbel_sample_rows(d_params, sr, sp, rows, d_noise, temperature, norm_params, d_out);
   if (!d_params) fail(PCM_ERR_ARG, "parameter matrix is null");
   if (rows < 1) fail(PCM_ERR_ARG, "need at least one parameter row, got %d", rows);
@@ -1168,11 +1182,7 @@ void HcltCircuit::gumbel_sample_rows(const float* d_params, int64_t sr, int64_t 
   build_kld_tables();
   const int64_t ns = (int64_t)sum_param_src_.size();
   const int64_t n = size(0);
-  if (d_blk2par_.n == 0) {
-    std::vector<int32_t> b2p((size_t)n_inner_ * K_ * K_, -1);
-    for (int64_t i = 0; i < ns; ++i) b2p[(size_t)sum_param_src_[i]] = (int32_t)i;
-    d_blk2par_.upload(b2p, stream);
-  }
+  build_block_params();
   const float* p = rows_packed_in(d_params, sr, sp, rows, n, d_rows_pk1_, stream);
   const int W = kl_waves(K_), D = kl_ahead(K_);
   const size_t nk = (size_t)n_inner_ * K_;
@@ -1231,7 +1241,7 @@ void HcltCircuit::gumbel_sample_backward_rows(const float* d_params, int64_t sr,
   // 16-byte rows on every side: the leaf kernel moves four categories at a time
   const bool aligned = C_ % 4 == 0 && n % 4 == 0 && ns % 4 == 0 && (reinterpret_cast<uintptr_t>(d_out_grad) & 15) == 0 &&
                        (!direct || ((reinterpret_cast<uintptr_t>(d_params) | reinterpret_cast<uintptr_t>(d_grads)) & 15) == 0);
-  if (!block_queries() || H_ > 0 || missing_ || !aligned)
+  if (!block_ || H_ > 0 || missing_ || !aligned)
     return general_structure()->gumbel_sample_backward_rows(d_params, sr, sp, rows, d_noise, temperature, norm_params,
                                                             grad_wrt_logparams, d_out_grad, d_grads);
   if (!d_params) fail(PCM_ERR_ARG, "parameter matrix is null");
@@ -1241,11 +1251,7 @@ void HcltCircuit::gumbel_sample_backward_rows(const float* d_params, int64_t sr,
   if (!d_out_grad || !d_grads) fail(PCM_ERR_ARG, "gradient pointer is null");
   if (!(temperature > 0.f)) fail(PCM_ERR_ARG, "temperature must be positive");
   build_kld_tables();
-  if (d_blk2par_.n == 0) {
-    std::vector<int32_t> b2p((size_t)n_inner_ * K_ * K_, -1);
-    for (int64_t i = 0; i < ns; ++i) b2p[(size_t)sum_param_src_[i]] = (int32_t)i;
-    d_blk2par_.upload(b2p, stream);
-  }
+  build_block_params();
   if (d_input_order_.n == 0) d_input_order_.upload(input_order_, stream);
   const float* p = rows_packed_in(d_params, sr, sp, rows, n, d_rows_pk1_, stream);
   float* gout = d_grads;
@@ -1309,7 +1315,7 @@ void HcltCircuit::gumbel_sample_backward_rows(const float* d_params, int64_t sr,
         hipLaunchKernelGGL(hclt_rows_soft_back_leaf_kernel<false>, lgrid, dim3(256), 0, stream, q, (size_t)n, (size_t)ns, C_, K_, Vu_,
                            n_inputs, d_input_order_.p, d_kl_tabs_.p + n_inner_, h, nk, og, vk, leaf_grad, out);
       hipLaunchKernelGGL(hclt_rows_soft_base2_kernel<KK>, dim3(n_inner_, rc), dim3(256), 0, stream, d_nodes_.p, d_child_leaf_.p,
-                         d_kl_pos_.p, n_inner_, leaf_grad, vk, pd, ell, base, rs, 0);
+                         d_kl_pos_.p, n_inner_, leaf_grad, vk, Vu_, pd, ell, base, rs, 0);
       chain(0);   // the gradients of the sum nodes, bottom-up
       hipLaunchKernelGGL(hclt_rows_soft_edge_grad_kernel<KK>, dim3((unsigned)ceil_div(ns, 256), ceil_div(rc, kEdgeGradRows)),
                          dim3(256), 0, stream, ns, d_sum_param_src_.p, d_kl_tabs_.p, d_kl_pos_.p, n_inner_, pd, z, klv, h, nk, rs,
@@ -1329,7 +1335,7 @@ static void check_rows_block_args(const void* p1, const void* p2, int64_t sr, in
 
 void HcltCircuit::kld_rows(const float* d_p1, const float* d_p2, int64_t sr, int64_t sp, int32_t rows, bool norm_params,
                            float* d_out) {
-  if (!block_queries() || H_ > 0 || missing_) return general_structure()->kld_rows(d_p1, d_p2, sr, sp, rows, norm_params, d_out);
+  if (!block_ || H_ > 0 || missing_) return general_structure()->kld_rows(d_p1, d_p2, sr, sp, rows, norm_params, d_out);
   check_rows_block_args(d_p1, d_p2, sr, sp, rows);
   if (!d_out) fail(PCM_ERR_ARG, "output pointer is null");
   kld_rows_block(d_p1, d_p2, sr, sp, rows, norm_params, d_out, nullptr, nullptr);
@@ -1340,7 +1346,7 @@ void HcltCircuit::kld_backward_rows(const float* d_p1, const float* d_p2, int64_
   const bool aligned = C_ % 4 == 0 && size(0) % 4 == 0 && (int64_t)sum_param_src_.size() % 4 == 0 &&
                        ((reinterpret_cast<uintptr_t>(d_p1) | reinterpret_cast<uintptr_t>(d_p2) | reinterpret_cast<uintptr_t>(d_g1) |
                          reinterpret_cast<uintptr_t>(d_g2)) & 15) == 0;
-  if (!block_queries() || H_ > 0 || missing_ || !aligned)
+  if (!block_ || H_ > 0 || missing_ || !aligned)
     return general_structure()->kld_backward_rows(d_p1, d_p2, sr, sp, rows, norm_params, d_g1, d_g2, d_klds);
   check_rows_block_args(d_p1, d_p2, sr, sp, rows);
   if (!d_g1 || !d_g2) fail(PCM_ERR_ARG, "parameter or gradient matrix is null");

@@ -481,6 +481,47 @@ def test_parameter_row_queries_match_oracle(gpu, oracle, kind, R, norm):
         P._lib.check(P._lib.lib.pcm_kld_rows(bpc.handle, None, None, n, 1, R, 0, None))
 
 
+@pytest.mark.parametrize("K,norm", [(16, True), (32, False)])
+@pytest.mark.parametrize("tree", [[-1] + [0] * 8,                                 # eight leaf children: two auxiliary nodes
+                                  [-1, 0, 0, 0, 0, 0, 1, 2, 3, 4, 5],             # five inner children
+                                  [-1, 0, 1, 1, 1, 1, 2, 3, 0, 8, 8, 8, 8, 8]])   # four and five children, mixed
+def test_parameter_rows_on_split_trees(gpu, oracle, tree, K, norm):
+    """The row queries of a tree whose nodes were split by auxiliary ones run on the block kernels: every row against
+    the oracle on the caller's tree."""
+    torch, P = gpu
+    O = oracle
+    from helpers import make_hclt, log_dirichlet
+    V, C, R, T = len(tree), 8, 3, 0.7
+    parent, theta, leaf, _ = make_hclt(V, K, C, 5, parent=np.array(tree, np.int32))
+    bpc = P.hclt_from_clt(parent, C, K)
+    fc = O.bits_compile(O.hclt_dag(parent, K, C, theta, leaf), C, V)
+    rng = np.random.default_rng(K + V)
+    n, ns = bpc.num_parameters(), bpc.num_inner_params()
+    p = np.empty((2, R, n), np.float32)
+    p[:, :, :ns] = np.stack([log_dirichlet(rng, K) for _ in range(2 * R * ns // K)]).reshape(2, R, ns)
+    lf = np.stack([log_dirichlet(rng, C) for _ in range(2 * R * (n - ns) // C)]).reshape(2, R, n - ns)
+    p[:, :, ns:] = np.exp(lf) if norm else lf
+    kl, (g1, g2) = P.kld(bpc, p[0], p[1], norm_params=norm), P.kld_backward(bpc, p[0], p[1], norm_params=norm)
+    noise = _gumbel(rng, (R, ns))
+    og = rng.normal(size=(R, V, C)).astype(np.float32)
+    soft = P.gumbel_sample_rows(bpc, p[0], temperature=T, noise=noise, norm_params=norm)
+    back = P.gumbel_sample_backward_rows(bpc, p[0], og, temperature=T, noise=noise, norm_params=norm)
+    for r in range(R):
+        f1, f2 = _row_oracle(O, fc, p[0, r], ns, norm), _row_oracle(O, fc, p[1, r], ns, norm)
+        klds, ek = O.kld(f1, f2, double=True, norm_params=norm)
+        _, eg1, eg2, lg1, lg2 = O.kld_backward(f1, f2, ek, double=True, norm_params=norm)
+        assert abs(kl[r] - klds[-1]) < KLD_RTOL * abs(klds[-1])
+        for got, want in ((g1[r], _grads_in_param_order(fc, eg1, lg1)), (g2[r], _grads_in_param_order(fc, eg2, lg2))):
+            assert np.abs(got - want).max() < GRAD_RTOL * np.abs(want).max()
+        g = np.zeros(fc.n_edges)
+        g[fc.sum_param_edges()] = noise[r]
+        _, want = O.gumbel_soft(f1, g, T, double=True, norm_params=norm)
+        np.testing.assert_allclose(soft[r], want, rtol=1e-4, atol=1e-7)
+        eg, lg = O.gumbel_soft_backward(f1, g, T, og[r], double=True, norm_params=norm)
+        want = _grads_in_param_order(fc, eg, lg)
+        assert np.abs(back[r] - want).max() < GRAD_RTOL * np.abs(want).max()
+
+
 def test_prealloc_wrappers_run_all_rows_at_once(gpu, oracle):
     """`kld_with_prealloc`, `kld_backward_with_prealloc`, `gumbel_sample_with_prealloc`
     (src/utils/cuda_preallocation.jl:47-78,189-203) with one parameter vector per example and the
