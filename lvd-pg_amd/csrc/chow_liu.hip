@@ -12,10 +12,10 @@
 // p(c) = (c + s)/Z, la[u][a] = log P_u[a]:
 //   MI[u,v] = sum over non-empty cells of g(c(cell))  -  M_u - M_v  +  C^2 * xlogx(p(0))  -  p(0) * C * (L_u + L_v)
 //   g(c) = xlogx(p(c)) - xlogx(p(0)),   M_u = (1/Z) sum_e la[u][x_eu],   L_u = sum_a la[u][a]
-// (the empty cells' terms are the closed-form remainder), so a pair costs two passes over its N examples against a
-// C x C table of counters in LDS -- count; then every example takes its cell's count away with it, and the one that
-// finds a count there adds the cell's term -- and no pass over the table itself.  Up to 65535
-// examples the counters are 16 bits wide and the whole table fits; beyond, they are 32 bits wide
+// (the empty cells' terms are the closed-form remainder).  The sum telescopes over a cell's examples -- the one that
+// raises a count from c to c + 1 brings g(c + 1) - g(c) -- so a pair costs ONE pass over its N examples against a C x C
+// table of counters in LDS: an atomic add that returns the old count, and a look-up of its difference; then the table is
+// cleared.  Up to 65535 examples the counters are 16 bits wide and the whole table fits; beyond, they are 32 bits wide
 // and the table is walked in bands of rows.
 #include "common.hpp"
 #include "chow_liu.hpp"
@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <cmath>
 #include <queue>
+#include <type_traits>
 
 namespace pcm {
 
@@ -63,20 +64,25 @@ __global__ __launch_bounds__(256) void mi_single_kernel(const uint8_t* __restric
   if (t == 0) { stat[2 * v] = M; stat[2 * v + 1] = red[0]; }
 }
 
-// g(c) = xlogx(p(c)) - xlogx(p(0)) for c = 0 .. N, the term of a cell that holds c examples, as a fixed-point integer of
-// kMiFrac fractional bits: |g| < 0.37, a pair adds at most N < 2^17 of them into 64 bits, and integer sums do not
-// depend on which thread adds which term (2^-44 per term is far below the float the sum ends as).
+// dg[c] = g(c + 1) - g(c) for c = 0 .. N - 1, g(c) = xlogx(p(c)) - xlogx(p(0)) the term of a cell that holds c examples
+// as a fixed-point integer of kMiFrac fractional bits: |g| < 0.37, the terms of a pair's cells are fewer than 2^17 and
+// add up in 64 bits, and integer sums do not depend on which thread adds which difference (2^-44 per cell is far below
+// the float the sum ends as).
 constexpr int kMiFrac = 44;
-__global__ void mi_table_kernel(int N, int C, float pc, long long* __restrict__ g) {
+__global__ void mi_table_kernel(int N, int C, float pc, long long* __restrict__ dg) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c > N) return;
+  if (c >= N) return;
   const double Z = (double)N + (double)pc, s = (double)pc / ((double)C * C);
   const double p0 = s / Z, x0 = p0 > 0.0 ? p0 * log(p0) : 0.0;
-  const double p = ((double)c + s) / Z;
-  g[c] = c ? llrint(ldexp(p * log(p) - x0, kMiFrac)) : 0ll;
+  auto g = [&](int64_t n) {
+    if (n == 0) return 0ll;
+    const double p = ((double)n + s) / Z;
+    return (long long)llrint(ldexp(p * log(p) - x0, kMiFrac));
+  };
+  dg[c] = g(c + 1) - g(c);
 }
 
-constexpr int kMiThreads = 1024;
+constexpr int kMiThreads = 1024;   // per workgroup; half of it where several workgroups share a compute unit (mi_launch)
 
 // Calls fn(a, b) for every example of a pair of staged rows; thread t owns examples 4t .. 4t+3
 // (+ 4096 per further round).
@@ -91,60 +97,37 @@ __device__ __forceinline__ void mi_each_example(const uint8_t* __restrict__ xu, 
   }
 }
 
-// The same with the words of the thread's first R rounds already in registers (R = 1, 2, 4 or 8: the host picks the
-// smallest that covers the examples; rounds are masked, not branched around): a pair's three passes read them
-// once, all of them requested before the first is used (a loop of a load and its use per round waits out one memory
-// latency per round and pass), and the next pair's are requested while this pair's passes run -- a persistent workgroup
-// owns its compute unit (the table fills the LDS), so nothing else hides the latency of its rows.
-template <int R>
-struct MiWords { uint32_t u[R], v[R]; };
-
-template <int R>
-__device__ __forceinline__ void mi_load_words(const uint8_t* __restrict__ xu, const uint8_t* __restrict__ xv, int N, int t,
-                                              MiWords<R>& w) {
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int64_t b4 = 4 * (int64_t)t + (int64_t)r * 4 * kMiThreads;
-    w.u[r] = w.v[r] = 0u;
-    if (b4 < N) {   // (the rows are padded to whole words past N)
-      w.u[r] = *reinterpret_cast<const uint32_t*>(xu + b4);
-      w.v[r] = *reinterpret_cast<const uint32_t*>(xv + b4);
-    }
-  }
-}
-
-template <int R, typename F>
-__device__ __forceinline__ void mi_each_example_from(const MiWords<R>& w, const uint8_t* __restrict__ xu,
-                                                     const uint8_t* __restrict__ xv, int N, int t, F&& fn) {
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int64_t b4 = 4 * (int64_t)t + (int64_t)r * 4 * kMiThreads;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (b4 + i < N) fn((int)((w.u[r] >> (8 * i)) & 0xffu), (int)((w.v[r] >> (8 * i)) & 0xffu));
-  }
-  for (int64_t b4 = 4 * (int64_t)t + (int64_t)R * 4 * kMiThreads; b4 < N; b4 += 4 * kMiThreads) {
-    const uint32_t wu = *reinterpret_cast<const uint32_t*>(xu + b4), wv = *reinterpret_cast<const uint32_t*>(xv + b4);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (b4 + i < N) fn((int)((wu >> (8 * i)) & 0xffu), (int)((wv >> (8 * i)) & 0xffu));
-  }
-}
-
-// Sum of acc over the workgroup, then the closed-form remainder; thread 0 writes both halves of the matrix.  su, sv: the
-// two variables' constants (M, L), read when the pair began -- read here they kept the whole workgroup waiting for
-// thread 0's trip to memory.  No barrier behind thread 0: whoever writes `red` next has passed a barrier that thread 0
-// reaches only after this.
+// Sum of acc over the workgroup, then the closed-form remainder; one lane writes both halves of the matrix.  su, sv: the
+// two variables' constants (M, L), read when the pair began -- read here they kept the whole workgroup waiting for a
+// trip to memory.  `red` is the pair's own half of a double buffer: nobody writes it again before two further barriers,
+// so what the first wave does here is behind no barrier of its own.
 struct MiStat { double m, l; };
-__device__ __forceinline__ void mi_finish_pair(long long acc, long long* red, int t, int u, int v, int V, int C, double p0,
-                                               double x0, MiStat su, MiStat sv, float* __restrict__ mi) {
+template <int kCtrl>
+__device__ __forceinline__ long long mi_dpp_add(long long x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)x, kCtrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(x >> 32), kCtrl, 0xf, 0xf, true);
+  return x + (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
+}
+// every lane: the sum over its row of 16 lanes (rotations by 8, 4, 2, 1: no trips through the LDS, which the table's
+// atomics keep busy)
+__device__ __forceinline__ long long mi_row_sum(long long x) {
+  return mi_dpp_add<0x121>(mi_dpp_add<0x122>(mi_dpp_add<0x124>(mi_dpp_add<0x128>(x))));
+}
+__device__ __forceinline__ void mi_leave_sum(long long acc, long long* red, int t) {
+  const long long x = mi_row_sum(acc);
+  long long sum = 0;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-  if ((t & 63) == 0) red[t >> 6] = acc;
-  __syncthreads();
+  for (int l = 0; l < 64; l += 16)
+    sum += (long long)(((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(x >> 32), l) << 32) |
+                       (unsigned)__builtin_amdgcn_readlane((int)(unsigned)x, l));
+  if ((t & 63) == 0) red[t >> 6] = sum;
+}
+template <int T>
+__device__ __forceinline__ void mi_finish_pair(const long long* red, int t, int u, int v, int V, int C, double p0, double x0,
+                                               MiStat su, MiStat sv, float* __restrict__ mi) {
+  if (t >= 16) return;
+  const long long sum = mi_row_sum(t < T / 64 ? red[t] : 0ll);
   if (t == 0) {
-    long long sum = 0;
-    for (int w = 0; w < kMiThreads / 64; ++w) sum += red[w];
     const double tot = ldexp((double)sum, -kMiFrac);
     double val = tot - su.m - sv.m + (double)C * C * x0;
     if (p0 > 0.0) val -= p0 * C * (su.l + sv.l);
@@ -153,99 +136,168 @@ __device__ __forceinline__ void mi_finish_pair(long long acc, long long* red, in
   }
 }
 
-// Pairs (u <= v) in row-major order of the upper triangle, dealt round-robin to persistent
-// workgroups.  At most 65535 examples: a cell's count fits 16 bits, two cells per LDS word.
-template <int R>
-__global__ __launch_bounds__(kMiThreads) void mi_pair_kernel(const uint8_t* __restrict__ xb, int N, int64_t Np, int V, int C,
-                                                             float pc, const long long* __restrict__ g, int g_lds,
-                                                             const double* __restrict__ stat, float* __restrict__ mi) {
-  extern __shared__ unsigned cells[];   // C*C 16-bit counters, two per word | 16 sums | the first g_lds entries of g
+// Rows u, v of the upper triangle's pairs in row-major order, `stride` pairs on at a time.
+struct MiPair { int u, v; };
+__device__ __forceinline__ void mi_advance(MiPair& p, int stride, int V) {
+  p.v += stride;
+  while (p.v >= V && p.u < V) { ++p.u; p.v += p.u - V; }   // (past the end of row u: on into row u + 1, which starts at its own diagonal)
+}
+
+// Words per row of the 16-bit table, an odd number: with rows of 128 words (C = 256) a cell's bank was that of its
+// column alone, and the columns of images bunch around the middle of the grey scale.
+__host__ __device__ constexpr int mi_row_words(int C) { return ((C + 1) / 2) | 1; }
+
+// Pairs (u <= v) in row-major order of the upper triangle, dealt round-robin to persistent workgroups.  At most 65535
+// examples: a cell's count fits 16 bits, two cells per LDS word.  A thread keeps the words of its first R rounds of four
+// examples in registers (R = 1, 2, 4 or 8: the host picks the smallest that covers the examples), all of them requested
+// before the first is used, and the next pair's are requested before this pair's pass: where the table fills the LDS
+// nothing else hides the latency of the rows.
+// What bounds it is the LDS: per 64 examples one atomic with return and one look-up, at 8.5 cycles each without bank
+// conflicts.  `sweep`: the table is cleared by 16-byte stores over all of it, else by a store per example into the
+// cells it touched.  3072 variables, 256 categories (4.72 M pairs): 36 -> 20 ms at 4096 examples, 88 -> 55 at 16384,
+// 170 -> 87 at 32768 against a pass that counts and one that takes the counts away, rows of 128 words and per-pair
+// overheads of 64-bit index arithmetic and shuffles through the LDS.
+template <int T, int R>
+__global__ __launch_bounds__(T) void mi_pair_kernel(const uint8_t* __restrict__ xb, int N, int Np, int V, int C, float pc,
+                                                    const long long* __restrict__ dg, int g_lds, int sweep,
+                                                    const double* __restrict__ stat, float* __restrict__ mi) {
+  extern __shared__ __align__(16) unsigned cells[];   // rows of 16-bit counters | 2 x 16 sums | the first g_lds entries of dg
   const int t = threadIdx.x;
-  const int words = (C * C + 1) / 2;
-  long long* red = reinterpret_cast<long long*>(cells + ((words + 1) & ~1));
-  long long* gl = red + kMiThreads / 64;   // what the LDS has left holds the table over counts from its start: a lookup
-  for (int i = t; i < words; i += kMiThreads) cells[i] = 0u;   // is then no trip to memory (counts past it are rare)
-  for (int i = t; i < g_lds; i += kMiThreads) gl[i] = g[i];
+  const int S = mi_row_words(C), words = (C * S + 3) & ~3;
+  long long* red2 = reinterpret_cast<long long*>(cells + words);
+  long long* gl = red2 + 2 * (kMiThreads / 64);   // what the LDS has left holds the table over counts from its start: a
+  auto clear_all = [&] {                          // look-up is then no trip to memory (counts past it are rare)
+    uint4* p = reinterpret_cast<uint4*>(cells);
+    const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+    int i = t;
+    for (; i + 3 * T < words / 4; i += 4 * T) p[i] = p[i + T] = p[i + 2 * T] = p[i + 3 * T] = zero;
+    for (; i < words / 4; i += T) p[i] = zero;
+  };
+  clear_all();
+  for (int i = t; i < g_lds; i += T) gl[i] = dg[i];
   __syncthreads();
-  const int64_t n_pairs = (int64_t)V * (V + 1) / 2;
   const double Z = (double)N + (double)pc, s = (double)pc / ((double)C * C);
   const double p0 = s / Z, x0 = p0 > 0.0 ? p0 * log(p0) : 0.0;
-  // row u of the triangle starts at pair u*V - u*(u-1)/2
-  int u = 0, un = 0;          // rows of this pair and of the workgroup's next one
-  int64_t row0 = 0, rown = 0;
-  MiWords<R> cur, nxt;
-  if ((int64_t)blockIdx.x < n_pairs) {
-    while ((int64_t)blockIdx.x >= rown + (V - un)) { rown += V - un; ++un; }
-    mi_load_words(xb + (size_t)un * Np, xb + (size_t)(un + (int)(blockIdx.x - rown)) * Np, N, t, cur);
-  }
-  for (int64_t p = blockIdx.x; p < n_pairs; p += gridDim.x) {
-    while (p >= row0 + (V - u)) { row0 += V - u; ++u; }
-    const int v = u + (int)(p - row0);
-    const uint8_t* xu = xb + (size_t)u * Np;
-    const uint8_t* xv = xb + (size_t)v * Np;
-    const MiStat su{stat[2 * u], stat[2 * u + 1]}, sv{stat[2 * v], stat[2 * v + 1]};
-    long long acc = 0;
-    mi_each_example_from(cur, xu, xv, N, t, [&](int a, int b) {
-      const int key = a * C + b;
-      atomicAdd(&cells[key >> 1], 1u << (16 * (key & 1)));
-    });
-    // the next pair's words, on their way while this pair is looked up and cleared
-    const int64_t pn = p + gridDim.x;
-    if (pn < n_pairs) {
-      while (pn >= rown + (V - un)) { rown += V - un; ++un; }
-      mi_load_words(xb + (size_t)un * Np, xb + (size_t)(un + (int)(pn - rown)) * Np, N, t, nxt);
+  uint32_t cu[R], cv[R], nu[R], nv[R];   // words of the pair under way and of the next one
+  auto request = [&](const MiPair& p, uint32_t (&wu)[R], uint32_t (&wv)[R]) {
+    const uint8_t* xu = xb + (size_t)p.u * Np;
+    const uint8_t* xv = xb + (size_t)p.v * Np;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {   // (past the end of a row: its last word, never counted)
+      const unsigned at = (unsigned)min(4 * (t + r * T), Np - 4);
+      wu[r] = *reinterpret_cast<const uint32_t*>(xu + at);
+      wv[r] = *reinterpret_cast<const uint32_t*>(xv + at);
     }
+  };
+  MiPair p{0, 0};
+  mi_advance(p, blockIdx.x, V);
+  if (p.u < V) request(p, cu, cv);
+  int half = 0;
+  while (p.u < V) {
+    const MiStat su{stat[2 * p.u], stat[2 * p.u + 1]}, sv{stat[2 * p.v], stat[2 * p.v + 1]};
+    MiPair pn = p;
+    mi_advance(pn, gridDim.x, V);
+    if (pn.u < V) request(pn, nu, nv);   // on their way while this pair is counted
+    long long acc = 0;
+    // Four examples at a time: their counts are all on the way back before the first is looked up.  Byte i of the words:
+    // row byte_i(u) of the table, word byte_i(v) >> 1 of it, the half by the lowest bit.
+    auto at = [&](uint32_t wu, uint32_t wv, int i) {
+      const uint32_t a = (wu >> (8 * i)) & 0xffu, col = (i ? wv >> (8 * i - 1) : wv << 1) & 0x1fcu;
+      return reinterpret_cast<unsigned*>(reinterpret_cast<char*>(cells) + (__umul24(a, 4 * S) + col));
+    };
+    auto count = [&](uint32_t wu, uint32_t wv, int n) {
+      unsigned old[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t sh = (i ? wv >> (8 * i - 4) : wv << 4) & 16u;
+        old[i] = 0u;
+        if (i < n) old[i] = (atomicAdd(at(wu, wv, i), 1u << sh) >> sh) & 0xffffu;
+      }
+      long long d[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) d[i] = gl[min(old[i], (unsigned)(g_lds - 1))];
+      // (kept apart from the loads below: a choice between the two tables' pointers becomes one flat load, which holds
+      // the LDS and the memory path together)
+      asm volatile("" : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]));
+      if (max(max(old[0], old[1]), max(old[2], old[3])) >= (unsigned)g_lds) {
+        long long far[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) far[i] = dg[min(old[i], (unsigned)(N - 1))];
+        asm volatile("" : "+v"(far[0]), "+v"(far[1]), "+v"(far[2]), "+v"(far[3]));   // waited for in here: the common path
+#pragma unroll                                                                             // waits for no memory
+        for (int i = 0; i < 4; ++i)
+          if (old[i] >= (unsigned)g_lds) d[i] = far[i];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i < n) acc += d[i];
+    };
+    auto wipe = [&](uint32_t wu, uint32_t wv, int n) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i < n) *at(wu, wv, i) = 0u;
+    };
+    // fn(word of u, word of v, examples in it) for the thread's words of the pair, whole rounds without a test per example
+    auto each_word = [&](auto&& fn) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if ((r + 1) * 4 * T <= N) fn(cu[r], cv[r], 4);
+        else if (4 * (t + r * T) < N) fn(cu[r], cv[r], min(4, N - 4 * (t + r * T)));
+      }
+      const uint8_t* xu = xb + (size_t)p.u * Np;
+      const uint8_t* xv = xb + (size_t)p.v * Np;
+      for (int b4 = 4 * (t + R * T); b4 < N; b4 += 4 * T)
+        fn(*reinterpret_cast<const uint32_t*>(xu + b4), *reinterpret_cast<const uint32_t*>(xv + b4), min(4, N - b4));
+    };
+    each_word(count);
+    mi_leave_sum(acc, red2 + half * (kMiThreads / 64), t);
+    __syncthreads();   // every example is counted
+    if (sweep) clear_all(); else each_word(wipe);
     __syncthreads();
-    // look up and clear in one: the first of a cell's examples to come takes the cell's count with it and adds the
-    // cell's term, the others find it empty (the sums are integers: who adds what does not show in the result)
-    mi_each_example_from(cur, xu, xv, N, t, [&](int a, int b) {
-      const int key = a * C + b, sh = 16 * (key & 1);
-      const int cnt = (int)((atomicAnd(&cells[key >> 1], ~(0xffffu << sh)) >> sh) & 0xffffu);
-      if (cnt) acc += cnt < g_lds ? gl[cnt] : g[cnt];
-    });
-    mi_finish_pair(acc, red, t, u, v, V, C, p0, x0, su, sv, mi);   // (its barrier also ends the clearing)
-    cur = nxt;
+    mi_finish_pair<T>(red2 + half * (kMiThreads / 64), t, p.u, p.v, V, C, p0, x0, su, sv, mi);
+    half ^= 1;
+    p = pn;
+#pragma unroll
+    for (int r = 0; r < R; ++r) { cu[r] = nu[r]; cv[r] = nv[r]; }
   }
 }
 
 // The same for any number of examples: 32-bit cells.  A C x C table of them can exceed the LDS, so
-// the categories of u are cut into bands of `band` rows and the three passes run once per band over
+// the categories of u are cut into bands of `band` rows and the pass runs once per band over
 // the examples whose u-category falls into it.
 __global__ __launch_bounds__(kMiThreads) void mi_pair_wide_kernel(const uint8_t* __restrict__ xb, int N, int64_t Np, int V,
-                                                                  int C, int band, float pc, const long long* __restrict__ g,
+                                                                  int C, int band, float pc, const long long* __restrict__ dg,
                                                                   const double* __restrict__ stat, float* __restrict__ mi) {
-  extern __shared__ unsigned cells[];   // band*C counters | 16 sums
+  extern __shared__ __align__(16) unsigned cells[];   // band rows of (C | 1) counters | 2 x 16 sums
   const int t = threadIdx.x;
-  const int words = band * C;
-  long long* red = reinterpret_cast<long long*>(cells + ((words + 1) & ~1));
-  for (int i = t; i < words; i += kMiThreads) cells[i] = 0u;
+  const int S = C | 1, words = (band * S + 3) & ~3;
+  long long* red2 = reinterpret_cast<long long*>(cells + words);
+  auto clear_all = [&] {
+    for (int i = 4 * t; i < words; i += 4 * kMiThreads) *reinterpret_cast<uint4*>(cells + i) = make_uint4(0u, 0u, 0u, 0u);
+  };
+  clear_all();
   __syncthreads();
-  const int64_t n_pairs = (int64_t)V * (V + 1) / 2;
   const double Z = (double)N + (double)pc, s = (double)pc / ((double)C * C);
   const double p0 = s / Z, x0 = p0 > 0.0 ? p0 * log(p0) : 0.0;
-  int u = 0;
-  int64_t row0 = 0;
-  for (int64_t p = blockIdx.x; p < n_pairs; p += gridDim.x) {
-    while (p >= row0 + (V - u)) { row0 += V - u; ++u; }
-    const int v = u + (int)(p - row0);
+  int half = 0;
+  MiPair p{0, 0};
+  for (mi_advance(p, blockIdx.x, V); p.u < V; mi_advance(p, gridDim.x, V)) {
+    const int u = p.u, v = p.v;
     const uint8_t* xu = xb + (size_t)u * Np;
     const uint8_t* xv = xb + (size_t)v * Np;
     const MiStat su{stat[2 * u], stat[2 * u + 1]}, sv{stat[2 * v], stat[2 * v + 1]};
     long long acc = 0;
     for (int a0 = 0; a0 < C; a0 += band) {
       mi_each_example(xu, xv, N, t, [&](int a, int b) {
-        if ((unsigned)(a - a0) < (unsigned)band) atomicAdd(&cells[(a - a0) * C + b], 1u);
+        if ((unsigned)(a - a0) < (unsigned)band) acc += dg[atomicAdd(&cells[(a - a0) * S + b], 1u)];
       });
+      if (a0 + band >= C) mi_leave_sum(acc, red2 + half * (kMiThreads / 64), t);
       __syncthreads();
-      mi_each_example(xu, xv, N, t, [&](int a, int b) {   // look up and clear in one, as above
-        if ((unsigned)(a - a0) < (unsigned)band) {
-          const unsigned cnt = atomicExch(&cells[(a - a0) * C + b], 0u);
-          if (cnt) acc += g[cnt];
-        }
-      });
+      clear_all();
       __syncthreads();
     }
-    mi_finish_pair(acc, red, t, u, v, V, C, p0, x0, su, sv, mi);
+    mi_finish_pair<kMiThreads>(red2 + half * (kMiThreads / 64), t, u, v, V, C, p0, x0, su, sv, mi);
+    half ^= 1;
   }
 }
 
@@ -272,43 +324,58 @@ void mi_launch(const uint8_t* d_data, int64_t stride_ex, int64_t stride_var, con
   PCM_HIP(hipGetDevice(&dev));
   PCM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   PCM_HIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-  const size_t red_bytes = (kMiThreads / 64) * sizeof(double);
+  const size_t red_bytes = 2 * (kMiThreads / 64) * sizeof(long long);
   const bool narrow = N <= 65535;
   int band = C;
   size_t lds;
   int g_lds = 0;
   if (narrow) {
-    const int words = (C * C + 1) / 2;
-    lds = ((size_t)((words + 1) & ~1)) * 4 + red_bytes;
-    // the rest of the LDS -- of half of it where two workgroups fit a compute unit -- holds the start of the g table
-    const size_t whole = std::min<size_t>((size_t)max_lds, 160 * 1024), share = lds <= whole / 4 ? whole / 2 : whole;
-    g_lds = (int)std::min<size_t>((size_t)N + 1, (share - lds) / sizeof(double));
+    lds = ((size_t)(C * mi_row_words(C) + 3) & ~(size_t)3) * 4 + red_bytes;
+    // The rest of the LDS -- of a workgroup's share of it -- holds the start of the dg table.  As many workgroups as
+    // possible, up to four, share a compute unit, each with table space for the counts to expect (a count past it is a
+    // trip to memory): their serial parts overlap (C = 64, 3072 variables, 16384 examples: four of 512 threads 37 ms, two
+    // of 1024 45 ms).
+    const size_t whole = std::min<size_t>((size_t)max_lds, 160 * 1024);
+    const size_t counts = std::min<size_t>((size_t)N, 512 + (size_t)32 * N / ((size_t)C * C));
+    size_t share = whole;
+    for (int n = 4; n > 1 && share == whole; n /= 2)
+      if (lds + counts * sizeof(long long) <= whole / n) share = whole / n;
+    g_lds = (int)std::min<size_t>((size_t)N, (share - lds) / sizeof(long long));
     lds += (size_t)g_lds * sizeof(long long);
   } else {
-    const size_t budget = std::min<size_t>((size_t)max_lds, 160 * 1024) - red_bytes - 8;
-    band = (int)std::min<size_t>((size_t)C, budget / ((size_t)C * 4));
+    const size_t budget = std::min<size_t>((size_t)max_lds, 160 * 1024) - red_bytes - 16;
+    band = (int)std::min<size_t>((size_t)C, budget / ((size_t)(C | 1) * 4));
     if (band < 1) fail(PCM_ERR_UNSUPPORTED, "one row of the pair table does not fit %d bytes of LDS", max_lds);
     band = ceil_div(C, ceil_div(C, band));         // equal bands
-    lds = ((size_t)((band * C + 1) & ~1)) * 4 + red_bytes;
+    lds = ((size_t)(band * (C | 1) + 3) & ~(size_t)3) * 4 + red_bytes;
   }
   if (lds > (size_t)max_lds) fail(PCM_ERR_UNSUPPORTED, "pair table needs %zu bytes of LDS, device offers %d", lds, max_lds);
   pcm_stage(d_data, stride_ex, stride_var, nullptr, N, sh.Np, V, C, w.xb, stream);
   hipLaunchKernelGGL(mi_single_kernel, dim3(V), dim3(256), 0, stream, w.xb, N, sh.Np, C, pseudocount, w.stat);
-  hipLaunchKernelGGL(mi_table_kernel, dim3(ceil_div((int64_t)N + 1, 256)), dim3(256), 0, stream, N, C, pseudocount, w.g);
+  hipLaunchKernelGGL(mi_table_kernel, dim3(ceil_div(N, 256)), dim3(256), 0, stream, N, C, pseudocount, w.g);
   const int64_t n_pairs = (int64_t)V * (V + 1) / 2;
   const int per_cu = std::max<int>(1, (int)(std::min<size_t>((size_t)max_lds, 160 * 1024) / lds));
-  const int grid = (int)std::min<int64_t>(n_pairs, (int64_t)cus * std::min(per_cu, 2));
+  const int grid = (int)std::min<int64_t>(n_pairs, (int64_t)cus * std::min(per_cu, 4));
   if (narrow) {
-    auto pairs = [&](auto kernel) {
+    // clearing the whole table costs what wiping after this many examples costs (measured at C = 256: equal at 16000
+    // examples, 38.9 against 32.5 ms at 8192, 86.8 against 103.5 at 32768; smaller tables favour the sweep a little more)
+    const int sweep = (int64_t)N * 8 > (int64_t)C * mi_row_words(C) * 3 ? 1 : 0;
+    const bool small = per_cu > 1;
+    auto pairs = [&](auto kernel, int threads) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-      hipLaunchKernelGGL(kernel, dim3(grid), dim3(kMiThreads), lds, stream, w.xb, N, sh.Np, V, C, pseudocount, w.g, g_lds, w.stat,
-                         d_mi);
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, stream, w.xb, N, (int)sh.Np, V, C, pseudocount, w.g, g_lds, sweep,
+                         w.stat, d_mi);
     };
-    // rounds of 4 * kMiThreads examples whose words a thread keeps in registers
-    if (N <= 4 * kMiThreads) pairs(&mi_pair_kernel<1>);
-    else if (N <= 8 * kMiThreads) pairs(&mi_pair_kernel<2>);
-    else if (N <= 16 * kMiThreads) pairs(&mi_pair_kernel<4>);
-    else pairs(&mi_pair_kernel<8>);
+    // rounds of 4 examples a thread whose words it keeps in registers
+    auto by_rounds = [&](auto t) {
+      constexpr int T = decltype(t)::value;
+      if (N <= 4 * T) pairs(&mi_pair_kernel<T, 1>, T);
+      else if (N <= 8 * T) pairs(&mi_pair_kernel<T, 2>, T);
+      else if (N <= 16 * T) pairs(&mi_pair_kernel<T, 4>, T);
+      else pairs(&mi_pair_kernel<T, 8>, T);
+    };
+    if (small) by_rounds(std::integral_constant<int, kMiThreads / 2>{});
+    else by_rounds(std::integral_constant<int, kMiThreads>{});
   } else {
     PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&mi_pair_wide_kernel),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));

@@ -117,6 +117,22 @@ def test_pairwise_mi_matches_oracle(gpu, N, V, C, pc):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,V,C", [(1, 2, 256), (3, 3, 255), (1500, 4, 100), (2049, 4, 100), (40000, 3, 64), (20000, 3, 2),
+                                   (12384, 3, 256), (12385, 3, 256), (32769, 3, 129), (16387, 4, 33)])
+def test_pairwise_mi_at_the_edges_of_its_launch_rules(gpu, N, V, C):
+    """Both ways of clearing the table on either side of their line, both workgroup sizes, rounds beyond the words a
+    thread keeps, counts past the part of the term table that the LDS holds (two categories), odd category counts, and
+    a constant column beside the others.  Same tolerance as above."""
+    torch, P = gpu
+    x = _data(N, V, C, N + V + C)
+    x[:, 0] = C - 1
+    want = S.pairwise_mi(x, C, 0.1)
+    got = P.pairwise_MI(torch.from_numpy(x).cuda(), C, 0.1).cpu().numpy()
+    assert np.abs(got - want).max() < 1e-4 * np.abs(want).max()
+    assert np.array_equal(got, got.T)
+
+
+@pytest.mark.gpu
 def test_learned_tree_and_hclt(gpu):
     torch, P = gpu
     x = _data(2000, 30, 8, 11)
