@@ -398,6 +398,39 @@ void pairwise_mi(const uint8_t* d_data, int64_t stride_ex, int64_t stride_var, i
   PCM_HIP(hipStreamSynchronize(stream));   // the scratch arrays die with this call
 }
 
+// One vertex of Prim's algorithm: its row's better links, and the largest of the vertices still outside (those inside
+// hold +inf in `best`, which no row beats, and are capped at -inf in `key`, the comparison).  Eight vertices at a time.
+using f8 = float __attribute__((ext_vector_type(8)));
+using i8 = int32_t __attribute__((ext_vector_type(8)));
+static float prim_take_row(const float* row, int32_t pick, int V, float* best, int32_t* link, const float* cap, float* key) {
+  f8 top = -INFINITY;
+  int v = 0;
+  for (; v + 8 <= V; v += 8) {
+    f8 r, b, c;
+    i8 l;
+    std::memcpy(&r, row + v, sizeof r);
+    std::memcpy(&b, best + v, sizeof b);
+    std::memcpy(&c, cap + v, sizeof c);
+    std::memcpy(&l, link + v, sizeof l);
+    const i8 better = r > b;
+    b = better ? r : b;
+    l = better ? (i8)pick : l;
+    const f8 k = b < c ? b : c;
+    top = k > top ? k : top;
+    std::memcpy(best + v, &b, sizeof b);
+    std::memcpy(link + v, &l, sizeof l);
+    std::memcpy(key + v, &k, sizeof k);
+  }
+  float most = -INFINITY;
+  for (int q = 0; q < 8; ++q) most = std::max(most, top[q]);
+  for (; v < V; ++v) {
+    if (row[v] > best[v]) { best[v] = row[v]; link[v] = pick; }
+    key[v] = std::min(best[v], cap[v]);
+    most = std::max(most, key[v]);
+  }
+  return most;
+}
+
 // Maximum spanning tree of a dense symmetric weight matrix (Prim; among equal weights the
 // lowest vertex index wins), rooted at the lowest-numbered centre of the tree (the vertex of
 // least eccentricity), as a parent array with -1 at the root.
@@ -405,22 +438,21 @@ void chow_liu_tree(const float* mi, int V, int32_t* parent_out) {
   if (!mi || !parent_out) fail(PCM_ERR_ARG, "matrix or output pointer is null");
   if (V < 1) fail(PCM_ERR_SHAPE, "num_vars must be positive, got %d", V);
   std::vector<float> best(V, -INFINITY);
-  std::vector<int32_t> link(V, -1);
-  std::vector<char> in(V, 0);
+  std::vector<int32_t> link(V, 0);
   std::vector<std::vector<int32_t>> adj(V);
-  in[0] = 1;
-  for (int v = 1; v < V; ++v) { best[v] = mi[v]; link[v] = 0; }
+  best[0] = INFINITY;
+  std::vector<float> cap(V, INFINITY), key(V);
+  cap[0] = -INFINITY;
+  int pick = 0;
   for (int it = 1; it < V; ++it) {
-    int pick = -1;
-    for (int v = 0; v < V; ++v)
-      if (!in[v] && (pick < 0 || best[v] > best[pick])) pick = v;
-    if (!(best[pick] > -INFINITY)) fail(PCM_ERR_ARG, "mutual information matrix holds NaN or -inf in row %d", pick);
-    in[pick] = 1;
+    const float most = prim_take_row(mi + (size_t)pick * V, pick, V, best.data(), link.data(), cap.data(), key.data());
+    if (!(most > -INFINITY)) fail(PCM_ERR_ARG, "mutual information matrix holds NaN or -inf in row %d",
+                                  (int)(std::find(cap.begin(), cap.end(), INFINITY) - cap.begin()));
+    pick = (int)(std::find(key.begin(), key.end(), most) - key.begin());
+    best[pick] = INFINITY;
+    cap[pick] = -INFINITY;
     adj[pick].push_back(link[pick]);
     adj[link[pick]].push_back(pick);
-    const float* row = mi + (size_t)pick * V;
-    for (int v = 0; v < V; ++v)
-      if (!in[v] && row[v] > best[v]) { best[v] = row[v]; link[v] = pick; }
   }
   for (auto& a : adj) std::sort(a.begin(), a.end());
   // centre: peel leaves layer by layer; the last one or two vertices are the centres
