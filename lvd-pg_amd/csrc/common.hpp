@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "../../include/pcmi355.h"
+#include "host_stage.hpp"
 
 namespace pcm {
 
@@ -138,6 +139,11 @@ struct pcm_circuit {
   // fscale of mini_batch_em_beta (src-jl/learning/em.jl:293, flow.jl:120-370): flows that feed the accumulators hand
   // a sum node's flow down in shares proportional to (posterior share)^(1 / flow_scale); 1: the ordinary flows
   float flow_scale = 1.f;
+  std::shared_ptr<pcm::HostStage> host_stage;   // held from the first large transfer on
+  pcm::HostStage& stage() {
+    if (!host_stage) host_stage = pcm::HostStage::shared();
+    return *host_stage;
+  }
   virtual ~pcm_circuit() {}
   virtual int64_t size(int what) const = 0;
   virtual void index_table(int which, int64_t* out, int64_t n) const = 0;

@@ -74,9 +74,6 @@ HcltCircuit::HcltCircuit(const int32_t* parent, int V, int K, int C, int num_hea
                               "every tile in LDS); use one handle per tree");
   if (!forest_) build_param_order();
 
-  // uniform parameters
-  std::vector<float> theta((size_t)Vu_ * K_ * K_, -std::log((float)K_));
-  std::vector<float> leaf((size_t)Vu_ * K_ * C_, -std::log((float)C_));
   d_leaf_.alloc((size_t)V_ * C_ * K_);
   d_logtheta_.alloc((size_t)n_inner_ * K_ * K_ + (size_t)T_ * H_ * K_);   // the head rows sit behind the blocks
   d_Wf_.alloc((size_t)n_inner_ * K_ * K_);
@@ -95,7 +92,7 @@ HcltCircuit::HcltCircuit(const int32_t* parent, int V, int K, int C, int num_hea
   d_leaf_flow_.alloc((size_t)V_ * C_ * K_);
   d_edge_aggr_.zero();
   d_leaf_flow_.zero();
-  set_block_params(theta.data(), leaf.data());
+  set_uniform();
 }
 
 // The lean walk kernels hold three children per tree node.  A forest meets that by construction: a node with
@@ -1077,39 +1074,65 @@ void HcltCircuit::heads_forward(const HcltDev& d, const float* d_mask, float* d_
   check_launch("heads_forward");
 }
 
+// the blocks of the tree nodes from a [Vu_][K][K] device array (null: uniform rows), and the operand layouts behind them
+void HcltCircuit::take_blocks(const float* d_theta) {
+  hipLaunchKernelGGL(hclt_blocks_in_kernel, dim3(n_inner_), dim3(256), 0, stream, d_nodes_.p, Vu_, K_, H_, d_theta,
+                     -std::log((float)K_), d_logtheta_.p);
+  check_launch("blocks_in");
+  rebuild_w();
+}
+
+void HcltCircuit::set_uniform() {
+  take_blocks(nullptr);
+  const int64_t own = (int64_t)Vu_ * C_ * K_, aux = (int64_t)(V_ - Vu_) * C_ * K_;   // (auxiliary variables: log 1 whatever the category)
+  hipLaunchKernelGGL(hclt_fill_kernel, dim3((unsigned)ceil_div(own, 256)), dim3(256), 0, stream, d_leaf_.p, own, -std::log((float)C_));
+  if (aux) hipLaunchKernelGGL(hclt_fill_kernel, dim3((unsigned)ceil_div(aux, 256)), dim3(256), 0, stream, d_leaf_.p + own, aux, 0.f);
+  check_launch("uniform parameters");
+  general_stale_ = true;
+  leaf_changed();
+  PCM_HIP(hipStreamSynchronize(stream));   // (the caller may go on on another stream)
+}
+
+// The caller's arrays go to the device as they are and are turned into the engine's layouts there (3072 variables, K = 32:
+// 32 -> 3.3 ms, and 36 -> 3.4 ms the other way, against one thread of the host over the leaf tables).
 void HcltCircuit::set_block_params(const float* theta, const float* leaf) {
-  const int K = K_, C = C_;
+  const size_t nt = (size_t)Vu_ * K_ * K_, nl = (size_t)Vu_ * K_ * C_;
+  d_param_vec_.ensure(std::max(theta ? nt : 0, leaf ? nl : 0));
   if (theta) {
-    std::vector<float> lt((size_t)n_inner_ * K * K);
-    for (int n = 0; n < n_inner_; ++n) {
-      float* dst = lt.data() + (size_t)n * K * K;
-      if (var_of_inner_[n] >= Vu_) {   // auxiliary node: identity
-        for (int i = 0; i < K * K; ++i) dst[i] = (i / K == i % K) ? 0.f : -INFINITY;
-        continue;
-      }
-      const float* src = theta + (size_t)var_of_inner_[n] * K * K;
-      std::copy(src, src + (size_t)K * K, dst);
-      if (parent_[var_of_inner_[n]] < 0) {
-        if (H_ > 0) {   // multi-head: identity block, the heads have their own rows
-          for (int i = 0; i < K * K; ++i) dst[i] = (i / K == i % K) ? 0.f : -INFINITY;
-        } else {
-          for (int i = K; i < K * K; ++i) dst[i] = -INFINITY;   // the root keeps one sum node
-        }
-      }
-    }
-    PCM_HIP(hipMemcpyAsync(d_logtheta_.p, lt.data(), lt.size() * sizeof(float), hipMemcpyHostToDevice, stream));
-    PCM_HIP(hipStreamSynchronize(stream));
-    rebuild_w();
+    stage().to_device(d_param_vec_.p, theta, nt * sizeof(float), stream);
+    take_blocks(d_param_vec_.p);
   }
   general_stale_ = true;
   if (leaf) {
-    std::vector<float> t((size_t)V_ * C * K, 0.f);   // (auxiliary variables: log 1 whatever the category)
-    for (int v = 0; v < Vu_; ++v)
-      for (int j = 0; j < K; ++j)
-        for (int c = 0; c < C; ++c) t[((size_t)v * C + c) * K + j] = leaf[((size_t)v * K + j) * C + c];
-    PCM_HIP(hipMemcpyAsync(d_leaf_.p, t.data(), t.size() * sizeof(float), hipMemcpyHostToDevice, stream));
-    PCM_HIP(hipStreamSynchronize(stream));
+    stage().to_device(d_param_vec_.p, leaf, nl * sizeof(float), stream);
+    leaf_vector(false, nullptr, d_leaf_.p, d_param_vec_.p);
     leaf_changed();
+  }
+  PCM_HIP(hipStreamSynchronize(stream));
+}
+
+void HcltCircuit::leaf_vector(bool to_vector, const int32_t* in_pos, float* d_leaf, float* d_vec) {
+  const int cats = std::min(64, 16384 / (K_ + 1));   // 64 KB of LDS at most, whatever the hidden size
+  const dim3 grid(Vu_, ceil_div(C_, cats));
+  const size_t lds = (size_t)cats * (K_ + 1) * sizeof(float);
+  if (to_vector) hipLaunchKernelGGL(hclt_leaf_vector_kernel<true>, grid, dim3(256), lds, stream, d_leaf, in_pos, K_, C_, cats, d_vec);
+  else hipLaunchKernelGGL(hclt_leaf_vector_kernel<false>, grid, dim3(256), lds, stream, d_leaf, in_pos, K_, C_, cats, d_vec);
+  check_launch("leaf_vector");
+}
+
+// an engine array of blocks and one of leaf rows as the caller holds them
+void HcltCircuit::fetch_blocks(const float* d_blocks, float* d_leaf, float* theta, float* leaf) {
+  const size_t nt = (size_t)Vu_ * K_ * K_, nl = (size_t)Vu_ * K_ * C_;
+  d_param_vec_.ensure(std::max(theta ? nt : 0, leaf ? nl : 0));
+  if (theta) {
+    hipLaunchKernelGGL(hclt_fill_kernel, dim3((unsigned)ceil_div((int64_t)nt, 256)), dim3(256), 0, stream, d_param_vec_.p, (int64_t)nt, 0.f);
+    hipLaunchKernelGGL(hclt_blocks_out_kernel, dim3(n_inner_), dim3(256), 0, stream, d_nodes_.p, Vu_, K_ * K_, d_blocks, d_param_vec_.p);
+    check_launch("blocks_out");
+    stage().to_host(theta, d_param_vec_.p, nt * sizeof(float), stream);
+  }
+  if (leaf) {
+    leaf_vector(true, nullptr, d_leaf, d_param_vec_.p);
+    stage().to_host(leaf, d_param_vec_.p, nl * sizeof(float), stream);
   }
 }
 
@@ -1184,37 +1207,15 @@ void HcltCircuit::get_heads(float* heads) {
   sync_checked();
 }
 
-static void fetch(std::vector<float>& h, const float* d, size_t n, hipStream_t s) {
-  h.resize(n);
-  PCM_HIP(hipMemcpyAsync(h.data(), d, n * sizeof(float), hipMemcpyDeviceToHost, s));
-  PCM_HIP(hipStreamSynchronize(s));
-}
-
 void HcltCircuit::get_block_params(float* theta, float* leaf) {
   sync_checked();   // (a void pass is reported before anything that came after it is handed out)
-  const int K = K_, C = C_;
-  std::vector<float> h;
-  if (theta) {
-    fetch(h, d_logtheta_.p, d_logtheta_.n, stream);
-    std::fill(theta, theta + (size_t)Vu_ * K * K, 0.f);
-    for (int n = 0; n < n_inner_; ++n)
-      if (var_of_inner_[n] < Vu_)
-        std::copy(h.begin() + (size_t)n * K * K, h.begin() + (size_t)(n + 1) * K * K,
-                  theta + (size_t)var_of_inner_[n] * K * K);
-  }
-  if (leaf) {
-    fetch(h, d_leaf_.p, d_leaf_.n, stream);
-    for (int v = 0; v < Vu_; ++v)
-      for (int j = 0; j < K; ++j)
-        for (int c = 0; c < C; ++c) leaf[((size_t)v * K + j) * C + c] = h[((size_t)v * C + c) * K + j];
-  }
+  fetch_blocks(d_logtheta_.p, d_leaf_.p, theta, leaf);
 }
 
 void HcltCircuit::get_block_flows(float* edge_aggr, float* leaf_flow) {
   sync_checked();
   if (!have_flows_) fail(PCM_ERR_STATE, "no flows have been computed on this circuit yet");
   const int K = K_, C = C_;
-  std::vector<float> h;
   if (flows_in_general_ || (!block_ && !wide_)) {   // from the layered engine's accumulators: up-edge / input-node order -> blocks
     std::vector<float> ea((size_t)n_edges_), lf((size_t)Vu_ * K * C);
     general_->get_aggregates(ea.data(), n_edges_, lf.data(), (int64_t)lf.size());
@@ -1231,20 +1232,7 @@ void HcltCircuit::get_block_flows(float* edge_aggr, float* leaf_flow) {
         std::copy(lf.begin() + q * C, lf.begin() + (q + 1) * C, leaf_flow + (size_t)input_order_[q] * C);
     return;
   }
-  if (edge_aggr) {
-    fetch(h, d_edge_aggr_.p, d_edge_aggr_.n, stream);
-    std::fill(edge_aggr, edge_aggr + (size_t)Vu_ * K * K, 0.f);
-    for (int n = 0; n < n_inner_; ++n)
-      if (var_of_inner_[n] < Vu_)
-        std::copy(h.begin() + (size_t)n * K * K, h.begin() + (size_t)(n + 1) * K * K,
-                  edge_aggr + (size_t)var_of_inner_[n] * K * K);
-  }
-  if (leaf_flow) {
-    fetch(h, d_leaf_flow_.p, d_leaf_flow_.n, stream);
-    for (int v = 0; v < Vu_; ++v)
-      for (int j = 0; j < K; ++j)
-        for (int c = 0; c < C; ++c) leaf_flow[((size_t)v * K + j) * C + c] = h[((size_t)v * C + c) * K + j];
-  }
+  fetch_blocks(d_edge_aggr_.p, d_leaf_flow_.p, edge_aggr, leaf_flow);
 }
 
 void HcltCircuit::vectorize(float* out, int64_t n) {
@@ -1258,12 +1246,9 @@ void HcltCircuit::vectorize(float* out, int64_t n) {
   if (ns > 0)
     hipLaunchKernelGGL(hclt_params_gather_kernel, dim3((unsigned)ceil_div(ns, 256)), dim3(256), 0, stream, ns,
                        d_sum_param_src_.p, d_logtheta_.p, d_param_vec_.p);
-  hipLaunchKernelGGL(hclt_leaf_vector_kernel<true>, dim3(Vu_, ceil_div(C_, kLeafVecCats)), dim3(256),
-                     (size_t)kLeafVecCats * (K_ + 1) * sizeof(float), stream, d_leaf_.p, d_in_pos_.p, K_, C_,
-                     d_param_vec_.p + ns);
+  leaf_vector(true, d_in_pos_.p, d_leaf_.p, d_param_vec_.p + ns);
   check_launch("vectorize");
-  PCM_HIP(hipMemcpyAsync(out, d_param_vec_.p, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, stream));
-  PCM_HIP(hipStreamSynchronize(stream));
+  stage().to_host(out, d_param_vec_.p, (size_t)n * sizeof(float), stream);
 }
 
 void HcltCircuit::update_parameters(const float* in, int64_t n) {
@@ -1273,15 +1258,12 @@ void HcltCircuit::update_parameters(const float* in, int64_t n) {
   if (!in) fail(PCM_ERR_ARG, "parameter vector is null");
   const int64_t ns = (int64_t)sum_param_src_.size();
   d_param_vec_.ensure((size_t)n);
-  PCM_HIP(hipMemcpyAsync(d_param_vec_.p, in, (size_t)n * sizeof(float), hipMemcpyHostToDevice, stream));
+  stage().to_device(d_param_vec_.p, in, (size_t)n * sizeof(float), stream);
   if (ns > 0)
     hipLaunchKernelGGL(hclt_params_scatter_kernel, dim3((unsigned)ceil_div(ns, 256)), dim3(256), 0, stream, ns,
                        d_sum_param_src_.p, d_param_vec_.p, d_logtheta_.p);
-  hipLaunchKernelGGL(hclt_leaf_vector_kernel<false>, dim3(Vu_, ceil_div(C_, kLeafVecCats)), dim3(256),
-                     (size_t)kLeafVecCats * (K_ + 1) * sizeof(float), stream, d_leaf_.p, d_in_pos_.p, K_, C_,
-                     d_param_vec_.p + ns);
+  leaf_vector(false, d_in_pos_.p, d_leaf_.p, d_param_vec_.p + ns);
   check_launch("update_parameters");
-  PCM_HIP(hipStreamSynchronize(stream));   // the caller's vector is free again
   rebuild_w();
   general_stale_ = true;
   leaf_changed();

@@ -378,6 +378,10 @@ class HcltCircuit : public pcm_circuit {
   HcltDev dev(int batch) const;
   void stage_batch(const BatchRef& b, bool tiles = true);
   void rebuild_w();
+  void take_blocks(const float* d_theta);
+  void set_uniform();
+  void leaf_vector(bool to_vector, const int32_t* in_pos, float* d_leaf, float* d_vec);
+  void fetch_blocks(const float* d_blocks, float* d_leaf, float* theta, float* leaf);
   bool lean_fits(int batch) const;
   void run_forward(const HcltDev& d, float* d_ll, int keep = kKeepAll);
   void run_backward(const HcltDev& d);

@@ -737,25 +737,53 @@ __global__ void hclt_params_scatter_kernel(int64_t ns, const int64_t* __restrict
   if (i < ns) logtheta[src[i]] = vec[i];
 }
 
-constexpr int kLeafVecCats = 64;
+// The block arrays [n_inner][K][K] of the engine as the caller holds them, [variables][K][K] (rows of leaf tree nodes
+// stay what they are), and back.  A workgroup takes a tree node.  In from the caller (theta null: uniform), what no
+// parameter stands for is set: an auxiliary node's block and a multi-head root's are the identity, a single root keeps
+// its first sum node.
+__global__ __launch_bounds__(256) void hclt_blocks_out_kernel(const HcltNode* __restrict__ nodes, int n_vars, int kk,
+                                                              const float* __restrict__ blocks, float* __restrict__ theta) {
+  const int n = blockIdx.x, v = nodes[n].var;
+  if (v >= n_vars) return;
+  for (int i = threadIdx.x; i < kk; i += 256) theta[(size_t)v * kk + i] = blocks[(size_t)n * kk + i];
+}
 
+__global__ __launch_bounds__(256) void hclt_blocks_in_kernel(const HcltNode* __restrict__ nodes, int n_vars, int K, int heads,
+                                                             const float* __restrict__ theta, float uniform,
+                                                             float* __restrict__ blocks) {
+  const int n = blockIdx.x, v = nodes[n].var, kk = K * K;
+  const bool root = nodes[n].parent < 0, identity = v >= n_vars || (root && heads);
+  for (int i = threadIdx.x; i < kk; i += 256) {
+    float x = identity ? (i / K == i % K ? 0.f : -INFINITY) : theta ? theta[(size_t)v * kk + i] : uniform;
+    if (root && !heads && i >= K) x = -INFINITY;
+    blocks[(size_t)n * kk + i] = x;
+  }
+}
+
+__global__ void hclt_fill_kernel(float* __restrict__ p, int64_t n, float value) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = value;
+}
+
+// Leaf tables [V][C][K] <-> runs of C values per input node: at in_pos[v * K + j] (parameter order), or at v * K + j
+// where in_pos is null ([V][K][C], the block form of the C ABI).  A workgroup turns `cats` categories of a variable in LDS.
 template <bool kToVector>
 __global__ __launch_bounds__(256) void hclt_leaf_vector_kernel(float* __restrict__ leaf, const int32_t* __restrict__ in_pos,
-                                                               int K, int C, float* __restrict__ vec) {
-  extern __shared__ float turn[];   // [kLeafVecCats][K + 1]
-  const int v = blockIdx.x, c0 = blockIdx.y * kLeafVecCats, nc = min(kLeafVecCats, C - c0);
+                                                               int K, int C, int cats, float* __restrict__ vec) {
+  extern __shared__ float turn[];   // [cats][K + 1]
+  const int v = blockIdx.x, c0 = blockIdx.y * cats, nc = min(cats, C - c0);
   float* rows = leaf + ((size_t)v * C + c0) * K;
   if (kToVector) {
     for (int i = threadIdx.x; i < nc * K; i += 256) turn[(i / K) * (K + 1) + i % K] = rows[i];
     __syncthreads();
     for (int i = threadIdx.x; i < nc * K; i += 256) {
       const int j = i / nc, cc = i % nc;
-      vec[(size_t)in_pos[v * K + j] * C + c0 + cc] = turn[cc * (K + 1) + j];
+      vec[(in_pos ? (size_t)in_pos[v * K + j] : (size_t)v * K + j) * C + c0 + cc] = turn[cc * (K + 1) + j];
     }
   } else {
     for (int i = threadIdx.x; i < nc * K; i += 256) {
       const int j = i / nc, cc = i % nc;
-      turn[cc * (K + 1) + j] = vec[(size_t)in_pos[v * K + j] * C + c0 + cc];
+      turn[cc * (K + 1) + j] = vec[(in_pos ? (size_t)in_pos[v * K + j] : (size_t)v * K + j) * C + c0 + cc];
     }
     __syncthreads();
     for (int i = threadIdx.x; i < nc * K; i += 256) rows[i] = turn[(i / K) * (K + 1) + i % K];

@@ -605,9 +605,8 @@ void HcltCircuit::kld_backward(pcm_circuit* q, float* gp, float* gq, int64_t n) 
   d1.alloc((size_t)std::max<int64_t>(n, 1));
   d2.alloc((size_t)std::max<int64_t>(n, 1));
   kld_backward_dev(q, d1.p, d2.p, n);
-  PCM_HIP(hipMemcpyAsync(gp, d1.p, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, stream));
-  PCM_HIP(hipMemcpyAsync(gq, d2.p, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, stream));
-  PCM_HIP(hipStreamSynchronize(stream));
+  stage().to_host(gp, d1.p, (size_t)n * sizeof(float), stream);
+  stage().to_host(gq, d2.p, (size_t)n * sizeof(float), stream);
 }
 
 void HcltCircuit::adam_step(const float* d_grad, float* d_params, float* d_m, float* d_v, float lr, float b1,

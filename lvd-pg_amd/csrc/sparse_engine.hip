@@ -1753,12 +1753,11 @@ static void fetch(std::vector<float>& h, const float* d, size_t n, hipStream_t s
 
 void SparseCircuit::vectorize(float* out, int64_t n) {
   if (n != size(0)) fail(PCM_ERR_ARG, "parameter vector has %lld entries, circuit has %lld", (long long)n, (long long)size(0));
-  std::vector<float> lp, lf;
+  std::vector<float> lp;
   fetch(lp, d_logp_.p, fc_.n_edges(), stream);
-  fetch(lf, d_leaf_.p, fc_.leaf_logp.size(), stream);
   const size_t ns = fc_.param2edge.size();
   for (size_t i = 0; i < ns; ++i) out[i] = lp[fc_.param2edge[i] - 1];
-  std::copy(lf.begin(), lf.end(), out + ns);
+  stage().to_host(out + ns, d_leaf_.p, fc_.leaf_logp.size() * sizeof(float), stream);
 }
 
 void SparseCircuit::update_parameters(const float* in, int64_t n) {
@@ -1769,7 +1768,7 @@ void SparseCircuit::update_parameters(const float* in, int64_t n) {
   for (size_t i = 0; i < ns; ++i) lp[fc_.param2edge[i] - 1] = in[i];
   if (!lp.empty()) PCM_HIP(hipMemcpyAsync(d_logp_.p, lp.data(), lp.size() * sizeof(float), hipMemcpyHostToDevice, stream));
   if (!fc_.leaf_logp.empty())
-    PCM_HIP(hipMemcpyAsync(d_leaf_.p, in + ns, fc_.leaf_logp.size() * sizeof(float), hipMemcpyHostToDevice, stream));
+    stage().to_device(d_leaf_.p, in + ns, fc_.leaf_logp.size() * sizeof(float), stream);
   PCM_HIP(hipStreamSynchronize(stream));
 }
 

@@ -123,6 +123,50 @@ def test_scores_do_not_depend_on_the_batch_size(gpu, K, V):
     assert torch.equal(P.loglikelihoods(a, d, batch_size=4499), want)
 
 
+@pytest.mark.parametrize("K,V,C,tree", [(16, 9, 7, None), (32, 700, 256, None), (8, 6, 5, None), (128, 5, 70, None),
+                                        (300, 2, 3, None), (16, 9, 5, [-1] + [0] * 8)])
+def test_parameters_come_back_as_they_went_in(gpu, K, V, C, tree):
+    """Block arrays and the parameter vector through the host copies of both sizes (plain below 1 MB, staged above: 23 MB
+    of leaf tables at V = 700) and the device-side layout changes, auxiliary nodes and hidden sizes without block kernels
+    included; a fresh handle is uniform."""
+    torch, P = gpu
+    rng = np.random.default_rng(K + V)
+    parent = np.array(tree, np.int32) if tree else np.array([-1] + [(i - 1) // 2 for i in range(1, V)], np.int32)
+    c = P.hclt_from_clt(parent, C, K)
+    inner = np.bincount(parent[1:], minlength=V) > 0
+    th0, lf0 = c.get_params()
+    assert np.allclose(lf0, -np.log(C)) and np.allclose(th0[inner][1:], -np.log(K)) and not th0[~inner].any()
+    assert np.allclose(th0[0, 0], -np.log(K)) and np.isneginf(th0[0, 1:]).all()
+    th, lf = rng.normal(size=(V, K, K)).astype(np.float32), rng.normal(size=(V, K, C)).astype(np.float32)
+    c.set_params(th, lf)
+    th1, lf1 = c.get_params()
+    assert np.array_equal(lf1, lf) and np.array_equal(th1[inner][1:], th[inner][1:]) and np.array_equal(th1[0, 0], th[0, 0])
+    vec = P.vectorize_parameters(c)
+    d = P.hclt_from_clt(parent, C, K)
+    P.update_parameters(d, vec)
+    th2, lf2 = d.get_params()
+    assert np.array_equal(th2, th1) and np.array_equal(lf2, lf1) and np.array_equal(P.vectorize_parameters(d), vec)
+
+
+def test_parameter_copies_from_several_threads(gpu):
+    """Transfers of several circuits at a time queue up at the shared pinned buffers."""
+    torch, P = gpu
+    from concurrent.futures import ThreadPoolExecutor
+    V, K, C = 90, 32, 256
+    parent = np.array([-1] + [(i - 1) // 2 for i in range(1, V)], np.int32)
+
+    def trip(seed):
+        c = P.hclt_from_clt(parent, C, K)
+        v = np.random.default_rng(seed).normal(size=c.num_parameters()).astype(np.float32)
+        for _ in range(3):
+            P.update_parameters(c, v)
+            if not np.array_equal(P.vectorize_parameters(c), v):
+                return False
+        return True
+    with ThreadPoolExecutor(4) as pool:
+        assert all(pool.map(trip, range(8)))
+
+
 def test_ragged_batch_and_example_ids(gpu, oracle):
     rng = np.random.default_rng(5)
     idx = rng.permutation(200)[:37].astype(np.int32)
