@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <map>
 #include <numeric>
 #include <tuple>
 #include <type_traits>
@@ -1195,16 +1196,24 @@ __global__ __launch_bounds__(256) void sparse_product_edge_kernel(const int2* __
 // Dense groups: sum nodes of one layer over one and the same set of (prime, sub) children (each may list them in an
 // order of its own), at least kGroupMinSide sums over at least kGroupMinSide children and at most kGroupMaxSide of
 // either (more sums: several groups over the same children).  group_of[node] = group or -1; edge_slot[edge] = the
-// child's number among all groups' children (its "slot") for the edges of a group's first sum, -1 for all others.
+// child's number among all groups' children (its "slot") for the edge of the first sum of a group that has it, -1 for all others.
+// Masked groups: sums that are in no such group -- pruning leaves the sums of one tree node with different subsets of
+// its products -- over the union of their children, W zero where a sum lacks a child; in reach of each other through
+// shared children, a layer at a time.  A block costs the same however thin it is (and a layer that is all blocks joins
+// the walks), an edge at a time the layer kernels cost little less for few edges: 192 variables, 128 heads, 16 batches of
+// 512, K = 32: 6.3 ms as blocks at any share of the pairs, edge by edge 9.9 at 60 %, 8.2 at 30 %, 8.0 at 15 %, 7.8 at 10
+// and 5 % (4 batches of 4096: 3.6 against 5.0 at 30 %, 4.4 at 10 %; K = 16, 512: 4.05 against 7.2 at 60 %, 7.0 at 30 %).
+// So the line is only one pair in kMaskedShare, two children of 32: sums that merely touch stay apart.
 // PCMI355_DENSE_GROUPS=0 in the environment keeps every node on the layer kernels (for comparisons).
-constexpr int kGroupMinSide = 4, kGroupMinEdges = 64, kGroupMaxSide = 128;
+constexpr int kGroupMinSide = 4, kGroupMinEdges = 64, kGroupMaxSide = 128, kMaskedShare = 16;
 static_assert(sizeof(GroupRec) == 2 * sizeof(int4), "a group's record is uploaded as two int4");
 
 void SparseCircuit::build_groups(std::vector<int32_t>& group_of, std::vector<int32_t>& edge_slot) {
   const int64_t nn = fc_.n_nodes();
   const char* env = std::getenv("PCMI355_DENSE_GROUPS");
   std::vector<int32_t> g_node, g_edge, g_prime;
-  struct Found { int layer; std::vector<int32_t> nodes; };
+  typedef std::pair<int32_t, int32_t> Child;   // (prime, sub)
+  struct Found { int layer; std::vector<int32_t> nodes; int children; std::vector<Child> set; };   // set: of a masked group
   std::vector<Found> found;
   // a sum's edges ordered by (prime, sub): the order of a group's children
   auto sorted_edges = [&](int32_t n) {
@@ -1250,16 +1259,59 @@ void SparseCircuit::build_groups(std::vector<int32_t>& group_of, std::vector<int
         for (size_t m0 = 0; m0 < members.size(); m0 += kGroupMaxSide) {
           const size_t g = std::min<size_t>(kGroupMaxSide, members.size() - m0);
           if ((int)g < kGroupMinSide || (int64_t)g * c < kGroupMinEdges) continue;
-          found.push_back(Found{fc_.layer[cand[i]], std::vector<int32_t>(members.begin() + m0, members.begin() + m0 + g)});
+          found.push_back(Found{fc_.layer[cand[i]], std::vector<int32_t>(members.begin() + m0, members.begin() + m0 + g), c, {}});
         }
+      }
+    }
+    std::vector<char> taken(nn, 0);
+    for (const Found& f : found)
+      for (int32_t n : f.nodes) taken[n] = 1;
+    // the sums that are left: sets of them that shared children connect
+    std::vector<int32_t> root_of(nn, -1);
+    auto root = [&](int32_t n) {
+      while (root_of[n] != n) n = root_of[n] = root_of[root_of[n]];
+      return n;
+    };
+    std::map<int32_t, std::vector<int32_t>> by_layer, connected;
+    for (int64_t n = 0; n < nn; ++n)
+      if (fc_.type[n] == kSum && !taken[n] && fc_.node_e1[n] - fc_.node_e0[n] <= kGroupMaxSide) by_layer[fc_.layer[n]].push_back((int32_t)n);
+    for (const auto& kv : by_layer) {
+      std::unordered_map<uint64_t, int32_t> last_with;   // child -> the last sum seen that has it
+      for (int32_t n : kv.second) root_of[n] = n;
+      for (int32_t n : kv.second) {
+        for (int32_t e = fc_.node_e0[n]; e < fc_.node_e1[n]; ++e) {
+          const auto at = last_with.emplace((uint64_t)(uint32_t)fc_.e_prime[e] << 32 | (uint32_t)fc_.e_sub[e], n);
+          if (at.second) continue;
+          if (at.first->second == n) taken[n] = 1;   // the same child twice: two parameters for one entry of W
+          const int32_t a = root(at.first->second), b = root(n);
+          root_of[std::max(a, b)] = std::min(a, b);
+          at.first->second = n;
+        }
+      }
+      for (int32_t n : kv.second)
+        if (!taken[n]) connected[root(n)].push_back(n);
+    }
+    for (const auto& kv : connected) {
+      for (size_t m0 = 0; m0 < kv.second.size(); m0 += kGroupMaxSide) {
+        const size_t g = std::min<size_t>(kGroupMaxSide, kv.second.size() - m0);
+        Found f{fc_.layer[kv.first], std::vector<int32_t>(kv.second.begin() + m0, kv.second.begin() + m0 + g), 0, {}};
+        int64_t edges = 0;
+        for (int32_t n : f.nodes)
+          for (int32_t e = fc_.node_e0[n]; e < fc_.node_e1[n]; ++e, ++edges) f.set.emplace_back(fc_.e_prime[e], fc_.e_sub[e]);
+        std::sort(f.set.begin(), f.set.end());
+        f.set.erase(std::unique(f.set.begin(), f.set.end()), f.set.end());
+        f.children = (int)f.set.size();
+        if ((int)g < kGroupMinSide || f.children < kGroupMinSide || f.children > kGroupMaxSide ||
+            (int64_t)g * f.children < kGroupMinEdges || edges * kMaskedShare < (int64_t)g * f.children)
+          continue;
+        found.push_back(f);
       }
     }
   }
   auto tiles = [](int x) { int t = 1; while (t * 16 < x) t *= 2; return t; };   // 16-row tiles, a power of two of them
   std::sort(found.begin(), found.end(), [&](const Found& a, const Found& b) {
-    const int ca = fc_.node_e1[a.nodes[0]] - fc_.node_e0[a.nodes[0]], cb = fc_.node_e1[b.nodes[0]] - fc_.node_e0[b.nodes[0]];
-    const auto ka = std::make_tuple(a.layer, tiles((int)a.nodes.size()), tiles(ca), a.nodes[0]);
-    const auto kb = std::make_tuple(b.layer, tiles((int)b.nodes.size()), tiles(cb), b.nodes[0]);
+    const auto ka = std::make_tuple(a.layer, tiles((int)a.nodes.size()), tiles(a.children), a.nodes[0]);
+    const auto kb = std::make_tuple(b.layer, tiles((int)b.nodes.size()), tiles(b.children), b.nodes[0]);
     return ka < kb;
   });
   for (size_t gi = 0; gi < found.size(); ++gi)
@@ -1293,8 +1345,8 @@ void SparseCircuit::build_groups(std::vector<int32_t>& group_of, std::vector<int
   int32_t n_slots = 0;
   for (size_t gi = 0; gi < found.size(); ++gi) {
     const Found& f = found[gi];
-    const std::vector<int32_t> first = sorted_edges(f.nodes[0]);
-    const int32_t c = (int32_t)first.size(), gn = (int32_t)f.nodes.size();
+    const int32_t c = f.children, gn = (int32_t)f.nodes.size();
+    std::vector<int32_t> first(c, -1);   // per child: the edge of the first sum that has it
     const int gt = tiles(gn), ct = tiles(c);
     shape_gt.push_back(gt);
     shape_ct.push_back(ct);
@@ -1305,9 +1357,14 @@ void SparseCircuit::build_groups(std::vector<int32_t>& group_of, std::vector<int
     elem.insert(elem.end(), (size_t)gt * 16 * ct * 16, (int32_t)gi);
     for (int i = 0; i < gt * 16; ++i) {
       g_node.push_back(i < gn ? f.nodes[i] : -1);
-      std::vector<int32_t> es;
+      std::vector<int32_t> es, row(ct * 16, -1);
       if (i < gn) es = sorted_edges(f.nodes[i]);
-      for (int k = 0; k < ct * 16; ++k) g_edge.push_back(i < gn && k < c ? es[k] : -1);
+      for (size_t k = 0; k < es.size(); ++k) {
+        const size_t at = f.set.empty() ? k : (size_t)(std::lower_bound(f.set.begin(), f.set.end(), Child(fc_.e_prime[es[k]], fc_.e_sub[es[k]])) - f.set.begin());
+        row[at] = es[k];
+        if (first[at] < 0) first[at] = es[k];
+      }
+      g_edge.insert(g_edge.end(), row.begin(), row.end());
     }
     for (int i = 0; i < ct * 16; ++i) {
       if (i >= c) { g_rows.push_back(int4{zrow, zrow, zrow, zrow}); g_own.push_back(-2); continue; }
@@ -1539,7 +1596,7 @@ SparseCircuit::SparseCircuit(FlatCircuit fc) : fc_(std::move(fc)) {
     const int32_t p = fc_.e_parent[e], pr = fc_.e_prime[e], sb = fc_.e_sub[e];
     if (group_of[p] >= 0) {
       const int32_t slot = edge_slot[e];
-      if (slot < 0) continue;   // (one record per child: from the edges of the group's first sum)
+      if (slot < 0) continue;   // (one record per child: from the group's first sum that has it)
       const int4 rec{(slot << 1) | 1, ~(int32_t)(nn + slot), zrow, zrow};
       in_list[pr].push_back(Entry{rec, -1 - slot, 0});
       if (sb >= 0) in_list[sb].push_back(Entry{rec, -1 - slot, 1});

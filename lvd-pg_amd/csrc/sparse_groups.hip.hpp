@@ -96,7 +96,8 @@ __global__ __launch_bounds__(256) void sparse_group_w_kernel(GroupDev d, const i
   const int64_t local = i - r.pw0;
   const int g = (int)(local / (16 * r.ct)), c = (int)(local % (16 * r.ct));
   const int e = d.edge[i];
-  const float w = e >= 0 ? __expf(d.logp[e] * d.inv_f) : 0.f;
+  float w = e >= 0 ? __expf(d.logp[e] * d.inv_f) : 0.f;
+  if (w < __FLT_MIN__) w = 0.f;   // (no denormal operands: see kLowSum)
   const_cast<float*>(d.wf)[r.pw0 + group_wf_index(g, c, r.ct)] = w;
   const_cast<float*>(d.wb)[r.pw0 + group_wb_index(g, c, r.gt)] = w;
 }
@@ -120,6 +121,49 @@ __device__ __forceinline__ float group_max4(float v) {
   const int b = __builtin_bit_cast(int, v);
   const auto r32 = __builtin_amdgcn_permlane32_swap(b, b, false, false);
   return fmaxf(__builtin_bit_cast(float, (int)r32[0]), __builtin_bit_cast(float, (int)r32[1]));
+}
+
+// Sums far below their group's maximum.  E = exp(X - m) leaves float's range 87 below m, and a sum without a share in
+// the children near m -- masked groups (build_groups) have many -- may own nothing above that.  A sum that comes out
+// below kLowSum is added up again with E = exp(X - m + off) for an offset raised step by step (per example, so the
+// matrix instruction's columns stay independent): 60 further, which brings out every child E still held, then to the
+// next child below.  Every second step takes in a child more, so the loop ends.  Going down, the sums with
+// m - value > kHighShare take the same road: their R is formed for value + off and met by E raised by off.  E is kept
+// under exp(kMaxRaise): a child above that has no share in the sum that asked (its W would be a denormal).
+constexpr float kLowSum = 1e-30f, kHighShare = 60.f, kMaxRaise = 88.f;
+
+template <int NK>
+__device__ __forceinline__ void group_low_sums(const float* xm, int64_t Bp, int hi, const float* w, float mx, bool (&low)[4], float (&val)[4]) {
+  float xs[NK], a[NK];
+#pragma unroll
+  for (int q = 0; q < NK; ++q) {
+    xs[q] = xm[(int64_t)(4 * q + hi) * Bp];   // (what this lane has just written)
+    a[q] = w[q * 64];
+  }
+  float off = 0.f;
+  for (int it = 0; it < 8 * NK + 2; ++it) {
+    if (!(it & 1)) {
+      off += kHighShare;
+    } else {
+      float next = -INFINITY;
+#pragma unroll
+      for (int q = 0; q < NK; ++q) if (xs[q] < -off - 40.f) next = fmaxf(next, xs[q]);
+      next = group_max4(next);
+      if (next > -INFINITY) off = -next;
+      else low[0] = low[1] = low[2] = low[3] = false;   // nothing further down: what S was, it is
+    }
+    if (!__any(low[0] | low[1] | low[2] | low[3])) break;
+    g4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < NK; ++q)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], xs[q] > -INFINITY ? __expf(fminf(xs[q] + off, kMaxRaise)) : 0.f, acc, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (low[i] && acc[i] >= kLowSum) {
+        val[i] = mx - off + __logf(acc[i]);
+        low[i] = false;
+      }
+  }
 }
 
 // Forward: values of the group's sums.  One wave per (group, 16 examples), nothing shared: lane 16 * hi + lo takes
@@ -186,15 +230,57 @@ __device__ __forceinline__ void group_forward_body(const GroupDev& d, const Grou
       acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, x[q], acc, 0, 0, 0);
     }
     const int nd[4] = {nd4[gt].x, nd4[gt].y, nd4[gt].z, nd4[gt].w};
+    float val[4];
+    bool low[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      val[i] = mx + __logf(acc[i]);
+      low[i] = nd[i] >= 0 && acc[i] < kLowSum;
+    }
+    if (__any(low[0] | low[1] | low[2] | low[3])) group_low_sums<NK>(xm, d.Bp, hi, wg + gt * NK * 64, mx, low, val);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (nd[i] >= 0) d.mars[(int64_t)nd[i] * d.Bp + col] = mx + __logf(acc[i]);
+      if (nd[i] >= 0) d.mars[(int64_t)nd[i] * d.Bp + col] = val[i];
   }
 }
 
 template <int GT, int CT>
 __global__ __launch_bounds__(64) void sparse_group_forward_kernel(GroupDev d, GroupBase base) {
   group_forward_body<GT, CT>(d, base, blockIdx.x, threadIdx.x, blockIdx.y);
+}
+
+// The part of the children's rows that comes from sums with m - value > kHighShare (see kLowSum): out[i] for the four
+// children whose X - m are e[i]; w: the children's tile of W in the backward order.
+template <int NG>
+__device__ __forceinline__ void group_high_shares(const GroupDev& d, const int32_t* node, int hi, int64_t col, float mb, const float* w,
+                                                  const float (&e)[4], float (&out)[4]) {
+  float f[NG], t[NG];
+#pragma unroll
+  for (int k = 0; k < NG; ++k) {
+    const int32_t nd = node[4 * k + hi];
+    const int64_t n = nd < 0 ? 0 : nd;
+    const float fl = d.flows[n * d.Bp + col], v = d.mars[n * d.Bp + col];
+    const float nv = d.norm_row < 0 ? d.norm[n * d.Bp + col] : 0.f;
+    f[k] = fl;
+    t[k] = nd >= 0 && fl > 0.f && v > -INFINITY ? (mb - v) * d.inv_f - nv : 0.f;
+  }
+  for (int it = 0; it < 4 * NG; ++it) {
+    float off = INFINITY;   // the nearest of the example's sums that are left
+#pragma unroll
+    for (int k = 0; k < NG; ++k) if (t[k] > kHighShare) off = fminf(off, t[k]);
+    off = -group_max4(-off);
+    if (!__any(off < INFINITY)) break;
+    g4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < NG; ++k) {
+      const bool now = t[k] > kHighShare && t[k] <= off + kHighShare && off < INFINITY;
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[k * 64], now ? f[k] * __expf(t[k] - off) : 0.f, acc, 0, 0, 0);
+      if (now) t[k] = 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (e[i] > -INFINITY && off < INFINITY) out[i] += __expf(fminf(e[i] * d.inv_f + off, kMaxRaise)) * acc[i];
+  }
 }
 
 // Backward, per layer: the rows the group hands its children, E[c] * sum_g W[g,c] R[g].  One wave per (group, 16
@@ -237,6 +323,7 @@ __device__ __forceinline__ void group_backward_body(const GroupDev& d, const Gro
     for (int ct = 0; ct < CT; ++ct) numbers(ct, ct);
   }
   float rv[NG];
+  bool high = false;
   {   // R = F / S = F * exp(m - value): no flow stays no flow where the value is -inf.  (All rows requested, then used:
       // written as one loop the compiler waits for every sum's rows in turn.)
     float f[NG], v[NG], nv[NG];
@@ -252,9 +339,14 @@ __device__ __forceinline__ void group_backward_body(const GroupDev& d, const Gro
       for (int k = 0; k < NG; ++k) nv[k] = d.norm[(nd[k] < 0 ? 0 : (int64_t)nd[k]) * d.Bp + col];
     }
 #pragma unroll
-    for (int k = 0; k < NG; ++k)
-      rv[k] = (nd[k] >= 0 && f[k] > 0.f && v[k] > -INFINITY) ? f[k] * __expf((mb - v[k]) * d.inv_f - nv[k]) : 0.f;
+    for (int k = 0; k < NG; ++k) {
+      const float t = (mb - v[k]) * d.inv_f - nv[k];
+      const bool some = nd[k] >= 0 && f[k] > 0.f && v[k] > -INFINITY;
+      high |= some && t > kHighShare;
+      rv[k] = some && !(t > kHighShare) ? f[k] * __expf(t) : 0.f;
+    }
   }
+  high = __any(high);
   if constexpr (kPre) {
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) values(ct, ct);
@@ -266,9 +358,13 @@ __device__ __forceinline__ void group_backward_body(const GroupDev& d, const Gro
     g4f acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < NG; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][k], rv[k], acc, 0, 0, 0);
+    float out[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[i] = (e[s][i] > -INFINITY ? __expf(e[s][i] * d.inv_f) : 0.f) * acc[i];
+    if (high) group_high_shares<NG>(d, node, hi, col, mb, wg + ct * NG * 64, e[s], out);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float f = (e[s][i] > -INFINITY ? __expf(e[s][i] * d.inv_f) : 0.f) * acc[i];
+      const float f = out[i];
       const int4 p = cpa[s][i], q = cpb[s][i];
       if (p.x >= 0) d.flows[(int64_t)p.x * d.Bp + col] = f;
       if (p.y >= 0) d.flows[(int64_t)p.y * d.Bp + col] = f;
@@ -320,6 +416,8 @@ __global__ __launch_bounds__(WV * 64) void sparse_group_walk_kernel(GroupDev d, 
 template <int GT, int CT>
 __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int first) {
   extern __shared__ float glds[];
+  __shared__ int next_pass[2];
+  constexpr int kLastPass = 1 << 20;
   const int group = d.order[first + blockIdx.x];
   const GroupRec r = d.rec[group];
   constexpr int Gp = GT * 16, Cp = CT * 16;
@@ -329,57 +427,75 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
   const int t = threadIdx.x;
   const int b = t & 63, part = guni(t >> 6);
   const float mb = d.m[(int64_t)group * d.Bp + b0 + b];
-  for (int cb = part; cb < Cp; cb += 32) {
-    float x[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int c = cb + 4 * q;
-      x[q] = c < Cp ? d.xm[(int64_t)(r.pslot0 + c) * d.Bp + b0 + b] : -INFINITY;
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int c = cb + 4 * q;
-      if (c < Cp) E[c * kGroupPad + b] = x[q] > -INFINITY ? __expf(x[q] * d.inv_f) : 0.f;
-    }
-  }
-  for (int gb = part; gb < Gp; gb += 32) {   // (eight sums' rows requested before the first is used, as above)
-    float f[8], v[8], nv[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int g = gb + 4 * q;
-      f[q] = 0.f;
-      v[q] = 0.f;
-      nv[q] = 0.f;
-      if (g < r.G) {
-        const int64_t n = guni(d.node[r.pnode0 + g]);
-        f[q] = d.flows[n * d.Bp + b0 + b];
-        v[q] = d.mars[n * d.Bp + b0 + b];
-        nv[q] = d.norm[(d.norm_row >= 0 ? d.norm_row : n) * d.Bp + b0 + b];
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int g = gb + 4 * q;
-      if (g < Gp) R[g * kGroupPad + b] = (f[q] > 0.f && v[q] > -INFINITY) ? f[q] * __expf((mb - v[q]) * d.inv_f - nv[q]) : 0.f;
-    }
-  }
-  __syncthreads();
   const int lane = t & 63, wave = t >> 6;
   const int lo = lane & 15, hi = lane >> 4;
   float* part_row = d.edge_part + (size_t)blockIdx.y * d.n_edges;
-  for (int tile = wave; tile < GT * CT; tile += 4) {
-    const int gt = tile / CT, ct = tile % CT;
-    g4f acc = {0.f, 0.f, 0.f, 0.f};
+  // a pass takes the (sum, example) pairs with m - value in one interval of kHighShare (see kLowSum): the first one
+  // everything below kHighShare, which is nearly always all there is, the next ones the nearest that is left
+  for (int pass = 0, turn = 0; pass <= kLastPass; turn ^= 1) {
+    const float off = kHighShare * (float)pass;
+    for (int cb = part; cb < Cp; cb += 32) {
+      float x[8];
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk)
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(R[(gt * 16 + lo) * kGroupPad + kk * 4 + hi], E[(ct * 16 + lo) * kGroupPad + kk * 4 + hi],
-                                                 acc, 0, 0, 0);
-    const int c = ct * 16 + lo;
+      for (int q = 0; q < 8; ++q) {
+        const int c = cb + 4 * q;
+        x[q] = c < Cp ? d.xm[(int64_t)(r.pslot0 + c) * d.Bp + b0 + b] : -INFINITY;
+      }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int g = gt * 16 + 4 * hi + i;
-      if (g < r.G && c < r.C) part_row[d.edge[r.pw0 + g * Cp + c]] = d.wf[r.pw0 + group_wf_index(g, c, CT)] * acc[i];
+      for (int q = 0; q < 8; ++q) {
+        const int c = cb + 4 * q;
+        if (c < Cp) E[c * kGroupPad + b] = x[q] > -INFINITY ? __expf(fminf(x[q] * d.inv_f + off, kMaxRaise)) : 0.f;
+      }
     }
+    int left = kLastPass + 1;
+    for (int gb = part; gb < Gp; gb += 32) {   // (eight sums' rows requested before the first is used, as above)
+      float f[8], v[8], nv[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int g = gb + 4 * q;
+        f[q] = 0.f;
+        v[q] = 0.f;
+        nv[q] = 0.f;
+        if (g < r.G) {
+          const int64_t n = guni(d.node[r.pnode0 + g]);
+          f[q] = d.flows[n * d.Bp + b0 + b];
+          v[q] = d.mars[n * d.Bp + b0 + b];
+          nv[q] = d.norm[(d.norm_row >= 0 ? d.norm_row : n) * d.Bp + b0 + b];
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int g = gb + 4 * q;
+        const bool some = f[q] > 0.f && v[q] > -INFINITY;
+        const float tq = (mb - v[q]) * d.inv_f - nv[q];
+        const int mine = tq > kHighShare ? (int)fminf(tq * (1.f / kHighShare), (float)kLastPass) : 0;
+        if (some && mine > pass) left = min(left, mine);
+        if (g < Gp) R[g * kGroupPad + b] = some && mine == pass ? f[q] * __expf(tq - off) : 0.f;
+      }
+    }
+    if (t == 0) next_pass[turn] = kLastPass + 1;
+    __syncthreads();
+    if (left <= kLastPass) atomicMin(&next_pass[turn], left);
+    for (int tile = wave; tile < GT * CT; tile += 4) {
+      const int gt = tile / CT, ct = tile % CT;
+      g4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < 16; ++kk)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(R[(gt * 16 + lo) * kGroupPad + kk * 4 + hi], E[(ct * 16 + lo) * kGroupPad + kk * 4 + hi],
+                                                   acc, 0, 0, 0);
+      const int c = ct * 16 + lo;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int g = gt * 16 + 4 * hi + i;
+        const int edge = g < r.G && c < r.C ? d.edge[r.pw0 + g * Cp + c] : -1;
+        if (edge < 0) continue;   // (in a masked group also a child the sum does not have)
+        const float w = d.wf[r.pw0 + group_wf_index(g, c, CT)];
+        const float flow = w > 0.f ? w * acc[i] : 0.f;
+        part_row[edge] = pass == 0 ? flow : part_row[edge] + flow;
+      }
+    }
+    __syncthreads();
+    pass = next_pass[turn];
   }
 }
 

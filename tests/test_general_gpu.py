@@ -765,6 +765,60 @@ def test_dense_groups_beside_ordinary_edges(gpu, oracle):
     assert grouped.size("dense_groups") == 2
 
 
+def _masked_multihead(O, rng, levels, G, J, H, keep, sharp, C):
+    """Heads over a chain of `levels` sets of G sums whose children are random parts of the J products below (two at
+    least); leaves whose log-probabilities lie `sharp` apart."""
+    from helpers import log_dirichlet
+
+    def leaf(v):
+        x = rng.normal(size=C) * sharp
+        x -= x.max()
+        return O.input_node(v, (x - np.log(np.exp(x).sum())).astype(np.float32))
+
+    subs = [O.multiply(leaf(0), leaf(1)) for _ in range(J)]
+    for l in range(levels):
+        sums = []
+        for _ in range(G):
+            kept = rng.random(J) < keep
+            kept[rng.choice(J, 2, replace=False)] = True
+            sums.append(O.summate(*[subs[j] for j in np.flatnonzero(kept)], logps=log_dirichlet(rng, int(kept.sum()))))
+        subs = [O.multiply(sums[j % G], leaf(2 + l)) for j in range(J)]
+    return [O.summate(*subs, logps=log_dirichlet(rng, J)) for _ in range(H)]
+
+
+@pytest.mark.parametrize("levels,G,J,H,keep,sharp,B,groups", [(3, 16, 16, 5, 0.6, 1.0, 100, 4), (2, 17, 33, 4, 0.5, 1.0, 65, 3),
+                                                              (2, 32, 32, 5, 0.5, 60.0, 130, 3), (2, 12, 20, 4, 0.4, 120.0, 90, 3),
+                                                              (2, 33, 65, 4, 0.4, 90.0, 64, 3), (1, 65, 128, 4, 0.3, 90.0, 40, 2),
+                                                              (2, 100, 100, 4, 0.0, 1.0, 50, 1), (2, 8, 12, 4, 0.3, 1.0, 33, 2)])
+def test_masked_groups(gpu, oracle, levels, G, J, H, keep, sharp, B, groups):
+    """Sums over different parts of one set of products run as one block with zeros (edges of tiles, sets too thin for
+    it); with sharp leaves a sum's own children lie hundreds below the block's maximum, where exp(X - m) is zero."""
+    rng = np.random.default_rng(71)
+    C = 5
+    heads = _masked_multihead(oracle, rng, levels, G, J, H, keep, sharp, C)
+    grouped, _ = _check_grouped_multihead(gpu, oracle, heads, 2 + levels, C, B, 72, min_groups=1)
+    assert grouped.size("dense_groups") == groups
+
+
+@pytest.mark.parametrize("fscale", [0.5, 2.5])
+def test_tempered_flows_of_masked_groups(gpu, oracle, fscale):
+    """Tempered flows of masked groups against the layer kernels', sharp leaves included."""
+    torch, P = gpu
+    rng = np.random.default_rng(73)
+    C, B, H = 5, 100, 4
+    for sharp in (1.0, 60.0):
+        heads = _masked_multihead(oracle, rng, 2, 20, 24, H, 0.5, sharp, C)
+        d = torch.from_numpy(rng.integers(0, C, size=(B, 4)).astype(np.uint8)).cuda()
+        hm = torch.from_numpy(rng.random((B, H)).astype(np.float32) + 0.05).cuda()
+        got = []
+        for c in _with_and_without_groups(P, heads, 4, C):
+            c.set_flow_scale(fscale)
+            P.probs_flows_circuit(c, d, head_mask=hm)
+            got.append((c.get_node_values(B)[1], *c.get_aggregates()))
+        for a, b in zip(*got):
+            assert np.abs(a - b).max() < FLOW_RTOL * max(np.abs(b).max(), 1.0)
+
+
 @pytest.mark.parametrize("fscale", [0.5, 2.5])
 def test_tempered_flows_match_the_oracle(gpu, oracle, fscale):
     """`fscale` of mini_batch_em_beta (src-jl/learning/flow.jl:120-373, `pcm_set_flow_scale`): node flows, edge and leaf
