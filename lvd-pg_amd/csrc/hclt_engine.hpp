@@ -323,8 +323,8 @@ class HcltCircuit : public pcm_circuit {
   DevBuf<int32_t> d_soft_tabs_;     // relaxed sampler: parents | leaf-feeding nodes | nodes by depth | level offsets
   DevBuf<float> d_soft_w_;          // ... exp(theta / T) in the two operand layouts
   int soft_levels_ = 0;
-  DevBuf<int32_t> d_sample_tabs_;   // sampler tables: parent of every inner node | state-giving node of every variable | level order
-  DevBuf<int32_t> d_sample_passes_;   // the sampler's levels from the root in records of 64 {node, parent} pairs
+  DevBuf<int32_t> d_sample_tabs_;   // sampler: place of the state-giving node of every variable
+  DevBuf<int32_t> d_sample_passes_;   // the sampler's levels from the root in records of kStateNodes(K) {node, parent's place, place, 0 or -1}
   int sample_passes_ = 0;
   DevBuf<int64_t> d_sum_param_src_;
   DevBuf<int32_t> d_in_pos_;   // input node (v, j) -> its position among the input nodes of the parameter vector

@@ -30,110 +30,91 @@ __device__ __forceinline__ float4 noise_word(const float* p) {
 // nodes) or of its parent (leaf tree nodes).  Same additions and comparisons, in the same
 // order, as the layered engine's sampler on the circuit's general form.
 
-// States of the inner tree nodes, a lane per tree node: a wave takes one example and walks the
-// levels from the root, 64 nodes of a level at a time (`passes` records of 64 {node, parent}
-// pairs, -1: no node).  A lane reads its node's K noise values and the parameter row its
-// parent's state selects (two contiguous rows of 4K bytes) and scans them in order: first
-// maximum wins, no exchange between lanes.  The noise does not depend on any state, so its
-// requests leave a pass ahead (up to K = 32, where a row fits the registers twice), or at
-// least before the parent's state is read.  The chosen states live in LDS (one byte
-// per node) and leave through a coalesced copy at the end; no barriers, a wave only reads its
-// own example's bytes.
+// States of the inner tree nodes.  A wave takes one example and walks the levels from the root; K / 4 lanes share a tree
+// node, so that its K noise values and the parameter row its parent's state selects are read by whole cache lines, and
+// kStateUnroll nodes per lane are under way together.  (A lane per node, as this kernel was before, has every lane read
+// rows of its own in 16-byte pieces: eight times the cache accesses for K = 32, which is what bounded it: 480 -> 356 us for 4096
+// samples of 2458 nodes, 1.06 GB of noise; what is left is the chain of a level, LDS byte -> parameter row -> byte.)
+// `passes` records of kStateNodes(K) {parameter block, place of the parent, place, 0 (-1: no node, the entry names node 0)}
+// entries; a node's place is the caller's number for it: its noise column and its byte of state.  The auxiliary nodes that
+// split a node of many children pass their parent's state on, so they are left out and the nodes below them hang from the
+// nearest node of the caller's: no pass for them, and the noise is read where it lies (4096 samples of a 3072-variable
+// circuit: the copy with columns for them, 1.1 GB in and 1.3 GB out, took 0.42 of 3.0 ms).
+// The noise does not depend on any state, so its requests leave a pass ahead.  First maximum wins: the lanes scan their
+// four values in order, and between lanes the larger value, then the lower state is kept; the first lane starts from
+// state 0 whatever its value, the others from nothing, so its result is that of one scan over the row.  The chosen states
+// live in LDS (one byte per node) and leave through a coalesced copy at the end; no barriers, a wave only reads its own
+// example's bytes.
+constexpr int kStateUnroll = 4;
+constexpr int kStateNodes(int K) { return 256 / K * kStateUnroll; }
+
+template <int kCtrl>
+__device__ __forceinline__ void state_take_dpp(float& bv, int& bi) {
+  const float ov = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, bv), kCtrl, 0xf, 0xf, true));
+  const int oi = __builtin_amdgcn_mov_dpp(bi, kCtrl, 0xf, 0xf, true);
+  if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+}
+
 template <int K>
 __global__ __launch_bounds__(256) void hclt_sample_states_node_kernel(const float* __restrict__ logtheta,
-                                                                      const int2* __restrict__ passes_tab, int passes,
+                                                                      const int4* __restrict__ passes_tab, int passes,
                                                                       const float* __restrict__ node_noise,
-                                                                      int n_inner, int stride, int batch,
+                                                                      int n_places, int stride, int batch,
                                                                       uint8_t* __restrict__ states) {
-  static_assert(K % 4 == 0, "rows are read as 16-byte words");
-  constexpr int CH = K < 32 ? K : 32;   // values scanned per round: 8 words of noise and 8 of parameters in registers
+  static_assert(K >= 4 && K <= 128 && (K & (K - 1)) == 0, "rows are read as 16-byte words by 1 to 32 lanes");
+  constexpr int U = kStateUnroll, LPN = K / 4, NPI = 64 / LPN;
   extern __shared__ uint8_t st[];   // [4 waves][stride]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int b = blockIdx.x * 4 + wave;
   if (b >= batch) return;
+  const int sub = lane % LPN, slot = lane / LPN;
   uint8_t* mine = st + (size_t)wave * stride;
-  const float* g = node_noise + (size_t)b * n_inner * K;
-  if constexpr (K <= 32) {
-    // the noise of a pass is requested one pass ahead (the table ends with two empty records)
-    int2 rec0 = passes_tab[lane], rec1 = passes_tab[64 + lane];
-    float4 z[K / 4];
+  const float* g = node_noise + (size_t)b * n_places * K + 4 * sub;
+  const float* th = logtheta + 4 * sub;
+  // (the table ends with two empty records; every entry names rows that exist, so no request needs a branch)
+  int4 rec0[U], rec1[U], rec2[U];
+  float4 z[U], zn[U], a[U];
 #pragma unroll
-    for (int i = 0; i < K / 4; ++i) z[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (rec0.x >= 0) {
-#pragma unroll
-      for (int i = 0; i < K / 4; ++i) z[i] = reinterpret_cast<const float4*>(g + (size_t)rec0.x * K)[i];
-    }
-    for (int ps = 0; ps < passes; ++ps) {
-      const int n = rec0.x, par = rec0.y;
-      const int2 rec2 = passes_tab[(size_t)(ps + 2) * 64 + lane];
-      const int k = (n >= 0 && par >= 0) ? mine[par] : 0;
-      float4 a[K / 4], zn[K / 4];
-      if (n >= 0) {
-        const float4* row = reinterpret_cast<const float4*>(logtheta + ((size_t)n * K + k) * K);
-#pragma unroll
-        for (int i = 0; i < K / 4; ++i) a[i] = row[i];
-      }
-#pragma unroll
-      for (int i = 0; i < K / 4; ++i) zn[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (rec1.x >= 0) {
-#pragma unroll
-        for (int i = 0; i < K / 4; ++i) zn[i] = reinterpret_cast<const float4*>(g + (size_t)rec1.x * K)[i];
-      }
-      if (n >= 0) {
-        float best = 0.f;
-        int idx = 0;
-#pragma unroll
-        for (int i = 0; i < K / 4; ++i) {
-          const float x[4] = {a[i].x + z[i].x, a[i].y + z[i].y, a[i].z + z[i].z, a[i].w + z[i].w};
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int j = 4 * i + e;
-            if (j == 0 || x[e] > best) { best = x[e]; idx = j; }
-          }
-        }
-        mine[n] = (uint8_t)idx;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-      for (int i = 0; i < K / 4; ++i) z[i] = zn[i];
-      rec0 = rec1;
-      rec1 = rec2;
-    }
-  } else {
-    // K = 64, 128: a row is scanned in rounds of 32 values, its noise requested with it
-  int2 rec = passes_tab[lane];
-    for (int ps = 0; ps < passes; ++ps) {
-      const int n = rec.x, par = rec.y;
-      if (ps + 1 < passes) rec = passes_tab[(size_t)(ps + 1) * 64 + lane];
-      if (n >= 0) {
-        const float4* gz = reinterpret_cast<const float4*>(g + (size_t)n * K);
-        float best = 0.f;
-        int idx = 0;
-  #pragma unroll
-        for (int j0 = 0; j0 < K; j0 += CH) {
-          float4 z[CH / 4], a[CH / 4];
-  #pragma unroll
-          for (int i = 0; i < CH / 4; ++i) z[i] = gz[j0 / 4 + i];   // default policy: a lane's row is one cache line read in pieces
-          const int k = par < 0 ? 0 : mine[par];
-          const float4* row = reinterpret_cast<const float4*>(logtheta + ((size_t)n * K + k) * K);
-  #pragma unroll
-          for (int i = 0; i < CH / 4; ++i) a[i] = row[j0 / 4 + i];
-  #pragma unroll
-          for (int i = 0; i < CH / 4; ++i) {
-            const float x[4] = {a[i].x + z[i].x, a[i].y + z[i].y, a[i].z + z[i].z, a[i].w + z[i].w};
-  #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int j = j0 + 4 * i + e;
-              if (j == 0 || x[e] > best) { best = x[e]; idx = j; }
-            }
-          }
-        }
-        mine[n] = (uint8_t)idx;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the next level's lanes read these bytes
-    }
+  for (int u = 0; u < U; ++u) {
+    rec0[u] = passes_tab[u * NPI + slot];
+    rec1[u] = passes_tab[(U + u) * NPI + slot];
   }
-  for (int i = lane; i < n_inner; i += 64) states[(size_t)b * n_inner + i] = mine[i];
+#pragma unroll
+  for (int u = 0; u < U; ++u) z[u] = noise_word(g + (size_t)rec0[u].z * K);
+  for (int ps = 0; ps < passes; ++ps) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = rec0[u].y >= 0 ? mine[rec0[u].y] : 0;
+      a[u] = *reinterpret_cast<const float4*>(th + ((size_t)rec0[u].x * K + k) * K);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) rec2[u] = passes_tab[((size_t)(ps + 2) * U + u) * NPI + slot];
+#pragma unroll
+    for (int u = 0; u < U; ++u) zn[u] = noise_word(g + (size_t)rec1[u].z * K);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float x[4] = {a[u].x + z[u].x, a[u].y + z[u].y, a[u].z + z[u].z, a[u].w + z[u].w};
+      float best = sub == 0 ? x[0] : -INFINITY;
+      int idx = sub == 0 ? 0 : 0x7fffffff;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (x[e] > best) { best = x[e]; idx = 4 * sub + e; }
+      if constexpr (LPN >= 2) state_take_dpp<0xB1>(best, idx);    // quad_perm [1, 0, 3, 2]
+      if constexpr (LPN >= 4) state_take_dpp<0x4E>(best, idx);    // quad_perm [2, 3, 0, 1]
+      if constexpr (LPN >= 8) state_take_dpp<0x141>(best, idx);   // mirror within 8 lanes
+      if constexpr (LPN >= 16) state_take_dpp<0x140>(best, idx);  // mirror within 16
+      if constexpr (LPN >= 32) {
+        const float ov = __shfl_xor(best, 16);
+        const int oi = __shfl_xor(idx, 16);
+        if (ov > best || (ov == best && oi < idx)) { best = ov; idx = oi; }
+      }
+      if (sub == 0 && rec0[u].w >= 0) mine[rec0[u].z] = (uint8_t)idx;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the next level's lanes read these bytes
+#pragma unroll
+    for (int u = 0; u < U; ++u) { z[u] = zn[u]; rec0[u] = rec1[u]; rec1[u] = rec2[u]; }
+  }
+  for (int i = lane; i < n_places; i += 64) states[(size_t)b * n_places + i] = mine[i];
 }
 
 // (value, category) of one lane against another's: the larger value, the lower category among equal values; a lane
@@ -363,7 +344,8 @@ void HcltCircuit::sample(const float* d_node_noise, const float* d_leaf_noise, i
   if ((reinterpret_cast<uintptr_t>(d_node_noise) | reinterpret_cast<uintptr_t>(d_leaf_noise)) & 15)
     fail(PCM_ERR_ARG, "noise pointers must be 16-byte aligned (rows are read as 16-byte words)");
   const bool rows_fit = K_ >= 4 && K_ <= 128 && (K_ & (K_ - 1)) == 0;   // rows of whole 16-byte words, states in a byte
-  const int stride = (n_inner_ + 15) & ~15;   // bytes of one example's states in LDS
+  const int places = n_user_inner_;
+  const int stride = (places + 15) & ~15;   // bytes of one example's states in LDS
   const size_t st_bytes = (size_t)4 * stride;
   if (!rows_fit || st_bytes > (size_t)64 * 1024) {   // other hidden sizes: the layered engine's sampler
     SparseCircuit* g = general();
@@ -373,38 +355,41 @@ void HcltCircuit::sample(const float* d_node_noise, const float* d_leaf_noise, i
     return;
   }
   if (d_sample_tabs_.n == 0) {
-    // per inner node: its parent | per variable: the node whose state picks its leaf row
-    std::vector<int32_t> t((size_t)n_inner_ + V_);
-    for (int n = 0; n < n_inner_; ++n) {
-      const int v = var_of_inner_[n];
-      t[n] = parent_[v] < 0 ? -1 : inner_of_var_[parent_[v]];
-    }
-    for (int v = 0; v < V_; ++v) t[(size_t)n_inner_ + v] = children_[v].empty() ? inner_of_var_[parent_[v]] : inner_of_var_[v];
-    // inner nodes level by level from the root in records of 64 {node, parent} pairs (-1: padding)
+    // per variable: the place of the node whose state picks its leaf row
+    auto place_of = [&](int32_t v) {   // (of the nearest node of the caller's, from v upwards)
+      while (user_index_[inner_of_var_[v]] < 0) v = parent_[v];
+      return user_index_[inner_of_var_[v]];
+    };
+    std::vector<int32_t> t((size_t)V_);
+    for (int v = 0; v < V_; ++v) t[v] = place_of(children_[v].empty() ? parent_[v] : v);
+    // the caller's inner nodes level by level from the root in records of kStateNodes(K) entries
     std::vector<std::vector<int32_t>> by_depth;
-    for (int n = 0; n < n_inner_; ++n) {
-      const size_t dep = (size_t)depth_[var_of_inner_[n]];
-      if (by_depth.size() <= dep) by_depth.resize(dep + 1);
-      by_depth[dep].push_back(n);
+    std::vector<int32_t> depth(n_inner_, 0);
+    for (int n = n_inner_ - 1; n >= 0; --n) {   // parents before children
+      const int v = var_of_inner_[n];
+      if (parent_[v] >= 0) depth[n] = depth[inner_of_var_[parent_[v]]] + (user_index_[n] >= 0);
+      if (user_index_[n] < 0) continue;
+      if ((int)by_depth.size() <= depth[n]) by_depth.resize(depth[n] + 1);
+      by_depth[depth[n]].push_back(n);
     }
     std::vector<int32_t> rec;
+    const size_t per_pass = 4 * (size_t)kStateNodes(K_);
     for (const auto& lvl : by_depth) {
       for (int32_t n : lvl) {
-        rec.push_back(n);
-        rec.push_back(t[n]);
+        const int32_t up = parent_[var_of_inner_[n]];
+        rec.insert(rec.end(), {n, up < 0 ? -1 : place_of(up), user_index_[n], 0});
       }
-      while (rec.size() % 128) rec.push_back(-1);
+      while (rec.size() % per_pass) rec.insert(rec.end(), {0, -1, 0, -1});
     }
-    sample_passes_ = (int)(rec.size() / 128);
-    rec.resize(rec.size() + 256, -1);   // two empty records: the walk requests records two passes ahead
+    sample_passes_ = (int)(rec.size() / per_pass);
+    for (size_t i = 0; i < 2 * per_pass / 4; ++i) rec.insert(rec.end(), {0, -1, 0, -1});   // two empty records: the walk requests records two passes ahead
     d_sample_passes_.upload(rec, stream);
     d_sample_tabs_.upload(t, stream);
   }
-  d_state_.ensure((size_t)batch * n_inner_);
+  d_state_.ensure((size_t)batch * places);
   auto node_states = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(ceil_div(batch, 4)), dim3(256), st_bytes, stream, d_logtheta_.p,
-                       reinterpret_cast<const int2*>(d_sample_passes_.p), sample_passes_, kernel_noise(d_node_noise, batch),
-                       n_inner_, stride, batch, d_state_.p);
+                       reinterpret_cast<const int4*>(d_sample_passes_.p), sample_passes_, d_node_noise, places, stride, batch, d_state_.p);
   };
   switch (K_) {
     case 4: node_states(&hclt_sample_states_node_kernel<4>); break;
@@ -422,7 +407,7 @@ void HcltCircuit::sample(const float* d_node_noise, const float* d_leaf_noise, i
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     // (leaves: the caller's variables, which come first; the auxiliary ones have nothing to draw)
     hipLaunchKernelGGL(hclt_sample_leaves_lds_kernel, dim3(Vu_, ceil_div(batch, kLeafExamples)), dim3(kLeafWaves * 64), lds,
-                       stream, d_leaf_.p, d_sample_tabs_.p + n_inner_, d_state_.p, d_leaf_noise, Vu_, K_, C_, n_inner_, batch,
+                       stream, d_leaf_.p, d_sample_tabs_.p, d_state_.p, d_leaf_noise, Vu_, K_, C_, places, batch,
                        d_out);
   } else {
     d_leaf_kc_.ensure((size_t)V_ * K_ * C_);
@@ -430,7 +415,7 @@ void HcltCircuit::sample(const float* d_node_noise, const float* d_leaf_noise, i
     hipLaunchKernelGGL(hclt_leaf_kc_kernel, dim3((unsigned)ceil_div(tot, 256)), dim3(256), 0, stream, d_leaf_.p, d_leaf_kc_.p,
                        V_, K_, C_);
     hipLaunchKernelGGL(hclt_sample_leaves_kernel, dim3(batch, ceil_div(Vu_, 4 * kVarsPerWave)), dim3(256), 0, stream, d_leaf_kc_.p,
-                       d_sample_tabs_.p + n_inner_, d_state_.p, d_leaf_noise, Vu_, K_, C_, n_inner_, batch, d_out);
+                       d_sample_tabs_.p, d_state_.p, d_leaf_noise, Vu_, K_, C_, places, batch, d_out);
   }
   check_launch_q("hclt_sample");
   sync_checked();

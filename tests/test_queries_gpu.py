@@ -191,6 +191,8 @@ def test_sampling_bit_exact_random_dag(gpu, oracle, V, C, width, B, seed):
     (7, 128, 8, 45, None), (5, 128, 128, 20, None),              # K = 128: block sampler; 6 KB and 68 KB of leaf table in LDS
     (5, 64, 256, 70, None), (3, 128, 252, 30, None),             # 67 KB and 131 KB
     (141, 8, 3, 33, [-1] + [0] * 70 + list(range(1, 71))),       # a level of more than 64 tree nodes
+    (37, 128, 3, 9, [-1] + [0] * 18 + list(range(1, 19))),       # levels of more nodes than a pass takes
+    (39, 64, 3, 9, [-1] + [0] * 19 + list(range(1, 20))), (85, 32, 3, 9, [-1] + [0] * 42 + list(range(1, 43))),
     (13, 16, 6, 50, [-1, 0, 1, 1, 1, 1, 2, 3, 0, 8, 8, 8, 8]),   # four children twice: split for the walks, the noise
     (11, 32, 5, 40, [-1, 0, 0, 0, 0, 0, 1, 2, 3, 4, 5])])        # stays indexed by the caller's tree nodes
 def test_sampling_bit_exact_hclt(gpu, oracle, V, K, C, B, tree):
@@ -209,6 +211,33 @@ def test_sampling_bit_exact_hclt(gpu, oracle, V, K, C, B, tree):
     for r, v in enumerate(inner):
         nk = len(fc.meta["sum_node"][v])
         e0 = fc.meta["edge_of"][v]
+        slot[e0:e0 + nk * K] = np.tile(r * K + np.arange(K), nk)
+    want = O.sample(fc, node_noise, leaf_noise, noise_slot=slot)
+    got = P.sample(bpc, torch.from_numpy(node_noise).cuda(), torch.from_numpy(leaf_noise).cuda()).cpu().numpy()
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("K", [4, 8, 16, 32, 64, 128])
+def test_sampling_takes_the_first_of_equal_states(gpu, oracle, K):
+    """Uniform parameters and noise of few values: nearly every maximum is shared; rows of -inf throughout give state 0."""
+    torch, P = gpu
+    O = oracle
+    from helpers import make_hclt, block_theta
+    V, C, B = 12, 4, 60
+    parent, theta, leaf, fc = make_hclt(V, K, C, 3)
+    rng = np.random.default_rng(K)
+    ch, root = O.clt_children(parent)
+    inner = [v for v in O.clt_bottom_up(parent) if ch[v]]
+    flat = {v: np.full_like(t, -np.log(np.float32(K))) for v, t in theta.items()}
+    fc = O.hclt_flat(parent, K, C, flat, leaf)
+    bpc = P.hclt_from_clt(parent, C, K)
+    bpc.set_params(block_theta(parent, K, flat), leaf)
+    node_noise = rng.integers(0, 2, (B, len(inner) * K)).astype(np.float32)
+    node_noise.reshape(B, len(inner), K)[rng.random((B, len(inner))) < 0.2] = -np.inf
+    leaf_noise = _gumbel(rng, (B, V, C))
+    slot = np.zeros(fc.n_edges, np.int64)
+    for r, v in enumerate(inner):
+        nk, e0 = len(fc.meta["sum_node"][v]), fc.meta["edge_of"][v]
         slot[e0:e0 + nk * K] = np.tile(r * K + np.arange(K), nk)
     want = O.sample(fc, node_noise, leaf_noise, noise_slot=slot)
     got = P.sample(bpc, torch.from_numpy(node_noise).cuda(), torch.from_numpy(leaf_noise).cuda()).cpu().numpy()
