@@ -1537,10 +1537,18 @@ HcltDev HcltCircuit::soft_stage(const SoftRef& s) {
   const int Cp = (C_ + 3) & ~3;
   const size_t lds = ((size_t)kEvExamples * (Cp + 4) + (size_t)Cp * (K_ + 16) + kEvExamples) * sizeof(float);
   PCM_DISPATCH_K(K_, {
-    PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&hclt_soft_leafval_kernel<KK>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(hclt_soft_leafval_kernel<KK>, dim3(ceil_div(V_, kEvVars), Bp64 / kEvExamples), dim3(4 * (KK / 16) * 64), lds,
-                       stream, s, d_leaf_.p, C_, V_, s.batch, Bp64, d_soft_lv_.p, d_soft_m_.p);
+    auto run = [&](auto kernel) {
+      PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      hipLaunchKernelGGL(kernel, dim3(ceil_div(V_, kEvVars), Bp64 / kEvExamples), dim3(4 * (KK / 16) * 64), lds, stream, s, d_leaf_.p,
+                         C_, V_, s.batch, Bp64, d_soft_lv_.p, d_soft_m_.p);
+    };
+    switch (soft_row_words(s, C_, KK)) {
+      case 0: run(&hclt_soft_leafval_kernel<KK, 0>); break;
+      case 2: run(&hclt_soft_leafval_kernel<KK, 2>); break;
+      case 4: run(&hclt_soft_leafval_kernel<KK, 4>); break;
+      case 8: run(&hclt_soft_leafval_kernel<KK, 8>); break;
+      default: run(&hclt_soft_leafval_kernel<KK, KK == 16 ? 16 : 8>); break;
+    }
   });
   check_launch("soft_leafval");
   d.leaf = d_soft_lv_.p;
@@ -1601,10 +1609,15 @@ void HcltCircuit::flows_soft(const SoftRef& s, float rate, const float* d_head_m
     const int split = ceil_div(chunks, std::min(chunks, want)) * kEvExamples;      // examples per split
     const int n_split = ceil_div(s.batch, split);
     if (n_split > 1) d_part_.ensure((size_t)n_split * n_leaf);
-    PCM_DISPATCH_K(K_, hipLaunchKernelGGL(hclt_soft_leafflow_kernel<KK>, dim3(ceil_div(C_, kEvCats), V_, n_split),
-                                          dim3(256), 0, stream, s, d_leaf_.p, d_soft_lv_.p, d_soft_m_.p, g_tiles,
-                                          d_soft_gnode_.p, C_, s.batch, Bp64, (size_t)d.tile_stride / 4, split,
-                                          d_leaf_flow_.p, n_split > 1 ? d_part_.p : (float*)nullptr));
+    PCM_DISPATCH_K(K_, {
+      auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(ceil_div(C_, kEvCats), V_, n_split), dim3(256), 0, stream, s, d_leaf_.p, d_soft_lv_.p,
+                           d_soft_m_.p, g_tiles, d_soft_gnode_.p, C_, s.batch, Bp64, (size_t)d.tile_stride / 4, split,
+                           d_leaf_flow_.p, n_split > 1 ? d_part_.p : (float*)nullptr);
+      };
+      if (soft_rows_aligned(s, C_)) run(&hclt_soft_leafflow_kernel<KK, true>);
+      else run(&hclt_soft_leafflow_kernel<KK, false>);
+    });
     if (n_split > 1)
       hipLaunchKernelGGL(sum_parts_kernel<false>, dim3(ceil_div(n_leaf, 64)), dim3(256), 0, stream, d_part_.p, n_split, n_leaf,
                          (const float*)nullptr, d_leaf_flow_.p);

@@ -437,3 +437,30 @@ def test_em_beta_with_soft_reg_and_tempered_flows_matches_oracle(gpu, fscale, up
     # the loop leaves the handle as it found it: an ordinary pass afterwards runs on the block kernels again
     ll = P.probs_flows_circuit(bpc, torch.from_numpy(data[:B]).cuda()).cpu().numpy()
     assert rel_err(ll, O.forward(cur, data[:B], double=True)[-1]).max() < 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,C,B", [(16, 4, 70), (16, 132, 64), (16, 256, 100), (32, 100, 65), (64, 128, 130), (64, 12, 1), (64, 7, 66)])
+def test_rows_in_registers_and_through_lds_agree(gpu, K, C, B):
+    """Evidence rows of whole aligned words stay in registers, rows of any other stride turn through LDS: the same bits,
+    for every place of the same numbers (a longer row, shifted by one, categories not contiguous)."""
+    torch, P = gpu
+    V = 6
+    parent = np.array([-1, 0, 0, 1, 1, 2], np.int32)
+    rng = np.random.default_rng(K + C)
+    bpc = P.hclt_from_clt(parent, C, K)
+    bpc.set_params(np.log(rng.dirichlet(np.ones(K), (V, K))).astype(np.float32), np.log(rng.dirichlet(np.ones(C), (V, K))).astype(np.float32))
+    ev = torch.from_numpy((rng.normal(size=(B, V, C)) * 8 - 300).astype(np.float32)).cuda()
+    ev[:, 1, 1:][torch.rand((B, C - 1), device="cuda") < 0.3] = float("-inf")
+    wide = torch.zeros((B, V, C + 5), device="cuda")
+    wide[:, :, 1:C + 1] = ev
+    turned = ev.permute(2, 1, 0).contiguous().permute(2, 1, 0)
+    ids = torch.randperm(B, dtype=torch.int32, device="cuda")
+    want = None
+    for x in (ev, wide[:, :, 1:C + 1], turned):
+        ll = P.probs_flows_circuit(bpc, x, example_ids=ids).cpu().numpy()
+        got = (ll, *bpc.get_flows())
+        if want is None:
+            want = got
+        for a, b in zip(got, want):
+            assert np.array_equal(np.asarray(a), np.asarray(b), equal_nan=True)
