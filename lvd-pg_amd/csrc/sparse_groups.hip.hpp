@@ -87,6 +87,14 @@ __host__ __device__ inline int64_t group_wb_index(int g, int c, int gt) {   // g
   return ((int64_t)(c >> 4) * (gt * 4) + (g >> 2)) * 64 + (g & 3) * 16 + (c & 15);
 }
 
+// W below float's normal range is kept as -0: nothing to a product, and the mark by which sums and shares that may hang on
+// such an edge (see kLowSum) find it and take its logarithm.
+__device__ __forceinline__ bool group_tiny_w(float w) { return __builtin_bit_cast(uint32_t, w) == 0x80000000u; }
+__device__ __forceinline__ float group_w(float lw) {
+  const float w = __expf(lw);
+  return w >= __FLT_MIN__ ? w : lw > -INFINITY ? -0.f : 0.f;
+}
+
 // exp of the groups' log-parameters in both orders, once per pass (the parameters may have moved): thread = (group,
 // entry of its padded Gp x Cp)
 __global__ __launch_bounds__(256) void sparse_group_w_kernel(GroupDev d, const int32_t* __restrict__ group_of_elem, int64_t total) {
@@ -96,8 +104,7 @@ __global__ __launch_bounds__(256) void sparse_group_w_kernel(GroupDev d, const i
   const int64_t local = i - r.pw0;
   const int g = (int)(local / (16 * r.ct)), c = (int)(local % (16 * r.ct));
   const int e = d.edge[i];
-  float w = e >= 0 ? __expf(d.logp[e] * d.inv_f) : 0.f;
-  if (w < __FLT_MIN__) w = 0.f;   // (no denormal operands: see kLowSum)
+  const float w = e >= 0 ? group_w(d.logp[e] * d.inv_f) : 0.f;
   const_cast<float*>(d.wf)[r.pw0 + group_wf_index(g, c, r.ct)] = w;
   const_cast<float*>(d.wb)[r.pw0 + group_wb_index(g, c, r.gt)] = w;
 }
@@ -130,15 +137,39 @@ __device__ __forceinline__ float group_max4(float v) {
 // next child below.  Every second step takes in a child more, so the loop ends.  Going down, the sums with
 // m - value > kHighShare take the same road: their R is formed for value + off and met by E raised by off.  E is kept
 // under exp(kMaxRaise): a child above that has no share in the sum that asked (its W would be a denormal).
+// Only such sums and shares can hang on a parameter below float's range; where a block has one (group_tiny_w) they
+// are added up in logarithms, edge by edge.
 constexpr float kLowSum = 1e-30f, kHighShare = 60.f, kMaxRaise = 88.f;
 
 template <int NK>
-__device__ __forceinline__ void group_low_sums(const float* xm, int64_t Bp, int hi, const float* w, float mx, bool (&low)[4], float (&val)[4]) {
+__device__ __forceinline__ void group_low_sums(const GroupDev& d, const float* xm, int hi, const float* w, const int32_t* edge, float mx,
+                                               bool (&low)[4], float (&val)[4]) {
   float xs[NK], a[NK];
+  bool tiny = false;
 #pragma unroll
   for (int q = 0; q < NK; ++q) {
-    xs[q] = xm[(int64_t)(4 * q + hi) * Bp];   // (what this lane has just written)
+    xs[q] = xm[(int64_t)(4 * q + hi) * d.Bp];   // (what this lane has just written)
     a[q] = w[q * 64];
+    tiny |= group_tiny_w(a[q]);
+  }
+  if (__any(tiny)) {   // edge: the tile's rows of d.edge, [16][4 NK]
+    __threadfence_block();   // (X - m of the children that the other lanes of the example hold)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (!low[i]) continue;
+      const int32_t* row = edge + (4 * hi + i) * (4 * NK);
+      float top = -INFINITY, sum = 0.f;
+#pragma clang loop unroll(disable)
+      for (int c = 0; c < 4 * NK; ++c)
+        if (row[c] >= 0) top = fmaxf(top, xm[(int64_t)c * d.Bp] + d.logp[row[c]] * d.inv_f);
+      if (top > -INFINITY) {
+#pragma clang loop unroll(disable)
+        for (int c = 0; c < 4 * NK; ++c)
+          if (row[c] >= 0) sum += __expf(xm[(int64_t)c * d.Bp] + d.logp[row[c]] * d.inv_f - top);
+      }
+      val[i] = mx + (top > -INFINITY ? top + __logf(sum) : -INFINITY);
+    }
+    return;
   }
   float off = 0.f;
   for (int it = 0; it < 8 * NK + 2; ++it) {
@@ -237,7 +268,8 @@ __device__ __forceinline__ void group_forward_body(const GroupDev& d, const Grou
       val[i] = mx + __logf(acc[i]);
       low[i] = nd[i] >= 0 && acc[i] < kLowSum;
     }
-    if (__any(low[0] | low[1] | low[2] | low[3])) group_low_sums<NK>(xm, d.Bp, hi, wg + gt * NK * 64, mx, low, val);
+    if (__any(low[0] | low[1] | low[2] | low[3]))
+      group_low_sums<NK>(d, xm, hi, wg + gt * NK * 64, d.edge + base.pw0 + ((int64_t)bx * Gp + gt * 16) * Cp, mx, low, val);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       if (nd[i] >= 0) d.mars[(int64_t)nd[i] * d.Bp + col] = val[i];
@@ -250,11 +282,13 @@ __global__ __launch_bounds__(64) void sparse_group_forward_kernel(GroupDev d, Gr
 }
 
 // The part of the children's rows that comes from sums with m - value > kHighShare (see kLowSum): out[i] for the four
-// children whose X - m are e[i]; w: the children's tile of W in the backward order.
-template <int NG>
+// children whose X - m are e[i]; w: the children's tile of W in the backward order; edge: the group's [4 NG][Cp] entries of
+// d.edge from these four children on.
+template <int NG, int Cp>
 __device__ __forceinline__ void group_high_shares(const GroupDev& d, const int32_t* node, int hi, int64_t col, float mb, const float* w,
-                                                  const float (&e)[4], float (&out)[4]) {
+                                                  const int32_t* edge, const float (&e)[4], float (&out)[4]) {
   float f[NG], t[NG];
+  bool tiny = false;
 #pragma unroll
   for (int k = 0; k < NG; ++k) {
     const int32_t nd = node[4 * k + hi];
@@ -263,6 +297,24 @@ __device__ __forceinline__ void group_high_shares(const GroupDev& d, const int32
     const float nv = d.norm_row < 0 ? d.norm[n * d.Bp + col] : 0.f;
     f[k] = fl;
     t[k] = nd >= 0 && fl > 0.f && v > -INFINITY ? (mb - v) * d.inv_f - nv : 0.f;
+    tiny |= group_tiny_w(w[k * 64]);
+  }
+  if (__any(tiny)) {
+#pragma clang loop unroll(disable)
+    for (int g = 0; g < 4 * NG; ++g) {
+      const int32_t n = node[g];
+      if (n < 0) continue;
+      const float fl = d.flows[(int64_t)n * d.Bp + col], v = d.mars[(int64_t)n * d.Bp + col];
+      const float tg = (mb - v) * d.inv_f - (d.norm_row < 0 ? d.norm[(int64_t)n * d.Bp + col] : 0.f);
+      if (!(fl > 0.f && v > -INFINITY && tg > kHighShare)) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int32_t ed = edge[(int64_t)g * Cp + i];
+        if (ed < 0) continue;
+        const float lw = d.logp[ed] * d.inv_f;
+        if (group_tiny_w(group_w(lw))) out[i] += fl * __expf(e[i] * d.inv_f + lw + tg);
+      }
+    }
   }
   for (int it = 0; it < 4 * NG; ++it) {
     float off = INFINITY;   // the nearest of the example's sums that are left
@@ -361,7 +413,8 @@ __device__ __forceinline__ void group_backward_body(const GroupDev& d, const Gro
     float out[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) out[i] = (e[s][i] > -INFINITY ? __expf(e[s][i] * d.inv_f) : 0.f) * acc[i];
-    if (high) group_high_shares<NG>(d, node, hi, col, mb, wg + ct * NG * 64, e[s], out);
+    if (high)
+      group_high_shares<NG, Cp>(d, node, hi, col, mb, wg + ct * NG * 64, d.edge + base.pw0 + (int64_t)bx * Gp * Cp + ct * 16 + 4 * hi, e[s], out);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float f = out[i];
@@ -432,7 +485,7 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
   float* part_row = d.edge_part + (size_t)blockIdx.y * d.n_edges;
   // a pass takes the (sum, example) pairs with m - value in one interval of kHighShare (see kLowSum): the first one
   // everything below kHighShare, which is nearly always all there is, the next ones the nearest that is left
-  for (int pass = 0, turn = 0; pass <= kLastPass; turn ^= 1) {
+  for (int pass = 0, turn = 0, nth = 0; pass <= kLastPass; turn ^= 1, ++nth) {
     const float off = kHighShare * (float)pass;
     for (int cb = part; cb < Cp; cb += 32) {
       float x[8];
@@ -490,7 +543,19 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
         const int edge = g < r.G && c < r.C ? d.edge[r.pw0 + g * Cp + c] : -1;
         if (edge < 0) continue;   // (in a masked group also a child the sum does not have)
         const float w = d.wf[r.pw0 + group_wf_index(g, c, CT)];
-        const float flow = w > 0.f ? w * acc[i] : 0.f;
+        float flow = w > 0.f ? w * acc[i] : 0.f;
+        if (group_tiny_w(w) && nth == 1) {   // (no pair above kHighShare: nothing goes through such an edge)
+          const int64_t n = d.node[r.pnode0 + g];
+          const float lw = d.logp[edge] * d.inv_f;
+#pragma clang loop unroll(disable)
+          for (int x = 0; x < 64; ++x) {
+            const float fl = d.flows[n * d.Bp + b0 + x], v = d.mars[n * d.Bp + b0 + x];
+            const float nv = d.norm[(d.norm_row >= 0 ? d.norm_row : n) * d.Bp + b0 + x];
+            const float mx = d.m[(int64_t)group * d.Bp + b0 + x];
+            if (fl > 0.f && v > -INFINITY)
+              flow += fl * __expf(d.xm[(int64_t)(r.pslot0 + c) * d.Bp + b0 + x] * d.inv_f + lw + ((mx - v) * d.inv_f - nv));
+          }
+        }
         part_row[edge] = pass == 0 ? flow : part_row[edge] + flow;
       }
     }

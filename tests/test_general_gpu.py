@@ -765,9 +765,9 @@ def test_dense_groups_beside_ordinary_edges(gpu, oracle):
     assert grouped.size("dense_groups") == 2
 
 
-def _masked_multihead(O, rng, levels, G, J, H, keep, sharp, C):
+def _masked_multihead(O, rng, levels, G, J, H, keep, sharp, C, tiny=0.0):
     """Heads over a chain of `levels` sets of G sums whose children are random parts of the J products below (two at
-    least); leaves whose log-probabilities lie `sharp` apart."""
+    least); leaves whose log-probabilities lie `sharp` apart; a share of `tiny` of the parameters lies below exp's range."""
     from helpers import log_dirichlet
 
     def leaf(v):
@@ -781,7 +781,12 @@ def _masked_multihead(O, rng, levels, G, J, H, keep, sharp, C):
         for _ in range(G):
             kept = rng.random(J) < keep
             kept[rng.choice(J, 2, replace=False)] = True
-            sums.append(O.summate(*[subs[j] for j in np.flatnonzero(kept)], logps=log_dirichlet(rng, int(kept.sum()))))
+            logps = log_dirichlet(rng, int(kept.sum()))
+            if tiny:
+                small = rng.random(len(logps)) < tiny
+                small[rng.integers(len(logps))] = False
+                logps[small] = -(88 + 40 * rng.random(int(small.sum()))).astype(np.float32)
+            sums.append(O.summate(*[subs[j] for j in np.flatnonzero(kept)], logps=logps))
         subs = [O.multiply(sums[j % G], leaf(2 + l)) for j in range(J)]
     return [O.summate(*subs, logps=log_dirichlet(rng, J)) for _ in range(H)]
 
@@ -798,6 +803,17 @@ def test_masked_groups(gpu, oracle, levels, G, J, H, keep, sharp, B, groups):
     heads = _masked_multihead(oracle, rng, levels, G, J, H, keep, sharp, C)
     grouped, _ = _check_grouped_multihead(gpu, oracle, heads, 2 + levels, C, B, 72, min_groups=1)
     assert grouped.size("dense_groups") == groups
+
+
+@pytest.mark.parametrize("G,J,keep,sharp,B", [(16, 16, 0.6, 100.0, 100), (33, 65, 0.4, 60.0, 65), (20, 20, 1.0, 100.0, 70),
+                                              (17, 20, 0.5, 1.0, 40)])
+def test_groups_with_parameters_below_the_range_of_exp(gpu, oracle, G, J, keep, sharp, B):
+    """exp of a log-parameter under -87.3 is no normal float any more; where the other children of a sum lie further down
+    still, its value and its flow go through that edge all the same (keep = 1: sums with the same children)."""
+    rng = np.random.default_rng(77)
+    heads = _masked_multihead(oracle, rng, 2, G, J, 4, keep, sharp, 5, tiny=0.5)
+    grouped, _ = _check_grouped_multihead(gpu, oracle, heads, 4, 5, B, 78, min_groups=2)
+    assert grouped.size("dense_groups") == 3
 
 
 @pytest.mark.parametrize("fscale", [0.5, 2.5])
