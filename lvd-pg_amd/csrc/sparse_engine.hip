@@ -1201,7 +1201,7 @@ __global__ __launch_bounds__(256) void sparse_product_edge_kernel(const int2* __
 // its products -- over the union of their children, W zero where a sum lacks a child; in reach of each other through
 // shared children, a layer at a time.  A block costs the same however thin it is (and a layer that is all blocks joins
 // the walks), an edge at a time the layer kernels cost little less for few edges: 192 variables, 128 heads, 16 batches of
-// 512, K = 32: 6.3 ms as blocks at any share of the pairs, edge by edge 9.9 at 60 %, 8.2 at 30 %, 8.0 at 15 %, 7.8 at 10
+// 512, K = 32: 6.45 ms as blocks at any share of the pairs, edge by edge 9.9 at 60 %, 8.2 at 30 %, 8.0 at 15 %, 7.8 at 10
 // and 5 % (4 batches of 4096: 3.6 against 5.0 at 30 %, 4.4 at 10 %; K = 16, 512: 4.05 against 7.2 at 60 %, 7.0 at 30 %).
 // So the line is only one pair in kMaskedShare, two children of 32: sums that merely touch stay apart.
 // PCMI355_DENSE_GROUPS=0 in the environment keeps every node on the layer kernels (for comparisons).
@@ -1219,9 +1219,10 @@ void SparseCircuit::build_groups(std::vector<int32_t>& group_of, std::vector<int
   auto sorted_edges = [&](int32_t n) {
     std::vector<int32_t> es(fc_.node_e1[n] - fc_.node_e0[n]);
     for (size_t i = 0; i < es.size(); ++i) es[i] = fc_.node_e0[n] + (int32_t)i;
-    std::sort(es.begin(), es.end(), [&](int32_t a, int32_t b) {
-      return std::make_tuple(fc_.e_prime[a], fc_.e_sub[a], a) < std::make_tuple(fc_.e_prime[b], fc_.e_sub[b], b);
-    });
+    auto before = [&](int32_t a, int32_t b) {
+      return std::tie(fc_.e_prime[a], fc_.e_sub[a], a) < std::tie(fc_.e_prime[b], fc_.e_sub[b], b);
+    };
+    if (!std::is_sorted(es.begin(), es.end(), before)) std::sort(es.begin(), es.end(), before);   // (builders mostly list them in order)
     return es;
   };
   if (!(env && env[0] == '0')) {
@@ -1273,31 +1274,40 @@ void SparseCircuit::build_groups(std::vector<int32_t>& group_of, std::vector<int
       return n;
     };
     std::map<int32_t, std::vector<int32_t>> by_layer, connected;
+    std::vector<int32_t> last_with_prime(nn, -1);   // child without a sub -> the last sum seen that has it
     for (int64_t n = 0; n < nn; ++n)
       if (fc_.type[n] == kSum && !taken[n] && fc_.node_e1[n] - fc_.node_e0[n] <= kGroupMaxSide) by_layer[fc_.layer[n]].push_back((int32_t)n);
     for (const auto& kv : by_layer) {
-      std::unordered_map<uint64_t, int32_t> last_with;   // child -> the last sum seen that has it
+      std::unordered_map<uint64_t, int32_t> last_with;   // child with a sub -> the last sum seen that has it
       for (int32_t n : kv.second) root_of[n] = n;
       for (int32_t n : kv.second) {
         for (int32_t e = fc_.node_e0[n]; e < fc_.node_e1[n]; ++e) {
-          const auto at = last_with.emplace((uint64_t)(uint32_t)fc_.e_prime[e] << 32 | (uint32_t)fc_.e_sub[e], n);
-          if (at.second) continue;
-          if (at.first->second == n) taken[n] = 1;   // the same child twice: two parameters for one entry of W
-          const int32_t a = root(at.first->second), b = root(n);
-          root_of[std::max(a, b)] = std::min(a, b);
-          at.first->second = n;
+          const int32_t prime = fc_.e_prime[e], sub = fc_.e_sub[e];
+          int32_t& last = sub < 0 ? last_with_prime[prime]
+                                  : last_with.emplace((uint64_t)(uint32_t)prime << 32 | (uint32_t)sub, -1).first->second;
+          if (last >= 0 && fc_.layer[last] == kv.first) {   // (a child may have sums in several layers)
+            if (last == n) taken[n] = 1;   // the same child twice: two parameters for one entry of W
+            const int32_t a = root(last), b = root(n);
+            root_of[std::max(a, b)] = std::min(a, b);
+          }
+          last = n;
         }
       }
       for (int32_t n : kv.second)
         if (!taken[n]) connected[root(n)].push_back(n);
     }
+    std::vector<int32_t> in_set_of(nn, -1);   // child without a sub -> the first sum of the last group that listed it
     for (const auto& kv : connected) {
       for (size_t m0 = 0; m0 < kv.second.size(); m0 += kGroupMaxSide) {
         const size_t g = std::min<size_t>(kGroupMaxSide, kv.second.size() - m0);
         Found f{fc_.layer[kv.first], std::vector<int32_t>(kv.second.begin() + m0, kv.second.begin() + m0 + g), 0, {}};
         int64_t edges = 0;
         for (int32_t n : f.nodes)
-          for (int32_t e = fc_.node_e0[n]; e < fc_.node_e1[n]; ++e, ++edges) f.set.emplace_back(fc_.e_prime[e], fc_.e_sub[e]);
+          for (int32_t e = fc_.node_e0[n]; e < fc_.node_e1[n]; ++e, ++edges) {
+            if (fc_.e_sub[e] < 0 && in_set_of[fc_.e_prime[e]] == f.nodes[0]) continue;
+            if (fc_.e_sub[e] < 0) in_set_of[fc_.e_prime[e]] = f.nodes[0];
+            f.set.emplace_back(fc_.e_prime[e], fc_.e_sub[e]);
+          }
         std::sort(f.set.begin(), f.set.end());
         f.set.erase(std::unique(f.set.begin(), f.set.end()), f.set.end());
         f.children = (int)f.set.size();
