@@ -825,18 +825,48 @@ __global__ __launch_bounds__(256) void sparse_leaf_flow_soft_kernel(SparseDev d,
     }
 }
 
-// (a record that names a dense group's row behind the node rows is not an edge: its flow is taken as it is)
-__global__ void sparse_gather_in_logp_kernel(const int4* __restrict__ in_rec, const float* __restrict__ logp, int64_t n,
-                                             int64_t n_nodes, float* __restrict__ in_logp) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int4 r = in_rec[i];
-  in_logp[i] = (r.y < 0 && (int64_t)~r.y >= n_nodes) ? 0.f : logp[r.x >> 1];
+// What a flow pass finds done: the accumulators scaled by what is kept of them (0: cleared, whatever they held), the rows of
+// partial edge flows cleared (an edge that no wave visits must read as zero), the parameters of the backward records
+// gathered.  Four kernels of about 5 us before, most of each its launch: one launch, a range of workgroups to each job
+// and 16-byte words (epoch of 16 batches, 192 variables, 128 heads: 6.43 -> 6.36 ms); parts and accumulators start at an allocation's first byte.
+struct FlowsStart {
+  float* edge_aggr; int64_t n_edges;
+  float* leaf_flow; int64_t n_leaf;
+  float* parts; int64_t n_parts;
+  const int4* in_rec; const float* logp; int64_t n_rec, n_nodes;
+  float* in_logp;
+  float rate;
+  int edge_blocks, leaf_blocks, part_blocks;   // workgroups of the first three jobs
+};
+constexpr int kStartFloats = 1024;   // per workgroup of the first three
+
+__device__ __forceinline__ void scale_words(float* __restrict__ p, int64_t n, float rate, int block) {
+  const int64_t i = (int64_t)block * kStartFloats + 4 * threadIdx.x;
+  if (i + 4 <= n) {
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (rate != 0.f) {
+      x = *reinterpret_cast<const float4*>(p + i);
+      x = make_float4(x.x * rate, x.y * rate, x.z * rate, x.w * rate);
+    }
+    *reinterpret_cast<float4*>(p + i) = x;
+  } else {
+    for (int64_t k = i; k < n; ++k) p[k] = rate != 0.f ? p[k] * rate : 0.f;
+  }
 }
 
-__global__ void sparse_scale_kernel(float* p, int64_t n, float rate) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = rate != 0.f ? p[i] * rate : 0.f;
+__global__ __launch_bounds__(256) void sparse_flows_start_kernel(FlowsStart f) {
+  int block = blockIdx.x;
+  if (block < f.edge_blocks) return scale_words(f.edge_aggr, f.n_edges, f.rate, block);
+  block -= f.edge_blocks;
+  if (block < f.leaf_blocks) return scale_words(f.leaf_flow, f.n_leaf, f.rate, block);
+  block -= f.leaf_blocks;
+  if (block < f.part_blocks) return scale_words(f.parts, f.n_parts, 0.f, block);
+  block -= f.part_blocks;
+  const int64_t i = (int64_t)block * 256 + threadIdx.x;
+  if (i >= f.n_rec) return;
+  // (a record that names a dense group's row behind the node rows is not an edge: its flow is taken as it is)
+  const int4 r = f.in_rec[i];
+  f.in_logp[i] = (r.y < 0 && (int64_t)~r.y >= f.n_nodes) ? 0.f : f.logp[r.x >> 1];
 }
 
 // EM update, one wave per node (lanes over the node's edges / categories): add_pseudocount,
@@ -1996,21 +2026,38 @@ void SparseCircuit::flows_soft(const SoftRef& s, float rate, const float* d_head
 void SparseCircuit::run_flows(int batch, const SoftRef* soft, float rate, const float* d_head_mask, float* d_ll, bool accumulate) {
   const int Bp = ceil_div(batch, 64) * 64;
   const int64_t ne = fc_.n_edges();
+  // edge flows summed over the batch: one row of partial sums per 64 examples, added into the accumulators in row
+  // order after the walk
+  const int n_parts = Bp / 64;
+  FlowsStart start{};
+  start.rate = rate;
   if (accumulate) {
-    hipLaunchKernelGGL(sparse_scale_kernel, dim3(ceil_div(std::max<int64_t>(ne, 1), 256)), dim3(256), 0, stream, d_edge_aggr_.p, ne, rate);
-    hipLaunchKernelGGL(sparse_scale_kernel, dim3(ceil_div((int64_t)fc_.leaf_logp.size(), 256)), dim3(256), 0, stream,
-                       d_leaf_flow_.p, (int64_t)fc_.leaf_logp.size(), rate);
+    start.edge_aggr = d_edge_aggr_.p;
+    start.n_edges = ne;
+    start.leaf_flow = d_leaf_flow_.p;
+    start.n_leaf = (int64_t)fc_.leaf_logp.size();
   }
+  if (ne) {
+    d_in_logp_.ensure(d_in_rec_.n);
+    d_edge_part_.ensure((size_t)n_parts * ne);
+    start.parts = d_edge_part_.p;
+    start.n_parts = (int64_t)n_parts * ne;
+    start.in_rec = d_in_rec_.p;
+    start.logp = d_logp_.p;
+    start.n_rec = (int64_t)d_in_rec_.n;
+    start.n_nodes = fc_.n_nodes();
+    start.in_logp = d_in_logp_.p;
+  }
+  start.edge_blocks = (int)ceil_div(start.n_edges, kStartFloats);
+  start.leaf_blocks = (int)ceil_div(start.n_leaf, kStartFloats);
+  start.part_blocks = (int)ceil_div(start.n_parts, kStartFloats);
+  const int64_t start_blocks = start.edge_blocks + start.leaf_blocks + (int64_t)start.part_blocks + ceil_div(start.n_rec, 256);
+  if (start_blocks) hipLaunchKernelGGL(sparse_flows_start_kernel, dim3((unsigned)start_blocks), dim3(256), 0, stream, start);
   SparseDev d = SPARSE_DEV(batch, Bp, d_visit_.p);
   d.n_flow_rows = n_flow_rows();
   if (soft) { d.ev = soft->d_ev; d.ev_se = soft->stride_ex; d.ev_sv = soft->stride_var; d.ev_sc = soft->stride_cat; d.ev_idx = soft->d_idx; }
   SparseDev db = d;
-  if (ne) {
-    d_in_logp_.ensure(d_in_rec_.n);
-    hipLaunchKernelGGL(sparse_gather_in_logp_kernel, dim3(ceil_div((int64_t)d_in_rec_.n, 256)), dim3(256), 0, stream,
-                       d_in_rec_.p, d_logp_.p, (int64_t)d_in_rec_.n, fc_.n_nodes(), d_in_logp_.p);
-    db.in_logp = d_in_logp_.p;
-  }
+  if (ne) db.in_logp = d_in_logp_.p;
   db.order = d_bwd_order_.p;   // the layers without the input nodes whose rows other nodes write
   const bool tempered = accumulate && flow_scale != 1.f;
   if (tempered) {
@@ -2020,14 +2067,6 @@ void SparseCircuit::run_flows(int batch, const SoftRef* soft, float rate, const 
     hipLaunchKernelGGL(sparse_tempered_norm_kernel, dim3((unsigned)(fc_.n_nodes() + 1), ceil_div(Bp, 256)), dim3(256), 0, stream, db,
                        d_norm_.p);
     refresh_group_w(db.inv_f);   // W^(1 / fscale) for this pass; the next forward pass puts W back
-  }
-  // edge flows summed over the batch: one row of partial sums per 64 examples, cleared first (an edge that
-  // no wave visits must read as zero), added into the accumulators in row order after the walk
-  const int n_parts = Bp / 64;
-  if (ne) {
-    d_edge_part_.ensure((size_t)n_parts * ne);
-    hipLaunchKernelGGL(sparse_scale_kernel, dim3(ceil_div((int64_t)n_parts * ne, 256)), dim3(256), 0, stream, d_edge_part_.p,
-                       (int64_t)n_parts * ne, 0.f);
   }
   int next_run = (int)group_runs_bwd_.size() - 1;
   for (int l = n_layers_ - 1; l >= 0; --l) {

@@ -231,6 +231,26 @@ def test_per_example_weights(gpu, oracle):
         P.mini_batch_em_with_reg(a, d, 1, batch_size=50, pseudocount=0.1, param_inertia=0.4, weights=w[:10])
 
 
+@pytest.mark.parametrize("V,C,width,B", [(2, 3, 1, 3), (3, 5, 2, 64), (5, 7, 3, 65), (6, 4, 5, 200)])
+def test_what_is_kept_of_the_accumulators(gpu, oracle, V, C, width, B):
+    """A second batch on top of `rate` of the first's statistics, and on nothing of them, NaN included; circuits whose numbers
+    of edges and leaf entries are no multiple of the words and workgroups that clear and scale them."""
+    torch, P = gpu
+    from helpers import random_dag
+    rng = np.random.default_rng(83)
+    bpc = _compile(P, [random_dag(V, C, rng, width=width)], V, C)
+    d = torch.from_numpy(rng.integers(0, C, size=(B, V)).astype(np.uint8)).cuda()
+    P.probs_flows_circuit(bpc, d)
+    first = bpc.get_aggregates()
+    P.probs_flows_circuit(bpc, d, rate=0.25)   # 0.25 a + a: one rounding of the sum where it is formed in order
+    for a, b in zip(first, bpc.get_aggregates()):
+        assert np.abs(b - 1.25 * a).max() <= 1e-5 * max(np.abs(a).max(), 1.0)
+    P.probs_flows_circuit(bpc, d, rate=float("nan"))
+    P.probs_flows_circuit(bpc, d)
+    for a, b in zip(first, bpc.get_aggregates()):
+        assert np.array_equal(a, b)
+
+
 def test_driver_called_again_without_clearing_its_flow_memory(gpu, oracle):
     """`init_clear_mem = false` (src-jl/multi_head_pc/em.jl:6,28-31): two calls of one epoch, the second keeping the
     accumulators, are one call of two epochs; with the default the second call starts from cleared ones."""
