@@ -133,13 +133,14 @@ __device__ __forceinline__ float group_max4(float v) {
 // Sums far below their group's maximum.  E = exp(X - m) leaves float's range 87 below m, and a sum without a share in
 // the children near m -- masked groups (build_groups) have many -- may own nothing above that.  A sum that comes out
 // below kLowSum is added up again with E = exp(X - m + off) for an offset raised step by step (per example, so the
-// matrix instruction's columns stay independent): 60 further, which brings out every child E still held, then to the
-// next child below.  Every second step takes in a child more, so the loop ends.  Going down, the sums with
-// m - value > kHighShare take the same road: their R is formed for value + off and met by E raised by off.  E is kept
-// under exp(kMaxRaise): a child above that has no share in the sum that asked (its W would be a denormal).
+// matrix instruction's columns stay independent).  A step raises the highest child that has not had its turn to
+// kHighShare, and with it the children up to kTurn below, which are then at kHighShare - kTurn = 20 or more: as W >= FLT_MIN,
+// W E >= 5.8e-30 shows any of them that the sum has.  So when E is cut off at exp(kMaxRaise), for children far above, no sum
+// that is still looked for has one of those, and every step takes in a child more, so the loop ends.  Going down, the sums with
+// m - value > kHighShare take the same road: their R is formed for value + off and met by E raised by off.
 // Only such sums and shares can hang on a parameter below float's range; where a block has one (group_tiny_w) they
 // are added up in logarithms, edge by edge.
-constexpr float kLowSum = 1e-30f, kHighShare = 60.f, kMaxRaise = 88.f;
+constexpr float kLowSum = 1e-30f, kHighShare = 60.f, kTurn = 40.f, kMaxRaise = 88.f;
 
 template <int NK>
 __device__ __forceinline__ void group_low_sums(const GroupDev& d, const float* xm, int hi, const float* w, const int32_t* edge, float mx,
@@ -171,19 +172,16 @@ __device__ __forceinline__ void group_low_sums(const GroupDev& d, const float* x
     }
     return;
   }
-  float off = 0.f;
-  for (int it = 0; it < 8 * NK + 2; ++it) {
-    if (!(it & 1)) {
-      off += kHighShare;
-    } else {
-      float next = -INFINITY;
+  float turned = INFINITY;   // the children from here up have had their turn
+  for (int it = 0; it <= 4 * NK; ++it) {
+    float next = -INFINITY;
 #pragma unroll
-      for (int q = 0; q < NK; ++q) if (xs[q] < -off - 40.f) next = fmaxf(next, xs[q]);
-      next = group_max4(next);
-      if (next > -INFINITY) off = -next;
-      else low[0] = low[1] = low[2] = low[3] = false;   // nothing further down: what S was, it is
-    }
+    for (int q = 0; q < NK; ++q) if (xs[q] < turned) next = fmaxf(next, xs[q]);
+    next = group_max4(next);
+    if (!(next > -INFINITY)) low[0] = low[1] = low[2] = low[3] = false;   // nothing further down: what S was, it is
     if (!__any(low[0] | low[1] | low[2] | low[3])) break;
+    const float off = next > -INFINITY ? kHighShare - next : 0.f;
+    turned = next - kTurn;
     g4f acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int q = 0; q < NK; ++q)

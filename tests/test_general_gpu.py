@@ -785,9 +785,10 @@ def test_dense_groups_beside_ordinary_edges(gpu, oracle):
     assert grouped.size("dense_groups") == 2
 
 
-def _masked_multihead(O, rng, levels, G, J, H, keep, sharp, C, tiny=0.0):
+def _masked_multihead(O, rng, levels, G, J, H, keep, sharp, C, tiny=0.0, down=(88, 128)):
     """Heads over a chain of `levels` sets of G sums whose children are random parts of the J products below (two at
-    least); leaves whose log-probabilities lie `sharp` apart; a share of `tiny` of the parameters lies below exp's range."""
+    least); leaves whose log-probabilities lie `sharp` apart; a share of `tiny` of the log-parameters lies `down` below
+    0 (the default: below exp's range)."""
     from helpers import log_dirichlet
 
     def leaf(v):
@@ -805,7 +806,7 @@ def _masked_multihead(O, rng, levels, G, J, H, keep, sharp, C, tiny=0.0):
             if tiny:
                 small = rng.random(len(logps)) < tiny
                 small[rng.integers(len(logps))] = False
-                logps[small] = -(88 + 40 * rng.random(int(small.sum()))).astype(np.float32)
+                logps[small] = -(down[0] + (down[1] - down[0]) * rng.random(int(small.sum()))).astype(np.float32)
             sums.append(O.summate(*[subs[j] for j in np.flatnonzero(kept)], logps=logps))
         subs = [O.multiply(sums[j % G], leaf(2 + l)) for j in range(J)]
     return [O.summate(*subs, logps=log_dirichlet(rng, J)) for _ in range(H)]
@@ -834,6 +835,37 @@ def test_groups_with_parameters_below_the_range_of_exp(gpu, oracle, G, J, keep, 
     heads = _masked_multihead(oracle, rng, 2, G, J, 4, keep, sharp, 5, tiny=0.5)
     grouped, _ = _check_grouped_multihead(gpu, oracle, heads, 4, 5, B, 78, min_groups=2)
     assert grouped.size("dense_groups") == 3
+
+
+@pytest.mark.parametrize("G,J,keep,sharp,B", [(16, 16, 0.6, 60.0, 100), (33, 65, 0.4, 60.0, 65), (20, 20, 1.0, 100.0, 70),
+                                              (12, 20, 0.5, 30.0, 64)])
+def test_groups_with_small_parameters_in_exps_range(gpu, oracle, G, J, keep, sharp, B):
+    """Log-parameters of -30 to -87 on children 0 to some hundreds below the block's maximum: normal floats whose
+    product with exp(X - m + offset) is below what shows unless the offset is the child's own."""
+    rng = np.random.default_rng(79)
+    heads = _masked_multihead(oracle, rng, 2, G, J, 4, keep, sharp, 5, tiny=0.6, down=(30, 87))
+    _check_grouped_multihead(gpu, oracle, heads, 4, 5, B, 80, min_groups=2)
+
+
+@pytest.mark.parametrize("gaps,logw", [((0, -95), (None, -40)), ((0, -80), (None, -60)), ((0, -95, -200), (None, -40, -1e-3)),
+                                       ((0, -41, -300), (None, -87, -87)), ((0, -60, -101), (None, -87, -46)), ((0, -1), (None, -87))])
+def test_a_sum_that_hangs_on_one_small_parameter(gpu, oracle, gaps, logw):
+    """Sums whose children lie at `gaps` below the block's maximum with log-parameters `logw` (None: not a child, so that
+    the maximum belongs to others), beside sums that have all the children."""
+    O = oracle
+    rng = np.random.default_rng(82)
+    C, J, G = 2, 16, 8
+    leaf = lambda v, x: O.input_node(v, np.float32([x, x]))
+    subs = [O.multiply(leaf(0, gaps[j] if j < len(gaps) else -400.0 - j), leaf(1, 0.0)) for j in range(J)]
+    own = [(subs[j], w) for j, w in enumerate(logw) if w is not None]
+    own += [(subs[-1], 0.0)] if len(own) < 2 else []         # (far below: no share in the sum)
+    sums = [O.summate(*[c for c, _ in own], logps=np.float32([w for _, w in own])) for _ in range(G)]
+    for g in range(G):                                       # (all but one each: no two of them the same children)
+        sums.append(O.summate(*[c for j, c in enumerate(subs) if j != 4 + g], logps=np.log(rng.dirichlet(np.ones(J - 1))).astype(np.float32)))
+    tops = [O.multiply(s, leaf(2, 0.0)) for s in sums]
+    heads = [O.summate(*tops, logps=np.full(2 * G, -np.log(2 * G), np.float32)) for _ in range(4)]
+    grouped, _ = _check_grouped_multihead(gpu, oracle, heads, 3, C, 70, 83, min_groups=2)
+    assert grouped.size("dense_groups") == 2                 # the masked one and the heads'
 
 
 @pytest.mark.parametrize("fscale", [0.5, 2.5])
