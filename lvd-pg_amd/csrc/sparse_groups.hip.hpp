@@ -464,27 +464,28 @@ __global__ __launch_bounds__(WV * 64) void sparse_group_walk_kernel(GroupDev d, 
 // examples, from the values and flows the pass has left.  A workgroup takes (group, 64 examples): E and R in LDS (a
 // wave stages every fourth child, whose row numbers are the same for its 64 lanes: scalar loads, the rows of eight
 // children requested before the first is used), the GT x CT tiles of the result dealt out over its four waves.
+// R E is share / W and is added up over the examples before W comes in, so the product only takes pairs (sum, example)
+// with m - value up to kHighShare.  The edges of a sum that has others as well are added up again in logarithms,
+// example by example: X and log R in the same LDS, every exponent then that of a share.
 template <int GT, int CT>
 __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int first) {
   extern __shared__ float glds[];
-  __shared__ int next_pass[2];
-  constexpr int kLastPass = 1 << 20;
+  __shared__ int row_high[GT * 16];
+  __shared__ int any_again;
   const int group = d.order[first + blockIdx.x];
   const GroupRec r = d.rec[group];
   constexpr int Gp = GT * 16, Cp = CT * 16;
-  const int b0 = blockIdx.y * 64;
   float* E = glds;
-  float* R = E + (size_t)Cp * kGroupPad;
+  float* R = E + Cp * kGroupPad;
+  const int b0 = blockIdx.y * 64;
   const int t = threadIdx.x;
   const int b = t & 63, part = guni(t >> 6);
   const float mb = d.m[(int64_t)group * d.Bp + b0 + b];
   const int lane = t & 63, wave = t >> 6;
   const int lo = lane & 15, hi = lane >> 4;
   float* part_row = d.edge_part + (size_t)blockIdx.y * d.n_edges;
-  // a pass takes the (sum, example) pairs with m - value in one interval of kHighShare (see kLowSum): the first one
-  // everything below kHighShare, which is nearly always all there is, the next ones the nearest that is left
-  for (int pass = 0, turn = 0, nth = 0; pass <= kLastPass; turn ^= 1, ++nth) {
-    const float off = kHighShare * (float)pass;
+  // child(c, X - m) for the wave's children, sum(g, flow (0: none), m - value) for its sums
+  auto stage = [&](auto&& child, auto&& sum) {
     for (int cb = part; cb < Cp; cb += 32) {
       float x[8];
 #pragma unroll
@@ -493,12 +494,9 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
         x[q] = c < Cp ? d.xm[(int64_t)(r.pslot0 + c) * d.Bp + b0 + b] : -INFINITY;
       }
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int c = cb + 4 * q;
-        if (c < Cp) E[c * kGroupPad + b] = x[q] > -INFINITY ? __expf(fminf(x[q] * d.inv_f + off, kMaxRaise)) : 0.f;
-      }
+      for (int q = 0; q < 8; ++q)
+        if (cb + 4 * q < Cp) child(cb + 4 * q, x[q] > -INFINITY ? x[q] * d.inv_f : -INFINITY);
     }
-    int left = kLastPass + 1;
     for (int gb = part; gb < Gp; gb += 32) {   // (eight sums' rows requested before the first is used, as above)
       float f[8], v[8], nv[8];
 #pragma unroll
@@ -515,50 +513,68 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
         }
       }
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int g = gb + 4 * q;
-        const bool some = f[q] > 0.f && v[q] > -INFINITY;
-        const float tq = (mb - v[q]) * d.inv_f - nv[q];
-        const int mine = tq > kHighShare ? (int)fminf(tq * (1.f / kHighShare), (float)kLastPass) : 0;
-        if (some && mine > pass) left = min(left, mine);
-        if (g < Gp) R[g * kGroupPad + b] = some && mine == pass ? f[q] * __expf(tq - off) : 0.f;
-      }
+      for (int q = 0; q < 8; ++q)
+        if (gb + 4 * q < Gp) sum(gb + 4 * q, f[q] > 0.f && v[q] > -INFINITY ? f[q] : 0.f, (mb - v[q]) * d.inv_f - nv[q]);
     }
-    if (t == 0) next_pass[turn] = kLastPass + 1;
-    __syncthreads();
-    if (left <= kLastPass) atomicMin(&next_pass[turn], left);
-    for (int tile = wave; tile < GT * CT; tile += 4) {
-      const int gt = tile / CT, ct = tile % CT;
-      g4f acc = {0.f, 0.f, 0.f, 0.f};
+  };
+  if (t == 0) any_again = 0;
+  stage([&](int c, float x) { E[c * kGroupPad + b] = __expf(x); },
+        [&](int g, float f, float tq) {
+          const bool high = f > 0.f && tq > kHighShare;
+          R[g * kGroupPad + b] = f > 0.f && !high ? f * __expf(tq) : 0.f;
+          const bool row = __any(high);
+          if (b == 0) row_high[g] = row;
+        });
+  __syncthreads();
+  uint64_t again = 0;   // a bit per (tile of the wave, i): edges to be added up in logarithms
+  int nth = 0;
+  for (int tile = wave; tile < GT * CT; tile += 4, ++nth) {
+    const int gt = tile / CT, ct = tile % CT;
+    g4f acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int kk = 0; kk < 16; ++kk)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(R[(gt * 16 + lo) * kGroupPad + kk * 4 + hi], E[(ct * 16 + lo) * kGroupPad + kk * 4 + hi],
-                                                   acc, 0, 0, 0);
-      const int c = ct * 16 + lo;
+    for (int kk = 0; kk < 16; ++kk)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(R[(gt * 16 + lo) * kGroupPad + kk * 4 + hi], E[(ct * 16 + lo) * kGroupPad + kk * 4 + hi],
+                                                 acc, 0, 0, 0);
+    const int c = ct * 16 + lo;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int g = gt * 16 + 4 * hi + i;
-        const int edge = g < r.G && c < r.C ? d.edge[r.pw0 + g * Cp + c] : -1;
-        if (edge < 0) continue;   // (in a masked group also a child the sum does not have)
-        const float w = d.wf[r.pw0 + group_wf_index(g, c, CT)];
-        float flow = w > 0.f ? w * acc[i] : 0.f;
-        if (group_tiny_w(w) && nth == 1) {   // (no pair above kHighShare: nothing goes through such an edge)
-          const int64_t n = d.node[r.pnode0 + g];
-          const float lw = d.logp[edge] * d.inv_f;
-#pragma clang loop unroll(disable)
-          for (int x = 0; x < 64; ++x) {
-            const float fl = d.flows[n * d.Bp + b0 + x], v = d.mars[n * d.Bp + b0 + x];
-            const float nv = d.norm[(d.norm_row >= 0 ? d.norm_row : n) * d.Bp + b0 + x];
-            const float mx = d.m[(int64_t)group * d.Bp + b0 + x];
-            if (fl > 0.f && v > -INFINITY)
-              flow += fl * __expf(d.xm[(int64_t)(r.pslot0 + c) * d.Bp + b0 + x] * d.inv_f + lw + ((mx - v) * d.inv_f - nv));
-          }
-        }
-        part_row[edge] = pass == 0 ? flow : part_row[edge] + flow;
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int g = gt * 16 + 4 * hi + i;
+      const int edge = g < r.G && c < r.C ? d.edge[r.pw0 + g * Cp + c] : -1;
+      if (edge < 0) continue;   // (in a masked group also a child the sum does not have)
+      if (row_high[g]) again |= (uint64_t)1 << (4 * nth + i);
+      else part_row[edge] = d.wf[r.pw0 + group_wf_index(g, c, CT)] * acc[i];
     }
-    __syncthreads();
-    pass = next_pass[turn];
+  }
+  if (again) any_again = 1;
+  __syncthreads();
+  if (!any_again) return;
+  stage([&](int c, float x) { E[c * kGroupPad + b] = x; },
+        [&](int g, float f, float tq) { R[g * kGroupPad + b] = f > 0.f ? __logf(f) + tq : -INFINITY; });
+  __syncthreads();
+  nth = 0;
+  for (int tile = wave; tile < GT * CT; tile += 4, ++nth) {
+    const int mine = (int)(again >> (4 * nth)) & 15;
+    if (!__any(mine)) continue;
+    const int gt = tile / CT, ct = tile % CT, c = ct * 16 + lo;
+    const float* Ec = E + c * kGroupPad;
+    const float* Rg = R + (gt * 16 + 4 * hi) * kGroupPad;
+    int edge[4];
+    float lw[4], flow[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      edge[i] = mine >> i & 1 ? d.edge[r.pw0 + (gt * 16 + 4 * hi + i) * Cp + c] : -1;
+      lw[i] = edge[i] >= 0 ? d.logp[edge[i]] * d.inv_f : -INFINITY;
+      flow[i] = 0.f;
+    }
+#pragma unroll 4
+    for (int x = 0; x < 64; ++x) {
+      const float e = Ec[x];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) flow[i] += __expf(e + Rg[i * kGroupPad + x] + lw[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (edge[i] >= 0) part_row[edge[i]] = flow[i];
   }
 }
 

@@ -847,14 +847,11 @@ def test_groups_with_small_parameters_in_exps_range(gpu, oracle, G, J, keep, sha
     _check_grouped_multihead(gpu, oracle, heads, 4, 5, B, 80, min_groups=2)
 
 
-@pytest.mark.parametrize("gaps,logw", [((0, -95), (None, -40)), ((0, -80), (None, -60)), ((0, -95, -200), (None, -40, -1e-3)),
-                                       ((0, -41, -300), (None, -87, -87)), ((0, -60, -101), (None, -87, -46)), ((0, -1), (None, -87))])
-def test_a_sum_that_hangs_on_one_small_parameter(gpu, oracle, gaps, logw):
-    """Sums whose children lie at `gaps` below the block's maximum with log-parameters `logw` (None: not a child, so that
-    the maximum belongs to others), beside sums that have all the children."""
-    O = oracle
+def _sums_beside_full_ones(O, gaps, logw, taken=0.0, G=8, J=16, H=4):
+    """Heads over sums whose children lie at `gaps` below the block's maximum with log-parameters `logw` (None: not a
+    child, so that the maximum belongs to others), beside sums that have nearly all the children; `taken` is what the
+    products over the first kind have on the others."""
     rng = np.random.default_rng(82)
-    C, J, G = 2, 16, 8
     leaf = lambda v, x: O.input_node(v, np.float32([x, x]))
     subs = [O.multiply(leaf(0, gaps[j] if j < len(gaps) else -400.0 - j), leaf(1, 0.0)) for j in range(J)]
     own = [(subs[j], w) for j, w in enumerate(logw) if w is not None]
@@ -862,10 +859,23 @@ def test_a_sum_that_hangs_on_one_small_parameter(gpu, oracle, gaps, logw):
     sums = [O.summate(*[c for c, _ in own], logps=np.float32([w for _, w in own])) for _ in range(G)]
     for g in range(G):                                       # (all but one each: no two of them the same children)
         sums.append(O.summate(*[c for j, c in enumerate(subs) if j != 4 + g], logps=np.log(rng.dirichlet(np.ones(J - 1))).astype(np.float32)))
-    tops = [O.multiply(s, leaf(2, 0.0)) for s in sums]
-    heads = [O.summate(*tops, logps=np.full(2 * G, -np.log(2 * G), np.float32)) for _ in range(4)]
-    grouped, _ = _check_grouped_multihead(gpu, oracle, heads, 3, C, 70, 83, min_groups=2)
+    tops = [O.multiply(s, leaf(2, taken if q < G else 0.0)) for q, s in enumerate(sums)]
+    return [O.summate(*tops, logps=np.full(2 * G, -np.log(2 * G), np.float32)) for _ in range(H)]
+
+
+@pytest.mark.parametrize("gaps,logw", [((0, -95), (None, -40)), ((0, -80), (None, -60)), ((0, -95, -200), (None, -40, -1e-3)),
+                                       ((0, -41, -300), (None, -87, -87)), ((0, -60, -101), (None, -87, -46)), ((0, -1), (None, -87))])
+def test_a_sum_that_hangs_on_one_small_parameter(gpu, oracle, gaps, logw):
+    grouped, _ = _check_grouped_multihead(gpu, oracle, _sums_beside_full_ones(oracle, gaps, logw), 3, 2, 70, 83, min_groups=2)
     assert grouped.size("dense_groups") == 2                 # the masked one and the heads'
+
+
+@pytest.mark.parametrize("logw", [-61.0, -80.0, -84.0, -86.0, -87.2, -88.0, -100.0])
+def test_all_flow_through_one_small_parameter(gpu, oracle, logw):
+    """The child at the block's maximum, all 64 examples of a block and their whole flow behind one edge: flow / W is
+    as far up as it goes."""
+    heads = _sums_beside_full_ones(oracle, (0,), (logw,), taken=-logw + 30.0)
+    _check_grouped_multihead(gpu, oracle, heads, 3, 2, 128, 84, min_groups=2)
 
 
 @pytest.mark.parametrize("fscale", [0.5, 2.5])
