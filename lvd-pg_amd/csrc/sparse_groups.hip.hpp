@@ -87,8 +87,8 @@ __host__ __device__ inline int64_t group_wb_index(int g, int c, int gt) {   // g
   return ((int64_t)(c >> 4) * (gt * 4) + (g >> 2)) * 64 + (g & 3) * 16 + (c & 15);
 }
 
-// W below float's normal range is kept as -0: nothing to a product, and the mark by which sums and shares that may hang on
-// such an edge (see kLowSum) find it and take its logarithm.
+// W below float's normal range is kept as -0: nothing to a product, and the mark by which sums that may hang on such an
+// edge (see kLowSum) find it and take its logarithm.
 __device__ __forceinline__ bool group_tiny_w(float w) { return __builtin_bit_cast(uint32_t, w) == 0x80000000u; }
 __device__ __forceinline__ float group_w(float lw) {
   const float w = __expf(lw);
@@ -136,10 +136,9 @@ __device__ __forceinline__ float group_max4(float v) {
 // matrix instruction's columns stay independent).  A step raises the highest child that has not had its turn to
 // kHighShare, and with it the children up to kTurn below, which are then at kHighShare - kTurn = 20 or more: as W >= FLT_MIN,
 // W E >= 5.8e-30 shows any of them that the sum has.  So when E is cut off at exp(kMaxRaise), for children far above, no sum
-// that is still looked for has one of those, and every step takes in a child more, so the loop ends.  Going down, the sums with
-// m - value > kHighShare take the same road: their R is formed for value + off and met by E raised by off.
-// Only such sums and shares can hang on a parameter below float's range; where a block has one (group_tiny_w) they
-// are added up in logarithms, edge by edge.
+// that is still looked for has one of those, and every step takes in a child more, so the loop ends.
+// Only such sums can hang on a parameter below float's range; where a block has one (group_tiny_w) they are added up in
+// logarithms, edge by edge.  Going down, so are the shares of all sums with m - value > kHighShare.
 constexpr float kLowSum = 1e-30f, kHighShare = 60.f, kTurn = 40.f, kMaxRaise = 88.f;
 
 template <int NK>
@@ -279,57 +278,39 @@ __global__ __launch_bounds__(64) void sparse_group_forward_kernel(GroupDev d, Gr
   group_forward_body<GT, CT>(d, base, blockIdx.x, threadIdx.x, blockIdx.y);
 }
 
-// The part of the children's rows that comes from sums with m - value > kHighShare (see kLowSum): out[i] for the four
-// children whose X - m are e[i]; w: the children's tile of W in the backward order; edge: the group's [4 NG][Cp] entries of
-// d.edge from these four children on.
+// The part of the children's rows that comes from sums with m - value > kHighShare (see kLowSum), edge by edge with the
+// exponent of the share: flow * W and exp(X - m) * share / W both leave float's range on the way to a share that does not.
+// out[i]: the rows of the four children whose X - m are e[i]; edge: the group's [4 NG][Cp] entries of d.edge from these
+// four children on (16-byte words).
 template <int NG, int Cp>
-__device__ __forceinline__ void group_high_shares(const GroupDev& d, const int32_t* node, int hi, int64_t col, float mb, const float* w,
-                                                  const int32_t* edge, const float (&e)[4], float (&out)[4]) {
-  float f[NG], t[NG];
-  bool tiny = false;
-#pragma unroll
-  for (int k = 0; k < NG; ++k) {
-    const int32_t nd = node[4 * k + hi];
-    const int64_t n = nd < 0 ? 0 : nd;
-    const float fl = d.flows[n * d.Bp + col], v = d.mars[n * d.Bp + col];
-    const float nv = d.norm_row < 0 ? d.norm[n * d.Bp + col] : 0.f;
-    f[k] = fl;
-    t[k] = nd >= 0 && fl > 0.f && v > -INFINITY ? (mb - v) * d.inv_f - nv : 0.f;
-    tiny |= group_tiny_w(w[k * 64]);
-  }
-  if (__any(tiny)) {
+__device__ __forceinline__ void group_shares_by_edge(const GroupDev& d, const int32_t* node, int64_t col, float mb, const int32_t* edge,
+                                                     const float (&e)[4], float (&out)[4]) {
 #pragma clang loop unroll(disable)
-    for (int g = 0; g < 4 * NG; ++g) {
-      const int32_t n = node[g];
-      if (n < 0) continue;
-      const float fl = d.flows[(int64_t)n * d.Bp + col], v = d.mars[(int64_t)n * d.Bp + col];
-      const float tg = (mb - v) * d.inv_f - (d.norm_row < 0 ? d.norm[(int64_t)n * d.Bp + col] : 0.f);
-      if (!(fl > 0.f && v > -INFINITY && tg > kHighShare)) continue;
+  for (int k = 0; k < NG; ++k) {
+    const int4 n4 = *reinterpret_cast<const int4*>(node + 4 * k);
+    const int nd[4] = {n4.x, n4.y, n4.z, n4.w};
+    float f[4], t[4];
+    bool take = false;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int64_t n = nd[g] < 0 ? 0 : nd[g];
+      f[g] = d.flows[n * d.Bp + col];
+      const float v = d.mars[n * d.Bp + col];
+      t[g] = (mb - v) * d.inv_f - (d.norm_row < 0 ? d.norm[n * d.Bp + col] : 0.f);
+      if (!(nd[g] >= 0 && f[g] > 0.f && v > -INFINITY && t[g] > kHighShare)) f[g] = 0.f;
+      take |= f[g] > 0.f;
+    }
+    if (!__any(take)) continue;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int4 e4 = *reinterpret_cast<const int4*>(edge + (int64_t)(4 * k + g) * Cp);
+      const int ed[4] = {e4.x, e4.y, e4.z, e4.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int32_t ed = edge[(int64_t)g * Cp + i];
-        if (ed < 0) continue;
-        const float lw = d.logp[ed] * d.inv_f;
-        if (group_tiny_w(group_w(lw))) out[i] += fl * __expf(e[i] * d.inv_f + lw + tg);
+        const float lw = ed[i] >= 0 ? d.logp[ed[i]] * d.inv_f : -INFINITY;
+        if (f[g] > 0.f) out[i] += f[g] * __expf(e[i] * d.inv_f + lw + t[g]);
       }
     }
-  }
-  for (int it = 0; it < 4 * NG; ++it) {
-    float off = INFINITY;   // the nearest of the example's sums that are left
-#pragma unroll
-    for (int k = 0; k < NG; ++k) if (t[k] > kHighShare) off = fminf(off, t[k]);
-    off = -group_max4(-off);
-    if (!__any(off < INFINITY)) break;
-    g4f acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < NG; ++k) {
-      const bool now = t[k] > kHighShare && t[k] <= off + kHighShare && off < INFINITY;
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[k * 64], now ? f[k] * __expf(t[k] - off) : 0.f, acc, 0, 0, 0);
-      if (now) t[k] = 0.f;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (e[i] > -INFINITY && off < INFINITY) out[i] += __expf(fminf(e[i] * d.inv_f + off, kMaxRaise)) * acc[i];
   }
 }
 
@@ -412,7 +393,7 @@ __device__ __forceinline__ void group_backward_body(const GroupDev& d, const Gro
 #pragma unroll
     for (int i = 0; i < 4; ++i) out[i] = (e[s][i] > -INFINITY ? __expf(e[s][i] * d.inv_f) : 0.f) * acc[i];
     if (high)
-      group_high_shares<NG, Cp>(d, node, hi, col, mb, wg + ct * NG * 64, d.edge + base.pw0 + (int64_t)bx * Gp * Cp + ct * 16 + 4 * hi, e[s], out);
+      group_shares_by_edge<NG, Cp>(d, node, col, mb, d.edge + base.pw0 + (int64_t)bx * Gp * Cp + ct * 16 + 4 * hi, e[s], out);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float f = out[i];

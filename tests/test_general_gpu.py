@@ -878,6 +878,38 @@ def test_all_flow_through_one_small_parameter(gpu, oracle, logw):
     _check_grouped_multihead(gpu, oracle, heads, 3, 2, 128, 84, min_groups=2)
 
 
+def _check_small_shares(gpu, O, heads, V, C, B, scale=1.0, edges=True):
+    """Flows (and edge statistics) of a grouped circuit one by one against the 64-bit oracle's, however small: rounding of
+    exponents of up to 128 (half an ulp: 4e-6) at about a dozen places from the heads down."""
+    torch, P = gpu
+    rng = np.random.default_rng(91)
+    bpc = _compile(P, heads, V, C, len(heads))
+    assert bpc.size("dense_groups") >= 1
+    fc = O.bits_compile(O.summate(*heads), C, V)
+    root_ids = (bpc.table("heads") - 1).astype(np.int32)
+    data = rng.integers(0, C, size=(B, V)).astype(np.uint8)
+    mask = ((rng.random((B, len(heads))) + 0.05) * scale).astype(np.float32)
+    skip = (fc.edge_parent() == fc.n_nodes - 1).astype(np.uint8)
+    flows_ref, ea_ref = O.backward(fc, O.forward(fc, data, double=True), skip=skip, root_ids=root_ids,
+                                   root_flow=np.ascontiguousarray(mask.T.astype(np.float64)), double=True)
+    order = fc.up_order()
+    order = order[fc.edge_parent()[order] != fc.n_nodes - 1]
+    P.probs_flows_circuit(bpc, torch.from_numpy(data).cuda(), head_mask=torch.from_numpy(mask).cuda())
+    pairs = [(bpc.get_node_values(B)[1], flows_ref[:-1])] + ([(bpc.get_aggregates()[0], ea_ref[order])] if edges else [])
+    for got, want in pairs:
+        at = want > 1e-30
+        assert at.any() and (np.abs(got[at] - want[at]) / want[at]).max() < 1e-4
+        assert (got[~at] < 2e-30).all()
+
+
+@pytest.mark.parametrize("logw", [-61.0, -70.0, -86.0, -87.2, -95.0])
+@pytest.mark.parametrize("scale", [1.0, 1e-6, 1e-12])
+def test_small_flows_behind_a_small_parameter(gpu, oracle, logw, scale):
+    """Flows of 1 to 1e-12 go through an edge of log-parameter -61 to -95 whole: W times such a flow is no normal float."""
+    heads = _sums_beside_full_ones(oracle, (0,), (logw,), taken=-logw + 30.0)
+    _check_small_shares(gpu, oracle, heads, 3, 2, 70, scale=scale, edges=False)
+
+
 @pytest.mark.parametrize("fscale", [0.5, 2.5])
 def test_tempered_flows_of_masked_groups(gpu, oracle, fscale):
     """Tempered flows of masked groups against the layer kernels', sharp leaves included."""
