@@ -109,6 +109,12 @@ __global__ __launch_bounds__(256) void sparse_group_w_kernel(GroupDev d, const i
   const_cast<float*>(d.wb)[r.pw0 + group_wb_index(g, c, r.gt)] = w;
 }
 
+// exp(x) * y with a product in float's range, whatever exp(x) alone would be
+__device__ __forceinline__ float group_exp_times(float x, float y) {
+  const float a = fmaxf(x, -2000.f) * 1.44269504f, n = rintf(a);   // (log2 e; -inf: far enough down)
+  return ldexpf(__builtin_amdgcn_exp2f(a - n) * y, (int)n);
+}
+
 __device__ __forceinline__ int guni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // X of a child for the example in column `col`: the value of its prime (the first three rows: the prime itself and
@@ -278,13 +284,15 @@ __global__ __launch_bounds__(64) void sparse_group_forward_kernel(GroupDev d, Gr
   group_forward_body<GT, CT>(d, base, blockIdx.x, threadIdx.x, blockIdx.y);
 }
 
-// The part of the children's rows that comes from sums with m - value > kHighShare (see kLowSum), edge by edge with the
-// exponent of the share: flow * W and exp(X - m) * share / W both leave float's range on the way to a share that does not.
+// The part of the children's rows that the product on the matrix cores leaves out, edge by edge with the exponent of the
+// share: what comes from sums with m - value > kHighShare (see kLowSum; flow * W and exp(X - m) * share / W both leave
+// float's range on the way to a share that does not) and, where the tile has such edges (tiny), what goes through a W below
+// float's range.
 // out[i]: the rows of the four children whose X - m are e[i]; edge: the group's [4 NG][Cp] entries of d.edge from these
 // four children on (16-byte words).
 template <int NG, int Cp>
-__device__ __forceinline__ void group_shares_by_edge(const GroupDev& d, const int32_t* node, int64_t col, float mb, const int32_t* edge,
-                                                     const float (&e)[4], float (&out)[4]) {
+__device__ __forceinline__ void group_shares_by_edge(const GroupDev& d, const int32_t* node, int64_t col, float mb, bool tiny,
+                                                     const int32_t* edge, const float (&e)[4], float (&out)[4]) {
 #pragma clang loop unroll(disable)
   for (int k = 0; k < NG; ++k) {
     const int4 n4 = *reinterpret_cast<const int4*>(node + 4 * k);
@@ -297,7 +305,7 @@ __device__ __forceinline__ void group_shares_by_edge(const GroupDev& d, const in
       f[g] = d.flows[n * d.Bp + col];
       const float v = d.mars[n * d.Bp + col];
       t[g] = (mb - v) * d.inv_f - (d.norm_row < 0 ? d.norm[n * d.Bp + col] : 0.f);
-      if (!(nd[g] >= 0 && f[g] > 0.f && v > -INFINITY && t[g] > kHighShare)) f[g] = 0.f;
+      if (!(nd[g] >= 0 && f[g] > 0.f && v > -INFINITY && (tiny || t[g] > kHighShare))) f[g] = 0.f;
       take |= f[g] > 0.f;
     }
     if (!__any(take)) continue;
@@ -308,7 +316,7 @@ __device__ __forceinline__ void group_shares_by_edge(const GroupDev& d, const in
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float lw = ed[i] >= 0 ? d.logp[ed[i]] * d.inv_f : -INFINITY;
-        if (f[g] > 0.f) out[i] += f[g] * __expf(e[i] * d.inv_f + lw + t[g]);
+        if (f[g] > 0.f && (t[g] > kHighShare || group_tiny_w(group_w(lw)))) out[i] += f[g] * __expf(e[i] * d.inv_f + lw + t[g]);
       }
     }
   }
@@ -391,9 +399,13 @@ __device__ __forceinline__ void group_backward_body(const GroupDev& d, const Gro
     for (int k = 0; k < NG; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][k], rv[k], acc, 0, 0, 0);
     float out[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) out[i] = (e[s][i] > -INFINITY ? __expf(e[s][i] * d.inv_f) : 0.f) * acc[i];
-    if (high)
-      group_shares_by_edge<NG, Cp>(d, node, col, mb, d.edge + base.pw0 + (int64_t)bx * Gp * Cp + ct * 16 + 4 * hi, e[s], out);
+    for (int i = 0; i < 4; ++i) out[i] = group_exp_times(e[s][i] * d.inv_f, acc[i]);   // (sum_g W R reaches e^kHighShare)
+    uint32_t signs = 0;   // W >= 0 but for the mark of a tiny one, -0
+#pragma unroll
+    for (int k = 0; k < NG; ++k) signs |= __builtin_bit_cast(uint32_t, a[s][k]);
+    const bool tiny = __any((int32_t)signs < 0);
+    if (high || tiny)
+      group_shares_by_edge<NG, Cp>(d, node, col, mb, tiny, d.edge + base.pw0 + (int64_t)bx * Gp * Cp + ct * 16 + 4 * hi, e[s], out);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float f = out[i];

@@ -910,6 +910,18 @@ def test_small_flows_behind_a_small_parameter(gpu, oracle, logw, scale):
     _check_small_shares(gpu, oracle, heads, 3, 2, 70, scale=scale, edges=False)
 
 
+SMALL_SHARES = [((0, -95), (None, 0), 50.0), ((0, -40, -100), (None, 0, 0), 40.0), ((0, -40, -101, -110), (None, -1, -0.5, -4), 41.0),
+                ((0, -50, -117.5), (None, 0, 0), 50.0), ((0, -55, 0), (None, 0, -88), 55.0), ((0, -50, -2), (None, 0, -100), 50.0)]
+
+
+@pytest.mark.parametrize("gaps,logw,taken", SMALL_SHARES)
+def test_small_shares_of_children_far_down(gpu, oracle, gaps, logw, taken):
+    """Shares of 1e-13 to 1e-30 in sums 30 to 60 below the block's maximum: of children more than 87 below it, where
+    exp(X - m) alone is no float any more, and through a W that is none."""
+    heads = _sums_beside_full_ones(oracle, gaps, logw, taken=taken + 30.0)
+    _check_small_shares(gpu, oracle, heads, 3, 2, 70, edges=False)
+
+
 @pytest.mark.parametrize("fscale", [0.5, 2.5])
 def test_tempered_flows_of_masked_groups(gpu, oracle, fscale):
     """Tempered flows of masked groups against the layer kernels', sharp leaves included."""
