@@ -109,10 +109,10 @@ __global__ __launch_bounds__(256) void sparse_group_w_kernel(GroupDev d, const i
   const_cast<float*>(d.wb)[r.pw0 + group_wb_index(g, c, r.gt)] = w;
 }
 
-// exp(x) * y with a product in float's range, whatever exp(x) alone would be
-__device__ __forceinline__ float group_exp_times(float x, float y) {
+// exp(x) * y * 2^bits with a product in float's range, whatever exp(x) alone would be
+__device__ __forceinline__ float group_exp_times(float x, float y, int bits = 0) {
   const float a = fmaxf(x, -2000.f) * 1.44269504f, n = rintf(a);   // (log2 e; -inf: far enough down)
-  return ldexpf(__builtin_amdgcn_exp2f(a - n) * y, (int)n);
+  return ldexpf(__builtin_amdgcn_exp2f(a - n) * y, (int)n + bits);
 }
 
 __device__ __forceinline__ int guni(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -458,12 +458,18 @@ __global__ __launch_bounds__(WV * 64) void sparse_group_walk_kernel(GroupDev d, 
 // wave stages every fourth child, whose row numbers are the same for its 64 lanes: scalar loads, the rows of eight
 // children requested before the first is used), the GT x CT tiles of the result dealt out over its four waves.
 // R E is share / W and is added up over the examples before W comes in, so the product only takes pairs (sum, example)
-// with m - value up to kHighShare.  The edges of a sum that has others as well are added up again in logarithms,
-// example by example: X and log R in the same LDS, every exponent then that of a share.
+// with m - value up to kHighShare.  In it E is kept 2^kEdgeBits up and R as much down, exactly: what is lost of a flow of 1
+// to zeros below float's range is then less than 2^-83 + e^-57 per pair, on both sides.  The edges of a sum that has pairs
+// above kHighShare, and those that come out below kLowFlow (or have a W below float's range, which is kept as -0) though
+// neither their sum is without flow nor their child impossible all over, are added up again in logarithms, example by
+// example: X and log R in the same LDS, every exponent then that of a share.
+constexpr int kEdgeBits = 43;
+constexpr float kLowFlow = 1e-15f;
+
 template <int GT, int CT>
 __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int first) {
   extern __shared__ float glds[];
-  __shared__ int row_high[GT * 16];
+  __shared__ int row_some[GT * 16], row_high[GT * 16], child_some[CT * 16];   // of a sum: any flow, any pair above kHighShare
   __shared__ int any_again;
   const int group = d.order[first + blockIdx.x];
   const GroupRec r = d.rec[group];
@@ -511,12 +517,19 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
     }
   };
   if (t == 0) any_again = 0;
-  stage([&](int c, float x) { E[c * kGroupPad + b] = __expf(x); },
+  stage([&](int c, float x) {
+          E[c * kGroupPad + b] = group_exp_times(x, 1.f, kEdgeBits);
+          const bool some = __any(x > -INFINITY);
+          if (b == 0) child_some[c] = some;
+        },
         [&](int g, float f, float tq) {
           const bool high = f > 0.f && tq > kHighShare;
-          R[g * kGroupPad + b] = f > 0.f && !high ? f * __expf(tq) : 0.f;
-          const bool row = __any(high);
-          if (b == 0) row_high[g] = row;
+          R[g * kGroupPad + b] = f > 0.f && !high ? group_exp_times(tq, f, -kEdgeBits) : 0.f;
+          const bool some = __any(f > 0.f), row = __any(high);
+          if (b == 0) {
+            row_some[g] = some;
+            row_high[g] = row;
+          }
         });
   __syncthreads();
   uint64_t again = 0;   // a bit per (tile of the wave, i): edges to be added up in logarithms
@@ -534,8 +547,10 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
       const int g = gt * 16 + 4 * hi + i;
       const int edge = g < r.G && c < r.C ? d.edge[r.pw0 + g * Cp + c] : -1;
       if (edge < 0) continue;   // (in a masked group also a child the sum does not have)
-      if (row_high[g]) again |= (uint64_t)1 << (4 * nth + i);
-      else part_row[edge] = d.wf[r.pw0 + group_wf_index(g, c, CT)] * acc[i];
+      const float w = d.wf[r.pw0 + group_wf_index(g, c, CT)], flow = w * acc[i];
+      const bool there = row_some[g] && child_some[c] && (w > 0.f || group_tiny_w(w));
+      if (there && (row_high[g] || flow < kLowFlow)) again |= (uint64_t)1 << (4 * nth + i);
+      else part_row[edge] = flow;
     }
   }
   if (again) any_again = 1;

@@ -922,6 +922,14 @@ def test_small_shares_of_children_far_down(gpu, oracle, gaps, logw, taken):
     _check_small_shares(gpu, oracle, heads, 3, 2, 70, edges=False)
 
 
+@pytest.mark.parametrize("gaps,logw,taken", SMALL_SHARES)
+@pytest.mark.parametrize("scale", [1.0, 1e-9])
+def test_edge_flows_of_small_shares(gpu, oracle, gaps, logw, taken, scale):
+    """... and the edges' own statistics, down to 1e-30 of a whole block's."""
+    heads = _sums_beside_full_ones(oracle, gaps, logw, taken=taken + 30.0)
+    _check_small_shares(gpu, oracle, heads, 3, 2, 70, scale=scale)
+
+
 @pytest.mark.parametrize("fscale", [0.5, 2.5])
 def test_tempered_flows_of_masked_groups(gpu, oracle, fscale):
     """Tempered flows of masked groups against the layer kernels', sharp leaves included."""
