@@ -287,7 +287,9 @@ __global__ __launch_bounds__(64) void sparse_group_forward_kernel(GroupDev d, Gr
 // The part of the children's rows that the product on the matrix cores leaves out, edge by edge with the exponent of the
 // share: what comes from sums with m - value > kHighShare (see kLowSum; flow * W and exp(X - m) * share / W both leave
 // float's range on the way to a share that does not) and, where the tile has such edges (tiny), what goes through a W below
-// float's range.
+// float's range from sums with m - value > kTinyShare (from others: shares below e^-67).
+constexpr float kTinyShare = 20.f;
+
 // out[i]: the rows of the four children whose X - m are e[i]; edge: the group's [4 NG][Cp] entries of d.edge from these
 // four children on (16-byte words).
 template <int NG, int Cp>
@@ -305,7 +307,7 @@ __device__ __forceinline__ void group_shares_by_edge(const GroupDev& d, const in
       f[g] = d.flows[n * d.Bp + col];
       const float v = d.mars[n * d.Bp + col];
       t[g] = (mb - v) * d.inv_f - (d.norm_row < 0 ? d.norm[n * d.Bp + col] : 0.f);
-      if (!(nd[g] >= 0 && f[g] > 0.f && v > -INFINITY && (tiny || t[g] > kHighShare))) f[g] = 0.f;
+      if (!(nd[g] >= 0 && f[g] > 0.f && v > -INFINITY && t[g] > (tiny ? kTinyShare : kHighShare))) f[g] = 0.f;
       take |= f[g] > 0.f;
     }
     if (!__any(take)) continue;
@@ -362,7 +364,7 @@ __device__ __forceinline__ void group_backward_body(const GroupDev& d, const Gro
     for (int ct = 0; ct < CT; ++ct) numbers(ct, ct);
   }
   float rv[NG];
-  bool high = false;
+  bool high = false, middle = false;
   {   // R = F / S = F * exp(m - value): no flow stays no flow where the value is -inf.  (All rows requested, then used:
       // written as one loop the compiler waits for every sum's rows in turn.)
     float f[NG], v[NG], nv[NG];
@@ -382,10 +384,12 @@ __device__ __forceinline__ void group_backward_body(const GroupDev& d, const Gro
       const float t = (mb - v[k]) * d.inv_f - nv[k];
       const bool some = nd[k] >= 0 && f[k] > 0.f && v[k] > -INFINITY;
       high |= some && t > kHighShare;
+      middle |= some && t > kTinyShare;
       rv[k] = some && !(t > kHighShare) ? f[k] * __expf(t) : 0.f;
     }
   }
   high = __any(high);
+  middle = __any(middle);
   if constexpr (kPre) {
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) values(ct, ct);
@@ -403,7 +407,7 @@ __device__ __forceinline__ void group_backward_body(const GroupDev& d, const Gro
     uint32_t signs = 0;   // W >= 0 but for the mark of a tiny one, -0
 #pragma unroll
     for (int k = 0; k < NG; ++k) signs |= __builtin_bit_cast(uint32_t, a[s][k]);
-    const bool tiny = __any((int32_t)signs < 0);
+    const bool tiny = middle && __any((int32_t)signs < 0);
     if (high || tiny)
       group_shares_by_edge<NG, Cp>(d, node, col, mb, tiny, d.edge + base.pw0 + (int64_t)bx * Gp * Cp + ct * 16 + 4 * hi, e[s], out);
 #pragma unroll
@@ -458,18 +462,22 @@ __global__ __launch_bounds__(WV * 64) void sparse_group_walk_kernel(GroupDev d, 
 // wave stages every fourth child, whose row numbers are the same for its 64 lanes: scalar loads, the rows of eight
 // children requested before the first is used), the GT x CT tiles of the result dealt out over its four waves.
 // R E is share / W and is added up over the examples before W comes in, so the product only takes pairs (sum, example)
-// with m - value up to kHighShare.  In it E is kept 2^kEdgeBits up and R as much down, exactly: what is lost of a flow of 1
-// to zeros below float's range is then less than 2^-83 + e^-57 per pair, on both sides.  The edges of a sum that has pairs
-// above kHighShare, and those that come out below kLowFlow (or have a W below float's range, which is kept as -0) though
-// neither their sum is without flow nor their child impossible all over, are added up again in logarithms, example by
-// example: X and log R in the same LDS, every exponent then that of a share.
-constexpr int kEdgeBits = 43;
-constexpr float kLowFlow = 1e-15f;
+// with m - value up to kEdgeShare.  In it E is kept 2^kEdgeBits up and R as much down, exactly: E then reaches down to
+// X - m = -109 and R to flow / S = e^-65, so a pair of a flow of 1 whose share falls out has one below e^-64.  The edges
+// of a sum that has pairs above kEdgeShare, and those that come out below kLowFlow (64 such pairs are 1e-5 of it) though
+// neither their sum is without flow nor their child impossible all over nor W zero, are added up again in logarithms,
+// example by example: X and log R in the same LDS, every exponent then that of a share.
+// 192 variables, 128 heads, K = 32, batches of 512: 12 us for the bodies' groups and 23 for the heads' with parameters as
+// training starts from, 19 and 37 after 20 epochs (all 64 examples of an edge instead of those with flow: 19 and 48).
+// With 30 or 60 as the limit, 21 or 43 bits and 1e-24 or 1e-18 for kLowFlow: 2 and 3 us more for the bodies' groups.
+constexpr float kEdgeShare = 45.f, kLowFlow = 1e-21f;
+constexpr int kEdgeBits = 32;
 
 template <int GT, int CT>
 __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int first) {
   extern __shared__ float glds[];
-  __shared__ int row_some[GT * 16], row_high[GT * 16], child_some[CT * 16];   // of a sum: any flow, any pair above kHighShare
+  __shared__ uint64_t row_some[GT * 16];                     // of a sum: the examples with flow
+  __shared__ int row_high[GT * 16], child_some[CT * 16];     // ... any pair above kEdgeShare; of a child: any example it is possible in
   __shared__ int any_again;
   const int group = d.order[first + blockIdx.x];
   const GroupRec r = d.rec[group];
@@ -523,9 +531,10 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
           if (b == 0) child_some[c] = some;
         },
         [&](int g, float f, float tq) {
-          const bool high = f > 0.f && tq > kHighShare;
+          const bool high = f > 0.f && tq > kEdgeShare;
           R[g * kGroupPad + b] = f > 0.f && !high ? group_exp_times(tq, f, -kEdgeBits) : 0.f;
-          const bool some = __any(f > 0.f), row = __any(high);
+          const uint64_t some = __ballot(f > 0.f);
+          const bool row = __any(high);
           if (b == 0) {
             row_some[g] = some;
             row_high[g] = row;
@@ -556,8 +565,14 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
   if (again) any_again = 1;
   __syncthreads();
   if (!any_again) return;
-  stage([&](int c, float x) { E[c * kGroupPad + b] = x; },
-        [&](int g, float f, float tq) { R[g * kGroupPad + b] = f > 0.f ? __logf(f) + tq : -INFINITY; });
+  stage([&](int c, float x) {
+          E[c * kGroupPad + b] = x;
+          if (b == 0) E[c * kGroupPad + 64] = 0.f;   // (column 64 stands for no example)
+        },
+        [&](int g, float f, float tq) {
+          R[g * kGroupPad + b] = f > 0.f ? __logf(f) + tq : -INFINITY;
+          if (b == 0) R[g * kGroupPad + 64] = -INFINITY;
+        });
   __syncthreads();
   nth = 0;
   for (int tile = wave; tile < GT * CT; tile += 4, ++nth) {
@@ -574,11 +589,26 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
       lw[i] = edge[i] >= 0 ? d.logp[edge[i]] * d.inv_f : -INFINITY;
       flow[i] = 0.f;
     }
-#pragma unroll 4
-    for (int x = 0; x < 64; ++x) {
-      const float e = Ec[x];
+    // the examples any of the tile's sums has flow in, four at a time
+    uint32_t left[2] = {0u, 0u};
+    for (int g = 0; g < 16; ++g) {
+      left[0] |= (uint32_t)row_some[gt * 16 + g];
+      left[1] |= (uint32_t)(row_some[gt * 16 + g] >> 32);
+    }
+    uint64_t examples = (uint64_t)(uint32_t)guni((int)left[1]) << 32 | (uint32_t)guni((int)left[0]);
+    while (examples) {
+      int x[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) flow[i] += __expf(e + Rg[i * kGroupPad + x] + lw[i]);
+      for (int u = 0; u < 4; ++u) {
+        x[u] = examples ? __builtin_ctzll(examples) : 64;
+        examples &= examples - 1;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float e = Ec[x[u]];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) flow[i] += __expf(e + Rg[i * kGroupPad + x[u]] + lw[i]);
+      }
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
