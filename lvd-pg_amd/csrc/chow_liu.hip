@@ -437,6 +437,8 @@ static float prim_take_row(const float* row, int32_t pick, int V, float* best, i
 void chow_liu_tree(const float* mi, int V, int32_t* parent_out) {
   if (!mi || !parent_out) fail(PCM_ERR_ARG, "matrix or output pointer is null");
   if (V < 1) fail(PCM_ERR_SHAPE, "num_vars must be positive, got %d", V);
+  for (int v = 1; v < V; ++v)   // (the first vertex's links start the tree; a later row's NaN is a link that is not there)
+    if (std::isnan(mi[v])) fail(PCM_ERR_ARG, "mutual information matrix holds NaN or -inf in row %d", v);
   std::vector<float> best(V, -INFINITY);
   std::vector<int32_t> link(V, 0);
   std::vector<std::vector<int32_t>> adj(V);

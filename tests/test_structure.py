@@ -88,6 +88,30 @@ def test_chow_liu_tree_host_entry_matches_oracle():
         P.chow_liu_tree(np.full((3, 3), np.nan, np.float32))
 
 
+@pytest.mark.parametrize("V", [2, 7, 10, 19])
+def test_chow_liu_tree_and_single_nans(V):
+    """A NaN among the first vertex's links is refused wherever it stands, as is a vertex without a link; any other NaN is
+    a link that is not there."""
+    import pcmi355 as P
+    rng = np.random.default_rng(V)
+    mi = rng.random((V, V)).astype(np.float32)
+    mi = mi + mi.T
+    for v in range(1, V):
+        bad = mi.copy()
+        bad[0, v] = np.nan
+        with pytest.raises(P.PcmError):
+            P.chow_liu_tree(bad)
+        bad[0, v], bad[:, v] = 1.0, -np.inf
+        bad[v] = -np.inf
+        with pytest.raises(P.PcmError):
+            P.chow_liu_tree(bad)
+    for u in range(1, V):
+        for v in range(V):
+            odd, none = mi.copy(), mi.copy()
+            odd[u, v], none[u, v] = np.nan, -np.inf
+            assert np.array_equal(P.chow_liu_tree(odd), P.chow_liu_tree(none))
+
+
 # ---- the HIP path -------------------------------------------------------------------------
 
 @pytest.fixture(scope="module")
