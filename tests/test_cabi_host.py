@@ -174,3 +174,27 @@ def test_describe_dag_is_topological():
     heads = simple_multihead_circuit(5)
     d = describe_dag(heads)
     assert d["node_type"][-2:].tolist() == [O.SUM, O.SUM] and len(d["node_type"]) == 10
+
+
+@pytest.mark.parametrize("n,batch_size,largest", [((3 << 20) + 7, 1000, 1 << 20), ((3 << 20) + 7, 2 << 20, 2 << 20), (5000, 1000, 5000),
+                                                  (5000, None, 5000)])
+def test_scoring_batches_stay_within_the_batch_argument(monkeypatch, n, batch_size, largest):
+    """Circuits on the lean walk score small batches together, but never all of a large data set in one call, whose batch
+    is a 32-bit integer; no batch is larger than the caller's for it."""
+    import torch
+    from pcmi355 import queries
+
+    class Lean:
+        num_heads = 0
+
+        def size(self, what):
+            return 1
+
+    calls = []
+    monkeypatch.setattr(queries, "_check_data", lambda bpc, data: None)
+    monkeypatch.setattr(queries, "_forward", lambda bpc, data, d_ptr, i_ptr, b, out_ptr: calls.append((d_ptr, b)))
+    data = torch.zeros((n, 1), dtype=torch.uint8)
+    out = queries.loglikelihoods(Lean(), data, batch_size=batch_size)
+    assert out.shape == (n,) and max(b for _, b in calls) == largest
+    assert [p - data.data_ptr() for p, _ in calls] == np.concatenate([[0], np.cumsum([b for _, b in calls])])[:-1].tolist()
+    assert sum(b for _, b in calls) == n
