@@ -1378,9 +1378,12 @@ const HcltCircuit::LeanPlan* HcltCircuit::fine_plan(int nslices) const {
   return best;
 }
 
-// the lean kernels address every array with 32-bit offsets from one descriptor
-bool HcltCircuit::lean_fits(int batch) const {
-  return lean_ && !force_general_walks_ && (size_t)(n_inner_ + 1) * tile_floats(ceil_div(batch, kSlice)) * 4 < ((size_t)1 << 31);
+// the lean kernels address every array with 32-bit offsets from one descriptor: the tiles, or where none are kept the
+// categories
+bool HcltCircuit::lean_fits(int batch, int keep) const {
+  const int ns = ceil_div(batch, kSlice);
+  const size_t per_node = keep == kKeepNone ? (size_t)ns * kSlice : tile_floats(ns);
+  return lean_ && !force_general_walks_ && (size_t)(n_inner_ + 1) * per_node * 4 < ((size_t)1 << 31);
 }
 
 void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
@@ -1390,7 +1393,7 @@ void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
     PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices), dim3(kWalkWaves * 64), lds, d, d_fwd_fields_.p, fwd_stride_,
                      d_fwd_sched_.p, n_fwd_steps_, d_ll);
   };
-  if (lean_fits(d.B)) {
+  if (lean_fits(d.B, keep)) {
     const size_t lean_lds = lds + kLeanFlagWords * 4;   // the slots' state words sit behind the slots
     auto launch_lean = [&](auto kernel) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
@@ -1504,7 +1507,7 @@ void HcltCircuit::loglikelihoods(const BatchRef& b, float* d_ll) {
     return;
   }
   // nobody reads a scoring pass's tiles: the lean walk keeps none (heads: the roots' only)
-  const bool lean = lean_fits(b.batch) && !wide_walk_;
+  const bool lean = lean_fits(b.batch, H_ > 0 ? kKeepRoots : kKeepNone) && !wide_walk_;
   stage_batch(b, !lean || H_ > 0);
   if (wide_walk_) return wide_forward(dev(b.batch), d_ll);
   if (H_ > 0) {   // per-head values [H][batch]

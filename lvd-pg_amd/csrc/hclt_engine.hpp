@@ -382,7 +382,7 @@ class HcltCircuit : public pcm_circuit {
   void set_uniform();
   void leaf_vector(bool to_vector, const int32_t* in_pos, float* d_leaf, float* d_vec);
   void fetch_blocks(const float* d_blocks, float* d_leaf, float* theta, float* leaf);
-  bool lean_fits(int batch) const;
+  bool lean_fits(int batch, int keep = kKeepAll) const;
   void run_forward(const HcltDev& d, float* d_ll, int keep = kKeepAll);
   void run_backward(const HcltDev& d);
   void run_stats(const HcltDev& d, float rate);

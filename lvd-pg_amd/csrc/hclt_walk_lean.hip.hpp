@@ -192,7 +192,7 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
   double msum = 0.0;   // sum of the row maxima of this wave's nodes: the part of the log-likelihood the tiles leave out
   Tile<K> o_prev;   // the value tile of the previous step, stored at the top of the next one
   tile_zero<K>(o_prev);
-  int store_prev = d.n_inner * (int)d.tile_stride;
+  int store_prev = (int)((uint32_t)d.n_inner * d.tile_stride);   // (kKeepNone: past 32 bits for all it matters)
   float m_prev = 0.f;
   int mrow_prev = d.n_inner * xrow;
 
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
     lean_w_load<K>(rW, vtile, lean_get(sc, kLW, s + 2), w);   // the block of step s+2, same registers
     o_prev = o;
     const int node = lean_get(sc, kLNode, s);
-    store_prev = node * (int)d.tile_stride;
+    store_prev = (int)((uint32_t)node * d.tile_stride);
     m_prev = m;
     mrow_prev = node * xrow;
     if (node != d.n_inner) msum += (double)m;   // (idle steps work on the trash tile)

@@ -123,6 +123,29 @@ def test_scores_do_not_depend_on_the_batch_size(gpu, K, V):
     assert torch.equal(P.loglikelihoods(a, d, batch_size=4499), want)
 
 
+def test_scoring_a_large_tree_keeps_no_tiles(gpu):
+    """4200 inner nodes at K = 32: the tiles of the 4096 examples that go through together would be more than the lean
+    walk addresses (and twice two gigabytes), but a scoring pass has none."""
+    torch, P = gpu
+    V, K, C, n = 4203, 32, 4, 4500
+    parent = np.maximum(np.arange(V) - 3, 0).astype(np.int32)   # three chains below the root
+    parent[0] = -1
+    a, b = P.hclt_from_clt(parent, C, K), P.hclt_from_clt(parent, C, K)
+    rng = np.random.default_rng(9)
+    theta, leaf = rng.random((V, K, K)).astype(np.float32) + 0.2, rng.random((V, K, C)).astype(np.float32) + 0.2
+    for c in (a, b):
+        c.set_params(np.log(theta / theta.sum(2, keepdims=True)), np.log(leaf / leaf.sum(2, keepdims=True)))
+    assert a.size("walk_kernels") == 1 and a.size("inner_tree_nodes") > 4096
+    d = torch.from_numpy(rng.integers(0, C, size=(n, V)).astype(np.uint8)).cuda()
+    want = torch.cat([P.probs_flows_circuit(b, d[:60].contiguous()), P.probs_flows_circuit(b, d[4060:4120].contiguous())])
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    got = P.loglikelihoods(a, d, batch_size=1000)
+    torch.cuda.synchronize()
+    assert before - torch.cuda.mem_get_info()[0] < 1 << 30
+    assert torch.equal(torch.cat([got[:60], got[4060:4120]]), want)
+
+
 @pytest.mark.parametrize("K,V,C,tree", [(16, 9, 7, None), (32, 700, 256, None), (8, 6, 5, None), (128, 5, 70, None),
                                         (300, 2, 3, None), (16, 9, 5, [-1] + [0] * 8)])
 def test_parameters_come_back_as_they_went_in(gpu, K, V, C, tree):
