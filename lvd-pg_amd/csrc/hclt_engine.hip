@@ -1097,6 +1097,7 @@ void HcltCircuit::set_uniform() {
 // 32 -> 3.3 ms, and 36 -> 3.4 ms the other way, against one thread of the host over the leaf tables).
 void HcltCircuit::set_block_params(const float* theta, const float* leaf) {
   const size_t nt = (size_t)Vu_ * K_ * K_, nl = (size_t)Vu_ * K_ * C_;
+  std::lock_guard<std::mutex> own(param_vec_mu_);
   d_param_vec_.ensure(std::max(theta ? nt : 0, leaf ? nl : 0));
   if (theta) {
     stage().to_device(d_param_vec_.p, theta, nt * sizeof(float), stream);
@@ -1123,6 +1124,7 @@ void HcltCircuit::leaf_vector(bool to_vector, const int32_t* in_pos, float* d_le
 // an engine array of blocks and one of leaf rows as the caller holds them
 void HcltCircuit::fetch_blocks(const float* d_blocks, float* d_leaf, float* theta, float* leaf) {
   const size_t nt = (size_t)Vu_ * K_ * K_, nl = (size_t)Vu_ * K_ * C_;
+  std::lock_guard<std::mutex> own(param_vec_mu_);
   d_param_vec_.ensure(std::max(theta ? nt : 0, leaf ? nl : 0));
   if (theta) {
     hipLaunchKernelGGL(hclt_fill_kernel, dim3((unsigned)ceil_div((int64_t)nt, 256)), dim3(256), 0, stream, d_param_vec_.p, (int64_t)nt, 0.f);
@@ -1242,6 +1244,7 @@ void HcltCircuit::vectorize(float* out, int64_t n) {
                          (long long)size(0));
   if (!out) fail(PCM_ERR_ARG, "parameter vector is null");
   const int64_t ns = (int64_t)sum_param_src_.size();
+  std::lock_guard<std::mutex> own(param_vec_mu_);
   d_param_vec_.ensure((size_t)n);
   if (ns > 0)
     hipLaunchKernelGGL(hclt_params_gather_kernel, dim3((unsigned)ceil_div(ns, 256)), dim3(256), 0, stream, ns,
@@ -1257,6 +1260,7 @@ void HcltCircuit::update_parameters(const float* in, int64_t n) {
                          (long long)size(0));
   if (!in) fail(PCM_ERR_ARG, "parameter vector is null");
   const int64_t ns = (int64_t)sum_param_src_.size();
+  std::lock_guard<std::mutex> own(param_vec_mu_);
   d_param_vec_.ensure((size_t)n);
   stage().to_device(d_param_vec_.p, in, (size_t)n * sizeof(float), stream);
   if (ns > 0)

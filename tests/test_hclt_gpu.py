@@ -190,6 +190,25 @@ def test_parameter_copies_from_several_threads(gpu):
         assert all(pool.map(trip, range(8)))
 
 
+def test_parameters_and_flows_of_one_circuit_from_several_threads(gpu):
+    """Each reader gets what it asked for (the library lets other Python threads run meanwhile)."""
+    torch, P = gpu
+    from concurrent.futures import ThreadPoolExecutor
+    from helpers import correlated_data
+    V, K, C = 90, 32, 256
+    parent = np.array([-1] + [(i - 1) // 2 for i in range(1, V)], np.int32)
+    c = P.hclt_from_clt(parent, C, K)
+    P.update_parameters(c, np.random.default_rng(1).normal(size=c.num_parameters()).astype(np.float32))
+    P.probs_flows_circuit(c, torch.from_numpy(correlated_data(200, V, C, 2, parent)).cuda())
+    reads = (c.get_params, c.get_flows, lambda: (P.vectorize_parameters(c),))
+    want = [r() for r in reads]
+
+    def read(i):
+        return all(np.array_equal(a, b) for a, b in zip(reads[i % 3](), want[i % 3]))
+    with ThreadPoolExecutor(6) as pool:
+        assert all(pool.map(read, range(60)))
+
+
 def test_ragged_batch_and_example_ids(gpu, oracle):
     rng = np.random.default_rng(5)
     idx = rng.permutation(200)[:37].astype(np.int32)
