@@ -1271,6 +1271,7 @@ void HcltCircuit::update_parameters(const float* in, int64_t n) {
   rebuild_w();
   general_stale_ = true;
   leaf_changed();
+  PCM_HIP(hipStreamSynchronize(stream));   // (the caller may go on on another stream)
 }
 
 // ---- batches ------------------------------------------------------------------------

@@ -209,6 +209,32 @@ def test_parameters_and_flows_of_one_circuit_from_several_threads(gpu):
         assert all(pool.map(read, range(60)))
 
 
+def test_new_parameters_are_there_for_any_stream(gpu):
+    """A circuit whose parameters were set on one stream is read and run on another without a wait in between."""
+    torch, P = gpu
+    from helpers import correlated_data
+    V, K, C = 400, 32, 256
+    parent = np.array([-1] + [(i - 1) // 2 for i in range(1, V)], np.int32)
+    c = P.hclt_from_clt(parent, C, K)
+    d = torch.from_numpy(correlated_data(100, V, C, 2, parent)).cuda()
+    one, two = torch.cuda.Stream(), torch.cuda.Stream()
+    rng = np.random.default_rng(1)
+    for _ in range(4):
+        p = rng.normal(size=c.num_parameters()).astype(np.float32)
+        c.set_stream(one.cuda_stream)
+        P.update_parameters(c, p)
+        c.set_stream(two.cuda_stream)
+        assert np.array_equal(P.vectorize_parameters(c), p)
+        c.set_stream(one.cuda_stream)
+        P.update_parameters(c, p)
+        c.set_stream(two.cuda_stream)
+        ll = P.loglikelihoods(c, d)
+        two.synchronize()
+        c.set_stream(0)
+        P.update_parameters(c, p)
+        assert torch.equal(ll, P.loglikelihoods(c, d))
+
+
 def test_ragged_batch_and_example_ids(gpu, oracle):
     rng = np.random.default_rng(5)
     idx = rng.permutation(200)[:37].astype(np.int32)
