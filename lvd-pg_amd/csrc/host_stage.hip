@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <map>
 #include <thread>
 
 #include "common.hpp"
@@ -11,10 +12,12 @@ namespace pcm {
 
 std::shared_ptr<HostStage> HostStage::shared() {
   static std::mutex mu;
-  static std::weak_ptr<HostStage> held;
+  static std::map<int, std::weak_ptr<HostStage>> held;   // by device
+  int dev = 0;
+  PCM_HIP(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lock(mu);
-  std::shared_ptr<HostStage> s = held.lock();
-  if (!s) held = s = std::shared_ptr<HostStage>(new HostStage);
+  std::shared_ptr<HostStage> s = held[dev].lock();
+  if (!s) held[dev] = s = std::shared_ptr<HostStage>(new HostStage);
   return s;
 }
 
@@ -22,17 +25,11 @@ HostStage::~HostStage() {
   for (Lane& l : lanes_) l.give_back();
 }
 
-// (events belong to the device that was current when they were made)
-void HostStage::Lane::make(int dev) {
-  for (int i = 0; i < 2; ++i)
+void HostStage::Lane::make() {
+  for (int i = 0; i < 2; ++i) {
     if (!buf[i]) PCM_HIP(hipHostMalloc((void**)&buf[i], kChunk, hipHostMallocPortable));
-  if (device == dev) return;
-  for (hipEvent_t& e : ev) {
-    if (e) (void)hipEventDestroy(e);
-    e = nullptr;
-    PCM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (!ev[i]) PCM_HIP(hipEventCreateWithFlags(&ev[i], hipEventDisableTiming));
   }
-  device = dev;
 }
 
 void HostStage::Lane::give_back() {
@@ -50,7 +47,7 @@ void HostStage::run(size_t bytes, F&& lane_work) {
   PCM_HIP(hipGetDevice(&dev));
   const int want = (int)std::min<size_t>(kThreads, std::max<size_t>(1, bytes / (4 * kChunk)));
   const int n = std::max(1, std::min(want, (int)std::thread::hardware_concurrency()));
-  for (int i = 0; i < n; ++i) lanes_[i].make(dev);
+  for (int i = 0; i < n; ++i) lanes_[i].make();
   std::atomic<size_t> next{0};
   std::atomic<int> failed{0};
   auto work = [&](int i) {
@@ -82,6 +79,7 @@ void HostStage::to_host(void* dst, const void* d_src, size_t bytes, hipStream_t 
     PCM_HIP(hipStreamSynchronize(stream));
     return;
   }
+  PCM_HIP(hipStreamSynchronize(stream));
   std::lock_guard<std::mutex> lock(mu_);
   run(bytes, [&](Lane& l, std::atomic<size_t>& next) {
     size_t at[2] = {bytes, bytes};
@@ -108,6 +106,7 @@ void HostStage::to_device(void* d_dst, const void* src, size_t bytes, hipStream_
     PCM_HIP(hipStreamSynchronize(stream));
     return;
   }
+  PCM_HIP(hipStreamSynchronize(stream));
   std::lock_guard<std::mutex> lock(mu_);
   run(bytes, [&](Lane& l, std::atomic<size_t>& next) {
     bool used[2] = {false, false};

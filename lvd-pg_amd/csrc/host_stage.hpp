@@ -18,12 +18,12 @@ namespace pcm {
 
 class HostStage {
  public:
-  // The process's stage: made on first use, given back (pinned memory and events) when the last circuit that asked for
-  // it is gone.  At most kThreads x 2 x kChunk bytes of pinned memory.
+  // The current device's stage: made on first use, given back (pinned memory and events) when the last circuit that asked
+  // for it is gone.  At most kThreads x 2 x kChunk bytes of pinned memory.
   static std::shared_ptr<HostStage> shared();
   ~HostStage();
-  // Both return when the whole copy is done.  Ordered behind what `stream` holds.  One transfer at a time: calls from
-  // several threads queue up.
+  // Both return when the whole copy is done.  Ordered behind what `stream` holds, which is waited for first: one transfer at a time goes through the buffers, and calls from several
+  // threads queue up for those that are moving, not for a stream that is still at work.
   void to_host(void* dst, const void* d_src, size_t bytes, hipStream_t stream);
   void to_device(void* d_dst, const void* src, size_t bytes, hipStream_t stream);
 
@@ -34,8 +34,7 @@ class HostStage {
   struct Lane {   // what one thread works with
     char* buf[2] = {nullptr, nullptr};
     hipEvent_t ev[2] = {nullptr, nullptr};
-    int device = -1;
-    void make(int device);
+    void make();
     void give_back();
   };
   HostStage() = default;

@@ -235,6 +235,38 @@ def test_new_parameters_are_there_for_any_stream(gpu):
         assert torch.equal(ll, P.loglikelihoods(c, d))
 
 
+def test_a_busy_stream_holds_up_nobody_elses_parameters(gpu):
+    """Parameters on their way into a circuit whose stream is at work wait for that stream; another circuit's do not."""
+    torch, P = gpu
+    import time
+    from concurrent.futures import ThreadPoolExecutor
+    V, K, C = 90, 32, 256
+    parent = np.array([-1] + [(i - 1) // 2 for i in range(1, V)], np.int32)
+    a, b = P.hclt_from_clt(parent, C, K), P.hclt_from_clt(parent, C, K)
+    va, vb = (np.random.default_rng(s).normal(size=a.num_parameters()).astype(np.float32) for s in (1, 2))
+    side = torch.cuda.Stream()
+    a.set_stream(side.cuda_stream)
+    x = torch.ones((8192, 8192), device="cuda")
+    for c, v in ((a, va), (b, vb)):                          # (buffers, events and the product's library are there)
+        P.update_parameters(c, v)
+    with torch.cuda.stream(side):
+        y = x @ x
+    torch.cuda.synchronize()
+    done = torch.cuda.Event()
+    with ThreadPoolExecutor(1) as pool:
+        with torch.cuda.stream(side):
+            for _ in range(100):                             # (each takes 7 ms and more)
+                torch.mm(x, x, out=y)
+            done.record()
+        waits = pool.submit(P.update_parameters, a, va)
+        time.sleep(0.1)                                      # (the other thread is inside its call)
+        P.update_parameters(b, vb)
+        got = P.vectorize_parameters(b)
+        busy = not done.query()
+        waits.result()
+    assert busy and np.array_equal(got, vb) and np.array_equal(P.vectorize_parameters(a), va)
+
+
 def test_ragged_batch_and_example_ids(gpu, oracle):
     rng = np.random.default_rng(5)
     idx = rng.permutation(200)[:37].astype(np.int32)
