@@ -42,7 +42,7 @@ void HostStage::Lane::give_back() {
 // lane_work(lane, next): takes chunk numbers from `next` until there are none.  Every thread has two chunks under way,
 // so a transfer is worth a thread per four; the caller's thread is one of them.
 template <typename F>
-void HostStage::run(size_t bytes, F&& lane_work) {
+void HostStage::run(size_t bytes, hipStream_t stream, F&& lane_work) {
   int dev = 0;
   PCM_HIP(hipGetDevice(&dev));
   const int want = (int)std::min<size_t>(kThreads, std::max<size_t>(1, bytes / (4 * kChunk)));
@@ -53,7 +53,7 @@ void HostStage::run(size_t bytes, F&& lane_work) {
   auto work = [&](int i) {
     try {
       lane_work(lanes_[i], next);
-    } catch (const Error&) {   // (reported by the caller's thread; the others run out of chunks)
+    } catch (...) {   // (reported by the caller's thread; the others run out of chunks)
       failed = 1;
       next = bytes;
     }
@@ -70,7 +70,10 @@ void HostStage::run(size_t bytes, F&& lane_work) {
   }
   work(0);
   for (std::thread& t : others) t.join();
-  if (failed) fail(PCM_ERR_HIP, "a staged copy of %zu bytes between host and device failed", bytes);
+  if (failed) {
+    (void)hipStreamSynchronize(stream);   // whatever is under way on the buffers or the caller's memory ends before they are free
+    fail(PCM_ERR_HIP, "a staged copy of %zu bytes between host and device failed", bytes);
+  }
 }
 
 void HostStage::to_host(void* dst, const void* d_src, size_t bytes, hipStream_t stream) {
@@ -81,7 +84,7 @@ void HostStage::to_host(void* dst, const void* d_src, size_t bytes, hipStream_t 
   }
   PCM_HIP(hipStreamSynchronize(stream));
   std::lock_guard<std::mutex> lock(mu_);
-  run(bytes, [&](Lane& l, std::atomic<size_t>& next) {
+  run(bytes, stream, [&](Lane& l, std::atomic<size_t>& next) {
     size_t at[2] = {bytes, bytes};
     auto request = [&](int b) {
       at[b] = std::min(bytes, next.fetch_add(1) * kChunk);
@@ -108,7 +111,7 @@ void HostStage::to_device(void* d_dst, const void* src, size_t bytes, hipStream_
   }
   PCM_HIP(hipStreamSynchronize(stream));
   std::lock_guard<std::mutex> lock(mu_);
-  run(bytes, [&](Lane& l, std::atomic<size_t>& next) {
+  run(bytes, stream, [&](Lane& l, std::atomic<size_t>& next) {
     bool used[2] = {false, false};
     for (int b = 0;; b ^= 1) {
       const size_t at = next.fetch_add(1) * kChunk;

@@ -22,7 +22,8 @@ class HostStage {
   // for it is gone.  At most kThreads x 2 x kChunk bytes of pinned memory.
   static std::shared_ptr<HostStage> shared();
   ~HostStage();
-  // Both return when the whole copy is done.  Ordered behind what `stream` holds, which is waited for first: one transfer at a time goes through the buffers, and calls from several
+  // Both return when the whole copy is done, or with an error when none of it is under way any more.  Ordered behind what
+  // `stream` holds, which is waited for first: one transfer at a time goes through the buffers, and calls from several
   // threads queue up for those that are moving, not for a stream that is still at work.
   void to_host(void* dst, const void* d_src, size_t bytes, hipStream_t stream);
   void to_device(void* d_dst, const void* src, size_t bytes, hipStream_t stream);
@@ -39,7 +40,7 @@ class HostStage {
   };
   HostStage() = default;
   template <typename F>
-  void run(size_t bytes, F&& lane_work);
+  void run(size_t bytes, hipStream_t stream, F&& lane_work);
   std::mutex mu_;
   Lane lanes_[kThreads];
 };
