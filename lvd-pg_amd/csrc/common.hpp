@@ -140,8 +140,9 @@ struct pcm_circuit {
   // a sum node's flow down in shares proportional to (posterior share)^(1 / flow_scale); 1: the ordinary flows
   float flow_scale = 1.f;
   std::shared_ptr<pcm::HostStage> host_stage;   // held from the first large transfer on
+  std::once_flag host_stage_made;
   pcm::HostStage& stage() {
-    if (!host_stage) host_stage = pcm::HostStage::shared();
+    std::call_once(host_stage_made, [this] { host_stage = pcm::HostStage::shared(); });
     return *host_stage;
   }
   virtual ~pcm_circuit() {}

@@ -1099,6 +1099,7 @@ void HcltCircuit::set_block_params(const float* theta, const float* leaf) {
   const size_t nt = (size_t)Vu_ * K_ * K_, nl = (size_t)Vu_ * K_ * C_;
   std::lock_guard<std::mutex> own(param_vec_mu_);
   d_param_vec_.ensure(std::max(theta ? nt : 0, leaf ? nl : 0));
+  stage().reserve((nt + nl) * sizeof(float));   // (the whole parameter vector may be asked for in one)
   if (theta) {
     stage().to_device(d_param_vec_.p, theta, nt * sizeof(float), stream);
     take_blocks(d_param_vec_.p);

@@ -39,14 +39,24 @@ void HostStage::Lane::give_back() {
     if (b) (void)hipHostFree(b);
 }
 
-// lane_work(lane, next): takes chunk numbers from `next` until there are none.  Every thread has two chunks under way,
-// so a transfer is worth a thread per four; the caller's thread is one of them.
+// Every thread has two chunks under way, so a transfer is worth a thread per four; the caller's thread is one of them.
+int HostStage::lanes_for(size_t bytes) const {
+  const int want = (int)std::min<size_t>(kThreads, std::max<size_t>(1, bytes / (4 * kChunk)));
+  return std::max(1, std::min(want, (int)std::thread::hardware_concurrency()));
+}
+
+void HostStage::reserve(size_t bytes) {
+  if (bytes < kSmall) return;
+  std::lock_guard<std::mutex> lock(mu_);
+  for (int i = 0; i < lanes_for(bytes); ++i) lanes_[i].make();
+}
+
+// lane_work(lane, next): takes chunk numbers from `next` until there are none.
 template <typename F>
 void HostStage::run(size_t bytes, hipStream_t stream, F&& lane_work) {
   int dev = 0;
   PCM_HIP(hipGetDevice(&dev));
-  const int want = (int)std::min<size_t>(kThreads, std::max<size_t>(1, bytes / (4 * kChunk)));
-  const int n = std::max(1, std::min(want, (int)std::thread::hardware_concurrency()));
+  const int n = lanes_for(bytes);
   for (int i = 0; i < n; ++i) lanes_[i].make();
   std::atomic<size_t> next{0};
   std::atomic<int> failed{0};

@@ -27,6 +27,8 @@ class HostStage {
   // threads queue up for those that are moving, not for a stream that is still at work.
   void to_host(void* dst, const void* d_src, size_t bytes, hipStream_t stream);
   void to_device(void* d_dst, const void* src, size_t bytes, hipStream_t stream);
+  // Makes the buffers for a transfer of this size, so that none is made within it.
+  void reserve(size_t bytes);
 
  private:
   static constexpr int kThreads = 6;
@@ -39,6 +41,7 @@ class HostStage {
     void give_back();
   };
   HostStage() = default;
+  int lanes_for(size_t bytes) const;
   template <typename F>
   void run(size_t bytes, hipStream_t stream, F&& lane_work);
   std::mutex mu_;
