@@ -109,10 +109,10 @@ __global__ __launch_bounds__(256) void sparse_group_w_kernel(GroupDev d, const i
   const_cast<float*>(d.wb)[r.pw0 + group_wb_index(g, c, r.gt)] = w;
 }
 
-// exp(x) * y * 2^bits with a product in float's range, whatever exp(x) alone would be
-__device__ __forceinline__ float group_exp_times(float x, float y, int bits = 0) {
+// exp(x) * y with a product in float's range, whatever exp(x) alone would be
+__device__ __forceinline__ float group_exp_times(float x, float y) {
   const float a = fmaxf(x, -2000.f) * 1.44269504f, n = rintf(a);   // (log2 e; -inf: far enough down)
-  return ldexpf(__builtin_amdgcn_exp2f(a - n) * y, (int)n + bits);
+  return ldexpf(__builtin_amdgcn_exp2f(a - n) * y, (int)n);
 }
 
 __device__ __forceinline__ int guni(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -462,22 +462,20 @@ __global__ __launch_bounds__(WV * 64) void sparse_group_walk_kernel(GroupDev d, 
 // wave stages every fourth child, whose row numbers are the same for its 64 lanes: scalar loads, the rows of eight
 // children requested before the first is used), the GT x CT tiles of the result dealt out over its four waves.
 // R E is share / W and is added up over the examples before W comes in, so the product only takes pairs (sum, example)
-// with m - value up to kEdgeShare.  In it E is kept 2^kEdgeBits up and R as much down, exactly: E then reaches down to
-// X - m = -109 and R to flow / S = e^-65, so a pair of a flow of 1 whose share falls out has one below e^-64.  The edges
-// of a sum that has pairs above kEdgeShare, and those that come out below kLowFlow (64 such pairs are 1e-5 of it) though
-// neither their sum is without flow nor their child impossible all over nor W zero, are added up again in logarithms,
-// example by example: X and log R in the same LDS, every exponent then that of a share.
-// 192 variables, 128 heads, K = 32, batches of 512: 12 us for the bodies' groups and 23 for the heads' with parameters as
-// training starts from, 19 and 37 after 20 epochs (all 64 examples of an edge instead of those with flow: 19 and 48).
-// With 30 or 60 as the limit, 21 or 43 bits and 1e-24 or 1e-18 for kLowFlow: 2 and 3 us more for the bodies' groups.
-constexpr float kEdgeShare = 45.f, kLowFlow = 1e-21f;
-constexpr int kEdgeBits = 32;
+// with m - value up to kEdgeShare; E is kept 2^kEdgeUp (e^kEdgeShare) up, so that it reaches down to X - m = -125 and no
+// share falls out for it, and R 2^kEdgeDown down, so that 64 pairs stay in range for flows of up to 1e9; what falls out for
+// that are flows of less than e^-73.  The other pairs, and for an edge with a W below float's range (kept as -0) all of
+// them, are added in logarithms, example by example: X and log R in the same LDS, every exponent then that of a share.
+// 192 variables, 128 heads, K = 32, batches of 512: 11 us for the bodies' groups and 20 for the heads' with parameters as
+// training starts from, 15 and 20 after 20 epochs (30 as the limit: 19 and 20; whole sums added up again instead of their
+// pairs above the limit: 18 and 21).
+constexpr float kEdgeShare = 38.f;
+constexpr int kEdgeUp = 55, kEdgeDown = 20;
 
 template <int GT, int CT>
 __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int first) {
   extern __shared__ float glds[];
-  __shared__ uint64_t row_some[GT * 16];                     // of a sum: the examples with flow
-  __shared__ int row_high[GT * 16], child_some[CT * 16];     // ... any pair above kEdgeShare; of a child: any example it is possible in
+  __shared__ uint64_t row_some[GT * 16], row_high[GT * 16];   // of a sum: the examples with flow, those above kEdgeShare
   __shared__ int any_again;
   const int group = d.order[first + blockIdx.x];
   const GroupRec r = d.rec[group];
@@ -526,22 +524,20 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
   };
   if (t == 0) any_again = 0;
   stage([&](int c, float x) {
-          E[c * kGroupPad + b] = group_exp_times(x, 1.f, kEdgeBits);
-          const bool some = __any(x > -INFINITY);
-          if (b == 0) child_some[c] = some;
+          const bool far = x < -64.f;   // (where exp(x) alone would run out of float's range on its way up)
+          E[c * kGroupPad + b] = __expf(far ? x + kEdgeUp * 0.69314718f : x) * (far ? 1.f : __builtin_ldexpf(1.f, kEdgeUp));
         },
         [&](int g, float f, float tq) {
           const bool high = f > 0.f && tq > kEdgeShare;
-          R[g * kGroupPad + b] = f > 0.f && !high ? group_exp_times(tq, f, -kEdgeBits) : 0.f;
-          const uint64_t some = __ballot(f > 0.f);
-          const bool row = __any(high);
+          R[g * kGroupPad + b] = f > 0.f && !high ? f * __expf(tq) * __builtin_ldexpf(1.f, -kEdgeDown) : 0.f;
+          const uint64_t some = __ballot(f > 0.f), above = __ballot(high);
           if (b == 0) {
             row_some[g] = some;
-            row_high[g] = row;
+            row_high[g] = above;
           }
         });
   __syncthreads();
-  uint64_t again = 0;   // a bit per (tile of the wave, i): edges to be added up in logarithms
+  uint64_t again = 0;   // a bit per (tile of the wave, i): edges with something to be added in logarithms
   int nth = 0;
   for (int tile = wave; tile < GT * CT; tile += 4, ++nth) {
     const int gt = tile / CT, ct = tile % CT;
@@ -556,10 +552,9 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
       const int g = gt * 16 + 4 * hi + i;
       const int edge = g < r.G && c < r.C ? d.edge[r.pw0 + g * Cp + c] : -1;
       if (edge < 0) continue;   // (in a masked group also a child the sum does not have)
-      const float w = d.wf[r.pw0 + group_wf_index(g, c, CT)], flow = w * acc[i];
-      const bool there = row_some[g] && child_some[c] && (w > 0.f || group_tiny_w(w));
-      if (there && (row_high[g] || flow < kLowFlow)) again |= (uint64_t)1 << (4 * nth + i);
-      else part_row[edge] = flow;
+      const float w = d.wf[r.pw0 + group_wf_index(g, c, CT)];
+      part_row[edge] = w * acc[i] * __builtin_ldexpf(1.f, kEdgeDown - kEdgeUp);
+      if (group_tiny_w(w) ? row_some[g] : row_high[g]) again |= (uint64_t)1 << (4 * nth + i);
     }
   }
   if (again) any_again = 1;
@@ -583,19 +578,24 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
     const float* Rg = R + (gt * 16 + 4 * hi) * kGroupPad;
     int edge[4];
     float lw[4], flow[4];
+    uint64_t own[4], examples = 0;   // the examples of each edge, and of any of the tile's
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      edge[i] = mine >> i & 1 ? d.edge[r.pw0 + (gt * 16 + 4 * hi + i) * Cp + c] : -1;
-      lw[i] = edge[i] >= 0 ? d.logp[edge[i]] * d.inv_f : -INFINITY;
+      const int g = gt * 16 + 4 * hi + i;
+      edge[i] = mine >> i & 1 ? d.edge[r.pw0 + g * Cp + c] : -1;
+      lw[i] = edge[i] >= 0 ? d.logp[edge[i]] * d.inv_f : 0.f;
+      own[i] = edge[i] < 0 ? 0 : group_tiny_w(group_w(lw[i])) ? row_some[g] : row_high[g];
       flow[i] = 0.f;
+      examples |= own[i];
     }
-    // the examples any of the tile's sums has flow in, four at a time
-    uint32_t left[2] = {0u, 0u};
-    for (int g = 0; g < 16; ++g) {
-      left[0] |= (uint32_t)row_some[gt * 16 + g];
-      left[1] |= (uint32_t)(row_some[gt * 16 + g] >> 32);
+    uint32_t half[2] = {(uint32_t)examples, (uint32_t)(examples >> 32)};
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      half[0] |= (uint32_t)__shfl_xor((int)half[0], o);
+      half[1] |= (uint32_t)__shfl_xor((int)half[1], o);
     }
-    uint64_t examples = (uint64_t)(uint32_t)guni((int)left[1]) << 32 | (uint32_t)guni((int)left[0]);
+    examples = (uint64_t)(uint32_t)guni((int)half[1]) << 32 | (uint32_t)guni((int)half[0]);
+    // four at a time
     while (examples) {
       int x[4];
 #pragma unroll
@@ -607,12 +607,15 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
       for (int u = 0; u < 4; ++u) {
         const float e = Ec[x[u]];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) flow[i] += __expf(e + Rg[i * kGroupPad + x[u]] + lw[i]);
+        for (int i = 0; i < 4; ++i) {
+          const float share = __expf(e + Rg[i * kGroupPad + x[u]] + lw[i]);
+          flow[i] += own[i] >> (x[u] & 63) & 1 ? share : 0.f;
+        }
       }
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (edge[i] >= 0) part_row[edge[i]] = flow[i];
+      if (edge[i] >= 0) part_row[edge[i]] += flow[i];
   }
 }
 

@@ -870,12 +870,14 @@ def test_a_sum_that_hangs_on_one_small_parameter(gpu, oracle, gaps, logw):
     assert grouped.size("dense_groups") == 2                 # the masked one and the heads'
 
 
-@pytest.mark.parametrize("logw", [-61.0, -80.0, -84.0, -86.0, -87.2, -88.0, -100.0])
+@pytest.mark.parametrize("logw", [-20.0, -37.5, -39.0, -61.0, -80.0, -84.0, -86.0, -87.2, -88.0, -100.0])
 def test_all_flow_through_one_small_parameter(gpu, oracle, logw):
     """The child at the block's maximum, all 64 examples of a block and their whole flow behind one edge: flow / W is
     as far up as it goes."""
     heads = _sums_beside_full_ones(oracle, (0,), (logw,), taken=-logw + 30.0)
     _check_grouped_multihead(gpu, oracle, heads, 3, 2, 128, 84, min_groups=2)
+    for scale in (1e3, 1e7):                                 # (weights of examples)
+        _check_small_shares(gpu, oracle, heads, 3, 2, 128, scale=scale)
 
 
 def _check_small_shares(gpu, O, heads, V, C, B, scale=1.0, edges=True):
