@@ -88,11 +88,11 @@ __host__ __device__ inline int64_t group_wb_index(int g, int c, int gt) {   // g
 }
 
 // W below float's normal range is kept as -0: nothing to a product, and the mark by which sums that may hang on such an
-// edge (see kLowSum) find it and take its logarithm.
+// edge (see kLowSum) find it and take its logarithm.  NaN stays NaN for the way up; going down, a sum it made NaN has no flow.
 __device__ __forceinline__ bool group_tiny_w(float w) { return __builtin_bit_cast(uint32_t, w) == 0x80000000u; }
 __device__ __forceinline__ float group_w(float lw) {
   const float w = __expf(lw);
-  return w >= __FLT_MIN__ ? w : lw > -INFINITY ? -0.f : 0.f;
+  return w >= __FLT_MIN__ ? w : lw > -INFINITY ? -0.f : lw == lw ? 0.f : lw;
 }
 
 // exp of the groups' log-parameters in both orders, once per pass (the parameters may have moved): thread = (group,
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256) void sparse_group_w_kernel(GroupDev d, const i
   const int e = d.edge[i];
   const float w = e >= 0 ? group_w(d.logp[e] * d.inv_f) : 0.f;
   const_cast<float*>(d.wf)[r.pw0 + group_wf_index(g, c, r.ct)] = w;
-  const_cast<float*>(d.wb)[r.pw0 + group_wb_index(g, c, r.gt)] = w;
+  const_cast<float*>(d.wb)[r.pw0 + group_wb_index(g, c, r.gt)] = w == w ? w : 0.f;
 }
 
 // exp(x) * y with a product in float's range, whatever exp(x) alone would be
@@ -144,7 +144,8 @@ __device__ __forceinline__ float group_max4(float v) {
 // W E >= 5.8e-30 shows any of them that the sum has.  So when E is cut off at exp(kMaxRaise), for children far above, no sum
 // that is still looked for has one of those, and every step takes in a child more, so the loop ends.
 // Only such sums can hang on a parameter below float's range; where a block has one (group_tiny_w) they are added up in
-// logarithms, edge by edge.  Going down, so are the shares of all sums with m - value > kHighShare.
+// logarithms, edge by edge.  So are sums that come out NaN: of the children's NaNs only those of a sum's own make it NaN.
+// Going down, the shares of all sums with m - value > kHighShare are added in logarithms.
 constexpr float kLowSum = 1e-30f, kHighShare = 60.f, kTurn = 40.f, kMaxRaise = 88.f;
 
 template <int NK>
@@ -156,7 +157,7 @@ __device__ __forceinline__ void group_low_sums(const GroupDev& d, const float* x
   for (int q = 0; q < NK; ++q) {
     xs[q] = xm[(int64_t)(4 * q + hi) * d.Bp];   // (what this lane has just written)
     a[q] = w[q * 64];
-    tiny |= group_tiny_w(a[q]);
+    tiny |= group_tiny_w(a[q]) || !(a[q] == a[q]) || !(xs[q] == xs[q]);
   }
   if (__any(tiny)) {   // edge: the tile's rows of d.edge, [16][4 NK]
     __threadfence_block();   // (X - m of the children that the other lanes of the example hold)
@@ -250,7 +251,7 @@ __device__ __forceinline__ void group_forward_body(const GroupDev& d, const Grou
     if (own[q] >= 0) d.mars[(int64_t)own[q] * d.Bp + col] = pv[q];
     const float xs = x[q] - mx;   // (-inf stays -inf)
     xm[(int64_t)(4 * q + hi) * d.Bp] = xs;
-    x[q] = x[q] > -INFINITY ? __expf(xs) : 0.f;
+    x[q] = __expf(xs);
   }
   if (hi == 0) d.m[(int64_t)group * d.Bp + col] = mx;
 #pragma unroll
@@ -269,7 +270,7 @@ __device__ __forceinline__ void group_forward_body(const GroupDev& d, const Grou
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       val[i] = mx + __logf(acc[i]);
-      low[i] = nd[i] >= 0 && acc[i] < kLowSum;
+      low[i] = nd[i] >= 0 && !(acc[i] >= kLowSum);
     }
     if (__any(low[0] | low[1] | low[2] | low[3]))
       group_low_sums<NK>(d, xm, hi, wg + gt * NK * 64, d.edge + base.pw0 + ((int64_t)bx * Gp + gt * 16) * Cp, mx, low, val);
@@ -317,7 +318,8 @@ __device__ __forceinline__ void group_shares_by_edge(const GroupDev& d, const in
       const int ed[4] = {e4.x, e4.y, e4.z, e4.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float lw = ed[i] >= 0 ? d.logp[ed[i]] * d.inv_f : -INFINITY;
+        if (ed[i] < 0) continue;
+        const float lw = d.logp[ed[i]] * d.inv_f;
         if (f[g] > 0.f && (t[g] > kHighShare || group_tiny_w(group_w(lw)))) out[i] += f[g] * __expf(e[i] * d.inv_f + lw + t[g]);
       }
     }
@@ -553,7 +555,7 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
       const int edge = g < r.G && c < r.C ? d.edge[r.pw0 + g * Cp + c] : -1;
       if (edge < 0) continue;   // (in a masked group also a child the sum does not have)
       const float w = d.wf[r.pw0 + group_wf_index(g, c, CT)];
-      part_row[edge] = w * acc[i] * __builtin_ldexpf(1.f, kEdgeDown - kEdgeUp);
+      part_row[edge] = w > 0.f ? w * acc[i] * __builtin_ldexpf(1.f, kEdgeDown - kEdgeUp) : 0.f;
       if (group_tiny_w(w) ? row_some[g] : row_high[g]) again |= (uint64_t)1 << (4 * nth + i);
     }
   }

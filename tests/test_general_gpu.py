@@ -933,6 +933,30 @@ def test_edge_flows_of_small_shares(gpu, oracle, gaps, logw, taken, scale):
     _check_small_shares(gpu, oracle, heads, 3, 2, 70, scale=scale)
 
 
+@pytest.mark.parametrize("keep", [1.0, 0.6])
+@pytest.mark.parametrize("where", ["parameter", "head", "leaf"])
+def test_nans_reach_the_sums_they_belong_to(gpu, oracle, keep, where):
+    """A NaN among a sum's own parameters or children makes its value NaN, in groups as on the layer kernels; sums that do
+    not have it keep theirs, and sums that are NaN hand no flow on."""
+    torch, P = gpu
+    rng = np.random.default_rng(95)
+    heads = _masked_multihead(oracle, rng, 2, 20, 24, 4, keep, 1.0, 5)
+    d = torch.from_numpy(rng.integers(0, 5, size=(70, 4)).astype(np.uint8)).cuda()
+    hm = torch.from_numpy(rng.random((70, 4)).astype(np.float32) + 0.05).cuda()
+    got = []
+    for c in _with_and_without_groups(P, heads, 4, 5):
+        p = P.vectorize_parameters(c)
+        p[c.num_inner_params() + {"parameter": 11 - c.num_inner_params(), "head": -1, "leaf": 7}[where]] = np.nan
+        P.update_parameters(c, p)
+        ll = P.probs_flows_circuit(c, d, head_mask=hm).cpu().numpy()
+        got.append((ll, *c.get_node_values(70), *c.get_aggregates()))
+    assert np.isnan(got[1][1]).any() and not np.isnan(got[1][1]).all()
+    for a, b in zip(*got):
+        assert np.array_equal(np.isnan(a), np.isnan(b))
+        ok = ~np.isnan(b) & np.isfinite(b)
+        assert np.array_equal(np.isfinite(a), np.isfinite(b)) and np.abs(a[ok] - b[ok]).max(initial=0.0) < FLOW_RTOL * np.abs(b[ok]).max(initial=1.0)
+
+
 @pytest.mark.parametrize("fscale", [0.5, 2.5])
 def test_tempered_flows_of_masked_groups(gpu, oracle, fscale):
     """Tempered flows of masked groups against the layer kernels', sharp leaves included."""
