@@ -357,8 +357,9 @@ void mi_launch(const uint8_t* d_data, int64_t stride_ex, int64_t stride_var, con
   const int per_cu = std::max<int>(1, (int)(std::min<size_t>((size_t)max_lds, 160 * 1024) / lds));
   const int grid = (int)std::min<int64_t>(n_pairs, (int64_t)cus * std::min(per_cu, 4));
   if (narrow) {
-    // clearing the whole table costs what wiping after this many examples costs (measured at C = 256: equal at 16000
-    // examples, 38.9 against 32.5 ms at 8192, 86.8 against 103.5 at 32768; smaller tables favour the sweep a little more)
+    // clearing the whole table costs what wiping after about this many examples costs: at 64 / 100 / 128 / 256 categories
+    // the line is at 790 / 1900 / 3100 / 12400, the two were equal at 500 / 2100 / 4100 / 15500 (700 variables; 256: 1.79 ms
+    // wiped, 2.16 swept at 8192, 5.52 and 4.65 at 32768)
     const int sweep = (int64_t)N * 8 > (int64_t)C * mi_row_words(C) * 3 ? 1 : 0;
     const bool small = per_cu > 1;
     auto pairs = [&](auto kernel, int threads) {

@@ -1231,8 +1231,10 @@ __global__ __launch_bounds__(256) void sparse_product_edge_kernel(const int2* __
 // its products -- over the union of their children, W zero where a sum lacks a child; in reach of each other through
 // shared children, a layer at a time.  A block costs the same however thin it is (and a layer that is all blocks joins
 // the walks), an edge at a time the layer kernels cost little less for few edges: 192 variables, 128 heads, 16 batches of
-// 512, K = 32: 6.45 ms as blocks at any share of the pairs, edge by edge 9.9 at 60 %, 8.2 at 30 %, 8.0 at 15 %, 7.8 at 10
-// and 5 % (4 batches of 4096: 3.6 against 5.0 at 30 %, 4.4 at 10 %; K = 16, 512: 4.05 against 7.2 at 60 %, 7.0 at 30 %).
+// 512, K = 32: 6.0 ms as blocks at any share of the pairs from 10 % on, edge by edge 8.3 at 60 %, 7.8 at 30 %, 7.6 at 15 %, 7.5
+// at 10 % (4 batches of 4096: 3.2 against 5.4 at 60 %, 4.7 at 30 %, 4.0 at 10 %; K = 16, 512: 3.9 against 7.0 at 60 %, 6.8 at
+// 10 %).  With trained parameters, whose sums lie further apart: 6.1 against 8.3 after 20 epochs, 7.3 with leaves 60 nats
+// apart; where nearly every block has parameters below exp's range 10.3 against 8.1 (not known when the blocks are chosen).
 // So the line is only one pair in kMaskedShare, two children of 32: sums that merely touch stay apart.
 // PCMI355_DENSE_GROUPS=0 in the environment keeps every node on the layer kernels (for comparisons).
 constexpr int kGroupMinSide = 4, kGroupMinEdges = 64, kGroupMaxSide = 128, kMaskedShare = 16;
