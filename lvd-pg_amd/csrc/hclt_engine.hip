@@ -12,6 +12,7 @@
 #include "hclt_walk_lean.hip.hpp"
 #include "hclt_soft_sample.hip.hpp"
 #include "hclt_heads.hip.hpp"
+#include "lean_schedule.hpp"
 #include "lean_schedule_check.hpp"
 #include "hclt_soft_evidence.hip.hpp"
 
@@ -235,15 +236,13 @@ void HcltCircuit::build_schedules() {
   const int trash_slot = lds_slots_ - 1;          // idle waves and childless nodes write here
 
   std::vector<std::vector<int32_t>> ic(n_inner_), lc(n_inner_);
-  std::vector<int32_t> par(n_inner_, -1), hin(n_inner_, 0);   // hin: longest chain of inner nodes below
-  std::vector<int32_t> below(n_inner_, 0);                    // inner nodes below (children come first in post-order)
-  const bool lean_k = K_ <= 32;                               // hidden sizes with lean walk kernels
+  std::vector<int32_t> par(n_inner_, -1);
   for (int n = 0; n < n_inner_; ++n) {
     const int v = var_of_inner_[n];
     if (parent_[v] >= 0) par[n] = inner_of_var_[parent_[v]];
     for (int c : children_[v]) {
       if (children_[c].empty()) lc[n].push_back(c);
-      else { ic[n].push_back(inner_of_var_[c]); hin[n] = std::max(hin[n], hin[inner_of_var_[c]] + 1); below[n] += 1 + below[inner_of_var_[c]]; }
+      else ic[n].push_back(inner_of_var_[c]);
     }
   }
   std::vector<uint32_t> ext;
@@ -303,87 +302,70 @@ void HcltCircuit::build_schedules() {
       }
     dst.upload(f);
   };
-  // lean schedule rows (see hclt_walk_lean.hip.hpp) from the padded items of a walk, or none
-  // if some node has more operands than the lean kernels hold
+  LeanTree lt;
+  lt.parent = par;
+  lt.inner = ic;
+  lt.tree = tree_of_inner_;
+  for (int n = 0; n < n_inner_; ++n) lt.depth.push_back(depth_[var_of_inner_[n]]);
+  lt.complete();
+  // field rows of the lean walks (see hclt_walk_lean.hip.hpp) from their own schedule, with the same padding, or none if
+  // some node has more operands than the lean kernels hold
   const size_t leaf_stride = (size_t)C_ * K_ * sizeof(float);
-  // (backward: ratio_slot[n] is the LDS slot in which node n finds its ratio tile, left there by its parent)
-  auto make_lean = [&](const std::vector<StepItem>& sched, bool forward, int stride, std::vector<int32_t>& dst,
-                       const std::vector<int32_t>* ratio_slot = nullptr) -> bool {
-    if (K_ > 32 || lds_slots_ > 255 || (size_t)V_ * leaf_stride >= ((size_t)1 << 31)) return false;
+  auto make_lean = [&](const LeanSchedule& sched, bool forward, int stride, std::vector<int32_t>& dst) -> bool {
+    if (!sched.ok || K_ > 32 || lds_slots_ >= (int)kLeanKept || (size_t)V_ * leaf_stride >= ((size_t)1 << 31)) return false;
     const size_t f0 = dst.size();   // (the rows of a further group of trees go behind those of the groups before)
     dst.resize(f0 + (size_t)kLeanFields * kWalkWaves * stride, 0);
     int32_t* f = dst.data() + f0;
+    auto at = [&](int field, int w, int st) -> int32_t& { return f[((size_t)field * kWalkWaves + w) * stride + st]; };
+    auto item = [&](int st, int w) { return st < sched.steps ? sched.item[(size_t)st * kWalkWaves + w] : -1; };
     // how often each slot has been filled so far: a step's reads see the fills of earlier steps only, so the
     // readers of a step are numbered before its writers
     std::vector<int32_t> fills(256, 0);
-    for (int s = 0; s < stride; ++s) {
+    for (int st = 0; st < sched.steps; ++st)
       for (int pass = 0; pass < 2; ++pass)
         for (int w = 0; w < kWalkWaves; ++w) {
-          const StepItem& it = sched[(size_t)s * kWalkWaves + w];
-          if (it.node < 0) continue;
-          int32_t& turns = f[((size_t)kLTurns * kWalkWaves + w) * stride + s];
-          if (!forward) {   // a node reads the slot its parent filled and fills one per inner child
-            const int n = it.node;
-            if (pass == 0) {
-              if (par[n] >= 0) turns |= (fills[(*ratio_slot)[n]] - 1) & 0x7f;
-            } else {
-              int q = 0;
-              for (int c : ic[n]) turns |= (fills[(*ratio_slot)[c]]++ & 0x7f) << (8 * ++q);
-            }
-            continue;
-          }
-          if (pass == 0) {
-            for (int c = 0; c < it.n_l; ++c) {
-              const int sl = (int)(it.l[c] >> kSlotShift) - 1;
-              if (sl >= 0) turns |= ((fills[sl] - 1) & 0x7f) << (8 * (c + 1));
-            }
-          } else if (it.out_slot != trash_slot) {
-            turns |= fills[it.out_slot]++ & 0x7f;
-          }
+          const int n = item(st, w);
+          if (n < 0) continue;
+          int32_t& turns = at(kLTurns, w, st);
+          auto turn = [&](int tile, int byte) {
+            const int sl = sched.slot[tile];
+            if (sl < kLeanSlotKept) turns |= ((pass == 0 ? fills[sl] - 1 : fills[sl]++) & 0x7f) << (8 * byte);
+          };
+          if (lt.inner[n].size() > 3) return false;
+          if ((pass == 0) == forward)   // the children's tiles are bytes 1 .. 3, the node's own is byte 0
+            for (size_t i = 0; i < lt.inner[n].size(); ++i) turn(lt.inner[n][i], 1 + (int)i);
+          else
+            turn(n, 0);
         }
-    }
-    for (int s = 0; s < stride; ++s)
+    for (int st = 0; st < stride; ++st)
       for (int w = 0; w < kWalkWaves; ++w) {
-        const StepItem& it = sched[(size_t)s * kWalkWaves + w];
-        auto put = [&](int field, int32_t v) { f[((size_t)field * kWalkWaves + w) * stride + s] = v; };
-        const int n = it.node;
-        put(kLA1, -1); put(kLA2, -1); put(kLA3, -1);
-        if (n < 0) {   // idle: trash tile, trash slot, block and leaf rows of node / variable 0
-          put(kLNode, n_inner_);
-          put(kLSlots, (int32_t)(0xffffff00u | (uint32_t)trash_slot));
-          continue;
+        const int n = item(st, w);
+        at(kLA1, w, st) = at(kLA2, w, st) = at(kLA3, w, st) = -1;
+        at(kLW, w, st) = -1;
+        at(kLSlots, w, st) = -1;
+        at(kLNode, w, st) = n < 0 ? n_inner_ : n;
+        if (n < 0) continue;   // idle: leaf rows of variable 0
+        if (lt.inner[n].size() + (forward ? 0 : lc[n].size()) > 3 || lc[n].size() > 3) return false;
+        if (forward || !lt.inner[n].empty()) at(kLW, w, st) = (int32_t)((size_t)n * K_ * K_ * sizeof(float));
+        at(kLA0, w, st) = (int32_t)((size_t)var_of_inner_[n] * leaf_stride);
+        at(kLFlags, w, st) = par[n] < 0 ? (H_ > 0 ? 3 : 1) : 0;
+        uint32_t slots = 0xffffff00u | (uint32_t)sched.slot[n];
+        int q = 0;
+        for (int c : lt.inner[n]) {
+          slots = (slots & ~(0xffu << (8 * (q + 1)))) | ((uint32_t)sched.slot[c] << (8 * (q + 1)));
+          if (!forward) at(kLA1 + q, w, st) = c << 3;
+          ++q;
         }
-        put(kLW, (int32_t)((size_t)n * K_ * K_ * sizeof(float)));
-        put(kLA0, (int32_t)((size_t)var_of_inner_[n] * leaf_stride));
-        put(kLNode, n);
-        put(kLFlags, par[n] < 0 ? (H_ > 0 ? 3 : 1) : 0);
-        if (forward) {
-          if (lc[n].size() > 3 || ic[n].size() > 3) return false;
-          for (size_t i = 0; i < lc[n].size(); ++i) put(kLA1 + (int)i, (int32_t)((size_t)lc[n][i] * leaf_stride));
-          uint32_t slots = (uint32_t)it.out_slot | 0xffffff00u;
-          for (int c = 0; c < it.n_l; ++c) {
-            const int sl = (int)(it.l[c] >> kSlotShift) - 1;
-            if (sl < 0) return false;
-            slots = (slots & ~(0xffu << (8 * (c + 1)))) | ((uint32_t)sl << (8 * (c + 1)));
-          }
-          put(kLSlots, (int32_t)slots);
-        } else {
-          if (lc[n].size() + ic[n].size() > 3) return false;
-          int q = 0;
-          uint32_t slots = (uint32_t)(par[n] < 0 ? trash_slot : (*ratio_slot)[n]) | 0xffffff00u;
-          for (int c : ic[n]) {
-            slots = (slots & ~(0xffu << (8 * (q + 1)))) | ((uint32_t)(*ratio_slot)[c] << (8 * (q + 1)));
-            put(kLA1 + q++, c << 3);
-          }
-          for (size_t i = 0; i < lc[n].size(); ++i)
-            put(kLA1 + q++, (int32_t)((size_t)lc[n][i] * leaf_stride) | 1 | (int32_t)((i + 1) << 1));
-          put(kLSlots, (int32_t)slots);
-        }
+        at(kLSlots, w, st) = (int32_t)slots;
+        if (forward) q = 0;
+        for (size_t i = 0; i < lc[n].size(); ++i)
+          at(kLA1 + q++, w, st) = (int32_t)((size_t)lc[n][i] * leaf_stride) | (forward ? 0 : 1 | (int32_t)((i + 1) << 1));
       }
     // the waits and posts of all waves, replayed: a schedule on which a wave would wait for ever is refused here
     static_assert(kLeanCheckA1 == kLA1 && kLeanCheckSlots == kLSlots && kLeanCheckTurns == kLTurns &&
-                  kLeanCheckFields == kLeanFields && kLeanCheckWaves == kWalkWaves, "lean_schedule_check.hpp follows the lean field rows");
-    const int stuck = lean_schedule_stuck_at(f, stride, stride, forward, trash_slot);
+                  kLeanCheckFields == kLeanFields && kLeanCheckWaves == kWalkWaves && kLeanCheckKept == kLeanKept &&
+                  kLeanSlotKept == kLeanKept && kLeanSchedWaves == kWalkWaves, "the lean schedule's headers follow the field rows");
+    const int stuck = lean_schedule_stuck_at(f, stride, stride, forward, kLeanSlotNone);
     if (stuck >= 0)
       fail(PCM_ERR_STATE, "%s walk schedule is unsound: wave %d would wait for ever in step %d", forward ? "forward" : "backward",
            stuck % kWalkWaves, stuck / kWalkWaves);
@@ -408,28 +390,18 @@ void HcltCircuit::build_schedules() {
     }
     return gr;
   };
-  const std::vector<std::pair<int, int>> groups = make_groups(forest_ ? std::max(1, std::min(4, T_ / 8)) : 1);
-  n_groups_ = (int)groups.size();
 
-  // ---- forward -----------------------------------------------------------------------
-  auto schedule_forward = [&](int g0, int g1, std::vector<StepItem>& sched, std::vector<PreItem>& pre, bool reserve) {
+  // (the general walk kernels' schedules: a step's nodes are put behind a barrier, every tile takes a slot)
+  auto schedule_forward = [&](std::vector<StepItem>& sched, std::vector<PreItem>& pre) {
     std::vector<int32_t> pending(n_inner_), slot(n_inner_, -1), free_slots;
     for (int s = trash_slot - 1; s >= 0; --s) free_slots.push_back(s);
-    // max-heap: deeper first, then lower id (post-order).  In a forest the earlier tree goes first whatever the
-    // depth: the trees then pass through the waves one behind the other, a few at a time, and the tiles that wait
-    // for a parent in LDS are those of a few trees instead of all.
-    auto cmp = [&](int a, int b) {
-      if (tree_of_inner_[a] != tree_of_inner_[b]) return tree_of_inner_[a] > tree_of_inner_[b];
-      return depth_of(a) != depth_of(b) ? depth_of(a) < depth_of(b) : a > b;
-    };
-    // with `reserve` (always in a forest) a node without inner children, which fills a slot and frees none, only
-    // starts while more than a step's worth of slots is free (or nothing else can run)
-    const int producer_reserve = kWalkWaves;
+    // max-heap: deeper first, then lower id (post-order)
+    auto cmp = [&](int a, int b) { return depth_of(a) != depth_of(b) ? depth_of(a) < depth_of(b) : a > b; };
     std::vector<int32_t> ready;
-    for (int n = g0; n < g1; ++n) { pending[n] = (int)ic[n].size(); if (!pending[n]) ready.push_back(n); }
+    for (int n = 0; n < n_inner_; ++n) { pending[n] = (int)ic[n].size(); if (!pending[n]) ready.push_back(n); }
     std::make_heap(ready.begin(), ready.end(), cmp);
     int done = 0;
-    while (done < g1 - g0) {
+    while (done < n_inner_) {
       // nodes whose flow tile needs an LDS slot wait while none is free (their turn comes
       // when children of earlier nodes have drained); only if nothing else is ready does a
       // tile go through HBM instead
@@ -439,23 +411,13 @@ void HcltCircuit::build_schedules() {
         std::pop_heap(ready.begin(), ready.end(), cmp);
         const int n = ready.back();
         ready.pop_back();
-        if (reserve) {
-          if (par[n] >= 0) {
-            if (slots_left <= (ic[n].empty() ? producer_reserve : 0)) { deferred.push_back(n); continue; }
-            --slots_left;
-          }
-        } else if (!ic[n].empty()) {
+        if (!ic[n].empty()) {
           if (slots_left == 0) { deferred.push_back(n); continue; }
           --slots_left;
         }
         step.push_back(n);
       }
-      if (step.empty() && !deferred.empty()) {
-        // nothing fits: the first of the waiting nodes in heap order / without a reserve the last one goes anyway
-        const size_t pick = reserve ? 0 : deferred.size() - 1;
-        step.push_back(deferred[pick]);
-        deferred.erase(deferred.begin() + (std::ptrdiff_t)pick);
-      }
+      if (step.empty() && !deferred.empty()) { step.push_back(deferred.back()); deferred.pop_back(); }
       for (int n : deferred) { ready.push_back(n); std::push_heap(ready.begin(), ready.end(), cmp); }
       if (step.empty()) fail(PCM_ERR_SHAPE, "forward schedule stalled (tree is inconsistent)");
       for (int w = 0; w < kWalkWaves; ++w) {
@@ -492,112 +454,36 @@ void HcltCircuit::build_schedules() {
       }
     }
   };
-  // The lean backward walk hands every inner child its own tile: a slot per (parent, inner child) pair, taken
-  // in the parent's step and free again from the step after the child's.  False if the slots run out.
-  auto assign_ratio_slots = [&](const std::vector<StepItem>& sched, std::vector<int32_t>& ratio_slot) {
-    const int g_steps = (int)sched.size() / kWalkWaves;
-    std::vector<int32_t> fs;
-    for (int sl = trash_slot - 1; sl >= 0; --sl) fs.push_back(sl);
-    for (int st = 0; st < g_steps; ++st) {
-      std::vector<int32_t> freed;
-      for (int w = 0; w < kWalkWaves; ++w) {
-        const int n = sched[(size_t)st * kWalkWaves + w].node;
-        if (n < 0) continue;
-        if (par[n] >= 0) freed.push_back(ratio_slot[n]);
-        for (int c : ic[n]) {
-          if (fs.empty()) return false;
-          ratio_slot[c] = fs.back();
-          fs.pop_back();
-        }
-      }
-      fs.insert(fs.end(), freed.begin(), freed.end());
-    }
-    return true;
-  };
-  auto pad_steps = [&](std::vector<StepItem>& sched, std::vector<PreItem>& pre, int steps) {
-    while ((int)sched.size() < steps * kWalkWaves) { sched.push_back(blank(-1)); pre.push_back(blank_pre(-1)); }
-  };
-  {
-    fwd_spill_ = false;
-    std::vector<std::vector<StepItem>> sched(n_groups_);
-    std::vector<std::vector<PreItem>> pre(n_groups_);
-    n_fwd_steps_ = 0;
-    for (int g = 0; g < n_groups_; ++g) {
-      schedule_forward(groups[g].first, groups[g].second, sched[g], pre[g], forest_);
-      n_fwd_steps_ = std::max(n_fwd_steps_, (int)sched[g].size() / kWalkWaves);
-    }
-    if (lean_k && !forest_ && fwd_spill_) {
-      // a single bushy tree whose waiting tiles overran the slots is scheduled again with a reserve (see kLeanStretch)
-      std::vector<StepItem> sched2;
-      std::vector<PreItem> pre2;
-      fwd_spill_ = false;
-      schedule_forward(0, n_inner_, sched2, pre2, true);
-      const int steps2 = (int)sched2.size() / kWalkWaves;
-      if (!fwd_spill_ && steps2 <= n_fwd_steps_ * kLeanStretch) {
-        n_fwd_steps_ = steps2;
-        sched[0].swap(sched2);
-        pre[0].swap(pre2);
-      } else {
-        fwd_spill_ = true;
-      }
-    }
-    std::vector<int32_t> lean_rows;
-    fwd_lean_ = !fwd_spill_;
-    for (int g = 0; g < n_groups_; ++g) {
-      pad_steps(sched[g], pre[g], n_fwd_steps_);   // the shorter groups idle at the end
-      if (g == 0) make_fields(sched[g], pre[g], true, fwd_stride_, d_fwd_fields_);
-      else pad_steps(sched[g], pre[g], fwd_stride_);
-      fwd_lean_ = fwd_lean_ && make_lean(sched[g], true, fwd_stride_, lean_rows);
-    }
-    if (fwd_lean_) d_fwd_lean_.upload(lean_rows);
-    d_fwd_sched_.upload(sched[0]);
-  }
-  // ---- backward ----------------------------------------------------------------------
   // Oldest-ready first (ties: longest chain below first): a parent's flow tile then leaves
   // its LDS slot a few steps after it was produced, so the number of live tiles stays near
   // the width of the tree instead of growing with every postponed short subtree.
-  auto schedule_backward = [&](int g0, int g1, std::vector<StepItem>& sched, std::vector<PreItem>& pre, bool counted) {
+  auto schedule_backward = [&](std::vector<StepItem>& sched, std::vector<PreItem>& pre) {
     std::vector<int32_t> remaining(n_inner_), slot(n_inner_, -1), ready_at(n_inner_, 0), free_slots;
     for (int s = trash_slot - 1; s >= 0; --s) free_slots.push_back(s);
     std::vector<int32_t> ready;
-    for (int n = g0; n < g1; ++n) { remaining[n] = (int)ic[n].size(); if (par[n] < 0) ready.push_back(n); }
-    int done = 0, step_no = 0, ratio_live = 0;
-    while (done < g1 - g0) {
+    for (int n = 0; n < n_inner_; ++n) { remaining[n] = (int)ic[n].size(); if (par[n] < 0) ready.push_back(n); }
+    int done = 0, step_no = 0;
+    while (done < n_inner_) {
       std::sort(ready.begin(), ready.end(), [&](int a, int b) {
-        if (tree_of_inner_[a] != tree_of_inner_[b]) return tree_of_inner_[a] < tree_of_inner_[b];   // a forest: tree after tree
         if (ready_at[a] != ready_at[b]) return ready_at[a] < ready_at[b];
-        return hin[a] != hin[b] ? hin[a] > hin[b] : a > b;
+        return lt.chain[a] != lt.chain[b] ? lt.chain[a] > lt.chain[b] : a > b;
       });
       // a node whose flow tile needs a slot waits while none is free; only if nothing else
       // is ready does a tile go through HBM instead
       std::vector<int32_t> step, rest;
       int slots_left = (int)free_slots.size();
       for (int n : ready) {
-        // with `counted` the ratio tiles of the lean walk (one per inner child, from the parent's step to the end of
-        // the child's) are counted along: a node only runs if its children's tiles fit.  In a forest a new tree only
-        // starts while half the slots are free, so that the trees under way can finish; in a single tree a node that
-        // adds tiles (two inner children or more) leaves kBranchReserve slots to the chains, which hand on as many
-        // tiles as they take.
-        const int need = (int)ic[n].size();
-        const int limit = !counted ? n_inner_ + trash_slot
-                          : T_ > 1 ? (par[n] < 0 ? trash_slot / 2 : trash_slot) : trash_slot - (need > 1 ? kBranchReserve : 0);
-        const bool ratio_ok = ratio_live + need <= limit;
-        if ((int)step.size() < kWalkWaves && (ic[n].empty() || slots_left > 0) && ratio_ok) {
+        if ((int)step.size() < kWalkWaves && (ic[n].empty() || slots_left > 0)) {
           step.push_back(n);
           if (!ic[n].empty()) --slots_left;
-          ratio_live += need;
         } else {
           rest.push_back(n);
         }
       }
       if (step.empty()) {
         if (rest.empty()) fail(PCM_ERR_SHAPE, "backward schedule stalled (tree is inconsistent)");
-        // (a single tree: the node with the fewest nodes below it, whose tiles are gone again soonest)
-        const auto pick = T_ > 1 || !counted ? rest.begin()
-                                             : std::min_element(rest.begin(), rest.end(), [&](int a, int b) { return below[a] < below[b]; });
-        ratio_live += (int)ic[*pick].size();
-        step.push_back(*pick);
-        rest.erase(pick);
+        step.push_back(rest.front());
+        rest.erase(rest.begin());
       }
       ready.swap(rest);
       for (int w = 0; w < kWalkWaves; ++w) {
@@ -620,110 +506,68 @@ void HcltCircuit::build_schedules() {
       }
       ++step_no;
       for (int n : step) {
-        if (par[n] >= 0) --ratio_live;
         if (par[n] >= 0 && --remaining[par[n]] == 0 && slot[par[n]] >= 0) free_slots.push_back(slot[par[n]]);
         for (int c : ic[n]) { ready.push_back(c); ready_at[c] = step_no; }
         ++done;
       }
     }
   };
-  {
-    bwd_spill_ = false;
-    std::vector<std::vector<StepItem>> scheds(n_groups_);
-    std::vector<std::vector<PreItem>> pres(n_groups_);
-    n_bwd_steps_ = 0;
-    for (int g = 0; g < n_groups_; ++g) {
-      schedule_backward(groups[g].first, groups[g].second, scheds[g], pres[g], forest_);
-      n_bwd_steps_ = std::max(n_bwd_steps_, (int)scheds[g].size() / kWalkWaves);
-    }
-    std::vector<int32_t> ratio_slot(n_inner_, -1);
-    bool slots_ok = true;
-    for (int g = 0; g < n_groups_ && slots_ok; ++g) slots_ok = assign_ratio_slots(scheds[g], ratio_slot);
-    if (lean_k && fwd_lean_ && !forest_ && !slots_ok) {
-      // a single tree whose ratio tiles overran the slots is scheduled again with the tiles counted
-      std::vector<StepItem> sched2;
-      std::vector<PreItem> pre2;
-      const bool spill = bwd_spill_;
-      bwd_spill_ = false;
-      schedule_backward(0, n_inner_, sched2, pre2, true);
-      std::vector<int32_t> ratio2(n_inner_, -1);
-      const int steps2 = (int)sched2.size() / kWalkWaves;
-      if (!bwd_spill_ && steps2 <= n_bwd_steps_ * kLeanStretch && assign_ratio_slots(sched2, ratio2)) {
-        slots_ok = true;
-        n_bwd_steps_ = steps2;
-        scheds[0].swap(sched2);
-        pres[0].swap(pre2);
-        ratio_slot.swap(ratio2);
-      } else {
-        bwd_spill_ = spill;
-      }
-    }
-    std::vector<int32_t> lean_rows;
-    bwd_lean_ = slots_ok;
-    for (int g = 0; g < n_groups_; ++g) {
-      pad_steps(scheds[g], pres[g], n_bwd_steps_);
-      if (g == 0) make_fields(scheds[g], pres[g], false, bwd_stride_, d_bwd_fields_);
-      else pad_steps(scheds[g], pres[g], bwd_stride_);
-      bwd_lean_ = bwd_lean_ && make_lean(scheds[g], false, bwd_stride_, lean_rows, &ratio_slot);
-    }
-    if (bwd_lean_) d_bwd_lean_.upload(lean_rows);
-    d_bwd_sched_.upload(scheds[0]);
+  fwd_spill_ = bwd_spill_ = false;
+  if (!forest_) {   // (a forest runs on the lean walks or not at all)
+    std::vector<StepItem> sched;
+    std::vector<PreItem> pre;
+    schedule_forward(sched, pre);
+    n_fwd_steps_ = (int)sched.size() / kWalkWaves;
+    make_fields(sched, pre, true, fwd_stride_, d_fwd_fields_);
+    d_fwd_sched_.upload(sched);
+    sched.clear();
+    pre.clear();
+    schedule_backward(sched, pre);
+    n_bwd_steps_ = (int)sched.size() / kWalkWaves;
+    make_fields(sched, pre, false, bwd_stride_, d_bwd_fields_);
+    d_bwd_sched_.upload(sched);
   }
-  // ---- a forest's finer plans --------------------------------------------------------------
-  // The same walks with two and four times as many, smaller groups of trees, for batches whose slices times the
-  // groups above leave most of the device idle (256 examples are 16 slices): the walk then takes the plan with
-  // the most groups that still gives every workgroup a compute unit of its own.  A tree's arithmetic does not
-  // depend on the group it is walked in, so the results are the same bits under every plan.
-  fine_plans_.clear();
-  if (forest_ && fwd_lean_ && bwd_lean_) {
-    const bool keep_fwd_spill = fwd_spill_, keep_bwd_spill = bwd_spill_;
-    for (int G = 2 * n_groups_; G <= 4 * n_groups_ && G <= T_ / 4; G *= 2) {
-      const std::vector<std::pair<int, int>> gr = make_groups(G);
-      if ((int)gr.size() <= (fine_plans_.empty() ? n_groups_ : fine_plans_.back()->n_groups)) break;
-      std::unique_ptr<LeanPlan> plan(new LeanPlan);
-      plan->n_groups = (int)gr.size();
-      bool ok = true;
+  // ---- lean walks ------------------------------------------------------------------------
+  // A plan: the schedules of a walk in G groups of whole trees, which the kernels take in blockIdx.y.  A tree's
+  // arithmetic does not depend on the group it is walked in, so the results are the same bits under every plan.
+  auto make_plan = [&](const std::vector<std::pair<int, int>>& groups) {
+    std::unique_ptr<LeanPlan> plan(new LeanPlan);
+    plan->n_groups = (int)groups.size();
+    for (const bool forward : {true, false}) {
+      std::vector<LeanSchedule> sched;
+      int steps = 0;
+      for (const auto& g : groups) {
+        sched.push_back(forward ? lean_schedule_up(lt, g.first, g.second, lds_slots_) : lean_schedule_down(lt, g.first, g.second, lds_slots_));
+        steps = std::max(steps, sched.back().steps);
+      }
+      const int stride = steps + 64;   // the shorter groups idle at the end
       std::vector<int32_t> rows;
-      {
-        fwd_spill_ = false;
-        std::vector<std::vector<StepItem>> sched(gr.size());
-        std::vector<std::vector<PreItem>> pre(gr.size());
-        for (size_t g = 0; g < gr.size(); ++g) {
-          schedule_forward(gr[g].first, gr[g].second, sched[g], pre[g], true);
-          plan->n_fwd_steps = std::max(plan->n_fwd_steps, (int)sched[g].size() / kWalkWaves);
-        }
-        ok = !fwd_spill_;
-        plan->fwd_stride = plan->n_fwd_steps + 64;
-        for (size_t g = 0; g < gr.size() && ok; ++g) {
-          pad_steps(sched[g], pre[g], plan->fwd_stride);
-          ok = make_lean(sched[g], true, plan->fwd_stride, rows);
-        }
-        if (ok) plan->fwd.upload(rows);
-      }
-      if (ok) {
-        bwd_spill_ = false;
-        std::vector<std::vector<StepItem>> sched(gr.size());
-        std::vector<std::vector<PreItem>> pre(gr.size());
-        for (size_t g = 0; g < gr.size(); ++g) {
-          schedule_backward(gr[g].first, gr[g].second, sched[g], pre[g], true);
-          plan->n_bwd_steps = std::max(plan->n_bwd_steps, (int)sched[g].size() / kWalkWaves);
-        }
-        ok = !bwd_spill_;
-        std::vector<int32_t> ratio_slot(n_inner_, -1);
-        for (size_t g = 0; g < gr.size() && ok; ++g) ok = assign_ratio_slots(sched[g], ratio_slot);
-        plan->bwd_stride = plan->n_bwd_steps + 64;
-        rows.clear();
-        for (size_t g = 0; g < gr.size() && ok; ++g) {
-          pad_steps(sched[g], pre[g], plan->bwd_stride);
-          ok = make_lean(sched[g], false, plan->bwd_stride, rows, &ratio_slot);
-        }
-        if (ok) plan->bwd.upload(rows);
-      }
-      if (!ok) break;
-      fine_plans_.push_back(std::move(plan));
+      for (const LeanSchedule& sc : sched)
+        if (!make_lean(sc, forward, stride, rows)) return std::unique_ptr<LeanPlan>();
+      (forward ? plan->n_fwd_steps : plan->n_bwd_steps) = steps;
+      (forward ? plan->fwd_stride : plan->bwd_stride) = stride;
+      (forward ? plan->fwd : plan->bwd).upload(rows);
     }
-    fwd_spill_ = keep_fwd_spill;
-    bwd_spill_ = keep_bwd_spill;
+    return plan;
+  };
+  // In order of their number of groups.  A forest's finer plans are for batches whose slices times the groups of the first
+  // leave most of the device idle (256 examples are 16 slices): a walk takes the plan with the most groups that still gives
+  // every workgroup a compute unit of its own.
+  plans_.clear();
+  if (K_ <= 32) {
+    const std::vector<std::pair<int, int>> groups = make_groups(forest_ ? std::max(1, std::min(4, T_ / 8)) : 1);
+    n_groups_ = (int)groups.size();
+    std::unique_ptr<LeanPlan> plan = make_plan(groups);
+    if (plan && !forest_ && (plan->n_fwd_steps > n_fwd_steps_ * kLeanStretch || plan->n_bwd_steps > n_bwd_steps_ * kLeanStretch))
+      plan.reset();   // (see kLeanStretch)
+    if (plan) plans_.push_back(std::move(plan));
+    for (int G = 2 * n_groups_; !plans_.empty() && G <= 4 * n_groups_ && G <= T_ / 4; G *= 2) {
+      const std::vector<std::pair<int, int>> gr = make_groups(G);
+      if ((int)gr.size() <= plans_.back()->n_groups) break;
+      plan = make_plan(gr);
+      if (!plan) break;
+      plans_.push_back(std::move(plan));
+    }
   }
   // ---- statistics: the static operands of every node ------------------------------------
   {
@@ -778,18 +622,16 @@ void HcltCircuit::build_schedules() {
       d_stat_claim_.upload(std::vector<uint32_t>(1, 0u));
     }
   }
-  lean_ = fwd_lean_ && bwd_lean_ && stat_lean_;
+  lean_ = !plans_.empty() && stat_lean_;
   if (ext.empty()) ext.push_back(0);
   d_ext_ops_.upload(ext);
-  if (getenv("PCM_VERBOSE"))
-    fprintf(stderr, "[pcmi355] hclt V=%d K=%d C=%d inner=%d trees=%d groups=%d: forward %d steps%s%s, backward %d steps%s%s, statistics%s, "
-            "%d LDS slots\n",
-            V_, K_, C_, n_inner_, T_, n_groups_, n_fwd_steps_, fwd_spill_ ? " (spills)" : "", fwd_lean_ ? " (lean)" : "", n_bwd_steps_,
-            bwd_spill_ ? " (spills)" : "", bwd_lean_ ? " (lean)" : "", stat_lean_ ? " (lean)" : "", lds_slots_);
-  if (getenv("PCM_VERBOSE"))
-    for (const auto& p : fine_plans_)
-      fprintf(stderr, "[pcmi355]   finer plan: %d groups, forward %d steps, backward %d steps\n", p->n_groups, p->n_fwd_steps,
-              p->n_bwd_steps);
+  if (getenv("PCM_VERBOSE")) {
+    fprintf(stderr, "[pcmi355] hclt V=%d K=%d C=%d inner=%d trees=%d: forward %d steps%s, backward %d steps%s, statistics%s, %d LDS slots\n",
+            V_, K_, C_, n_inner_, T_, n_fwd_steps_, fwd_spill_ ? " (spills)" : "", n_bwd_steps_, bwd_spill_ ? " (spills)" : "",
+            stat_lean_ ? " (lean)" : "", lds_slots_);
+    for (const auto& p : plans_)
+      fprintf(stderr, "[pcmi355]   lean: %d groups, forward %d steps, backward %d steps\n", p->n_groups, p->n_fwd_steps, p->n_bwd_steps);
+  }
 }
 
 // Numbering the reference would give this circuit.  Nodes are created in depth-first
@@ -1377,9 +1219,9 @@ void HcltCircuit::stage_batch(const BatchRef& b, bool tiles) {
 
 // The finer plan a batch of `nslices` slices walks a forest with, or null for the plan of the constructor: the
 // most groups whose workgroups still get a compute unit each.
-const HcltCircuit::LeanPlan* HcltCircuit::fine_plan(int nslices) const {
-  const LeanPlan* best = nullptr;
-  for (const auto& p : fine_plans_)
+const HcltCircuit::LeanPlan* HcltCircuit::lean_plan(int nslices) const {
+  const LeanPlan* best = plans_.front().get();
+  for (const auto& p : plans_)
     if ((int64_t)nslices * p->n_groups <= n_cus_) best = p.get();
   return best;
 }
@@ -1403,13 +1245,9 @@ void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
     const size_t lean_lds = lds + kLeanFlagWords * 4;   // the slots' state words sit behind the slots
     auto launch_lean = [&](auto kernel) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
-      const LeanPlan* fp = fine_plan(d.nslices);
-      if (fp)
-        PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices, fp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, fp->fwd.p,
-                         fp->fwd_stride, fp->n_fwd_steps, d_ll, lds_slots_);
-      else
-        PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices, n_groups_), dim3(kWalkWaves * 64), lean_lds, d, d_fwd_lean_.p, fwd_stride_,
-                         n_fwd_steps_, d_ll, lds_slots_);
+      const LeanPlan* lp = lean_plan(d.nslices);
+      PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, lp->fwd.p, lp->fwd_stride,
+                       lp->n_fwd_steps, d_ll, lds_slots_);
     };
     PCM_DISPATCH_LEAN_K(K_, {
       if (keep == kKeepAll) launch_lean(&hclt_forward_lean_kernel<KK, kKeepAll>);
@@ -1435,13 +1273,9 @@ void HcltCircuit::run_backward(const HcltDev& d) {
     const size_t lean_lds = lds + kLeanFlagWords * 4;
     auto launch_lean = [&](auto kernel) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
-      const LeanPlan* fp = fine_plan(d.nslices);
-      if (fp)
-        PCM_LAUNCH_PHASE(1, kernel, dim3(d.nslices, fp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, fp->bwd.p,
-                         fp->bwd_stride, fp->n_bwd_steps, lds_slots_);
-      else
-        PCM_LAUNCH_PHASE(1, kernel, dim3(d.nslices, n_groups_), dim3(kWalkWaves * 64), lean_lds, d, d_bwd_lean_.p, bwd_stride_,
-                         n_bwd_steps_, lds_slots_);
+      const LeanPlan* lp = lean_plan(d.nslices);
+      PCM_LAUNCH_PHASE(1, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, lp->bwd.p, lp->bwd_stride,
+                       lp->n_bwd_steps, lds_slots_);
     };
     PCM_DISPATCH_LEAN_K(K_, {
       if (H_ > 0) launch_lean(&hclt_backward_lean_kernel<KK, true>); else launch_lean(&hclt_backward_lean_kernel<KK, false>);

@@ -27,15 +27,10 @@ constexpr int kXSelShift = 28;               // leaf operand: which byte of the 
 constexpr int kSlotShift = 22;               // LDS operand: (slot + 1) << kSlotShift | inner id
 constexpr int kItemRoot = 1, kItemHasInnerChild = 2, kItemOverflow = 4, kItemSpillOut = 8;
 enum { kKeepNone = 0, kKeepRoots, kKeepAll };   // what the lean forward walk leaves in memory (hclt_walk_lean.hip.hpp)
-// A single tree (K <= 32) whose tiles overrun the LDS slots under the plain greedy schedules is scheduled again with the
-// tiles counted, at up to kLeanStretch times the steps, before it goes to the general walk kernels: those take 1.45 times
-// as long per EM step (2.40 against 1.65 ms on a 3072-variable Chow-Liu tree at 4096 examples, which needed 80 ratio
-// tiles of the 78 that fit and needs no step more, 164, with the tiles counted).  Of 66 random trees of 1000 to 3072
-// variables, 15 are scheduled again without a step more and one with 40 for 39 (0.56 against 0.80 ms).  Beyond the line: a forward walk
-// of 1.45 times the steps beside a backward one of 0.6 still gains (2000 variables: 1.87 against 2.32 ms), a backward one
-// of 2.8 times loses (3072 variables, binary: 2.71 against 2.33 ms).  A branching node leaves
-// kBranchReserve slots free to the chains; 0 / 16 / 24 gave 164 / 164 / 165 steps there.
-constexpr int kBranchReserve = 8;
+// A single tree (K <= 32) runs on the lean walks if their schedules, which keep every tile in registers or LDS, take at most
+// kLeanStretch times the steps of the general walks' schedules, which may send tiles through memory: the general kernels
+// take 1.45 times as long per EM step of as many steps (2.40 against 1.65 ms on a 3072-variable Chow-Liu tree at 4096
+// examples).
 constexpr double kLeanStretch = 1.4;
 constexpr int kPre = 3;          // static operand tiles a wave requests one step ahead
 
@@ -236,13 +231,14 @@ class HcltCircuit : public pcm_circuit {
   bool forest_ = false;
   int T_ = 1;                      // trees (1 unless a forest)
   int n_groups_ = 1;               // groups of trees the walk kernels take side by side (blockIdx.y)
-  // a forest's walk schedules with more, smaller groups of trees, for batches whose slices do not fill the device
+  // schedules of the lean walks, in one group of trees or more (a forest's finer plans are for batches whose slices do not
+  // fill the device), fewest groups first
   struct LeanPlan {
     int n_groups = 1, n_fwd_steps = 0, fwd_stride = 0, n_bwd_steps = 0, bwd_stride = 0;
     DevBuf<int32_t> fwd, bwd;
   };
-  std::vector<std::unique_ptr<LeanPlan>> fine_plans_;
-  const LeanPlan* fine_plan(int nslices) const;
+  std::vector<std::unique_ptr<LeanPlan>> plans_;   // empty: the lean kernels do not take this tree
+  const LeanPlan* lean_plan(int nslices) const;
   std::vector<int32_t> roots_;     // root variable of every tree, in variable order
   std::vector<int32_t> tree_of_inner_;   // tree of every inner node
   // inner nodes of the caller's tree, and every node's index among them (auxiliary nodes keep the post-order of the
@@ -299,9 +295,9 @@ class HcltCircuit : public pcm_circuit {
   DevBuf<HcltNode> d_nodes_;
   DevBuf<int32_t> d_child_inner_, d_child_leaf_;
   DevBuf<StepItem> d_fwd_sched_, d_bwd_sched_, d_stat_items_;
-  DevBuf<int32_t> d_fwd_fields_, d_bwd_fields_, d_fwd_lean_, d_bwd_lean_;
-  bool fwd_lean_ = false, bwd_lean_ = false, stat_lean_ = false;   // each lean kernel could run this tree ...
-  bool lean_ = false;   // ... and all three do (they share the stored row maxima, so it is all or none)
+  DevBuf<int32_t> d_fwd_fields_, d_bwd_fields_;   // the general walk kernels' schedules
+  bool stat_lean_ = false;   // the lean statistics kernel could run this tree ...
+  bool lean_ = false;        // ... and all three lean kernels do (they share the stored row maxima, so it is all or none)
   DevBuf<float> d_M_;
   int* walk_err_ = nullptr;    // pinned host word the walk kernels raise (HcltDev::err); checked by check_walks()
   void check_walks();

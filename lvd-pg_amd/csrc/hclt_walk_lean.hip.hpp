@@ -15,7 +15,13 @@
 //     zero-filled, selected or copied;
 //   * the parameter block is requested right after the contraction that used its
 //     predecessor, into the same registers, so nothing rotates between steps.
-// Idle waves work on a trash tile (row n_inner of the value arrays) and the trash LDS slot.
+//   * a wave follows a chain of the tree (lean_schedule.hpp): the tile of its last node is in registers when the next one
+//     needs it, and four tiles in five go through no LDS slot, no wait and no post;
+//   * idle steps only keep the requests going.
+// What bounds a step (walks with pieces left out, 784 variables, K = 32, 512 examples, 53 steps of 16 nodes, 97 us): all its
+// memory requests without the arithmetic 95 us, all the arithmetic without the requests 84, neither 33.  The fp32 matrix
+// instructions of a SIMD's four waves (4 x 512 cycles) and their vector instructions (4 x 600) add up, as both use the same
+// units; the requests of a compute unit (140 KB a step) do so beside them.
 #pragma once
 
 #include "hclt_kernels.hip.hpp"
@@ -23,20 +29,21 @@
 namespace pcm {
 
 // Field rows of a lean schedule, [field][wave][stride] like the general one.
-//   kLW     byte offset of the node's parameter block
+//   kLW     byte offset of the node's parameter block (-1: none wanted)
 //   kLA0    byte offset of the node's own leaf rows (variable * leaf_stride)
 //   kLA1..3 forward: leaf children's rows (-1: none; their categories are bytes 1..3 of the
 //           packed word).  backward: children, inner ones first, -1: none, leaf child: row
 //           offset | 1 | category byte << 1, inner child: node index << 3 (its value tile)
 //   kLNode  node index (value / flow tile, packed-category row, row of maxima); idle waves:
-//           n_inner, the trash tile (its category row is out of range and reads as zero)
+//           n_inner (that category row is out of range and reads as zero)
 //   kLSlots forward: out slot | child slots << 8, 16, 24 (0xff: none); backward: slot holding
 //           this node's ratio tile | slots of the inner children's ratio tiles << 8, 16, 24
-//           (0xff: that child is a leaf or absent)
+//           (0xff: that child is a leaf or absent); kLeanKept: in registers
 //   kLFlags bit 0: root; bit 1: root of a multi-head circuit
 //   kLTurns which use of its slot a tile is, modulo 128, in the byte layout of kLSlots: a slot passes through
 //           the states 2t (free for its t-th tile), 2t + 1 (that tile is there), 2t + 2 (read, free again)
 enum { kLW = 0, kLA0, kLA1, kLA2, kLA3, kLNode, kLSlots, kLFlags, kLTurns, kLeanFields };
+constexpr uint32_t kLeanKept = 0xfe;       // in place of a slot: the tile stays in the registers of the wave (one that stays nowhere: 0xff)
 constexpr int kLeanFlagWords = 256;        // one state word per LDS slot, behind the slots
 constexpr int kLeanSpinLimit = 1 << 22;    // polls before a wave gives up on a tile (never reached by a sound schedule)
 
@@ -76,17 +83,11 @@ __device__ __forceinline__ void lean_tile_load(__amdgpu_buffer_rsrc_t r, uint32_
     t.v[kt] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(voff + kt * 1024), soff, kStreamLoad));
 }
 
-#ifndef PCM_ST_O
-#define PCM_ST_O kStreamStore
-#endif
-#ifndef PCM_ST_R
-#define PCM_ST_R kStreamStore
-#endif
-template <int K, int kAux = kStreamStore>
+template <int K>
 __device__ __forceinline__ void lean_tile_store(__amdgpu_buffer_rsrc_t r, uint32_t voff, int soff, const Tile<K>& t) {
 #pragma unroll
   for (int kt = 0; kt < K / 16; ++kt)
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, t.v[kt]), r, (int)(voff + kt * 1024), soff, kAux);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, t.v[kt]), r, (int)(voff + kt * 1024), soff, kStreamStore);
 }
 
 template <int K>
@@ -94,6 +95,16 @@ __device__ __forceinline__ void lean_w_load(__amdgpu_buffer_rsrc_t r, uint32_t v
 #pragma unroll
   for (int i = 0; i < (K / 16) * (K / 16); ++i)
     w.a[i] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(voff + (i & 3) * 1024), soff + (i >> 2) * 4096, 0));
+}
+
+// The same where the block may be absent (-1: idle steps; going down, nodes without inner children): the requests go out
+// all the same, past the end of the array, where the buffer unit answers with zeros and fetches nothing.  Behind a branch
+// they would cost more than they save: the compiler counts the requests in flight for the shorter way, so the wait for
+// the next step's rows would also wait for this block, two steps early.
+constexpr uint32_t kLeanNowhere = 0x80000000u;   // (every array is shorter)
+template <int K>
+__device__ __forceinline__ void lean_w_load_if(__amdgpu_buffer_rsrc_t r, uint32_t vtile, int soff, WTile<K>& w) {
+  lean_w_load<K>(r, soff < 0 ? kLeanNowhere + vtile : vtile, max(soff, 0), w);
 }
 
 // byte offset of this lane's part of leaf row x (byte `sel` of the packed word)
@@ -144,6 +155,10 @@ __device__ __forceinline__ void lean_post(unsigned* state, unsigned value) {
 // but the log-likelihoods: a scoring pass has nobody behind it, and value stores are 512 of a step's 1340 requests.
 // 10300 examples of 3072 variables (K = 32), which no longer need tile arrays and so go through 4096 at a time
 // whatever the caller's batch size: 3.93 ms in batches of 1000 -> 1.08 ms.
+//
+// With chains kept in registers, against the schedule that picked the sixteen most urgent nodes of every step anew (a tile per
+// node through LDS): 784 variables, 512 examples 111 -> 97 us, 192 variables 55 -> 42, 64 variables (K = 16) 19 -> 16.5;
+// 3072 variables at 4096 examples, where the stores of the tiles count, 390 -> 384.
 template <int K, int kKeep>
 __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
     HcltDev d, const int32_t* __restrict__ fields, int stride, int n_steps, float* __restrict__ ll_out, int n_slots) {
@@ -185,34 +200,24 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
     if (a1 >= 0) lean_row_load<K>(rL, lean_row_off<K>(x0, 1, vleaf), a1, P1);
     if (a2 >= 0) lean_row_load<K>(rL, lean_row_off<K>(x0, 2, vleaf), a2, P2);
     if (a3 >= 0) lean_row_load<K>(rL, lean_row_off<K>(x0, 3, vleaf), a3, P3);
-    lean_w_load<K>(rW, vtile, lean_get(sc, kLW, 0), wA);
-    lean_w_load<K>(rW, vtile, lean_get(sc, kLW, 1), wB);
+    lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, 0), wA);
+    __builtin_amdgcn_sched_barrier(0);   // (in this order: the waits inside the loop are counted for both ways into it)
+    lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, 1), wB);
+    __builtin_amdgcn_sched_barrier(0);
   }
   float ll = 0.f;
+  bool root_here = false;
   double msum = 0.0;   // sum of the row maxima of this wave's nodes: the part of the log-likelihood the tiles leave out
-  Tile<K> o_prev;   // the value tile of the previous step, stored at the top of the next one
-  tile_zero<K>(o_prev);
-  int store_prev = (int)((uint32_t)d.n_inner * d.tile_stride);   // (kKeepNone: past 32 bits for all it matters)
-  float m_prev = 0.f;
-  int mrow_prev = d.n_inner * xrow;
+  Tile<K> o;           // the value tile of this wave's last node: its parent takes it from here if it comes next in the wave
+  tile_zero<K>(o);
 
-  bool root_prev = false;
-  auto keep_prev = [&]() {
-    if (kKeep == kKeepAll || (kKeep == kKeepRoots && root_prev)) lean_tile_store<K, PCM_ST_O>(rO, vtile, store_prev, o_prev);
-    if (kKeep != kKeepNone)
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, m_prev), rM, (int)vm, mrow_prev, kStreamStore);
-  };
-
-  // the schedule is consumed in chunks of kLeanChunk steps (a chunk's registers also serve
-  // the two steps of look-ahead past its end)
   auto step = [&](const int s, WTile<K>& w) {
     // (1) the static operands of this step have landed
     Tile<K> z = P0;
     if (a1 >= 0) tile_add<K>(z, P1);
     if (a2 >= 0) tile_add<K>(z, P2);
     if (a3 >= 0) tile_add<K>(z, P3);
-    // the previous step's value tile goes out now
-    keep_prev();
+    const int node = lean_get(sc, kLNode, s);
     // (2) request the leaf rows of step s+1 and the categories of step s+2
     {
       // (the categories first: everything that later waits for a leaf row then covers them)
@@ -224,44 +229,53 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
       if (a2 >= 0) lean_row_load<K>(rL, lean_row_off<K>(xc, 2, vleaf), a2, P2);
       if (a3 >= 0) lean_row_load<K>(rL, lean_row_off<K>(xc, 3, vleaf), a3, P3);
     }
-    // (3) children from LDS, logsumexp through the matrix cores
-    const uint32_t slots = (uint32_t)lean_get(sc, kLSlots, s), turns = (uint32_t)lean_get(sc, kLTurns, s);
+    if (node != d.n_inner) {   // (idle steps only keep the requests going)
+      // (3) inner children, from LDS or, the one this wave computed last, from registers; logsumexp through the matrix cores
+      const uint32_t slots = (uint32_t)lean_get(sc, kLSlots, s), turns = (uint32_t)lean_get(sc, kLTurns, s);
 #pragma unroll
-    for (int c = 1; c <= 3; ++c) {
-      const uint32_t sl = (slots >> (8 * c)) & 0xffu, tn = (turns >> (8 * c)) & 0x7fu;
-      if (sl != 0xffu) {
-        lean_wait(state + sl, (2 * tn + 1) & 0xffu, d);
-        Tile<K> t;
-        lds_tile_load<K>(lds, (int)sl, lane, t);
-        tile_add<K>(z, t);
-        lean_post(state + sl, (2 * tn + 2) & 0xffu);   // read: the slot may take its next tile
+      for (int c = 1; c <= 3; ++c) {
+        const uint32_t sl = (slots >> (8 * c)) & 0xffu, tn = (turns >> (8 * c)) & 0x7fu;
+        if (sl == 0xffu) break;
+        if (sl == kLeanKept) {
+          tile_add<K>(z, o);
+        } else {
+          lean_wait(state + sl, (2 * tn + 1) & 0xffu, d);
+          Tile<K> t;
+          lds_tile_load<K>(lds, (int)sl, lane, t);
+          tile_add<K>(z, t);
+          lean_post(state + sl, (2 * tn + 2) & 0xffu);   // read: the slot may take its next tile
+        }
       }
-    }
-    const float m = tile_rowmax<K>(z);
-    tile_exp_sub<K>(z, m);
-    Tile<K> o;
-    contract<K>(w, z, o);
+      const float m = tile_rowmax<K>(z);
+      tile_exp_sub<K>(z, m);
+      contract<K>(w, z, o);
 #pragma unroll
-    for (int kt = 0; kt < K / 16; ++kt)
+      for (int kt = 0; kt < K / 16; ++kt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o.v[kt][i] = __builtin_amdgcn_logf(o.v[kt][i]) * kLn2;
-    lean_w_load<K>(rW, vtile, lean_get(sc, kLW, s + 2), w);   // the block of step s+2, same registers
-    o_prev = o;
-    const int node = lean_get(sc, kLNode, s);
-    store_prev = (int)((uint32_t)node * d.tile_stride);
-    m_prev = m;
-    mrow_prev = node * xrow;
-    if (node != d.n_inner) msum += (double)m;   // (idle steps work on the trash tile)
-    {
-      // idle steps and the root write the trash slot, which nobody reads: no hand-over there
+        for (int i = 0; i < 4; ++i) o.v[kt][i] = __builtin_amdgcn_logf(o.v[kt][i]) * kLn2;
+      // hand the tile on first (the root's, and one whose reader is this wave's next node, go nowhere)
       const uint32_t so = slots & 0xffu, tn = turns & 0x7fu;
-      const bool handed = so != (uint32_t)(n_slots - 1);
-      if (handed) lean_wait(state + so, (2 * tn) & 0xffu, d);
-      lds_tile_store<K>(lds, (int)so, lane, o);
-      if (handed) lean_post(state + so, (2 * tn + 1) & 0xffu);
+      if (so < kLeanKept) {
+        lean_wait(state + so, (2 * tn) & 0xffu, d);
+        lds_tile_store<K>(lds, (int)so, lane, o);
+        lean_post(state + so, (2 * tn + 1) & 0xffu);
+      }
+      msum += (double)m;
+      const bool root = (lean_get(sc, kLFlags, s) & 1) != 0;
+      if (root) {
+        ll = o.v[0][0];
+        root_here = true;
+      }
+      if (kKeep == kKeepAll || (kKeep == kKeepRoots && root))
+        lean_tile_store<K>(rO, vtile, (int)((uint32_t)node * d.tile_stride), o);
+      if (kKeep != kKeepNone)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, m), rM, (int)vm, node * xrow, kStreamStore);
     }
-    root_prev = (lean_get(sc, kLFlags, s) & 1) != 0;
-    if (root_prev) ll = o.v[0][0];
+    // (4) the block of step s+2, into the registers of this step's; behind the stores, so that a step's wait for its
+    // leaf rows finds exactly these requests behind them, whether there were stores or not
+    __builtin_amdgcn_sched_barrier(0);
+    lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, s + 2), w);
+    __builtin_amdgcn_sched_barrier(0);
   };
   // The schedule is consumed in chunks of kLeanChunk steps (a chunk's registers also serve the
   // two steps of look-ahead past its end), two steps per trip: the parameter blocks alternate
@@ -275,19 +289,22 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
       step(s + 1, wB);
     }
   }
-  keep_prev();
   // log-likelihood of a single-root circuit: the root's (scaled) value plus the row maxima of all nodes, the
   // waves' sums added in wave order (a multi-head circuit's head kernel adds up the stored maxima per tree)
   if (!ll_out) return;
   __syncthreads();   // every wave is through its steps: the slots are free
   double* part = reinterpret_cast<double*>(lds);
-  if (lane < 16) part[wave * 16 + lane] = msum;
+  float* top = lds + 2 * kWalkWaves * 16;
+  if (lane < 16) {
+    part[wave * 16 + lane] = msum;
+    if (root_here) top[lane] = ll;
+  }
   __syncthreads();
-  if (wave == 0 && lane < 16 && bcol < d.B) {   // the root is item 0 of the last step
+  if (wave == 0 && lane < 16 && bcol < d.B) {
     double tot = 0.0;
 #pragma unroll
     for (int w = 0; w < kWalkWaves; ++w) tot += part[w * 16 + lane];
-    ll_out[bcol] = (float)(tot + (double)ll);
+    ll_out[bcol] = (float)(tot + (double)top[lane]);
   }
 }
 
@@ -302,6 +319,8 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
 // child gives probability zero (O'_c = -inf) has flow 0 and keeps ratio 0.  A node without inner children
 // only stores its tile.
 // kHeads: multi-head circuit, whose head kernel has left the root's ratio tile in memory.
+// 192 variables at 4096 examples 77 -> 53 us, 784 at 4096 184 -> 170 with the first child's tile in registers and the blocks
+// requested whether wanted or not; 3072 at 4096 stays at 625: 3.2 GB at 5.2 TB/s.
 template <int K, bool kHeads>
 __global__ __launch_bounds__(kWalkWaves * 64) void hclt_backward_lean_kernel(
     HcltDev d, const int32_t* __restrict__ fields, int stride, int n_steps, int n_slots) {
@@ -350,10 +369,13 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_backward_lean_kernel(
     if (c1 >= 0) child_load(c1, x0, C1);
     if (c2 >= 0) child_load(c2, x0, C2);
     if (c3 >= 0) child_load(c3, x0, C3);
-    // (a node without inner children has no use for its parameter block)
-    if (is_inner(c1)) lean_w_load<K>(rW, vtile, lean_get(sc, kLW, 0), wA);
-    if (is_inner(lean_get(sc, kLA1, 1))) lean_w_load<K>(rW, vtile, lean_get(sc, kLW, 1), wB);
+    lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, 0), wA);
+    __builtin_amdgcn_sched_barrier(0);   // (in this order: the waits inside the loop are counted for both ways into it)
+    lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, 1), wB);
+    __builtin_amdgcn_sched_barrier(0);
   }
+  Tile<K> r;   // the ratio tile of the node under way; behind a step, that of its first child, which comes next in this wave
+  tile_zero<K>(r);
 
   // exponent tile of inner child `own` among the landed operands: the other operands minus m_v,
   // in base-2 units; -inf where the child's own value is -inf
@@ -373,23 +395,21 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_backward_lean_kernel(
   auto step = [&](const int s, WTile<K>& w) {
     // (1) from the landed operands: the exponent tiles of the inner children (they come first).  The first
     // stays in registers; a second and third wait in the LDS slots their ratio tiles will take.
+    const int node = lean_get(sc, kLNode, s);
     const bool in1 = is_inner(c1), in2 = is_inner(c2), in3 = is_inner(c3);
     const uint32_t slots = (uint32_t)lean_get(sc, kLSlots, s), turns = (uint32_t)lean_get(sc, kLTurns, s);
-    {   // the children's slots are this wave's from here (scratch first, their ratio tiles at the end)
-      if (in1) lean_wait(state + ((slots >> 8) & 0xffu), (2 * ((turns >> 8) & 0x7fu)) & 0xffu, d);
-      if (in2) lean_wait(state + ((slots >> 16) & 0xffu), (2 * ((turns >> 16) & 0x7fu)) & 0xffu, d);
-      if (in3) lean_wait(state + ((slots >> 24) & 0xffu), (2 * ((turns >> 24) & 0x7fu)) & 0xffu, d);
-    }
     Tile<K> X1;
     if (in1) exponent(C1, c2 >= 0, C2, c3 >= 0, C3, X1);
-    if (in2) {
+    if (in2) {   // the children's slots are this wave's from here (scratch first, their ratio tiles at the end)
       Tile<K> x;
       exponent(C2, true, C1, c3 >= 0, C3, x);
+      lean_wait(state + ((slots >> 16) & 0xffu), (2 * ((turns >> 16) & 0x7fu)) & 0xffu, d);
       lds_tile_store<K>(lds, (int)((slots >> 16) & 0xffu), lane, x);
     }
     if (in3) {
       Tile<K> x;
       exponent(C3, true, C1, true, C2, x);
+      lean_wait(state + ((slots >> 24) & 0xffu), (2 * ((turns >> 24) & 0x7fu)) & 0xffu, d);
       lds_tile_store<K>(lds, (int)((slots >> 24) & 0xffu), lane, x);
     }
     // (2) request the operands of step s+1 and the categories of step s+2
@@ -403,55 +423,53 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_backward_lean_kernel(
       if (c2 >= 0) child_load(c2, xc, C2);
       if (c3 >= 0) child_load(c3, xc, C3);
     }
-    // (3) this node's ratio tile: left in LDS by the parent (the root and idle steps read the trash slot)
-    Tile<K> r;
-    const bool handed = (slots & 0xffu) != (uint32_t)(n_slots - 1);
-    if (handed) lean_wait(state + (slots & 0xffu), (2 * (turns & 0x7fu) + 1) & 0xffu, d);
-    lds_tile_load<K>(lds, (int)(slots & 0xffu), lane, r);
-    if (handed) lean_post(state + (slots & 0xffu), (2 * (turns & 0x7fu) + 2) & 0xffu);
-    const int fl = lean_get(sc, kLFlags, s);
-    if (kHeads && (fl & 2)) {   // multi-head circuit: the head kernel has left the root's ratio tile in memory
-      lean_tile_load<K>(rR, vtile, lean_get(sc, kLNode, s) * (int)d.tile_stride, r);
-    } else if (fl & 1) {   // flow 1 into the single root sum node of every live example: R = 1 / S = exp(-O')
-      const float o00 = __builtin_bit_cast(
-          float, __builtin_amdgcn_raw_buffer_load_b32(rO, (int)vtile, lean_get(sc, kLNode, s) * (int)d.tile_stride, 0));
-      const bool live = lane < 16 && bcol < d.B;
-      const float wgt = (d.w && live) ? d.w[bcol] : 1.f;   // per-example weights: the flow the example starts with
-      const float r00 = live ? wgt * fminf(__builtin_amdgcn_exp2f(o00 * -kLog2e), kFlowRatioCap) : 0.f;
-      tile_zero<K>(r);
-      r.v[0][0] = r00;
-    }
-    lean_tile_store<K, PCM_ST_R>(rR, vtile, lean_get(sc, kLNode, s) * (int)d.tile_stride, r);
-    // (4) the inner children's ratio tiles
-    if (in1) {
-      Tile<K> t;
-      contract<K>(w, r, t);
-      auto emit = [&](const Tile<K>& x, uint32_t slot) {
-        Tile<K> rc;
-#pragma unroll
-        for (int kt = 0; kt < K / 16; ++kt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) rc.v[kt][i] = t.v[kt][i] * fminf(__builtin_amdgcn_exp2f(x.v[kt][i]), kFlowRatioCap);
-        lds_tile_store<K>(lds, (int)slot, lane, rc);
-      };
-      emit(X1, (slots >> 8) & 0xffu);
-      if (in2) {
-        Tile<K> x;
-        lds_tile_load<K>(lds, (int)((slots >> 16) & 0xffu), lane, x);
-        emit(x, (slots >> 16) & 0xffu);
+    if (node != d.n_inner) {   // (idle steps only keep the requests going)
+      // (3) this node's ratio tile: in registers from the step before, or left in LDS by the parent
+      const uint32_t so = slots & 0xffu;
+      if (so < kLeanKept) {
+        lean_wait(state + so, (2 * (turns & 0x7fu) + 1) & 0xffu, d);
+        lds_tile_load<K>(lds, (int)so, lane, r);
+        lean_post(state + so, (2 * (turns & 0x7fu) + 2) & 0xffu);
       }
-      if (in3) {
-        Tile<K> x;
-        lds_tile_load<K>(lds, (int)((slots >> 24) & 0xffu), lane, x);
-        emit(x, (slots >> 24) & 0xffu);
+      const int fl = lean_get(sc, kLFlags, s);
+      if (kHeads && (fl & 2)) {   // multi-head circuit: the head kernel has left the root's ratio tile in memory
+        lean_tile_load<K>(rR, vtile, node * (int)d.tile_stride, r);
+      } else if (fl & 1) {   // flow 1 into the single root sum node of every live example: R = 1 / S = exp(-O')
+        const float o00 = __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(rO, (int)vtile, node * (int)d.tile_stride, 0));
+        const bool live = lane < 16 && bcol < d.B;
+        const float wgt = (d.w && live) ? d.w[bcol] : 1.f;   // per-example weights: the flow the example starts with
+        const float r00 = live ? wgt * fminf(__builtin_amdgcn_exp2f(o00 * -kLog2e), kFlowRatioCap) : 0.f;
+        tile_zero<K>(r);
+        r.v[0][0] = r00;
       }
-      {
-        lean_post(state + ((slots >> 8) & 0xffu), (2 * ((turns >> 8) & 0x7fu) + 1) & 0xffu);
-        if (in2) lean_post(state + ((slots >> 16) & 0xffu), (2 * ((turns >> 16) & 0x7fu) + 1) & 0xffu);
-        if (in3) lean_post(state + ((slots >> 24) & 0xffu), (2 * ((turns >> 24) & 0x7fu) + 1) & 0xffu);
+      lean_tile_store<K>(rR, vtile, node * (int)d.tile_stride, r);
+      // (4) the inner children's ratio tiles; the first child is this wave's next node
+      if (in1) {
+        Tile<K> t;
+        contract<K>(w, r, t);
+        auto ratio = [&](const Tile<K>& x, Tile<K>& rc) {
+#pragma unroll
+          for (int kt = 0; kt < K / 16; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) rc.v[kt][i] = t.v[kt][i] * fminf(__builtin_amdgcn_exp2f(x.v[kt][i]), kFlowRatioCap);
+        };
+        auto hand_on = [&](int c) {
+          const uint32_t sl = (slots >> (8 * c)) & 0xffu;
+          Tile<K> x;
+          lds_tile_load<K>(lds, (int)sl, lane, x);
+          ratio(x, x);
+          lds_tile_store<K>(lds, (int)sl, lane, x);
+          lean_post(state + sl, (2 * ((turns >> (8 * c)) & 0x7fu) + 1) & 0xffu);
+        };
+        if (in2) hand_on(2);
+        if (in3) hand_on(3);
+        ratio(X1, r);
       }
     }
-    if (is_inner(lean_get(sc, kLA1, s + 2))) lean_w_load<K>(rW, vtile, lean_get(sc, kLW, s + 2), w);
+    __builtin_amdgcn_sched_barrier(0);
+    lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, s + 2), w);
+    __builtin_amdgcn_sched_barrier(0);
   };
   for (int base = 0; base < n_steps; base += kLeanChunk) {
     if (base) lean_refill(fields, stride, wave, lane, base, sc);

@@ -19,6 +19,7 @@ namespace pcm {
 
 // field rows of a lean schedule, [field][wave][stride]; the names are those of hclt_walk_lean.hip.hpp
 constexpr int kLeanCheckA1 = 2, kLeanCheckSlots = 6, kLeanCheckTurns = 8, kLeanCheckFields = 9, kLeanCheckWaves = 16;
+constexpr uint8_t kLeanCheckKept = 0xfe;   // from here on a slot byte names no slot (kept in registers / nobody hands it on)
 
 struct LeanSlotOp {
   uint8_t slot, value;
@@ -33,11 +34,11 @@ inline void lean_step_ops(const int32_t* f, int stride, int w, int s, bool forwa
   auto st = [&](int c, int add) { return (uint8_t)((2u * ((turns >> (8 * c)) & 0x7fu) + (uint32_t)add) & 0xffu); };
   if (forward) {
     for (int c = 1; c <= 3; ++c)
-      if (sl(c) != 0xffu) {   // a child's tile: wait for it, read it, free the slot
+      if (sl(c) < kLeanCheckKept) {   // a child's tile: wait for it, read it, free the slot
         ops.push_back({sl(c), st(c, 1), true});
         ops.push_back({sl(c), st(c, 2), false});
       }
-    if (sl(0) != (uint8_t)trash_slot) {   // the node's own tile goes into its slot once that is free
+    if (sl(0) != (uint8_t)trash_slot && sl(0) < kLeanCheckKept) {   // the node's own tile goes into its slot once that is free
       ops.push_back({sl(0), st(0, 0), true});
       ops.push_back({sl(0), st(0, 1), false});
     }
@@ -49,14 +50,14 @@ inline void lean_step_ops(const int32_t* f, int stride, int w, int s, bool forwa
     inner[c] = a >= 0 && !(a & 1);
   }
   for (int c = 1; c <= 3; ++c)
-    if (inner[c]) ops.push_back({sl(c), st(c, 0), true});   // the children's slots must be free
-  if (sl(0) != (uint8_t)trash_slot) {                       // the node's ratio tile, left by its parent
+    if (inner[c] && sl(c) < kLeanCheckKept) ops.push_back({sl(c), st(c, 0), true});   // the children's slots must be free
+  if (sl(0) != (uint8_t)trash_slot && sl(0) < kLeanCheckKept) {   // the node's ratio tile, left by its parent
     ops.push_back({sl(0), st(0, 1), true});
     ops.push_back({sl(0), st(0, 2), false});
   }
   if (inner[1])
     for (int c = 1; c <= 3; ++c)
-      if (inner[c]) ops.push_back({sl(c), st(c, 1), false});
+      if (inner[c] && sl(c) < kLeanCheckKept) ops.push_back({sl(c), st(c, 1), false});
 }
 
 // -1 if every wave gets through its `n_steps` steps; otherwise step * 16 + wave of the first wave found stuck.

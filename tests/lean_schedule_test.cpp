@@ -1,0 +1,122 @@
+// Host test of csrc/lean_schedule.hpp: schedules of chains, stars, binary and random trees, one tree or several, for many
+// and few slots.  Every schedule is replayed step by step.  Prints "<name> <number>" lines.
+#include <cstdio>
+#include <random>
+
+#include "lean_schedule.hpp"
+
+using namespace pcm;
+
+// inner nodes only, children before their parents: parent[v] > v, or -1
+static LeanTree make(const std::vector<int>& parent) {
+  LeanTree t;
+  const int n = (int)parent.size();
+  t.parent.assign(parent.begin(), parent.end());
+  t.inner.resize(n);
+  t.tree.assign(n, 0);
+  t.depth.assign(n, 0);
+  for (int v = 0; v < n; ++v)
+    if (parent[v] >= 0) t.inner[parent[v]].push_back(v);
+  for (int v = n - 1; v >= 0; --v) t.depth[v] = parent[v] < 0 ? 0 : t.depth[parent[v]] + 1;
+  for (int v = 0, k = 0; v < n; ++v) {
+    t.tree[v] = k;
+    if (parent[v] < 0) ++k;
+  }
+  t.complete();
+  return t;
+}
+
+// 0 if the schedule is right: every node once, what a node reads was written in an earlier step and is where it looks for it
+static int fault(const LeanTree& t, const LeanSchedule& s, int g0, int g1, int n_slots, bool up) {
+  std::vector<int> step(t.parent.size(), -1), in_slot(n_slots, -1), last(kLeanSchedWaves, -1);
+  int done = 0;
+  for (int st = 0; st < s.steps; ++st) {
+    std::vector<std::pair<int, int>> put;
+    for (int w = 0; w < kLeanSchedWaves; ++w) {
+      const int v = s.item[(size_t)st * kLeanSchedWaves + w];
+      if (v < 0) continue;
+      if (v < g0 || v >= g1 || step[v] >= 0) return 1;
+      const std::vector<int32_t> reads = up ? t.inner[v] : std::vector<int32_t>{v};
+      for (int r : reads) {
+        const int from = up ? r : t.parent[v];
+        if (from < 0) { if (s.slot[v] != kLeanSlotNone) return 2; continue; }
+        if (step[from] < 0 || step[from] >= st) return 3;
+        if (s.slot[r] == kLeanSlotKept) {
+          if (last[w] != from || (!up && t.inner[from][0] != v)) return 4;
+        } else {
+          if (s.slot[r] < 0 || s.slot[r] >= n_slots || in_slot[s.slot[r]] != r) return 5;
+          in_slot[s.slot[r]] = -1;
+        }
+      }
+      const std::vector<int32_t> writes = up ? std::vector<int32_t>{v} : t.inner[v];
+      for (int x : writes)
+        if (s.slot[x] < kLeanSlotKept) put.push_back({s.slot[x], x});
+      step[v] = st;
+      ++done;
+      last[w] = v;
+    }
+    for (auto& p : put) {
+      if (in_slot[p.first] >= 0) return 6;
+      in_slot[p.first] = p.second;
+    }
+  }
+  return done == g1 - g0 ? 0 : 7;
+}
+
+int main() {
+  std::mt19937 rng(3);
+  auto chain = [](int n) { std::vector<int> p(n); for (int v = 0; v < n; ++v) p[v] = v + 1 < n ? v + 1 : -1; return p; };
+  {
+    const LeanTree t = make(chain(40));
+    const LeanSchedule a = lean_schedule_up(t, 0, 40, 20), b = lean_schedule_down(t, 0, 40, 20);
+    int kept = 0;
+    for (int v = 0; v < 40; ++v) kept += (a.slot[v] == kLeanSlotKept) + (b.slot[v] == kLeanSlotKept);
+    std::printf("chain_steps %d\nchain_kept %d\n", a.steps + b.steps, kept);
+  }
+  int faults = 0, refused_many = 0, refused_few = 0, long_ones = 0, handed = 0;
+  for (int i = 0; i < 600; ++i) {
+    const int n = 1 + (int)(rng() % (i % 10 == 0 ? 1500 : 200));
+    const int span = i % 3 == 0 ? n : 1 + (int)(rng() % 12), trees = i % 4 == 0 ? 1 + (int)(rng() % 6) : 1;
+    std::vector<int> p(n), kids(n, 0);
+    for (int v = 0; v < n; ++v) {   // parents with fewer than three children, within `span` of the node
+      p[v] = -1;
+      for (int tries = 0; tries < 40 && p[v] < 0 && v + 1 < n; ++tries) {
+        const int q = std::min(n - 1, v + 1 + (int)(rng() % span));
+        if (kids[q] < 3 && q != v) { p[v] = q; ++kids[q]; }
+      }
+      for (int q = v + 1; q < n && p[v] < 0; ++q)
+        if (kids[q] < 3) { p[v] = q; ++kids[q]; }
+    }
+    // post-order numbering, tree after tree: relabel a forest of `trees` copies
+    std::vector<int> all;
+    {
+      std::vector<std::vector<int>> ch(n);
+      for (int v = 0; v < n; ++v) if (p[v] >= 0) ch[p[v]].push_back(v);
+      std::vector<int> id(n, -1), post;
+      std::vector<std::pair<int, size_t>> st{{n - 1, 0}};
+      while (!st.empty()) {
+        auto& top = st.back();
+        if (top.second < ch[top.first].size()) { const int c = ch[top.first][top.second++]; st.push_back({c, 0}); }
+        else { id[top.first] = (int)post.size(); post.push_back(top.first); st.pop_back(); }
+      }
+      for (int k = 0; k < trees; ++k)
+        for (size_t v = 0; v < post.size(); ++v) all.push_back(p[post[v]] < 0 ? -1 : id[p[post[v]]] + k * (int)post.size());
+    }
+    const LeanTree t = make(all);
+    const int m = (int)all.size();
+    int deep = 0;
+    for (int v = 0; v < m; ++v) deep = std::max(deep, t.depth[v] + 1);
+    for (int n_slots : {79, 24}) {
+      const LeanSchedule a = lean_schedule_up(t, 0, m, n_slots), b = lean_schedule_down(t, 0, m, n_slots);
+      for (const LeanSchedule* s : {&a, &b}) {
+        if (!s->ok) { ++(n_slots == 79 ? refused_many : refused_few); continue; }
+        const int f = fault(t, *s, 0, m, n_slots, s == &a);
+        if (f) { ++faults; std::fprintf(stderr, "tree %d (%d nodes), %d slots, %s: fault %d\n", i, m, n_slots, s == &a ? "up" : "down", f); }
+        if (n_slots == 79 && s->steps > std::max(deep, (m + 15) / 16) * 1.4 + 4) ++long_ones;
+        for (int v = 0; v < m; ++v) handed += s->slot[v] == kLeanSlotKept;
+      }
+    }
+  }
+  std::printf("faults %d\nrefused_many %d\nrefused_few %d\nlong %d\nhanded %d\n", faults, refused_many, refused_few, long_ones, handed > 0);
+  return 0;
+}

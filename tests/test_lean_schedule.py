@@ -1,0 +1,20 @@
+"""The schedules of the lean tree walks (csrc/lean_schedule.hpp): chains handed on in a wave's registers, everything else
+through LDS slots; compiled with g++ and replayed over hand-made and random trees."""
+import os
+import subprocess
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "lvd-pg_amd", "csrc")
+
+
+def test_lean_schedule(tmp_path):
+    exe = str(tmp_path / "lean_schedule")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-I", CSRC, "-o", exe,
+                    os.path.join(HERE, "lean_schedule_test.cpp")], check=True)
+    out = subprocess.run([exe], check=True, capture_output=True, text=True).stdout
+    got = dict((l.split()[0], int(l.split()[1])) for l in out.splitlines())
+    assert got["chain_steps"] == 80 and got["chain_kept"] == 78
+    assert got["faults"] == 0
+    assert got["refused_many"] == 0 and got["refused_few"] <= 5
+    assert got["long"] <= 60   # of 1200, more than 1.4 times the fewest steps there could be
+    assert got["handed"] == 1
