@@ -311,8 +311,9 @@ void HcltCircuit::build_schedules() {
   // field rows of the lean walks (see hclt_walk_lean.hip.hpp) from their own schedule, with the same padding, or none if
   // some node has more operands than the lean kernels hold
   const size_t leaf_stride = (size_t)C_ * K_ * sizeof(float);
-  auto make_lean = [&](const LeanSchedule& sched, bool forward, int stride, std::vector<int32_t>& dst) -> bool {
-    if (!sched.ok || K_ > 32 || lds_slots_ >= (int)kLeanKept || (size_t)V_ * leaf_stride >= ((size_t)1 << 31)) return false;
+  auto make_lean = [&](const LeanScope& in, const LeanSchedule& sched, const std::vector<int32_t>& xid, bool forward, int stride,
+                       std::vector<int32_t>& dst) -> bool {
+    if (!sched.ok || K_ > 32 || lds_slots_ >= (int)kLeanAway || (size_t)V_ * leaf_stride >= ((size_t)1 << 31)) return false;
     const size_t f0 = dst.size();   // (the rows of a further group of trees go behind those of the groups before)
     dst.resize(f0 + (size_t)kLeanFields * kWalkWaves * stride, 0);
     int32_t* f = dst.data() + f0;
@@ -329,7 +330,7 @@ void HcltCircuit::build_schedules() {
           int32_t& turns = at(kLTurns, w, st);
           auto turn = [&](int tile, int byte) {
             const int sl = sched.slot[tile];
-            if (sl < kLeanSlotKept) turns |= ((pass == 0 ? fills[sl] - 1 : fills[sl]++) & 0x7f) << (8 * byte);
+            if (sl < kLeanSlotAway) turns |= ((pass == 0 ? fills[sl] - 1 : fills[sl]++) & 0x7f) << (8 * byte);
           };
           if (lt.inner[n].size() > 3) return false;
           if ((pass == 0) == forward)   // the children's tiles are bytes 1 .. 3, the node's own is byte 0
@@ -357,14 +358,20 @@ void HcltCircuit::build_schedules() {
           ++q;
         }
         at(kLSlots, w, st) = (int32_t)slots;
+        if (par[n] >= 0 && !in.in[par[n]]) at(kLAway, w, st) = xid[n];
+        for (size_t i = lt.inner[n].size(); i-- > 0;) {
+          if (in.in[lt.inner[n][i]]) continue;
+          at(kLAway, w, st) = xid[lt.inner[n][i]];   // (those of one node are numbered in order)
+          at(kLFlags, w, st) |= 4 << i;
+        }
         if (forward) q = 0;
         for (size_t i = 0; i < lc[n].size(); ++i)
           at(kLA1 + q++, w, st) = (int32_t)((size_t)lc[n][i] * leaf_stride) | (forward ? 0 : 1 | (int32_t)((i + 1) << 1));
       }
     // the waits and posts of all waves, replayed: a schedule on which a wave would wait for ever is refused here
-    static_assert(kLeanCheckA1 == kLA1 && kLeanCheckSlots == kLSlots && kLeanCheckTurns == kLTurns &&
-                  kLeanCheckFields == kLeanFields && kLeanCheckWaves == kWalkWaves && kLeanCheckKept == kLeanKept &&
-                  kLeanSlotKept == kLeanKept && kLeanSchedWaves == kWalkWaves, "the lean schedule's headers follow the field rows");
+    static_assert(kLeanCheckA1 == kLA1 && kLeanCheckSlots == kLSlots && kLeanCheckTurns == kLTurns && kLeanCheckFlags == kLFlags &&
+                  kLeanCheckFields == kLeanFields && kLeanCheckWaves == kWalkWaves && kLeanCheckKept == kLeanAway &&
+                  kLeanSlotKept == kLeanKept && kLeanSlotAway == kLeanAway && kLeanSchedWaves == kWalkWaves, "the lean schedule's headers follow the field rows");
     const int stuck = lean_schedule_stuck_at(f, stride, stride, forward, kLeanSlotNone);
     if (stuck >= 0)
       fail(PCM_ERR_STATE, "%s walk schedule is unsound: wave %d would wait for ever in step %d", forward ? "forward" : "backward",
@@ -528,46 +535,94 @@ void HcltCircuit::build_schedules() {
     d_bwd_sched_.upload(sched);
   }
   // ---- lean walks ------------------------------------------------------------------------
-  // A plan: the schedules of a walk in G groups of whole trees, which the kernels take in blockIdx.y.  A tree's
-  // arithmetic does not depend on the group it is walked in, so the results are the same bits under every plan.
-  auto make_plan = [&](const std::vector<std::pair<int, int>>& groups) {
+  // A plan: the schedules of a walk in G groups, which the kernels take in blockIdx.y: groups of whole trees, or the parts of
+  // one tree.  A node's arithmetic does not depend on the group it is walked in, so its results are the same bits under
+  // every plan.  Going up the top of a tree is the last group, going down the first: whoever is waited for comes first.
+  auto make_plan = [&](const std::vector<LeanScope>& scopes, const std::vector<int32_t>& part) {
     std::unique_ptr<LeanPlan> plan(new LeanPlan);
-    plan->n_groups = (int)groups.size();
+    const int G = (int)scopes.size();
+    plan->n_groups = G;
+    std::vector<int32_t> xid(n_inner_, -1);
+    if (!part.empty())
+      for (int n = 0; n < n_inner_; ++n)
+        for (int c : lt.inner[n])
+          if (part[c] != part[n]) xid[c] = plan->n_away++;
     for (const bool forward : {true, false}) {
-      std::vector<LeanSchedule> sched;
+      std::vector<LeanScope> in = scopes;
+      std::vector<LeanSchedule> sched(G);
       int steps = 0;
-      for (const auto& g : groups) {
-        sched.push_back(forward ? lean_schedule_up(lt, g.first, g.second, lds_slots_) : lean_schedule_down(lt, g.first, g.second, lds_slots_));
-        steps = std::max(steps, sched.back().steps);
+      for (int i = 0; i < G; ++i) {
+        const int g = forward ? (i + 1) % G : i;   // (part 0 is the top: going up it is scheduled last, as it runs)
+        if (!part.empty() && (g == 0) == forward) {
+          in[g].release.assign(n_inner_, 0);
+          for (int n = 0; n < n_inner_; ++n)
+            for (int c : lt.inner[n])
+              if (part[c] != part[n] && (forward ? n : c) >= 0) {
+                const int from = forward ? c : n;
+                int32_t& at = in[g].release[forward ? n : c];
+                for (const LeanSchedule& sc : sched)
+                  if (!sc.step_of.empty() && sc.step_of[from] >= 0) at = std::max(at, sc.step_of[from] + 1 + kLeanAwaySteps);
+              }
+        }
+        sched[g] = forward ? lean_schedule_up(lt, in[g], lds_slots_) : lean_schedule_down(lt, in[g], lds_slots_);
+        steps = std::max(steps, sched[g].steps);
       }
       const int stride = steps + 64;   // the shorter groups idle at the end
       std::vector<int32_t> rows;
-      for (const LeanSchedule& sc : sched)
-        if (!make_lean(sc, forward, stride, rows)) return std::unique_ptr<LeanPlan>();
+      for (int i = 0; i < G; ++i) {
+        const int g = forward && !part.empty() ? (i + 1) % G : i;
+        if (!make_lean(in[g], sched[g], xid, forward, stride, rows)) return std::unique_ptr<LeanPlan>();
+      }
       (forward ? plan->n_fwd_steps : plan->n_bwd_steps) = steps;
       (forward ? plan->fwd_stride : plan->bwd_stride) = stride;
       (forward ? plan->fwd : plan->bwd).upload(rows);
     }
     return plan;
   };
-  // In order of their number of groups.  A forest's finer plans are for batches whose slices times the groups of the first
-  // leave most of the device idle (256 examples are 16 slices): a walk takes the plan with the most groups that still gives
-  // every workgroup a compute unit of its own.
+  auto whole_trees = [&](int G) {
+    std::vector<LeanScope> sc;
+    for (const auto& g : make_groups(G)) sc.push_back(LeanScope(lt, g.first, g.second));
+    return sc;
+  };
+  // In order of their number of groups.  The finer plans are for batches whose slices times the groups of the first leave most
+  // of the device idle (256 examples are 16 slices): a walk takes the plan with the most groups that still gives every
+  // workgroup a compute unit of its own.
   plans_.clear();
+  size_t away_tiles = 0, away_parts = 0;
+  int most_nodes = n_inner_;
   if (K_ <= 32) {
-    const std::vector<std::pair<int, int>> groups = make_groups(forest_ ? std::max(1, std::min(4, T_ / 8)) : 1);
-    n_groups_ = (int)groups.size();
-    std::unique_ptr<LeanPlan> plan = make_plan(groups);
+    std::unique_ptr<LeanPlan> plan = make_plan(whole_trees(forest_ ? std::max(1, std::min(4, T_ / 8)) : 1), {});
     if (plan && !forest_ && (plan->n_fwd_steps > n_fwd_steps_ * kLeanStretch || plan->n_bwd_steps > n_bwd_steps_ * kLeanStretch))
       plan.reset();   // (see kLeanStretch)
     if (plan) plans_.push_back(std::move(plan));
-    for (int G = 2 * n_groups_; !plans_.empty() && G <= 4 * n_groups_ && G <= T_ / 4; G *= 2) {
-      const std::vector<std::pair<int, int>> gr = make_groups(G);
-      if ((int)gr.size() <= plans_.back()->n_groups) break;
-      plan = make_plan(gr);
+    for (int G = plans_.empty() ? 0 : 2 * plans_[0]->n_groups; G; G *= 2) {
+      if (forest_ ? G > 4 * plans_[0]->n_groups || G > T_ / 4 : G > kLeanMostParts || n_inner_ < G * kLeanPartNodes) break;
+      std::vector<int32_t> part;
+      std::vector<LeanScope> scopes;
+      if (forest_) {
+        scopes = whole_trees(G);
+      } else {
+        int largest = 0;
+        part = lean_parts(lt, G, &largest);
+        if (largest > 3 * most_nodes / 4) break;   // (the top alone is most of it)
+        most_nodes = largest;
+        for (int g = 0; g < G; ++g) scopes.push_back(LeanScope(part, g));
+      }
+      if ((int)scopes.size() <= plans_.back()->n_groups) break;
+      plan = make_plan(scopes, part);
       if (!plan) break;
+      const size_t slices = (size_t)n_cus_ / G;
+      away_tiles = std::max(away_tiles, (size_t)plan->n_away * slices);
+      away_parts = std::max(away_parts, (size_t)plan->n_groups * slices);
       plans_.push_back(std::move(plan));
     }
+  }
+  if (away_parts) {
+    d_away_tiles_.alloc(std::max<size_t>(away_tiles, 1) * kSlice * K_);
+    d_away_sums_.alloc(away_parts * kSlice);
+    d_away_flags_.alloc(away_tiles + away_parts);
+    d_away_flags_.zero();
+    away_tiles_ = away_tiles;
   }
   // ---- statistics: the static operands of every node ------------------------------------
   {
@@ -1217,8 +1272,7 @@ void HcltCircuit::stage_batch(const BatchRef& b, bool tiles) {
   check_launch("pack_x");
 }
 
-// The finer plan a batch of `nslices` slices walks a forest with, or null for the plan of the constructor: the
-// most groups whose workgroups still get a compute unit each.
+// The plan a batch of `nslices` slices is walked with: the most groups whose workgroups still get a compute unit each.
 const HcltCircuit::LeanPlan* HcltCircuit::lean_plan(int nslices) const {
   const LeanPlan* best = plans_.front().get();
   for (const auto& p : plans_)
@@ -1234,6 +1288,10 @@ bool HcltCircuit::lean_fits(int batch, int keep) const {
   return lean_ && !force_general_walks_ && (size_t)(n_inner_ + 1) * per_node * 4 < ((size_t)1 << 31);
 }
 
+LeanAway HcltCircuit::away() const {
+  return {d_away_tiles_.p, d_away_flags_.p, d_away_sums_.p, d_away_flags_.p + away_tiles_};
+}
+
 void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
   const size_t lds = (size_t)lds_slots_ * kSlice * K_ * sizeof(float);
   auto launch = [&](auto kernel) {
@@ -1247,7 +1305,7 @@ void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
       const LeanPlan* lp = lean_plan(d.nslices);
       PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, lp->fwd.p, lp->fwd_stride,
-                       lp->n_fwd_steps, d_ll, lds_slots_);
+                       lp->n_fwd_steps, d_ll, lds_slots_, away());
     };
     PCM_DISPATCH_LEAN_K(K_, {
       if (keep == kKeepAll) launch_lean(&hclt_forward_lean_kernel<KK, kKeepAll>);
@@ -1275,7 +1333,7 @@ void HcltCircuit::run_backward(const HcltDev& d) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
       const LeanPlan* lp = lean_plan(d.nslices);
       PCM_LAUNCH_PHASE(1, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, lp->bwd.p, lp->bwd_stride,
-                       lp->n_bwd_steps, lds_slots_);
+                       lp->n_bwd_steps, lds_slots_, away());
     };
     PCM_DISPATCH_LEAN_K(K_, {
       if (H_ > 0) launch_lean(&hclt_backward_lean_kernel<KK, true>); else launch_lean(&hclt_backward_lean_kernel<KK, false>);
@@ -1655,6 +1713,7 @@ void HcltCircuit::check_walks() {
     *walk_err_ = 0;
     if (d_walk_void_.p) (void)hipMemsetAsync(d_walk_void_.p, 0, sizeof(int32_t), stream);
     if (d_stat_claim_.p) (void)hipMemsetAsync(d_stat_claim_.p, 0, sizeof(uint32_t), stream);
+    if (d_away_flags_.p) (void)hipMemsetAsync(d_away_flags_.p, 0, d_away_flags_.n * sizeof(uint32_t), stream);
     have_flows_ = false;
     fail(PCM_ERR_HIP, "a tree-walk kernel gave up waiting for a tile of an earlier step; the results of that pass are void");
   }

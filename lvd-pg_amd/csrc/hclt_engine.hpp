@@ -32,6 +32,11 @@ enum { kKeepNone = 0, kKeepRoots, kKeepAll };   // what the lean forward walk le
 // take 1.45 times as long per EM step of as many steps (2.40 against 1.65 ms on a 3072-variable Chow-Liu tree at 4096
 // examples).
 constexpr double kLeanStretch = 1.4;
+// One tree over several workgroups (hclt_walk_lean.hip.hpp): up to kLeanMostParts parts of at least kLeanPartNodes nodes on
+// average, while the largest part goes on shrinking by a quarter.  Below that the crossings cost what the parts gain: 153
+// nodes at 512 examples forward 42 us in one part, 50 in six; 632 nodes 97 in one, 95 in four (backward 125 and 107).  A tile
+// from another workgroup is expected kLeanAwaySteps steps after the step it is sent in.
+constexpr int kLeanMostParts = 16, kLeanPartNodes = 80, kLeanAwaySteps = 4;
 constexpr int kPre = 3;          // static operand tiles a wave requests one step ahead
 
 struct HcltNode {     // one non-leaf tree node, device-resident
@@ -141,6 +146,8 @@ struct HcltDev {
     default: fail(PCM_ERR_UNSUPPORTED, "hidden size %d not supported by the block engine", K_); \
   }
 
+struct LeanAway;
+
 class HcltCircuit : public pcm_circuit {
  public:
   // num_heads > 0: a multi-head circuit, num_heads sum nodes over the root's K products instead of one.
@@ -231,14 +238,20 @@ class HcltCircuit : public pcm_circuit {
   bool forest_ = false;
   int T_ = 1;                      // trees (1 unless a forest)
   int n_groups_ = 1;               // groups of trees the walk kernels take side by side (blockIdx.y)
-  // schedules of the lean walks, in one group of trees or more (a forest's finer plans are for batches whose slices do not
-  // fill the device), fewest groups first
+  // schedules of the lean walks, in one group of trees or more, or one tree in several parts (the finer plans are for batches
+  // whose slices do not fill the device), fewest groups first
   struct LeanPlan {
-    int n_groups = 1, n_fwd_steps = 0, fwd_stride = 0, n_bwd_steps = 0, bwd_stride = 0;
+    int n_groups = 1, n_away = 0, n_fwd_steps = 0, fwd_stride = 0, n_bwd_steps = 0, bwd_stride = 0;
     DevBuf<int32_t> fwd, bwd;
   };
   std::vector<std::unique_ptr<LeanPlan>> plans_;   // empty: the lean kernels do not take this tree
   const LeanPlan* lean_plan(int nslices) const;
+  // what crosses the parts of a tree: for every plan with as many slices as it is taken for
+  DevBuf<float> d_away_tiles_;
+  DevBuf<double> d_away_sums_;
+  DevBuf<uint32_t> d_away_flags_;   // zero between launches
+  size_t away_tiles_ = 0;
+  LeanAway away() const;
   std::vector<int32_t> roots_;     // root variable of every tree, in variable order
   std::vector<int32_t> tree_of_inner_;   // tree of every inner node
   // inner nodes of the caller's tree, and every node's index among them (auxiliary nodes keep the post-order of the

@@ -39,10 +39,12 @@ namespace pcm {
 //   kLSlots forward: out slot | child slots << 8, 16, 24 (0xff: none); backward: slot holding
 //           this node's ratio tile | slots of the inner children's ratio tiles << 8, 16, 24
 //           (0xff: that child is a leaf or absent); kLeanKept: in registers
-//   kLFlags bit 0: root; bit 1: root of a multi-head circuit
+//   kLFlags bit 0: root; bit 1: root of a multi-head circuit; bits 2..4, backward: child 1..3 is away
 //   kLTurns which use of its slot a tile is, modulo 128, in the byte layout of kLSlots: a slot passes through
 //           the states 2t (free for its t-th tile), 2t + 1 (that tile is there), 2t + 2 (read, free again)
-enum { kLW = 0, kLA0, kLA1, kLA2, kLA3, kLNode, kLSlots, kLFlags, kLTurns, kLeanFields };
+//   kLAway  place in the exchange of this node's tile, or of the first of its children's, that crosses workgroups (below)
+enum { kLW = 0, kLA0, kLA1, kLA2, kLA3, kLNode, kLSlots, kLFlags, kLTurns, kLAway, kLeanFields };
+constexpr uint32_t kLeanAway = 0xfd;       // in place of a slot: the tile comes from or goes to another workgroup
 constexpr uint32_t kLeanKept = 0xfe;       // in place of a slot: the tile stays in the registers of the wave (one that stays nowhere: 0xff)
 constexpr int kLeanFlagWords = 256;        // one state word per LDS slot, behind the slots
 constexpr int kLeanSpinLimit = 1 << 22;    // polls before a wave gives up on a tile (never reached by a sound schedule)
@@ -141,6 +143,73 @@ __device__ __forceinline__ void lean_post(unsigned* state, unsigned value) {
   __hip_atomic_store(state, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// ---- a tree over several workgroups ----------------------------------------------------------
+// A batch of few slices leaves most compute units idle while one of them per slice walks the whole tree.  So a single tree
+// is also scheduled in 2, 4, 8 .. parts (lean_parts), blockIdx.y of the walk: the top of the tree and, dealt to the parts,
+// the subtrees below it.  A tile that crosses goes through memory, once on the way up or down, with a flag per (tile, slice)
+// that its one reader puts back to zero, so that a launch leaves the flags as it found them (also one that a graph replays).
+// The data is written and read with device-scope accesses of its own, which pass the L2s of the eight dies; a release or
+// acquire fence would write back or drop a whole L2 each time.  Only the top waits going up, only the others going down,
+// and whoever is waited for comes first in the grid: it does not depend on a workgroup that is dispatched later.  The waits
+// are bounded like those for LDS tiles.  3072 variables, K = 32, 512 examples: forward 336 -> 194 us, backward 444 -> 235 in
+// eight parts; 1024 examples 338 -> 201 and 480 -> 271 in four; 784 variables, 512 examples: 97 -> 97 and 125 -> 107.
+struct LeanAway {
+  float* tiles;        // [tile][slice][16 * K]
+  unsigned* flags;     // [tile][slice]
+  double* sums;        // [part][Bp] a part's share of the log-likelihood
+  unsigned* sum_flags; // [part][slice]
+};
+
+__device__ __forceinline__ void away_wait(unsigned* flag, const HcltDev& d) {
+  int polls = 0;
+  while (__builtin_amdgcn_readfirstlane((int)__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 1) {
+    if (++polls > kLeanSpinLimit) {
+      if ((threadIdx.x & 63) == 0) {
+        __hip_atomic_store(d.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(d.err_dev, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      break;
+    }
+    __builtin_amdgcn_s_sleep(2);
+  }
+  asm volatile("" ::: "memory");   // (what the flag announces is read behind this)
+}
+
+// everything this wave has written or read so far is through before the flag changes
+__device__ __forceinline__ void away_flag(unsigned* flag, unsigned value) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if ((threadIdx.x & 63) == 0) __hip_atomic_store(flag, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <int K>
+__device__ __forceinline__ void away_put(const LeanAway& x, const HcltDev& d, int tile, int slice, int lane, const Tile<K>& t) {
+  const size_t at = (size_t)tile * d.nslices + slice;
+  unsigned long long* p = reinterpret_cast<unsigned long long*>(x.tiles + at * (kSlice * K)) + lane * 2;
+#pragma unroll
+  for (int kt = 0; kt < K / 16; ++kt)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      __hip_atomic_store(p + kt * 128 + h, __builtin_bit_cast(unsigned long long, make_float2(t.v[kt][2 * h], t.v[kt][2 * h + 1])),
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  away_flag(x.flags + at, 1u);
+}
+
+template <int K>
+__device__ __forceinline__ void away_get(const LeanAway& x, const HcltDev& d, int tile, int slice, int lane, Tile<K>& t) {
+  const size_t at = (size_t)tile * d.nslices + slice;
+  away_wait(x.flags + at, d);
+  unsigned long long* p = reinterpret_cast<unsigned long long*>(x.tiles + at * (kSlice * K)) + lane * 2;
+#pragma unroll
+  for (int kt = 0; kt < K / 16; ++kt)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float2 v = __builtin_bit_cast(float2, __hip_atomic_load(p + kt * 128 + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      t.v[kt][2 * h] = v.x;
+      t.v[kt][2 * h + 1] = v.y;
+    }
+  away_flag(x.flags + at, 0u);
+}
+
 // ---- forward ------------------------------------------------------------------------------
 // A node's value is kept in two parts: the tile holds O'_v[k] = log S_v[k] = log sum_j W[k,j] exp(Z'_v[j] - m_v), numbers
 // of order one, and the row of maxima holds m_v = max_j Z'_v[j], where Z'_v is the sum of the node's leaf rows and of its
@@ -161,7 +230,7 @@ __device__ __forceinline__ void lean_post(unsigned* state, unsigned value) {
 // 3072 variables at 4096 examples, where the stores of the tiles count, 390 -> 384.
 template <int K, int kKeep>
 __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
-    HcltDev d, const int32_t* __restrict__ fields, int stride, int n_steps, float* __restrict__ ll_out, int n_slots) {
+    HcltDev d, const int32_t* __restrict__ fields, int stride, int n_steps, float* __restrict__ ll_out, int n_slots, LeanAway away) {
   extern __shared__ float lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -232,12 +301,17 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
     if (node != d.n_inner) {   // (idle steps only keep the requests going)
       // (3) inner children, from LDS or, the one this wave computed last, from registers; logsumexp through the matrix cores
       const uint32_t slots = (uint32_t)lean_get(sc, kLSlots, s), turns = (uint32_t)lean_get(sc, kLTurns, s);
+      int next_away = lean_get(sc, kLAway, s);
 #pragma unroll
       for (int c = 1; c <= 3; ++c) {
         const uint32_t sl = (slots >> (8 * c)) & 0xffu, tn = (turns >> (8 * c)) & 0x7fu;
         if (sl == 0xffu) break;
         if (sl == kLeanKept) {
           tile_add<K>(z, o);
+        } else if (sl == kLeanAway) {
+          Tile<K> t;
+          away_get<K>(away, d, next_away++, slice, lane, t);
+          tile_add<K>(z, t);
         } else {
           lean_wait(state + sl, (2 * tn + 1) & 0xffu, d);
           Tile<K> t;
@@ -255,10 +329,12 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
         for (int i = 0; i < 4; ++i) o.v[kt][i] = __builtin_amdgcn_logf(o.v[kt][i]) * kLn2;
       // hand the tile on first (the root's, and one whose reader is this wave's next node, go nowhere)
       const uint32_t so = slots & 0xffu, tn = turns & 0x7fu;
-      if (so < kLeanKept) {
+      if (so < kLeanAway) {
         lean_wait(state + so, (2 * tn) & 0xffu, d);
         lds_tile_store<K>(lds, (int)so, lane, o);
         lean_post(state + so, (2 * tn + 1) & 0xffu);
+      } else if (so == kLeanAway) {
+        away_put<K>(away, d, lean_get(sc, kLAway, s), slice, lane, o);
       }
       msum += (double)m;
       const bool root = (lean_get(sc, kLFlags, s) & 1) != 0;
@@ -300,11 +376,24 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
     if (root_here) top[lane] = ll;
   }
   __syncthreads();
-  if (wave == 0 && lane < 16 && bcol < d.B) {
+  if (wave == 0) {
     double tot = 0.0;
 #pragma unroll
-    for (int w = 0; w < kWalkWaves; ++w) tot += part[w * 16 + lane];
-    ll_out[bcol] = (float)(tot + (double)top[lane]);
+    for (int w = 0; w < kWalkWaves; ++w) tot += part[w * 16 + (lane & 15)];
+    // (a tree over several workgroups: the top, which comes last, adds up the shares of the others in order)
+    const int last = (int)gridDim.y - 1;
+    if ((int)blockIdx.y < last) {
+      if (lane < 16) __hip_atomic_store(away.sums + (size_t)blockIdx.y * d.Bp + bcol, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      away_flag(away.sum_flags + (size_t)blockIdx.y * d.nslices + slice, 1u);
+    } else {
+      for (int g = 0; g < last; ++g) {
+        unsigned* flag = away.sum_flags + (size_t)g * d.nslices + slice;
+        away_wait(flag, d);
+        tot += __hip_atomic_load(away.sums + (size_t)g * d.Bp + bcol, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        away_flag(flag, 0u);
+      }
+      if (lane < 16 && bcol < d.B) ll_out[bcol] = (float)(tot + (double)top[lane]);
+    }
   }
 }
 
@@ -323,7 +412,7 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
 // requested whether wanted or not; 3072 at 4096 stays at 625: 3.2 GB at 5.2 TB/s.
 template <int K, bool kHeads>
 __global__ __launch_bounds__(kWalkWaves * 64) void hclt_backward_lean_kernel(
-    HcltDev d, const int32_t* __restrict__ fields, int stride, int n_steps, int n_slots) {
+    HcltDev d, const int32_t* __restrict__ fields, int stride, int n_steps, int n_slots, LeanAway away) {
   extern __shared__ float lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -374,7 +463,7 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_backward_lean_kernel(
     lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, 1), wB);
     __builtin_amdgcn_sched_barrier(0);
   }
-  Tile<K> r;   // the ratio tile of the node under way; behind a step, that of its first child, which comes next in this wave
+  Tile<K> r;   // the ratio tile of the node under way; behind a step, that of its first child, which comes next in this wave (or is away)
   tile_zero<K>(r);
 
   // exponent tile of inner child `own` among the landed operands: the other operands minus m_v,
@@ -426,7 +515,9 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_backward_lean_kernel(
     if (node != d.n_inner) {   // (idle steps only keep the requests going)
       // (3) this node's ratio tile: in registers from the step before, or left in LDS by the parent
       const uint32_t so = slots & 0xffu;
-      if (so < kLeanKept) {
+      if (so == kLeanAway) {
+        away_get<K>(away, d, lean_get(sc, kLAway, s), slice, lane, r);
+      } else if (so < kLeanAway) {
         lean_wait(state + so, (2 * (turns & 0x7fu) + 1) & 0xffu, d);
         lds_tile_load<K>(lds, (int)so, lane, r);
         lean_post(state + so, (2 * (turns & 0x7fu) + 2) & 0xffu);
@@ -454,17 +545,26 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_backward_lean_kernel(
 #pragma unroll
             for (int i = 0; i < 4; ++i) rc.v[kt][i] = t.v[kt][i] * fminf(__builtin_amdgcn_exp2f(x.v[kt][i]), kFlowRatioCap);
         };
+        int next_away = lean_get(sc, kLAway, s);
+        const bool first_away = (fl & 4) != 0;
+        if (first_away) ++next_away;
         auto hand_on = [&](int c) {
           const uint32_t sl = (slots >> (8 * c)) & 0xffu;
           Tile<K> x;
           lds_tile_load<K>(lds, (int)sl, lane, x);
           ratio(x, x);
-          lds_tile_store<K>(lds, (int)sl, lane, x);
-          lean_post(state + sl, (2 * ((turns >> (8 * c)) & 0x7fu) + 1) & 0xffu);
+          if (fl & (2 << c)) {   // away: the slot was only to work in
+            away_put<K>(away, d, next_away++, slice, lane, x);
+            lean_post(state + sl, (2 * ((turns >> (8 * c)) & 0x7fu) + 2) & 0xffu);
+          } else {
+            lds_tile_store<K>(lds, (int)sl, lane, x);
+            lean_post(state + sl, (2 * ((turns >> (8 * c)) & 0x7fu) + 1) & 0xffu);
+          }
         };
         if (in2) hand_on(2);
         if (in3) hand_on(3);
         ratio(X1, r);
+        if (first_away) away_put<K>(away, d, lean_get(sc, kLAway, s), slice, lane, r);
       }
     }
     __builtin_amdgcn_sched_barrier(0);

@@ -23,6 +23,7 @@ namespace pcm {
 constexpr int kLeanSchedWaves = 16;
 constexpr int32_t kLeanSlotKept = 0xfe;   // the tile stays in the registers of the wave
 constexpr int32_t kLeanSlotNone = 0xff;   // nobody hands this tile on (a root)
+constexpr int32_t kLeanSlotAway = 0xfd;   // the tile goes to or comes from another workgroup
 
 struct LeanTree {   // inner nodes, children before their parents
   std::vector<int32_t> parent;               // -1: a root
@@ -58,9 +59,29 @@ struct LeanTree {   // inner nodes, children before their parents
   }
 };
 
+// The nodes one workgroup walks: whole trees, or a part of one whose other parts other workgroups walk.
+struct LeanScope {
+  std::vector<int32_t> nodes;     // in ascending order
+  std::vector<char> in;           // by node
+  std::vector<int32_t> release;   // by node: the step before which a tile from another part is not to be expected; may be empty
+
+  LeanScope(const LeanTree& t, int g0, int g1) : in(t.parent.size(), 0) {
+    for (int v = g0; v < g1; ++v) add(v);
+  }
+  LeanScope(const std::vector<int32_t>& part, int g) : in(part.size(), 0) {
+    for (int v = 0; v < (int)part.size(); ++v)
+      if (part[v] == g) add(v);
+  }
+  void add(int v) { nodes.push_back(v); in[v] = 1; }
+  int ready_at(int v) const { return release.empty() ? 0 : release[v]; }
+};
+
 struct LeanSchedule {
   std::vector<int32_t> item;   // [steps][16 waves] node, -1: idle
-  std::vector<int32_t> slot;   // by node: the slot of its tile (going down: of its ratio tile), kLeanSlotKept or kLeanSlotNone
+  // by node: the slot of its tile (going down: of its ratio tile), kLeanSlotKept, kLeanSlotNone or kLeanSlotAway.  Going down,
+  // a node's second and third child that are away have a slot too: their parent works there before it sends the tile.
+  std::vector<int32_t> slot;
+  std::vector<int32_t> step_of;   // by node
   int steps = 0;
   bool ok = false;             // false: the slots do not do
 };
@@ -87,13 +108,13 @@ struct LeanHeap {
 };
 
 // The slot that has been free longest is taken first: a wave then hardly ever waits for the reader of the tile before.
-inline bool lean_place(const LeanTree& t, LeanSchedule& s, int n_slots, bool up) {
+inline bool lean_place(const LeanTree& t, const LeanScope& in, LeanSchedule& s, int n_slots, bool up) {
   std::vector<int32_t> ring(n_slots), freed;   // the free slots, first in first out
   for (int i = 0; i < n_slots; ++i) ring[i] = i;
   size_t head = 0;
   int n_free = n_slots;
   auto take = [&](int tile) {
-    if (s.slot[tile] >= 0) return true;   // (kept, or nobody's)
+    if (s.slot[tile] >= 0) return true;   // (kept, away or nobody's)
     if (!n_free) return false;
     s.slot[tile] = ring[head];
     head = (head + 1) % n_slots;
@@ -101,7 +122,7 @@ inline bool lean_place(const LeanTree& t, LeanSchedule& s, int n_slots, bool up)
     return true;
   };
   auto free_after = [&](int tile) {
-    if (s.slot[tile] < kLeanSlotKept) freed.push_back(s.slot[tile]);
+    if (s.slot[tile] >= 0 && s.slot[tile] < kLeanSlotAway) freed.push_back(s.slot[tile]);
   };
   for (int st = 0; st < s.steps; ++st) {
     freed.clear();
@@ -109,12 +130,15 @@ inline bool lean_place(const LeanTree& t, LeanSchedule& s, int n_slots, bool up)
       const int n = s.item[(size_t)st * kLeanSchedWaves + w];
       if (n < 0) continue;
       if (up) {
-        for (int c : t.inner[n]) free_after(c);
+        for (int c : t.inner[n])
+          if (in.in[c]) free_after(c);
         if (!take(n)) return false;
       } else {
         free_after(n);
-        for (int c : t.inner[n])
+        for (int c : t.inner[n]) {
           if (!take(c)) return false;
+          if (!in.in[c]) free_after(c);   // (a slot to work in)
+        }
       }
     }
     for (int x : freed) ring[(head + n_free++) % n_slots] = x;
@@ -122,28 +146,41 @@ inline bool lean_place(const LeanTree& t, LeanSchedule& s, int n_slots, bool up)
   return true;
 }
 
-// Nodes g0 .. g1 - 1 (whole trees) from the leaves up.
-inline LeanSchedule lean_schedule_up(const LeanTree& t, int g0, int g1, int n_slots) {
+// From the leaves up.
+inline LeanSchedule lean_schedule_up(const LeanTree& t, const LeanScope& in, int n_slots) {
   constexpr int W = kLeanSchedWaves;
   LeanSchedule s;
   s.slot.assign(t.parent.size(), -1);
+  s.step_of.assign(t.parent.size(), -1);
   std::vector<int32_t> pending(t.parent.size(), 0), last(W, -1);
-  std::vector<char> waiting(t.parent.size(), 0);
-  // [0]: nodes without inner children, [1]: the others; the most urgent first (a forest: earlier trees first) / in the order
-  // that finishes subtrees
-  LeanHeap by_depth[2], by_order[2];
+  std::vector<char> waiting(t.parent.size(), 0), all(t.parent.size(), 1), starts(t.parent.size(), 0);
+  // [0]: nodes without inner children here, [1]: the others; the most urgent first (a forest: earlier trees first) / in the
+  // order that finishes subtrees; `later`: nodes that would be ready but for a tile from another part
+  LeanHeap by_depth[2], by_order[2], later;
   auto add = [&](int v) {
-    const int kind = t.inner[v].empty() ? 0 : 1;
+    if (in.ready_at(v) > s.steps) return later.push(in.ready_at(v), 0, v);
+    const int kind = starts[v] ? 0 : 1;
     waiting[v] = 1;
     by_depth[kind].push(t.tree[v], -t.depth[v], v);
     by_order[kind].push(t.order[v], 0, v);
   };
-  for (int v = g0; v < g1; ++v) {
-    pending[v] = (int32_t)t.inner[v].size();
-    if (!pending[v]) add(v);
+  for (int v : in.nodes) {
+    for (int c : t.inner[v]) {
+      pending[v] += in.in[c];
+      if (!in.in[c]) s.slot[c] = kLeanSlotAway;
+    }
+    starts[v] = pending[v] == 0;
+    if (starts[v]) add(v);
+    if (t.parent[v] < 0) s.slot[v] = kLeanSlotNone;
+    else if (!in.in[t.parent[v]]) s.slot[v] = kLeanSlotAway;
   }
   int live = 0;   // tiles nobody has taken yet, those in registers among them
-  for (int done = 0; done < g1 - g0;) {
+  for (size_t done = 0; done < in.nodes.size(); ++s.steps) {
+    for (int v; (v = later.top(all)) >= 0 && in.ready_at(v) <= s.steps;) {
+      std::pop_heap(later.e.begin(), later.e.end());
+      later.e.pop_back();
+      add(v);
+    }
     std::vector<int32_t> now(W, -1);
     int taken = 0;
     for (int w = 0; w < W; ++w) {   // chains first; of several children that could hand on in registers the first does
@@ -173,66 +210,85 @@ inline LeanSchedule lean_schedule_up(const LeanTree& t, int g0, int g1, int n_sl
       waiting[pick] = 0;
       ++taken;
     }
-    if (!taken) return s;   // only nodes that need a slot, and none is left
+    if (!taken && later.top(all) < 0) {
+      // tiles wait for a subtree that has not begun (its nodes came late): the deepest node may use the slots left free
+      const int start = by_depth[0].top(waiting);
+      if (start < 0 || live + 2 > n_slots) return s;
+      now[0] = start;
+      waiting[start] = 0;
+    }
     for (int w = 0; w < W; ++w) {
       const int v = now[w];
       if (v < 0) continue;
       for (int c : t.inner[v]) {
+        if (!in.in[c]) continue;
         if (last[w] == c) s.slot[c] = kLeanSlotKept;
         --live;
       }
-      if (t.parent[v] >= 0) ++live; else s.slot[v] = kLeanSlotNone;
+      if (s.slot[v] != kLeanSlotNone && s.slot[v] != kLeanSlotAway) ++live;
     }
     for (int w = 0; w < W; ++w) {
       const int v = now[w];
       s.item.push_back(v);
       if (v < 0) continue;
       last[w] = v;
+      s.step_of[v] = s.steps;
       ++done;
       const int p = t.parent[v];
-      if (p >= 0 && --pending[p] == 0) add(p);
+      if (p >= 0 && in.in[p] && --pending[p] == 0) add(p);
     }
-    ++s.steps;
   }
-  s.ok = lean_place(t, s, n_slots, true);
+  s.ok = lean_place(t, in, s, n_slots, true);
   return s;
 }
 
-// Nodes g0 .. g1 - 1 (whole trees) from the roots down.  A node's first child always follows it on its wave, and its other
-// children take a slot each.  A chain that finds none waits, its tile in registers; `careful`: so that not all waves end up
-// waiting, a chain is only started if the slots do for what it and the chains under way (but the greediest) still take.
-inline LeanSchedule lean_schedule_down(const LeanTree& t, int g0, int g1, int n_slots, bool careful) {
+// From the roots down.  A node's first child always follows it on its wave (unless it is away), and its other children take
+// a slot each.  A chain that finds none waits, its tile in registers; `careful`: so that not all waves end up waiting, a
+// chain is only started if the slots do for what it and the chains under way (but the greediest) still take.
+inline LeanSchedule lean_schedule_down(const LeanTree& t, const LeanScope& in, int n_slots, bool careful) {
   constexpr int W = kLeanSchedWaves;
   LeanSchedule s;
   s.slot.assign(t.parent.size(), -1);
+  s.step_of.assign(t.parent.size(), -1);
   std::vector<int32_t> last(W, -1), rest(t.parent.size(), 0);
-  std::vector<char> waiting(t.parent.size(), 0);
-  auto extra = [&](int v) { return std::max(0, (int)t.inner[v].size() - 1); };   // slots a node's children take
-  for (int v = g0; v < g1; ++v) rest[v] = extra(v) + (t.inner[v].empty() ? 0 : rest[t.inner[v][0]]);   // ... a chain's
-  LeanHeap by_chain, by_size;   // longest chain first (a forest: earlier trees first) / those soonest gone again first
+  std::vector<char> waiting(t.parent.size(), 0), all(t.parent.size(), 1);
+  auto next = [&](int v) { return t.inner[v].empty() || !in.in[t.inner[v][0]] ? -1 : t.inner[v][0]; };   // on the same wave
+  std::vector<int32_t> extra(t.parent.size(), 0);   // slots a node's children take
+  for (int v : in.nodes) {
+    for (size_t i = 1; i < t.inner[v].size(); ++i) extra[v] += in.in[t.inner[v][i]];
+    rest[v] = extra[v] + (next(v) < 0 ? 0 : rest[next(v)]);   // ... a chain's
+    if (!t.inner[v].empty() && next(v) < 0) s.slot[t.inner[v][0]] = kLeanSlotAway;
+  }
+  LeanHeap by_chain, by_size, later;   // longest chain first (a forest: earlier trees first) / those soonest gone again first
   auto add = [&](int v) {
+    if (in.ready_at(v) > s.steps) return later.push(in.ready_at(v), 0, v);
     waiting[v] = 1;
     by_chain.push(t.tree[v], -t.chain[v], v);
     by_size.push(t.below[v], -s.steps, v);
   };
-  for (int v = g0; v < g1; ++v)
-    if (t.parent[v] < 0) {
+  for (int v : in.nodes)
+    if (t.parent[v] < 0 || !in.in[t.parent[v]]) {
       add(v);
-      s.slot[v] = kLeanSlotNone;
+      s.slot[v] = t.parent[v] < 0 ? kLeanSlotNone : kLeanSlotAway;
     }
   int live = 0;
-  for (int done = 0; done < g1 - g0; ++s.steps) {
+  for (size_t done = 0; done < in.nodes.size(); ++s.steps) {
+    for (int v; (v = later.top(all)) >= 0 && in.ready_at(v) <= s.steps;) {
+      std::pop_heap(later.e.begin(), later.e.end());
+      later.e.pop_back();
+      add(v);
+    }
     std::vector<int32_t> now(W, -1);
     std::vector<char> held(W, 0);
     int taken = 0, freed = 0, open = 0, widest = 0;
     for (int w = 0; w < W; ++w) {
-      if (last[w] < 0 || t.inner[last[w]].empty()) continue;
+      const int c = last[w] < 0 ? -1 : next(last[w]);
+      if (c < 0) continue;
       held[w] = 1;
-      const int c = t.inner[last[w]][0];
       int left = rest[c];
-      if (live + extra(c) <= n_slots) {
-        live += extra(c);
-        left -= extra(c);
+      if (live + extra[c] <= n_slots) {
+        live += extra[c];
+        left -= extra[c];
         now[w] = c;
         s.slot[c] = kLeanSlotKept;
         ++taken;
@@ -245,36 +301,66 @@ inline LeanSchedule lean_schedule_down(const LeanTree& t, int g0, int g1, int n_
       last[w] = -1;
       const int v = (2 * live <= n_slots && !careful ? by_chain : by_size).top(waiting);
       if (v < 0) continue;
-      const int left = rest[v] - extra(v);
+      const int left = rest[v] - extra[v];
       const bool fits = rest[v] == 0 || (careful ? live + open + rest[v] - std::max(widest, left) <= n_slots
-                                                 : live + extra(v) <= n_slots - W / 2);
+                                                 : live + extra[v] <= n_slots - W / 2);
       if (!fits) continue;
       waiting[v] = 0;
-      live += extra(v);
+      live += extra[v];
       open += left;
       widest = std::max(widest, left);
-      if (t.parent[v] >= 0) ++freed;   // its slot is free again after the step
+      if (s.slot[v] == -1) ++freed;   // its slot is free again after the step
       now[w] = v;
       ++taken;
     }
-    if (!taken) return s;
+    if (!taken && later.top(all) < 0) return s;
     live -= freed;
     for (int w = 0; w < W; ++w) {
       const int v = now[w];
       s.item.push_back(v);
       if (v < 0) continue;
       last[w] = v;
+      s.step_of[v] = s.steps;
       ++done;
-      for (size_t i = 1; i < t.inner[v].size(); ++i) add(t.inner[v][i]);
+      for (size_t i = 1; i < t.inner[v].size(); ++i)
+        if (in.in[t.inner[v][i]]) add(t.inner[v][i]);
     }
   }
-  s.ok = lean_place(t, s, n_slots, false);
+  s.ok = lean_place(t, in, s, n_slots, false);
   return s;
 }
 
-inline LeanSchedule lean_schedule_down(const LeanTree& t, int g0, int g1, int n_slots) {
-  LeanSchedule s = lean_schedule_down(t, g0, g1, n_slots, false);
-  return s.ok ? s : lean_schedule_down(t, g0, g1, n_slots, true);
+inline LeanSchedule lean_schedule_down(const LeanTree& t, const LeanScope& in, int n_slots) {
+  LeanSchedule s = lean_schedule_down(t, in, n_slots, false);
+  return s.ok ? s : lean_schedule_down(t, in, n_slots, true);
+}
+
+// One tree cut for `G` workgroups: part 0 has the top of the tree, everything more than 1 / (2 G) of the nodes hang from,
+// and the subtrees below it are dealt to the parts, largest first, each to the part with the fewest nodes.  So a tile
+// crosses at most once on its way up or down, and only part 0 waits (going up) or is waited for (going down).  A subtree of
+// fewer than kLeanCutNodes nodes is not worth the crossing and stays with the top.  `*largest`: nodes of the largest part.
+constexpr int kLeanCutNodes = 6;
+inline std::vector<int32_t> lean_parts(const LeanTree& t, int G, int* largest) {
+  const int n = (int)t.parent.size(), most = std::max(kLeanCutNodes, n / (2 * G));
+  std::vector<int32_t> part(n, 0), load(G, 0), cut;
+  for (int v = 0; v < n; ++v) {
+    const bool small = t.below[v] + 1 <= most;
+    if (!small || t.parent[v] < 0) ++load[0];
+    else if (t.below[t.parent[v]] + 1 > most || t.parent[t.parent[v]] < 0) {
+      if (t.below[v] + 1 < kLeanCutNodes) load[0] += t.below[v] + 1;
+      else cut.push_back(v);
+    }
+  }
+  std::stable_sort(cut.begin(), cut.end(), [&](int a, int b) { return t.below[a] > t.below[b]; });
+  for (int v : cut) {
+    const int g = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+    part[v] = g;
+    load[g] += t.below[v] + 1;
+  }
+  for (int v = n - 1; v >= 0; --v)   // (parents have higher numbers)
+    if (t.parent[v] >= 0 && part[v] == 0) part[v] = part[t.parent[v]];
+  *largest = *std::max_element(load.begin(), load.end());
+  return part;
 }
 
 }  // namespace pcm

@@ -26,20 +26,23 @@ static LeanTree make(const std::vector<int>& parent) {
   return t;
 }
 
-// 0 if the schedule is right: every node once, what a node reads was written in an earlier step and is where it looks for it
-static int fault(const LeanTree& t, const LeanSchedule& s, int g0, int g1, int n_slots, bool up) {
+// 0 if the schedule is right: every node of the scope once, what a node reads was written in an earlier step and is where it
+// looks for it (tiles from other workgroups excepted)
+static int fault(const LeanTree& t, const LeanSchedule& s, const LeanScope& in, int n_slots, bool up) {
   std::vector<int> step(t.parent.size(), -1), in_slot(n_slots, -1), last(kLeanSchedWaves, -1);
-  int done = 0;
+  size_t done = 0;
   for (int st = 0; st < s.steps; ++st) {
     std::vector<std::pair<int, int>> put;
+    std::vector<int> scratch;
     for (int w = 0; w < kLeanSchedWaves; ++w) {
       const int v = s.item[(size_t)st * kLeanSchedWaves + w];
       if (v < 0) continue;
-      if (v < g0 || v >= g1 || step[v] >= 0) return 1;
+      if (!in.in[v] || step[v] >= 0 || s.step_of[v] != st) return 1;
       const std::vector<int32_t> reads = up ? t.inner[v] : std::vector<int32_t>{v};
       for (int r : reads) {
         const int from = up ? r : t.parent[v];
         if (from < 0) { if (s.slot[v] != kLeanSlotNone) return 2; continue; }
+        if (!in.in[from]) { if (s.slot[r] != kLeanSlotAway) return 8; continue; }
         if (step[from] < 0 || step[from] >= st) return 3;
         if (s.slot[r] == kLeanSlotKept) {
           if (last[w] != from || (!up && t.inner[from][0] != v)) return 4;
@@ -48,19 +51,26 @@ static int fault(const LeanTree& t, const LeanSchedule& s, int g0, int g1, int n
           in_slot[s.slot[r]] = -1;
         }
       }
+      if (up && t.parent[v] >= 0 && !in.in[t.parent[v]] && s.slot[v] != kLeanSlotAway) return 9;
       const std::vector<int32_t> writes = up ? std::vector<int32_t>{v} : t.inner[v];
       for (int x : writes)
-        if (s.slot[x] < kLeanSlotKept) put.push_back({s.slot[x], x});
+        if (s.slot[x] < kLeanSlotAway) {
+          put.push_back({s.slot[x], x});
+          if (!up && !in.in[x]) scratch.push_back(s.slot[x]);
+        } else if (!up && !in.in[x] && x != t.inner[v][0]) {
+          return 10;
+        }
       step[v] = st;
       ++done;
       last[w] = v;
     }
     for (auto& p : put) {
-      if (in_slot[p.first] >= 0) return 6;
+      if (p.first < 0 || p.first >= n_slots || in_slot[p.first] >= 0) return 6;
       in_slot[p.first] = p.second;
     }
+    for (int x : scratch) in_slot[x] = -1;
   }
-  return done == g1 - g0 ? 0 : 7;
+  return done == in.nodes.size() ? 0 : 7;
 }
 
 int main() {
@@ -68,7 +78,7 @@ int main() {
   auto chain = [](int n) { std::vector<int> p(n); for (int v = 0; v < n; ++v) p[v] = v + 1 < n ? v + 1 : -1; return p; };
   {
     const LeanTree t = make(chain(40));
-    const LeanSchedule a = lean_schedule_up(t, 0, 40, 20), b = lean_schedule_down(t, 0, 40, 20);
+    const LeanSchedule a = lean_schedule_up(t, LeanScope(t, 0, 40), 20), b = lean_schedule_down(t, LeanScope(t, 0, 40), 20);
     int kept = 0;
     for (int v = 0; v < 40; ++v) kept += (a.slot[v] == kLeanSlotKept) + (b.slot[v] == kLeanSlotKept);
     std::printf("chain_steps %d\nchain_kept %d\n", a.steps + b.steps, kept);
@@ -107,16 +117,59 @@ int main() {
     int deep = 0;
     for (int v = 0; v < m; ++v) deep = std::max(deep, t.depth[v] + 1);
     for (int n_slots : {79, 24}) {
-      const LeanSchedule a = lean_schedule_up(t, 0, m, n_slots), b = lean_schedule_down(t, 0, m, n_slots);
+      const LeanSchedule a = lean_schedule_up(t, LeanScope(t, 0, m), n_slots), b = lean_schedule_down(t, LeanScope(t, 0, m), n_slots);
       for (const LeanSchedule* s : {&a, &b}) {
         if (!s->ok) { ++(n_slots == 79 ? refused_many : refused_few); continue; }
-        const int f = fault(t, *s, 0, m, n_slots, s == &a);
+        const int f = fault(t, *s, LeanScope(t, 0, m), n_slots, s == &a);
         if (f) { ++faults; std::fprintf(stderr, "tree %d (%d nodes), %d slots, %s: fault %d\n", i, m, n_slots, s == &a ? "up" : "down", f); }
         if (n_slots == 79 && s->steps > std::max(deep, (m + 15) / 16) * 1.4 + 4) ++long_ones;
         for (int v = 0; v < m; ++v) handed += s->slot[v] == kLeanSlotKept;
       }
     }
   }
+  // trees over several workgroups: a tile crosses once, between the top and another part, and every part's schedule is right
+  int cut_faults = 0, cut_refused = 0;
+  for (int i = 0; i < 120; ++i) {
+    const int n = 60 + (int)(rng() % 2000), span = i % 3 == 0 ? n : 2 + (int)(rng() % 10);
+    std::vector<int> up_to(n, -1), kids(n, 0);   // numbered from the root, every node below one of its `span` predecessors
+    for (int v = 1; v < n; ++v)
+      do { up_to[v] = std::max(0, v - 1 - (int)(rng() % span)); for (; kids[up_to[v]] >= 3; ++up_to[v]) {} } while (up_to[v] >= v);
+    for (int v = 1; v < n; ++v) ++kids[up_to[v]];
+    std::vector<std::vector<int>> ch(n);
+    for (int v = 1; v < n; ++v) ch[up_to[v]].push_back(v);
+    std::vector<int> id(n), post, parent(n, -1);
+    std::vector<std::pair<int, size_t>> st{{0, 0}};
+    while (!st.empty()) {
+      auto& top = st.back();
+      if (top.second < ch[top.first].size()) { const int c = ch[top.first][top.second++]; st.push_back({c, 0}); }
+      else { id[top.first] = (int)post.size(); post.push_back(top.first); st.pop_back(); }
+    }
+    for (int v = 1; v < n; ++v) parent[id[v]] = id[up_to[v]];
+    bool wide = false;
+    for (auto& c : ch) wide = wide || c.size() > 3;
+    if (wide) continue;
+    const LeanTree t = make(parent);
+    for (int G : {2, 4, 8, 16}) {
+      int largest = 0, most = 0;
+      const std::vector<int32_t> part = lean_parts(t, G, &largest);
+      for (int g = 0; g < G; ++g) most = std::max(most, (int)std::count(part.begin(), part.end(), g));
+      if (most != largest) ++cut_faults;
+      for (int v = 0; v < n; ++v)
+        if (part[v] < 0 || part[v] >= G || (t.parent[v] >= 0 && part[v] != part[t.parent[v]] && part[t.parent[v]] != 0)) ++cut_faults;
+      for (int g = 0; g < G; ++g) {
+        LeanScope in(part, g);
+        in.release.assign(n, 0);
+        for (int v = 0; v < n; ++v) in.release[v] = (int)(rng() % 40);
+        const LeanSchedule a = lean_schedule_up(t, in, 79), b = lean_schedule_down(t, in, 79);
+        for (const LeanSchedule* s : {&a, &b}) {
+          if (!s->ok) { ++cut_refused; continue; }
+          const int f = fault(t, *s, in, 79, s == &a);
+          if (f) { ++cut_faults; std::fprintf(stderr, "cut tree %d (%d nodes), part %d of %d, %s: fault %d\n", i, n, g, G, s == &a ? "up" : "down", f); }
+        }
+      }
+    }
+  }
+  std::printf("cut_faults %d\ncut_refused %d\n", cut_faults, cut_refused);
   std::printf("faults %d\nrefused_many %d\nrefused_few %d\nlong %d\nhanded %d\n", faults, refused_many, refused_few, long_ones, handed > 0);
   return 0;
 }

@@ -104,6 +104,32 @@ def test_bushy_trees_keep_the_lean_walks(gpu, oracle, shape):
     assert bpc.size("walk_kernels") == 1
 
 
+@pytest.mark.parametrize("V,K,B,reach", [(70, 32, 1, 6), (160, 16, 40, 4), (700, 32, 200, 8), (1300, 32, 33, 40)])
+def test_a_tree_over_several_workgroups(gpu, oracle, V, K, B, reach):
+    """Batches of few slices walk one tree in parts, a workgroup each, whose tiles cross through memory: against the
+    oracle, and the same bits on every pass (the flags that announce the tiles are back at zero behind each), with
+    batches that are walked in fewer parts in between."""
+    torch, P = gpu
+    from helpers import correlated_data
+    rng = np.random.default_rng(V)
+    kids, tree = np.zeros(V, int), [-1]
+    for v in range(1, V):
+        near = [u for u in range(max(0, v - reach), v) if kids[u] < 3]
+        tree.append(int(near[rng.integers(len(near))]))
+        kids[tree[-1]] += 1
+    bpc = _compare_step(gpu, oracle, V, K, 6, B, seed=V, tree=tree)
+    assert bpc.size("walk_kernels") == 1
+    d = torch.from_numpy(correlated_data(2100, V, 6, 9, np.array(tree))).cuda()
+    first = [t.cpu().numpy() for t in (P.loglikelihoods(bpc, d[:B]), P.probs_flows_circuit(bpc, d[:B]))]
+    flows = bpc.get_flows()
+    for n in (2100, 700, B, B):
+        other = P.probs_flows_circuit(bpc, d[:n]).cpu().numpy()
+        np.testing.assert_allclose(other[:B], first[0], rtol=1e-6)   # (the parts' shares of a likelihood add up in another order)
+        again = [t.cpu().numpy() for t in (P.loglikelihoods(bpc, d[:B]), P.probs_flows_circuit(bpc, d[:B]))]
+        assert all(np.array_equal(a, b) for a, b in zip(first, again))
+        assert all(np.array_equal(a, b) for a, b in zip(flows, bpc.get_flows()))
+
+
 @pytest.mark.parametrize("K,V", [(16, 9), (32, 40), (64, 6), (8, 5)])
 def test_scores_do_not_depend_on_the_batch_size(gpu, K, V):
     """A scoring pass on the lean walk keeps no tiles and takes the examples in batches of its own; the other kernels

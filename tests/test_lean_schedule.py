@@ -1,5 +1,5 @@
 """The schedules of the lean tree walks (csrc/lean_schedule.hpp): chains handed on in a wave's registers, everything else
-through LDS slots; compiled with g++ and replayed over hand-made and random trees."""
+through LDS slots, one tree cut for several workgroups; compiled with g++ and replayed over hand-made and random trees."""
 import os
 import subprocess
 
@@ -18,3 +18,4 @@ def test_lean_schedule(tmp_path):
     assert got["refused_many"] == 0 and got["refused_few"] <= 5
     assert got["long"] <= 60   # of 1200, more than 1.4 times the fewest steps there could be
     assert got["handed"] == 1
+    assert got["cut_faults"] == 0 and got["cut_refused"] == 0
