@@ -315,10 +315,22 @@ void HcltCircuit::build_schedules() {
                        std::vector<int32_t>& dst) -> bool {
     if (!sched.ok || K_ > 32 || lds_slots_ >= (int)kLeanAway || (size_t)V_ * leaf_stride >= ((size_t)1 << 31)) return false;
     const size_t f0 = dst.size();   // (the rows of a further group of trees go behind those of the groups before)
-    dst.resize(f0 + (size_t)kLeanFields * kWalkWaves * stride, 0);
+    dst.resize(f0 + (size_t)kLeanFields * kWalkWaves * stride + kWalkWaves, 0);
     int32_t* f = dst.data() + f0;
     auto at = [&](int field, int w, int st) -> int32_t& { return f[((size_t)field * kWalkWaves + w) * stride + st]; };
-    auto item = [&](int st, int w) { return st < sched.steps ? sched.item[(size_t)st * kWalkWaves + w] : -1; };
+    auto item = [&](int st, int w) { return sched.item[(size_t)st * kWalkWaves + w]; };
+    // A wave takes its nodes one behind the other: where the schedule has it idle it is the tile it waits for that holds it
+    // up.  place[st][w]: the step of the wave itself.  The rest of the rows is padding: no node, leaf rows of variable 0.
+    std::vector<int32_t> place((size_t)sched.steps * kWalkWaves, 0);
+    int32_t* const n_own = f + (size_t)kLeanFields * kWalkWaves * stride;
+    for (int st = 0; st < sched.steps; ++st)
+      for (int w = 0; w < kWalkWaves; ++w)
+        if (item(st, w) >= 0) place[(size_t)st * kWalkWaves + w] = n_own[w]++;
+    for (int w = 0; w < kWalkWaves; ++w)
+      for (int i = 0; i < stride; ++i) {
+        for (const int field : {kLW, kLA1, kLA2, kLA3, kLSlots}) at(field, w, i) = -1;
+        at(kLNode, w, i) = n_inner_;
+      }
     // how often each slot has been filled so far: a step's reads see the fills of earlier steps only, so the
     // readers of a step are numbered before its writers
     std::vector<int32_t> fills(256, 0);
@@ -327,7 +339,7 @@ void HcltCircuit::build_schedules() {
         for (int w = 0; w < kWalkWaves; ++w) {
           const int n = item(st, w);
           if (n < 0) continue;
-          int32_t& turns = at(kLTurns, w, st);
+          int32_t& turns = at(kLTurns, w, place[(size_t)st * kWalkWaves + w]);
           auto turn = [&](int tile, int byte) {
             const int sl = sched.slot[tile];
             if (sl < kLeanSlotAway) turns |= ((pass == 0 ? fills[sl] - 1 : fills[sl]++) & 0x7f) << (8 * byte);
@@ -338,38 +350,35 @@ void HcltCircuit::build_schedules() {
           else
             turn(n, 0);
         }
-    for (int st = 0; st < stride; ++st)
+    for (int st = 0; st < sched.steps; ++st)
       for (int w = 0; w < kWalkWaves; ++w) {
-        const int n = item(st, w);
-        at(kLA1, w, st) = at(kLA2, w, st) = at(kLA3, w, st) = -1;
-        at(kLW, w, st) = -1;
-        at(kLSlots, w, st) = -1;
-        at(kLNode, w, st) = n < 0 ? n_inner_ : n;
-        if (n < 0) continue;   // idle: leaf rows of variable 0
+        const int n = item(st, w), i = place[(size_t)st * kWalkWaves + w];
+        if (n < 0) continue;
+        at(kLNode, w, i) = n;
         if (lt.inner[n].size() + (forward ? 0 : lc[n].size()) > 3 || lc[n].size() > 3) return false;
-        if (forward || !lt.inner[n].empty()) at(kLW, w, st) = (int32_t)((size_t)n * K_ * K_ * sizeof(float));
-        at(kLA0, w, st) = (int32_t)((size_t)var_of_inner_[n] * leaf_stride);
-        at(kLFlags, w, st) = par[n] < 0 ? (H_ > 0 ? 3 : 1) : 0;
+        if (forward || !lt.inner[n].empty()) at(kLW, w, i) = (int32_t)((size_t)n * K_ * K_ * sizeof(float));
+        at(kLA0, w, i) = (int32_t)((size_t)var_of_inner_[n] * leaf_stride);
+        if (par[n] < 0) at(kLTurns, w, i) |= 0x80;
         uint32_t slots = 0xffffff00u | (uint32_t)sched.slot[n];
         int q = 0;
         for (int c : lt.inner[n]) {
           slots = (slots & ~(0xffu << (8 * (q + 1)))) | ((uint32_t)sched.slot[c] << (8 * (q + 1)));
-          if (!forward) at(kLA1 + q, w, st) = c << 3;
+          if (!forward) at(kLA1 + q, w, i) = c << 3 | (lt.inner[n].size() == 1 && in.in[c] ? 2 : 0);
           ++q;
         }
-        at(kLSlots, w, st) = (int32_t)slots;
-        if (par[n] >= 0 && !in.in[par[n]]) at(kLAway, w, st) = xid[n];
-        for (size_t i = lt.inner[n].size(); i-- > 0;) {
-          if (in.in[lt.inner[n][i]]) continue;
-          at(kLAway, w, st) = xid[lt.inner[n][i]];   // (those of one node are numbered in order)
-          at(kLFlags, w, st) |= 4 << i;
+        at(kLSlots, w, i) = (int32_t)slots;
+        if (par[n] >= 0 && !in.in[par[n]]) at(kLAway, w, i) = xid[n];
+        for (size_t k = lt.inner[n].size(); k-- > 0;) {
+          if (in.in[lt.inner[n][k]]) continue;
+          at(kLAway, w, i) = xid[lt.inner[n][k]];   // (those of one node are numbered in order)
+          if (!forward) at(kLTurns, w, i) |= (int32_t)(0x80u << (8 * (k + 1)));
         }
         if (forward) q = 0;
-        for (size_t i = 0; i < lc[n].size(); ++i)
-          at(kLA1 + q++, w, st) = (int32_t)((size_t)lc[n][i] * leaf_stride) | (forward ? 0 : 1 | (int32_t)((i + 1) << 1));
+        for (size_t k = 0; k < lc[n].size(); ++k)
+          at(kLA1 + q++, w, i) = (int32_t)((size_t)lc[n][k] * leaf_stride) | (forward ? 0 : 1 | (int32_t)((k + 1) << 1));
       }
     // the waits and posts of all waves, replayed: a schedule on which a wave would wait for ever is refused here
-    static_assert(kLeanCheckA1 == kLA1 && kLeanCheckSlots == kLSlots && kLeanCheckTurns == kLTurns && kLeanCheckFlags == kLFlags &&
+    static_assert(kLeanCheckA1 == kLA1 && kLeanCheckSlots == kLSlots && kLeanCheckTurns == kLTurns &&
                   kLeanCheckFields == kLeanFields && kLeanCheckWaves == kWalkWaves && kLeanCheckKept == kLeanAway &&
                   kLeanSlotKept == kLeanKept && kLeanSlotAway == kLeanAway && kLeanSchedWaves == kWalkWaves, "the lean schedule's headers follow the field rows");
     const int stuck = lean_schedule_stuck_at(f, stride, stride, forward, kLeanSlotNone);
@@ -965,7 +974,7 @@ void HcltCircuit::rebuild_heads() {
 void HcltCircuit::heads_forward(const HcltDev& d, const float* d_mask, float* d_ll_heads, float* d_ll_mix, bool flows_follow,
                                 float rate) {
   PCM_DISPATCH_LEAN_K(K_, hipLaunchKernelGGL(hclt_heads_forward_kernel<KK>, dim3(d.nslices, T_), dim3(kHeadWaves * 64), 0,
-                                             stream, d.O, d.M, d.Bp, d_root_node_.p, (int64_t)(d.tile_stride / 4), d_head_wf_.p,
+                                             stream, d.O, d.M, lean_fits(d.B) ? ~1 : ~0, d.Bp, d_root_node_.p, (int64_t)(d.tile_stride / 4), d_head_wf_.p,
                                              H_, Hp_, d.B, d_mask, d_ll_heads, d_ll_mix,
                                              flows_follow ? head_aggr() : (float*)nullptr, rate, d_flow_shift_.p));
   check_launch("heads_forward");
@@ -1304,8 +1313,8 @@ void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
     auto launch_lean = [&](auto kernel) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
       const LeanPlan* lp = lean_plan(d.nslices);
-      PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, lp->fwd.p, lp->fwd_stride,
-                       lp->n_fwd_steps, d_ll, lds_slots_, away());
+      PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, lp->fwd.p, lp->fwd_stride, d_ll,
+                       lds_slots_, away());
     };
     PCM_DISPATCH_LEAN_K(K_, {
       if (keep == kKeepAll) launch_lean(&hclt_forward_lean_kernel<KK, kKeepAll>);
@@ -1333,7 +1342,7 @@ void HcltCircuit::run_backward(const HcltDev& d) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
       const LeanPlan* lp = lean_plan(d.nslices);
       PCM_LAUNCH_PHASE(1, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, lp->bwd.p, lp->bwd_stride,
-                       lp->n_bwd_steps, lds_slots_, away());
+                       lds_slots_, away());
     };
     PCM_DISPATCH_LEAN_K(K_, {
       if (H_ > 0) launch_lean(&hclt_backward_lean_kernel<KK, true>); else launch_lean(&hclt_backward_lean_kernel<KK, false>);

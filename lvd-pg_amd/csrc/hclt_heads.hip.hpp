@@ -80,7 +80,7 @@ __device__ __forceinline__ v4f heads_contract_f(const float* __restrict__ hwf, i
 //   logsumexp_h(ll_h + log mask_h) - log sum_h mask_h   (src-jl/multi_head_pc/likelihood.jl:3-12).
 template <int K>
 __global__ __launch_bounds__(kHeadWaves * 64) void hclt_heads_forward_kernel(const float* __restrict__ O,
-                                                                             const float* __restrict__ M, int Bp,
+                                                                             const float* __restrict__ M, int m_mask, int Bp,
                                                                              const int32_t* __restrict__ root_node,
                                                                              int64_t tile_floats,
                                                                              const float* __restrict__ hwf, int H, int Hp,
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kHeadWaves * 64) void hclt_heads_forward_kernel(con
   {
     const int n_lo = tree > 0 ? root_node[tree - 1] + 1 : 0, n_hi = root_node[tree];
     double acc = 0.0;
-    for (int n = n_lo + wave * 4 + g; n <= n_hi; n += kHeadWaves * 4) acc += (double)M[(size_t)n * Bp + col];
+    for (int n = n_lo + wave * 4 + g; n <= n_hi; n += kHeadWaves * 4) acc += (double)__builtin_bit_cast(float, __builtin_bit_cast(int, M[(size_t)n * Bp + col]) & m_mask);
     pb[wave * 4 + g][b] = acc;
     __syncthreads();
     base = 0.0;

@@ -18,7 +18,7 @@
 //   * a wave follows a chain of the tree (lean_schedule.hpp): the tile of its last node is in registers when the next one
 //     needs it, and four tiles in five go through no LDS slot, no wait and no post;
 //   * idle steps only keep the requests going.
-// What bounds a step (walks with pieces left out, 784 variables, K = 32, 512 examples, 53 steps of 16 nodes, 97 us): all its
+// What bounds a step (forward walk with pieces left out, 784 variables, K = 32, 512 examples, 53 steps, then 97 us): all its
 // memory requests without the arithmetic 95 us, all the arithmetic without the requests 84, neither 33.  The fp32 matrix
 // instructions of a SIMD's four waves (4 x 512 cycles) and their vector instructions (4 x 600) add up, as both use the same
 // units; the requests of a compute unit (140 KB a step) do so beside them.
@@ -28,28 +28,30 @@
 
 namespace pcm {
 
-// Field rows of a lean schedule, [field][wave][stride] like the general one.
+// Field rows of a lean schedule, [field][wave][stride] like the general one, and behind them [wave] the number of steps up
+// to the wave's last node: a wave that is through leaves the compute unit to the others.
 //   kLW     byte offset of the node's parameter block (-1: none wanted)
 //   kLA0    byte offset of the node's own leaf rows (variable * leaf_stride)
 //   kLA1..3 forward: leaf children's rows (-1: none; their categories are bytes 1..3 of the
 //           packed word).  backward: children, inner ones first, -1: none, leaf child: row
-//           offset | 1 | category byte << 1, inner child: node index << 3 (its value tile)
+//           offset | 1 | category byte << 1, inner child: node index << 3 (its value tile), | 2
+//           if it is the only one and comes next in this wave: its value tile is not wanted
 //   kLNode  node index (value / flow tile, packed-category row, row of maxima); idle waves:
 //           n_inner (that category row is out of range and reads as zero)
 //   kLSlots forward: out slot | child slots << 8, 16, 24 (0xff: none); backward: slot holding
 //           this node's ratio tile | slots of the inner children's ratio tiles << 8, 16, 24
 //           (0xff: that child is a leaf or absent); kLeanKept: in registers
-//   kLFlags bit 0: root; bit 1: root of a multi-head circuit; bits 2..4, backward: child 1..3 is away
 //   kLTurns which use of its slot a tile is, modulo 128, in the byte layout of kLSlots: a slot passes through
-//           the states 2t (free for its t-th tile), 2t + 1 (that tile is there), 2t + 2 (read, free again)
+//           the states 2t (free for its t-th tile), 2t + 1 (that tile is there), 2t + 2 (read, free again).  Bit 7 of byte 0:
+//           the root; bit 7 of bytes 1..3, backward: that child is away
 //   kLAway  place in the exchange of this node's tile, or of the first of its children's, that crosses workgroups (below)
-enum { kLW = 0, kLA0, kLA1, kLA2, kLA3, kLNode, kLSlots, kLFlags, kLTurns, kLAway, kLeanFields };
+enum { kLW = 0, kLA0, kLA1, kLA2, kLA3, kLNode, kLSlots, kLTurns, kLAway, kLeanFields };
 constexpr uint32_t kLeanAway = 0xfd;       // in place of a slot: the tile comes from or goes to another workgroup
 constexpr uint32_t kLeanKept = 0xfe;       // in place of a slot: the tile stays in the registers of the wave (one that stays nowhere: 0xff)
 constexpr int kLeanFlagWords = 256;        // one state word per LDS slot, behind the slots
 constexpr int kLeanSpinLimit = 1 << 22;    // polls before a wave gives up on a tile (never reached by a sound schedule)
 
-constexpr int kLeanChunk = 62;   // steps per refill: 64 lanes minus two steps of look-ahead
+constexpr int kLeanChunk = 60;   // steps per refill (even): 64 lanes minus what the last two steps look ahead
 
 struct LeanChunk {
   int v[kLeanFields];
@@ -107,6 +109,26 @@ constexpr uint32_t kLeanNowhere = 0x80000000u;   // (every array is shorter)
 template <int K>
 __device__ __forceinline__ void lean_w_load_if(__amdgpu_buffer_rsrc_t r, uint32_t vtile, int soff, WTile<K>& w) {
   lean_w_load<K>(r, soff < 0 ? kLeanNowhere + vtile : vtile, max(soff, 0), w);
+}
+
+// Places the requests of the block of code it stands in between the block's matrix instructions: three reads (words, rows) and
+// the first half of the next parameter block behind every second one, the other half as its registers are through.  A wave
+// that issues a matrix instruction waits for the one before; these slots are free.  (K = 32; a K = 16 contraction is four
+// instructions.)  632 nodes in four parts, 512 examples, forward: 96 -> 91 us.  The same in the backward walk, whose requests
+// would then stand in three branches, loses: the compiler no longer knows how many are in flight where they join (75 -> 118).
+template <int K>
+__device__ __forceinline__ void lean_between() {
+  if constexpr (K == 32) {
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);   // matrix instructions
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);   // reads
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+  }
 }
 
 // byte offset of this lane's part of leaf row x (byte `sel` of the packed word)
@@ -181,32 +203,27 @@ __device__ __forceinline__ void away_flag(unsigned* flag, unsigned value) {
   if ((threadIdx.x & 63) == 0) __hip_atomic_store(flag, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+constexpr int kDeviceScope = 16;   // (sc1)
 template <int K>
-__device__ __forceinline__ void away_put(const LeanAway& x, const HcltDev& d, int tile, int slice, int lane, const Tile<K>& t) {
-  const size_t at = (size_t)tile * d.nslices + slice;
-  unsigned long long* p = reinterpret_cast<unsigned long long*>(x.tiles + at * (kSlice * K)) + lane * 2;
+__device__ __forceinline__ void away_put(const LeanAway& x, const HcltDev& d, int tile, int slice, uint32_t vtile, const Tile<K>& t) {
+  const int at = tile * d.nslices + slice;
+  const __amdgpu_buffer_rsrc_t r = make_rsrc(x.tiles + (size_t)at * (kSlice * K), kSlice * K * 4);
 #pragma unroll
   for (int kt = 0; kt < K / 16; ++kt)
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-      __hip_atomic_store(p + kt * 128 + h, __builtin_bit_cast(unsigned long long, make_float2(t.v[kt][2 * h], t.v[kt][2 * h + 1])),
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, t.v[kt]), r, (int)(vtile + kt * 1024), 0, kDeviceScope);
   away_flag(x.flags + at, 1u);
 }
 
 template <int K>
-__device__ __forceinline__ void away_get(const LeanAway& x, const HcltDev& d, int tile, int slice, int lane, Tile<K>& t) {
-  const size_t at = (size_t)tile * d.nslices + slice;
+__device__ __forceinline__ void away_get(const LeanAway& x, const HcltDev& d, int tile, int slice, uint32_t vtile, Tile<K>& t) {
+  const int at = tile * d.nslices + slice;
+  const __amdgpu_buffer_rsrc_t r = make_rsrc(x.tiles + (size_t)at * (kSlice * K), kSlice * K * 4);
   away_wait(x.flags + at, d);
-  unsigned long long* p = reinterpret_cast<unsigned long long*>(x.tiles + at * (kSlice * K)) + lane * 2;
 #pragma unroll
   for (int kt = 0; kt < K / 16; ++kt)
+    t.v[kt] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(vtile + kt * 1024), 0, kDeviceScope));
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const float2 v = __builtin_bit_cast(float2, __hip_atomic_load(p + kt * 128 + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-      t.v[kt][2 * h] = v.x;
-      t.v[kt][2 * h + 1] = v.y;
-    }
+  for (int kt = 0; kt < K / 16; ++kt) asm volatile("" : "+v"(t.v[kt]));   // (waited for here, not where the ways join)
   away_flag(x.flags + at, 0u);
 }
 
@@ -219,18 +236,34 @@ __device__ __forceinline__ void away_get(const LeanAway& x, const HcltDev& d, in
 // (values near -14000) an absolute error of 1e-3, which is a relative error of 1e-3 on every flow; in two parts the
 // flows keep float32's relative accuracy at any depth.
 //
+// The lowest bit of a stored maximum is not part of the number: m is rounded to an even last place before anything is scaled
+// by it (any number near the maximum does), and the bit says that some example of the slice has a state of probability zero
+// (a value of -inf) at this node.  A node with one inner child then needs that child's tile on the way down only where the
+// bit is set: its ratio tile is made of the OTHER operands, and of its own values only "is it zero" counts.
+__device__ __forceinline__ float lean_scale(float m) { return __builtin_bit_cast(float, __builtin_bit_cast(int, m) & ~1); }
+template <int K>
+__device__ __forceinline__ float lean_mark(float m, const Tile<K>& o) {
+  float least = o.v[0][0];
+#pragma unroll
+  for (int kt = 0; kt < K / 16; ++kt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) least = fminf(least, o.v[kt][i]);
+  return __builtin_bit_cast(float, __builtin_bit_cast(int, m) | (__ballot(least == -INFINITY) != 0ull ? 1 : 0));
+}
+
 // kKeep: what the walk leaves in memory.  kKeepAll: every node's tile and row of maxima, for the passes behind it;
 // kKeepRoots: the maxima and the roots' tiles, what the head kernel of a multi-head circuit reads; kKeepNone: nothing
 // but the log-likelihoods: a scoring pass has nobody behind it, and value stores are 512 of a step's 1340 requests.
 // 10300 examples of 3072 variables (K = 32), which no longer need tile arrays and so go through 4096 at a time
 // whatever the caller's batch size: 3.93 ms in batches of 1000 -> 1.08 ms.
 //
-// With chains kept in registers, against the schedule that picked the sixteen most urgent nodes of every step anew (a tile per
-// node through LDS): 784 variables, 512 examples 111 -> 97 us, 192 variables 55 -> 42, 64 variables (K = 16) 19 -> 16.5;
-// 3072 variables at 4096 examples, where the stores of the tiles count, 390 -> 384.
+// Measured (us; the schedule that picked the sixteen most urgent nodes of every step anew and put a tile per node through LDS /
+// chains in registers / and requests that never wait for a store, two steps ahead, waves that leave when they are through):
+// 784 variables, 512 examples 111 / 97 / 70, 192 variables 55 / 42 / 37, 64 variables (K = 16) 19 / 16.5 / 13; 3072 variables
+// at 512 examples (in parts) 336 / 194 / 141, at 4096, where the stores of the tiles count, 390 / 384 / 372.
 template <int K, int kKeep>
 __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
-    HcltDev d, const int32_t* __restrict__ fields, int stride, int n_steps, float* __restrict__ ll_out, int n_slots, LeanAway away) {
+    HcltDev d, const int32_t* __restrict__ fields, int stride, float* __restrict__ ll_out, int n_slots, LeanAway away) {
   extern __shared__ float lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -252,25 +285,31 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
   // kernel scale by exactly these numbers (lanes 16..63 hold copies: their stores fall outside the buffer)
   const __amdgpu_buffer_rsrc_t rM =
       make_rsrc(d.M + (size_t)slice * kSlice, (uint32_t)(d.n_inner + 1) * (uint32_t)d.Bp * 4u - (uint32_t)slice * (kSlice * 4));
-  const uint32_t vm = lane < 16 ? vx : 0x7ffffff0u;
+  const uint32_t vm = lane < 16 ? vx : 0x70000000u;   // (past the end with kLeanNowhere added, too)
 
-  fields += (size_t)blockIdx.y * (kLeanFields * kWalkWaves) * stride;   // a forest's groups of trees: a schedule each
+  fields += (size_t)blockIdx.y * (kLeanFields * kWalkWaves * (size_t)stride + kWalkWaves);   // groups of trees, parts: a schedule each
+  const int n_steps = __builtin_amdgcn_readfirstlane(fields[(size_t)kLeanFields * kWalkWaves * stride + wave]);
   LeanChunk sc;
   lean_refill(fields, stride, wave, lane, 0, sc);
-  Tile<K> P0, P1, P2, P3;
-  WTile<K> wA, wB;   // parameter blocks of the even / odd steps
-  uint32_t xs;
-  int a1, a2, a3;   // leaf children of the step whose operands are in flight
+  // What is in flight: a node's own leaf rows and its parameter block are requested two steps ahead, into the registers of
+  // the step that has just used them (so there are two sets, of the even and the odd steps), the rows of its leaf children
+  // one step ahead, the categories three.
+  Tile<K> PA, PB, P1, P2;   // (a third leaf child is rare: its rows are fetched at the point of use)
+  WTile<K> wA, wB;
+  uint32_t x0, x1, x2;  // packed categories of this step, of the next and of the one after
+  int a1, a2, a3;       // leaf children of the step whose operands are in flight
+  auto load_x = [&](int s) { return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rX, (int)vx, lean_get(sc, kLNode, s) * xrow, 0); };
   {
-    const uint32_t x0 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rX, (int)vx, lean_get(sc, kLNode, 0) * xrow, 0);
-    xs = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rX, (int)vx, lean_get(sc, kLNode, 1) * xrow, 0);
-    lean_row_load<K>(rL, lean_row_off<K>(x0, 0, vleaf), lean_get(sc, kLA0, 0), P0);
+    x0 = load_x(0);
+    x1 = load_x(1);
+    x2 = load_x(2);
+    lean_row_load<K>(rL, lean_row_off<K>(x0, 0, vleaf), lean_get(sc, kLA0, 0), PA);
     a1 = lean_get(sc, kLA1, 0); a2 = lean_get(sc, kLA2, 0); a3 = lean_get(sc, kLA3, 0);
     if (a1 >= 0) lean_row_load<K>(rL, lean_row_off<K>(x0, 1, vleaf), a1, P1);
     if (a2 >= 0) lean_row_load<K>(rL, lean_row_off<K>(x0, 2, vleaf), a2, P2);
-    if (a3 >= 0) lean_row_load<K>(rL, lean_row_off<K>(x0, 3, vleaf), a3, P3);
     lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, 0), wA);
     __builtin_amdgcn_sched_barrier(0);   // (in this order: the waits inside the loop are counted for both ways into it)
+    lean_row_load<K>(rL, lean_row_off<K>(x1, 0, vleaf), lean_get(sc, kLA0, 1), PB);
     lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, 1), wB);
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -279,79 +318,113 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
   double msum = 0.0;   // sum of the row maxima of this wave's nodes: the part of the log-likelihood the tiles leave out
   Tile<K> o;           // the value tile of this wave's last node: its parent takes it from here if it comes next in the wave
   tile_zero<K>(o);
+  // what of it is to be stored, in the step after (kLeanNowhere: nothing)
+  uint32_t keep_o = kLeanNowhere, keep_m = kLeanNowhere;
+  int o_at = 0, m_at = 0;
+  float m_prev = 0.f;
 
-  auto step = [&](const int s, WTile<K>& w) {
-    // (1) the static operands of this step have landed
-    Tile<K> z = P0;
-    if (a1 >= 0) tile_add<K>(z, P1);
-    if (a2 >= 0) tile_add<K>(z, P2);
-    if (a3 >= 0) tile_add<K>(z, P3);
-    const int node = lean_get(sc, kLNode, s);
-    // (2) request the leaf rows of step s+1 and the categories of step s+2
-    {
-      // (the categories first: everything that later waits for a leaf row then covers them)
-      const uint32_t xc = xs;
-      xs = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rX, (int)vx, lean_get(sc, kLNode, s + 2) * xrow, 0);
-      lean_row_load<K>(rL, lean_row_off<K>(xc, 0, vleaf), lean_get(sc, kLA0, s + 1), P0);
-      a1 = lean_get(sc, kLA1, s + 1); a2 = lean_get(sc, kLA2, s + 1); a3 = lean_get(sc, kLA3, s + 1);
-      if (a1 >= 0) lean_row_load<K>(rL, lean_row_off<K>(xc, 1, vleaf), a1, P1);
-      if (a2 >= 0) lean_row_load<K>(rL, lean_row_off<K>(xc, 2, vleaf), a2, P2);
-      if (a3 >= 0) lean_row_load<K>(rL, lean_row_off<K>(xc, 3, vleaf), a3, P3);
+  // A step sends its requests whatever it does, those with nothing to fetch or to store past the end of their array: the wait
+  // for one is then for a known number of requests behind it, and none is waited for less than a step after it went out.
+  auto ahead = [&](const int s, WTile<K>& w, Tile<K>& P) {
+    const uint32_t x3 = load_x(s + 3);
+    lean_row_load<K>(rL, lean_row_off<K>(x2, 0, vleaf), lean_get(sc, kLA0, s + 2), P);
+    lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, s + 2), w);
+    x0 = x1;
+    x1 = x2;
+    x2 = x3;
+  };
+  auto step = [&](const int s, WTile<K>& w, Tile<K>& P) {
+    // (1) the leaf rows of this step have landed
+    Tile<K> z = P;
+    if (a1 >= 0) {
+      tile_add<K>(z, P1);
+      if (a2 >= 0) tile_add<K>(z, P2);
+      if (a3 >= 0) {
+        Tile<K> t;
+        lean_row_load<K>(rL, lean_row_off<K>(x0, 3, vleaf), a3, t);
+        tile_add<K>(z, t);
+#pragma unroll
+        for (int kt = 0; kt < K / 16; ++kt) asm volatile("" : "+v"(z.v[kt]));   // (waited for here, not where the ways join)
+      }
     }
+    // (2) request the rows of the next step's leaf children, the node's own of the step after, the categories of the third;
+    // the previous step's tile goes out
+    a1 = lean_get(sc, kLA1, s + 1);
+    if (a1 >= 0) {
+      a2 = lean_get(sc, kLA2, s + 1); a3 = lean_get(sc, kLA3, s + 1);
+      lean_row_load<K>(rL, lean_row_off<K>(x1, 1, vleaf), a1, P1);
+      if (a2 >= 0) lean_row_load<K>(rL, lean_row_off<K>(x1, 2, vleaf), a2, P2);
+    }
+    if (kKeep != kKeepNone) {
+      lean_tile_store<K>(rO, keep_o + vtile, o_at, o);
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, m_prev), rM, (int)(keep_m + vm), m_at, kStreamStore);
+      keep_o = keep_m = kLeanNowhere;
+    }
+    const int node = lean_get(sc, kLNode, s);
     if (node != d.n_inner) {   // (idle steps only keep the requests going)
       // (3) inner children, from LDS or, the one this wave computed last, from registers; logsumexp through the matrix cores
       const uint32_t slots = (uint32_t)lean_get(sc, kLSlots, s), turns = (uint32_t)lean_get(sc, kLTurns, s);
-      int next_away = lean_get(sc, kLAway, s);
+      if ((slots >> 8) == (0xffff00u | kLeanKept)) {   // (most nodes: one inner child, and this wave has it)
+        tile_add<K>(z, o);
+      } else {
+        int next_away = lean_get(sc, kLAway, s);
 #pragma unroll
-      for (int c = 1; c <= 3; ++c) {
-        const uint32_t sl = (slots >> (8 * c)) & 0xffu, tn = (turns >> (8 * c)) & 0x7fu;
-        if (sl == 0xffu) break;
-        if (sl == kLeanKept) {
-          tile_add<K>(z, o);
-        } else if (sl == kLeanAway) {
-          Tile<K> t;
-          away_get<K>(away, d, next_away++, slice, lane, t);
-          tile_add<K>(z, t);
-        } else {
-          lean_wait(state + sl, (2 * tn + 1) & 0xffu, d);
-          Tile<K> t;
-          lds_tile_load<K>(lds, (int)sl, lane, t);
-          tile_add<K>(z, t);
-          lean_post(state + sl, (2 * tn + 2) & 0xffu);   // read: the slot may take its next tile
+        for (int c = 1; c <= 3; ++c) {
+          const uint32_t sl = (slots >> (8 * c)) & 0xffu, tn = (turns >> (8 * c)) & 0x7fu;
+          if (sl == 0xffu) break;
+          if (sl == kLeanKept) {
+            tile_add<K>(z, o);
+          } else if (sl == kLeanAway) {
+            Tile<K> t;
+            away_get<K>(away, d, next_away++, slice, vtile, t);
+            tile_add<K>(z, t);
+          } else {
+            lean_wait(state + sl, (2 * tn + 1) & 0xffu, d);
+            Tile<K> t;
+            lds_tile_load<K>(lds, (int)sl, lane, t);
+            tile_add<K>(z, t);
+            lean_post(state + sl, (2 * tn + 2) & 0xffu);   // read: the slot may take its next tile
+          }
         }
       }
-      const float m = tile_rowmax<K>(z);
+      const float m = lean_scale(tile_rowmax<K>(z));
       tile_exp_sub<K>(z, m);
+      // the requests go out between the matrix instructions, which leave the wave's issue slots free
       contract<K>(w, z, o);
+      ahead(s, w, P);
+      lean_between<K>();
 #pragma unroll
       for (int kt = 0; kt < K / 16; ++kt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) o.v[kt][i] = __builtin_amdgcn_logf(o.v[kt][i]) * kLn2;
-      // hand the tile on first (the root's, and one whose reader is this wave's next node, go nowhere)
-      const uint32_t so = slots & 0xffu, tn = turns & 0x7fu;
-      if (so < kLeanAway) {
-        lean_wait(state + so, (2 * tn) & 0xffu, d);
-        lds_tile_store<K>(lds, (int)so, lane, o);
-        lean_post(state + so, (2 * tn + 1) & 0xffu);
-      } else if (so == kLeanAway) {
-        away_put<K>(away, d, lean_get(sc, kLAway, s), slice, lane, o);
+      // hand the tile on (the root's, and one whose reader is this wave's next node, go nowhere)
+      const uint32_t so = slots & 0xffu;
+      if (so <= kLeanAway) {
+        const uint32_t tn = turns & 0x7fu;
+        if (so == kLeanAway) {
+          away_put<K>(away, d, lean_get(sc, kLAway, s), slice, vtile, o);
+        } else {
+          lean_wait(state + so, (2 * tn) & 0xffu, d);
+          lds_tile_store<K>(lds, (int)so, lane, o);
+          lean_post(state + so, (2 * tn + 1) & 0xffu);
+        }
       }
       msum += (double)m;
-      const bool root = (lean_get(sc, kLFlags, s) & 1) != 0;
+      const bool root = (turns & 0x80u) != 0;
       if (root) {
         ll = o.v[0][0];
         root_here = true;
       }
-      if (kKeep == kKeepAll || (kKeep == kKeepRoots && root))
-        lean_tile_store<K>(rO, vtile, (int)((uint32_t)node * d.tile_stride), o);
-      if (kKeep != kKeepNone)
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, m), rM, (int)vm, node * xrow, kStreamStore);
+      if (kKeep == kKeepAll || (kKeep == kKeepRoots && root)) keep_o = 0;
+      if (kKeep != kKeepNone) {
+        keep_m = 0;
+        m_prev = lean_mark<K>(m, o);
+      }
+      o_at = (int)((uint32_t)node * d.tile_stride);
+      m_at = node * xrow;
+    } else {
+      ahead(s, w, P);
     }
-    // (4) the block of step s+2, into the registers of this step's; behind the stores, so that a step's wait for its
-    // leaf rows finds exactly these requests behind them, whether there were stores or not
-    __builtin_amdgcn_sched_barrier(0);
-    lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, s + 2), w);
-    __builtin_amdgcn_sched_barrier(0);
   };
   // The schedule is consumed in chunks of kLeanChunk steps (a chunk's registers also serve the
   // two steps of look-ahead past its end), two steps per trip: the parameter blocks alternate
@@ -361,9 +434,13 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
     if (base) lean_refill(fields, stride, wave, lane, base, sc);
     const int s_end = min(base + kLeanChunk, n_steps);
     for (int s = base; s < s_end; s += 2) {
-      step(s, wA);
-      step(s + 1, wB);
+      step(s, wA, PA);
+      step(s + 1, wB, PB);
     }
+  }
+  if (kKeep != kKeepNone) {
+    lean_tile_store<K>(rO, keep_o + vtile, o_at, o);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, m_prev), rM, (int)(keep_m + vm), m_at, kStreamStore);
   }
   // log-likelihood of a single-root circuit: the root's (scaled) value plus the row maxima of all nodes, the
   // waves' sums added in wave order (a multi-head circuit's head kernel adds up the stored maxima per tree)
@@ -408,11 +485,11 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
 // child gives probability zero (O'_c = -inf) has flow 0 and keeps ratio 0.  A node without inner children
 // only stores its tile.
 // kHeads: multi-head circuit, whose head kernel has left the root's ratio tile in memory.
-// 192 variables at 4096 examples 77 -> 53 us, 784 at 4096 184 -> 170 with the first child's tile in registers and the blocks
-// requested whether wanted or not; 3072 at 4096 stays at 625: 3.2 GB at 5.2 TB/s.
+// Measured as above: 192 variables at 4096 examples 77 / 53 / 43 us, 784 at 4096 184 / 170 / 151, at 512 125 / 107 / 75; 3072
+// at 4096 625 / 625 / 572 (the tiles of only children, 0.8 of 1.3 GB of the value tiles, are no longer read).
 template <int K, bool kHeads>
 __global__ __launch_bounds__(kWalkWaves * 64) void hclt_backward_lean_kernel(
-    HcltDev d, const int32_t* __restrict__ fields, int stride, int n_steps, int n_slots, LeanAway away) {
+    HcltDev d, const int32_t* __restrict__ fields, int stride, int n_slots, LeanAway away) {
   extern __shared__ float lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -441,130 +518,159 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_backward_lean_kernel(
   };
   auto is_inner = [](int c) { return c >= 0 && !(c & 1); };
 
-  fields += (size_t)blockIdx.y * (kLeanFields * kWalkWaves) * stride;   // a forest's groups of trees: a schedule each
+  fields += (size_t)blockIdx.y * (kLeanFields * kWalkWaves * (size_t)stride + kWalkWaves);   // groups of trees, parts: a schedule each
+  const int n_steps = __builtin_amdgcn_readfirstlane(fields[(size_t)kLeanFields * kWalkWaves * stride + wave]);
   LeanChunk sc;
   lean_refill(fields, stride, wave, lane, 0, sc);
-  Tile<K> P0, C1, C2, C3;
+  // in flight: a node's own leaf rows, row maxima and parameter block two steps ahead, its children's operands one, the
+  // categories three (see the forward walk)
+  Tile<K> PA, PB, C1, C2, C3;
   WTile<K> wA, wB;
-  uint32_t xs;
+  uint32_t x1, x2;
   int c1, c2, c3;
-  float mv;
+  float m0, m1;   // row maxima of this step and of the next, as stored
+  auto load_x = [&](int s) { return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rX, (int)vx, lean_get(sc, kLNode, s) * xrow, 0); };
+  auto load_m = [&](int s) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rM, (int)vx, lean_get(sc, kLNode, s) * xrow, 0));
+  };
+  auto load_children = [&](int s, uint32_t xpack) {
+    c1 = lean_get(sc, kLA1, s); c2 = lean_get(sc, kLA2, s); c3 = lean_get(sc, kLA3, s);
+    if (c1 >= 0) {
+      if ((c1 & 3) != 2) child_load(c1, xpack, C1);
+      if (c2 >= 0) child_load(c2, xpack, C2);
+      if (c3 >= 0) child_load(c3, xpack, C3);
+    }
+  };
   {
-    const uint32_t x0 = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rX, (int)vx, lean_get(sc, kLNode, 0) * xrow, 0);
-    xs = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rX, (int)vx, lean_get(sc, kLNode, 1) * xrow, 0);
-    mv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rM, (int)vx, lean_get(sc, kLNode, 0) * xrow, 0));
-    lean_row_load<K>(rL, lean_row_off<K>(x0, 0, vleaf), lean_get(sc, kLA0, 0), P0);
-    c1 = lean_get(sc, kLA1, 0); c2 = lean_get(sc, kLA2, 0); c3 = lean_get(sc, kLA3, 0);
-    if (c1 >= 0) child_load(c1, x0, C1);
-    if (c2 >= 0) child_load(c2, x0, C2);
-    if (c3 >= 0) child_load(c3, x0, C3);
+    const uint32_t x0 = load_x(0);
+    x1 = load_x(1);
+    x2 = load_x(2);
+    m0 = load_m(0);
+    m1 = load_m(1);
+    lean_row_load<K>(rL, lean_row_off<K>(x0, 0, vleaf), lean_get(sc, kLA0, 0), PA);
+    load_children(0, x0);
     lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, 0), wA);
     __builtin_amdgcn_sched_barrier(0);   // (in this order: the waits inside the loop are counted for both ways into it)
+    lean_row_load<K>(rL, lean_row_off<K>(x1, 0, vleaf), lean_get(sc, kLA0, 1), PB);
     lean_w_load_if<K>(rW, vtile, lean_get(sc, kLW, 1), wB);
     __builtin_amdgcn_sched_barrier(0);
   }
   Tile<K> r;   // the ratio tile of the node under way; behind a step, that of its first child, which comes next in this wave (or is away)
   tile_zero<K>(r);
 
-  // exponent tile of inner child `own` among the landed operands: the other operands minus m_v,
-  // in base-2 units; -inf where the child's own value is -inf
-  auto exponent = [&](const Tile<K>& own, bool has_a, const Tile<K>& a, bool has_b, const Tile<K>& b, Tile<K>& x) {
-    const float dm = -mv * kLog2e;
-#pragma unroll
-    for (int kt = 0; kt < K / 16; ++kt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float rest = P0.v[kt][i];
-        if (has_a) rest += a.v[kt][i];
-        if (has_b) rest += b.v[kt][i];
-        x.v[kt][i] = own.v[kt][i] == -INFINITY ? -INFINITY : fmaf(rest, kLog2e, dm);
-      }
-  };
-
-  auto step = [&](const int s, WTile<K>& w) {
-    // (1) from the landed operands: the exponent tiles of the inner children (they come first).  The first
-    // stays in registers; a second and third wait in the LDS slots their ratio tiles will take.
+  auto step = [&](const int s, WTile<K>& w, Tile<K>& P) {
+    // (1) from the landed operands: what an inner child's ratio tile is made of besides t, exp of the other operands minus
+    // m_v, zero where the child's own value is -inf.  The inner children come first; the first's factors stay in registers,
+    // a second's and third's wait in the LDS slots their ratio tiles will take.
     const int node = lean_get(sc, kLNode, s);
-    const bool in1 = is_inner(c1), in2 = is_inner(c2), in3 = is_inner(c3);
+    const bool in1 = is_inner(c1), in2 = is_inner(c2), in3 = is_inner(c3), alone = (c1 & 3) == 2 && in1;
+    const int own1 = c1;
     const uint32_t slots = (uint32_t)lean_get(sc, kLSlots, s), turns = (uint32_t)lean_get(sc, kLTurns, s);
+    const float dm = -lean_scale(m0) * kLog2e;
+    auto factor = [&](bool check, const Tile<K>& own, bool has_a, const Tile<K>& a, bool has_b, const Tile<K>& b, Tile<K>& x) {
+      Tile<K> rest = P;
+      if (has_a) tile_add<K>(rest, a);
+      if (has_b) tile_add<K>(rest, b);
+#pragma unroll
+      for (int kt = 0; kt < K / 16; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float e = fminf(__builtin_amdgcn_exp2f(fmaf(rest.v[kt][i], kLog2e, dm)), kFlowRatioCap);
+          x.v[kt][i] = check && own.v[kt][i] == -INFINITY ? 0.f : e;
+        }
+    };
     Tile<K> X1;
-    if (in1) exponent(C1, c2 >= 0, C2, c3 >= 0, C3, X1);
+    if (in1) {
+      if (alone) factor(false, C1, c2 >= 0, C2, c3 >= 0, C3, X1);
+      else factor(true, C1, c2 >= 0, C2, c3 >= 0, C3, X1);
+    }
     if (in2) {   // the children's slots are this wave's from here (scratch first, their ratio tiles at the end)
       Tile<K> x;
-      exponent(C2, true, C1, c3 >= 0, C3, x);
+      factor(true, C2, true, C1, c3 >= 0, C3, x);
       lean_wait(state + ((slots >> 16) & 0xffu), (2 * ((turns >> 16) & 0x7fu)) & 0xffu, d);
       lds_tile_store<K>(lds, (int)((slots >> 16) & 0xffu), lane, x);
+      if (in3) {
+        factor(true, C3, true, C1, true, C2, x);
+        lean_wait(state + ((slots >> 24) & 0xffu), (2 * ((turns >> 24) & 0x7fu)) & 0xffu, d);
+        lds_tile_store<K>(lds, (int)((slots >> 24) & 0xffu), lane, x);
+      }
     }
-    if (in3) {
-      Tile<K> x;
-      exponent(C3, true, C1, true, C2, x);
-      lean_wait(state + ((slots >> 24) & 0xffu), (2 * ((turns >> 24) & 0x7fu)) & 0xffu, d);
-      lds_tile_store<K>(lds, (int)((slots >> 24) & 0xffu), lane, x);
-    }
-    // (2) request the operands of step s+1 and the categories of step s+2
+    // (2) requests: the operands of the next step's children, own rows and maxima of the step after, categories of the third
+    load_children(s + 1, x1);
     {
-      const uint32_t xc = xs;
-      xs = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rX, (int)vx, lean_get(sc, kLNode, s + 2) * xrow, 0);
-      mv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rM, (int)vx, lean_get(sc, kLNode, s + 1) * xrow, 0));
-      lean_row_load<K>(rL, lean_row_off<K>(xc, 0, vleaf), lean_get(sc, kLA0, s + 1), P0);
-      c1 = lean_get(sc, kLA1, s + 1); c2 = lean_get(sc, kLA2, s + 1); c3 = lean_get(sc, kLA3, s + 1);
-      if (c1 >= 0) child_load(c1, xc, C1);
-      if (c2 >= 0) child_load(c2, xc, C2);
-      if (c3 >= 0) child_load(c3, xc, C3);
+      const uint32_t x3 = load_x(s + 3);
+      m0 = m1;
+      m1 = load_m(s + 2);
+      lean_row_load<K>(rL, lean_row_off<K>(x2, 0, vleaf), lean_get(sc, kLA0, s + 2), P);
+      x1 = x2;
+      x2 = x3;
     }
     if (node != d.n_inner) {   // (idle steps only keep the requests going)
       // (3) this node's ratio tile: in registers from the step before, or left in LDS by the parent
       const uint32_t so = slots & 0xffu;
-      if (so == kLeanAway) {
-        away_get<K>(away, d, lean_get(sc, kLAway, s), slice, lane, r);
-      } else if (so < kLeanAway) {
-        lean_wait(state + so, (2 * (turns & 0x7fu) + 1) & 0xffu, d);
-        lds_tile_load<K>(lds, (int)so, lane, r);
-        lean_post(state + so, (2 * (turns & 0x7fu) + 2) & 0xffu);
-      }
-      const int fl = lean_get(sc, kLFlags, s);
-      if (kHeads && (fl & 2)) {   // multi-head circuit: the head kernel has left the root's ratio tile in memory
-        lean_tile_load<K>(rR, vtile, node * (int)d.tile_stride, r);
-      } else if (fl & 1) {   // flow 1 into the single root sum node of every live example: R = 1 / S = exp(-O')
-        const float o00 = __builtin_bit_cast(
-            float, __builtin_amdgcn_raw_buffer_load_b32(rO, (int)vtile, node * (int)d.tile_stride, 0));
-        const bool live = lane < 16 && bcol < d.B;
-        const float wgt = (d.w && live) ? d.w[bcol] : 1.f;   // per-example weights: the flow the example starts with
-        const float r00 = live ? wgt * fminf(__builtin_amdgcn_exp2f(o00 * -kLog2e), kFlowRatioCap) : 0.f;
-        tile_zero<K>(r);
-        r.v[0][0] = r00;
+      if (so != kLeanKept) {
+        if (so == kLeanAway) {
+          away_get<K>(away, d, lean_get(sc, kLAway, s), slice, vtile, r);
+        } else if (so < kLeanAway) {
+          lean_wait(state + so, (2 * (turns & 0x7fu) + 1) & 0xffu, d);
+          lds_tile_load<K>(lds, (int)so, lane, r);
+          lean_post(state + so, (2 * (turns & 0x7fu) + 2) & 0xffu);
+        } else if (kHeads) {   // a root of a multi-head circuit: the head kernel has left its ratio tile in memory
+          lean_tile_load<K>(rR, vtile, node * (int)d.tile_stride, r);
+#pragma unroll
+          for (int kt = 0; kt < K / 16; ++kt) asm volatile("" : "+v"(r.v[kt]));   // (waited for here, not where the ways join)
+        } else {   // flow 1 into the single root sum node of every live example: R = 1 / S = exp(-O')
+          const float o00 = __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(rO, (int)vtile, node * (int)d.tile_stride, 0));
+          const bool live = lane < 16 && bcol < d.B;
+          const float wgt = (d.w && live) ? d.w[bcol] : 1.f;   // per-example weights: the flow the example starts with
+          float r00 = live ? wgt * fminf(__builtin_amdgcn_exp2f(o00 * -kLog2e), kFlowRatioCap) : 0.f;
+          asm volatile("" : "+v"(r00));
+          tile_zero<K>(r);
+          r.v[0][0] = r00;
+        }
       }
       lean_tile_store<K>(rR, vtile, node * (int)d.tile_stride, r);
       // (4) the inner children's ratio tiles; the first child is this wave's next node
       if (in1) {
         Tile<K> t;
         contract<K>(w, r, t);
-        auto ratio = [&](const Tile<K>& x, Tile<K>& rc) {
+        // (alone: the child comes next, so m0 is its row of maxima by now, with the mark of a state of probability zero)
+        if (alone && (__builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, m0)) & 1)) {
+          Tile<K> own;
+          lean_tile_load<K>(rO, vtile, (own1 >> 3) * (int)d.tile_stride, own);
 #pragma unroll
           for (int kt = 0; kt < K / 16; ++kt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) rc.v[kt][i] = t.v[kt][i] * fminf(__builtin_amdgcn_exp2f(x.v[kt][i]), kFlowRatioCap);
+            for (int i = 0; i < 4; ++i) X1.v[kt][i] = own.v[kt][i] == -INFINITY ? 0.f : X1.v[kt][i];
+#pragma unroll
+          for (int kt = 0; kt < K / 16; ++kt) asm volatile("" : "+v"(X1.v[kt]));
+        }
+        auto ratio = [&](const Tile<K>& x, Tile<K>& rc) {
+#pragma unroll
+          for (int kt = 0; kt < K / 16; ++kt) rc.v[kt] = t.v[kt] * x.v[kt];
         };
-        int next_away = lean_get(sc, kLAway, s);
-        const bool first_away = (fl & 4) != 0;
-        if (first_away) ++next_away;
-        auto hand_on = [&](int c) {
-          const uint32_t sl = (slots >> (8 * c)) & 0xffu;
-          Tile<K> x;
-          lds_tile_load<K>(lds, (int)sl, lane, x);
-          ratio(x, x);
-          if (fl & (2 << c)) {   // away: the slot was only to work in
-            away_put<K>(away, d, next_away++, slice, lane, x);
-            lean_post(state + sl, (2 * ((turns >> (8 * c)) & 0x7fu) + 2) & 0xffu);
-          } else {
-            lds_tile_store<K>(lds, (int)sl, lane, x);
-            lean_post(state + sl, (2 * ((turns >> (8 * c)) & 0x7fu) + 1) & 0xffu);
-          }
-        };
-        if (in2) hand_on(2);
-        if (in3) hand_on(3);
+        const bool first_away = (turns & 0x8000u) != 0;
+        if (in2) {
+          int next_away = lean_get(sc, kLAway, s) + (first_away ? 1 : 0);
+          auto hand_on = [&](int c) {
+            const uint32_t sl = (slots >> (8 * c)) & 0xffu;
+            Tile<K> x;
+            lds_tile_load<K>(lds, (int)sl, lane, x);
+            ratio(x, x);
+            if ((turns >> (8 * c)) & 0x80u) {   // away: the slot was only to work in
+              away_put<K>(away, d, next_away++, slice, vtile, x);
+              lean_post(state + sl, (2 * ((turns >> (8 * c)) & 0x7fu) + 2) & 0xffu);
+            } else {
+              lds_tile_store<K>(lds, (int)sl, lane, x);
+              lean_post(state + sl, (2 * ((turns >> (8 * c)) & 0x7fu) + 1) & 0xffu);
+            }
+          };
+          hand_on(2);
+          if (in3) hand_on(3);
+        }
         ratio(X1, r);
-        if (first_away) away_put<K>(away, d, lean_get(sc, kLAway, s), slice, lane, r);
+        if (first_away) away_put<K>(away, d, lean_get(sc, kLAway, s), slice, vtile, r);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -575,8 +681,8 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_backward_lean_kernel(
     if (base) lean_refill(fields, stride, wave, lane, base, sc);
     const int s_end = min(base + kLeanChunk, n_steps);
     for (int s = base; s < s_end; s += 2) {
-      step(s, wA);
-      step(s + 1, wB);
+      step(s, wA, PA);
+      step(s + 1, wB, PB);
     }
   }
 }
@@ -795,7 +901,7 @@ __global__ __launch_bounds__(kStatLeanWaves * 64) void hclt_stats_lean_kernel(
         if (t_c1 >= 0) child_load(t_c1, xc, so1, C1);
         if (t_c2 >= 0) child_load(t_c2, xc, so1, C2);
         // (2) E, the edge flows, then G = E .* (R W)
-        tile_exp_sub<K>(e, m);
+        tile_exp_sub<K>(e, lean_scale(m));
         {
           // A += R^T E over the 16 examples of the tile (contraction over examples): both operands
           // go through the wave's pad to reach the [state][example] operand layout.  A wave's LDS

@@ -18,7 +18,7 @@
 namespace pcm {
 
 // field rows of a lean schedule, [field][wave][stride]; the names are those of hclt_walk_lean.hip.hpp
-constexpr int kLeanCheckA1 = 2, kLeanCheckSlots = 6, kLeanCheckFlags = 7, kLeanCheckTurns = 8, kLeanCheckFields = 10, kLeanCheckWaves = 16;
+constexpr int kLeanCheckA1 = 2, kLeanCheckSlots = 6, kLeanCheckTurns = 7, kLeanCheckFields = 9, kLeanCheckWaves = 16;
 constexpr uint8_t kLeanCheckKept = 0xfd;   // from here on a slot byte names no slot (another workgroup's / kept in registers / nobody's)
 
 struct LeanSlotOp {
@@ -58,7 +58,7 @@ inline void lean_step_ops(const int32_t* f, int stride, int w, int s, bool forwa
   if (inner[1])
     for (int c = 1; c <= 3; ++c)
       if (inner[c] && sl(c) < kLeanCheckKept)   // (a child in another workgroup: its slot is free again at once)
-        ops.push_back({sl(c), st(c, (get(kLeanCheckFlags) >> (c + 1)) & 1u ? 2 : 1), false});
+        ops.push_back({sl(c), st(c, (turns >> (8 * c)) & 0x80u ? 2 : 1), false});
 }
 
 // -1 if every wave gets through its `n_steps` steps; otherwise step * 16 + wave of the first wave found stuck.

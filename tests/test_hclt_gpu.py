@@ -104,6 +104,44 @@ def test_bushy_trees_keep_the_lean_walks(gpu, oracle, shape):
     assert bpc.size("walk_kernels") == 1
 
 
+@pytest.mark.parametrize("K", [16, 32])
+def test_states_of_probability_zero(gpu, oracle, K):
+    """Half of a node's states without the shown category, and half of the sums over those states only: their value is
+    zero, so their ratio tile must be zero too.  On the way down a node with one inner child reads that child's values only
+    where the forward walk has marked such a state; nodes with two and three inner children beside it."""
+    torch, P = gpu
+    from helpers import correlated_data
+    tree = np.array([-1, 0, 1, 2, 3, 4, 2, 6, 7, 4, 9, 10, 1, 12, 13, 5, 5], np.int32)
+    V, C, B = len(tree), 6, 100
+    rng = np.random.default_rng(K)
+    theta, leaf = oracle.random_hclt_params(tree, K, C, rng)
+    even = np.arange(K) % 2 == 0
+    never = -200.0   # e^-200 is zero in float32 and a number in the float64 oracle, which has no use for log 0
+    normalised = lambda p: np.where(p > 0, np.log(np.maximum(p / p.sum(-1, keepdims=True), 1e-300)), never).astype(np.float32)
+    for v in [v for v in theta if v >= 4]:   # even sums over even states only, below the top
+        t = np.exp(theta[v].astype(np.float64))
+        t[::2] *= even
+        theta[v] = normalised(t)
+    p = np.exp(leaf.astype(np.float64).reshape(V, K, C))
+    p[4:, even, 1::2] = 0.0   # even states never show an odd category
+    leaf = normalised(p).reshape(leaf.shape)
+    fc = oracle.hclt_flat(tree, K, C, theta, leaf)
+    data = correlated_data(B, V, C, 3, tree)
+    ll_ref, _, _, ea_ref, lf_ref = oracle.em_step(fc, data, np.arange(B, dtype=np.int32), 0.1, 0.9, double=True)
+    bpc = P.hclt_from_clt(tree, C, K)
+    th = np.zeros((V, K, K), np.float32)
+    for v, t in theta.items():
+        th[v, :t.shape[0]] = t
+    bpc.set_params(th, leaf)
+    ll = P.probs_flows_circuit(bpc, torch.from_numpy(data).cuda()).cpu().numpy()
+    np.testing.assert_allclose(ll, ll_ref, rtol=1e-5)
+    ea, lf = bpc.get_flows()
+    assert np.isfinite(ea).all() and np.isfinite(lf).all()
+    np.testing.assert_allclose(lf, np.asarray(lf_ref).reshape(V, K, C), rtol=1e-4, atol=1e-5)
+    for v, blk in oracle.hclt_block_aggr(fc, ea_ref).items():
+        np.testing.assert_allclose(ea[v][:blk.shape[0]], blk, rtol=1e-4, atol=1e-5)
+
+
 @pytest.mark.parametrize("V,K,B,reach", [(70, 32, 1, 6), (160, 16, 40, 4), (700, 32, 200, 8), (1300, 32, 33, 40)])
 def test_a_tree_over_several_workgroups(gpu, oracle, V, K, B, reach):
     """Batches of few slices walk one tree in parts, a workgroup each, whose tiles cross through memory: against the
