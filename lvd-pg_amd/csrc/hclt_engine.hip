@@ -205,6 +205,13 @@ void HcltCircuit::build_structure() {
     nd.lc_cnt = (int)cl.size() - nd.lc_off;
     nd.has_inner_child = nd.ic_cnt > 0;
   }
+  std::vector<int32_t> pv((size_t)4 * n_inner_, -1);
+  for (int n = 0; n < n_inner_; ++n) {
+    if (nodes[n].var < Vu_) pv[4 * n] = nodes[n].var;
+    for (int i = 0; i < nodes[n].lc_cnt && i < 3; ++i)
+      if (cl[nodes[n].lc_off + i] < Vu_) pv[4 * n + 1 + i] = cl[nodes[n].lc_off + i];
+  }
+  d_pack_vars_.upload(pv);
   if (ci.empty()) ci.push_back(0);
   if (cl.empty()) cl.push_back(0);
   d_nodes_.upload(nodes);
@@ -1274,6 +1281,12 @@ void HcltCircuit::stage_batch(const BatchRef& b, bool tiles) {
   if (b.batch < 1) fail(PCM_ERR_ARG, "batch must be positive, got %d", b.batch);
   if (tiles) ensure_batch(b.batch); else ensure_staged(b.batch);
   const int Bp = ceil_div(b.batch, kSlice) * kSlice;
+  if (!wide_walk_ && lean_fits(b.batch, tiles ? kKeepAll : kKeepNone) && (int64_t)Bp * Vu_ <= kGatherBytes) {
+    hipLaunchKernelGGL(hclt_gather_x_kernel, dim3(Bp / kSlice, ceil_div(n_inner_, kGatherNodes)), dim3(256), 0, stream,
+                       reinterpret_cast<const int4*>(d_pack_vars_.p), b.d_data, b.stride_ex, b.stride_var, b.d_idx, b.batch, Bp, C_,
+                       n_inner_, d_xn_.p);
+    return check_launch("gather_x");
+  }
   pcm_stage(b.d_data, b.stride_ex, b.stride_var, b.d_idx, b.batch, Bp, Vu_, C_, d_xb_.p, stream);   // (auxiliary rows stay 0)
   check_launch("stage_batch");
   hipLaunchKernelGGL(hclt_pack_x_kernel, dim3(ceil_div(Bp, 1024), n_inner_), dim3(256), 0, stream, d_nodes_.p,

@@ -329,6 +329,7 @@ class HcltCircuit : public pcm_circuit {
   DevBuf<uint32_t> d_ext_ops_;
   DevBuf<float> d_leaf_, d_logtheta_, d_Wf_, d_Wb_, d_edge_aggr_, d_leaf_flow_, d_O_, d_R_, d_G_;
   DevBuf<uint8_t> d_xb_;
+  DevBuf<int32_t> d_pack_vars_;   // per node: the variables of its packed word, -1 where there is none
   DevBuf<uint32_t> d_xn_;
   DevBuf<float> d_leaf_kc_;      // [V][K][C] copy for sampling
   DevBuf<float> d_kld_;          // scratch of the KL recursion
