@@ -1469,6 +1469,7 @@ void SparseCircuit::build_groups(std::vector<int32_t>& group_of, std::vector<int
   g.xm = d_grp_xm_.p;                                                                                                \
   g.logp = d_logp_.p; g.mars = d_mars_.p; g.flows = d_flows_.p; g.edge_part = d_edge_part_.p;                        \
   g.n_nodes = fc_.n_nodes(); g.n_edges = fc_.n_edges(); g.B = batch_; g.Bp = bp_;                                   \
+  g.flow_bytes = d_flows_.n < ((size_t)1 << 29) ? (uint32_t)(d_flows_.n * 4) : 0u;                                   \
   g.inv_f = 1.f; g.norm = d_mars_.p; g.norm_row = fc_.n_nodes()   /* (not tempered: the row of zeros for every sum) */
 
 // exp of the groups' log-parameters, before a forward pass

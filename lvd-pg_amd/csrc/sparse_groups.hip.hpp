@@ -62,6 +62,7 @@ struct GroupDev {
   float* edge_part;       // [Bp / 64][n_edges]
   int64_t n_nodes, n_edges;
   int32_t B, Bp;
+  uint32_t flow_bytes;    // size of the flow array, 0 from 2 GiB on (its rows are then addressed by pointers)
   // tempered flows (fscale of mini_batch_em_beta): shares to the power inv_f = 1 / fscale, normalised again by the
   // sums' rows of `norm` (row norm_row for every sum if it is >= 0: the row of zeros of a pass that is not tempered)
   float inv_f;
@@ -412,6 +413,28 @@ __device__ __forceinline__ void group_backward_body(const GroupDev& d, const Gro
     const bool tiny = middle && __any((int32_t)signs < 0);
     if (high || tiny)
       group_shares_by_edge<NG, Cp>(d, node, col, mb, tiny, d.edge + base.pw0 + (int64_t)bx * Gp * Cp + ct * 16 + 4 * hi, e[s], out);
+    if (d.flow_bytes) {
+      // Row -1 of a buffer lies past its end and a store there goes nowhere, so the copies go out without a branch per row;
+      // one test in eight is left, whether any child of the tile has a copy of that rank (they fill up from the front).
+      // (A branch per row, 32 a tile: 192 variables, 128 heads, 512 examples: a walk down 37 layers 137 us, without 102.  The
+      // same for the rows read and written on the way up loses, 48 -> 102 us a walk.)
+      const __amdgpu_buffer_rsrc_t rf = __builtin_amdgcn_make_buffer_rsrc(d.flows, 0, (int)d.flow_bytes, 0x00020000);
+      const int col4 = (int)col * 4;
+      auto put = [&](const int r0, const int r1, const int r2, const int r3) {
+        if (!__any((r0 & r1 & r2 & r3) >= 0)) return false;
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, out[0]), rf, r0 * (d.Bp * 4) + col4, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, out[1]), rf, r1 * (d.Bp * 4) + col4, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, out[2]), rf, r2 * (d.Bp * 4) + col4, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, out[3]), rf, r3 * (d.Bp * 4) + col4, 0, 0);
+        return true;
+      };
+      const int4* const p = cpa[s];
+      const int4* const q = cpb[s];
+      (void)(put(p[0].x, p[1].x, p[2].x, p[3].x) && put(p[0].y, p[1].y, p[2].y, p[3].y) && put(p[0].z, p[1].z, p[2].z, p[3].z) &&
+             put(p[0].w, p[1].w, p[2].w, p[3].w) && put(q[0].x, q[1].x, q[2].x, q[3].x) && put(q[0].y, q[1].y, q[2].y, q[3].y) &&
+             put(q[0].z, q[1].z, q[2].z, q[3].z) && put(q[0].w, q[1].w, q[2].w, q[3].w));
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float f = out[i];
