@@ -221,6 +221,22 @@ void HcltCircuit::build_structure() {
   if (block_) build_schedules();
 }
 
+LeanTree HcltCircuit::lean_tree() const {
+  LeanTree t;
+  t.parent.assign(n_inner_, -1);
+  t.inner.resize(n_inner_);
+  t.tree = tree_of_inner_;
+  for (int n = 0; n < n_inner_; ++n) {
+    const int v = var_of_inner_[n];
+    t.depth.push_back(depth_[v]);
+    if (parent_[v] >= 0) t.parent[n] = inner_of_var_[parent_[v]];
+    for (int c : children_[v])
+      if (!children_[c].empty()) t.inner[n].push_back(inner_of_var_[c]);
+  }
+  t.complete();
+  return t;
+}
+
 // Step schedules of the two tree walks.  Every step holds at most kWalkWaves nodes whose
 // dependencies were produced in earlier steps; among the ready nodes those with the longest
 // remaining chain go first (for unit-time tasks on a tree this greedy rule gives the fewest
@@ -309,12 +325,7 @@ void HcltCircuit::build_schedules() {
       }
     dst.upload(f);
   };
-  LeanTree lt;
-  lt.parent = par;
-  lt.inner = ic;
-  lt.tree = tree_of_inner_;
-  for (int n = 0; n < n_inner_; ++n) lt.depth.push_back(depth_[var_of_inner_[n]]);
-  lt.complete();
+  const LeanTree lt = lean_tree();
   // field rows of the lean walks (see hclt_walk_lean.hip.hpp) from their own schedule, with the same padding, or none if
   // some node has more operands than the lean kernels hold
   const size_t leaf_stride = (size_t)C_ * K_ * sizeof(float);
@@ -554,6 +565,7 @@ void HcltCircuit::build_schedules() {
   // A plan: the schedules of a walk in G groups, which the kernels take in blockIdx.y: groups of whole trees, or the parts of
   // one tree.  A node's arithmetic does not depend on the group it is walked in, so its results are the same bits under
   // every plan.  Going up the top of a tree is the last group, going down the first: whoever is waited for comes first.
+  std::vector<int32_t> lean_rows;   // of all plans: one upload
   auto make_plan = [&](const std::vector<LeanScope>& scopes, const std::vector<int32_t>& part) {
     std::unique_ptr<LeanPlan> plan(new LeanPlan);
     const int G = (int)scopes.size();
@@ -591,7 +603,8 @@ void HcltCircuit::build_schedules() {
       }
       (forward ? plan->n_fwd_steps : plan->n_bwd_steps) = steps;
       (forward ? plan->fwd_stride : plan->bwd_stride) = stride;
-      (forward ? plan->fwd : plan->bwd).upload(rows);
+      (forward ? plan->fwd_at : plan->bwd_at) = lean_rows.size();
+      lean_rows.insert(lean_rows.end(), rows.begin(), rows.end());
     }
     return plan;
   };
@@ -634,6 +647,7 @@ void HcltCircuit::build_schedules() {
       plans_.push_back(std::move(plan));
     }
   }
+  if (!plans_.empty()) d_lean_rows_.upload(lean_rows);
   if (away_parts) {
     d_away_tiles_.alloc(std::max<size_t>(away_tiles, 1) * kSlice * K_);
     d_away_sums_.alloc(away_parts * kSlice);
@@ -1327,7 +1341,7 @@ void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
     auto launch_lean = [&](auto kernel) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
       const LeanPlan* lp = lean_plan(d.nslices);
-      PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, lp->fwd.p, lp->fwd_stride, d_ll,
+      PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, d_lean_rows_.p + lp->fwd_at, lp->fwd_stride, d_ll,
                        lds_slots_, away());
     };
     PCM_DISPATCH_LEAN_K(K_, {
@@ -1355,7 +1369,7 @@ void HcltCircuit::run_backward(const HcltDev& d) {
     auto launch_lean = [&](auto kernel) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
       const LeanPlan* lp = lean_plan(d.nslices);
-      PCM_LAUNCH_PHASE(1, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, lp->bwd.p, lp->bwd_stride,
+      PCM_LAUNCH_PHASE(1, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, d_lean_rows_.p + lp->bwd_at, lp->bwd_stride,
                        lds_slots_, away());
     };
     PCM_DISPATCH_LEAN_K(K_, {

@@ -36,6 +36,8 @@ constexpr double kLeanStretch = 1.4;
 // average, while the largest part goes on shrinking by a quarter.  Below that the crossings cost what the parts gain: 153
 // nodes at 512 examples forward 42 us in one part, 50 in six; 632 nodes 97 in one, 95 in four (backward 125 and 107).  A tile
 // from another workgroup is expected kLeanAwaySteps steps after the step it is sent in.
+// The chains of the row queries: parts, and nodes that make a part worth its launches.
+constexpr int kKlMostParts = 8, kKlPartNodes = 24;
 constexpr int kLeanMostParts = 16, kLeanPartNodes = 80, kLeanAwaySteps = 4;
 constexpr int kPre = 3;          // static operand tiles a wave requests one step ahead
 
@@ -147,6 +149,8 @@ struct HcltDev {
   }
 
 struct LeanAway;
+struct LeanTree;
+struct KlRowStrides;
 
 class HcltCircuit : public pcm_circuit {
  public:
@@ -230,6 +234,11 @@ class HcltCircuit : public pcm_circuit {
   }
   void read_timing(float* ms, int n);
 
+  // a workgroup's walk over its part of the tree in the KL recursion's chains: its first item, its steps, and what it needs
+  // of other parts
+  struct KlWalk { int32_t item0, steps, away0, n_away; };
+  struct KlPart { KlWalk up, down; };
+
  private:
   int V_, K_, C_, n_inner_, root_;
   int Vu_ = 0;                     // the caller's variables; V_ - Vu_ auxiliary ones behind them (forests only)
@@ -242,9 +251,10 @@ class HcltCircuit : public pcm_circuit {
   // whose slices do not fill the device), fewest groups first
   struct LeanPlan {
     int n_groups = 1, n_away = 0, n_fwd_steps = 0, fwd_stride = 0, n_bwd_steps = 0, bwd_stride = 0;
-    DevBuf<int32_t> fwd, bwd;
+    size_t fwd_at = 0, bwd_at = 0;   // its field rows in d_lean_rows_
   };
   std::vector<std::unique_ptr<LeanPlan>> plans_;   // empty: the lean kernels do not take this tree
+  DevBuf<int32_t> d_lean_rows_;
   const LeanPlan* lean_plan(int nslices) const;
   // what crosses the parts of a tree: for every plan with as many slices as it is taken for
   DevBuf<float> d_away_tiles_;
@@ -380,6 +390,27 @@ class HcltCircuit : public pcm_circuit {
   DevBuf<int32_t> d_kl_ext_;              // chain slots of the children past the second, of nodes with more than three
   int kl_up_steps_ = 0, kl_down_steps_ = 0;
   int kl_ring_slots_ = 0;                 // slots of the chains' LDS ring; 0: levels too wide, the ring is the whole chain in device memory
+  // the chains of the row queries (see kl_view): tables of one workgroup per row, or of a tree in parts
+  struct KlPlan {
+    bool ok = false;
+    int W = 0, slots = 0, most_away = 0;
+    size_t su = 0, sd = 0;
+    DevBuf<int32_t> tab;
+    size_t up = 0, down = 0, pos = 0, ext = 0, away = 0, parts = 0;   // where in `tab`
+  };
+  struct KlView {
+    int G, W, mask;
+    bool lds;
+    size_t lds_bytes, su, sd;
+    const int32_t *up, *down, *ext, *pos, *away;
+    const KlPart* parts;
+  };
+  KlPlan kl_plans_[2];
+  KlView kl_view(int rows);
+  void build_kl_plan(const LeanTree& t, KlPlan& p, int G);
+  void kl_chain(const KlView& v, bool up, int rows, const float* pu, const float* base, const float* ell, const float* pd,
+                float* ring_up, float* ring_down, float* klv, float* z, float* h, const KlRowStrides& strides);
+  LeanTree lean_tree() const;
   HcltCircuit* same_tree(pcm_circuit* q);
   void build_kld_tables();
   void build_block_params();

@@ -21,6 +21,7 @@
 // the chain runs at the rate one compute unit pulls the parameters from L2.  Everything else is
 // a data-parallel kernel.
 #include "hclt_engine.hpp"
+#include "lean_schedule.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -74,6 +75,12 @@ static_assert(sizeof(KlItem) == 16, "KlItem is read as one 16-byte word");
 // requested ahead: as many as its registers hold.
 constexpr int kl_waves(int K) { return K > 32 ? 8 : 16; }
 constexpr int kl_ahead(int K) { return K > 32 ? 2 : 4; }
+
+// A chain over several workgroups: the part of a tree one of them walks (lean_parts), in the order of HcltCircuit::KlPart.
+// The vectors its nodes need from another part are in device memory when its launch begins (the parts below the top go up
+// in a launch before it and down in one behind it) and are brought into LDS, behind the ring, before the first step:
+// slot kKlAway + e names the e-th of them.
+constexpr int kKlAway = 1 << 28;
 
 // Operand layout of the chains: lane (part, r) of a wave, part = lane / K, r = lane % K, owns
 // rows part * JP .. + JP (JP = K * K / 64) of its node's K x K operand at column r; the JP values
@@ -145,17 +152,23 @@ struct KlRowStrides {
 // operand and constants of a step are requested D = kl_ahead(K) steps before it; the chains are
 // padded to a multiple of D steps and the tables by D idle steps more, so the requests need no
 // bounds and every lane's requests complete in the order the steps use them.
+// `parts` (null: the whole tree): blockIdx.x is a part from `part0` on, and rs.down_only says which way it goes; the number of
+// waves is the launch's.  A step of sixteen nodes is 66 KB of operands, which one compute unit pulls at 75 GB/s, so a matrix
+// of few rows spends its time here with most of the device idle: 16 rows of the 3072-variable circuit, a chain 278 us on 16
+// workgroups, 111 in eight parts each (the parts below the top in one launch, the top in another).
 template <int K, bool kLds>
 __global__ __launch_bounds__(kl_waves(K) * 64) void hclt_kld_chain_kernel(
     const KlItem* __restrict__ up_items, int up_steps, const KlItem* __restrict__ down_items, int down_steps,
     const int32_t* __restrict__ ext, const float* __restrict__ pu, const float* __restrict__ base,
     const float* __restrict__ ell, const float* __restrict__ pd, int ring_mask, float* ring_up, float* ring_down,
-    float* __restrict__ klv, float* __restrict__ z, float* __restrict__ h, KlRowStrides rs) {
-  constexpr int PARTS = 64 / K, JP = K / PARTS, Q = JP / 4, W = kl_waves(K), D = kl_ahead(K);
+    float* klv, float* __restrict__ z, float* h, KlRowStrides rs, const HcltCircuit::KlPart* __restrict__ parts, int part0,
+    const int32_t* __restrict__ away) {
+  constexpr int PARTS = 64 / K, JP = K / PARTS, Q = JP / 4, D = kl_ahead(K);
+  const int W = blockDim.x >> 6;
   extern __shared__ float lds_ring[];   // kLds: [ring_mask + 1][K]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane % K, part = lane / K;
-  const bool up = blockIdx.x == 0 && !rs.down_only;
+  const bool up = parts ? !rs.down_only : blockIdx.x == 0 && !rs.down_only;
   {   // a row of a parameter matrix per blockIdx.y: its operands, constants and results sit rs.* floats further on
     const size_t row = blockIdx.y;
     pu += row * rs.pu; pd += row * rs.pd; base += row * rs.vec; ell += row * rs.vec;
@@ -163,17 +176,26 @@ __global__ __launch_bounds__(kl_waves(K) * 64) void hclt_kld_chain_kernel(
     if (ring_up) ring_up += row * rs.ring_up;
     if (ring_down) ring_down += row * rs.ring_down;
   }
-  const int steps = up ? up_steps : down_steps;
+  HcltCircuit::KlWalk walk{0, up ? up_steps : down_steps, 0, 0};
+  if (parts) walk = up ? parts[part0 + blockIdx.x].up : parts[part0 + blockIdx.x].down;
+  const int steps = walk.steps;
   const int4* __restrict__ items = reinterpret_cast<const int4*>(up ? up_items : down_items);
   const float4* __restrict__ par = reinterpret_cast<const float4*>(up ? pu : pd);
   float* ring_dev = up ? ring_up : ring_down;
   auto ring_at = [&](int slot) -> float* {
-    if constexpr (kLds) return lds_ring + (size_t)(slot & ring_mask) * K;
+    if constexpr (kLds) return lds_ring + (size_t)(slot >= kKlAway ? ring_mask + 1 + (slot - kKlAway) : slot & ring_mask) * K;
     else return ring_dev + (size_t)slot * K;
   };
   // The first round (q0 = -D) computes nothing and only places the requests of steps 0 .. D-1:
   // with every request issued from the same place in the loop, the waits the compiler counts
   // from the order of issue let D - 1 steps of requests stay in flight.
+  if constexpr (kLds)
+    if (walk.n_away) {
+      const float* const from = up ? klv : h;
+      for (int i = threadIdx.x; i < walk.n_away * K; i += blockDim.x)
+        lds_ring[(size_t)(ring_mask + 1) * K + i] = from[(size_t)away[walk.away0 + i / K] * K + i % K];
+      __syncthreads();
+    }
   int4 it[D];
   float4 p[D][Q];
   float bs[D], el[D];
@@ -230,7 +252,7 @@ __global__ __launch_bounds__(kl_waves(K) * 64) void hclt_kld_chain_kernel(
           }
         }
       }
-      const size_t nx = (size_t)(slot + D * W);
+      const size_t nx = (size_t)(walk.item0 + slot + D * W);
       it[d] = items[nx];
 #pragma unroll
       for (int e = 0; e < Q; ++e) p[d][e] = par[(nx * Q + e) * 64 + lane];
@@ -515,7 +537,194 @@ void HcltCircuit::build_kld_tables() {
     t[(size_t)n_inner_ + v] = children_[v].empty() ? inner_of_var_[parent_[v]] : inner_of_var_[v];
   for (size_t q = 0; q < input_order_.size(); ++q) t[(size_t)n_inner_ + V_ + input_order_[q]] = (int32_t)q;
   d_kl_tabs_.upload(t, stream);
+  // (both plans now: a call for other numbers of rows builds nothing)
+  if (block_ && n_inner_ >= kKlMostParts / 2 * kKlPartNodes) {
+    const LeanTree lt = lean_tree();
+    for (int i = 0; i < 2; ++i)
+      if (n_inner_ >= (kKlMostParts >> i) * kKlPartNodes) build_kl_plan(lt, kl_plans_[i], kKlMostParts >> i);
+  }
   d_kl_up_.upload(raw, stream);   // last: marks the tables as built
+}
+
+// The chains of the row queries: in parts where the rows leave most of the device idle 
+// and LDS holds every vector of a part, else on the tables above.
+HcltCircuit::KlView HcltCircuit::kl_view(int rows) {
+  build_kld_tables();
+  const int D = kl_ahead(K_);
+  KlView v;
+  v.G = 1;
+  v.W = kl_waves(K_);
+  v.lds = kl_ring_slots_ > 0;
+  v.mask = kl_ring_slots_ - 1;
+  v.lds_bytes = (size_t)kl_ring_slots_ * K_ * sizeof(float);
+  v.su = (size_t)(kl_up_steps_ + D) * v.W;
+  v.sd = (size_t)(kl_down_steps_ + D) * v.W;
+  v.up = d_kl_up_.p;
+  v.down = d_kl_down_.p;
+  v.ext = d_kl_ext_.p;
+  v.pos = d_kl_pos_.p;
+  v.parts = nullptr;
+  v.away = nullptr;
+  for (int i = 0; i < 2; ++i) {
+    const int G = kKlMostParts >> i;
+    const KlPlan& p = kl_plans_[i];
+    if (!p.ok || (int64_t)rows * G > n_cus_) continue;
+    v.G = G;
+    v.W = p.W;
+    v.lds = true;
+    v.mask = p.slots - 1;
+    v.lds_bytes = (size_t)(p.slots + p.most_away) * K_ * sizeof(float);
+    v.su = p.su;
+    v.sd = p.sd;
+    v.up = p.tab.p + p.up;
+    v.down = p.tab.p + p.down;
+    v.ext = p.tab.p + p.ext;
+    v.pos = p.tab.p + p.pos;
+    v.away = p.tab.p + p.away;
+    v.parts = reinterpret_cast<const KlPart*>(p.tab.p + p.parts);
+    break;
+  }
+  return v;
+}
+
+void HcltCircuit::build_kl_plan(const LeanTree& t, KlPlan& p, int G) {
+  const int D = kl_ahead(K_), W = p.W = std::max(4, kl_waves(K_) * 2 / G);
+  int largest = 0;
+  const std::vector<int32_t> part = lean_parts(t, G, &largest);
+  if (largest > n_inner_ / 2) return;   // (the top alone is most of the tree)
+  std::vector<int32_t> pos((size_t)2 * n_inner_, 0), ext, away;
+  std::vector<KlItem> all[2];
+  std::vector<KlPart> parts(G);
+  std::vector<std::vector<int32_t>> nodes(G);
+  for (int n = 0; n < n_inner_; ++n) nodes[part[n]].push_back(n);
+  std::vector<int32_t> pending(n_inner_);
+  std::vector<char> waiting(n_inner_);
+  all[0].reserve((size_t)4 * n_inner_);
+  all[1].reserve((size_t)4 * n_inner_);
+  int reach = 0;
+  for (int dir = 0; dir < 2; ++dir) {
+    const bool up = dir == 0;
+    std::fill(pending.begin(), pending.end(), 0);
+    std::fill(waiting.begin(), waiting.end(), 0);
+    int32_t* const at = pos.data() + (up ? 0 : n_inner_);
+    for (int g = 0; g < G; ++g) {
+      KlWalk& walk = up ? parts[g].up : parts[g].down;
+      const int first = (int)all[dir].size();
+      walk.item0 = first;
+      walk.away0 = (int)away.size();
+      // a step takes up to W nodes whose neighbours came in earlier steps, deepest (down: longest chain) first
+      LeanHeap ready;
+      auto add = [&](int n) {
+        waiting[n] = 1;
+        ready.push(up ? -t.depth[n] : -t.chain[n], 0, n);
+      };
+      int left = (int)nodes[g].size();
+      for (const int n : nodes[g]) {
+        if (up) {
+          for (int c : t.inner[n]) pending[n] += part[c] == g;
+        } else {
+          pending[n] = t.parent[n] >= 0 && part[t.parent[n]] == g;
+        }
+        if (!pending[n]) add(n);
+      }
+      const KlItem idle{-1, {-1, -1, -1}};
+      std::vector<KlItem>& items = all[dir];   // (slots count from the part's first)
+      std::vector<int32_t> now, cs;
+      while (left > 0) {
+        now.clear();
+        for (int v; (int)now.size() < W && (v = ready.top(waiting)) >= 0;) {
+          waiting[v] = 0;
+          now.push_back(v);
+        }
+        for (int n : now) {
+          KlItem it = idle;
+          it.n = n;
+          const int32_t me = (int32_t)items.size() - first;
+          auto slot_of = [&](int from) -> int32_t {   // where the vector of a neighbour is: in the ring, or behind it
+            if (part[from] == g) {
+              const int32_t sl = at[from] - first;
+              reach = std::max(reach, me - sl);
+              return sl;
+            }
+            away.push_back(from);
+            return kKlAway + (int32_t)away.size() - 1 - walk.away0;
+          };
+          if (up) {
+            cs.clear();
+            for (int c : t.inner[n]) cs.push_back(slot_of(c));
+            for (size_t i = 0; i < cs.size() && i < 3; ++i) it.c[i] = cs[i];
+            if (cs.size() > 3) {
+              it.c[2] = -((int32_t)ext.size() + 2);
+              ext.push_back((int32_t)cs.size() - 2);
+              ext.insert(ext.end(), cs.begin() + 2, cs.end());
+            }
+          } else if (t.parent[n] >= 0) {
+            it.c[0] = slot_of(t.parent[n]);
+          }
+          at[n] = first + me;
+          items.push_back(it);
+          --left;
+        }
+        while ((items.size() - first) % W) items.push_back(idle);
+        for (int n : now) {
+          if (up) {
+            if (t.parent[n] >= 0 && part[t.parent[n]] == g && --pending[t.parent[n]] == 0) add(t.parent[n]);
+          } else {
+            for (int c : t.inner[n])
+              if (part[c] == g) add(c);
+          }
+        }
+      }
+      while ((items.size() - first) % ((size_t)D * W)) items.push_back(idle);   // whole rounds of D steps
+      walk.steps = (int)((items.size() - first) / W);
+      walk.n_away = (int)away.size() - walk.away0;
+      p.most_away = std::max(p.most_away, walk.n_away);
+      items.resize(items.size() + (size_t)D * W, idle);   // idle steps for the requests that run ahead
+    }
+  }
+  p.slots = 1;
+  while (p.slots < reach + W) p.slots <<= 1;
+  if ((size_t)(p.slots + p.most_away) * K_ * sizeof(float) > (size_t)max_lds_) return;
+  p.su = all[0].size();
+  p.sd = all[1].size();
+  std::vector<int32_t> tab;   // one upload
+  auto put = [&](const void* q, size_t bytes) {
+    while (tab.size() % 4) tab.push_back(0);
+    const size_t at = tab.size();
+    tab.resize(at + bytes / 4);
+    if (bytes) std::memcpy(tab.data() + at, q, bytes);
+    return at;
+  };
+  p.up = put(all[0].data(), all[0].size() * sizeof(KlItem));
+  p.down = put(all[1].data(), all[1].size() * sizeof(KlItem));
+  p.pos = put(pos.data(), pos.size() * 4);
+  p.ext = put(ext.data(), ext.size() * 4);
+  p.away = put(away.data(), away.size() * 4);
+  p.parts = put(parts.data(), parts.size() * sizeof(KlPart));
+  p.tab.upload(tab, stream);
+  p.ok = true;
+}
+
+void HcltCircuit::kl_chain(const KlView& v, bool up, int rows, const float* pu, const float* base, const float* ell, const float* pd,
+                           float* ring_up, float* ring_down, float* klv, float* z, float* h, const KlRowStrides& strides) {
+  KlRowStrides rs = strides;
+  rs.down_only = up ? 0 : 1;
+  PCM_DISPATCH_K(K_, {
+    auto launch = [&](auto kernel, int part0, int n_parts) {
+      if (v.lds_bytes > (size_t)64 * 1024)
+        PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)v.lds_bytes));
+      hipLaunchKernelGGL(kernel, dim3(n_parts, rows), dim3(v.W * 64), v.lds ? v.lds_bytes : 0, stream,
+                         reinterpret_cast<const KlItem*>(v.up), kl_up_steps_, reinterpret_cast<const KlItem*>(v.down),
+                         kl_down_steps_, v.ext, pu, base, ell, pd, v.mask, ring_up, ring_down, klv, z, h, rs, v.parts, part0, v.away);
+    };
+    auto all = [&](auto kernel) {
+      if (v.G == 1) return launch(kernel, 0, 1);
+      if (up) launch(kernel, 1, v.G - 1);
+      launch(kernel, 0, 1);
+      if (!up) launch(kernel, 1, v.G - 1);
+    };
+    if (v.lds) all(&hclt_kld_chain_kernel<KK, true>); else all(&hclt_kld_chain_kernel<KK, false>);
+  });
 }
 
 // Runs the recursion of this circuit (p) against q; with_down also leaves h.
@@ -550,7 +759,8 @@ void HcltCircuit::kld_device(HcltCircuit* q, bool with_down) {
       hipLaunchKernelGGL(kernel, dim3(with_down ? 2 : 1), dim3(kl_waves(KK) * 64), lds, stream,
                          reinterpret_cast<const KlItem*>(d_kl_up_.p), kl_up_steps_,
                          reinterpret_cast<const KlItem*>(d_kl_down_.p), kl_down_steps_, d_kl_ext_.p, pu, base, ell, pd,
-                         kl_ring_slots_ - 1, ring_up, ring_down, klv, z, h, KlRowStrides{0, 0, 0, 0, 0, 0, 0});
+                         kl_ring_slots_ - 1, ring_up, ring_down, klv, z, h, KlRowStrides{0, 0, 0, 0, 0, 0, 0},
+                         (const KlPart*)nullptr, 0, (const int32_t*)nullptr);
     };
     if (kl_ring_slots_) chain(&hclt_kld_chain_kernel<KK, true>, (size_t)kl_ring_slots_ * KK * sizeof(float));
     else chain(&hclt_kld_chain_kernel<KK, false>, 0);
@@ -861,7 +1071,7 @@ void HcltCircuit::build_block_params() {
 void HcltCircuit::kld_rows_block(const float* d_p1, const float* d_p2, int64_t sr, int64_t sp, int32_t rows, bool norm,
                                  float* d_klds, float* d_g1, float* d_g2) {
   const bool with_down = d_g1 != nullptr;
-  build_kld_tables();
+  const KlView kv = kl_view(rows);
   const int64_t ns = (int64_t)sum_param_src_.size();
   const int64_t n = size(0);
   build_block_params();
@@ -877,16 +1087,15 @@ void HcltCircuit::kld_rows_block(const float* d_p1, const float* d_p2, int64_t s
     g1 = d_rows_pg1_.p;
     g2 = d_rows_pg2_.p;
   }
-  const int W = kl_waves(K_), D = kl_ahead(K_);
   const size_t nk = (size_t)n_inner_ * K_, vk = (size_t)V_ * K_;
-  const size_t su = (size_t)(kl_up_steps_ + D) * W, sd = (size_t)(kl_down_steps_ + D) * W, sm = std::max(su, sd);
+  const size_t su = kv.su, sd = kv.sd, sm = std::max(su, sd);
   KlRowStrides rs;
   rs.pu = su * K_ * K_;
   rs.pd = with_down ? sd * K_ * K_ : 0;
   rs.vec = sm * K_;
   rs.out = nk;
-  rs.ring_up = kl_ring_slots_ ? 0 : su * K_;
-  rs.ring_down = kl_ring_slots_ ? 0 : sd * K_;
+  rs.ring_up = kv.lds ? 0 : su * K_;
+  rs.ring_down = kv.lds ? 0 : sd * K_;
   rs.down_only = 0;
   const size_t per_row = vk + 2 * rs.vec + rs.pu + rs.pd + 3 * nk + rs.ring_up + rs.ring_down;
   // rows at a time: what keeps the scratch arrays within 8 GB
@@ -900,8 +1109,8 @@ void HcltCircuit::kld_rows_block(const float* d_p1, const float* d_p2, int64_t s
   float* klv = pu + (size_t)chunk * (rs.pu + rs.pd);
   float* z = klv + (size_t)chunk * nk;
   float* h = z + (size_t)chunk * nk;
-  float* ring_up = kl_ring_slots_ ? nullptr : h + (size_t)chunk * nk;
-  float* ring_down = kl_ring_slots_ ? nullptr : ring_up + (size_t)chunk * rs.ring_up;
+  float* ring_up = kv.lds ? nullptr : h + (size_t)chunk * nk;
+  float* ring_down = kv.lds ? nullptr : ring_up + (size_t)chunk * rs.ring_up;
   // (klv, z and h of a row sit nk apart per row, not behind one another: rs.out strides each of them)
   const int n_inputs = (int)input_order_.size();
   const bool vec = C_ % 4 == 0 && n % 4 == 0 && ns % 4 == 0 && ((reinterpret_cast<uintptr_t>(p1) | reinterpret_cast<uintptr_t>(p2)) & 15) == 0;
@@ -912,23 +1121,10 @@ void HcltCircuit::kld_rows_block(const float* d_p1, const float* d_p2, int64_t s
     const int rc = std::min(chunk, rows - r0);
     const float* q1 = p1 + (size_t)r0 * n;
     const float* q2 = p2 + (size_t)r0 * n;
-    auto chain = [&](int down_only) {   // one workgroup per row, up the tree or down it
-      KlRowStrides r2 = rs;
-      r2.down_only = down_only;
-      PCM_DISPATCH_K(K_, {
-        auto launch = [&](auto kernel, size_t lds) {
-          hipLaunchKernelGGL(kernel, dim3(1, rc), dim3(kl_waves(KK) * 64), lds, stream,
-                             reinterpret_cast<const KlItem*>(d_kl_up_.p), kl_up_steps_,
-                             reinterpret_cast<const KlItem*>(d_kl_down_.p), kl_down_steps_, d_kl_ext_.p, pu, base, ell, pd,
-                             kl_ring_slots_ - 1, ring_up, ring_down, klv, z, h, r2);
-        };
-        if (kl_ring_slots_) launch(&hclt_kld_chain_kernel<KK, true>, (size_t)kl_ring_slots_ * KK * sizeof(float));
-        else launch(&hclt_kld_chain_kernel<KK, false>, 0);
-      });
-    };
+    auto chain = [&](int down_only) { kl_chain(kv, !down_only, rc, pu, base, ell, pd, ring_up, ring_down, klv, z, h, rs); };
     auto base_pass = [&](const float* leaf_terms, float* up, float* down) {
       PCM_DISPATCH_K(K_, hipLaunchKernelGGL(hclt_rows_base_kernel<KK>, dim3(n_inner_, rc), dim3(256), 0, stream, d_nodes_.p,
-                                            d_child_leaf_.p, d_kl_pos_.p, n_inner_, d_blk2par_.p, q1, q2, (size_t)n, leaf_terms,
+                                            d_child_leaf_.p, kv.pos, n_inner_, d_blk2par_.p, q1, q2, (size_t)n, leaf_terms,
                                             vk, Vu_, ell, base, up, down, rs));
     };
     if (!with_down) {
@@ -957,7 +1153,7 @@ void HcltCircuit::kld_rows_block(const float* d_p1, const float* d_p2, int64_t s
         hipLaunchKernelGGL(hclt_rows_leaf_kl_grad_kernel<false>, ggrid, dim3(256), 0, stream, q1, q2, (size_t)n, (size_t)ns, C_, K_,
                            n_inputs, L, d_input_order_.p, d_kl_tabs_.p + n_inner_, h, nk, vk, kl_leaf, o1, o2);
       PCM_DISPATCH_K(K_, hipLaunchKernelGGL(hclt_rows_soft_base2_kernel<KK>, dim3(n_inner_, rc), dim3(256), 0, stream, d_nodes_.p,
-                                            d_child_leaf_.p, d_kl_pos_.p, n_inner_, kl_leaf, vk, Vu_, pd, ell, base, rs, 1));
+                                            d_child_leaf_.p, kv.pos, n_inner_, kl_leaf, vk, Vu_, pd, ell, base, rs, 1));
       chain(0);
       hipLaunchKernelGGL(hclt_rows_edge_grad_kernel, dim3((unsigned)ceil_div(ns, 256), ceil_div(rc, kEdgeGradRows)), dim3(256), 0,
                          stream, ns, K_, d_sum_param_src_.p, d_kl_tabs_.p, q1, q2, (size_t)n, z, h, nk, rc, o1, o2);
@@ -1178,21 +1374,20 @@ void HcltCircuit::gumbel_sample_rows(const float* d_params, int64_t sr, int64_t 
   if (sr == 0 || sp == 0) fail(PCM_ERR_ARG, "parameter matrix strides must not be zero");
   if (!d_out) fail(PCM_ERR_ARG, "output pointer is null");
   if (!(temperature > 0.f)) fail(PCM_ERR_ARG, "temperature must be positive");
-  build_kld_tables();
+  const KlView kv = kl_view(rows);
   const int64_t ns = (int64_t)sum_param_src_.size();
   const int64_t n = size(0);
   build_block_params();
   const float* p = rows_packed_in(d_params, sr, sp, rows, n, d_rows_pk1_, stream);
-  const int W = kl_waves(K_), D = kl_ahead(K_);
   const size_t nk = (size_t)n_inner_ * K_;
-  const size_t su = (size_t)(kl_up_steps_ + D) * W, sd = (size_t)(kl_down_steps_ + D) * W, sm = std::max(su, sd);
+  const size_t su = kv.su, sd = kv.sd, sm = std::max(su, sd);
   KlRowStrides rs;
   rs.pu = 0;               // (a chain that walks down reads no upward operand; the constants it requests are not used)
   rs.pd = sd * K_ * K_;
   rs.vec = sm * K_;
   rs.out = nk;
   rs.ring_up = 0;
-  rs.ring_down = kl_ring_slots_ ? 0 : sd * K_;
+  rs.ring_down = kv.lds ? 0 : sd * K_;
   rs.down_only = 1;
   const size_t per_row = rs.pd + rs.vec + nk + rs.ring_down;
   const int chunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)rows, ((size_t)2 << 30) / per_row));
@@ -1200,7 +1395,7 @@ void HcltCircuit::gumbel_sample_rows(const float* d_params, int64_t sr, int64_t 
   float* pd = d_rows_scratch_.p;
   float* vec = pd + (size_t)chunk * rs.pd;
   float* h = vec + (size_t)chunk * rs.vec;
-  float* ring_down = kl_ring_slots_ ? nullptr : h + (size_t)chunk * nk;
+  float* ring_down = kv.lds ? nullptr : h + (size_t)chunk * nk;
   float* pu = d_rows_scratch_.p + (size_t)chunk * per_row;   // never used, but named by the kernel's requests
   const float inv_t = 1.f / temperature;
   for (int r0 = 0; r0 < rows; r0 += chunk) {
@@ -1208,17 +1403,10 @@ void HcltCircuit::gumbel_sample_rows(const float* d_params, int64_t sr, int64_t 
     const float* q = p + (size_t)r0 * n;
     const float* g = d_noise ? d_noise + (size_t)r0 * ns : nullptr;
     PCM_DISPATCH_K(K_, {
-      hipLaunchKernelGGL(hclt_rows_soft_base_kernel<KK>, dim3(n_inner_, rc), dim3(256), 0, stream, d_kl_pos_.p, n_inner_,
+      hipLaunchKernelGGL(hclt_rows_soft_base_kernel<KK>, dim3(n_inner_, rc), dim3(256), 0, stream, kv.pos, n_inner_,
                          d_blk2par_.p, q, (size_t)n, g, (size_t)ns, inv_t, pd, (float*)nullptr, rs);
-      auto chain = [&](auto kernel, size_t lds) {
-        hipLaunchKernelGGL(kernel, dim3(1, rc), dim3(kl_waves(KK) * 64), lds, stream,
-                           reinterpret_cast<const KlItem*>(d_kl_up_.p), kl_up_steps_,
-                           reinterpret_cast<const KlItem*>(d_kl_down_.p), kl_down_steps_, d_kl_ext_.p, pu, vec, vec, pd,
-                           kl_ring_slots_ - 1, (float*)nullptr, ring_down, h, h, h, rs);
-      };
-      if (kl_ring_slots_) chain(&hclt_kld_chain_kernel<KK, true>, (size_t)kl_ring_slots_ * KK * sizeof(float));
-      else chain(&hclt_kld_chain_kernel<KK, false>, 0);
     });
+    kl_chain(kv, false, rc, pu, vec, vec, pd, nullptr, ring_down, h, h, h, rs);
     float* out = d_out + (size_t)r0 * Vu_ * C_;
     const dim3 lgrid(Vu_, rc);
     if (norm_params)
@@ -1249,7 +1437,7 @@ void HcltCircuit::gumbel_sample_backward_rows(const float* d_params, int64_t sr,
   if (sr == 0 || sp == 0) fail(PCM_ERR_ARG, "parameter matrix strides must not be zero");
   if (!d_out_grad || !d_grads) fail(PCM_ERR_ARG, "gradient pointer is null");
   if (!(temperature > 0.f)) fail(PCM_ERR_ARG, "temperature must be positive");
-  build_kld_tables();
+  const KlView kv = kl_view(rows);
   build_block_params();
   if (d_input_order_.n == 0) d_input_order_.upload(input_order_, stream);
   const float* p = rows_packed_in(d_params, sr, sp, rows, n, d_rows_pk1_, stream);
@@ -1258,16 +1446,15 @@ void HcltCircuit::gumbel_sample_backward_rows(const float* d_params, int64_t sr,
     d_rows_pg1_.ensure((size_t)rows * n);
     gout = d_rows_pg1_.p;
   }
-  const int W = kl_waves(K_), D = kl_ahead(K_);
   const size_t nk = (size_t)n_inner_ * K_, vk = (size_t)V_ * K_;
-  const size_t su = (size_t)(kl_up_steps_ + D) * W, sd = (size_t)(kl_down_steps_ + D) * W, sm = std::max(su, sd);
+  const size_t su = kv.su, sd = kv.sd, sm = std::max(su, sd);
   KlRowStrides rs;
   rs.pu = su * K_ * K_;
   rs.pd = sd * K_ * K_;
   rs.vec = sm * K_;
   rs.out = nk;
-  rs.ring_up = kl_ring_slots_ ? 0 : su * K_;
-  rs.ring_down = kl_ring_slots_ ? 0 : sd * K_;
+  rs.ring_up = kv.lds ? 0 : su * K_;
+  rs.ring_down = kv.lds ? 0 : sd * K_;
   rs.down_only = 0;
   const size_t per_row = rs.pu + rs.pd + 2 * rs.vec + 3 * nk + vk + rs.ring_up + rs.ring_down;
   const int chunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)rows, ((size_t)2 << 30) / per_row));
@@ -1280,8 +1467,8 @@ void HcltCircuit::gumbel_sample_backward_rows(const float* d_params, int64_t sr,
   float* klv = h + (size_t)chunk * nk;
   float* z = klv + (size_t)chunk * nk;
   float* leaf_grad = z + (size_t)chunk * nk;
-  float* ring_up = kl_ring_slots_ ? nullptr : leaf_grad + (size_t)chunk * vk;
-  float* ring_down = kl_ring_slots_ ? nullptr : ring_up + (size_t)chunk * rs.ring_up;
+  float* ring_up = kv.lds ? nullptr : leaf_grad + (size_t)chunk * vk;
+  float* ring_down = kv.lds ? nullptr : ring_up + (size_t)chunk * rs.ring_up;
   const float inv_t = 1.f / temperature;
   const int n_inputs = (int)input_order_.size();
   for (int r0 = 0; r0 < rows; r0 += chunk) {
@@ -1291,19 +1478,8 @@ void HcltCircuit::gumbel_sample_backward_rows(const float* d_params, int64_t sr,
     const float* og = d_out_grad + (size_t)r0 * Vu_ * C_;
     float* out = gout + (size_t)r0 * n;
     PCM_DISPATCH_K(K_, {
-      auto chain = [&](int down_only) {
-        KlRowStrides r2 = rs;
-        r2.down_only = down_only;
-        auto launch = [&](auto kernel, size_t lds) {
-          hipLaunchKernelGGL(kernel, dim3(1, rc), dim3(kl_waves(KK) * 64), lds, stream,
-                             reinterpret_cast<const KlItem*>(d_kl_up_.p), kl_up_steps_,
-                             reinterpret_cast<const KlItem*>(d_kl_down_.p), kl_down_steps_, d_kl_ext_.p, pu, base, ell, pd,
-                             kl_ring_slots_ - 1, ring_up, ring_down, klv, z, h, r2);
-        };
-        if (kl_ring_slots_) launch(&hclt_kld_chain_kernel<KK, true>, (size_t)kl_ring_slots_ * KK * sizeof(float));
-        else launch(&hclt_kld_chain_kernel<KK, false>, 0);
-      };
-      hipLaunchKernelGGL(hclt_rows_soft_base_kernel<KK>, dim3(n_inner_, rc), dim3(256), 0, stream, d_kl_pos_.p, n_inner_,
+      auto chain = [&](int down_only) { kl_chain(kv, !down_only, rc, pu, base, ell, pd, ring_up, ring_down, klv, z, h, rs); };
+      hipLaunchKernelGGL(hclt_rows_soft_base_kernel<KK>, dim3(n_inner_, rc), dim3(256), 0, stream, kv.pos, n_inner_,
                          d_blk2par_.p, q, (size_t)n, g, (size_t)ns, inv_t, pd, pu, rs);
       chain(1);   // the top-down probabilities
       const dim3 lgrid(ceil_div(n_inputs, 8), rc);
@@ -1314,10 +1490,10 @@ void HcltCircuit::gumbel_sample_backward_rows(const float* d_params, int64_t sr,
         hipLaunchKernelGGL(hclt_rows_soft_back_leaf_kernel<false>, lgrid, dim3(256), 0, stream, q, (size_t)n, (size_t)ns, C_, K_, Vu_,
                            n_inputs, d_input_order_.p, d_kl_tabs_.p + n_inner_, h, nk, og, vk, leaf_grad, out);
       hipLaunchKernelGGL(hclt_rows_soft_base2_kernel<KK>, dim3(n_inner_, rc), dim3(256), 0, stream, d_nodes_.p, d_child_leaf_.p,
-                         d_kl_pos_.p, n_inner_, leaf_grad, vk, Vu_, pd, ell, base, rs, 0);
+                         kv.pos, n_inner_, leaf_grad, vk, Vu_, pd, ell, base, rs, 0);
       chain(0);   // the gradients of the sum nodes, bottom-up
       hipLaunchKernelGGL(hclt_rows_soft_edge_grad_kernel<KK>, dim3((unsigned)ceil_div(ns, 256), ceil_div(rc, kEdgeGradRows)),
-                         dim3(256), 0, stream, ns, d_sum_param_src_.p, d_kl_tabs_.p, d_kl_pos_.p, n_inner_, pd, z, klv, h, nk, rs,
+                         dim3(256), 0, stream, ns, d_sum_param_src_.p, d_kl_tabs_.p, kv.pos, n_inner_, pd, z, klv, h, nk, rs,
                          inv_t, grad_wrt_logparams ? 1 : 0, rc, (size_t)n, out);
     });
   }

@@ -796,3 +796,45 @@ def test_row_queries_on_the_block_form_agree_with_the_layer_kernels(gpu, oracle,
         for wrt_log in (True, False):
             close(P.gumbel_sample_backward_rows(blk, p1, G, grad_wrt_logparams=wrt_log, **kw),
                   P.gumbel_sample_backward_rows(gen, p1, G, grad_wrt_logparams=wrt_log, **kw), "reverse pass")
+
+
+@pytest.mark.parametrize("shape,V,K,C", [("near", 700, 32, 8), ("near", 300, 64, 4), ("binary", 4095, 16, 4), ("wide", 400, 16, 8)])
+def test_a_row_does_not_depend_on_the_rows_beside_it(gpu, oracle, shape, V, K, C):
+    """The chains of the row queries walk a tree in eight parts, four or one by the number of rows: the same rows alone and
+    among others, in parts and in one (with vectors in LDS, and for the binary tree's wide levels in device memory)."""
+    torch, P = gpu
+    from helpers import make_hclt
+    rng = np.random.default_rng(V)
+    if shape == "binary":
+        parent = [-1] + [(v - 1) // 2 for v in range(1, V)]
+    else:   # wide: up to six children a node
+        parent, kids = [-1], np.zeros(V, int)
+        for v in range(1, V):
+            near = [u for u in range(max(0, v - 8), v) if kids[u] < (6 if shape == "wide" else 3)]
+            parent.append(int(near[rng.integers(len(near))]))
+            kids[parent[-1]] += 1
+    parent, _, _, _ = make_hclt(V, K, C, 1, parent=np.array(parent, np.int32))
+    bpc = P.hclt_from_clt(parent, C, K)
+    n, ns, R = bpc.num_parameters(), bpc.num_inner_params(), 70
+    gen = torch.Generator(device="cuda").manual_seed(V)
+
+    def draw():
+        x = torch.rand((R, n), device="cuda", generator=gen) + 0.05
+        for part, size in ((x[:, :ns], K), (x[:, ns:], C)):
+            part.view(R, -1, size).div_(part.reshape(R, -1, size).sum(-1, keepdim=True)) if part.is_contiguous() else \
+                part.copy_((part.reshape(R, -1, size) / part.reshape(R, -1, size).sum(-1, keepdim=True)).reshape(R, -1))
+        return x.log_()
+    p, q = draw(), draw()
+    noise = -torch.log(-torch.log(torch.rand((R, ns), device="cuda", generator=gen).clamp_(1e-6, 1 - 1e-6)))
+    G = torch.randn((R, V, C), device="cuda", generator=gen)
+
+    def queries(lo, hi):
+        a, b, g, z = p[lo:hi].contiguous(), q[lo:hi].contiguous(), G[lo:hi].contiguous(), noise[lo:hi].contiguous()
+        kw = dict(temperature=0.7, noise=z)
+        return [P.kld(bpc, a, b), *P.kld_backward(bpc, a, b), P.gumbel_sample_rows(bpc, a, **kw),
+                P.gumbel_sample_backward_rows(bpc, a, g, **kw)]
+    whole = queries(0, R)
+    for lo, hi in ((0, 40), (65, 70), (3, 4)):
+        for got, ref in zip(queries(lo, hi), whole):
+            ref = ref[lo:hi]
+            assert (got - ref).abs().max() <= 1e-5 * ref.abs().max()
