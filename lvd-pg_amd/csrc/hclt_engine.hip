@@ -1341,7 +1341,7 @@ void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
     auto launch_lean = [&](auto kernel) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
       const LeanPlan* lp = lean_plan(d.nslices);
-      PCM_LAUNCH_PHASE(0, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, d_lean_rows_.p + lp->fwd_at, lp->fwd_stride, d_ll,
+      PCM_LAUNCH_PHASE(0, kernel, dim3(lp->grid(d.nslices), lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, d_lean_rows_.p + lp->fwd_at, lp->fwd_stride, d_ll,
                        lds_slots_, away());
     };
     PCM_DISPATCH_LEAN_K(K_, {
@@ -1369,7 +1369,7 @@ void HcltCircuit::run_backward(const HcltDev& d) {
     auto launch_lean = [&](auto kernel) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
       const LeanPlan* lp = lean_plan(d.nslices);
-      PCM_LAUNCH_PHASE(1, kernel, dim3(d.nslices, lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, d_lean_rows_.p + lp->bwd_at, lp->bwd_stride,
+      PCM_LAUNCH_PHASE(1, kernel, dim3(lp->grid(d.nslices), lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, d_lean_rows_.p + lp->bwd_at, lp->bwd_stride,
                        lds_slots_, away());
     };
     PCM_DISPATCH_LEAN_K(K_, {

@@ -36,9 +36,9 @@ constexpr double kLeanStretch = 1.4;
 // average, while the largest part goes on shrinking by a quarter.  Below that the crossings cost what the parts gain: 153
 // nodes at 512 examples forward 42 us in one part, 50 in six; 632 nodes 97 in one, 95 in four (backward 125 and 107).  A tile
 // from another workgroup is expected kLeanAwaySteps steps after the step it is sent in.
+constexpr int kLeanMostParts = 16, kLeanPartNodes = 80, kLeanAwaySteps = 4;
 // The chains of the row queries: parts, and nodes that make a part worth its launches.
 constexpr int kKlMostParts = 8, kKlPartNodes = 24;
-constexpr int kLeanMostParts = 16, kLeanPartNodes = 80, kLeanAwaySteps = 4;
 constexpr int kPre = 3;          // static operand tiles a wave requests one step ahead
 
 struct HcltNode {     // one non-leaf tree node, device-resident
@@ -246,12 +246,13 @@ class HcltCircuit : public pcm_circuit {
   std::vector<std::vector<int32_t>> uchildren_;   // the caller's tree (children of every variable) where nodes were split
   bool forest_ = false;
   int T_ = 1;                      // trees (1 unless a forest)
-  int n_groups_ = 1;               // groups of trees the walk kernels take side by side (blockIdx.y)
   // schedules of the lean walks, in one group of trees or more, or one tree in several parts (the finer plans are for batches
   // whose slices do not fill the device), fewest groups first
   struct LeanPlan {
     int n_groups = 1, n_away = 0, n_fwd_steps = 0, fwd_stride = 0, n_bwd_steps = 0, bwd_stride = 0;
     size_t fwd_at = 0, bwd_at = 0;   // its field rows in d_lean_rows_
+    // workgroups side by side for so many slices: the parts of a tree stay on one of the eight dies (see hclt_walk_lean.hip.hpp)
+    unsigned grid(int nslices) const { return n_away ? (nslices + 7) / 8 * 8 : nslices; }
   };
   std::vector<std::unique_ptr<LeanPlan>> plans_;   // empty: the lean kernels do not take this tree
   DevBuf<int32_t> d_lean_rows_;

@@ -172,8 +172,10 @@ __device__ __forceinline__ void lean_post(unsigned* state, unsigned value) {
 // that its one reader puts back to zero, so that a launch leaves the flags as it found them (also one that a graph replays).
 // The data is written and read with device-scope accesses of its own, which pass the L2s of the eight dies; a release or
 // acquire fence would write back or drop a whole L2 each time.  Only the top waits going up, only the others going down,
-// and whoever is waited for comes first in the grid: it does not depend on a workgroup that is dispatched later.  The waits
-// are bounded like those for LDS tiles.  3072 variables, K = 32, 512 examples: forward 336 -> 194 us, backward 444 -> 235 in
+// and whoever is waited for comes first in the grid.  Workgroups go to the dies in turn and are dispatched in order within a
+// die, so the grid's first dimension is a multiple of their number: the parts of a slice are then on one die, and a
+// workgroup never holds a compute unit while the one it waits for still queues behind another stream's.  The waits are
+// bounded like those for LDS tiles.  3072 variables, K = 32, 512 examples: forward 336 -> 194 us, backward 444 -> 235 in
 // eight parts; 1024 examples 338 -> 201 and 480 -> 271 in four; 784 variables, 512 examples: 97 -> 97 and 125 -> 107.
 struct LeanAway {
   float* tiles;        // [tile][slice][16 * K]
@@ -268,6 +270,7 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int slice = blockIdx.x;
+  if (slice >= d.nslices) return;   // (the grid of a tree in parts is rounded up)
   unsigned* state = reinterpret_cast<unsigned*>(lds + (size_t)n_slots * (kSlice * K));
   for (int i = threadIdx.x; i < kLeanFlagWords; i += blockDim.x) state[i] = 0u;
   __syncthreads();
@@ -494,6 +497,7 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_backward_lean_kernel(
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int slice = blockIdx.x;
+  if (slice >= d.nslices) return;   // (the grid of a tree in parts is rounded up)
   unsigned* state = reinterpret_cast<unsigned*>(lds + (size_t)n_slots * (kSlice * K));
   for (int i = threadIdx.x; i < kLeanFlagWords; i += blockDim.x) state[i] = 0u;
   __syncthreads();
