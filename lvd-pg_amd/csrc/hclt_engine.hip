@@ -221,8 +221,9 @@ void HcltCircuit::build_structure() {
   if (block_) build_schedules();
 }
 
-LeanTree HcltCircuit::lean_tree() const {
-  LeanTree t;
+void HcltCircuit::build_lean_tree() {
+  const auto tree = std::make_shared<LeanTree>();
+  LeanTree& t = *tree;
   t.parent.assign(n_inner_, -1);
   t.inner.resize(n_inner_);
   t.tree = tree_of_inner_;
@@ -234,7 +235,7 @@ LeanTree HcltCircuit::lean_tree() const {
       if (!children_[c].empty()) t.inner[n].push_back(inner_of_var_[c]);
   }
   t.complete();
-  return t;
+  lean_tree_ = tree;
 }
 
 // Step schedules of the two tree walks.  Every step holds at most kWalkWaves nodes whose
@@ -325,7 +326,8 @@ void HcltCircuit::build_schedules() {
       }
     dst.upload(f);
   };
-  const LeanTree lt = lean_tree();
+  build_lean_tree();
+  const LeanTree& lt = *lean_tree_;
   // field rows of the lean walks (see hclt_walk_lean.hip.hpp) from their own schedule, with the same padding, or none if
   // some node has more operands than the lean kernels hold
   const size_t leaf_stride = (size_t)C_ * K_ * sizeof(float);

@@ -382,13 +382,19 @@ class HcltCircuit : public pcm_circuit {
   SparseCircuit* general();
   SparseCircuit* general_structure();   // the same object without bringing its parameters up to date
   // KL recursion on the block form
-  DevBuf<int32_t> d_kl_up_, d_kl_down_;   // chain steps (KlItem records) bottom-up / top-down
+  // the tables of the chains, one allocation and one copy for all of them (build_kld_tables)
+  struct KlTab {
+    const int32_t* p = nullptr;
+    size_t n = 0;
+  };
+  DevBuf<int32_t> d_kl_all_;
+  KlTab d_kl_up_, d_kl_down_;   // chain steps (KlItem records) bottom-up / top-down
   DevBuf<int32_t> d_blk2par_;             // entry of the [n_inner][K][K] blocks -> parameter, for the row queries (build_block_params)
   DevBuf<float> d_rows_scratch_, d_rows_pk1_, d_rows_pk2_, d_rows_pg1_, d_rows_pg2_;   // row queries: per-row arrays; re-laid-out matrices
-  DevBuf<int32_t> d_kl_tabs_;             // parent of every inner node | h-giving node of every variable | input-node positions
-  DevBuf<int32_t> d_kl_pos_;              // chain slot of every inner node: upward | downward
+  KlTab d_kl_tabs_;             // parent of every inner node | h-giving node of every variable | input-node positions
+  KlTab d_kl_pos_;              // chain slot of every inner node: upward | downward
   DevBuf<float> d_kl_leaf_, d_kl_vec_, d_kl_par_;
-  DevBuf<int32_t> d_kl_ext_;              // chain slots of the children past the second, of nodes with more than three
+  KlTab d_kl_ext_;              // chain slots of the children past the second, of nodes with more than three
   int kl_up_steps_ = 0, kl_down_steps_ = 0;
   int kl_ring_slots_ = 0;                 // slots of the chains' LDS ring; 0: levels too wide, the ring is the whole chain in device memory
   // the chains of the row queries (see kl_view): tables of one workgroup per row, or of a tree in parts
@@ -396,8 +402,7 @@ class HcltCircuit : public pcm_circuit {
     bool ok = false;
     int W = 0, slots = 0, most_away = 0;
     size_t su = 0, sd = 0;
-    DevBuf<int32_t> tab;
-    size_t up = 0, down = 0, pos = 0, ext = 0, away = 0, parts = 0;   // where in `tab`
+    size_t up = 0, down = 0, pos = 0, ext = 0, away = 0, parts = 0;   // where in d_kl_all_
   };
   struct KlView {
     int G, W, mask;
@@ -408,10 +413,11 @@ class HcltCircuit : public pcm_circuit {
   };
   KlPlan kl_plans_[2];
   KlView kl_view(int rows);
-  void build_kl_plan(const LeanTree& t, KlPlan& p, int G);
+  void build_kl_plan(const LeanTree& t, KlPlan& p, int G, std::vector<int32_t>& tab);
   void kl_chain(const KlView& v, bool up, int rows, const float* pu, const float* base, const float* ell, const float* pd,
                 float* ring_up, float* ring_down, float* klv, float* z, float* h, const KlRowStrides& strides);
-  LeanTree lean_tree() const;
+  std::shared_ptr<const LeanTree> lean_tree_;   // the tree of inner nodes as the schedulers see it
+  void build_lean_tree();
   HcltCircuit* same_tree(pcm_circuit* q);
   void build_kld_tables();
   void build_block_params();

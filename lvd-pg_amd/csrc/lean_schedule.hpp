@@ -43,13 +43,15 @@ struct LeanTree {   // inner nodes, children before their parents
         chain[v] = std::max(chain[v], chain[c] + 1);
         below[v] += below[c] + 1;
       }
-      std::stable_sort(inner[v].begin(), inner[v].end(), [&](int a, int b) { return chain[a] > chain[b]; });
+      if (inner[v].size() > 1)
+        std::stable_sort(inner[v].begin(), inner[v].end(), [&](int a, int b) { return chain[a] > chain[b]; });
     }
+    std::vector<int32_t> c;
     // post-order places: a node's subtree ends at its own place; the larger child's subtree comes first
     for (int v = n - 1; v >= 0; --v) {
       if (parent[v] < 0) order[v] = v;   // (trees are runs of node numbers that end with their root)
-      std::vector<int32_t> c = inner[v];
-      std::stable_sort(c.begin(), c.end(), [&](int a, int b) { return below[a] < below[b]; });
+      c.assign(inner[v].begin(), inner[v].end());
+      if (c.size() > 1) std::stable_sort(c.begin(), c.end(), [&](int a, int b) { return below[a] < below[b]; });
       int at = order[v] - 1;
       for (int k : c) {
         order[k] = at;
