@@ -399,10 +399,11 @@ class HcltCircuit : public pcm_circuit {
   int kl_ring_slots_ = 0;                 // slots of the chains' LDS ring; 0: levels too wide, the ring is the whole chain in device memory
   // the chains of the row queries (see kl_view): tables of one workgroup per row, or of a tree in parts
   struct KlPlan {
-    bool ok = false;
+    bool tried = false, ok = false;
+    DevBuf<int32_t> tab;
     int W = 0, slots = 0, most_away = 0;
     size_t su = 0, sd = 0;
-    size_t up = 0, down = 0, pos = 0, ext = 0, away = 0, parts = 0;   // where in d_kl_all_
+    size_t up = 0, down = 0, pos = 0, ext = 0, away = 0, parts = 0;   // where in `tab`
   };
   struct KlView {
     int G, W, mask;
@@ -413,7 +414,7 @@ class HcltCircuit : public pcm_circuit {
   };
   KlPlan kl_plans_[2];
   KlView kl_view(int rows);
-  void build_kl_plan(const LeanTree& t, KlPlan& p, int G, std::vector<int32_t>& tab);
+  void build_kl_plan(const LeanTree& t, KlPlan& p, int G);
   void kl_chain(const KlView& v, bool up, int rows, const float* pu, const float* base, const float* ell, const float* pd,
                 float* ring_up, float* ring_down, float* klv, float* z, float* h, const KlRowStrides& strides);
   std::shared_ptr<const LeanTree> lean_tree_;   // the tree of inner nodes as the schedulers see it

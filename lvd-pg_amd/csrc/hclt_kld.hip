@@ -528,10 +528,9 @@ void HcltCircuit::build_kld_tables() {
   int ring = 1;
   while (ring < reach + W) ring <<= 1;
   kl_ring_slots_ = (size_t)ring * K_ * sizeof(float) <= (size_t)64 * 1024 ? ring : 0;
-  // Everything in one buffer: an allocation, a copy and a wait instead of seven (first KL and gradient of 16 rows of a
-  // 3072-variable circuit 6.6 -> 6.0 ms, which is what it took without the plans)
+  // Everything in one buffer: an allocation, a copy and a wait instead of five
   std::vector<int32_t> tab;
-  tab.reserve(4 * (up.size() + down.size()) + pos.size() + ext.size() + (size_t)(K_ + 2) * V_ + (size_t)96 * n_inner_);
+  tab.reserve(4 * (up.size() + down.size()) + pos.size() + ext.size() + (size_t)(K_ + 3) * V_);
   // per inner node: its parent | per variable: the inner node whose h reaches its leaf |
   // per input node (v, j): its position among the input nodes of the parameter vector
   std::vector<int32_t> t((size_t)n_inner_ + V_ + (size_t)V_ * K_, 0);
@@ -545,11 +544,6 @@ void HcltCircuit::build_kld_tables() {
   const size_t at_up = kl_table(tab, up.data(), up.size() * sizeof(KlItem)), at_down = kl_table(tab, down.data(), down.size() * sizeof(KlItem));
   const size_t at_pos = kl_table(tab, pos.data(), pos.size() * 4), at_ext = kl_table(tab, ext.data(), ext.size() * 4);
   const size_t at_t = kl_table(tab, t.data(), t.size() * 4);
-  // (both plans now: a call for other numbers of rows builds nothing)
-  if (block_ && n_inner_ >= kKlMostParts / 2 * kKlPartNodes) {
-    for (int i = 0; i < 2; ++i)
-      if (n_inner_ >= (kKlMostParts >> i) * kKlPartNodes) build_kl_plan(*lean_tree_, kl_plans_[i], kKlMostParts >> i, tab);
-  }
   d_kl_all_.upload(tab, stream);
   d_kl_down_ = {d_kl_all_.p + at_down, down.size() * 4};
   d_kl_pos_ = {d_kl_all_.p + at_pos, pos.size()};
@@ -578,8 +572,14 @@ HcltCircuit::KlView HcltCircuit::kl_view(int rows) {
   v.away = nullptr;
   for (int i = 0; i < 2; ++i) {
     const int G = kKlMostParts >> i;
-    const KlPlan& p = kl_plans_[i];
-    if (!p.ok || (int64_t)rows * G > n_cus_) continue;
+    KlPlan& p = kl_plans_[i];
+    if (!block_ || n_inner_ < G * kKlPartNodes || (int64_t)rows * G > n_cus_) continue;
+    if (!p.tried) {   // a plan is built by the first call that takes it (not under capture: that call takes the tables above)
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) continue;
+      build_kl_plan(*lean_tree_, p, G);
+    }
+    if (!p.ok) continue;
     v.G = G;
     v.W = p.W;
     v.lds = true;
@@ -587,21 +587,22 @@ HcltCircuit::KlView HcltCircuit::kl_view(int rows) {
     v.lds_bytes = (size_t)(p.slots + p.most_away) * K_ * sizeof(float);
     v.su = p.su;
     v.sd = p.sd;
-    v.up = d_kl_all_.p + p.up;
-    v.down = d_kl_all_.p + p.down;
-    v.ext = d_kl_all_.p + p.ext;
-    v.pos = d_kl_all_.p + p.pos;
-    v.away = d_kl_all_.p + p.away;
-    v.parts = reinterpret_cast<const KlPart*>(d_kl_all_.p + p.parts);
+    v.up = p.tab.p + p.up;
+    v.down = p.tab.p + p.down;
+    v.ext = p.tab.p + p.ext;
+    v.pos = p.tab.p + p.pos;
+    v.away = p.tab.p + p.away;
+    v.parts = reinterpret_cast<const KlPart*>(p.tab.p + p.parts);
     break;
   }
   return v;
 }
 
-void HcltCircuit::build_kl_plan(const LeanTree& t, KlPlan& p, int G, std::vector<int32_t>& tab) {
+void HcltCircuit::build_kl_plan(const LeanTree& t, KlPlan& p, int G) {
   const int D = kl_ahead(K_), W = p.W = std::max(4, kl_waves(K_) * 2 / G);
   int largest = 0;
   const std::vector<int32_t> part = lean_parts(t, G, &largest);
+  p.tried = true;
   if (largest > n_inner_ / 2) return;   // (the top alone is most of the tree)
   std::vector<int32_t> pos((size_t)2 * n_inner_, 0), ext, away;
   std::vector<KlItem> all[2];
@@ -696,8 +697,10 @@ void HcltCircuit::build_kl_plan(const LeanTree& t, KlPlan& p, int G, std::vector
   p.slots = 1;
   while (p.slots < reach + W) p.slots <<= 1;
   if ((size_t)(p.slots + p.most_away) * K_ * sizeof(float) > (size_t)max_lds_) return;
+  p.tried = false;   // (until its table is there)
   p.su = all[0].size();
   p.sd = all[1].size();
+  std::vector<int32_t> tab;   // one upload
   auto put = [&](const void* q, size_t bytes) { return kl_table(tab, q, bytes); };
   p.up = put(all[0].data(), all[0].size() * sizeof(KlItem));
   p.down = put(all[1].data(), all[1].size() * sizeof(KlItem));
@@ -705,7 +708,8 @@ void HcltCircuit::build_kl_plan(const LeanTree& t, KlPlan& p, int G, std::vector
   p.ext = put(ext.data(), ext.size() * 4);
   p.away = put(away.data(), away.size() * 4);
   p.parts = put(parts.data(), parts.size() * sizeof(KlPart));
-  p.ok = true;
+  p.tab.upload(tab, stream);
+  p.ok = p.tried = true;
 }
 
 void HcltCircuit::kl_chain(const KlView& v, bool up, int rows, const float* pu, const float* base, const float* ell, const float* pd,
