@@ -995,11 +995,12 @@ void HcltCircuit::rebuild_heads() {
 }
 
 // head values from the root tile the forward walk has left (identity block: the root's Z)
-void HcltCircuit::heads_forward(const HcltDev& d, const float* d_mask, float* d_ll_heads, float* d_ll_mix, bool flows_follow,
+// (`row`: examples of a row of the mask and of the results, of which this batch is a part)
+void HcltCircuit::heads_forward(const HcltDev& d, int row, const float* d_mask, float* d_ll_heads, float* d_ll_mix, bool flows_follow,
                                 float rate) {
   PCM_DISPATCH_LEAN_K(K_, hipLaunchKernelGGL(hclt_heads_forward_kernel<KK>, dim3(d.nslices, T_), dim3(kHeadWaves * 64), 0,
                                              stream, d.O, d.M, lean_fits(d.B) ? ~1 : ~0, d.Bp, d_root_node_.p, (int64_t)(d.tile_stride / 4), d_head_wf_.p,
-                                             H_, Hp_, d.B, d_mask, d_ll_heads, d_ll_mix,
+                                             H_, Hp_, d.B, row, d_mask, d_ll_heads, d_ll_mix,
                                              flows_follow ? head_aggr() : (float*)nullptr, rate, d_flow_shift_.p));
   check_launch("heads_forward");
 }
@@ -1284,6 +1285,20 @@ int HcltCircuit::walk_chunk(int batch) const {
   return (H_ == 0 && block_ && !wide_walk_ && batch > chunk) ? chunk : 0;
 }
 
+// A forest runs on the lean walks alone, which address its tiles with 31-bit offsets: a batch whose tiles are more goes
+// through in as few, equal chunks as they allow (16 trees of 192 variables: from 7000 examples on).  Returns the chunk size, or
+// 0 for a batch that goes through as it is.
+int HcltCircuit::forest_chunk(int batch) const {
+  if (!forest_ || batch < 1 || lean_fits(batch)) return 0;
+  const int ns = ceil_div(batch, kSlice);
+  const int most = (int)((((size_t)1 << 31) - 1) / ((size_t)(n_inner_ + 1) * kSlice * K_ * 4));
+  for (int parts = ceil_div(ns, std::max(most, 1)); parts <= ns; ++parts) {
+    const int chunk = ceil_div(ns, parts) * kSlice;
+    if (lean_fits(chunk)) return chunk;
+  }
+  fail(PCM_ERR_UNSUPPORTED, "the tiles of a forest of %d tree nodes are too large for any batch", n_inner_);
+}
+
 BatchRef HcltCircuit::chunk_of(const BatchRef& b, int off, int chunk) {
   BatchRef part = b;
   part.batch = std::min(chunk, b.batch - off);
@@ -1331,6 +1346,10 @@ LeanAway HcltCircuit::away() const {
   return {d_away_tiles_.p, d_away_flags_.p, d_away_sums_.p, d_away_flags_.p + away_tiles_};
 }
 
+void HcltCircuit::need_general_schedules() const {
+  if (!d_fwd_fields_.p || !d_bwd_fields_.p) fail(PCM_ERR_STATE, "the general walk kernels have no schedules of this circuit");
+}
+
 void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
   const size_t lds = (size_t)lds_slots_ * kSlice * K_ * sizeof(float);
   auto launch = [&](auto kernel) {
@@ -1352,6 +1371,7 @@ void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
       else launch_lean(&hclt_forward_lean_kernel<KK, kKeepNone>);
     });
   } else {
+    need_general_schedules();
     PCM_DISPATCH_K(K_, {
       if (fwd_spill_) launch(&hclt_forward_kernel<KK, true>); else launch(&hclt_forward_kernel<KK, false>);
     });
@@ -1378,6 +1398,7 @@ void HcltCircuit::run_backward(const HcltDev& d) {
       if (H_ > 0) launch_lean(&hclt_backward_lean_kernel<KK, true>); else launch_lean(&hclt_backward_lean_kernel<KK, false>);
     });
   } else {
+    need_general_schedules();
     PCM_DISPATCH_K(K_, {
       if (H_ > 0) {
         if (bwd_spill_) launch(&hclt_backward_kernel<KK, true, true>); else launch(&hclt_backward_kernel<KK, false, true>);
@@ -1443,16 +1464,22 @@ void HcltCircuit::loglikelihoods(const BatchRef& b, float* d_ll) {
     for (int off = 0; off < b.batch; off += chunk) loglikelihoods(chunk_of(b, off, chunk), d_ll + off);
     return;
   }
-  // nobody reads a scoring pass's tiles: the lean walk keeps none (heads: the roots' only)
-  const bool lean = lean_fits(b.batch, H_ > 0 ? kKeepRoots : kKeepNone) && !wide_walk_;
-  stage_batch(b, !lean || H_ > 0);
-  if (wide_walk_) return wide_forward(dev(b.batch), d_ll);
   if (H_ > 0) {   // per-head values [H][batch]
-    const HcltDev d = dev(b.batch);
-    run_forward(d, nullptr, kKeepRoots);   // (the head kernel reads the root tiles and the row maxima)
-    heads_forward(d, nullptr, d_ll, nullptr);
+    const int chunk = forest_chunk(b.batch);
+    for (int off = 0; off == 0 || off < b.batch; off += chunk) {
+      const BatchRef part = chunk ? chunk_of(b, off, chunk) : b;
+      stage_batch(part);
+      const HcltDev d = dev(part.batch);
+      run_forward(d, nullptr, kKeepRoots);   // (the head kernel reads the root tiles and the row maxima)
+      heads_forward(d, b.batch, nullptr, d_ll + off, nullptr);
+      if (!chunk) break;
+    }
     return;
   }
+  // nobody reads a scoring pass's tiles: the lean walk keeps none
+  const bool lean = lean_fits(b.batch, kKeepNone) && !wide_walk_;
+  stage_batch(b, !lean);
+  if (wide_walk_) return wide_forward(dev(b.batch), d_ll);
   run_forward(dev(b.batch), d_ll, kKeepNone);
 }
 
@@ -1623,29 +1650,19 @@ void HcltCircuit::flows(const BatchRef& b, float rate, const float* d_head_mask,
       flows(chunk_of(b, off, chunk), off == 0 ? rate : 1.f, weights ? weights + off : nullptr, d_ll + off);
     return;
   }
+  if (H_ > 0) {
+    const int chunk = forest_chunk(b.batch);
+    if (!chunk) head_flows(b, b.batch, rate, d_head_mask, d_ll);
+    for (int off = 0; chunk && off < b.batch; off += chunk)
+      head_flows(chunk_of(b, off, chunk), b.batch, off == 0 ? rate : 1.f, d_head_mask + off, d_ll + off);
+    return;
+  }
   stage_batch(b);
   HcltDev d = dev(b.batch);
   d.w = weights;
   if (weights) {   // bound on the flow of one example, as a power of two, for the statistics' fixed-point counters
     hipLaunchKernelGGL(hclt_weight_shift_kernel, dim3(1), dim3(256), 0, stream, weights, b.batch, d_flow_shift_.p);
     check_launch("weight_shift");
-  }
-  if (H_ > 0) {
-    run_forward(d, nullptr);
-    heads_forward(d, d_head_mask, nullptr, d_ll, true, rate);
-    const size_t lds = ((size_t)16 * Hp_ + 16 * K_ + (size_t)kHeadWaves * 16 * K_ + (size_t)kHeadWaves * 16) * sizeof(float);
-    d_part_.ensure((size_t)T_ * d.nslices * H_ * K_);
-    PCM_DISPATCH_LEAN_K(K_, hipLaunchKernelGGL(hclt_heads_backward_kernel<KK>, dim3(d.nslices, T_), dim3(kHeadWaves * 64), lds,
-                                               stream, d.O, d.R, d_root_node_.p, (int64_t)(d.tile_stride / 4), d_head_wf_.p,
-                                               d_head_wb_.p, H_, Hp_, d.B, d_head_mask, d_part_.p, d_flow_shift_.p));
-    hipLaunchKernelGGL(sum_parts_kernel<true>, dim3(ceil_div((int64_t)H_ * K_, 64), T_), dim3(256), 0, stream, d_part_.p,
-                       d.nslices, (int64_t)H_ * K_, head_logp(), head_aggr());
-    check_launch("heads_backward");
-    run_backward(d);
-    run_stats(d, rate);
-    have_flows_ = true;
-    if (timing) ++n_timed_;
-    return;
   }
   if (wide_walk_) {
     wide_forward(d, d_ll);
@@ -1655,6 +1672,26 @@ void HcltCircuit::flows(const BatchRef& b, float rate, const float* d_head_mask,
     return;
   }
   run_forward(d, d_ll);
+  run_backward(d);
+  run_stats(d, rate);
+  have_flows_ = true;
+  if (timing) ++n_timed_;
+}
+
+// Flows of a batch that is `row` examples of the caller's, or a chunk of it (mask and results: rows of the caller's batch).
+void HcltCircuit::head_flows(const BatchRef& b, int row, float rate, const float* d_head_mask, float* d_ll) {
+  stage_batch(b);
+  const HcltDev d = dev(b.batch);
+  run_forward(d, nullptr);
+  heads_forward(d, row, d_head_mask, nullptr, d_ll, true, rate);
+  const size_t lds = ((size_t)16 * Hp_ + 16 * K_ + (size_t)kHeadWaves * 16 * K_ + (size_t)kHeadWaves * 16) * sizeof(float);
+  d_part_.ensure((size_t)T_ * d.nslices * H_ * K_);
+  PCM_DISPATCH_LEAN_K(K_, hipLaunchKernelGGL(hclt_heads_backward_kernel<KK>, dim3(d.nslices, T_), dim3(kHeadWaves * 64), lds,
+                                             stream, d.O, d.R, d_root_node_.p, (int64_t)(d.tile_stride / 4), d_head_wf_.p,
+                                             d_head_wb_.p, H_, Hp_, d.B, row, d_head_mask, d_part_.p, d_flow_shift_.p));
+  hipLaunchKernelGGL(sum_parts_kernel<true>, dim3(ceil_div((int64_t)H_ * K_, 64), T_), dim3(256), 0, stream, d_part_.p,
+                     d.nslices, (int64_t)H_ * K_, head_logp(), head_aggr());
+  check_launch("heads_backward");
   run_backward(d);
   run_stats(d, rate);
   have_flows_ = true;

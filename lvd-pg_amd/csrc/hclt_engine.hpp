@@ -301,7 +301,7 @@ class HcltCircuit : public pcm_circuit {
   float* head_logp() { return d_logtheta_.p + (size_t)n_inner_ * K_ * K_; }   // [trees][H][K], behind the blocks
   float* head_aggr() { return d_edge_aggr_.p + (size_t)n_inner_ * K_ * K_; }
   void rebuild_heads();
-  void heads_forward(const HcltDev& d, const float* d_mask, float* d_ll_heads, float* d_ll_mix, bool flows_follow = false,
+  void heads_forward(const HcltDev& d, int row, const float* d_mask, float* d_ll_heads, float* d_ll_mix, bool flows_follow = false,
                      float rate = 0.f);
   bool block_ = true;   // the hidden size has walk kernels (block tiles in registers)
   bool wide_ = false;   // the hidden size has the wide block kernels (likelihoods, flows, EM); neither: layered engine
@@ -328,6 +328,9 @@ class HcltCircuit : public pcm_circuit {
   void sync_checked();   // waits for the stream, then check_walks()
   DevBuf<int32_t> d_walk_void_;   // device copy of the word: non-zero after a void pass, read by the update kernels
   int walk_chunk(int batch) const;
+  int forest_chunk(int batch) const;
+  void head_flows(const BatchRef& b, int row, float rate, const float* d_head_mask, float* d_ll);
+  void need_general_schedules() const;
   static BatchRef chunk_of(const BatchRef& b, int off, int chunk);
   // Floats per node in the tile arrays.  The walk engines keep an odd number of tiles per node: with a power
   // of two (a batch of 4096), the tiles that one step reads from different nodes at equal slice offsets fell on

@@ -21,7 +21,8 @@
 //
 // A forest (several trees over one batch, H heads each) runs the same kernels with the tree in
 // blockIdx.y: every per-tree array is [tree][...], the root tiles are found through `root_node`
-// (each tree's root node, whose tiles start `tile_floats` floats per node into the value / ratio arrays).
+// (each tree's root node, whose tiles start `tile_floats` floats per node into the value / ratio arrays).  A batch that
+// goes through in chunks has its mask and results in rows of `row` examples, of which a launch takes B.
 #pragma once
 
 #include "hclt_kernels.hip.hpp"
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(kHeadWaves * 64) void hclt_heads_forward_kernel(con
                                                                              const int32_t* __restrict__ root_node,
                                                                              int64_t tile_floats,
                                                                              const float* __restrict__ hwf, int H, int Hp,
-                                                                             int B, const float* __restrict__ mask,
+                                                                             int B, int row, const float* __restrict__ mask,
                                                                              float* __restrict__ ll_heads,
                                                                              float* __restrict__ ll_mix,
                                                                              float* __restrict__ head_aggr, float rate,
@@ -94,9 +95,9 @@ __global__ __launch_bounds__(kHeadWaves * 64) void hclt_heads_forward_kernel(con
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, slice = blockIdx.x, tree = blockIdx.y;
   const float* __restrict__ O_root = O + (size_t)root_node[tree] * tile_floats;
   hwf += (size_t)tree * Hp * K;
-  if (mask) mask += (size_t)tree * H * B;
-  if (ll_heads) ll_heads += (size_t)tree * H * B;
-  if (ll_mix) ll_mix += (size_t)tree * B;
+  if (mask) mask += (size_t)tree * H * row;
+  if (ll_heads) ll_heads += (size_t)tree * H * row;
+  if (ll_mix) ll_mix += (size_t)tree * row;
   if (head_aggr) head_aggr += (size_t)tree * H * K;
   if (head_aggr) {   // ahead of a flow pass: previous head statistics times the flow memory rate, flow bound cleared
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < H * K; i += gridDim.x * blockDim.x)
@@ -127,9 +128,9 @@ __global__ __launch_bounds__(kHeadWaves * 64) void hclt_heads_forward_kernel(con
       const int h = ht * 16 + 4 * g + i;
       if (h >= H || col >= B) continue;
       const float val = (float)(base + (double)(m + __logf(s[i])));
-      if (ll_heads) ll_heads[(size_t)h * B + col] = val;
+      if (ll_heads) ll_heads[(size_t)h * row + col] = val;
       if (mask) {
-        const float mk = mask[(size_t)h * B + col];
+        const float mk = mask[(size_t)h * row + col];
         tot += mk;
         const float t = val + __logf(mk);
         if (t > mx) { sm = sm * __expf(mx - t) + 1.f; mx = t; }
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(kHeadWaves * 64) void hclt_heads_forward_kernel(con
 template <int K>
 __global__ __launch_bounds__(kHeadWaves * 64) void hclt_heads_backward_kernel(
     const float* __restrict__ O, float* __restrict__ R, const int32_t* __restrict__ root_node, int64_t tile_floats,
-    const float* __restrict__ hwf, const float* __restrict__ hwb, int H, int Hp, int B, const float* __restrict__ mask,
+    const float* __restrict__ hwf, const float* __restrict__ hwb, int H, int Hp, int B, int row, const float* __restrict__ mask,
     float* __restrict__ head_part, int* __restrict__ flow_shift) {
   extern __shared__ float lds[];   // R [16][Hp] | E [16][K] | partial T tiles [waves][16*K] | mask totals [waves][16]
   float* Rl = lds;
@@ -166,7 +167,7 @@ __global__ __launch_bounds__(kHeadWaves * 64) void hclt_heads_backward_kernel(
   float* __restrict__ R_root = R + (size_t)root_node[tree] * tile_floats;
   hwf += (size_t)tree * Hp * K;
   hwb += (size_t)tree * Hp * K;
-  mask += (size_t)tree * H * B;
+  mask += (size_t)tree * H * row;
   const int b = lane & 15, g = lane >> 4, col = slice * kSlice + b;
   Tile<K> e;
   heads_load_e<K>(O_root, slice, lane, e);
@@ -184,7 +185,7 @@ __global__ __launch_bounds__(kHeadWaves * 64) void hclt_heads_backward_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int h = ht * 16 + 4 * g + i;
-      const float f = (h < H && col < B) ? mask[(size_t)h * B + col] : 0.f;
+      const float f = (h < H && col < B) ? mask[(size_t)h * row + col] : 0.f;
       ftot += fmaxf(f, 0.f);
       r[i] = (f > 0.f && s[i] > 0.f) ? f / s[i] : 0.f;
       Rl[b * Hp + h] = r[i];

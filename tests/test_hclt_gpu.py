@@ -821,6 +821,60 @@ def test_forest_handle_with_example_ids_and_flow_memory(gpu, oracle):
             np.testing.assert_array_equal(heads_f[t], c.get_heads(), err_msg=f"batch {it} tree {t}")
 
 
+@pytest.mark.parametrize("T,n", [(2, 300), (16, 100)])
+def test_a_forest_batch_beyond_two_gigabytes_of_tiles(gpu, oracle, T, n):
+    """The lean walks, a forest's only ones, address less than 2 GiB of tiles: a larger batch goes through in chunks, its
+    masks and results in rows of the whole batch.  The likelihoods are those of the same examples in batches that fit, to
+    the bit; the accumulators those of the batches one after the other, with example ids and flow memory."""
+    torch, P = gpu
+    from pcmi355._lib import lib, check
+    K, C, H, Vt = 32, 4, 3, [n] * T
+    rng = np.random.default_rng(T)
+    V, parent, gvars, trees = _forest_case(P, oracle, rng, T, Vt, K, C, H)
+    a, b = (P.hclt_forest_from_clts(parent, C, K, H) for _ in range(2))
+    theta, leaf = np.zeros((V, K, K), np.float32), np.zeros((V, K, C), np.float32)
+    for gv, (_, theta_t, leaf_t, _) in zip(gvars, trees):
+        theta[gv], leaf[gv] = theta_t, leaf_t
+    for f in (a, b):
+        f.set_params(theta, leaf)
+        f.set_heads(np.stack([t[3] for t in trees]))
+    fits = ((1 << 31) - 1) // ((a.size("inner_tree_nodes") + 1) * K * 4)   # examples (auxiliary nodes aside)
+    B = 2 * fits + 77                                                       # three chunks, the last one ragged
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    d = torch.randint(0, C, (B + 100, V), device="cuda", generator=gen, dtype=torch.uint8)
+    ids = torch.randperm(B + 100, device="cuda", generator=gen)[:B].int()
+    mask = torch.rand((T, H, B), device="cuda", generator=gen)
+    mask[0, 0, ::5] = 0
+    mix, ll = torch.empty((T, B), device="cuda"), torch.empty((T, H, B), device="cuda")
+
+    def call(f, lo, hi, rate, out, heads=False):
+        m, i = mask[:, :, lo:hi].contiguous(), ids[lo:hi].contiguous()
+        args = (f.handle, d.data_ptr(), d.stride(0), d.stride(1), i.data_ptr(), hi - lo)
+        check(lib.pcm_loglikelihoods(*args, out.data_ptr()) if heads else
+              lib.pcm_flows(*args, rate, m.data_ptr(), out.data_ptr()))
+        torch.cuda.synchronize()
+    call(a, 0, B, 0.0, ll, heads=True)
+    call(a, 0, B, 0.0, mix)
+    call(a, 0, B, 0.5, mix)
+    step = fits // 3 // 16 * 16
+    for turn in range(2):
+        for lo in range(0, B, step):
+            hi = min(lo + step, B)
+            one, many = torch.empty((T, hi - lo), device="cuda"), torch.empty((T, H, hi - lo), device="cuda")
+            if turn == 0:
+                call(b, lo, hi, 0.0, many, heads=True)
+                assert torch.equal(many, ll[:, :, lo:hi])
+            call(b, lo, hi, 1.0 if lo else 0.5 * turn, one)
+            assert torch.equal(one, mix[:, lo:hi])
+    for f in (a, b):
+        check(lib.pcm_em_update(f.handle, 0.1, 0.5))
+    for x, y in zip((*a.get_flows(), *a.get_params(), a.get_heads()), (*b.get_flows(), *b.get_params(), b.get_heads())):
+        # sums over the batch in 32 bits and, for the leaves, in fixed point, cut into chunks in another way
+        some = np.isfinite(y)
+        np.testing.assert_array_equal(np.isfinite(x), some)
+        assert np.abs(x[some] - y[some]).max() <= 1e-4 * np.abs(y[some]).max()
+
+
 def test_em_driver_of_a_forest_follows_the_driver_of_every_tree(gpu, oracle):
     """mini_batch_em_for_forest against mini_batch_em_for_multihead_pc on a handle per tree: three epochs in the
     given order of examples, rising inertia, flow memory."""
