@@ -624,8 +624,6 @@ void HcltCircuit::build_schedules() {
   int most_nodes = n_inner_;
   if (K_ <= 32) {
     std::unique_ptr<LeanPlan> plan = make_plan(whole_trees(forest_ ? std::max(1, std::min(4, T_ / 8)) : 1), {});
-    if (plan && !forest_ && (plan->n_fwd_steps > n_fwd_steps_ * kLeanStretch || plan->n_bwd_steps > n_bwd_steps_ * kLeanStretch))
-      plan.reset();   // (see kLeanStretch)
     if (plan) plans_.push_back(std::move(plan));
     for (int G = plans_.empty() ? 0 : 2 * plans_[0]->n_groups; G; G *= 2) {
       if (forest_ ? G > 8 * plans_[0]->n_groups || G > T_ / 2 : G > kLeanMostParts || n_inner_ < G * kLeanPartNodes) break;

@@ -27,11 +27,6 @@ constexpr int kXSelShift = 28;               // leaf operand: which byte of the 
 constexpr int kSlotShift = 22;               // LDS operand: (slot + 1) << kSlotShift | inner id
 constexpr int kItemRoot = 1, kItemHasInnerChild = 2, kItemOverflow = 4, kItemSpillOut = 8;
 enum { kKeepNone = 0, kKeepRoots, kKeepAll };   // what the lean forward walk leaves in memory (hclt_walk_lean.hip.hpp)
-// A single tree (K <= 32) runs on the lean walks if their schedules, which keep every tile in registers or LDS, take at most
-// kLeanStretch times the steps of the general walks' schedules, which may send tiles through memory: the general kernels
-// take 1.45 times as long per EM step of as many steps (2.40 against 1.65 ms on a 3072-variable Chow-Liu tree at 4096
-// examples).
-constexpr double kLeanStretch = 1.4;
 // One tree over several workgroups (hclt_walk_lean.hip.hpp): up to kLeanMostParts parts of at least kLeanPartNodes nodes on
 // average, while the largest part goes on shrinking by a quarter.  Below that the crossings cost what the parts gain: 153
 // nodes at 512 examples forward 42 us in one part, 50 in six; 632 nodes 97 in one, 95 in four (backward 125 and 107).  A tile

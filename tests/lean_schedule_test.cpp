@@ -127,6 +127,55 @@ int main() {
       }
     }
   }
+  // rows of equally long chains off a column, crowns with chains below: what the steps cost, over the fewest there could be
+  double worst = 0;
+  int shapes = 0, shape_faults = 0;
+  auto look = [&](const std::vector<int>& up_to) {   // numbered from the root
+    const int n = (int)up_to.size();
+    std::vector<std::vector<int>> ch(n);
+    for (int v = 1; v < n; ++v) ch[up_to[v]].push_back(v);
+    std::vector<int> id(n), parent(n, -1);
+    std::vector<std::pair<int, size_t>> st{{0, 0}};
+    for (int k = 0; !st.empty();) {
+      auto& top = st.back();
+      if (top.second < ch[top.first].size()) { const int c = ch[top.first][top.second++]; st.push_back({c, 0}); }
+      else { id[top.first] = k++; st.pop_back(); }
+    }
+    for (int v = 1; v < n; ++v) parent[id[v]] = id[up_to[v]];
+    const LeanTree t = make(parent);
+    int deep = 0;
+    for (int v = 0; v < n; ++v) deep = std::max(deep, t.depth[v] + 1);
+    const LeanScope in(t, 0, n);
+    const LeanSchedule a = lean_schedule_up(t, in, 79), b = lean_schedule_down(t, in, 79);
+    if (!a.ok || !b.ok || fault(t, a, in, 79, true) || fault(t, b, in, 79, false)) ++shape_faults;
+    worst = std::max(worst, lean_steps_cost(a.steps + b.steps, 2 * n) / lean_steps_cost(2 * std::max(deep, (n + 15) / 16), 2 * n));
+    ++shapes;
+  };
+  auto chain_at = [](std::vector<int>& up, int p, int length) {
+    for (int i = 0; i < length; ++i) { up.push_back(p); p = (int)up.size() - 1; }
+    return p;
+  };
+  for (int rows : {2, 15, 16, 17, 18, 20, 24, 31, 32, 33, 40, 47, 48, 49, 64, 100})
+    for (int length : {1, 9, 20, 28, 32, 60, 170}) {
+      std::vector<int> up{-1}, column{0};
+      for (int r = 1; r < rows; ++r) column.push_back(chain_at(up, column.back(), 1));
+      for (int r = 0; r < rows; ++r) chain_at(up, column[r], length);
+      if (up.size() < 4000) look(up);
+    }
+  for (int levels : {1, 3, 5, 7})
+    for (int above : {0, 50, 150})
+      for (int length : {0, 3, 10, 40}) {
+        std::vector<int> up{-1}, now;
+        now.push_back(chain_at(up, 0, above));
+        for (int l = 0; l < levels; ++l) {
+          std::vector<int> next;
+          for (int p : now) { next.push_back(chain_at(up, p, 1)); next.push_back(chain_at(up, p, 1)); }
+          now.swap(next);
+        }
+        for (int p : now) chain_at(up, p, length);
+        look(up);
+      }
+  std::printf("shapes %d\nshape_faults %d\nshape_cost %d\n", shapes, shape_faults, (int)(worst * 100));
   // trees over several workgroups: a tile crosses once, between the top and another part, and every part's schedule is right
   int cut_faults = 0, cut_refused = 0;
   for (int i = 0; i < 120; ++i) {

@@ -104,6 +104,19 @@ def test_bushy_trees_keep_the_lean_walks(gpu, oracle, shape):
     assert bpc.size("walk_kernels") == 1
 
 
+@pytest.mark.parametrize("rows,length", [(17, 60), (20, 47)])
+def test_rows_of_equal_chains_keep_the_lean_walks(gpu, oracle, rows, length):
+    """A few chains more than waves, all equally long, run one behind the other in half as many steps again as a schedule
+    that picks the most urgent nodes of every step anew: still on the lean walks, which take two thirds of the
+    general kernels' time."""
+    tree = [-1] + list(range(rows - 1))
+    for r in range(rows):
+        tree += [r] + [len(tree) + i for i in range(length)]
+    assert np.bincount(np.array(tree[1:])).max() <= 3
+    bpc = _compare_step(gpu, oracle, len(tree), 32, 5, 19, seed=rows, tree=tree)
+    assert bpc.size("walk_kernels") == 1
+
+
 @pytest.mark.parametrize("K", [16, 32])
 def test_states_of_probability_zero(gpu, oracle, K):
     """Half of a node's states without the shown category, and half of the sums over those states only: their value is

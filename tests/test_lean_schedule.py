@@ -19,3 +19,6 @@ def test_lean_schedule(tmp_path):
     assert got["long"] <= 60   # of 1200, more than 1.4 times the fewest steps there could be
     assert got["handed"] == 1
     assert got["cut_faults"] == 0 and got["cut_refused"] == 0
+    # equal chains behind one another: what their steps cost stays below what makes the general walk kernels the better ones
+    # (those take about 1.7 times as long for the same steps)
+    assert got["shapes"] > 130 and got["shape_faults"] == 0 and got["shape_cost"] <= 130
