@@ -238,11 +238,26 @@ void HcltCircuit::build_lean_tree() {
   lean_tree_ = tree;
 }
 
-// Step schedules of the two tree walks.  Every step holds at most kWalkWaves nodes whose
-// dependencies were produced in earlier steps; among the ready nodes those with the longest
-// remaining chain go first (for unit-time tasks on a tree this greedy rule gives the fewest
-// steps).  The host also places every produced tile into one of the LDS slots, for as long
-// as a later step still reads it.
+// per inner node: inner and leaf children in the order of the variables, and the parent
+struct HcltCircuit::InnerTree {
+  std::vector<std::vector<int32_t>> ic, lc;
+  std::vector<int32_t> par;
+};
+HcltCircuit::InnerTree HcltCircuit::inner_tree() const {
+  InnerTree t{std::vector<std::vector<int32_t>>(n_inner_), std::vector<std::vector<int32_t>>(n_inner_), std::vector<int32_t>(n_inner_, -1)};
+  for (int n = 0; n < n_inner_; ++n) {
+    const int v = var_of_inner_[n];
+    if (parent_[v] >= 0) t.par[n] = inner_of_var_[parent_[v]];
+    for (int c : children_[v]) {
+      if (children_[c].empty()) t.lc[n].push_back(c);
+      else t.ic[n].push_back(inner_of_var_[c]);
+    }
+  }
+  return t;
+}
+
+// Step schedules of the tree walks.  The host also places every produced tile that changes waves into one of the LDS
+// slots, for as long as a later step still reads it.
 void HcltCircuit::build_schedules() {
   if (!walk_err_) {
     PCM_HIP(hipHostMalloc((void**)&walk_err_, sizeof(int), hipHostMallocMapped));
@@ -257,75 +272,9 @@ void HcltCircuit::build_schedules() {
   // (the lean walks keep one state word per slot behind the slots)
   lds_slots_ = std::min((max_lds_ - kLeanFlagWords * 4) / tile_bytes, (1 << (31 - kSlotShift)) - 2);
   if (lds_slots_ < 3) fail(PCM_ERR_UNSUPPORTED, "device offers %d bytes of LDS, a value tile needs %d", max_lds_, tile_bytes);
-  const int trash_slot = lds_slots_ - 1;          // idle waves and childless nodes write here
-
-  std::vector<std::vector<int32_t>> ic(n_inner_), lc(n_inner_);
-  std::vector<int32_t> par(n_inner_, -1);
-  for (int n = 0; n < n_inner_; ++n) {
-    const int v = var_of_inner_[n];
-    if (parent_[v] >= 0) par[n] = inner_of_var_[parent_[v]];
-    for (int c : children_[v]) {
-      if (children_[c].empty()) lc[n].push_back(c);
-      else ic[n].push_back(inner_of_var_[c]);
-    }
-  }
-  std::vector<uint32_t> ext;
-  // a leaf child's row operand: its category is byte 1 + i of the node's packed word (the
-  // word holds the first three leaf children; later ones only occur beyond the kPre
-  // requested-ahead operands, where the category is fetched on the spot)
-  auto leaf_child_op = [&](int var, size_t i) {
-    return kOpLeaf | (uint32_t)var | ((uint32_t)std::min<size_t>(i + 1, 3) << kXSelShift);
-  };
-  auto fill_ops = [&](StepItem& it, PreItem& q, const std::vector<uint32_t>& ops) {
-    it.n_g = (int32_t)std::min<size_t>(ops.size(), kInlineOps);
-    for (int i = 0; i < kInlineOps; ++i) it.g[i] = i < it.n_g ? ops[i] : 0;
-    for (int i = 0; i < kPre; ++i) q.g[i] = i < (int)ops.size() ? ops[i] : kOpNone;
-    it.ext_off = (int32_t)ext.size();
-    it.ext_cnt = 0;
-    if (ops.size() > (size_t)kPre) it.flags |= kItemOverflow;
-    if (ops.size() > (size_t)kInlineOps) {
-      it.ext_cnt = (int32_t)(ops.size() - kInlineOps);
-      ext.insert(ext.end(), ops.begin() + kInlineOps, ops.end());
-    }
-  };
-  auto blank = [&](int n) {
-    StepItem it;
-    std::memset(&it, 0, sizeof it);
-    it.node = n;
-    it.out_slot = trash_slot; it.in_slot = trash_slot; it.parent = n >= 0 ? par[n] : -1;
-    if (n >= 0) it.flags = (par[n] < 0 ? kItemRoot : 0) | (ic[n].empty() ? 0 : kItemHasInnerChild);
-    return it;
-  };
-  auto blank_pre = [&](int n) {
-    PreItem q;
-    std::memset(&q, 0, sizeof q);
-    q.node = n;
-    q.wnode = n;
-    for (int i = 0; i < kPre; ++i) q.g[i] = kOpNone;
-    return q;
-  };
-  // field rows [field][wave][stride] with 64 idle steps of padding (a chunk refill reads
-  // 64 steps starting anywhere below n_steps)
-  auto make_fields = [&](std::vector<StepItem>& sched, std::vector<PreItem>& pre, bool forward, int& stride,
-                         DevBuf<int32_t>& dst) {
-    const int n_steps = (int)sched.size() / kWalkWaves;
-    for (int i = 0; i < 64 * kWalkWaves; ++i) { sched.push_back(blank(-1)); pre.push_back(blank_pre(-1)); }
-    stride = n_steps + 64;
-    std::vector<int32_t> f((size_t)kSchedFields * kWalkWaves * stride, 0);
-    for (int s = 0; s < stride; ++s)
-      for (int w = 0; w < kWalkWaves; ++w) {
-        const StepItem& it = sched[(size_t)s * kWalkWaves + w];
-        const PreItem& q = pre[(size_t)s * kWalkWaves + w];
-        auto put = [&](int field, int32_t v) { f[((size_t)field * kWalkWaves + w) * stride + s] = v; };
-        put(kFNode, q.node); put(kFWnode, q.wnode);
-        put(kFG0, (int32_t)q.g[0]); put(kFG1, (int32_t)q.g[1]); put(kFG2, (int32_t)q.g[2]);
-        put(kFStore, it.node); put(kFOutSlot, it.out_slot);
-        put(kFFlags, it.flags | (it.n_l << 8));
-        if (forward) { put(kFL0, (int32_t)it.l[0]); put(kFL1, (int32_t)it.l[1]); put(kFL2, (int32_t)it.l[2]); }
-        else { put(kFL0, it.in_slot); put(kFL1, it.parent < 0 ? 0 : it.parent); put(kFL2, 0); }
-      }
-    dst.upload(f);
-  };
+  const InnerTree kin = inner_tree();
+  const std::vector<std::vector<int32_t>>&ic = kin.ic, &lc = kin.lc;
+  const std::vector<int32_t>& par = kin.par;
   build_lean_tree();
   const LeanTree& lt = *lean_tree_;
   // field rows of the lean walks (see hclt_walk_lean.hip.hpp) from their own schedule, with the same padding, or none if
@@ -401,14 +350,12 @@ void HcltCircuit::build_schedules() {
     static_assert(kLeanCheckA1 == kLA1 && kLeanCheckSlots == kLSlots && kLeanCheckTurns == kLTurns &&
                   kLeanCheckFields == kLeanFields && kLeanCheckWaves == kWalkWaves && kLeanCheckKept == kLeanAway &&
                   kLeanSlotKept == kLeanKept && kLeanSlotAway == kLeanAway && kLeanSchedWaves == kWalkWaves, "the lean schedule's headers follow the field rows");
-    const int stuck = lean_schedule_stuck_at(f, stride, stride, forward, kLeanSlotNone);
+    const int stuck = lean_schedule_stuck_at(f, stride, sched.steps, forward, kLeanSlotNone);
     if (stuck >= 0)
       fail(PCM_ERR_STATE, "%s walk schedule is unsound: wave %d would wait for ever in step %d", forward ? "forward" : "backward",
            stuck % kWalkWaves, stuck / kWalkWaves);
     return true;
   };
-  auto depth_of = [&](int n) { return depth_[var_of_inner_[n]]; };
-
   // A forest's trees are walked in groups side by side (blockIdx.y of the walk kernels): each group of whole trees
   // has a schedule of its own, so that a batch too small to fill the device with its slices (1024 examples are 64
   // workgroups) still does.  Groups are node ranges (post-order goes tree after tree) of about equal size.
@@ -426,6 +373,221 @@ void HcltCircuit::build_schedules() {
     }
     return gr;
   };
+
+  // ---- lean walks ------------------------------------------------------------------------
+  // A plan: the schedules of a walk in G groups, which the kernels take in blockIdx.y: groups of whole trees, or the parts of
+  // one tree.  A node's arithmetic does not depend on the group it is walked in, so its results are the same bits under
+  // every plan.  Going up the top of a tree is the last group, going down the first: whoever is waited for comes first.
+  std::vector<int32_t> lean_rows;   // of all plans: one upload
+  auto make_plan = [&](const std::vector<LeanScope>& scopes, const std::vector<int32_t>& part) {
+    std::unique_ptr<LeanPlan> plan(new LeanPlan);
+    const int G = (int)scopes.size();
+    plan->n_groups = G;
+    std::vector<int32_t> xid(n_inner_, -1);
+    if (!part.empty())
+      for (int n = 0; n < n_inner_; ++n)
+        for (int c : lt.inner[n])
+          if (part[c] != part[n]) xid[c] = plan->n_away++;
+    for (const bool forward : {true, false}) {
+      std::vector<LeanScope> in = scopes;
+      std::vector<LeanSchedule> sched(G);
+      int steps = 0;
+      for (int i = 0; i < G; ++i) {
+        const int g = forward ? (i + 1) % G : i;   // (part 0 is the top: going up it is scheduled last, as it runs)
+        if (!part.empty() && (g == 0) == forward) {
+          in[g].release.assign(n_inner_, 0);
+          for (int n = 0; n < n_inner_; ++n)
+            for (int c : lt.inner[n])
+              if (part[c] != part[n] && (forward ? n : c) >= 0) {
+                const int from = forward ? c : n;
+                int32_t& at = in[g].release[forward ? n : c];
+                for (const LeanSchedule& sc : sched)
+                  if (!sc.step_of.empty() && sc.step_of[from] >= 0) at = std::max(at, sc.step_of[from] + 1 + kLeanAwaySteps);
+              }
+        }
+        sched[g] = forward ? lean_schedule_up(lt, in[g], lds_slots_) : lean_schedule_down(lt, in[g], lds_slots_);
+        steps = std::max(steps, sched[g].steps);
+      }
+      const int stride = steps + 64;   // the shorter groups idle at the end
+      std::vector<int32_t> rows;
+      for (int i = 0; i < G; ++i) {
+        const int g = forward && !part.empty() ? (i + 1) % G : i;
+        if (!make_lean(in[g], sched[g], xid, forward, stride, rows)) return std::unique_ptr<LeanPlan>();
+      }
+      (forward ? plan->n_fwd_steps : plan->n_bwd_steps) = steps;
+      (forward ? plan->fwd_stride : plan->bwd_stride) = stride;
+      (forward ? plan->fwd_at : plan->bwd_at) = lean_rows.size();
+      lean_rows.insert(lean_rows.end(), rows.begin(), rows.end());
+    }
+    return plan;
+  };
+  auto whole_trees = [&](int G) {
+    std::vector<LeanScope> sc;
+    for (const auto& g : make_groups(G)) sc.push_back(LeanScope(lt, g.first, g.second));
+    return sc;
+  };
+  // In order of their number of groups.  The finer plans are for batches whose slices times the groups of the first leave most
+  // of the device idle (256 examples are 16 slices): a walk takes the plan with the most groups that still gives every
+  // workgroup a compute unit of its own.  A forest goes down to two trees a group (sixteen trees of 192 variables, 512 examples:
+  // an epoch of 16 steps 11.5 ms in groups of four trees, 10.5 in groups of two).
+  plans_.clear();
+  size_t away_tiles = 0, away_parts = 0;
+  int most_nodes = n_inner_;
+  if (K_ <= 32) {
+    std::unique_ptr<LeanPlan> plan = make_plan(whole_trees(forest_ ? std::max(1, std::min(4, T_ / 8)) : 1), {});
+    if (plan) plans_.push_back(std::move(plan));
+    for (int G = plans_.empty() ? 0 : 2 * plans_[0]->n_groups; G; G *= 2) {
+      if (forest_ ? G > 8 * plans_[0]->n_groups || G > T_ / 2 : G > kLeanMostParts || n_inner_ < G * kLeanPartNodes) break;
+      std::vector<int32_t> part;
+      std::vector<LeanScope> scopes;
+      if (forest_) {
+        scopes = whole_trees(G);
+      } else {
+        int largest = 0;
+        part = lean_parts(lt, G, &largest);
+        if (largest > 3 * most_nodes / 4) break;   // (the top alone is most of it)
+        most_nodes = largest;
+        for (int g = 0; g < G; ++g) scopes.push_back(LeanScope(part, g));
+      }
+      if ((int)scopes.size() <= plans_.back()->n_groups) break;
+      plan = make_plan(scopes, part);
+      if (!plan) break;
+      const size_t slices = (size_t)n_cus_ / G;
+      away_tiles = std::max(away_tiles, (size_t)plan->n_away * slices);
+      away_parts = std::max(away_parts, (size_t)plan->n_groups * slices);
+      plans_.push_back(std::move(plan));
+    }
+  }
+  if (!plans_.empty()) d_lean_rows_.upload(lean_rows);
+  if (away_parts) {
+    d_away_tiles_.alloc(std::max<size_t>(away_tiles, 1) * kSlice * K_);
+    d_away_sums_.alloc(away_parts * kSlice);
+    d_away_flags_.alloc(away_tiles + away_parts);
+    d_away_flags_.zero();
+    away_tiles_ = away_tiles;
+  }
+  // ---- statistics: the static operands of every node (with at most three children) ------------
+  {
+    stat_lean_ = K_ <= 32;
+    std::vector<StatNode> sn(n_inner_);
+    for (int n = 0; n < n_inner_ && stat_lean_; ++n) {
+      StatNode& q = sn[n];
+      std::memset(&q, 0, sizeof q);
+      if (ic[n].size() + lc[n].size() > 3) { stat_lean_ = false; break; }
+      q.var = var_of_inner_[n];
+      q.node = n;
+      q.c[0] = q.c[1] = q.c[2] = -1;
+      int k = 0;
+      for (int c : ic[n]) q.c[k++] = c << 3;
+      q.n_hist = 1;
+      q.hvar[0] = q.var;
+      for (size_t i = 0; i < lc[n].size(); ++i) {
+        q.c[k++] = (lc[n][i] << 3) | 1 | (int32_t)((i + 1) << 1);
+        q.hvar[q.n_hist++] = lc[n][i];
+      }
+    }
+    {   // its LDS: two histograms if they fit, else one (or the parked edge-flow blocks, if larger) | per-wave pads
+      const size_t hist = 2 * (size_t)C_ * K_, park = (size_t)kStatLeanWaves * K_ * K_, pads = (size_t)kStatLeanWaves * kSlice * K_;
+      stat_lean_hists_ = (std::max(2 * hist, park) + pads) * 4 <= (size_t)max_lds_ ? 2 : 1;
+      if ((std::max(hist, park) + pads) * 4 > (size_t)max_lds_) stat_lean_ = false;
+    }
+    if (stat_lean_) {
+      // The workgroups draw the records in this order, and the kernel ends when the last drawn node is done: the
+      // costliest nodes (passes over the batch, then histograms, then operands) go first, so that what is left for
+      // the end are the short ones.
+      const int nh_pass = stat_lean_hists_;
+      auto cost = [&](const StatNode& q) {
+        const int children = (q.c[0] >= 0) + (q.c[1] >= 0) + (q.c[2] >= 0);
+        return ((q.n_hist + nh_pass - 1) / nh_pass) * 100 + std::min(q.n_hist, nh_pass) * 10 + children;
+      };
+      std::stable_sort(sn.begin(), sn.end(), [&](const StatNode& a, const StatNode& b) { return cost(a) > cost(b); });
+      d_stat_lean_.upload(sn);
+      d_stat_claim_.upload(std::vector<uint32_t>(1, 0u));
+    }
+  }
+  lean_ = !plans_.empty() && stat_lean_;
+  // Most trees never need the other walk kernels (soft evidence and, of 4096 tree nodes and more, batches whose tiles the
+  // lean walks cannot address): their schedules are built by the first call that takes them, for 784 variables 2 of 19 ms
+  // of building a circuit.
+  if (!forest_ && !(lean_ && lean_fits(n_cus_ * kSlice))) build_general_schedules();
+  if (getenv("PCM_VERBOSE")) {
+    fprintf(stderr, "[pcmi355] hclt V=%d K=%d C=%d inner=%d trees=%d: statistics%s, %d LDS slots\n", V_, K_, C_, n_inner_, T_,
+            stat_lean_ ? " (lean)" : "", lds_slots_);
+    for (const auto& p : plans_)
+      fprintf(stderr, "[pcmi355]   lean: %d groups, forward %d steps, backward %d steps\n", p->n_groups, p->n_fwd_steps, p->n_bwd_steps);
+  }
+}
+
+// The general walk kernels' schedules and operand lists, if they are not there yet.  Every step holds at most kWalkWaves nodes
+// whose dependencies were produced in earlier steps; among the ready nodes those with the longest remaining chain go first (for
+// unit-time tasks on a tree this greedy rule gives the fewest steps).
+void HcltCircuit::build_general_schedules() {
+  if (d_stat_items_.p) return;
+  if (forest_) fail(PCM_ERR_STATE, "the general walk kernels do not take a forest");
+  const int trash_slot = lds_slots_ - 1;          // idle waves and childless nodes write here
+
+  const InnerTree kin = inner_tree();
+  const std::vector<std::vector<int32_t>>&ic = kin.ic, &lc = kin.lc;
+  const std::vector<int32_t>& par = kin.par;
+  const LeanTree& lt = *lean_tree_;
+  std::vector<uint32_t> ext;
+  // a leaf child's row operand: its category is byte 1 + i of the node's packed word (the
+  // word holds the first three leaf children; later ones only occur beyond the kPre
+  // requested-ahead operands, where the category is fetched on the spot)
+  auto leaf_child_op = [&](int var, size_t i) {
+    return kOpLeaf | (uint32_t)var | ((uint32_t)std::min<size_t>(i + 1, 3) << kXSelShift);
+  };
+  auto fill_ops = [&](StepItem& it, PreItem& q, const std::vector<uint32_t>& ops) {
+    it.n_g = (int32_t)std::min<size_t>(ops.size(), kInlineOps);
+    for (int i = 0; i < kInlineOps; ++i) it.g[i] = i < it.n_g ? ops[i] : 0;
+    for (int i = 0; i < kPre; ++i) q.g[i] = i < (int)ops.size() ? ops[i] : kOpNone;
+    it.ext_off = (int32_t)ext.size();
+    it.ext_cnt = 0;
+    if (ops.size() > (size_t)kPre) it.flags |= kItemOverflow;
+    if (ops.size() > (size_t)kInlineOps) {
+      it.ext_cnt = (int32_t)(ops.size() - kInlineOps);
+      ext.insert(ext.end(), ops.begin() + kInlineOps, ops.end());
+    }
+  };
+  auto blank = [&](int n) {
+    StepItem it;
+    std::memset(&it, 0, sizeof it);
+    it.node = n;
+    it.out_slot = trash_slot; it.in_slot = trash_slot; it.parent = n >= 0 ? par[n] : -1;
+    if (n >= 0) it.flags = (par[n] < 0 ? kItemRoot : 0) | (ic[n].empty() ? 0 : kItemHasInnerChild);
+    return it;
+  };
+  auto blank_pre = [&](int n) {
+    PreItem q;
+    std::memset(&q, 0, sizeof q);
+    q.node = n;
+    q.wnode = n;
+    for (int i = 0; i < kPre; ++i) q.g[i] = kOpNone;
+    return q;
+  };
+  // field rows [field][wave][stride] with 64 idle steps of padding (a chunk refill reads
+  // 64 steps starting anywhere below n_steps)
+  auto make_fields = [&](std::vector<StepItem>& sched, std::vector<PreItem>& pre, bool forward, int& stride,
+                         DevBuf<int32_t>& dst) {
+    const int n_steps = (int)sched.size() / kWalkWaves;
+    for (int i = 0; i < 64 * kWalkWaves; ++i) { sched.push_back(blank(-1)); pre.push_back(blank_pre(-1)); }
+    stride = n_steps + 64;
+    std::vector<int32_t> f((size_t)kSchedFields * kWalkWaves * stride, 0);
+    for (int s = 0; s < stride; ++s)
+      for (int w = 0; w < kWalkWaves; ++w) {
+        const StepItem& it = sched[(size_t)s * kWalkWaves + w];
+        const PreItem& q = pre[(size_t)s * kWalkWaves + w];
+        auto put = [&](int field, int32_t v) { f[((size_t)field * kWalkWaves + w) * stride + s] = v; };
+        put(kFNode, q.node); put(kFWnode, q.wnode);
+        put(kFG0, (int32_t)q.g[0]); put(kFG1, (int32_t)q.g[1]); put(kFG2, (int32_t)q.g[2]);
+        put(kFStore, it.node); put(kFOutSlot, it.out_slot);
+        put(kFFlags, it.flags | (it.n_l << 8));
+        if (forward) { put(kFL0, (int32_t)it.l[0]); put(kFL1, (int32_t)it.l[1]); put(kFL2, (int32_t)it.l[2]); }
+        else { put(kFL0, it.in_slot); put(kFL1, it.parent < 0 ? 0 : it.parent); put(kFL2, 0); }
+      }
+    dst.upload(f, stream);
+  };
+  auto depth_of = [&](int n) { return depth_[var_of_inner_[n]]; };
 
   // (the general walk kernels' schedules: a step's nodes are put behind a barrier, every tile takes a slot)
   auto schedule_forward = [&](std::vector<StepItem>& sched, std::vector<PreItem>& pre) {
@@ -549,112 +711,18 @@ void HcltCircuit::build_schedules() {
     }
   };
   fwd_spill_ = bwd_spill_ = false;
-  if (!forest_) {   // (a forest runs on the lean walks or not at all)
-    std::vector<StepItem> sched;
-    std::vector<PreItem> pre;
-    schedule_forward(sched, pre);
-    n_fwd_steps_ = (int)sched.size() / kWalkWaves;
-    make_fields(sched, pre, true, fwd_stride_, d_fwd_fields_);
-    d_fwd_sched_.upload(sched);
-    sched.clear();
-    pre.clear();
-    schedule_backward(sched, pre);
-    n_bwd_steps_ = (int)sched.size() / kWalkWaves;
-    make_fields(sched, pre, false, bwd_stride_, d_bwd_fields_);
-    d_bwd_sched_.upload(sched);
-  }
-  // ---- lean walks ------------------------------------------------------------------------
-  // A plan: the schedules of a walk in G groups, which the kernels take in blockIdx.y: groups of whole trees, or the parts of
-  // one tree.  A node's arithmetic does not depend on the group it is walked in, so its results are the same bits under
-  // every plan.  Going up the top of a tree is the last group, going down the first: whoever is waited for comes first.
-  std::vector<int32_t> lean_rows;   // of all plans: one upload
-  auto make_plan = [&](const std::vector<LeanScope>& scopes, const std::vector<int32_t>& part) {
-    std::unique_ptr<LeanPlan> plan(new LeanPlan);
-    const int G = (int)scopes.size();
-    plan->n_groups = G;
-    std::vector<int32_t> xid(n_inner_, -1);
-    if (!part.empty())
-      for (int n = 0; n < n_inner_; ++n)
-        for (int c : lt.inner[n])
-          if (part[c] != part[n]) xid[c] = plan->n_away++;
-    for (const bool forward : {true, false}) {
-      std::vector<LeanScope> in = scopes;
-      std::vector<LeanSchedule> sched(G);
-      int steps = 0;
-      for (int i = 0; i < G; ++i) {
-        const int g = forward ? (i + 1) % G : i;   // (part 0 is the top: going up it is scheduled last, as it runs)
-        if (!part.empty() && (g == 0) == forward) {
-          in[g].release.assign(n_inner_, 0);
-          for (int n = 0; n < n_inner_; ++n)
-            for (int c : lt.inner[n])
-              if (part[c] != part[n] && (forward ? n : c) >= 0) {
-                const int from = forward ? c : n;
-                int32_t& at = in[g].release[forward ? n : c];
-                for (const LeanSchedule& sc : sched)
-                  if (!sc.step_of.empty() && sc.step_of[from] >= 0) at = std::max(at, sc.step_of[from] + 1 + kLeanAwaySteps);
-              }
-        }
-        sched[g] = forward ? lean_schedule_up(lt, in[g], lds_slots_) : lean_schedule_down(lt, in[g], lds_slots_);
-        steps = std::max(steps, sched[g].steps);
-      }
-      const int stride = steps + 64;   // the shorter groups idle at the end
-      std::vector<int32_t> rows;
-      for (int i = 0; i < G; ++i) {
-        const int g = forward && !part.empty() ? (i + 1) % G : i;
-        if (!make_lean(in[g], sched[g], xid, forward, stride, rows)) return std::unique_ptr<LeanPlan>();
-      }
-      (forward ? plan->n_fwd_steps : plan->n_bwd_steps) = steps;
-      (forward ? plan->fwd_stride : plan->bwd_stride) = stride;
-      (forward ? plan->fwd_at : plan->bwd_at) = lean_rows.size();
-      lean_rows.insert(lean_rows.end(), rows.begin(), rows.end());
-    }
-    return plan;
-  };
-  auto whole_trees = [&](int G) {
-    std::vector<LeanScope> sc;
-    for (const auto& g : make_groups(G)) sc.push_back(LeanScope(lt, g.first, g.second));
-    return sc;
-  };
-  // In order of their number of groups.  The finer plans are for batches whose slices times the groups of the first leave most
-  // of the device idle (256 examples are 16 slices): a walk takes the plan with the most groups that still gives every
-  // workgroup a compute unit of its own.  A forest goes down to two trees a group (sixteen trees of 192 variables, 512 examples:
-  // an epoch of 16 steps 11.5 ms in groups of four trees, 10.5 in groups of two).
-  plans_.clear();
-  size_t away_tiles = 0, away_parts = 0;
-  int most_nodes = n_inner_;
-  if (K_ <= 32) {
-    std::unique_ptr<LeanPlan> plan = make_plan(whole_trees(forest_ ? std::max(1, std::min(4, T_ / 8)) : 1), {});
-    if (plan) plans_.push_back(std::move(plan));
-    for (int G = plans_.empty() ? 0 : 2 * plans_[0]->n_groups; G; G *= 2) {
-      if (forest_ ? G > 8 * plans_[0]->n_groups || G > T_ / 2 : G > kLeanMostParts || n_inner_ < G * kLeanPartNodes) break;
-      std::vector<int32_t> part;
-      std::vector<LeanScope> scopes;
-      if (forest_) {
-        scopes = whole_trees(G);
-      } else {
-        int largest = 0;
-        part = lean_parts(lt, G, &largest);
-        if (largest > 3 * most_nodes / 4) break;   // (the top alone is most of it)
-        most_nodes = largest;
-        for (int g = 0; g < G; ++g) scopes.push_back(LeanScope(part, g));
-      }
-      if ((int)scopes.size() <= plans_.back()->n_groups) break;
-      plan = make_plan(scopes, part);
-      if (!plan) break;
-      const size_t slices = (size_t)n_cus_ / G;
-      away_tiles = std::max(away_tiles, (size_t)plan->n_away * slices);
-      away_parts = std::max(away_parts, (size_t)plan->n_groups * slices);
-      plans_.push_back(std::move(plan));
-    }
-  }
-  if (!plans_.empty()) d_lean_rows_.upload(lean_rows);
-  if (away_parts) {
-    d_away_tiles_.alloc(std::max<size_t>(away_tiles, 1) * kSlice * K_);
-    d_away_sums_.alloc(away_parts * kSlice);
-    d_away_flags_.alloc(away_tiles + away_parts);
-    d_away_flags_.zero();
-    away_tiles_ = away_tiles;
-  }
+  std::vector<StepItem> sched;
+  std::vector<PreItem> pre;
+  schedule_forward(sched, pre);
+  n_fwd_steps_ = (int)sched.size() / kWalkWaves;
+  make_fields(sched, pre, true, fwd_stride_, d_fwd_fields_);
+  d_fwd_sched_.upload(sched, stream);
+  sched.clear();
+  pre.clear();
+  schedule_backward(sched, pre);
+  n_bwd_steps_ = (int)sched.size() / kWalkWaves;
+  make_fields(sched, pre, false, bwd_stride_, d_bwd_fields_);
+  d_bwd_sched_.upload(sched, stream);
   // ---- statistics: the static operands of every node ------------------------------------
   {
     std::vector<StepItem> items;
@@ -669,55 +737,14 @@ void HcltCircuit::build_schedules() {
       for (int i = 0; i < kPre; ++i) it.g[i] = q.g[i];   // absent operands name the zero tile
       items.push_back(it);
     }
-    d_stat_items_.upload(items);
-    // the same for the lean statistics kernel (nodes with at most three children)
-    stat_lean_ = K_ <= 32;
-    std::vector<StatNode> sn(n_inner_);
-    for (int n = 0; n < n_inner_ && stat_lean_; ++n) {
-      StatNode& q = sn[n];
-      std::memset(&q, 0, sizeof q);
-      if (ic[n].size() + lc[n].size() > 3) { stat_lean_ = false; break; }
-      q.var = var_of_inner_[n];
-      q.node = n;
-      q.c[0] = q.c[1] = q.c[2] = -1;
-      int k = 0;
-      for (int c : ic[n]) q.c[k++] = c << 3;
-      q.n_hist = 1;
-      q.hvar[0] = q.var;
-      for (size_t i = 0; i < lc[n].size(); ++i) {
-        q.c[k++] = (lc[n][i] << 3) | 1 | (int32_t)((i + 1) << 1);
-        q.hvar[q.n_hist++] = lc[n][i];
-      }
-    }
-    {   // its LDS: two histograms if they fit, else one (or the parked edge-flow blocks, if larger) | per-wave pads
-      const size_t hist = 2 * (size_t)C_ * K_, park = (size_t)kStatLeanWaves * K_ * K_, pads = (size_t)kStatLeanWaves * kSlice * K_;
-      stat_lean_hists_ = (std::max(2 * hist, park) + pads) * 4 <= (size_t)max_lds_ ? 2 : 1;
-      if ((std::max(hist, park) + pads) * 4 > (size_t)max_lds_) stat_lean_ = false;
-    }
-    if (stat_lean_) {
-      // The workgroups draw the records in this order, and the kernel ends when the last drawn node is done: the
-      // costliest nodes (passes over the batch, then histograms, then operands) go first, so that what is left for
-      // the end are the short ones.
-      const int nh_pass = stat_lean_hists_;
-      auto cost = [&](const StatNode& q) {
-        const int children = (q.c[0] >= 0) + (q.c[1] >= 0) + (q.c[2] >= 0);
-        return ((q.n_hist + nh_pass - 1) / nh_pass) * 100 + std::min(q.n_hist, nh_pass) * 10 + children;
-      };
-      std::stable_sort(sn.begin(), sn.end(), [&](const StatNode& a, const StatNode& b) { return cost(a) > cost(b); });
-      d_stat_lean_.upload(sn);
-      d_stat_claim_.upload(std::vector<uint32_t>(1, 0u));
-    }
+    if (ext.empty()) ext.push_back(0);
+    d_ext_ops_.upload(ext, stream);
+    if (bwd_spill_ && cap_slices_) d_G_.alloc((size_t)n_inner_ * tile_floats(cap_slices_));
+    d_stat_items_.upload(items, stream);   // last: marks the tables as built
   }
-  lean_ = !plans_.empty() && stat_lean_;
-  if (ext.empty()) ext.push_back(0);
-  d_ext_ops_.upload(ext);
-  if (getenv("PCM_VERBOSE")) {
-    fprintf(stderr, "[pcmi355] hclt V=%d K=%d C=%d inner=%d trees=%d: forward %d steps%s, backward %d steps%s, statistics%s, %d LDS slots\n",
-            V_, K_, C_, n_inner_, T_, n_fwd_steps_, fwd_spill_ ? " (spills)" : "", n_bwd_steps_, bwd_spill_ ? " (spills)" : "",
-            stat_lean_ ? " (lean)" : "", lds_slots_);
-    for (const auto& p : plans_)
-      fprintf(stderr, "[pcmi355]   lean: %d groups, forward %d steps, backward %d steps\n", p->n_groups, p->n_fwd_steps, p->n_bwd_steps);
-  }
+  if (getenv("PCM_VERBOSE"))
+    fprintf(stderr, "[pcmi355]   general walks: forward %d steps%s, backward %d steps%s\n", n_fwd_steps_, fwd_spill_ ? " (spills)" : "",
+            n_bwd_steps_, bwd_spill_ ? " (spills)" : "");
 }
 
 // Numbering the reference would give this circuit.  Nodes are created in depth-first
@@ -1309,9 +1336,11 @@ void HcltCircuit::stage_batch(const BatchRef& b, bool tiles) {
   check_walks();
   if (!b.d_data) fail(PCM_ERR_ARG, "data pointer is null");
   if (b.batch < 1) fail(PCM_ERR_ARG, "batch must be positive, got %d", b.batch);
+  const bool lean = !wide_walk_ && lean_fits(b.batch, tiles ? kKeepAll : kKeepNone);
+  if (!wide_walk_ && !lean) build_general_schedules();
   if (tiles) ensure_batch(b.batch); else ensure_staged(b.batch);
   const int Bp = ceil_div(b.batch, kSlice) * kSlice;
-  if (!wide_walk_ && lean_fits(b.batch, tiles ? kKeepAll : kKeepNone) && (int64_t)Bp * Vu_ <= kGatherBytes) {
+  if (lean && (int64_t)Bp * Vu_ <= kGatherBytes) {
     hipLaunchKernelGGL(hclt_gather_x_kernel, dim3(Bp / kSlice, ceil_div(n_inner_, kGatherNodes)), dim3(256), 0, stream,
                        reinterpret_cast<const int4*>(d_pack_vars_.p), b.d_data, b.stride_ex, b.stride_var, b.d_idx, b.batch, Bp, C_,
                        n_inner_, d_xn_.p);
@@ -1345,7 +1374,7 @@ LeanAway HcltCircuit::away() const {
 }
 
 void HcltCircuit::need_general_schedules() const {
-  if (!d_fwd_fields_.p || !d_bwd_fields_.p) fail(PCM_ERR_STATE, "the general walk kernels have no schedules of this circuit");
+  if (!d_stat_items_.p) fail(PCM_ERR_STATE, "the general walk kernels have no schedules of this circuit");
 }
 
 void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
@@ -1435,6 +1464,7 @@ void HcltCircuit::run_stats(const HcltDev& d, float rate) {
       return;
     }
   }
+  need_general_schedules();
   // LDS layout of hclt_stats_kernel
   const size_t pads = (size_t)kStatWaves * kSlice * (K_ + 16);
   auto hist_words = [&](int nh) { return std::max((((size_t)nh * hist + 3) & ~(size_t)3), (size_t)K_ * K_); };
@@ -1488,6 +1518,7 @@ void HcltCircuit::loglikelihoods(const BatchRef& b, float* d_ll) {
 HcltDev HcltCircuit::soft_stage(const SoftRef& s) {
   if (!s.d_ev) fail(PCM_ERR_ARG, "evidence pointer is null");
   if (s.batch < 1) fail(PCM_ERR_ARG, "batch must be positive, got %d", s.batch);
+  if (!wide_walk_) build_general_schedules();
   ensure_batch(s.batch);
   HcltDev d = dev(s.batch);
   if ((size_t)d.Bp * K_ * 4 >= ((size_t)1 << 31)) fail(PCM_ERR_UNSUPPORTED, "batch of %d examples is too large for one call", s.batch);

@@ -424,6 +424,9 @@ class HcltCircuit : public pcm_circuit {
   void pull_from_general();
   void build_structure();
   void build_schedules();
+  void build_general_schedules();
+  struct InnerTree;
+  InnerTree inner_tree() const;
   void build_param_order();
   void ensure_batch(int batch);
   void ensure_staged(int batch);

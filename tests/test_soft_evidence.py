@@ -464,3 +464,40 @@ def test_rows_in_registers_and_through_lds_agree(gpu, K, C, B):
             want = got
         for a, b in zip(got, want):
             assert np.array_equal(np.asarray(a), np.asarray(b), equal_nan=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", ["binary", "near"])
+@pytest.mark.parametrize("K", [16, 32])
+def test_soft_evidence_before_and_after_categorical_batches(gpu, shape, K):
+    """Soft evidence runs on the general walk kernels, whose schedules a circuit gets with its first such call: one-hot
+    evidence on a circuit that has seen categorical batches (of more examples, so that its tiles are there already) and on a
+    fresh one, against the categorical batch on the lean walks.  The binary tree's tiles overrun the general kernels' LDS
+    in both directions."""
+    torch, P = gpu
+    V, C, B = (2047 if shape == "binary" else 150), 4, 40
+    rng = np.random.default_rng(K)
+    parent = [-1] + [(v - 1) // 2 if shape == "binary" else int(rng.integers(max(0, v - 2), v)) for v in range(1, V)]
+    theta, leaf = rng.random((V, K, K)).astype(np.float32) + 0.1, rng.random((V, K, C)).astype(np.float32) + 0.1
+    a, b = (P.hclt_from_clt(np.array(parent, np.int32), C, K) for _ in range(2))
+    for c in (a, b):
+        c.set_params(np.log(theta / theta.sum(2, keepdims=True)), np.log(leaf / leaf.sum(2, keepdims=True)))
+    data = rng.integers(0, C, (90, V)).astype(np.uint8)
+    d = torch.from_numpy(data).cuda()
+    ev = torch.from_numpy(_one_hot_evidence(data[:B], C)).cuda()
+
+    def passes(c, x):
+        ll, mix = P.loglikelihoods(c, x).cpu().numpy(), P.probs_flows_circuit(c, x).cpu().numpy()
+        return [ll, mix, *c.get_flows()]
+    assert a.size("walk_kernels") == 1
+    passes(a, d)
+    hard, soft = passes(a, d[:B]), passes(a, ev)
+    fresh = passes(b, ev)
+    for x, y in zip(soft, fresh):
+        np.testing.assert_array_equal(x, y)
+    for x, y in zip(hard, passes(b, d[:B])):
+        np.testing.assert_array_equal(x, y)
+    np.testing.assert_allclose(soft[0], hard[0], rtol=1e-5)
+    np.testing.assert_allclose(soft[1], hard[1], rtol=1e-5)
+    for x, y in zip(soft[2:], hard[2:]):   # sums of 40 flows, each through a few hundred 32-bit products
+        assert np.abs(x - y).max() < 2e-4 * y.max()
