@@ -282,7 +282,9 @@ void HcltCircuit::build_schedules() {
   const size_t leaf_stride = (size_t)C_ * K_ * sizeof(float);
   auto make_lean = [&](const LeanScope& in, const LeanSchedule& sched, const std::vector<int32_t>& xid, bool forward, int stride,
                        std::vector<int32_t>& dst) -> bool {
-    if (!sched.ok || K_ > 32 || lds_slots_ >= (int)kLeanAway || (size_t)V_ * leaf_stride >= ((size_t)1 << 31)) return false;
+    if (!sched.ok || K_ > 32 || lds_slots_ >= (int)kLeanAway || !lean_array_fits(V_, (size_t)C_ * K_) ||
+        !lean_array_fits(n_inner_, (size_t)K_ * K_))
+      return false;
     const size_t f0 = dst.size();   // (the rows of a further group of trees go behind those of the groups before)
     dst.resize(f0 + (size_t)kLeanFields * kWalkWaves * stride + kWalkWaves, 0);
     int32_t* f = dst.data() + f0;
@@ -398,7 +400,7 @@ void HcltCircuit::build_schedules() {
           in[g].release.assign(n_inner_, 0);
           for (int n = 0; n < n_inner_; ++n)
             for (int c : lt.inner[n])
-              if (part[c] != part[n] && (forward ? n : c) >= 0) {
+              if (part[c] != part[n]) {
                 const int from = forward ? c : n;
                 int32_t& at = in[g].release[forward ? n : c];
                 for (const LeanSchedule& sc : sched)
@@ -1366,7 +1368,7 @@ const HcltCircuit::LeanPlan* HcltCircuit::lean_plan(int nslices) const {
 bool HcltCircuit::lean_fits(int batch, int keep) const {
   const int ns = ceil_div(batch, kSlice);
   const size_t per_node = keep == kKeepNone ? (size_t)ns * kSlice : tile_floats(ns);
-  return lean_ && !force_general_walks_ && (size_t)(n_inner_ + 1) * per_node * 4 < ((size_t)1 << 31);
+  return lean_ && !force_general_walks_ && lean_array_fits((size_t)n_inner_ + 1, per_node);
 }
 
 LeanAway HcltCircuit::away() const {

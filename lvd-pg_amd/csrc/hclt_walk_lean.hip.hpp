@@ -1,6 +1,6 @@
 // Lean tree-walk kernels: the same slice-persistent forward / backward walks as in
 // hclt_kernels.hip.hpp, for the common case (no tile ever leaves LDS, at most three children
-// per tree node, every array below 4 GiB), written for the fewest instructions per step.
+// per tree node, every array below 2 GiB), written for the fewest instructions per step.
 //
 // Why a second pair of kernels.  With one 16-example tile per wave and step, a step is only
 // ~100 useful vector instructions (8 exp, 8 log, 16 MFMA, a few adds), and four waves share a
@@ -105,7 +105,7 @@ __device__ __forceinline__ void lean_w_load(__amdgpu_buffer_rsrc_t r, uint32_t v
 // all the same, past the end of the array, where the buffer unit answers with zeros and fetches nothing.  Behind a branch
 // they would cost more than they save: the compiler counts the requests in flight for the shorter way, so the wait for
 // the next step's rows would also wait for this block, two steps early.
-constexpr uint32_t kLeanNowhere = 0x80000000u;   // (every array is shorter)
+constexpr uint32_t kLeanNowhere = 0x80000000u;   // (every array is shorter: lean_array_fits)
 template <int K>
 __device__ __forceinline__ void lean_w_load_if(__amdgpu_buffer_rsrc_t r, uint32_t vtile, int soff, WTile<K>& w) {
   lean_w_load<K>(r, soff < 0 ? kLeanNowhere + vtile : vtile, max(soff, 0), w);

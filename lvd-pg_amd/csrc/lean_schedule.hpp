@@ -34,6 +34,11 @@ constexpr int32_t kLeanSlotKept = 0xfe;   // the tile stays in the registers of 
 constexpr int32_t kLeanSlotNone = 0xff;   // nobody hands this tile on (a root)
 constexpr int32_t kLeanSlotAway = 0xfd;   // the tile goes to or comes from another workgroup
 
+// The lean kernels reach every array with a 32-bit offset from one descriptor, and send a request that is to fetch or store
+// nothing 2 GiB further on, past the end: so each array -- parameter blocks and leaf tables here, tiles and categories by the
+// batch -- has to be shorter than that.
+inline bool lean_array_fits(size_t rows, size_t floats_per_row) { return rows * floats_per_row * 4 < ((size_t)1 << 31); }
+
 struct LeanTree {   // inner nodes, children before their parents
   std::vector<int32_t> parent;               // -1: a root
   std::vector<std::vector<int32_t>> inner;   // inner children, longest chain first

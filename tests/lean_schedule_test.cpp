@@ -83,6 +83,9 @@ int main() {
     for (int v = 0; v < 40; ++v) kept += (a.slot[v] == kLeanSlotKept) + (b.slot[v] == kLeanSlotKept);
     std::printf("chain_steps %d\nchain_kept %d\n", a.steps + b.steps, kept);
   }
+  // arrays the lean kernels can address: blocks of K = 32 are 4 KB, 2^19 of them 2 GiB
+  std::printf("array_fits %d\narray_too_long %d\n", lean_array_fits((1 << 19) - 1, 32 * 32) + lean_array_fits((1 << 21) - 1, 16 * 16) + lean_array_fits(1, 1),
+              !lean_array_fits(1 << 19, 32 * 32) + !lean_array_fits(1 << 21, 16 * 16) + !lean_array_fits((size_t)1 << 30, (size_t)1 << 31));
   int faults = 0, refused_many = 0, refused_few = 0, long_ones = 0, handed = 0;
   for (int i = 0; i < 600; ++i) {
     const int n = 1 + (int)(rng() % (i % 10 == 0 ? 1500 : 200));

@@ -22,3 +22,4 @@ def test_lean_schedule(tmp_path):
     # equal chains behind one another: what their steps cost stays below what makes the general walk kernels the better ones
     # (those take about 1.7 times as long for the same steps)
     assert got["shapes"] > 130 and got["shape_faults"] == 0 and got["shape_cost"] <= 130
+    assert got["array_fits"] == 3 and got["array_too_long"] == 3
