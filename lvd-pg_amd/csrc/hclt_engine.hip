@@ -12,7 +12,7 @@
 #include "hclt_walk_lean.hip.hpp"
 #include "hclt_soft_sample.hip.hpp"
 #include "hclt_heads.hip.hpp"
-#include "lean_schedule.hpp"
+#include "lean_rows.hpp"
 #include "lean_schedule_check.hpp"
 #include "hclt_soft_evidence.hip.hpp"
 
@@ -274,90 +274,10 @@ void HcltCircuit::build_schedules() {
   if (lds_slots_ < 3) fail(PCM_ERR_UNSUPPORTED, "device offers %d bytes of LDS, a value tile needs %d", max_lds_, tile_bytes);
   const InnerTree kin = inner_tree();
   const std::vector<std::vector<int32_t>>&ic = kin.ic, &lc = kin.lc;
-  const std::vector<int32_t>& par = kin.par;
   build_lean_tree();
   const LeanTree& lt = *lean_tree_;
-  // field rows of the lean walks (see hclt_walk_lean.hip.hpp) from their own schedule, with the same padding, or none if
-  // some node has more operands than the lean kernels hold
-  const size_t leaf_stride = (size_t)C_ * K_ * sizeof(float);
-  auto make_lean = [&](const LeanScope& in, const LeanSchedule& sched, const std::vector<int32_t>& xid, bool forward, int stride,
-                       std::vector<int32_t>& dst) -> bool {
-    if (!sched.ok || K_ > 32 || lds_slots_ >= (int)kLeanAway || !lean_array_fits(V_, (size_t)C_ * K_) ||
-        !lean_array_fits(n_inner_, (size_t)K_ * K_))
-      return false;
-    const size_t f0 = dst.size();   // (the rows of a further group of trees go behind those of the groups before)
-    dst.resize(f0 + (size_t)kLeanFields * kWalkWaves * stride + kWalkWaves, 0);
-    int32_t* f = dst.data() + f0;
-    auto at = [&](int field, int w, int st) -> int32_t& { return f[((size_t)field * kWalkWaves + w) * stride + st]; };
-    auto item = [&](int st, int w) { return sched.item[(size_t)st * kWalkWaves + w]; };
-    // A wave takes its nodes one behind the other: where the schedule has it idle it is the tile it waits for that holds it
-    // up.  place[st][w]: the step of the wave itself.  The rest of the rows is padding: no node, leaf rows of variable 0.
-    std::vector<int32_t> place((size_t)sched.steps * kWalkWaves, 0);
-    int32_t* const n_own = f + (size_t)kLeanFields * kWalkWaves * stride;
-    for (int st = 0; st < sched.steps; ++st)
-      for (int w = 0; w < kWalkWaves; ++w)
-        if (item(st, w) >= 0) place[(size_t)st * kWalkWaves + w] = n_own[w]++;
-    for (int w = 0; w < kWalkWaves; ++w)
-      for (int i = 0; i < stride; ++i) {
-        for (const int field : {kLW, kLA1, kLA2, kLA3, kLSlots}) at(field, w, i) = -1;
-        at(kLNode, w, i) = n_inner_;
-      }
-    // how often each slot has been filled so far: a step's reads see the fills of earlier steps only, so the
-    // readers of a step are numbered before its writers
-    std::vector<int32_t> fills(256, 0);
-    for (int st = 0; st < sched.steps; ++st)
-      for (int pass = 0; pass < 2; ++pass)
-        for (int w = 0; w < kWalkWaves; ++w) {
-          const int n = item(st, w);
-          if (n < 0) continue;
-          int32_t& turns = at(kLTurns, w, place[(size_t)st * kWalkWaves + w]);
-          auto turn = [&](int tile, int byte) {
-            const int sl = sched.slot[tile];
-            if (sl < kLeanSlotAway) turns |= ((pass == 0 ? fills[sl] - 1 : fills[sl]++) & 0x7f) << (8 * byte);
-          };
-          if (lt.inner[n].size() > 3) return false;
-          if ((pass == 0) == forward)   // the children's tiles are bytes 1 .. 3, the node's own is byte 0
-            for (size_t i = 0; i < lt.inner[n].size(); ++i) turn(lt.inner[n][i], 1 + (int)i);
-          else
-            turn(n, 0);
-        }
-    for (int st = 0; st < sched.steps; ++st)
-      for (int w = 0; w < kWalkWaves; ++w) {
-        const int n = item(st, w), i = place[(size_t)st * kWalkWaves + w];
-        if (n < 0) continue;
-        at(kLNode, w, i) = n;
-        if (lt.inner[n].size() + (forward ? 0 : lc[n].size()) > 3 || lc[n].size() > 3) return false;
-        if (forward || !lt.inner[n].empty()) at(kLW, w, i) = (int32_t)((size_t)n * K_ * K_ * sizeof(float));
-        at(kLA0, w, i) = (int32_t)((size_t)var_of_inner_[n] * leaf_stride);
-        if (par[n] < 0) at(kLTurns, w, i) |= 0x80;
-        uint32_t slots = 0xffffff00u | (uint32_t)sched.slot[n];
-        int q = 0;
-        for (int c : lt.inner[n]) {
-          slots = (slots & ~(0xffu << (8 * (q + 1)))) | ((uint32_t)sched.slot[c] << (8 * (q + 1)));
-          if (!forward) at(kLA1 + q, w, i) = c << 3 | (lt.inner[n].size() == 1 && in.in[c] ? 2 : 0);
-          ++q;
-        }
-        at(kLSlots, w, i) = (int32_t)slots;
-        if (par[n] >= 0 && !in.in[par[n]]) at(kLAway, w, i) = xid[n];
-        for (size_t k = lt.inner[n].size(); k-- > 0;) {
-          if (in.in[lt.inner[n][k]]) continue;
-          at(kLAway, w, i) = xid[lt.inner[n][k]];   // (those of one node are numbered in order)
-          if (!forward) at(kLTurns, w, i) |= (int32_t)(0x80u << (8 * (k + 1)));
-        }
-        if (forward) q = 0;
-        for (size_t k = 0; k < lc[n].size(); ++k)
-          at(kLA1 + q++, w, i) = (int32_t)((size_t)lc[n][k] * leaf_stride) | (forward ? 0 : 1 | (int32_t)((k + 1) << 1));
-      }
-    // the waits and posts of all waves, replayed: a schedule on which a wave would wait for ever is refused here
-    static_assert(kLeanCheckA1 == kLA1 && kLeanCheckSlots == kLSlots && kLeanCheckTurns == kLTurns &&
-                  kLeanCheckFields == kLeanFields && kLeanCheckWaves == kWalkWaves && kLeanCheckKept == kLeanAway &&
-                  kLeanSlotKept == kLeanKept && kLeanSlotAway == kLeanAway && kLeanSchedWaves == kWalkWaves, "the lean schedule's headers follow the field rows");
-    const int stuck = lean_schedule_stuck_at(f, stride, sched.steps, forward, kLeanSlotNone);
-    if (stuck >= 0)
-      fail(PCM_ERR_STATE, "%s walk schedule is unsound: wave %d would wait for ever in step %d", forward ? "forward" : "backward",
-           stuck % kWalkWaves, stuck / kWalkWaves);
-    return true;
-  };
+  LeanNodes nd{lc, {}, K_, (size_t)C_ * K_ * sizeof(float)};
+  for (int n = 0; n < n_inner_; ++n) nd.var.push_back(var_of_inner_[n]);
   // A forest's trees are walked in groups side by side (blockIdx.y of the walk kernels): each group of whole trees
   // has a schedule of its own, so that a batch too small to fill the device with its slices (1024 examples are 64
   // workgroups) still does.  Groups are node ranges (post-order goes tree after tree) of about equal size.
@@ -382,45 +302,30 @@ void HcltCircuit::build_schedules() {
   // every plan.  Going up the top of a tree is the last group, going down the first: whoever is waited for comes first.
   std::vector<int32_t> lean_rows;   // of all plans: one upload
   auto make_plan = [&](const std::vector<LeanScope>& scopes, const std::vector<int32_t>& part) {
-    std::unique_ptr<LeanPlan> plan(new LeanPlan);
-    const int G = (int)scopes.size();
-    plan->n_groups = G;
-    std::vector<int32_t> xid(n_inner_, -1);
-    if (!part.empty())
-      for (int n = 0; n < n_inner_; ++n)
-        for (int c : lt.inner[n])
-          if (part[c] != part[n]) xid[c] = plan->n_away++;
+    LeanPlanRows r;
+    std::unique_ptr<LeanPlan> plan;
+    if (!lean_plan_rows(lt, nd, scopes, part, lds_slots_, r)) return plan;
+    // the waits and posts of all waves of all groups, replayed: rows on which a wave would wait for ever are refused here
+    static_assert(kLeanCheckA1 == kLA1 && kLeanCheckSlots == kLSlots && kLeanCheckTurns == kLTurns && kLeanCheckAway == kLAway &&
+                  kLeanCheckFields == kLeanFields && kLeanCheckWaves == kWalkWaves && kLeanCheckKept == kLeanAway &&
+                  kLeanSchedWaves == kWalkWaves, "the check follows the field rows, the schedules the kernels");
     for (const bool forward : {true, false}) {
-      std::vector<LeanScope> in = scopes;
-      std::vector<LeanSchedule> sched(G);
-      int steps = 0;
-      for (int i = 0; i < G; ++i) {
-        const int g = forward ? (i + 1) % G : i;   // (part 0 is the top: going up it is scheduled last, as it runs)
-        if (!part.empty() && (g == 0) == forward) {
-          in[g].release.assign(n_inner_, 0);
-          for (int n = 0; n < n_inner_; ++n)
-            for (int c : lt.inner[n])
-              if (part[c] != part[n]) {
-                const int from = forward ? c : n;
-                int32_t& at = in[g].release[forward ? n : c];
-                for (const LeanSchedule& sc : sched)
-                  if (!sc.step_of.empty() && sc.step_of[from] >= 0) at = std::max(at, sc.step_of[from] + 1 + kLeanAwaySteps);
-              }
-        }
-        sched[g] = forward ? lean_schedule_up(lt, in[g], lds_slots_) : lean_schedule_down(lt, in[g], lds_slots_);
-        steps = std::max(steps, sched[g].steps);
-      }
-      const int stride = steps + 64;   // the shorter groups idle at the end
-      std::vector<int32_t> rows;
-      for (int i = 0; i < G; ++i) {
-        const int g = forward && !part.empty() ? (i + 1) % G : i;
-        if (!make_lean(in[g], sched[g], xid, forward, stride, rows)) return std::unique_ptr<LeanPlan>();
-      }
-      (forward ? plan->n_fwd_steps : plan->n_bwd_steps) = steps;
-      (forward ? plan->fwd_stride : plan->bwd_stride) = stride;
-      (forward ? plan->fwd_at : plan->bwd_at) = lean_rows.size();
-      lean_rows.insert(lean_rows.end(), rows.begin(), rows.end());
+      const int stuck = lean_rows_stuck_at(r.rows[!forward].data(), r.n_groups, r.stride[!forward], r.steps[!forward], forward, kLeanSlotNone);
+      if (stuck >= 0)
+        fail(PCM_ERR_STATE, "%s walk schedule is unsound: wave %d of group %d of %d would wait for ever in step %d", forward ? "forward" : "backward",
+             stuck % kWalkWaves, stuck / kWalkWaves % r.n_groups, r.n_groups, stuck / kWalkWaves / r.n_groups);
     }
+    plan.reset(new LeanPlan);
+    plan->n_groups = r.n_groups;
+    plan->n_away = r.n_away;
+    plan->n_fwd_steps = r.steps[0];
+    plan->n_bwd_steps = r.steps[1];
+    plan->fwd_stride = r.stride[0];
+    plan->bwd_stride = r.stride[1];
+    plan->fwd_at = lean_rows.size();
+    lean_rows.insert(lean_rows.end(), r.rows[0].begin(), r.rows[0].end());
+    plan->bwd_at = lean_rows.size();
+    lean_rows.insert(lean_rows.end(), r.rows[1].begin(), r.rows[1].end());
     return plan;
   };
   auto whole_trees = [&](int G) {
@@ -435,7 +340,7 @@ void HcltCircuit::build_schedules() {
   plans_.clear();
   size_t away_tiles = 0, away_parts = 0;
   int most_nodes = n_inner_;
-  if (K_ <= 32) {
+  if (K_ <= 32 && lds_slots_ < (int)kLeanAway && lean_array_fits(V_, (size_t)C_ * K_) && lean_array_fits(n_inner_, (size_t)K_ * K_)) {
     std::unique_ptr<LeanPlan> plan = make_plan(whole_trees(forest_ ? std::max(1, std::min(4, T_ / 8)) : 1), {});
     if (plan) plans_.push_back(std::move(plan));
     for (int G = plans_.empty() ? 0 : 2 * plans_[0]->n_groups; G; G *= 2) {

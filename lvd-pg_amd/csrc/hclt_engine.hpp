@@ -28,10 +28,17 @@ constexpr int kSlotShift = 22;               // LDS operand: (slot + 1) << kSlot
 constexpr int kItemRoot = 1, kItemHasInnerChild = 2, kItemOverflow = 4, kItemSpillOut = 8;
 enum { kKeepNone = 0, kKeepRoots, kKeepAll };   // what the lean forward walk leaves in memory (hclt_walk_lean.hip.hpp)
 // One tree over several workgroups (hclt_walk_lean.hip.hpp): up to kLeanMostParts parts of at least kLeanPartNodes nodes on
-// average, while the largest part goes on shrinking by a quarter.  Below that the crossings cost what the parts gain: 153
-// nodes at 512 examples forward 42 us in one part, 50 in six; 632 nodes 97 in one, 95 in four (backward 125 and 107).  A tile
-// from another workgroup is expected kLeanAwaySteps steps after the step it is sent in.
-constexpr int kLeanMostParts = 16, kLeanPartNodes = 80, kLeanAwaySteps = 4;
+// average, while the largest part goes on shrinking by a quarter.  Below that the crossings cost what the parts gain.  Walks up /
+// down of 512 examples through Chow-Liu trees of images, K = 32, us in one, two, four and eight parts (-: the largest part is
+// that of four):
+//    145 nodes   32 /  32    31 /  31    33 /  32    -
+//    319 nodes   57 /  55    47 /  48    46 /  49    -
+//    642 nodes  105 / 107    72 /  78    70 /  76    -
+//    972 nodes  135 / 148    93 / 106    82 / 101    -
+//   2498 nodes  322 / 368   208 / 216   162 / 189   156 / 171
+// At K = 16, whose steps take half as long, every part counts from about 320 nodes on (642 nodes 56 / 61, 50 / 56, 53 / 58;
+// 2498 nodes 166 / 187, 114 / 130, 106 / 126, 118 / 129): the same line there is up to a tenth above the best.
+constexpr int kLeanMostParts = 16, kLeanPartNodes = 80;
 // The chains of the row queries: parts, and nodes that make a part worth its launches.
 constexpr int kKlMostParts = 8, kKlPartNodes = 24;
 constexpr int kPre = 3;          // static operand tiles a wave requests one step ahead

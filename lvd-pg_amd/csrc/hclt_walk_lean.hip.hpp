@@ -25,29 +25,10 @@
 #pragma once
 
 #include "hclt_kernels.hip.hpp"
+#include "lean_rows.hpp"
 
 namespace pcm {
 
-// Field rows of a lean schedule, [field][wave][stride] like the general one, and behind them [wave] the number of steps up
-// to the wave's last node: a wave that is through leaves the compute unit to the others.
-//   kLW     byte offset of the node's parameter block (-1: none wanted)
-//   kLA0    byte offset of the node's own leaf rows (variable * leaf_stride)
-//   kLA1..3 forward: leaf children's rows (-1: none; their categories are bytes 1..3 of the
-//           packed word).  backward: children, inner ones first, -1: none, leaf child: row
-//           offset | 1 | category byte << 1, inner child: node index << 3 (its value tile), | 2
-//           if it is the only one and comes next in this wave: its value tile is not wanted
-//   kLNode  node index (value / flow tile, packed-category row, row of maxima); idle waves:
-//           n_inner (that category row is out of range and reads as zero)
-//   kLSlots forward: out slot | child slots << 8, 16, 24 (0xff: none); backward: slot holding
-//           this node's ratio tile | slots of the inner children's ratio tiles << 8, 16, 24
-//           (0xff: that child is a leaf or absent); kLeanKept: in registers
-//   kLTurns which use of its slot a tile is, modulo 128, in the byte layout of kLSlots: a slot passes through
-//           the states 2t (free for its t-th tile), 2t + 1 (that tile is there), 2t + 2 (read, free again).  Bit 7 of byte 0:
-//           the root; bit 7 of bytes 1..3, backward: that child is away
-//   kLAway  place in the exchange of this node's tile, or of the first of its children's, that crosses workgroups (below)
-enum { kLW = 0, kLA0, kLA1, kLA2, kLA3, kLNode, kLSlots, kLTurns, kLAway, kLeanFields };
-constexpr uint32_t kLeanAway = 0xfd;       // in place of a slot: the tile comes from or goes to another workgroup
-constexpr uint32_t kLeanKept = 0xfe;       // in place of a slot: the tile stays in the registers of the wave (one that stays nowhere: 0xff)
 constexpr int kLeanFlagWords = 256;        // one state word per LDS slot, behind the slots
 constexpr int kLeanSpinLimit = 1 << 22;    // polls before a wave gives up on a tile (never reached by a sound schedule)
 

@@ -89,5 +89,17 @@ int main() {
     q.bwd(0, 1, 99, 0, {{0, 0}});
     std::printf("backward_child_first %d\n", lean_schedule_stuck_at(q.f.data(), q.stride, 2, false, 99));
   }
+  // two workgroups: a tile of the first crosses to the second through the exchange, there / never sent / read in the wrong place
+  for (const int fault : {0, 1, 2}) {
+    Sched low(1), top(1);
+    low.fwd(4, 0, fault == 1 ? 99 : kLeanCheckKept, 0);
+    top.fwd(6, 0, 99, 0, {{kLeanCheckKept, 0}});
+    low.at(kLeanCheckAway, 4, 0) = top.at(kLeanCheckAway, 6, 0) = 3;
+    if (fault == 2) top.at(kLeanCheckAway, 6, 0) = 2;
+    std::vector<int32_t> f(low.f);
+    f.resize(f.size() + kLeanCheckWaves, 0);
+    f.insert(f.end(), top.f.begin(), top.f.end());
+    std::printf("exchange_%d %d\n", fault, lean_rows_stuck_at(f.data(), 2, 1, 1, true, 99));
+  }
   return 0;
 }

@@ -1,9 +1,10 @@
-// Host test of csrc/lean_schedule.hpp: schedules of chains, stars, binary and random trees, one tree or several, for many
+// Host test of csrc/lean_schedule.hpp and csrc/lean_rows.hpp: schedules of chains, stars, binary and random trees, one tree or several, for many
 // and few slots.  Every schedule is replayed step by step.  Prints "<name> <number>" lines.
 #include <cstdio>
 #include <random>
 
-#include "lean_schedule.hpp"
+#include "lean_rows.hpp"
+#include "lean_schedule_check.hpp"
 
 using namespace pcm;
 
@@ -24,6 +25,22 @@ static LeanTree make(const std::vector<int>& parent) {
   }
   t.complete();
   return t;
+}
+
+// the same tree, given from the root (up_to[v] < v), with children before their parents
+static std::vector<int> from_root(const std::vector<int>& up_to) {
+  const int n = (int)up_to.size();
+  std::vector<std::vector<int>> ch(n);
+  for (int v = 1; v < n; ++v) ch[up_to[v]].push_back(v);
+  std::vector<int> id(n), parent(n, -1);
+  std::vector<std::pair<int, size_t>> st{{0, 0}};
+  for (int k = 0; !st.empty();) {
+    auto& top = st.back();
+    if (top.second < ch[top.first].size()) { const int c = ch[top.first][top.second++]; st.push_back({c, 0}); }
+    else { id[top.first] = k++; st.pop_back(); }
+  }
+  for (int v = 1; v < n; ++v) parent[id[v]] = id[up_to[v]];
+  return parent;
 }
 
 // 0 if the schedule is right: every node of the scope once, what a node reads was written in an earlier step and is where it
@@ -135,17 +152,7 @@ int main() {
   int shapes = 0, shape_faults = 0;
   auto look = [&](const std::vector<int>& up_to) {   // numbered from the root
     const int n = (int)up_to.size();
-    std::vector<std::vector<int>> ch(n);
-    for (int v = 1; v < n; ++v) ch[up_to[v]].push_back(v);
-    std::vector<int> id(n), parent(n, -1);
-    std::vector<std::pair<int, size_t>> st{{0, 0}};
-    for (int k = 0; !st.empty();) {
-      auto& top = st.back();
-      if (top.second < ch[top.first].size()) { const int c = ch[top.first][top.second++]; st.push_back({c, 0}); }
-      else { id[top.first] = k++; st.pop_back(); }
-    }
-    for (int v = 1; v < n; ++v) parent[id[v]] = id[up_to[v]];
-    const LeanTree t = make(parent);
+    const LeanTree t = make(from_root(up_to));
     int deep = 0;
     for (int v = 0; v < n; ++v) deep = std::max(deep, t.depth[v] + 1);
     const LeanScope in(t, 0, n);
@@ -179,49 +186,90 @@ int main() {
         look(up);
       }
   std::printf("shapes %d\nshape_faults %d\nshape_cost %d\n", shapes, shape_faults, (int)(worst * 100));
-  // trees over several workgroups: a tile crosses once, between the top and another part, and every part's schedule is right
-  int cut_faults = 0, cut_refused = 0;
+  // trees over several workgroups: a tile crosses once, between the top and another part, every part's schedule is right, and
+  // the field rows of all parts together let every wave through and leave the exchange empty.  taken[G]: cuts the engine's
+  // rule takes (the largest part no more than three quarters of that of the cut before).
+  int cut_trees = 0, cut_pairs = 0, cut_faults = 0, cut_refused = 0, cut_stuck = 0, taken[17] = {0};
   for (int i = 0; i < 120; ++i) {
-    const int n = 60 + (int)(rng() % 2000), span = i % 3 == 0 ? n : 2 + (int)(rng() % 10);
+    const int n = 60 + (int)(rng() % 2500), span = i % 3 == 0 ? n : i % 3 == 1 ? 2 + (int)(rng() % 10) : 20 + (int)(rng() % 200);
     std::vector<int> up_to(n, -1), kids(n, 0);   // numbered from the root, every node below one of its `span` predecessors
-    for (int v = 1; v < n; ++v)
-      do { up_to[v] = std::max(0, v - 1 - (int)(rng() % span)); for (; kids[up_to[v]] >= 3; ++up_to[v]) {} } while (up_to[v] >= v);
-    for (int v = 1; v < n; ++v) ++kids[up_to[v]];
-    std::vector<std::vector<int>> ch(n);
-    for (int v = 1; v < n; ++v) ch[up_to[v]].push_back(v);
-    std::vector<int> id(n), post, parent(n, -1);
-    std::vector<std::pair<int, size_t>> st{{0, 0}};
-    while (!st.empty()) {
-      auto& top = st.back();
-      if (top.second < ch[top.first].size()) { const int c = ch[top.first][top.second++]; st.push_back({c, 0}); }
-      else { id[top.first] = (int)post.size(); post.push_back(top.first); st.pop_back(); }
+    for (int v = 1; v < n; ++v) {
+      int q = std::max(0, v - 1 - (int)(rng() % span));
+      while (kids[q] >= 3) q = q + 1 < v ? q + 1 : 0;
+      up_to[v] = q;
+      ++kids[q];
     }
-    for (int v = 1; v < n; ++v) parent[id[v]] = id[up_to[v]];
-    bool wide = false;
-    for (auto& c : ch) wide = wide || c.size() > 3;
-    if (wide) continue;
-    const LeanTree t = make(parent);
+    const LeanTree t = make(from_root(up_to));
+    LeanNodes nd;
+    nd.K = 32;
+    nd.leaf_stride = 512;
+    for (int v = 0, var = 0; v < n; ++v) {
+      nd.var.push_back(var++);
+      nd.leaves.push_back({});
+      for (size_t room = 3 - t.inner[v].size(), k = t.inner[v].empty() ? 1 + rng() % room : rng() % (room + 1); k > 0; --k) nd.leaves[v].push_back(var++);
+    }
+    ++cut_trees;
+    int before = n;
+    bool going = true;
     for (int G : {2, 4, 8, 16}) {
       int largest = 0, most = 0;
       const std::vector<int32_t> part = lean_parts(t, G, &largest);
       for (int g = 0; g < G; ++g) most = std::max(most, (int)std::count(part.begin(), part.end(), g));
       if (most != largest) ++cut_faults;
+      going = going && largest <= 3 * before / 4;
+      before = largest;
+      taken[G] += going;
+      ++cut_pairs;
       for (int v = 0; v < n; ++v)
         if (part[v] < 0 || part[v] >= G || (t.parent[v] >= 0 && part[v] != part[t.parent[v]] && part[t.parent[v]] != 0)) ++cut_faults;
+      std::vector<LeanScope> scopes;
       for (int g = 0; g < G; ++g) {
-        LeanScope in(part, g);
-        in.release.assign(n, 0);
-        for (int v = 0; v < n; ++v) in.release[v] = (int)(rng() % 40);
-        const LeanSchedule a = lean_schedule_up(t, in, 79), b = lean_schedule_down(t, in, 79);
+        scopes.push_back(LeanScope(part, g));
+        LeanScope in = scopes.back(), late = in;   // tiles from other parts: the top waits for them going up, the others going down
+        late.release.assign(n, 0);
+        for (int v = 0; v < n; ++v)
+          if (t.parent[v] >= 0 && part[v] != part[t.parent[v]]) {
+            const int x = g == 0 ? t.parent[v] : v;
+            late.release[x] = std::max(late.release[x], (int32_t)(rng() % 40));
+          }
+        const LeanSchedule a = lean_schedule_up(t, g == 0 ? late : in, 79), b = lean_schedule_down(t, g == 0 ? in : late, 79);
         for (const LeanSchedule* s : {&a, &b}) {
           if (!s->ok) { ++cut_refused; continue; }
           const int f = fault(t, *s, in, 79, s == &a);
           if (f) { ++cut_faults; std::fprintf(stderr, "cut tree %d (%d nodes), part %d of %d, %s: fault %d\n", i, n, g, G, s == &a ? "up" : "down", f); }
         }
       }
+      LeanPlanRows p;
+      if (!lean_plan_rows(t, nd, scopes, part, 79, p)) { ++cut_refused; continue; }
+      int crossing = 0;
+      for (int v = 0; v < n; ++v) crossing += t.parent[v] >= 0 && part[v] != part[t.parent[v]];
+      if (crossing != p.n_away) ++cut_faults;
+      for (const bool forward : {true, false}) {
+        std::vector<uint8_t> flags;
+        const int stuck = lean_rows_stuck_at(p.rows[!forward].data(), G, p.stride[!forward], p.steps[!forward], forward, kLeanSlotNone, &flags);
+        if (stuck >= 0 || (int)flags.size() != p.n_away || std::count(flags.begin(), flags.end(), 0) != p.n_away) {
+          ++cut_stuck;
+          std::fprintf(stderr, "cut tree %d (%d nodes), %d parts, %s: stuck at %d, %d flags of %d\n", i, n, G, forward ? "up" : "down", stuck,
+                       (int)flags.size(), p.n_away);
+        }
+        // every node in one group, a wave's last step where the row behind says
+        std::vector<int> seen(n, 0);
+        const size_t per_group = (size_t)kLeanFields * kLeanSchedWaves * p.stride[!forward] + kLeanSchedWaves;
+        for (int g = 0; g < G; ++g)
+          for (int w = 0; w < kLeanSchedWaves; ++w) {
+            const int32_t* const f = p.rows[!forward].data() + g * per_group;
+            for (int st = 0; st < p.stride[!forward]; ++st) {
+              const int v = f[((size_t)kLNode * kLeanSchedWaves + w) * p.stride[!forward] + st];
+              if ((v != n) != (st < f[per_group - kLeanSchedWaves + w])) ++cut_faults;
+              if (v != n) ++seen[v];
+            }
+          }
+        cut_faults += (int)(n - std::count(seen.begin(), seen.end(), 1));
+      }
     }
   }
-  std::printf("cut_faults %d\ncut_refused %d\n", cut_faults, cut_refused);
+  std::printf("cut_trees %d\ncut_pairs %d\ncut_faults %d\ncut_refused %d\ncut_stuck %d\n", cut_trees, cut_pairs, cut_faults, cut_refused, cut_stuck);
+  for (int G : {2, 4, 8, 16}) std::printf("taken_%d %d\n", G, taken[G]);
   std::printf("faults %d\nrefused_many %d\nrefused_few %d\nlong %d\nhanded %d\n", faults, refused_many, refused_few, long_ones, handed > 0);
   return 0;
 }

@@ -18,7 +18,10 @@ def test_lean_schedule(tmp_path):
     assert got["refused_many"] == 0 and got["refused_few"] <= 5
     assert got["long"] <= 60   # of 1200, more than 1.4 times the fewest steps there could be
     assert got["handed"] == 1
-    assert got["cut_faults"] == 0 and got["cut_refused"] == 0
+    assert got["cut_faults"] == 0 and got["cut_refused"] == 0 and got["cut_stuck"] == 0
+    assert got["cut_trees"] == 120 and got["cut_pairs"] == 480
+    # cuts into 2, 4, 8 and 16 parts that the engine would take among them
+    assert got["taken_2"] >= 60 and got["taken_4"] >= 40 and got["taken_8"] >= 30 and got["taken_16"] >= 20
     # equal chains behind one another: what their steps cost stays below what makes the general walk kernels the better ones
     # (those take about 1.7 times as long for the same steps)
     assert got["shapes"] > 130 and got["shape_faults"] == 0 and got["shape_cost"] <= 130

@@ -23,3 +23,6 @@ def test_lean_schedule_check(tmp_path):
     assert got["forward_overwrite"] == 1 * 16 + 4         # the second writer waits for a read that never comes
     assert got["backward_tree"] == -1
     assert got["backward_child_first"] == 0 * 16 + 0
+    assert got["exchange_0"] == -1                        # a tile from one workgroup to another
+    assert got["exchange_1"] == (0 * 2 + 1) * 16 + 6      # never sent: step 0, group 1, wave 6
+    assert got["exchange_2"] == (0 * 2 + 1) * 16 + 6      # looked for in another place
