@@ -183,7 +183,9 @@ int pcm_set_stream(pcm_circuit* c, void* hip_stream);
  * results agree to rounding), 17 nodes whose values the per-layer kernels compute (the others are the groups'), 18 layers
  * of groups that go inside walk launches: runs of consecutive layers that hold groups of one shape and nothing else take
  * one launch per direction where their groups are few (PCMI355_GROUP_WALK=0 at creation: a launch per layer, the same
- * bits). */
+ * bits), 19 workgroups that walked a slice of 16 examples in the last likelihood or flow pass on the tree walks (parts of
+ * one tree, groups of a forest's trees; 0: no such pass yet), 20 workgroups that walked a row in the last row query on the
+ * block kernels (0: none yet). */
 int64_t pcm_size(const pcm_circuit* c, int32_t what);
 
 /* Index tables of src/bits_circuit.jl:9-36, 1-based as the reference holds them.

@@ -865,6 +865,8 @@ int64_t HcltCircuit::size(int what) const {
     case 16: return 0;
     case 17: return 0;
     case 18: return 0;
+    case 19: return walk_parts_;
+    case 20: return row_parts_;
     default: fail(PCM_ERR_ARG, "unknown size selector %d", what);
   }
 }
@@ -1285,6 +1287,7 @@ void HcltCircuit::need_general_schedules() const {
 }
 
 void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
+  walk_parts_ = lean_fits(d.B, keep) ? lean_plan(d.nslices)->n_groups : 1;
   const size_t lds = (size_t)lds_slots_ * kSlice * K_ * sizeof(float);
   auto launch = [&](auto kernel) {
     PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));

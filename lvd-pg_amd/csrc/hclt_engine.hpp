@@ -259,6 +259,7 @@ class HcltCircuit : public pcm_circuit {
   std::vector<std::unique_ptr<LeanPlan>> plans_;   // empty: the lean kernels do not take this tree
   DevBuf<int32_t> d_lean_rows_;
   const LeanPlan* lean_plan(int nslices) const;
+  int walk_parts_ = 0, row_parts_ = 0;   // workgroups per slice of the last forward walk, per row of the last row query (for pcm_size)
   // what crosses the parts of a tree: for every plan with as many slices as it is taken for
   DevBuf<float> d_away_tiles_;
   DevBuf<double> d_away_sums_;

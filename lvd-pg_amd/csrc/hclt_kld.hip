@@ -595,6 +595,7 @@ HcltCircuit::KlView HcltCircuit::kl_view(int rows) {
     v.parts = reinterpret_cast<const KlPart*>(p.tab.p + p.parts);
     break;
   }
+  row_parts_ = v.G;
   return v;
 }
 

@@ -1816,6 +1816,8 @@ int64_t SparseCircuit::size(int what) const {
     case 16: return n_groups_;
     case 17: return n_layer_nodes_;
     case 18: return n_walk_levels_;
+    case 19: return 0;
+    case 20: return 0;
     default: fail(PCM_ERR_ARG, "unknown size selector %d", what);
   }
 }

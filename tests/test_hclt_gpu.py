@@ -109,9 +109,7 @@ def test_rows_of_equal_chains_keep_the_lean_walks(gpu, oracle, rows, length):
     """A few chains more than waves, all equally long, run one behind the other in half as many steps again as a schedule
     that picks the most urgent nodes of every step anew: still on the lean walks, which take two thirds of the
     general kernels' time."""
-    tree = [-1] + list(range(rows - 1))
-    for r in range(rows):
-        tree += [r] + [len(tree) + i for i in range(length)]
+    tree = _tree_of_shape((rows, length), rows * (length + 2))
     assert np.bincount(np.array(tree[1:])).max() <= 3
     bpc = _compare_step(gpu, oracle, len(tree), 32, 5, 19, seed=rows, tree=tree)
     assert bpc.size("walk_kernels") == 1
@@ -155,30 +153,163 @@ def test_states_of_probability_zero(gpu, oracle, K):
         np.testing.assert_allclose(ea[v][:blk.shape[0]], blk, rtol=1e-4, atol=1e-5)
 
 
-@pytest.mark.parametrize("V,K,B,reach", [(70, 32, 1, 6), (160, 16, 40, 4), (700, 32, 200, 8), (1300, 32, 33, 40)])
-def test_a_tree_over_several_workgroups(gpu, oracle, V, K, B, reach):
-    """Batches of few slices walk one tree in parts, a workgroup each, whose tiles cross through memory: against the
-    oracle, and the same bits on every pass (the flags that announce the tiles are back at zero behind each), with
-    batches that are walked in fewer parts in between."""
-    torch, P = gpu
-    from helpers import correlated_data
-    rng = np.random.default_rng(V)
-    kids, tree = np.zeros(V, int), [-1]
+def _tree_of_shape(shape, V):
+    """"binary", (rows, length): rows of equal chains off a column, or n: every variable below one of the n before it"""
+    if shape == "binary":
+        return [-1] + [(v - 1) // 2 for v in range(1, V)]
+    tree = [-1]
+    if isinstance(shape, tuple):
+        tree += list(range(shape[0] - 1))
+        for r in range(shape[0]):
+            tree += [r] + [len(tree) + i for i in range(shape[1])]
+        assert len(tree) == V
+        return tree
+    rng, kids = np.random.default_rng(V), np.zeros(V, int)
     for v in range(1, V):
-        near = [u for u in range(max(0, v - reach), v) if kids[u] < 3]
+        near = [u for u in range(max(0, v - shape), v) if kids[u] < 3]
         tree.append(int(near[rng.integers(len(near))]))
         kids[tree[-1]] += 1
-    bpc = _compare_step(gpu, oracle, V, K, 6, B, seed=V, tree=tree)
-    assert bpc.size("walk_kernels") == 1
-    d = torch.from_numpy(correlated_data(2100, V, 6, 9, np.array(tree))).cuda()
+    return tree
+
+
+@pytest.mark.parametrize("shape,V,K,B,parts", [(6, 70, 32, 1, 1), ((16, 20), 352, 32, 1, 4), (40, 330, 16, 70, 2),
+                                               (300, 700, 16, 40, 4), (300, 2200, 32, 19, 8), ("binary", 2600, 32, 33, 16),
+                                               ("binary", 2600, 16, 16, 16)])
+def test_a_tree_over_several_workgroups(gpu, oracle, shape, V, K, B, parts):
+    """Batches of few slices walk one tree in parts, a workgroup each, whose tiles cross through memory: against the
+    oracle; the same bits on every pass (the flags that announce the tiles are back at zero behind each) with batches in
+    fewer parts in between; and the most slices every number of parts is taken for against one-hot soft evidence, which
+    takes the general walk kernels."""
+    torch, P = gpu
+    from helpers import correlated_data
+    tree, C = _tree_of_shape(shape, V), 6
+    bpc = _compare_step(gpu, oracle, V, K, C, B, seed=V, tree=tree)
+    assert bpc.size("walk_kernels") == 1 and bpc.size("walk_parts") == parts
+    d = torch.from_numpy(correlated_data(2100, V, C, 9, np.array(tree))).cuda()
     first = [t.cpu().numpy() for t in (P.loglikelihoods(bpc, d[:B]), P.probs_flows_circuit(bpc, d[:B]))]
+    assert bpc.size("walk_parts") == parts
     flows = bpc.get_flows()
-    for n in (2100, 700, B, B):
+    fill = [(256 // g * 16, g) for g in (1, 2, 4, 8, 16) if 1 < g <= parts]
+    for n, g in [(2100, 1), (700, min(parts, 4)), (B, parts), *fill]:
         other = P.probs_flows_circuit(bpc, d[:n]).cpu().numpy()
+        assert bpc.size("walk_parts") == g
         np.testing.assert_allclose(other[:B], first[0], rtol=1e-6)   # (the parts' shares of a likelihood add up in another order)
+        if (n, g) in fill:
+            hard = bpc.get_flows()
+            ev = torch.full((n, V, C), -float("inf"), device="cuda")
+            ev.scatter_(2, d[:n].long().unsqueeze(-1), 0.0)
+            soft = P.probs_flows_circuit(bpc, ev).cpu().numpy()
+            del ev
+            np.testing.assert_allclose(other, soft, rtol=1e-5)
+            for x, y in zip(hard, bpc.get_flows()):
+                assert np.abs(x - y).max() < FLOW_RTOL * y.max()
         again = [t.cpu().numpy() for t in (P.loglikelihoods(bpc, d[:B]), P.probs_flows_circuit(bpc, d[:B]))]
         assert all(np.array_equal(a, b) for a, b in zip(first, again))
         assert all(np.array_equal(a, b) for a, b in zip(flows, bpc.get_flows()))
+
+
+@pytest.mark.parametrize("K", [16, 32])
+@pytest.mark.parametrize("kind,shape,parts", [("root", (16, 20), 4), ("heads", (16, 20), 4), ("heads", (2, 20), 1), ("forest", (5, 12), 1)])
+def test_states_of_probability_zero_in_parts_and_under_heads(gpu, oracle, kind, shape, parts, K):
+    """The mark of a state of probability zero in the row of maxima, where the tree is walked in parts, where the head
+    kernel adds up the maxima, and in a forest: states of even variables never show an odd category, and the sums over even
+    states only are zero with them.  Every example seeds head 0, so a tree's flows are those of a single root with that
+    head's parameters."""
+    torch, P = gpu
+    from helpers import correlated_data
+    tree = np.array(_tree_of_shape(shape, shape[0] + shape[0] * (shape[1] + 1)), np.int32)
+    V, C, B, T, H = len(tree), 6, 100, 2 if kind == "forest" else 1, 3
+    rng = np.random.default_rng(K)
+    even, never = np.arange(K) % 2 == 0, -200.0
+    normalised = lambda p: np.where(p > 0, np.log(np.maximum(p / p.sum(-1, keepdims=True), 1e-300)), never).astype(np.float32)
+    th, lf, heads, data, ref = np.zeros((T, V, K, K), np.float32), np.zeros((T, V, K, C), np.float32), [], [], []
+    for t in range(T):
+        theta, leaf = oracle.random_hclt_params(tree, K, C, rng)
+        for v in [v for v in theta if v % 2 and v > 1]:
+            w = np.exp(theta[v].astype(np.float64))
+            w[::2] *= even
+            theta[v] = normalised(w)
+        p = np.exp(leaf.astype(np.float64).reshape(V, K, C))
+        p[2::2, even, 1::2] = 0.0
+        leaf = normalised(p).reshape(leaf.shape)
+        fc = oracle.hclt_flat(tree, K, C, theta, leaf)
+        x = correlated_data(B, V, C, 3 + t, tree)
+        ll, _, _, ea, lflow = oracle.em_step(fc, x, np.arange(B, dtype=np.int32), 0.1, 0.9, double=True)
+        for v, w in theta.items():
+            th[t, v, :w.shape[0]] = w
+        lf[t] = leaf
+        hd = np.log(rng.dirichlet(np.ones(K), size=H)).astype(np.float32)
+        hd[0] = theta[0][0]
+        heads.append(hd)
+        data.append(x)
+        ref.append((ll, oracle.hclt_block_aggr(fc, ea), np.asarray(lflow).reshape(V, K, C)))
+    parent = np.concatenate([np.where(tree < 0, -1, tree + t * V) for t in range(T)]).astype(np.int32)
+    bpc = (P.hclt_from_clt(parent, C, K) if kind == "root" else P.multihead_hclt_from_clt(parent, C, K, H) if kind == "heads"
+           else P.hclt_forest_from_clts(parent, C, K, H))
+    bpc.set_params(th.reshape(T * V, K, K), lf.reshape(T * V, K, C))
+    d = torch.from_numpy(np.concatenate(data, axis=1)).cuda()
+    if kind != "root":
+        bpc.set_heads(np.stack(heads) if kind == "forest" else heads[0])
+        mask = torch.zeros((T, H, B), device="cuda")
+        mask[:, 0] = 1.0
+    if kind == "root":
+        got = P.probs_flows_circuit(bpc, d).cpu().numpy()[None]
+    elif kind == "heads":
+        got = P.probs_flows_circuit(bpc, d, head_mask=mask[0].t().contiguous()).cpu().numpy()[None]
+    else:
+        got = P.forest_flows(bpc, d, mask).cpu().numpy()
+    assert bpc.size("walk_kernels") == 1 and bpc.size("walk_parts") == parts
+    ea, lflow = (x.reshape((T, V) + x.shape[1:]) for x in bpc.get_flows())
+    for t, (ll, ea_ref, lf_ref) in enumerate(ref):
+        np.testing.assert_allclose(got[t], ll, rtol=1e-5)
+        assert np.isfinite(ea[t]).all() and np.isfinite(lflow[t]).all()
+        assert np.abs(lflow[t] - lf_ref).max() < FLOW_RTOL * lf_ref.max()
+        np.testing.assert_array_equal(lflow[t][lf_ref < 1e-30], 0.0)
+        for v, blk in ea_ref.items():
+            if v:   # (the root's are the heads')
+                assert np.abs(ea[t, v][:blk.shape[0]] - blk).max() < FLOW_RTOL * max(blk.max(), 1e-3), v
+
+
+@pytest.mark.parametrize("K", [16, 32])
+def test_batches_gathered_and_staged_agree(gpu, K):
+    """Up to 2 MB of batch the lean walks' categories come straight from the caller's rows, above it from a staged copy:
+    one batch of 4000 examples of 700 variables against the same examples in batches of 1000, with example ids, rows and
+    columns apart, and categories past the last (which stand for the last)."""
+    torch, P = gpu
+    from pcmi355._lib import lib, check
+    V, C, N = 700, 7, 4000
+    parent = np.array(_tree_of_shape(8, V), np.int32)
+    rng = np.random.default_rng(K)
+    theta, leaf = rng.random((V, K, K)).astype(np.float32) + 0.1, rng.random((V, K, C)).astype(np.float32) + 0.1
+    a, b = (P.hclt_from_clt(parent, C, K) for _ in range(2))
+    for c in (a, b):
+        c.set_params(np.log(theta / theta.sum(2, keepdims=True)), np.log(leaf / leaf.sum(2, keepdims=True)))
+    x = rng.integers(0, C, (N + 50, V)).astype(np.uint8)
+    x[::7, ::5] = 255
+    ids = torch.from_numpy(rng.permutation(N + 50)[:N].astype(np.int32)).cuda()
+    wide = torch.zeros((N + 50, V + 9), dtype=torch.uint8, device="cuda")
+    wide[:, :V] = torch.from_numpy(x).cuda()
+    columns = torch.from_numpy(np.ascontiguousarray(x.T)).cuda()
+    layouts = [(wide, wide.stride(0), 1), (columns, 1, columns.stride(0))]
+
+    def call(c, layout, lo, hi, rate, out):
+        data, se, sv = layout
+        i = ids[lo:hi].contiguous()
+        check(lib.pcm_loglikelihoods(c.handle, data.data_ptr(), se, sv, i.data_ptr(), hi - lo, out.data_ptr()) if rate is None else
+              lib.pcm_flows(c.handle, data.data_ptr(), se, sv, i.data_ptr(), hi - lo, rate, None, out.data_ptr()))
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+    new = lambda n: torch.empty(n, device="cuda")
+    whole = None
+    for layout in layouts:
+        got = [call(a, layout, 0, N, None, new(N)), call(a, layout, 0, N, 0.0, new(N)), *a.get_flows()]
+        whole = whole or got
+        assert all(np.array_equal(p, q) for p, q in zip(whole, got))
+        for rate in (None, 0.0):
+            few = np.concatenate([call(b, layout, lo, lo + 1000, rate if rate is None or not lo else 1.0, new(1000)) for lo in range(0, N, 1000)])
+            np.testing.assert_allclose(few, whole[0], rtol=1e-6)
+        for p, q in zip(b.get_flows(), whole[2:]):
+            assert np.abs(p - q).max() < 1e-5 * q.max()
 
 
 @pytest.mark.parametrize("K,V", [(16, 9), (32, 40), (64, 6), (8, 5)])
@@ -575,7 +706,8 @@ def test_config_hclt48_k128(gpu, oracle):
 @pytest.mark.parametrize("V,K,C,H,B,tree", [(7, 16, 5, 3, 40, None), (12, 32, 9, 128, 70, None), (2, 16, 4, 16, 16, [-1, 0]),
                                             (9, 32, 256, 40, 33, [-1, 0, 0, 1, 1, 2, 2, 3, 3]),
                                             (13, 16, 7, 20, 50, [-1, 0, 1, 1, 1, 1, 2, 3, 0, 8, 8, 8, 8]),     # four children twice
-                                            (7, 32, 6, 5, 30, [-1, 0, 0, 0, 0, 0, 0])])                        # a star
+                                            (7, 32, 6, 5, 30, [-1, 0, 0, 0, 0, 0, 0]),                         # a star
+                                            (352, 16, 4, 5, 70, (16, 20))])                                    # in four parts
 def test_multihead_hclt_on_the_block_engine(gpu, oracle, V, K, C, H, B, tree):
     """H heads over the root's products (src-jl/multi_head_pc/bit_circuit.jl:14-56): the block
     engine (body through the walk kernels, heads in two small kernels) against the layered engine
@@ -586,6 +718,8 @@ def test_multihead_hclt_on_the_block_engine(gpu, oracle, V, K, C, H, B, tree):
     from helpers import multihead_hclt, describe_dag, correlated_data
     from pcmi355._lib import lib, check
     rng = np.random.default_rng(V * 100 + H)
+    parts = 4 if isinstance(tree, tuple) else 1
+    tree = _tree_of_shape(tree, V) if isinstance(tree, tuple) else tree
     parent = O.random_tree(V, rng, 3) if tree is None else np.array(tree, np.int32)
     heads, _ = multihead_hclt(parent, K, C, H, rng)
     g = describe_dag(heads)
@@ -615,6 +749,7 @@ def test_multihead_hclt_on_the_block_engine(gpu, oracle, V, K, C, H, B, tree):
         hm = torch.from_numpy(mask).cuda()
         mix_g = P.probs_flows_circuit(gen, d, head_mask=hm, rate=0.25 if soft else 0.0).cpu().numpy()
         mix_b = P.probs_flows_circuit(blk, d, head_mask=hm, rate=0.25 if soft else 0.0).cpu().numpy()
+        assert blk.size("walk_parts") == parts
         np.testing.assert_allclose(mix_b, mix_g, rtol=2e-5)
         np.testing.assert_allclose(mix_b, P.multihead_loglikelihoods(blk, d, hm).cpu().numpy(), rtol=2e-5)
         check(lib.pcm_em_update(gen.handle, 0.1, 0.7))

@@ -798,19 +798,22 @@ def test_row_queries_on_the_block_form_agree_with_the_layer_kernels(gpu, oracle,
                   P.gumbel_sample_backward_rows(gen, p1, G, grad_wrt_logparams=wrt_log, **kw), "reverse pass")
 
 
-@pytest.mark.parametrize("shape,V,K,C", [("near", 700, 32, 8), ("near", 300, 64, 4), ("binary", 4095, 16, 4), ("wide", 400, 16, 8)])
-def test_a_row_does_not_depend_on_the_rows_beside_it(gpu, oracle, shape, V, K, C):
+@pytest.mark.parametrize("reach,most,V,K,C", [(300, 3, 700, 32, 8), (300, 6, 640, 64, 4), (None, 2, 4095, 16, 4), (300, 6, 640, 16, 8),
+                                              (8, 3, 700, 32, 8)])
+def test_a_row_does_not_depend_on_the_rows_beside_it(gpu, oracle, reach, most, V, K, C):
     """The chains of the row queries walk a tree in eight parts, four or one by the number of rows: the same rows alone and
-    among others, in parts and in one (with vectors in LDS, and for the binary tree's wide levels in device memory)."""
+    among others, in parts and in one (with vectors in LDS, and for the binary tree's wide levels in device memory).  At
+    K = 64 nodes have up to six children (in several parts), at K = 16 auxiliary nodes below them; the last tree, mostly
+    one chain, does not come apart."""
     torch, P = gpu
     from helpers import make_hclt
     rng = np.random.default_rng(V)
-    if shape == "binary":
+    if reach is None:
         parent = [-1] + [(v - 1) // 2 for v in range(1, V)]
-    else:   # wide: up to six children a node
+    else:
         parent, kids = [-1], np.zeros(V, int)
         for v in range(1, V):
-            near = [u for u in range(max(0, v - 8), v) if kids[u] < (6 if shape == "wide" else 3)]
+            near = [u for u in range(max(0, v - reach), v) if kids[u] < most]
             parent.append(int(near[rng.integers(len(near))]))
             kids[parent[-1]] += 1
     parent, _, _, _ = make_hclt(V, K, C, 1, parent=np.array(parent, np.int32))
@@ -833,8 +836,12 @@ def test_a_row_does_not_depend_on_the_rows_beside_it(gpu, oracle, shape, V, K, C
         kw = dict(temperature=0.7, noise=z)
         return [P.kld(bpc, a, b), *P.kld_backward(bpc, a, b), P.gumbel_sample_rows(bpc, a, **kw),
                 P.gumbel_sample_backward_rows(bpc, a, g, **kw)]
+    in_parts = reach != 8
     whole = queries(0, R)
-    for lo, hi in ((0, 40), (65, 70), (3, 4)):
-        for got, ref in zip(queries(lo, hi), whole):
+    assert bpc.size("row_parts") == 1
+    for lo, hi, parts in ((0, 40, 4), (65, 70, 8), (3, 4, 8), (0, 32, 8), (0, 33, 4), (0, 64, 4), (0, 65, 1)):
+        some = queries(lo, hi)
+        assert bpc.size("row_parts") == (parts if in_parts else 1)
+        for got, ref in zip(some, whole):
             ref = ref[lo:hi]
             assert (got - ref).abs().max() <= 1e-5 * ref.abs().max()
