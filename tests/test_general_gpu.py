@@ -143,8 +143,8 @@ def test_layered_engine_on_a_batch_that_saturates_the_device(gpu, oracle):
 
 
 def test_layered_engine_with_value_arrays_beyond_two_gigabytes(gpu, oracle):
-    """From 2 GiB of node values on, the layer kernels address rows through pointers instead of buffer descriptors:
-    a circuit of about 7900 nodes (K = 32 HCLT over 128 variables) on 73728 examples, 96 copies of 768 distinct ones.  The
+    """From 2 GiB of node values on, the layer kernels address rows through pointers instead of buffer descriptors, and so do
+    the dense groups' kernels the flow rows their children's copies go to: a circuit of about 7900 nodes (K = 32 HCLT over 128 variables) on 73728 examples, 96 copies of 768 distinct ones.  The
     likelihood of a copy is that of its original in a 768-example batch (the descriptor path) and the same bits in
     every copy, and with no
     pseudocount the EM update of the large batch is the update of the small one up to rounding."""
@@ -164,6 +164,7 @@ def test_layered_engine_with_value_arrays_beyond_two_gigabytes(gpu, oracle):
                                  d["input_logp"], V, C)
     small, large = compiled(), compiled()
     assert small.num_nodes() * base * 4 < 2 ** 31 <= large.num_nodes() * base * copies * 4
+    assert large.size("dense_groups") > 60   # (with the descriptor in the small batch, by pointers in the large one)
     data = rng.integers(0, C, size=(base, V)).astype(np.uint8)
     ds = torch.from_numpy(data).cuda()
     dl = torch.from_numpy(np.tile(data, (copies, 1))).cuda()
