@@ -152,50 +152,54 @@ struct KlRowStrides {
 // operand and constants of a step are requested D = kl_ahead(K) steps before it; the chains are
 // padded to a multiple of D steps and the tables by D idle steps more, so the requests need no
 // bounds and every lane's requests complete in the order the steps use them.
-// `parts` (null: the whole tree): blockIdx.x is a part from `part0` on, and rs.down_only says which way it goes; the number of
-// waves is the launch's.  A step of sixteen nodes is 66 KB of operands, which one compute unit pulls at 75 GB/s, so a matrix
+// kParts: blockIdx.x is a part of `parts` from `part0` on, and rs.down_only says which way it goes; the number of waves is the
+// launch's.  (A build of its own: what the parts need costs a step over the whole tree 25 ns, 2 % of a query of one row.)  A step of sixteen nodes is 66 KB of operands, which one compute unit pulls at 75 GB/s, so a matrix
 // of few rows spends its time here with most of the device idle: 16 rows of the 3072-variable circuit, a chain 278 us on 16
 // workgroups, 111 in eight parts each (the parts below the top in one launch, the top in another).
-template <int K, bool kLds>
+template <int K, bool kLds, bool kParts>
 __global__ __launch_bounds__(kl_waves(K) * 64) void hclt_kld_chain_kernel(
     const KlItem* __restrict__ up_items, int up_steps, const KlItem* __restrict__ down_items, int down_steps,
     const int32_t* __restrict__ ext, const float* __restrict__ pu, const float* __restrict__ base,
     const float* __restrict__ ell, const float* __restrict__ pd, int ring_mask, float* ring_up, float* ring_down,
-    float* klv, float* __restrict__ z, float* h, KlRowStrides rs, const HcltCircuit::KlPart* __restrict__ parts, int part0,
+    float* klv_, float* __restrict__ z, float* h_, KlRowStrides rs, const HcltCircuit::KlPart* __restrict__ parts, int part0,
     const int32_t* __restrict__ away) {
+  static_assert(kLds || !kParts, "a part's vectors are in LDS");
   constexpr int PARTS = 64 / K, JP = K / PARTS, Q = JP / 4, D = kl_ahead(K);
-  const int W = blockDim.x >> 6;
+  const int W = kParts ? (int)(blockDim.x >> 6) : kl_waves(K);
   extern __shared__ float lds_ring[];   // kLds: [ring_mask + 1][K]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane % K, part = lane / K;
-  const bool up = parts ? !rs.down_only : blockIdx.x == 0 && !rs.down_only;
+  const bool up = (kParts || blockIdx.x == 0) && !rs.down_only;
   {   // a row of a parameter matrix per blockIdx.y: its operands, constants and results sit rs.* floats further on
     const size_t row = blockIdx.y;
     pu += row * rs.pu; pd += row * rs.pd; base += row * rs.vec; ell += row * rs.vec;
-    klv += row * rs.out; z += row * rs.out; h += row * rs.out;
+    klv_ += row * rs.out; z += row * rs.out; h_ += row * rs.out;
     if (ring_up) ring_up += row * rs.ring_up;
     if (ring_down) ring_down += row * rs.ring_down;
   }
   HcltCircuit::KlWalk walk{0, up ? up_steps : down_steps, 0, 0};
-  if (parts) walk = up ? parts[part0 + blockIdx.x].up : parts[part0 + blockIdx.x].down;
+  if constexpr (kParts) walk = up ? parts[part0 + blockIdx.x].up : parts[part0 + blockIdx.x].down;
   const int steps = walk.steps;
   const int4* __restrict__ items = reinterpret_cast<const int4*>(up ? up_items : down_items);
   const float4* __restrict__ par = reinterpret_cast<const float4*>(up ? pu : pd);
   float* ring_dev = up ? ring_up : ring_down;
   auto ring_at = [&](int slot) -> float* {
-    if constexpr (kLds) return lds_ring + (size_t)(slot >= kKlAway ? ring_mask + 1 + (slot - kKlAway) : slot & ring_mask) * K;
+    if constexpr (kParts) return lds_ring + (size_t)(slot >= kKlAway ? ring_mask + 1 + (slot - kKlAway) : slot & ring_mask) * K;
+    else if constexpr (kLds) return lds_ring + (size_t)(slot & ring_mask) * K;
     else return ring_dev + (size_t)slot * K;
   };
-  // The first round (q0 = -D) computes nothing and only places the requests of steps 0 .. D-1:
-  // with every request issued from the same place in the loop, the waits the compiler counts
-  // from the order of issue let D - 1 steps of requests stay in flight.
-  if constexpr (kLds)
+  if constexpr (kParts)
     if (walk.n_away) {
-      const float* const from = up ? klv : h;
+      const float* const from = up ? klv_ : h_;
       for (int i = threadIdx.x; i < walk.n_away * K; i += blockDim.x)
         lds_ring[(size_t)(ring_mask + 1) * K + i] = from[(size_t)away[walk.away0 + i / K] * K + i % K];
       __syncthreads();
     }
+  float* __restrict__ const klv = klv_;   // (written only from here on)
+  float* __restrict__ const h = h_;
+  // The first round (q0 = -D) computes nothing and only places the requests of steps 0 .. D-1:
+  // with every request issued from the same place in the loop, the waits the compiler counts
+  // from the order of issue let D - 1 steps of requests stay in flight.
   int4 it[D];
   float4 p[D][Q];
   float bs[D], el[D];
@@ -725,13 +729,16 @@ void HcltCircuit::kl_chain(const KlView& v, bool up, int rows, const float* pu, 
                          reinterpret_cast<const KlItem*>(v.up), kl_up_steps_, reinterpret_cast<const KlItem*>(v.down),
                          kl_down_steps_, v.ext, pu, base, ell, pd, v.mask, ring_up, ring_down, klv, z, h, rs, v.parts, part0, v.away);
     };
-    auto all = [&](auto kernel) {
-      if (v.G == 1) return launch(kernel, 0, 1);
+    if (v.G > 1) {
+      auto* const kernel = &hclt_kld_chain_kernel<KK, true, true>;
       if (up) launch(kernel, 1, v.G - 1);
       launch(kernel, 0, 1);
       if (!up) launch(kernel, 1, v.G - 1);
-    };
-    if (v.lds) all(&hclt_kld_chain_kernel<KK, true>); else all(&hclt_kld_chain_kernel<KK, false>);
+    } else if (v.lds) {
+      launch(&hclt_kld_chain_kernel<KK, true, false>, 0, 1);
+    } else {
+      launch(&hclt_kld_chain_kernel<KK, false, false>, 0, 1);
+    }
   });
 }
 
@@ -770,8 +777,8 @@ void HcltCircuit::kld_device(HcltCircuit* q, bool with_down) {
                          kl_ring_slots_ - 1, ring_up, ring_down, klv, z, h, KlRowStrides{0, 0, 0, 0, 0, 0, 0},
                          (const KlPart*)nullptr, 0, (const int32_t*)nullptr);
     };
-    if (kl_ring_slots_) chain(&hclt_kld_chain_kernel<KK, true>, (size_t)kl_ring_slots_ * KK * sizeof(float));
-    else chain(&hclt_kld_chain_kernel<KK, false>, 0);
+    if (kl_ring_slots_) chain(&hclt_kld_chain_kernel<KK, true, false>, (size_t)kl_ring_slots_ * KK * sizeof(float));
+    else chain(&hclt_kld_chain_kernel<KK, false, false>, 0);
   });
   check_launch_k("hclt_kld");
 }
