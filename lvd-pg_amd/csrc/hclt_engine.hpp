@@ -39,8 +39,13 @@ enum { kKeepNone = 0, kKeepRoots, kKeepAll };   // what the lean forward walk le
 // At K = 16, whose steps take half as long, every part counts from about 320 nodes on (642 nodes 56 / 61, 50 / 56, 53 / 58;
 // 2498 nodes 166 / 187, 114 / 130, 106 / 126, 118 / 129): the same line there is up to a tenth above the best.
 constexpr int kLeanMostParts = 16, kLeanPartNodes = 80;
-// The chains of the row queries: parts, and nodes that make a part worth its launches.
-constexpr int kKlMostParts = 8, kKlPartNodes = 24;
+// The chains of the row queries in parts: how many, and the nodes a tree needs for them.  Parts cost a second launch per chain and
+// save steps, whose length goes with the operands of a node, K x K.  Gradient of the KL of eight rows, us in one part / in eight:
+// K = 64 390 / 297 at about 200 nodes, 522 / 407 at 290; K = 32 141 / 122 at 200, 347 / 285 at 610; but K = 16 85 / 91 at 200,
+// 97 / 110 at 290, 162 / 177 at 610, 192 / 175 at 770, 319 / 268 at 1370.  Of 64 rows, in four parts: K = 16 586 / 593 at 610 and
+// 732 / 715 at 770.
+constexpr int kKlMostParts = 8;
+constexpr int kl_part_nodes(int K, int parts) { return K > 16 ? 24 * parts : 700; }
 constexpr int kPre = 3;          // static operand tiles a wave requests one step ahead
 
 struct HcltNode {     // one non-leaf tree node, device-resident

@@ -577,7 +577,7 @@ HcltCircuit::KlView HcltCircuit::kl_view(int rows) {
   for (int i = 0; i < 2; ++i) {
     const int G = kKlMostParts >> i;
     KlPlan& p = kl_plans_[i];
-    if (!block_ || n_inner_ < G * kKlPartNodes || (int64_t)rows * G > n_cus_) continue;
+    if (!block_ || n_inner_ < kl_part_nodes(K_, G) || (int64_t)rows * G > n_cus_) continue;
     if (!p.tried) {   // a plan is built by the first call that takes it (not under capture: that call takes the tables above)
       hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
       if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) continue;
