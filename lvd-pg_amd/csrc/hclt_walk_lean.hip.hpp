@@ -156,8 +156,8 @@ __device__ __forceinline__ void lean_post(unsigned* state, unsigned value) {
 // and whoever is waited for comes first in the grid.  Workgroups go to the dies in turn and are dispatched in order within a
 // die, so the grid's first dimension is a multiple of their number: the parts of a slice are then on one die, and a
 // workgroup never holds a compute unit while the one it waits for still queues behind another stream's.  The waits are
-// bounded like those for LDS tiles.  3072 variables, K = 32, 512 examples: forward 336 -> 194 us, backward 444 -> 235 in
-// eight parts; 1024 examples 338 -> 201 and 480 -> 271 in four; 784 variables, 512 examples: 97 -> 97 and 125 -> 107.
+// bounded like those for LDS tiles.  3072 variables, K = 32, 512 examples: forward 322 -> 156 us, backward 368 -> 171 in
+// eight parts; 1024 examples 322 -> 173 and 394 -> 221 in four; 784 variables, 512 examples: 105 -> 70 and 107 -> 76.
 struct LeanAway {
   float* tiles;        // [tile][slice][16 * K]
   unsigned* flags;     // [tile][slice]
