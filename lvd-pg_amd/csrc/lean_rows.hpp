@@ -57,11 +57,9 @@ inline bool lean_field_rows(const LeanTree& t, const LeanNodes& nd, const LeanSc
   for (int st = 0; st < sched.steps; ++st)
     for (int w = 0; w < W; ++w)
       if (item(st, w) >= 0) place[(size_t)st * W + w] = n_own[w]++;
-  for (int w = 0; w < W; ++w)
-    for (int i = 0; i < stride; ++i) {
-      for (const int field : {kLW, kLA1, kLA2, kLA3, kLSlots}) at(field, w, i) = -1;
-      at(kLNode, w, i) = (int32_t)t.parent.size();
-    }
+  const size_t field = (size_t)W * stride;
+  for (const int none : {kLW, kLA1, kLA2, kLA3, kLSlots}) std::fill_n(f + none * field, field, -1);
+  std::fill_n(f + kLNode * field, field, (int32_t)t.parent.size());
   // how often each slot has been filled so far: a step's reads see the fills of earlier steps only, so the
   // readers of a step are numbered before its writers
   std::vector<int32_t> fills(256, 0);
@@ -151,6 +149,7 @@ inline bool lean_plan_rows(const LeanTree& t, const LeanNodes& nd, const std::ve
     }
     p.steps[!forward] = steps;
     p.stride[!forward] = steps + 64;   // the shorter groups idle at the end
+    p.rows[!forward].reserve((size_t)G * (kLeanFields * kLeanSchedWaves * (size_t)(steps + 64) + kLeanSchedWaves));
     for (int i = 0; i < G; ++i) {
       const int g = forward && !part.empty() ? (i + 1) % G : i;
       if (!lean_field_rows(t, nd, in[g], sched[g], xid, forward, steps + 64, p.rows[!forward])) return false;

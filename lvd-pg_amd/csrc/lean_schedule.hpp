@@ -190,6 +190,7 @@ inline LeanSchedule lean_schedule_up(const LeanTree& t, const LeanScope& in, int
     if (t.parent[v] < 0) s.slot[v] = kLeanSlotNone;
     else if (!in.in[t.parent[v]]) s.slot[v] = kLeanSlotAway;
   }
+  int32_t now[W];
   int live = 0;   // tiles nobody has taken yet, those in registers among them
   for (size_t done = 0; done < in.nodes.size(); ++s.steps) {
     for (int v; (v = later.top(all)) >= 0 && in.ready_at(v) <= s.steps;) {
@@ -197,7 +198,7 @@ inline LeanSchedule lean_schedule_up(const LeanTree& t, const LeanScope& in, int
       later.e.pop_back();
       add(v);
     }
-    std::vector<int32_t> now(W, -1);
+    std::fill_n(now, W, -1);
     int taken = 0;
     for (int w = 0; w < W; ++w) {   // chains first; of several children that could hand on in registers the first does
       const int c = last[w], p = c < 0 ? -1 : t.parent[c];
@@ -287,6 +288,8 @@ inline LeanSchedule lean_schedule_down(const LeanTree& t, const LeanScope& in, i
       add(v);
       s.slot[v] = t.parent[v] < 0 ? kLeanSlotNone : kLeanSlotAway;
     }
+  int32_t now[W];
+  bool held[W];
   int live = 0;
   for (size_t done = 0; done < in.nodes.size(); ++s.steps) {
     for (int v; (v = later.top(all)) >= 0 && in.ready_at(v) <= s.steps;) {
@@ -294,8 +297,8 @@ inline LeanSchedule lean_schedule_down(const LeanTree& t, const LeanScope& in, i
       later.e.pop_back();
       add(v);
     }
-    std::vector<int32_t> now(W, -1);
-    std::vector<char> held(W, 0);
+    std::fill_n(now, W, -1);
+    std::fill_n(held, W, false);
     int taken = 0, freed = 0, open = 0, widest = 0;
     for (int w = 0; w < W; ++w) {
       const int c = last[w] < 0 ? -1 : next(last[w]);

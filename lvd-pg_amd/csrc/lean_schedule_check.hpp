@@ -34,6 +34,7 @@ constexpr int kLeanCheckFlag = 256;   // (a tile in the exchange: 0 not there, 1
 inline void lean_step_ops(const int32_t* f, int stride, int w, int s, bool forward, int trash_slot, std::vector<LeanSlotOp>& ops) {
   auto get = [&](int field) { return (uint32_t)f[((size_t)field * kLeanCheckWaves + w) * stride + s]; };
   const uint32_t slots = get(kLeanCheckSlots), turns = get(kLeanCheckTurns);
+  if (slots == 0xffffffffu) return;   // (an idle step, or nothing to hand over)
   auto sl = [&](int c) { return (uint8_t)((slots >> (8 * c)) & 0xffu); };
   auto st = [&](int c, int add) { return (uint8_t)((2u * ((turns >> (8 * c)) & 0x7fu) + (uint32_t)add) & 0xffu); };
   auto is_away = [&](int c) { return sl(c) == kLeanCheckKept && sl(c) != (uint8_t)trash_slot; };
@@ -90,13 +91,13 @@ inline int lean_rows_stuck_at(const int32_t* f, int n_groups, int stride, int n_
   const size_t per_group = (size_t)kLeanCheckFields * kLeanCheckWaves * stride + kLeanCheckWaves;
   const int n_waves = n_groups * kLeanCheckWaves;
   std::vector<std::vector<LeanSlotOp>> ops(n_waves);
-  std::vector<std::vector<int>> step_of(n_waves);
+  std::vector<std::vector<uint32_t>> step_end(n_waves, std::vector<uint32_t>(n_steps));   // operations up to a step's end
   int n_flags = 0;
   for (int w = 0; w < n_waves; ++w)
     for (int s = 0; s < n_steps; ++s) {
       const size_t before = ops[w].size();
       lean_step_ops(f + (size_t)(w / kLeanCheckWaves) * per_group, stride, w % kLeanCheckWaves, s, forward, trash_slot, ops[w]);
-      step_of[w].resize(ops[w].size(), s);
+      step_end[w][s] = (uint32_t)ops[w].size();
       for (size_t i = before; i < ops[w].size(); ++i) {
         if (ops[w][i].slot < kLeanCheckFlag) ops[w][i].slot += w / kLeanCheckWaves * kLeanCheckFlag;
         else n_flags = std::max(n_flags, (ops[w][i].slot += (n_groups - 1) * kLeanCheckFlag) - n_groups * kLeanCheckFlag + 1);
@@ -117,7 +118,10 @@ inline int lean_rows_stuck_at(const int32_t* f, int n_groups, int stride, int n_
   }
   if (flags) flags->assign(state.begin() + (size_t)n_groups * kLeanCheckFlag, state.end());
   for (int w = 0; w < n_waves; ++w)
-    if (pos[w] < ops[w].size()) return (step_of[w][pos[w]] * n_groups + w / kLeanCheckWaves) * kLeanCheckWaves + w % kLeanCheckWaves;
+    if (pos[w] < ops[w].size()) {
+      const int step = (int)(std::upper_bound(step_end[w].begin(), step_end[w].end(), (uint32_t)pos[w]) - step_end[w].begin());
+      return (step * n_groups + w / kLeanCheckWaves) * kLeanCheckWaves + w % kLeanCheckWaves;
+    }
   return -1;
 }
 
