@@ -13,7 +13,7 @@
 //
 // A chain never leaves its wave, so a few chains more than waves, all about equally long, run one behind the other: 17 rows of
 // 60 nodes off a column take 121 steps where the most urgent sixteen of every step, picked anew, would take 77.  That costs
-// little, as a step's time goes with the waves at work in it (0.3 of a full step's with one: lean_steps_cost), and a tree with
+// little, as a step's time goes with the waves at work in it (0.3 of a full step's with one), and a tree with
 // such schedules (K <= 32) runs on the lean walks whatever the general walk kernels' would be: scores of 4096 examples
 // of those 17 rows 149 us against 220, 18 rows of 170 386 against 576.  Letting a chain give up its wave to a more
 // urgent node, its tile in a slot, saves the steps but hardly time: 140 us there, and where chains and turns are closer it
@@ -353,10 +353,6 @@ inline LeanSchedule lean_schedule_down(const LeanTree& t, const LeanScope& in, i
   LeanSchedule s = lean_schedule_down(t, in, n_slots, false);
   return s.ok ? s : lean_schedule_down(t, in, n_slots, true);
 }
-
-// What the steps of a walk over so many nodes cost, a step with all sixteen waves at work being 1.  (17 rows of 60 nodes against
-// 16: 45 steps with one wave more, 22 us more; the 76 others take 128.)
-inline double lean_steps_cost(int steps, size_t nodes) { return 0.3 * steps + 0.7 * (double)nodes / kLeanSchedWaves; }
 
 // One tree cut for `G` workgroups: part 0 has the top of the tree, everything more than 1 / (2 G) of the nodes hang from,
 // and the subtrees below it are dealt to the parts, largest first, each to the part with the fewest nodes.  So a tile
