@@ -341,6 +341,7 @@ void HcltCircuit::build_schedules() {
   plans_.clear();
   size_t away_tiles = 0, away_parts = 0;
   int most_nodes = n_inner_;
+  double walk_us = lean_walk_us(lt, std::vector<int32_t>(n_inner_, 0), n_inner_, K_);
   if (K_ <= 32 && lds_slots_ < (int)kLeanAway && lean_array_fits(V_, (size_t)C_ * K_) && lean_array_fits(n_inner_, (size_t)K_ * K_)) {
     std::unique_ptr<LeanPlan> plan = make_plan(whole_trees(forest_ ? std::max(1, std::min(4, T_ / 8)) : 1), {});
     if (plan) plans_.push_back(std::move(plan));
@@ -355,6 +356,9 @@ void HcltCircuit::build_schedules() {
         part = lean_parts(lt, G, &largest);
         if (largest > 3 * most_nodes / 4) break;   // (the top alone is most of it)
         most_nodes = largest;
+        const double us = lean_walk_us(lt, part, largest, K_);
+        if (us > walk_us) break;   // (it waits for tiles that cross)
+        walk_us = us;
         for (int g = 0; g < G; ++g) scopes.push_back(LeanScope(part, g));
       }
       if ((int)scopes.size() <= plans_.back()->n_groups) break;

@@ -36,8 +36,9 @@ enum { kKeepNone = 0, kKeepRoots, kKeepAll };   // what the lean forward walk le
 //    642 nodes  105 / 107    72 /  78    70 /  76    -
 //    972 nodes  135 / 148    93 / 106    82 / 101    -
 //   2498 nodes  322 / 368   208 / 216   162 / 189   156 / 171
-// At K = 16, whose steps take half as long, every part counts from about 320 nodes on (642 nodes 56 / 61, 50 / 56, 53 / 58;
-// 2498 nodes 166 / 187, 114 / 130, 106 / 126, 118 / 129): the same line there is up to a tenth above the best.
+// At K = 16, whose steps take half as long and whose tiles cross no faster, fewer parts gain (642 nodes 56 / 61, 50 / 56, 53 / 58;
+// 2498 nodes 166 / 187, 114 / 130, 106 / 126, 118 / 129), and trees with branches all along a long chain lose at any K: more parts
+// are taken only where lean_walk_us says that the walk gets shorter.
 constexpr int kLeanMostParts = 16, kLeanPartNodes = 80;
 // The chains of the row queries in parts: how many, and the nodes a tree needs for them.  Parts cost a second launch per chain and
 // save steps, whose length goes with the operands of a node, K x K.  Gradient of the KL of eight rows, us in one part / in eight:

@@ -192,7 +192,7 @@ int main() {
   std::printf("shapes %d\nshape_faults %d\nshape_cost %d\n", shapes, shape_faults, (int)(worst * 100));
   // trees over several workgroups: a tile crosses once, between the top and another part, every part's schedule is right, and
   // the field rows of all parts together let every wave through and leave the exchange empty.  taken[G]: cuts the engine's
-  // rule takes (the largest part no more than three quarters of that of the cut before).
+  // rule takes at K = 32 (the largest part no more than three quarters of that of the cut before, and the walk shorter).
   int cut_trees = 0, cut_pairs = 0, cut_faults = 0, cut_refused = 0, cut_stuck = 0, taken[17] = {0};
   for (int i = 0; i < 120; ++i) {
     const int n = 60 + (int)(rng() % 2500), span = i % 3 == 0 ? n : i % 3 == 1 ? 2 + (int)(rng() % 10) : 20 + (int)(rng() % 200);
@@ -215,13 +215,16 @@ int main() {
     ++cut_trees;
     int before = n;
     bool going = true;
+    double us = lean_walk_us(t, std::vector<int32_t>(n, 0), n, 32);
     for (int G : {2, 4, 8, 16}) {
       int largest = 0, most = 0;
       const std::vector<int32_t> part = lean_parts(t, G, &largest);
       for (int g = 0; g < G; ++g) most = std::max(most, (int)std::count(part.begin(), part.end(), g));
       if (most != largest) ++cut_faults;
-      going = going && largest <= 3 * before / 4;
+      const double part_us = lean_walk_us(t, part, largest, 32);
+      going = going && largest <= 3 * before / 4 && part_us <= us;
       before = largest;
+      us = part_us;
       taken[G] += going;
       ++cut_pairs;
       for (int v = 0; v < n; ++v)
@@ -274,6 +277,36 @@ int main() {
   }
   std::printf("cut_trees %d\ncut_pairs %d\ncut_faults %d\ncut_refused %d\ncut_stuck %d\n", cut_trees, cut_pairs, cut_faults, cut_refused, cut_stuck);
   for (int G : {2, 4, 8, 16}) std::printf("taken_%d %d\n", G, taken[G]);
+  // a spine with a branch at every node waits for what crosses, a crown of chains does not: parts that gain, of 2, 4, 8 and 16
+  auto gains = [&](int spine, int branch, int levels, int K) {
+    std::vector<int> up{-1}, ends{0};
+    if (spine)
+      for (int i = 0, p = 0; i < spine; ++i, p = (int)up.size() - 1) {
+        chain_at(up, p, branch);
+        up.push_back(p);
+      }
+    for (int l = 0; l < levels; ++l) {
+      std::vector<int> below;
+      for (int u : ends)
+        for (int k = 0; k < 2; ++k) below.push_back(chain_at(up, u, l + 1 < levels ? 1 : branch));
+      ends = below;
+    }
+    const LeanTree t = make(from_root(up));
+    const int n = (int)up.size();
+    double us = lean_walk_us(t, std::vector<int32_t>(n, 0), n, K);
+    int best = 1;
+    for (int G : {2, 4, 8, 16}) {
+      int largest = 0;
+      const std::vector<int32_t> part = lean_parts(t, G, &largest);
+      const double x = lean_walk_us(t, part, largest, K);
+      if (x > us) break;
+      us = x;
+      best = G;
+    }
+    return best;
+  };
+  std::printf("gain_spine_16 %d\ngain_spine_32 %d\ngain_crown_16 %d\ngain_crown_32 %d\n", gains(200, 7, 0, 16), gains(200, 7, 0, 32),
+              gains(0, 40, 5, 16), gains(0, 40, 5, 32));
   std::printf("faults %d\nrefused_many %d\nrefused_few %d\nlong %d\nhanded %d\n", faults, refused_many, refused_few, long_ones, handed > 0);
   return 0;
 }

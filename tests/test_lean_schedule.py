@@ -26,3 +26,5 @@ def test_lean_schedule(tmp_path):
     # (those take about 1.7 times as long for the same steps)
     assert got["shapes"] > 130 and got["shape_faults"] == 0 and got["shape_cost"] <= 130
     assert got["array_fits"] == 3 and got["array_too_long"] == 3
+    assert got["gain_spine_16"] == 1 and got["gain_spine_32"] <= 2   # (measured best: one part, and 251 us in one against 261 in two)
+    assert got["gain_crown_16"] >= 8 and got["gain_crown_32"] >= 8
