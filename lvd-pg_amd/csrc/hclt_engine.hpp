@@ -40,13 +40,10 @@ enum { kKeepNone = 0, kKeepRoots, kKeepAll };   // what the lean forward walk le
 // 2498 nodes 166 / 187, 114 / 130, 106 / 126, 118 / 129), and trees with branches all along a long chain lose at any K: more parts
 // are taken only where lean_walk_us says that the walk gets shorter.
 constexpr int kLeanMostParts = 16, kLeanPartNodes = 80;
-// The chains of the row queries in parts: how many, and the nodes a tree needs for them.  Parts cost a second launch per chain and
-// save steps, whose length goes with the operands of a node, K x K.  Gradient of the KL of eight rows, us in one part / in eight:
-// K = 64 390 / 297 at about 200 nodes, 522 / 407 at 290; K = 32 141 / 122 at 200, 347 / 285 at 610; but K = 16 85 / 91 at 200,
-// 97 / 110 at 290, 162 / 177 at 610, 192 / 175 at 770, 319 / 268 at 1370.  Of 64 rows, in four parts: K = 16 586 / 593 at 610 and
-// 732 / 715 at 770.
-constexpr int kKlMostParts = 8;
-constexpr int kl_part_nodes(int K, int parts) { return K > 16 ? 24 * parts : 700; }
+// The chains of the row queries in parts: how many, and the nodes that make a part worth its launches (whether a tree comes apart
+// at all is kl_chains_us's to say).  Gradient of the KL of eight rows, us in one part / in eight: K = 64 390 / 297 at 200 nodes,
+// 522 / 407 at 290; K = 32 141 / 122 at 200, 347 / 285 at 610; K = 16, random trees, 69 / 63 at 420, bushy ones 88 / 79 at 670.
+constexpr int kKlMostParts = 8, kKlPartNodes = 24;
 constexpr int kPre = 3;          // static operand tiles a wave requests one step ahead
 
 struct HcltNode {     // one non-leaf tree node, device-resident
@@ -413,7 +410,7 @@ class HcltCircuit : public pcm_circuit {
   struct KlPlan {
     bool tried = false, ok = false;
     DevBuf<int32_t> tab;
-    int W = 0, slots = 0, most_away = 0;
+    int W = 0, slots = 0, most_away = 0, steps = 0;
     size_t su = 0, sd = 0;
     size_t up = 0, down = 0, pos = 0, ext = 0, away = 0, parts = 0;   // where in `tab`
   };

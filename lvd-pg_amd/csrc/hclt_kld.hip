@@ -556,7 +556,20 @@ void HcltCircuit::build_kld_tables() {
   d_kl_up_ = {d_kl_all_.p + at_up, up.size() * 4};   // last: marks the tables as built
 }
 
-// The chains of the row queries: in parts where the rows leave most of the device idle and LDS holds every vector of a part, else on the tables above.
+// What the chains up and down of a row query take, in us: their steps (in parts those of the largest part and of the top, one
+// behind the other) and, in one workgroup of sixteen waves, the nodes in them; in parts a launch more each way; and the
+// operands of all slots, idle ones too, for every row.  Where a tree is mostly a few chains as long as a part, parts walk them
+// one behind the other: sixteen chains of 60 nodes, KL of one row, K = 16, 52 us in one part, 60 in eight; K = 32, 64 rows,
+// relaxed samples in four parts 12 % above one.  From the differences between one part and eight or four in three queries of 1, 8,
+// 32 and 64 rows on 17 trees of 211 to 1600 nodes (spines, crowns, random and Chow-Liu trees).
+static double kl_chains_us(int K, bool parts, int steps, int nodes, size_t slots, int rows) {
+  const double step = parts ? (K == 64 ? 0.45 : K == 32 ? 0.3 : 0.31) : K == 64 ? 1.3 : K == 32 ? 0.34 : 0.19;
+  const double node = parts || K == 64 ? 0.0 : K == 32 ? 0.03 : 0.022;
+  return step * steps + node * 2 * nodes + (parts ? 6.0 : 0.0) + 0.3e-6 * (double)slots * K * K * rows;
+}
+
+// The chains of the row queries: in parts where the rows leave most of the device idle, LDS holds every vector of a part
+// and the chains get shorter, else on the tables above.
 HcltCircuit::KlView HcltCircuit::kl_view(int rows) {
   build_kld_tables();
   const int D = kl_ahead(K_);
@@ -574,16 +587,17 @@ HcltCircuit::KlView HcltCircuit::kl_view(int rows) {
   v.pos = d_kl_pos_.p;
   v.parts = nullptr;
   v.away = nullptr;
+  const double whole_us = kl_chains_us(K_, false, kl_up_steps_ + kl_down_steps_, n_inner_, v.su + v.sd, rows);
   for (int i = 0; i < 2; ++i) {
     const int G = kKlMostParts >> i;
     KlPlan& p = kl_plans_[i];
-    if (!block_ || n_inner_ < kl_part_nodes(K_, G) || (int64_t)rows * G > n_cus_) continue;
+    if (!block_ || n_inner_ < G * kKlPartNodes || (int64_t)rows * G > n_cus_) continue;
     if (!p.tried) {   // a plan is built by the first call that takes it (not under capture: that call takes the tables above)
       hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
       if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) continue;
       build_kl_plan(*lean_tree_, p, G);
     }
-    if (!p.ok) continue;
+    if (!p.ok || kl_chains_us(K_, true, p.steps, n_inner_, p.su + p.sd, rows) > whole_us) continue;
     v.G = G;
     v.W = p.W;
     v.lds = true;
@@ -619,8 +633,10 @@ void HcltCircuit::build_kl_plan(const LeanTree& t, KlPlan& p, int G) {
   all[0].reserve((size_t)4 * n_inner_);
   all[1].reserve((size_t)4 * n_inner_);
   int reach = 0;
+  p.steps = 0;
   for (int dir = 0; dir < 2; ++dir) {
     const bool up = dir == 0;
+    int longest = 0;   // of the parts below the top
     std::fill(pending.begin(), pending.end(), 0);
     std::fill(waiting.begin(), waiting.end(), 0);
     int32_t* const at = pos.data() + (up ? 0 : n_inner_);
@@ -694,10 +710,13 @@ void HcltCircuit::build_kl_plan(const LeanTree& t, KlPlan& p, int G) {
       }
       while ((items.size() - first) % ((size_t)D * W)) items.push_back(idle);   // whole rounds of D steps
       walk.steps = (int)((items.size() - first) / W);
+      if (g) longest = std::max(longest, walk.steps);
+      else p.steps += walk.steps;
       walk.n_away = (int)away.size() - walk.away0;
       p.most_away = std::max(p.most_away, walk.n_away);
       items.resize(items.size() + (size_t)D * W, idle);   // idle steps for the requests that run ahead
     }
+    p.steps += longest;
   }
   p.slots = 1;
   while (p.slots < reach + W) p.slots <<= 1;

@@ -799,17 +799,19 @@ def test_row_queries_on_the_block_form_agree_with_the_layer_kernels(gpu, oracle,
 
 
 @pytest.mark.parametrize("reach,most,V,K,C", [(300, 3, 700, 32, 8), (300, 6, 640, 64, 4), (None, 2, 4095, 16, 4), (300, 6, 1400, 16, 8),
-                                              (8, 3, 700, 32, 8), (300, 6, 640, 16, 8)])
+                                              (300, 6, 640, 16, 8), (8, 3, 700, 32, 8), (0, 2, 991, 16, 4)])
 def test_a_row_does_not_depend_on_the_rows_beside_it(gpu, oracle, reach, most, V, K, C):
     """The chains of the row queries walk a tree in eight parts, four or one by the number of rows: the same rows alone and
     among others, in parts and in one (with vectors in LDS, and for the binary tree's wide levels in device memory).  At
     K = 64 nodes have up to six children (in several parts), at K = 16 auxiliary nodes below them; the last two trees, one
-    mostly one chain, the other small for K = 16, are not taken apart."""
+    mostly one chain, one of sixteen chains as long as a part, are not taken apart."""
     torch, P = gpu
     from helpers import make_hclt
     rng = np.random.default_rng(V)
     if reach is None:
         parent = [-1] + [(v - 1) // 2 for v in range(1, V)]
+    elif reach == 0:
+        parent = [-1] + [(v - 1) // 2 if v < 31 else v - 16 for v in range(1, V)]
     else:
         parent, kids = [-1], np.zeros(V, int)
         for v in range(1, V):
@@ -836,7 +838,7 @@ def test_a_row_does_not_depend_on_the_rows_beside_it(gpu, oracle, reach, most, V
         kw = dict(temperature=0.7, noise=z)
         return [P.kld(bpc, a, b), *P.kld_backward(bpc, a, b), P.gumbel_sample_rows(bpc, a, **kw),
                 P.gumbel_sample_backward_rows(bpc, a, g, **kw)]
-    in_parts = reach != 8 and (K, V) != (16, 640)
+    in_parts = reach not in (0, 8)
     whole = queries(0, R)
     assert bpc.size("row_parts") == 1
     for lo, hi, parts in ((0, 40, 4), (65, 70, 8), (3, 4, 8), (0, 32, 8), (0, 33, 4), (0, 64, 4), (0, 65, 1)):
