@@ -16,7 +16,7 @@
 // raises a count from c to c + 1 brings g(c + 1) - g(c) -- so a pair costs ONE pass over its N examples against a C x C
 // table of counters in LDS: an atomic add that returns the old count, and a look-up of its difference; then the table is
 // cleared.  Up to 65535 examples the counters are 16 bits wide and the whole table fits; beyond, they are 32 bits wide
-// and the table is walked in bands of rows.
+// and the table is walked in bands of rows.  Many variables go to another kernel, a pair per lane (mi_lanes.hip.hpp).
 #include "common.hpp"
 #include "chow_liu.hpp"
 #include "stage_kernel.hip.hpp"
@@ -122,17 +122,21 @@ __device__ __forceinline__ void mi_leave_sum(long long acc, long long* red, int 
                        (unsigned)__builtin_amdgcn_readlane((int)(unsigned)x, l));
   if ((t & 63) == 0) red[t >> 6] = sum;
 }
+__device__ __forceinline__ float mi_value(long long sum, int C, double p0, double x0, MiStat su, MiStat sv) {
+  const double tot = ldexp((double)sum, -kMiFrac);
+  double val = tot - su.m - sv.m + (double)C * C * x0;
+  if (p0 > 0.0) val -= p0 * C * (su.l + sv.l);
+  return (float)val;
+}
 template <int T>
 __device__ __forceinline__ void mi_finish_pair(const long long* red, int t, int u, int v, int V, int C, double p0, double x0,
                                                MiStat su, MiStat sv, float* __restrict__ mi) {
   if (t >= 16) return;
   const long long sum = mi_row_sum(t < T / 64 ? red[t] : 0ll);
   if (t == 0) {
-    const double tot = ldexp((double)sum, -kMiFrac);
-    double val = tot - su.m - sv.m + (double)C * C * x0;
-    if (p0 > 0.0) val -= p0 * C * (su.l + sv.l);
-    mi[(size_t)u * V + v] = (float)val;
-    mi[(size_t)v * V + u] = (float)val;
+    const float val = mi_value(sum, C, p0, x0, su, sv);
+    mi[(size_t)u * V + v] = val;
+    mi[(size_t)v * V + u] = val;
   }
 }
 
@@ -386,17 +390,42 @@ void mi_launch(const uint8_t* d_data, int64_t stride_ex, int64_t stride_var, con
   check_launch_c("pairwise_mi");
 }
 
+}  // namespace pcm
+#include "mi_lanes.hip.hpp"
+namespace pcm {
+
 void pairwise_mi(const uint8_t* d_data, int64_t stride_ex, int64_t stride_var, int64_t n_examples, int num_vars,
                  int num_cats, float pseudocount, float* d_mi, hipStream_t stream) {
   const MiShape sh = mi_check(d_data, n_examples, num_vars, num_cats, pseudocount, d_mi);
-  DevBuf<uint8_t> xb;
-  DevBuf<double> stat;
-  DevBuf<long long> g;
-  xb.alloc((size_t)sh.V * sh.Np);
-  stat.alloc((size_t)2 * sh.V);
-  g.alloc((size_t)sh.N + 1);
-  mi_launch(d_data, stride_ex, stride_var, sh, pseudocount, MiScratch{xb.p, stat.p, g.p}, d_mi, stream);
-  PCM_HIP(hipStreamSynchronize(stream));   // the scratch arrays die with this call
+  MiLanesPlan p = mi_lanes_plan(sh);
+  DevBuf<uint8_t> scratch;   // one allocation: each costs more than a small call's kernels
+  size_t bytes = 0;
+  auto take = [&](size_t n) { const size_t at = bytes; bytes += (n + 255) & ~(size_t)255; return at; };
+  const size_t xb = take((size_t)sh.V * sh.Np), stat = take((size_t)2 * sh.V * sizeof(double)),
+               terms = take(((size_t)sh.N + 1) * sizeof(long long));
+  const size_t pairs_bytes = bytes;
+  const size_t xt = take((size_t)p.blocks * sh.N * 128), order = take((size_t)sh.V * p.stride * sizeof(uint32_t)),
+               begin = take((size_t)sh.V * (p.parts + 1) * sizeof(int)),
+               partial = take(p.parts > 1 ? (size_t)sh.V * 64 * p.blocks * sizeof(long long) : 0);
+  if (p.items) {
+    try {
+      scratch.alloc(bytes);
+    } catch (const Error&) {   // a device that is nearly full: the pairs go to workgroups, whose lists of examples are the data
+      (void)hipGetLastError();
+      p.items = 0;
+    }
+  }
+  if (!p.items) scratch.alloc(pairs_bytes);
+  const MiScratch w{scratch.p + xb, reinterpret_cast<double*>(scratch.p + stat), reinterpret_cast<long long*>(scratch.p + terms)};
+  if (p.items)
+    mi_lanes_launch(d_data, stride_ex, stride_var, sh, p, pseudocount, w,
+                    MiLanesScratch{reinterpret_cast<uint32_t*>(scratch.p + xt), reinterpret_cast<uint32_t*>(scratch.p + order),
+                                   reinterpret_cast<int*>(scratch.p + begin),
+                                   reinterpret_cast<unsigned long long*>(scratch.p + partial)},
+                    d_mi, stream);
+  else
+    mi_launch(d_data, stride_ex, stride_var, sh, pseudocount, w, d_mi, stream);
+  PCM_HIP(hipStreamSynchronize(stream));   // the scratch array dies with this call
 }
 
 // One vertex of Prim's algorithm: its row's better links, and the largest of the vertices still outside (those inside

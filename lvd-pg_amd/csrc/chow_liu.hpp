@@ -20,7 +20,7 @@ struct MiShape {
 // Argument checks shared by the entry points; throws pcm::Error.
 MiShape mi_check(const uint8_t* d_data, int64_t n_examples, int num_vars, int num_cats, float pseudocount, const float* d_mi);
 
-// Queues staging, marginals, the count table and the pair kernel on `stream`; allocates nothing and
+// Queues staging, marginals, the count table and the pair kernel (a pair per workgroup) on `stream`; allocates nothing and
 // does not wait.  w.xb holds V * Np bytes, w.stat 2 * V doubles, w.g N 64-bit integers.
 void mi_launch(const uint8_t* d_data, int64_t stride_ex, int64_t stride_var, const MiShape& sh, float pseudocount,
                const MiScratch& w, float* d_mi, hipStream_t stream);

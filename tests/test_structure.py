@@ -157,6 +157,41 @@ def test_pairwise_mi_at_the_edges_of_its_launch_rules(gpu, N, V, C):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,V,C", [(1, 450, 256), (17, 461, 255), (300, 1100, 129), (2000, 1030, 130), (2500, 700, 256),
+                                   (2500, 700, 200), (4096, 640, 256), (4097, 1000, 128), (14000, 1152, 64), (15000, 1100, 33),
+                                   (16000, 1024, 256), (3000, 900, 1), (3000, 900, 100)])
+def test_pairwise_mi_with_a_pair_per_lane(gpu, N, V, C):
+    """Enough variables for the kernel that sorts a variable's examples by category, against the one with a pair per
+    workgroup (`pcm_pairwise_mi_static`, the oracle's tests' kernel): both add the same integers, so the results are the same
+    bits.  Columns whose categories hold 8, 9, 16, 17, 255, 256 and 257 examples (ends of chunks, the last 8-bit count), one
+    that is constant, one with nine tenths of its examples in one category (counts past the terms in LDS); variables past a
+    whole block of 64; categories shared out among several waves and not."""
+    torch, P = gpu
+    from pcmi355._lib import lib, check
+    rng = np.random.default_rng(N + V + C)
+    base = rng.normal(size=(N, 1)) * 0.6 + rng.normal(size=(N, V))
+    x = np.clip((base / 6 + 0.5) * C, 0, C - 1).astype(np.uint8)
+    edges = np.repeat(np.arange(7), [8, 9, 16, 17, 255, 256, 257])[:N] % C
+    for v in (0, 64, V - 1):
+        x[:, v] = C - 1
+        x[:len(edges), v] = edges
+        x[:, v] = x[rng.permutation(N), v]
+    x[:, 5] = C // 2
+    x[rng.random(N) < 0.9, 9] = 0
+    x[rng.random(N) < 0.9, 70] = C - 1
+    d = torch.from_numpy(x).cuda()
+    got = P.pairwise_MI(d, C, 0.1)
+    want = torch.full((V, V), float("nan"), device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    check(lib.pcm_pairwise_mi_static(d.data_ptr(), d.stride(0), d.stride(1), N, V, C, 0.1, want.data_ptr(), stream))
+    assert torch.equal(got, want)
+    wide = torch.zeros((N, V + 3), dtype=torch.uint8, device="cuda")
+    wide[:, 1:V + 1] = d
+    assert torch.equal(P.pairwise_MI(wide[:, 1:V + 1], C, 0.1), got)
+    assert torch.equal(P.pairwise_MI(d.t().contiguous().t(), C, 0.1), got)
+
+
+@pytest.mark.gpu
 def test_learned_tree_and_hclt(gpu):
     torch, P = gpu
     x = _data(2000, 30, 8, 11)
