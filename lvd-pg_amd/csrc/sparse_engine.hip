@@ -1485,7 +1485,7 @@ void SparseCircuit::refresh_group_w(float inv_f) {
 // (sparse_group_walk_kernel) instead of a launch per layer, where a layer's groups are few.  Going up and going down have
 // runs of their own: a node the layer kernels compute going up may take its flow from a group's kernel going down.
 // PCMI355_GROUP_WALK=0 in the environment when the circuit is created keeps the launch per layer (for comparisons).
-void SparseCircuit::build_group_runs() {
+void SparseCircuit::build_group_runs(const std::vector<int32_t>& group_of) {
   group_runs_fwd_.clear();
   group_runs_bwd_.clear();
   n_walk_levels_ = 0;
@@ -1530,7 +1530,161 @@ void SparseCircuit::build_group_runs() {
   // the walk going down takes a run's layers from the last to the first
   for (GroupRun& r : group_runs_bwd_) std::reverse(levels.begin() + r.level0, levels.begin() + r.level0 + r.n_levels);
   for (const GroupRun& r : group_runs_fwd_) n_walk_levels_ += r.n_levels;
+  plan_group_stages(group_of, levels);
   if (!levels.empty()) d_grp_levels_.upload(levels);
+}
+
+// Every run's plans in parts (sparse_group_parts_kernel), by an estimate of their time: a launch, and for the part with the most to do a
+// layer's chain of requests per layer and a compute unit's time per group.  Which cuts between a run's layers, all together
+// or none, is a shortest path over them: for every pair of cuts the connected sets of the groups between them, dealt to the
+// parts largest first.  A plan of one stage and one part is not kept.
+void SparseCircuit::plan_group_stages(const std::vector<int32_t>& group_of, const std::vector<int2>& levels) {
+  group_stages_fwd_.assign(group_runs_fwd_.size(), {});
+  group_stages_bwd_.assign(group_runs_bwd_.size(), {});
+  // the groups whose sums a group's children reach without another group's sums between: whose values it reads going up and
+  // whose flows it may write going down
+  std::vector<std::vector<int32_t>> below(n_groups_);
+  {
+    std::vector<int32_t> seen(fc_.n_nodes(), -1), todo;
+    std::vector<int> lowest(n_groups_, 0);   // nothing below its run's first layer matters
+    for (const std::vector<GroupRun>* runs : {&group_runs_fwd_, &group_runs_bwd_})
+      for (const GroupRun& r : *runs)
+        for (int g = r.group0; g < r.group0 + r.n_groups; ++g)
+          lowest[g] = lowest[g] ? std::min(lowest[g], r.layer_first) : r.layer_first;
+    std::vector<std::vector<int32_t>> sums(n_groups_);
+    for (int64_t n = 0; n < fc_.n_nodes(); ++n)
+      if (group_of[n] >= 0) sums[group_of[n]].push_back((int32_t)n);
+    for (int64_t g = 0; g < n_groups_; ++g) {
+      if (!lowest[g]) continue;
+      todo = sums[g];
+      while (!todo.empty()) {
+        const int32_t n = todo.back();
+        todo.pop_back();
+        for (int32_t e = fc_.node_e0[n]; e < fc_.node_e1[n]; ++e)
+          for (const int32_t c : {fc_.e_prime[e], fc_.e_sub[e]}) {
+            if (c < 0 || seen[c] == (int32_t)g || fc_.layer[c] < lowest[g]) continue;
+            seen[c] = (int32_t)g;
+            if (group_of[c] < 0) todo.push_back(c);
+            else if (below[g].empty() || below[g].back() != group_of[c]) below[g].push_back(group_of[c]);
+          }
+      }
+    }
+  }
+  std::vector<int2> items;
+  auto plan = [&](const GroupRun& r, bool forward, std::array<std::vector<GroupStage>, 3>& out) {
+    // microseconds: a launch; a layer; a group
+    const float kLaunch = 5.f, kLayer = forward ? 1.5f : 2.f, kGroup = forward ? 0.6f : 0.8f;
+    const int n = r.n_levels;
+    std::vector<int2> own(levels.begin() + r.level0, levels.begin() + r.level0 + n);   // from the leaves on
+    if (!forward) std::reverse(own.begin(), own.end());
+    std::vector<int> level_of(r.n_groups);
+    for (int l = 0; l < n; ++l)
+      for (int i = 0; i < own[l].y; ++i) level_of[own[l].x + i] = l;
+    // cuts: every layer's, or fewer where that would take long
+    const int step = std::max(1, (int)std::ceil(std::sqrt((double)n * n * r.n_groups / 4e5)));
+    std::vector<int> cuts;
+    for (int l = 0; l < n; l += step) cuts.push_back(l);
+    cuts.push_back(n);
+    const int n_cuts = (int)cuts.size();
+    struct Set { int first, last, size, root; };
+    std::vector<int> root(r.n_groups);
+    auto find = [&](int g) {
+      while (root[g] != g) g = root[g] = root[root[g]];
+      return g;
+    };
+    // the connected sets of the layers cuts[a] .. cuts[b] - 1, given those up to cuts[b - 1]
+    auto extend = [&](int a, int b) {
+      for (int l = cuts[b - 1]; l < cuts[b]; ++l)
+        for (int g = own[l].x; g < own[l].x + own[l].y; ++g) {
+          root[g] = g;
+          for (const int32_t c : below[r.group0 + g]) {
+            const int o = c - r.group0;
+            if (o < 0 || o >= r.n_groups || level_of[o] < cuts[a]) continue;
+            root[find(o)] = find(g);
+          }
+        }
+    };
+    std::vector<int> at(r.n_groups, -1);
+    auto sets_of = [&](int a, int b) {
+      std::vector<Set> sets;
+      for (int l = cuts[a]; l < cuts[b]; ++l)
+        for (int g = own[l].x; g < own[l].x + own[l].y; ++g) {
+          const int q = find(g);
+          if (at[q] < 0) { at[q] = (int)sets.size(); sets.push_back(Set{l, l, 0, q}); }
+          sets[at[q]].last = l;
+          sets[at[q]].size++;
+        }
+      for (const Set& s : sets) at[s.root] = -1;
+      std::stable_sort(sets.begin(), sets.end(), [](const Set& x, const Set& y) { return x.size > y.size; });
+      return sets;
+    };
+    // the sets' parts, and the time of the longest
+    auto deal = [&](const std::vector<Set>& sets, int most, std::vector<int>* part_of) {
+      const int parts = std::min<int>(most, (int)sets.size());
+      std::vector<float> work(parts, 0.f), span(parts, 0.f);
+      for (size_t i = 0; i < sets.size(); ++i) {
+        int to = 0;
+        for (int p = 1; p < parts; ++p)
+          if (work[p] < work[to]) to = p;
+        work[to] += kGroup * sets[i].size;
+        span[to] = std::max(span[to], kLayer * (sets[i].last - sets[i].first + 1));
+        if (part_of) (*part_of)[i] = to;
+      }
+      float longest = 0.f;
+      for (int p = 0; p < parts; ++p) longest = std::max(longest, work[p] + span[p]);
+      return kLaunch + longest;
+    };
+    constexpr int kPlans = 3;
+    std::vector<std::array<float, kPlans>> best(n_cuts);
+    std::vector<std::array<int, kPlans>> from(n_cuts);
+    for (int b = 0; b < n_cuts; ++b) best[b].fill(b ? INFINITY : 0.f);
+    for (int a = 0; a + 1 < n_cuts; ++a)
+      for (int b = a + 1; b < n_cuts; ++b) {
+        extend(a, b);
+        const std::vector<Set> sets = sets_of(a, b);
+        for (int k = 0; k < kPlans; ++k) {
+          const float t = best[a][k] + deal(sets, kGroupParts[k], nullptr);
+          if (t < best[b][k]) { best[b][k] = t; from[b][k] = a; }
+        }
+      }
+    for (int k = 0; k < kPlans; ++k) {
+      std::vector<std::pair<int, int>> stages;
+      for (int b = n_cuts - 1; b > 0; b = from[b][k]) stages.emplace_back(from[b][k], b);
+      if (forward) std::reverse(stages.begin(), stages.end());
+      std::vector<GroupStage> kept;
+      for (const auto& [a, b] : stages) {
+        for (int c = a + 1; c <= b; ++c) extend(a, c);
+        const std::vector<Set> sets = sets_of(a, b);
+        std::vector<int> part_of(sets.size());
+        deal(sets, kGroupParts[k], &part_of);
+        const int parts = std::min<int>(kGroupParts[k], (int)sets.size()), depth = cuts[b] - cuts[a];
+        for (size_t i = 0; i < sets.size(); ++i) at[sets[i].root] = part_of[i];
+        // a part's groups of a layer go round its waves, each layer starting where the one before ended
+        std::vector<std::vector<int2>> own_items(parts * kPartWaves);
+        for (int p = 0; p < parts; ++p) {
+          int wave = 0;
+          for (int i = 0; i < depth; ++i) {
+            const int l = forward ? cuts[a] + i : cuts[b] - 1 - i;
+            for (int g = own[l].x; g < own[l].x + own[l].y; ++g)
+              if (at[find(g)] == p) own_items[p * kPartWaves + wave++ % kPartWaves].push_back(int2{g, i});
+          }
+        }
+        size_t most = 0;
+        for (const auto& v : own_items) most = std::max(most, v.size());
+        const GroupStage st{(int)items.size(), (int)most, depth, parts};
+        for (auto& v : own_items) {
+          v.resize(most, int2{-1, 0});
+          items.insert(items.end(), v.begin(), v.end());
+        }
+        for (const Set& s : sets) at[s.root] = -1;
+        kept.push_back(st);
+      }
+      if (kept.size() > 1 || kept[0].parts > 1) out[k] = kept;
+    }
+  };
+  for (size_t i = 0; i < group_runs_fwd_.size(); ++i) plan(group_runs_fwd_[i], true, group_stages_fwd_[i]);
+  for (size_t i = 0; i < group_runs_bwd_.size(); ++i) plan(group_runs_bwd_[i], false, group_stages_bwd_[i]);
+  if (!items.empty()) d_grp_items_.upload(items);
 }
 
 // a run goes as one walk launch if its layers' groups are few: each slice of 16 examples is one workgroup whose waves
@@ -1539,27 +1693,58 @@ static bool run_walks(int max_count, int Bp) {
   return max_count <= 32 && (int64_t)max_count * (Bp / 16) <= 4096;
 }
 
-bool SparseCircuit::launch_group_walk(const GroupRun& r, bool forward, int Bp, int batch, bool tempered) {
-  if (!run_walks(r.max_count, Bp)) return false;
-  PCM_GROUP_DEV(g, batch, Bp);
-  if (tempered) { g.inv_f = 1.f / flow_scale; g.norm = d_norm_.p; g.norm_row = -1; }
-  GroupWalk w;
-  w.levels = d_grp_levels_.p + r.level0;
-  w.n_levels = r.n_levels;
-  w.base = GroupBase{r.group0, r.pnode0, r.pslot0, r.pw0};
-  const dim3 grid(Bp / 16);
+static void run_group_walk(const GroupDev& g, const GroupWalk& w, int gt, bool forward, dim3 grid, hipStream_t stream) {
   // waves per workgroup: as many as the kernel's registers allow (going down a 32 x 32 group takes 128 and more)
 #define PCM_WALK(GT_, WVF_, WVB_)                                                                                              \
   do {                                                                                                                         \
     if (forward) hipLaunchKernelGGL((sparse_group_walk_kernel<GT_, GT_, WVF_, true>), grid, dim3(WVF_ * 64), 0, stream, g, w);  \
     else hipLaunchKernelGGL((sparse_group_walk_kernel<GT_, GT_, WVB_, false>), grid, dim3(WVB_ * 64), 0, stream, g, w);         \
   } while (0)
-  switch (r.gt) {
+  switch (gt) {
     case 1: PCM_WALK(1, 16, 16); break;
     case 2: PCM_WALK(2, 16, 8); break;
     default: PCM_WALK(4, 4, 4); break;
   }
 #undef PCM_WALK
+}
+
+bool SparseCircuit::launch_group_walk(int run, bool forward, int Bp, int batch, bool tempered) {
+  const GroupRun& r = (forward ? group_runs_fwd_ : group_runs_bwd_)[run];
+  if (!run_walks(r.max_count, Bp)) return false;
+  PCM_GROUP_DEV(g, batch, Bp);
+  if (tempered) { g.inv_f = 1.f / flow_scale; g.norm = d_norm_.p; g.norm_row = -1; }
+  // In parts where they find compute units of their own and every array is below 2 GiB (GroupBuffers).  192 variables, K = 32,
+  // 128 heads, 60 % of the edges, an epoch of 16 batches: 5.45 -> 4.25 ms at 512 examples (25 layers up 96 -> 53 us a batch,
+  // down 100 -> 54), 4.94 -> 3.75 at 64; 48 variables and 1024 examples, 2.67 -> 2.60.
+  const int slices = Bp / 16;
+  const size_t gib2 = (size_t)1 << 31;
+  const bool small = g.flow_bytes && d_grp_rows_.n * (size_t)Bp * 4 < gib2 && (size_t)n_group_elems_ * 4 < gib2 &&
+                     d_grp_copies_.n * sizeof(int4) < gib2;
+  const std::vector<GroupStage>* stages = nullptr;
+  walk_parts_ = 1;
+  for (int k = 0; k < 3; ++k)
+    if (small && slices * kGroupParts[k] <= 256) stages = &(forward ? group_stages_fwd_ : group_stages_bwd_)[run][k];
+  if (stages && !stages->empty()) {
+    for (const GroupStage& st : *stages) {
+      walk_parts_ = std::max(walk_parts_, st.parts);
+      const GroupParts w{d_grp_items_.p + st.item0, st.n_items, st.n_levels, GroupBase{r.group0, r.pnode0, r.pslot0, r.pw0}};
+      const dim3 grid(slices, st.parts), block(kPartWaves * 64);
+#define PCM_PARTS(GT_)                                                                                          \
+  do {                                                                                                          \
+    if (forward) hipLaunchKernelGGL((sparse_group_parts_kernel<GT_, GT_, true>), grid, block, 0, stream, g, w);  \
+    else hipLaunchKernelGGL((sparse_group_parts_kernel<GT_, GT_, false>), grid, block, 0, stream, g, w);         \
+  } while (0)
+      switch (r.gt) {
+        case 1: PCM_PARTS(1); break;
+        case 2: PCM_PARTS(2); break;
+        default: PCM_PARTS(4); break;
+      }
+#undef PCM_PARTS
+    }
+  } else {
+    run_group_walk(g, GroupWalk{d_grp_levels_.p + r.level0, r.n_levels, GroupBase{r.group0, r.pnode0, r.pslot0, r.pw0}},
+                   r.gt, forward, dim3(slices), stream);
+  }
   return true;
 }
 
@@ -1785,7 +1970,7 @@ SparseCircuit::SparseCircuit(FlatCircuit fc) : fc_(std::move(fc)) {
     d_bwd_rec_.upload(br);
     d_bwd_alias_.upload(ar);
   }
-  build_group_runs();
+  build_group_runs(group_of);
   // normalisation groups over the sum parameters
   std::vector<int32_t> gp(1, 0), p2e;
   for (int64_t s : fc_.pargroup_sizes) gp.push_back(gp.back() + (int32_t)s);
@@ -1816,7 +2001,7 @@ int64_t SparseCircuit::size(int what) const {
     case 16: return n_groups_;
     case 17: return n_layer_nodes_;
     case 18: return n_walk_levels_;
-    case 19: return 0;
+    case 19: return walk_parts_;
     case 20: return 0;
     default: fail(PCM_ERR_ARG, "unknown size selector %d", what);
   }
@@ -1959,7 +2144,7 @@ void SparseCircuit::run_forward(const BatchRef* b, const SoftRef* s) {
     const int n0 = fwd_layer0_[l], cnt = fwd_layer0_[l + 1] - n0;
     while (next_run < group_runs_fwd_.size() && group_runs_fwd_[next_run].layer_first < l) ++next_run;
     if (next_run < group_runs_fwd_.size() && group_runs_fwd_[next_run].layer_first == l &&
-        launch_group_walk(group_runs_fwd_[next_run], true, Bp, batch, false)) {
+        launch_group_walk((int)next_run, true, Bp, batch, false)) {
       l = group_runs_fwd_[next_run].layer_last;   // the run's layers hold nothing but these groups
       continue;
     }
@@ -2077,7 +2262,7 @@ void SparseCircuit::run_flows(int batch, const SoftRef* soft, float rate, const 
   for (int l = n_layers_ - 1; l >= 0; --l) {
     while (next_run >= 0 && group_runs_bwd_[next_run].layer_last > l) --next_run;
     if (next_run >= 0 && group_runs_bwd_[next_run].layer_last == l &&
-        launch_group_walk(group_runs_bwd_[next_run], false, Bp, batch, tempered)) {
+        launch_group_walk(next_run, false, Bp, batch, tempered)) {
       l = group_runs_bwd_[next_run].layer_first;   // (the loop's --l moves on below the run)
       continue;
     }

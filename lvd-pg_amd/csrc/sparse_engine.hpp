@@ -7,6 +7,8 @@
 // its result once -- no atomics on node values or flows.
 #pragma once
 
+#include <array>
+
 #include <memory>
 
 #include "common.hpp"
@@ -128,9 +130,16 @@ class SparseCircuit : public pcm_circuit {
   struct GroupRun { int layer_first, layer_last, gt, ct, group0, n_groups; int32_t pnode0, pslot0; int64_t pw0; int level0, n_levels, max_count; };
   std::vector<GroupRun> group_runs_fwd_, group_runs_bwd_;
   DevBuf<int2> d_grp_levels_;
+  // a run in parts (sparse_group_parts_kernel): its stages in the order of the walk, {first of its items in d_grp_items_, ...}
+  struct GroupStage { int item0, n_items, n_levels, parts; };
+  static constexpr int kGroupParts[3] = {4, 8, 16};   // most parts a plan has
+  std::vector<std::array<std::vector<GroupStage>, 3>> group_stages_fwd_, group_stages_bwd_;   // per run, per entry of kGroupParts
+  DevBuf<int2> d_grp_items_;
+  int walk_parts_ = 0;                        // most parts of the last walk (0: none yet)
   int64_t n_walk_levels_ = 0;                 // layers of groups inside forward runs
-  void build_group_runs();
-  bool launch_group_walk(const GroupRun& r, bool forward, int Bp, int batch, bool tempered);
+  void build_group_runs(const std::vector<int32_t>& group_of);
+  void plan_group_stages(const std::vector<int32_t>& group_of, const std::vector<int2>& levels);
+  bool launch_group_walk(int run, bool forward, int Bp, int batch, bool tempered);
   std::vector<GroupLaunch> group_stat_launches_;   // per shape: ranges of d_grp_order_ (layer and bases unused)
   std::vector<int> fwd_layer0_;               // ranges of d_fwd_rec_ per layer: the nodes no group computes
   bool layer0_inputs_only_ = true;            // the first layer holds input nodes and nothing else

@@ -118,15 +118,6 @@ __device__ __forceinline__ float group_exp_times(float x, float y) {
 
 __device__ __forceinline__ int guni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// X of a child for the example in column `col`: the value of its prime (the first three rows: the prime itself and
-// two rows of zeros, or the factors of a product the group computes) plus its sub's (the last row; zeros: none)
-__device__ __forceinline__ float group_prime_value(const GroupDev& d, const int4 rw, int64_t col) {
-  return (d.mars[(int64_t)rw.x * d.Bp + col] + d.mars[(int64_t)rw.y * d.Bp + col]) + d.mars[(int64_t)rw.z * d.Bp + col];
-}
-__device__ __forceinline__ float group_x(const GroupDev& d, const int4 rw, int64_t col) {
-  return group_prime_value(d, rw, col) + d.mars[(int64_t)rw.w * d.Bp + col];
-}
-
 // maximum over the four lanes that hold one example (lane, lane ^ 16, lane ^ 32, lane ^ 48)
 __device__ __forceinline__ float group_max4(float v) {
   const int a = __builtin_bit_cast(int, v);
@@ -136,6 +127,71 @@ __device__ __forceinline__ float group_max4(float v) {
   const auto r32 = __builtin_amdgcn_permlane32_swap(b, b, false, false);
   return fmaxf(__builtin_bit_cast(float, (int)r32[0]), __builtin_bit_cast(float, (int)r32[1]));
 }
+
+// How the group kernels reach memory: `at` is the same for a wave, `own` a lane's, `row` a row of values or flows of which
+// the lane's example is taken (row -1: a store goes nowhere).  By pointers, whatever the arrays' sizes:
+struct GroupPointers {
+  const GroupDev& d;
+  int64_t col;
+  __device__ __forceinline__ GroupPointers(const GroupDev& dev, int slice, int lane) : d(dev), col((int64_t)slice * 16 + (lane & 15)) {}
+  __device__ __forceinline__ int4 rows(int at, int own) const { return d.rows[(int64_t)at + own]; }
+  __device__ __forceinline__ int own(int at, int own_) const { return d.own[(int64_t)at + own_]; }
+  __device__ __forceinline__ int node(int at, int own) const { return d.node[(int64_t)at + own]; }
+  __device__ __forceinline__ int4 node4(int at, int own) const { return *reinterpret_cast<const int4*>(d.node + at + own); }
+  __device__ __forceinline__ int4 copies(int64_t at, int own) const { return d.copies[at + own]; }
+  __device__ __forceinline__ float wf(int64_t at, int own) const { return d.wf[at + own]; }
+  __device__ __forceinline__ float wb(int64_t at, int own) const { return d.wb[at + own]; }
+  __device__ __forceinline__ float m(int group) const { return d.m[(int64_t)group * d.Bp + col]; }
+  __device__ __forceinline__ void put_m(int group, float v) const { d.m[(int64_t)group * d.Bp + col] = v; }
+  __device__ __forceinline__ float xm(int at, int own) const { return d.xm[((int64_t)at + own) * d.Bp + col]; }
+  __device__ __forceinline__ void put_xm(int at, int own, float v) const { d.xm[((int64_t)at + own) * d.Bp + col] = v; }
+  __device__ __forceinline__ float value(int row) const { return d.mars[(int64_t)row * d.Bp + col]; }
+  __device__ __forceinline__ void put_value(int row, float v) const { if (row >= 0) d.mars[(int64_t)row * d.Bp + col] = v; }
+  __device__ __forceinline__ float flow(int row) const { return d.flows[(int64_t)row * d.Bp + col]; }
+  __device__ __forceinline__ float norm(int row) const { return d.norm[(int64_t)row * d.Bp + col]; }
+};
+// ... and by buffer descriptors where every array stays below 2 GiB and a row below 64 KB: a row's address is one
+// 24-bit multiply-add, the tables' offsets are in the requests.
+struct GroupBuffers {
+  __amdgpu_buffer_rsrc_t r_rows, r_own, r_node, r_copies, r_wf, r_wb, r_m, r_xm, r_mars, r_flows, r_norm;
+  int bp4, col4;
+  template <typename T>
+  __device__ __forceinline__ static __amdgpu_buffer_rsrc_t all(const T* p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), 0, 0x7fffffff, 0x00020000);
+  }
+  __device__ __forceinline__ GroupBuffers(const GroupDev& d, int slice, int lane)
+      : r_rows(all(d.rows)), r_own(all(d.own)), r_node(all(d.node)), r_copies(all(d.copies)), r_wf(all(d.wf)), r_wb(all(d.wb)),
+        r_m(all(d.m)), r_xm(all(d.xm)), r_mars(all(d.mars)), r_flows(all(d.flows)), r_norm(all(d.norm)), bp4(d.Bp * 4),
+        col4(slice * 64 + (lane & 15) * 4) {}
+  __device__ __forceinline__ static float one(__amdgpu_buffer_rsrc_t r, int own, int at) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, own, at, 0));
+  }
+  __device__ __forceinline__ static int4 four(__amdgpu_buffer_rsrc_t r, int own, int at) {
+    return __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(r, own, at, 0));
+  }
+  __device__ __forceinline__ int at_row(int row) const { return (int)__umul24(row, bp4) + col4; }
+  __device__ __forceinline__ int4 rows(int at, int own) const { return four(r_rows, 16 * own, 16 * at); }
+  __device__ __forceinline__ int own(int at, int own_) const { return (int)__builtin_amdgcn_raw_buffer_load_b32(r_own, 4 * own_, 4 * at, 0); }
+  __device__ __forceinline__ int node(int at, int own) const { return (int)__builtin_amdgcn_raw_buffer_load_b32(r_node, 4 * own, 4 * at, 0); }
+  __device__ __forceinline__ int4 node4(int at, int own) const { return four(r_node, 4 * own, 4 * at); }
+  __device__ __forceinline__ int4 copies(int64_t at, int own) const { return four(r_copies, 16 * own, (int)(16 * at)); }
+  __device__ __forceinline__ float wf(int64_t at, int own) const { return one(r_wf, 4 * own, (int)(4 * at)); }
+  __device__ __forceinline__ float wb(int64_t at, int own) const { return one(r_wb, 4 * own, (int)(4 * at)); }
+  __device__ __forceinline__ float m(int group) const { return one(r_m, col4, group * bp4); }
+  __device__ __forceinline__ void put_m(int group, float v) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r_m, col4, group * bp4, 0);
+  }
+  __device__ __forceinline__ float xm(int at, int own) const { return one(r_xm, own * bp4 + col4, at * bp4); }
+  __device__ __forceinline__ void put_xm(int at, int own, float v) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r_xm, own * bp4 + col4, at * bp4, 0);
+  }
+  __device__ __forceinline__ float value(int row) const { return one(r_mars, at_row(row), 0); }
+  __device__ __forceinline__ void put_value(int row, float v) const {   // (past the descriptor's end: nowhere)
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r_mars, row >= 0 ? at_row(row) : -1, 0, 0);
+  }
+  __device__ __forceinline__ float flow(int row) const { return one(r_flows, at_row(row), 0); }
+  __device__ __forceinline__ float norm(int row) const { return one(r_norm, at_row(row), 0); }
+};
 
 // Sums far below their group's maximum.  E = exp(X - m) leaves float's range 87 below m, and a sum without a share in
 // the children near m -- masked groups (build_groups) have many -- may own nothing above that.  A sum that comes out
@@ -209,76 +265,130 @@ __device__ __forceinline__ void group_low_sums(const GroupDev& d, const float* x
 // before anything of it is used and no branch around a load: a layer's launch lasts as long as its longest chain of
 // requests.  The maximum goes to d.m for the backward kernels.
 template <int GT, int CT>
-__device__ __forceinline__ void group_forward_body(const GroupDev& d, const GroupBase& base, int bx, int lane, int slice) {
-  constexpr int NK = CT * 4, Gp = GT * 16, Cp = CT * 16;
-  constexpr bool kPre = GT * NK <= 64;   // W in registers before the rows arrive
-  const int group = base.group0 + bx;
-  const int lo = lane & 15, hi = lane >> 4;
-  const int64_t col = (int64_t)slice * 16 + lo;
-  const int4* rows = d.rows + base.pslot0 + (int64_t)bx * Cp;
-  const int32_t* owns = d.own + base.pslot0 + (int64_t)bx * Cp;
-  const int32_t* node = d.node + base.pnode0 + (int64_t)bx * Gp;
-  const float* wg = d.wf + base.pw0 + (int64_t)bx * Gp * Cp + lane;
-  int4 rw[NK];
+struct GroupUpTables {   // what the forward kernel reads of a group in its first round
+  static constexpr int NK = CT * 4;
+  static constexpr bool kPre = GT * NK <= 64;   // W in registers before the rows arrive
+  int4 rw[NK], nd4[GT];
   int own[NK];
-#pragma unroll
-  for (int q = 0; q < NK; ++q) { rw[q] = rows[4 * q + hi]; own[q] = owns[4 * q + hi]; }
   float a[kPre ? GT : 1][kPre ? NK : 1];
-  if constexpr (kPre) {
-#pragma unroll
-    for (int gt = 0; gt < GT; ++gt)
-#pragma unroll
-      for (int q = 0; q < NK; ++q) a[gt][q] = wg[(gt * NK + q) * 64];
-  }
-  int4 nd4[GT];   // (the four sums of a lane's output rows are neighbours in the table: one request per tile)
-#pragma unroll
-  for (int gt = 0; gt < GT; ++gt) nd4[gt] = *reinterpret_cast<const int4*>(node + gt * 16 + 4 * hi);
-  float x[NK], pv[NK];
-#pragma unroll
-  for (int q = 0; q < NK; ++q) {
-    pv[q] = group_prime_value(d, rw[q], col);
-    x[q] = pv[q] + d.mars[(int64_t)rw[q].w * d.Bp + col];
-  }
-#pragma unroll
-  for (int q = 0; q < NK; ++q) if (own[q] == -2) x[q] = -INFINITY;
-  float mx = x[0];
-#pragma unroll
-  for (int q = 1; q < NK; ++q) mx = fmaxf(mx, x[q]);
-  mx = group_max4(mx);
-  if (!(mx > -INFINITY)) mx = 0.f;   // every child impossible: E = 0, the sums come out as -inf
-  float* xm = d.xm + (base.pslot0 + (int64_t)bx * Cp) * d.Bp + col;
-#pragma unroll
-  for (int q = 0; q < NK; ++q) {
-    if (own[q] >= 0) d.mars[(int64_t)own[q] * d.Bp + col] = pv[q];
-    const float xs = x[q] - mx;   // (-inf stays -inf)
-    xm[(int64_t)(4 * q + hi) * d.Bp] = xs;
-    x[q] = __expf(xs);
-  }
-  if (hi == 0) d.m[(int64_t)group * d.Bp + col] = mx;
-#pragma unroll
-  for (int gt = 0; gt < GT; ++gt) {
-    g4f acc = {0.f, 0.f, 0.f, 0.f};
+  template <typename M>
+  __device__ __forceinline__ void load(const M& mem, const GroupBase& base, int bx, int lane) {
+    constexpr int Gp = GT * 16, Cp = CT * 16;
+    const int hi = lane >> 4;
 #pragma unroll
     for (int q = 0; q < NK; ++q) {
-      float av;
-      if constexpr (kPre) av = a[gt][q];
-      else av = wg[(gt * NK + q) * 64];
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, x[q], acc, 0, 0, 0);
+      rw[q] = mem.rows(base.pslot0 + bx * Cp + 4 * q, hi);
+      own[q] = mem.own(base.pslot0 + bx * Cp + 4 * q, hi);
     }
-    const int nd[4] = {nd4[gt].x, nd4[gt].y, nd4[gt].z, nd4[gt].w};
-    float val[4];
-    bool low[4];
+    if constexpr (kPre) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      val[i] = mx + __logf(acc[i]);
-      low[i] = nd[i] >= 0 && !(acc[i] >= kLowSum);
+      for (int gt = 0; gt < GT; ++gt)
+#pragma unroll
+        for (int q = 0; q < NK; ++q) a[gt][q] = mem.wf(base.pw0 + (int64_t)bx * Gp * Cp + (gt * NK + q) * 64, lane);
     }
-    if (__any(low[0] | low[1] | low[2] | low[3]))
-      group_low_sums<NK>(d, xm, hi, wg + gt * NK * 64, d.edge + base.pw0 + ((int64_t)bx * Gp + gt * 16) * Cp, mx, low, val);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (nd[i] >= 0) d.mars[(int64_t)nd[i] * d.Bp + col] = val[i];
+#pragma unroll   // (the four sums of a lane's output rows are neighbours in the table: one request per tile)
+    for (int gt = 0; gt < GT; ++gt) nd4[gt] = mem.node4(base.pnode0 + bx * Gp + gt * 16, 4 * hi);
   }
+};
+// A group going up, in two steps: the sums' values, which the groups above wait for, and what later passes read.
+template <int GT, int CT>
+struct GroupUp {
+  static constexpr int NK = CT * 4;
+  float xs[NK], pv[NK], mx;   // X - m and the value of the prime, per child; m
+  bool kept;                  // X - m is in memory
+  template <typename M>
+  __device__ __forceinline__ void keep_xm(const M& mem, const GroupBase& base, int bx, int lane) {
+#pragma unroll
+    for (int q = 0; q < NK; ++q) mem.put_xm(base.pslot0 + bx * CT * 16 + 4 * q, lane >> 4, xs[q]);
+  }
+  // X of a child: the value of its prime (the first three rows: the prime itself and two rows of zeros, or the factors of a
+  // product the group computes) plus its sub's (the last row; zeros: none).  kAll: what later passes read is stored on the
+  // way, where it takes the fewest registers, and there is no rest.
+  template <bool kAll, typename M>
+  __device__ __forceinline__ void values(const GroupDev& d, const GroupBase& base, int bx, int lane, int slice, const M& mem,
+                                         const GroupUpTables<GT, CT>& tb) {
+    constexpr int Gp = GT * 16, Cp = CT * 16;
+    constexpr bool kPre = GroupUpTables<GT, CT>::kPre;
+    const int lo = lane & 15, hi = lane >> 4;
+    float e[NK];
+#pragma unroll
+    for (int q = 0; q < NK; ++q) {
+      pv[q] = (mem.value(tb.rw[q].x) + mem.value(tb.rw[q].y)) + mem.value(tb.rw[q].z);
+      xs[q] = pv[q] + mem.value(tb.rw[q].w);
+    }
+#pragma unroll
+    for (int q = 0; q < NK; ++q) if (tb.own[q] == -2) xs[q] = -INFINITY;
+    mx = xs[0];
+#pragma unroll
+    for (int q = 1; q < NK; ++q) mx = fmaxf(mx, xs[q]);
+    mx = group_max4(mx);
+    if (!(mx > -INFINITY)) mx = 0.f;   // every child impossible: E = 0, the sums come out as -inf
+#pragma unroll
+    for (int q = 0; q < NK; ++q) {
+      xs[q] -= mx;   // (-inf stays -inf)
+      e[q] = __expf(xs[q]);
+    }
+    kept = false;
+    if constexpr (kAll) {
+      rest(base, bx, lane, mem, tb);
+      kept = true;
+    }
+    float val[GT][4];
+    bool low[GT][4], any = false;
+    g4f acc[GT];
+#pragma unroll
+    for (int gt = 0; gt < GT; ++gt) acc[gt] = g4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < NK; ++q)
+#pragma unroll
+      for (int gt = 0; gt < GT; ++gt) {
+        float av;
+        if constexpr (kPre) av = tb.a[gt][q];
+        else av = mem.wf(base.pw0 + (int64_t)bx * Gp * Cp + (gt * NK + q) * 64, lane);
+        acc[gt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, e[q], acc[gt], 0, 0, 0);
+      }
+#pragma unroll
+    for (int gt = 0; gt < GT; ++gt) {
+      const int nd[4] = {tb.nd4[gt].x, tb.nd4[gt].y, tb.nd4[gt].z, tb.nd4[gt].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        val[gt][i] = mx + __logf(acc[gt][i]);
+        low[gt][i] = nd[i] >= 0 && !(acc[gt][i] >= kLowSum);
+        any |= low[gt][i];
+      }
+    }
+    if (__any(any)) {
+      if (!kept) keep_xm(mem, base, bx, lane);
+      kept = true;
+      const float* xm = d.xm + (base.pslot0 + (int64_t)bx * Cp) * d.Bp + (int64_t)slice * 16 + lo;
+      const float* wg = d.wf + base.pw0 + (int64_t)bx * Gp * Cp + lane;
+#pragma unroll
+      for (int gt = 0; gt < GT; ++gt)
+        if (__any(low[gt][0] | low[gt][1] | low[gt][2] | low[gt][3]))
+          group_low_sums<NK>(d, xm, hi, wg + gt * NK * 64, d.edge + base.pw0 + ((int64_t)bx * Gp + gt * 16) * Cp, mx, low[gt], val[gt]);
+    }
+#pragma unroll
+    for (int gt = 0; gt < GT; ++gt) {
+      const int nd[4] = {tb.nd4[gt].x, tb.nd4[gt].y, tb.nd4[gt].z, tb.nd4[gt].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mem.put_value(nd[i], val[gt][i]);
+    }
+  }
+  template <typename M>
+  __device__ __forceinline__ void rest(const GroupBase& base, int bx, int lane, const M& mem, const GroupUpTables<GT, CT>& tb) {
+    if (!kept) keep_xm(mem, base, bx, lane);
+#pragma unroll
+    for (int q = 0; q < NK; ++q) mem.put_value(tb.own[q], pv[q]);
+    if ((lane >> 4) == 0) mem.put_m(base.group0 + bx, mx);
+  }
+};
+template <int GT, int CT>
+__device__ __forceinline__ void group_forward_body(const GroupDev& d, const GroupBase& base, int bx, int lane, int slice) {
+  const GroupPointers mem(d, slice, lane);
+  GroupUpTables<GT, CT> tb;
+  tb.load(mem, base, bx, lane);
+  GroupUp<GT, CT> up;
+  up.template values<true>(d, base, bx, lane, slice, mem, tb);
 }
 
 template <int GT, int CT>
@@ -331,56 +441,81 @@ __device__ __forceinline__ void group_shares_by_edge(const GroupDev& d, const in
 // examples) as going up: R of the sums g = 4 k + hi is the B operand of k-step k as it is loaded.  The same two
 // rounds of requests where the registers hold a group's W and row numbers (kPre); 16 children at a time otherwise.
 template <int GT, int CT>
-__device__ __forceinline__ void group_backward_body(const GroupDev& d, const GroupBase& base, int bx, int lane, int slice) {
-  constexpr int NG = GT * 4, Gp = GT * 16, Cp = CT * 16;
-  constexpr bool kPre = CT <= 2 && GT * CT <= 16;
-  constexpr int CL = kPre ? CT : 1;
-  const int group = base.group0 + bx;
-  const int lo = lane & 15, hi = lane >> 4;
-  const int64_t col = (int64_t)slice * 16 + lo;
-  const float* xm = d.xm + (base.pslot0 + (int64_t)bx * Cp) * d.Bp + col;
-  const int4* copies = d.copies + 2 * (base.pslot0 + (int64_t)bx * Cp);
-  const int32_t* node = d.node + base.pnode0 + (int64_t)bx * Gp;
-  const float* wg = d.wb + base.pw0 + (int64_t)bx * Gp * Cp + lane;
-  const float mb = d.m[(int64_t)group * d.Bp + col];
+struct GroupDownTables {   // what the backward kernel reads of a group without waiting for anything
+  static constexpr int NG = GT * 4;
+  static constexpr bool kPre = CT <= 2 && GT * CT <= 16;
+  static constexpr int CL = kPre ? CT : 1;
   int nd[NG];
-#pragma unroll
-  for (int k = 0; k < NG; ++k) nd[k] = node[4 * k + hi];
   int4 cpa[CL][4], cpb[CL][4];
-  float a[CL][NG], e[CL][4];
-  auto numbers = [&](int ct, int s) {   // row numbers and W for the children 16 ct + 4 hi + i
+  float a[CL][NG], e[CL][4], mb, v[NG];
+  template <typename M>   // row numbers and W for the children 16 ct + 4 hi + i
+  __device__ __forceinline__ void numbers(const M& mem, const GroupBase& base, int bx, int lane, int ct, int s) {
+    constexpr int Gp = GT * 16, Cp = CT * 16;
+    const int hi = lane >> 4;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int c = ct * 16 + 4 * hi + i;
-      cpa[s][i] = copies[2 * c];
-      cpb[s][i] = copies[2 * c + 1];
+      const int64_t at = 2 * (base.pslot0 + (int64_t)bx * Cp + ct * 16);
+      cpa[s][i] = mem.copies(at + 2 * i, 8 * hi);
+      cpb[s][i] = mem.copies(at + 2 * i + 1, 8 * hi);
     }
 #pragma unroll
-    for (int k = 0; k < NG; ++k) a[s][k] = wg[(ct * NG + k) * 64];
-  };
-  auto values = [&](int ct, int s) {   // X - m as the forward kernel left it (a child that is not there: -inf)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) e[s][i] = xm[(int64_t)(ct * 16 + 4 * hi + i) * d.Bp];
-  };
-  if constexpr (kPre) {
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) numbers(ct, ct);
+    for (int k = 0; k < NG; ++k) a[s][k] = mem.wb(base.pw0 + (int64_t)bx * Gp * Cp + (ct * NG + k) * 64, lane);
   }
+  template <typename M>
+  __device__ __forceinline__ void load(const M& mem, const GroupBase& base, int bx, int lane) {
+    mb = mem.m(base.group0 + bx);
+#pragma unroll
+    for (int k = 0; k < NG; ++k) nd[k] = mem.node(base.pnode0 + bx * GT * 16 + 4 * k, lane >> 4);
+    if constexpr (kPre) {
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) numbers(mem, base, bx, lane, ct, ct);
+    }
+  }
+  template <typename M>   // X - m as the forward kernel left it (a child that is not there: -inf)
+  __device__ __forceinline__ void children(const M& mem, const GroupBase& base, int bx, int lane, int ct, int s) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) e[s][i] = mem.xm(base.pslot0 + bx * CT * 16 + ct * 16 + i, 4 * (lane >> 4));
+  }
+  template <typename M>   // the sums' values, and the children's where the registers hold them
+  __device__ __forceinline__ void values(const M& mem, const GroupBase& base, int bx, int lane) {
+#pragma unroll
+    for (int k = 0; k < NG; ++k) v[k] = mem.value(max(nd[k], 0));
+    if constexpr (kPre) {
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) children(mem, base, bx, lane, ct, ct);
+    }
+  }
+};
+template <int GT, int CT, typename M>
+__device__ __forceinline__ void group_backward_body(const GroupDev& d, const GroupBase& base, int bx, int lane, int slice,
+                                                    const M& mem, GroupDownTables<GT, CT>& tb) {
+  constexpr int NG = GT * 4, Gp = GT * 16, Cp = CT * 16;
+  constexpr bool kPre = GroupDownTables<GT, CT>::kPre;
+  constexpr int CL = GroupDownTables<GT, CT>::CL;
+  const int lo = lane & 15, hi = lane >> 4;
+  const int64_t col = (int64_t)slice * 16 + lo;
+  const int32_t* node = d.node + base.pnode0 + (int64_t)bx * Gp;
+  const float mb = tb.mb;
+  const int (&nd)[NG] = tb.nd;
+  const auto& cpa = tb.cpa;
+  const auto& cpb = tb.cpb;
+  const auto& a = tb.a;
+  const auto& e = tb.e;
+  const auto& v = tb.v;
   float rv[NG];
   bool high = false, middle = false;
   {   // R = F / S = F * exp(m - value): no flow stays no flow where the value is -inf.  (All rows requested, then used:
       // written as one loop the compiler waits for every sum's rows in turn.)
-    float f[NG], v[NG], nv[NG];
+    float f[NG], nv[NG];
 #pragma unroll
     for (int k = 0; k < NG; ++k) {
-      const int64_t n = nd[k] < 0 ? 0 : nd[k];
-      f[k] = d.flows[n * d.Bp + col];
-      v[k] = d.mars[n * d.Bp + col];
+      const int n = max(nd[k], 0);
+      f[k] = mem.flow(n);
       nv[k] = 0.f;
     }
     if (d.norm_row < 0) {   // tempered flows only (the same for every lane: a branch around requests, none around a wait)
 #pragma unroll
-      for (int k = 0; k < NG; ++k) nv[k] = d.norm[(nd[k] < 0 ? 0 : (int64_t)nd[k]) * d.Bp + col];
+      for (int k = 0; k < NG; ++k) nv[k] = mem.norm(max(nd[k], 0));
     }
 #pragma unroll
     for (int k = 0; k < NG; ++k) {
@@ -393,14 +528,10 @@ __device__ __forceinline__ void group_backward_body(const GroupDev& d, const Gro
   }
   high = __any(high);
   middle = __any(middle);
-  if constexpr (kPre) {
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) values(ct, ct);
-  }
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const int s = kPre ? ct : 0;
-    if constexpr (!kPre) { numbers(ct, 0); values(ct, 0); }
+    if constexpr (!kPre) { tb.numbers(mem, base, bx, lane, ct, 0); tb.children(mem, base, bx, lane, ct, 0); }
     g4f acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < NG; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][k], rv[k], acc, 0, 0, 0);
@@ -452,6 +583,15 @@ __device__ __forceinline__ void group_backward_body(const GroupDev& d, const Gro
 }
 
 template <int GT, int CT>
+__device__ __forceinline__ void group_backward_body(const GroupDev& d, const GroupBase& base, int bx, int lane, int slice) {
+  const GroupPointers mem(d, slice, lane);
+  GroupDownTables<GT, CT> tb;
+  tb.load(mem, base, bx, lane);
+  tb.values(mem, base, bx, lane);
+  group_backward_body<GT, CT>(d, base, bx, lane, slice, mem, tb);
+}
+
+template <int GT, int CT>
 __global__ __launch_bounds__(64) void sparse_group_backward_kernel(GroupDev d, GroupBase base) {
   group_backward_body<GT, CT>(d, base, blockIdx.x, threadIdx.x, blockIdx.y);
 }
@@ -480,6 +620,58 @@ __global__ __launch_bounds__(WV * 64) void sparse_group_walk_kernel(GroupDev d, 
     }
     __syncthreads();
   }
+}
+
+// The same where a batch has few slices.  What a compute unit spends on a layer grows with the layer's groups (each is 70
+// to 100 requests of four cache lines), while most compute units have nothing to do.  Groups that nothing of some
+// consecutive layers connects can be walked by workgroups of their own, so a run is cut into stages, a launch each, whose
+// groups are dealt to several workgroups per slice (blockIdx.y), whole connected sets to one of them.  With few groups left in
+// a layer, its time is that of one group's chain of requests and instructions (up: rows 500 + 230 cycles, values 1500), so what
+// no group of the next layer waits for -- rows for later passes, the tables of the wave's next group -- is left for behind the
+// barrier, where the next layer's groups are other waves' (a part's groups go round its waves).
+// 192 variables, K = 32, 512 examples, 25 layers: up 96 us (two walks) -> 53 (four launches), down 100 -> 54 (three); a layer of
+// one group takes 1.7 us, of which its own instructions are the most.  Tried: the next tables asked for behind the rows under
+// way (2.0 us), the rows of earlier launches asked for at the start (to no effect: 1 us a launch longer).
+constexpr int kPartWaves = 4;
+struct GroupParts {
+  const int2* items;   // [part][wave][n_items]: {group, counted from the run's first, or -1: no more; its layer of the stage}
+  int n_items, n_levels;
+  GroupBase base;
+};
+
+template <int GT, int CT, bool kForward>
+__global__ __launch_bounds__(kPartWaves * 64) void sparse_group_parts_kernel(GroupDev d, GroupParts w) {
+  const int lane = threadIdx.x & 63, wave = guni(threadIdx.x >> 6);
+  // (read as constants: by the scalar unit, beside the requests that are under way)
+  typedef const __attribute__((address_space(4))) int* list_at;
+  const list_at items = (list_at)(uintptr_t)(w.items + ((size_t)blockIdx.y * kPartWaves + wave) * w.n_items);
+  using Tables = std::conditional_t<kForward, GroupUpTables<GT, CT>, GroupDownTables<GT, CT>>;
+  const GroupBuffers mem(d, blockIdx.x, lane);
+  Tables tb;
+  int level = 0;
+  int2 item{guni(items[0]), guni(items[1])};
+  if (item.x >= 0) tb.load(mem, w.base, item.x, lane);
+  for (int k = 1; item.x >= 0; ++k) {
+    const int2 after = k < w.n_items ? int2{guni(items[2 * k]), guni(items[2 * k + 1])} : int2{-1, 0};
+    if constexpr (!kForward) tb.values(mem, w.base, item.x, lane);
+    for (; level < item.y; ++level) __syncthreads();
+    // what the next layer waits for; then, unless this wave has more of the layer, the layer is over for it
+    auto over = [&] {
+      if ((after.x < 0 || after.y > level) && level + 1 < w.n_levels) { __syncthreads(); ++level; }
+    };
+    if constexpr (kForward) {
+      GroupUp<GT, CT> up;
+      up.template values<false>(d, w.base, item.x, lane, blockIdx.x, mem, tb);
+      over();
+      up.rest(w.base, item.x, lane, mem, tb);
+    } else {
+      group_backward_body<GT, CT>(d, w.base, item.x, lane, blockIdx.x, mem, tb);
+      over();
+    }
+    item = after;
+    if (item.x >= 0) tb.load(mem, w.base, item.x, lane);
+  }
+  for (; level + 1 < w.n_levels; ++level) __syncthreads();   // (as many barriers for every wave)
 }
 
 // Edge flows of the groups of one shape, after the backward pass: W[g,c] * sum_b R[b,g] E[b,c] over a block of 64

@@ -736,6 +736,44 @@ def test_dense_groups_of_a_multihead_hclt(gpu, oracle, V, K, C, H, B, max_childr
         assert grouped.size("layer_nodes") == grouped.size("input_nodes") + K
 
 
+@pytest.mark.parametrize("V,K,H,keep,B", [(40, 16, 7, 1.0, 64), (60, 32, 9, 0.6, 250), (60, 32, 9, 0.6, 257), (60, 32, 9, 0.7, 520),
+                                          (30, 32, 5, 1.0, 1024), (30, 32, 5, 1.0, 1030), (40, 64, 5, 0.8, 70)])
+def test_walks_of_groups_in_parts(gpu, oracle, V, K, H, keep, B):
+    """Walks whose groups are dealt to several workgroups per slice (4, 8 and 16 of them, by the batch's slices, on either side
+    of the lines) against a launch per layer: the same bits, going up, going down and in the statistics."""
+    torch, P = gpu
+    from helpers import multihead_hclt
+    import pcmi355._lib as L
+    rng = np.random.default_rng(V + K + B)
+    parent = np.full(V, -1, np.int32)
+    for v in range(1, V):      # two long branches and short ones beside them
+        parent[v] = max(0, v - 2) if rng.random() < 0.6 else int(rng.integers(max(0, v - 12), v))
+    heads, _ = multihead_hclt(parent, K, 5, H, rng)
+    if keep < 1.0:             # no two sums of a group with the same children
+        import dag_oracle
+        for n in dag_oracle.topo(list(heads)):
+            if n.kind == oracle.SUM and len(n.children) == K and not any(n is h for h in heads):
+                kept = np.sort(rng.permutation(K)[: int(keep * K)])
+                n.children = [n.children[i] for i in kept]
+                n.logps = np.asarray(n.logps)[kept] - np.logaddexp.reduce(np.asarray(n.logps)[kept])
+    parts = _compile(P, heads, V, 5, H)
+    layered = _without_group_walks(P, heads, V, 5)
+    data = torch.from_numpy(rng.integers(0, 5, size=(B, V)).astype(np.uint8)).cuda()
+    mask = torch.from_numpy((rng.random((B, H)) + 0.05).astype(np.float32)).cuda()
+    got = []
+    for c in (parts, layered):
+        ll = P.probs_flows_circuit(c, data, head_mask=mask).cpu().numpy()
+        mars, flows = c.get_node_values(B)
+        ea, lf = c.get_aggregates()
+        L.check(L.lib.pcm_em_update(c.handle, 0.1, 0.7))
+        got.append((ll, mars, flows, ea, lf, P.vectorize_parameters(c)))
+    assert parts.size("walk_levels") >= 4 and parts.size("dense_groups") > 0
+    most = 1 if B > 1024 else 16 if B <= 256 else 8 if B <= 512 else 4
+    assert 1 <= parts.size("walk_parts") <= most and (parts.size("walk_parts") > 1) == (most > 1)
+    for a, b in zip(*got):
+        assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 def test_dense_groups_after_pruning_and_growing(gpu, oracle):
     """prune_pc takes edges out of some of a group's sums (their lists of children differ from then on) and
     grow_heads_by_flows doubles sums and products: what is left of the groups, and the new ones, still compute what
