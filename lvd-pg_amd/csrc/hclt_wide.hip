@@ -192,8 +192,8 @@ __device__ __forceinline__ WideSlot wide_slot_at(const WideSlot* __restrict__ tb
 //                tile and maximum in LDS (a maximum agreed on first would cost a barrier and an LDS round trip more);
 //   second half: the next slot's value tiles are requested; every wave reads all tiles and maxima, rescales tile w
 //                by exp(m_w - m), m the largest of them, and contracts; logarithms; the tile goes to memory.
-// The barrier after the first half waits for the wave's memory traffic (the group is ahead of the other there
-// anyway), the one after the second half only for LDS: a tile is in memory for the other group three half-steps
+// What one group stores before the barrier in the middle of its slot the other reads behind it through the same compute
+// unit's cache; the barrier after the second half orders LDS only: a tile is there for the other group three half-steps
 // after its slot began.
 // The maxima m go to d.M: the backward walk takes them from there.
 template <int K>
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_forwa
   WideLds<K>& L = Lg[grp];
   wide_stage_slots(tbl, 2 * n_steps, tbl_in_lds, slots_mem);
   const WideRsrc rs = wide_rsrcs<K>(d, s, lane);
-  v4f w[NW], pre[kWidePre][Q], prev_o[Q];
+  v4f pre[kWidePre][Q], prev_o[Q];
   auto request_leaves = [&](const WideSlot& sl, uint32_t xpack) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) wide_request_leaf<K>(rs, sl.op[i], xpack, wave, pre[i]);
@@ -228,7 +228,7 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_forwa
     idle.node = -1;
     return idle;
   };
-  auto cats_of = [&](const WideSlot& sl) { return sl.node >= 0 ? d.xn[(size_t)sl.node * d.Bp + col] : 0u; };
+  auto cats_of = [&](const WideSlot& sl) { return d.xn[(size_t)max(sl.node, 0) * d.Bp + col]; };   // (an idle slot's are not looked at)
   WideSlot nxt = slot_or_idle(0);
   uint32_t xnext = cats_of(nxt);   // packed categories of the slot after the current one
   if (nxt.node >= 0) { request_leaves(nxt, xnext); request_tiles(nxt); }
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_forwa
     const int nn = __builtin_amdgcn_readfirstlane(nxt.node);
     // ---- first half
     if (n >= 0) {
-      v4f z[Q];
+      v4f w[NW], z[Q];
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
         z[q] = pre[0][q];
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_forwa
         for (int i = 0; i < NW; ++i) w[i] = wf[((wave * Q + i / KT) * KT + i % KT) * 64 + lane];
       }
       if (cur.extra_cnt) wide_extras<K>(d, extra, cur.extra_off, cur.extra_cnt, s, lane, wave, z);
-      if (nn >= 0) request_leaves(nxt, xnext);   // (they depend on no other node; the tiles wait for the second half)
+      request_leaves(nxt, xnext);   // (they depend on no other node; the tiles wait for the second half)
       float mw = -INFINITY;
 #pragma unroll
       for (int q = 0; q < Q; ++q)
@@ -285,14 +285,10 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_forwa
         L.e[wave * Q + q][lane] = x;
       }
       if (g == 0) L.mx[wave][b] = mw;
-    } else if (nn >= 0) {
-      request_leaves(nxt, xnext);
-    }
-    __syncthreads();   // (with everything of this wave in memory: the tile of its slot before, which the other group may ask for from here on)
-    // ---- second half
-    if (nn >= 0) request_tiles(nxt);
-    xnext = cats_of(slot_or_idle(t + 2));
-    if (n >= 0) {
+      __syncthreads();   // (behind the tile of the slot before, which the other group may ask for from here on)
+      // ---- second half
+      request_tiles(nxt);
+      xnext = cats_of(slot_or_idle(t + 2));
       float mall[WV], m = -INFINITY;
 #pragma unroll
       for (int w2 = 0; w2 < WV; ++w2) {
@@ -322,6 +318,11 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_forwa
         prev_o[q] = o;
         if ((cur.flags & kWideRoot) && wave == 0 && q == 0) { root_o = o[0]; has_root = true; }
       }
+    } else {   // nothing in this slot (paths of their own: where they join, the compiler waits for the parameter block)
+      request_leaves(nxt, xnext);
+      __syncthreads();
+      request_tiles(nxt);
+      xnext = cats_of(slot_or_idle(t + 2));
     }
     wide_lds_barrier();   // (the tile's store and the next slot's requests stay in flight)
   }
@@ -348,6 +349,9 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_backw
                                                                                            float* __restrict__ ES) {
   constexpr int KT = K / 16, WV = wide_walk_waves<K>(), Q = KT / WV;
   constexpr int NW = Q * KT;
+  // the leaf rows are asked for in the half that is shorter without: the groups swap when the longer one is done (64 variables in
+  // a row, K = 64: a step 2430 + 1700 cycles, then 2050 + 2050; at K = 128 the second half has the more matrix instructions)
+  constexpr bool kLeavesLate = K < 128;
   __shared__ WideLdsB<K> Lg[2];
   extern __shared__ uint32_t slots_mem[];
   const int lane = threadIdx.x & 63, wave_all = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -357,15 +361,18 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_backw
   wide_stage_slots(tbl, 2 * n_steps, tbl_in_lds, slots_mem);
   const WideRsrc rs = wide_rsrcs<K>(d, s, lane);
   const bool live = col < d.B;
-  v4f w[NW], pre[kWidePre][Q], o_next[Q], f_next[Q], prev_g[Q];
+  v4f pre[kWidePre][Q], o_next[Q], f_next[Q], prev_g[Q];
   float m_next = 0.f;
   const uint32_t voff = (uint32_t)s * (kSlice * K * 4) + (uint32_t)lane * 16;
-  // what depends on no other node of this walk: the operands of Z, the node's own value tile and its row maxima
-  auto request_own = [&](const WideSlot& sl, uint32_t xpack) {
-    const int n = __builtin_amdgcn_readfirstlane(sl.node);
-    m_next = d.M[(size_t)n * d.Bp + col];
+  // what depends on no other node of this walk: the tiles of Z, the node's own value tile and its row maxima
+  auto request_leaves = [&](const WideSlot& sl, uint32_t xpack) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) wide_request_leaf<K>(rs, sl.op[i], xpack, wave, pre[i]);
+  };
+  auto request_own = [&](const WideSlot& sl, uint32_t xpack) {
+    if (!kLeavesLate) request_leaves(sl, xpack);
+    const int n = max(__builtin_amdgcn_readfirstlane(sl.node), 0);   // (an idle slot asks for node 0's tile to no purpose, without a branch)
+    m_next = d.M[(size_t)n * d.Bp + col];
 #pragma unroll
     for (int i = 4; i < kWidePre; ++i) wide_request_tile<K>(rs, sl.op[i], wave, pre[i]);
     const __amdgpu_buffer_rsrc_t ro = wide_rsrc(reinterpret_cast<const char*>(d.O) + (size_t)n * d.tile_stride, d.tile_stride);
@@ -374,7 +381,8 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_backw
       o_next[q] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(ro, (int)(voff + (wave * Q + q) * 1024), 0, 0));
   };
   // the parent's flow tile
-  auto request_flow = [&](const WideSlot& sl) {
+  auto request_flow = [&](const WideSlot& sl, uint32_t xpack) {
+    if (kLeavesLate) request_leaves(sl, xpack);
     const int par = __builtin_amdgcn_readfirstlane(sl.parent);
     const bool from_mem = par >= 0 && !(sl.flags & kWidePrev);   // otherwise: the root, or the flows are still in registers
     const __amdgpu_buffer_rsrc_t rg = wide_rsrc(reinterpret_cast<const char*>(G) + (size_t)max(par, 0) * d.tile_stride,
@@ -389,10 +397,10 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_backw
     idle.node = -1;
     return idle;
   };
-  auto cats_of = [&](const WideSlot& sl) { return sl.node >= 0 ? d.xn[(size_t)sl.node * d.Bp + col] : 0u; };
+  auto cats_of = [&](const WideSlot& sl) { return d.xn[(size_t)max(sl.node, 0) * d.Bp + col]; };   // (an idle slot's are not looked at)
   WideSlot nxt = slot_or_idle(0);
   uint32_t xnext = cats_of(nxt);   // packed categories of the slot after the current one
-  if (nxt.node >= 0) { request_own(nxt, xnext); request_flow(nxt); }
+  if (nxt.node >= 0) { request_own(nxt, xnext); request_flow(nxt, xnext); }
   xnext = cats_of(slot_or_idle(1));
 #pragma unroll
   for (int q = 0; q < Q; ++q) prev_g[q] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -403,10 +411,9 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_backw
     nxt = slot_or_idle(t + 1);
     const int nn = __builtin_amdgcn_readfirstlane(nxt.node);
     const size_t tile = ((size_t)max(n, 0) * d.nslices + s) * kSlice * K;
-    v4f e[Q];
     // ---- first half
     if (n >= 0) {
-      v4f z[Q];
+      v4f w[NW], e[Q], z[Q];
       const float m = m_next;
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
@@ -439,13 +446,11 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_backw
         }
         L.r[kt][lane] = r;
       }
-    }
-    if (nn >= 0) request_own(nxt, xnext);
-    __syncthreads();   // (with everything of this wave in memory: the flow tile of its slot before, which the other group may ask for from here on)
-    // ---- second half
-    if (nn >= 0) request_flow(nxt);
-    xnext = cats_of(slot_or_idle(t + 2));
-    if (n >= 0) {
+      request_own(nxt, xnext);
+      __syncthreads();   // (behind the flow tile of the slot before, which the other group may ask for from here on)
+      // ---- second half
+      request_flow(nxt, xnext);
+      xnext = cats_of(slot_or_idle(t + 2));
       v4f* gout = reinterpret_cast<v4f*>(G + tile);
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
@@ -478,6 +483,11 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_backw
         reinterpret_cast<v4f*>(RS + tile)[kt * 64 + lane] = rst;
         reinterpret_cast<v4f*>(ES + tile)[kt * 64 + lane] = est;
       }
+    } else {
+      request_own(nxt, xnext);
+      __syncthreads();
+      request_flow(nxt, xnext);
+      xnext = cats_of(slot_or_idle(t + 2));
     }
     wide_lds_barrier();   // (the stores and the next slot's request stay in flight)
   }

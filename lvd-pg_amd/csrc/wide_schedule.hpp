@@ -34,7 +34,38 @@ inline bool wide_slot_ok(const WideSchedule& s, const std::vector<int>& deps, in
   return true;
 }
 
-// parent[n] = parent node or -1; greedy list scheduling, the node with the longest way still to go first
+// parent[n] = parent node or -1; greedy list scheduling, the node with the longest way still to go first -- or one that is
+// at most `slack` steps behind it and has its operand in the group's registers: going down, two branches of about one length
+// otherwise take turns on one group, each waiting for tiles that the turns have put out of the registers.
+inline WideSchedule wide_greedy_schedule(const std::vector<std::vector<int>>& deps, const std::vector<int>& priority, int slack) {
+  const int n = (int)deps.size();
+  WideSchedule s;
+  s.step.assign(n, -1);
+  s.group.assign(n, -1);
+  int placed = 0;
+  for (int time = 0; placed < n; ++time) {
+    const int t = time / 2, g = time % 2;
+    int best = -1, follower = -1;
+    for (int v = 0; v < n; ++v) {
+      if (s.step[v] >= 0 || !wide_slot_ok(s, deps[v], t, g)) continue;
+      if (best < 0 || priority[v] > priority[best]) best = v;
+      bool follows = false;
+      for (int x : deps[v]) follows |= s.group[x] == g && s.step[x] == t - 1;
+      if (follows && (follower < 0 || priority[v] > priority[follower])) follower = v;
+    }
+    if (best < 0) continue;   // (the root of the remaining work is always placeable two half-steps later at most)
+    if (follower >= 0 && priority[follower] >= priority[best] - slack) best = follower;
+    s.step[best] = t;
+    s.group[best] = g;
+    s.n_steps = t + 1;
+    ++placed;
+  }
+  return s;
+}
+
+// The shortest of the greedy schedules for a few values of the slack, or the first that has nearly as few steps as there can be
+// (64 variables in a row going down: 56 steps where the longest way alone decides, 32 with any slack; bushy trees come out
+// the same with all of them, or shortest with little).
 inline WideSchedule wide_two_group_schedule(const std::vector<int>& parent, bool forward) {
   const int n = (int)parent.size();
   std::vector<std::vector<int>> deps(n);
@@ -49,25 +80,14 @@ inline WideSchedule wide_two_group_schedule(const std::vector<int>& parent, bool
   for (int d = n; d >= 0; --d)   // heights, deepest nodes first
     for (int v = 0; v < n; ++v)
       if (depth[v] == d && parent[v] >= 0) height[parent[v]] = std::max(height[parent[v]], height[v] + 1);
-  const std::vector<int>& priority = forward ? depth : height;
-  WideSchedule s;
-  s.step.assign(n, -1);
-  s.group.assign(n, -1);
-  int placed = 0;
-  for (int time = 0; placed < n; ++time) {
-    const int t = time / 2, g = time % 2;
-    int best = -1;
-    for (int v = 0; v < n; ++v) {
-      if (s.step[v] >= 0 || !wide_slot_ok(s, deps[v], t, g)) continue;
-      if (best < 0 || priority[v] > priority[best]) best = v;
-    }
-    if (best < 0) continue;   // (the root of the remaining work is always placeable two half-steps later at most)
-    s.step[best] = t;
-    s.group[best] = g;
-    s.n_steps = t + 1;
-    ++placed;
+  WideSchedule best;
+  const int least = std::max((n + 1) / 2, n ? *std::max_element(height.begin(), height.end()) : 0);
+  for (const int slack : {0, -n, 1, 2, 4, n}) {   // (-n: the longest way alone decides)
+    if (best.n_steps > 0 && best.n_steps <= least + 2) break;
+    WideSchedule s = wide_greedy_schedule(deps, forward ? depth : height, slack);
+    if (best.n_steps == 0 || s.n_steps < best.n_steps) best = std::move(s);
   }
-  return s;
+  return best;
 }
 
 // -1 when every node's operands are where its slot expects them and no slot is taken twice, else the first node at fault

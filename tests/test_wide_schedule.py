@@ -19,6 +19,7 @@ def test_wide_schedule(tmp_path):
     assert got["chain_forward_fault"] == -1 and got["chain_backward_fault"] == -1
     assert got["chain_one_group"] == 1
     assert got["two_chains_steps"] <= 5 and got["two_chains_fault"] == -1 and got["two_chains_split"] == 1
+    assert got["two_branches_down_steps"] <= 23 and got["two_branches_down_fault"] == -1
     assert got["cross_too_early"] == 2
     assert got["cross_late_enough"] == -1
     assert got["slot_twice"] == 1

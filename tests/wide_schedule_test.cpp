@@ -39,6 +39,13 @@ int main() {
     std::printf("two_chains_fault %d\n", wide_schedule_fault(par, true, f));
     std::printf("two_chains_split %d\n", (int)(f.group[0] != f.group[3] && f.group[0] == f.group[1] && f.group[3] == f.group[4]));
   }
+  {   // two chains of twenty under a root, going down: a group for each, not both by turns on one
+    std::vector<int> par(41, -1);
+    for (int v = 0; v < 40; ++v) par[v] = v % 20 == 19 ? 40 : v + 1;
+    const WideSchedule s = wide_two_group_schedule(par, false);
+    std::printf("two_branches_down_steps %d\n", s.n_steps);
+    std::printf("two_branches_down_fault %d\n", wide_schedule_fault(par, false, s));
+  }
   {   // faults are found: a parent in the slot right after its child of the OTHER group, a slot taken twice
     std::vector<int> par = {2, 2, -1};
     WideSchedule s;
