@@ -270,7 +270,9 @@ void HcltCircuit::build_schedules() {
   PCM_HIP(hipDeviceGetAttribute(&n_cus_, hipDeviceAttributeMultiprocessorCount, dev_id));
   const int tile_bytes = kSlice * K_ * (int)sizeof(float);
   // (the lean walks keep one state word per slot behind the slots)
-  lds_slots_ = std::min((max_lds_ - kLeanFlagWords * 4) / tile_bytes, (1 << (31 - kSlotShift)) - 2);
+  // (the packed categories of a small tree's slice have their place behind the slots' states: LeanRows)
+  const int row_bytes = n_inner_ <= kLeanRowNodes ? (n_inner_ + 1) * kSlice * 4 : 0;
+  lds_slots_ = std::min((max_lds_ - kLeanFlagWords * 4 - row_bytes) / tile_bytes, (1 << (31 - kSlotShift)) - 2);
   if (lds_slots_ < 3) fail(PCM_ERR_UNSUPPORTED, "device offers %d bytes of LDS, a value tile needs %d", max_lds_, tile_bytes);
   const InnerTree kin = inner_tree();
   const std::vector<std::vector<int32_t>>&ic = kin.ic, &lc = kin.lc;
@@ -1252,10 +1254,20 @@ BatchRef HcltCircuit::chunk_of(const BatchRef& b, int off, int chunk) {
   return part;
 }
 
-void HcltCircuit::stage_batch(const BatchRef& b, bool tiles) {
+void HcltCircuit::check_batch(const BatchRef& b) {
   check_walks();
   if (!b.d_data) fail(PCM_ERR_ARG, "data pointer is null");
   if (b.batch < 1) fail(PCM_ERR_ARG, "batch must be positive, got %d", b.batch);
+}
+
+// whether a scoring walk packs its categories itself: a small tree's, where the batch's rows stay in the caches (the line of
+// hclt_gather_x_kernel)
+bool HcltCircuit::packs_in_walk(int batch) const {
+  return n_inner_ <= kLeanRowNodes && (int64_t)batch * Vu_ <= kGatherBytes;
+}
+
+void HcltCircuit::stage_batch(const BatchRef& b, bool tiles) {
+  check_batch(b);
   const bool lean = !wide_walk_ && lean_fits(b.batch, tiles ? kKeepAll : kKeepNone);
   if (!wide_walk_ && !lean) build_general_schedules();
   if (tiles) ensure_batch(b.batch); else ensure_staged(b.batch);
@@ -1297,7 +1309,7 @@ void HcltCircuit::need_general_schedules() const {
   if (!d_stat_items_.p) fail(PCM_ERR_STATE, "the general walk kernels have no schedules of this circuit");
 }
 
-void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
+void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep, const BatchRef* rows) {
   walk_parts_ = lean_fits(d.B, keep) ? lean_plan(d.nslices)->n_groups : 1;
   const size_t lds = (size_t)lds_slots_ * kSlice * K_ * sizeof(float);
   auto launch = [&](auto kernel) {
@@ -1306,17 +1318,21 @@ void HcltCircuit::run_forward(const HcltDev& d, float* d_ll, int keep) {
                      d_fwd_sched_.p, n_fwd_steps_, d_ll);
   };
   if (lean_fits(d.B, keep)) {
-    const size_t lean_lds = lds + kLeanFlagWords * 4;   // the slots' state words sit behind the slots
+    // the slots' state words sit behind the slots, the categories behind them
+    const size_t lean_lds = lds + kLeanFlagWords * 4 + (rows ? (size_t)(n_inner_ + 1) * kSlice * 4 : 0);
+    LeanRows from{};
+    if (rows) from = {reinterpret_cast<const int4*>(d_pack_vars_.p), rows->d_data, rows->stride_ex, rows->stride_var, rows->d_idx};
     auto launch_lean = [&](auto kernel) {
       PCM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lean_lds));
       const LeanPlan* lp = lean_plan(d.nslices);
       PCM_LAUNCH_PHASE(0, kernel, dim3(lp->grid(d.nslices), lp->n_groups), dim3(kWalkWaves * 64), lean_lds, d, d_lean_rows_.p + lp->fwd_at, lp->fwd_stride, d_ll,
-                       lds_slots_, away());
+                       lds_slots_, away(), from);
     };
     PCM_DISPATCH_LEAN_K(K_, {
-      if (keep == kKeepAll) launch_lean(&hclt_forward_lean_kernel<KK, kKeepAll>);
-      else if (keep == kKeepRoots) launch_lean(&hclt_forward_lean_kernel<KK, kKeepRoots>);
-      else launch_lean(&hclt_forward_lean_kernel<KK, kKeepNone>);
+      if (keep == kKeepAll) launch_lean(&hclt_forward_lean_kernel<KK, kKeepAll, false>);
+      else if (keep == kKeepRoots) launch_lean(&hclt_forward_lean_kernel<KK, kKeepRoots, false>);
+      else if (rows) launch_lean(&hclt_forward_lean_kernel<KK, kKeepNone, true>);
+      else launch_lean(&hclt_forward_lean_kernel<KK, kKeepNone, false>);
     });
   } else {
     need_general_schedules();
@@ -1427,6 +1443,11 @@ void HcltCircuit::loglikelihoods(const BatchRef& b, float* d_ll) {
   }
   // nobody reads a scoring pass's tiles: the lean walk keeps none
   const bool lean = lean_fits(b.batch, kKeepNone) && !wide_walk_;
+  if (lean && packs_in_walk(b.batch)) {
+    check_batch(b);
+    ensure_staged(b.batch);
+    return run_forward(dev(b.batch), d_ll, kKeepNone, &b);
+  }
   stage_batch(b, !lean);
   if (wide_walk_) return wide_forward(dev(b.batch), d_ll);
   run_forward(dev(b.batch), d_ll, kKeepNone);

@@ -449,7 +449,9 @@ class HcltCircuit : public pcm_circuit {
   void leaf_vector(bool to_vector, const int32_t* in_pos, float* d_leaf, float* d_vec);
   void fetch_blocks(const float* d_blocks, float* d_leaf, float* theta, float* leaf);
   bool lean_fits(int batch, int keep = kKeepAll) const;
-  void run_forward(const HcltDev& d, float* d_ll, int keep = kKeepAll);
+  void run_forward(const HcltDev& d, float* d_ll, int keep = kKeepAll, const BatchRef* rows = nullptr);
+  void check_batch(const BatchRef& b);
+  bool packs_in_walk(int batch) const;
   void run_backward(const HcltDev& d);
   void run_stats(const HcltDev& d, float rate);
   // wide block kernels

@@ -244,9 +244,21 @@ __device__ __forceinline__ float lean_mark(float m, const Tile<K>& o) {
 // chains in registers / and requests that never wait for a store, two steps ahead, waves that leave when they are through):
 // 784 variables, 512 examples 111 / 97 / 70, 192 variables 55 / 42 / 37, 64 variables (K = 16) 19 / 16.5 / 13; 3072 variables
 // at 512 examples (in parts) 336 / 194 / 141, at 4096, where the stores of the tiles count, 390 / 384 / 372.
-template <int K, int kKeep>
+//
+// kRows: the packed categories come from the caller's rows, each workgroup packing its slice's into LDS before it starts
+// (small trees, scores of small batches: the kernel in front that packs them took a quarter as long as the walk; 64 variables,
+// K = 16, 100 examples 14.6 -> 11.1 us).
+struct LeanRows {
+  const int4* vars;   // per inner node: its own variable and its first three leaf children (-1: none)
+  const uint8_t* data;
+  int64_t stride_ex, stride_var;
+  const int32_t* idx;
+};
+constexpr int kLeanRowNodes = 256;   // most inner nodes of a tree whose categories a workgroup keeps: 64 bytes each
+
+template <int K, int kKeep, bool kRows>
 __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
-    HcltDev d, const int32_t* __restrict__ fields, int stride, float* __restrict__ ll_out, int n_slots, LeanAway away) {
+    HcltDev d, const int32_t* __restrict__ fields, int stride, float* __restrict__ ll_out, int n_slots, LeanAway away, LeanRows rows) {
   extern __shared__ float lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -254,6 +266,18 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
   if (slice >= d.nslices) return;   // (the grid of a tree in parts is rounded up)
   unsigned* state = reinterpret_cast<unsigned*>(lds + (size_t)n_slots * (kSlice * K));
   for (int i = threadIdx.x; i < kLeanFlagWords; i += blockDim.x) state[i] = 0u;
+  uint32_t* const xs = state + kLeanFlagWords;   // kRows: [n_inner + 1][16 examples], behind the state words
+  if constexpr (kRows) {
+    const int b = slice * kSlice + (int)(threadIdx.x & 15);
+    const uint8_t* row = rows.data + (b < d.B ? (int64_t)(rows.idx ? rows.idx[b] : b) * rows.stride_ex : 0);
+    auto category = [&](int var) -> uint32_t {
+      return var >= 0 && b < d.B ? min((uint32_t)row[var * rows.stride_var], (uint32_t)(d.C - 1)) : 0u;   // (in range whatever the caller sent)
+    };
+    for (int n = threadIdx.x >> 4; n <= d.n_inner; n += kWalkWaves * 4) {
+      const int4 v = n < d.n_inner ? rows.vars[n] : make_int4(-1, -1, -1, -1);
+      xs[n * kSlice + (threadIdx.x & 15)] = category(v.x) | category(v.y) << 8 | category(v.z) << 16 | category(v.w) << 24;
+    }
+  }
   __syncthreads();
   const uint32_t vtile = (uint32_t)lane * 16, vleaf = (uint32_t)(lane >> 4) * 16, vx = (uint32_t)(lane & 15) * 4;
   const int bcol = slice * kSlice + (lane & 15);
@@ -282,7 +306,10 @@ __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(
   WTile<K> wA, wB;
   uint32_t x0, x1, x2;  // packed categories of this step, of the next and of the one after
   int a1, a2, a3;       // leaf children of the step whose operands are in flight
-  auto load_x = [&](int s) { return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rX, (int)vx, lean_get(sc, kLNode, s) * xrow, 0); };
+  auto load_x = [&](int s) {
+    if constexpr (kRows) return xs[lean_get(sc, kLNode, s) * kSlice + (lane & 15)];
+    else return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rX, (int)vx, lean_get(sc, kLNode, s) * xrow, 0);
+  };
   {
     x0 = load_x(0);
     x1 = load_x(1);

@@ -313,6 +313,28 @@ def test_batches_gathered_and_staged_agree(gpu, K):
             assert np.abs(p - q).max() < 1e-5 * q.max()
 
 
+@pytest.mark.parametrize("K,V,B", [(16, 2, 1), (16, 64, 100), (32, 64, 15), (32, 65, 17), (16, 257, 33), (32, 257, 16), (32, 258, 20),
+                                   (16, 258, 4097)])
+def test_scores_of_small_trees_pack_their_own_categories(gpu, K, V, B):
+    """Up to 256 inner nodes a scoring walk packs its categories itself; the flow pass and larger trees (257: the last two)
+    have them packed by a kernel in front.  The same bits for rows of bytes, columns, a window of wider rows and ids, and
+    for categories past the last one."""
+    torch, P = gpu
+    rng = np.random.default_rng(V + B)
+    C = 7
+    parent = np.array([-1] + [max(0, v - 1 - int(rng.integers(0, 2))) if V < 200 else v - 1 for v in range(1, V)], np.int32)
+    bpc = P.hclt_from_clt(parent, C, K)
+    x = torch.from_numpy(rng.integers(0, C + 2, size=(B, V)).astype(np.uint8)).cuda()
+    want = P.probs_flows_circuit(bpc, x)
+    assert torch.isfinite(want).all()
+    wide = torch.zeros((B, V + 5), dtype=torch.uint8, device="cuda")
+    wide[:, 3:V + 3] = x
+    ids = rng.permutation(B).astype(np.int32)
+    for got in (P.loglikelihoods(bpc, x), P.loglikelihoods(bpc, x.t().contiguous().t()), P.loglikelihoods(bpc, wide[:, 3:V + 3])):
+        assert torch.equal(got, want)
+    assert torch.equal(P.loglikelihoods(bpc, x, example_ids=ids), want[torch.from_numpy(ids).long().cuda()])
+
+
 @pytest.mark.parametrize("K,V", [(16, 9), (32, 40), (64, 6), (8, 5)])
 def test_scores_do_not_depend_on_the_batch_size(gpu, K, V):
     """A scoring pass on the lean walk keeps no tiles and takes the examples in batches of its own; the other kernels
