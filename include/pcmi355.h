@@ -421,10 +421,20 @@ int pcm_flows_soft(pcm_circuit* c, const float* d_evidence, int64_t stride_ex, i
  * pcm_chow_liu_tree: host matrix [num_vars][num_vars] -> maximum spanning tree (ties: lowest
  * index), directed away from the lowest-numbered centre of the tree; clt_parent[v] = parent
  * of v, -1 at the root: the argument of pcm_hclt_create.
+ *
+ * pcm_chow_liu_edges: the edges of the same spanning tree from a matrix on the device, where they can be told without a rule
+ * for ties.  d_edges (device, [2 num_vars - 1]): {1, then the num_vars - 1 edges as pairs, in no order}, or 0 in the first
+ * place where the matrix is not symmetric and finite off its diagonal or may have more than one maximum spanning tree (take it
+ * to pcm_chow_liu_tree then).  d_workspace: pcm_chow_liu_edges_workspace(num_vars) bytes, 0 for numbers of variables that it does not
+ * take (fewer than 2, more than 8192: PCM_ERR_UNSUPPORTED).  Queued on `stream`; waits for nothing and allocates nothing.
+ * pcm_chow_liu_root: host, the tree of those edges directed as pcm_chow_liu_tree directs it.
  */
 int pcm_pairwise_mi(const uint8_t* d_data, int64_t stride_ex, int64_t stride_var, int64_t num_examples,
                     int32_t num_vars, int32_t num_cats, float pseudocount, float* d_mi, void* stream);
 int pcm_chow_liu_tree(const float* mi, int32_t num_vars, int32_t* clt_parent);
+int64_t pcm_chow_liu_edges_workspace(int32_t num_vars);
+int pcm_chow_liu_edges(const float* d_mi, int32_t num_vars, int32_t* d_edges, void* d_workspace, void* stream);
+int pcm_chow_liu_root(const int32_t* edges, int32_t num_vars, int32_t* clt_parent);
 
 /*
  * pcm_pairwise_mi without any allocation.  No counterpart in the reference: it is for callers that

@@ -355,6 +355,16 @@ int pcm_chow_liu_tree(const float* mi, int32_t num_vars, int32_t* clt_parent) {
   return guarded([&] { pcm::chow_liu_tree(mi, num_vars, clt_parent); });
 }
 
+int64_t pcm_chow_liu_edges_workspace(int32_t num_vars) { return pcm::chow_liu_edges_workspace(num_vars); }
+
+int pcm_chow_liu_edges(const float* d_mi, int32_t num_vars, int32_t* d_edges, void* d_workspace, void* stream) {
+  return guarded([&] { pcm::chow_liu_edges(d_mi, num_vars, d_edges, d_workspace, static_cast<hipStream_t>(stream)); });
+}
+
+int pcm_chow_liu_root(const int32_t* edges, int32_t num_vars, int32_t* clt_parent) {
+  return guarded([&] { pcm::chow_liu_root(edges, num_vars, clt_parent); });
+}
+
 int pcm_stream_probe(const void* d_src, void* d_dst, int64_t lanes, int32_t reads, int32_t writes, int32_t grid, void* stream) {
   return guarded([&] { pcm::stream_probe(d_src, d_dst, lanes, reads, writes, grid, static_cast<hipStream_t>(stream)); });
 }

@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <numeric>
 #include <queue>
 #include <type_traits>
 
@@ -461,31 +462,9 @@ static float prim_take_row(const float* row, int32_t pick, int V, float* best, i
   return most;
 }
 
-// Maximum spanning tree of a dense symmetric weight matrix (Prim; among equal weights the
-// lowest vertex index wins), rooted at the lowest-numbered centre of the tree (the vertex of
-// least eccentricity), as a parent array with -1 at the root.
-void chow_liu_tree(const float* mi, int V, int32_t* parent_out) {
-  if (!mi || !parent_out) fail(PCM_ERR_ARG, "matrix or output pointer is null");
-  if (V < 1) fail(PCM_ERR_SHAPE, "num_vars must be positive, got %d", V);
-  for (int v = 1; v < V; ++v)   // (the first vertex's links start the tree; a later row's NaN is a link that is not there)
-    if (std::isnan(mi[v])) fail(PCM_ERR_ARG, "mutual information matrix holds NaN or -inf in row %d", v);
-  std::vector<float> best(V, -INFINITY);
-  std::vector<int32_t> link(V, 0);
-  std::vector<std::vector<int32_t>> adj(V);
-  best[0] = INFINITY;
-  std::vector<float> cap(V, INFINITY), key(V);
-  cap[0] = -INFINITY;
-  int pick = 0;
-  for (int it = 1; it < V; ++it) {
-    const float most = prim_take_row(mi + (size_t)pick * V, pick, V, best.data(), link.data(), cap.data(), key.data());
-    if (!(most > -INFINITY)) fail(PCM_ERR_ARG, "mutual information matrix holds NaN or -inf in row %d",
-                                  (int)(std::find(cap.begin(), cap.end(), INFINITY) - cap.begin()));
-    pick = (int)(std::find(key.begin(), key.end(), most) - key.begin());
-    best[pick] = INFINITY;
-    cap[pick] = -INFINITY;
-    adj[pick].push_back(link[pick]);
-    adj[link[pick]].push_back(pick);
-  }
+// The tree with these links directed away from its lowest-numbered centre (the vertex of least eccentricity).
+static void root_at_centre(std::vector<std::vector<int32_t>>& adj, int32_t* parent_out) {
+  const int V = (int)adj.size();
   for (auto& a : adj) std::sort(a.begin(), a.end());
   // centre: peel leaves layer by layer; the last one or two vertices are the centres
   std::vector<int> deg(V);
@@ -511,6 +490,55 @@ void chow_liu_tree(const float* mi, int V, int32_t* parent_out) {
     for (int32_t w : adj[v])
       if (parent_out[w] == -2) { parent_out[w] = v; q.push(w); }
   }
+}
+
+// Maximum spanning tree of a dense symmetric weight matrix (Prim; among equal weights the
+// lowest vertex index wins), rooted at the lowest-numbered centre of the tree (the vertex of
+// least eccentricity), as a parent array with -1 at the root.
+void chow_liu_tree(const float* mi, int V, int32_t* parent_out) {
+  if (!mi || !parent_out) fail(PCM_ERR_ARG, "matrix or output pointer is null");
+  if (V < 1) fail(PCM_ERR_SHAPE, "num_vars must be positive, got %d", V);
+  for (int v = 1; v < V; ++v)   // (the first vertex's links start the tree; a later row's NaN is a link that is not there)
+    if (std::isnan(mi[v])) fail(PCM_ERR_ARG, "mutual information matrix holds NaN or -inf in row %d", v);
+  std::vector<float> best(V, -INFINITY);
+  std::vector<int32_t> link(V, 0);
+  std::vector<std::vector<int32_t>> adj(V);
+  best[0] = INFINITY;
+  std::vector<float> cap(V, INFINITY), key(V);
+  cap[0] = -INFINITY;
+  int pick = 0;
+  for (int it = 1; it < V; ++it) {
+    const float most = prim_take_row(mi + (size_t)pick * V, pick, V, best.data(), link.data(), cap.data(), key.data());
+    if (!(most > -INFINITY)) fail(PCM_ERR_ARG, "mutual information matrix holds NaN or -inf in row %d",
+                                  (int)(std::find(cap.begin(), cap.end(), INFINITY) - cap.begin()));
+    pick = (int)(std::find(key.begin(), key.end(), most) - key.begin());
+    best[pick] = INFINITY;
+    cap[pick] = -INFINITY;
+    adj[pick].push_back(link[pick]);
+    adj[link[pick]].push_back(pick);
+  }
+  root_at_centre(adj, parent_out);
+}
+
+// The same from the V - 1 edges of a spanning tree.
+void chow_liu_root(const int32_t* edges, int V, int32_t* parent_out) {
+  if (!edges || !parent_out) fail(PCM_ERR_ARG, "edges or output pointer is null");
+  if (V < 1) fail(PCM_ERR_SHAPE, "num_vars must be positive, got %d", V);
+  std::vector<std::vector<int32_t>> adj(V);
+  std::vector<int32_t> part(V);   // (a cycle or an edge out of range is refused: the peeling below would not end)
+  std::iota(part.begin(), part.end(), 0);
+  auto find = [&](int32_t v) {
+    while (part[v] != v) v = part[v] = part[part[v]];
+    return v;
+  };
+  for (int i = 0; i < V - 1; ++i) {
+    const int32_t a = edges[2 * i], b = edges[2 * i + 1];
+    if (a < 0 || b < 0 || a >= V || b >= V || find(a) == find(b)) fail(PCM_ERR_ARG, "edge %d (%d, %d) does not belong to a tree", i, a, b);
+    part[find(a)] = find(b);
+    adj[a].push_back(b);
+    adj[b].push_back(a);
+  }
+  root_at_centre(adj, parent_out);
 }
 
 }  // namespace pcm

@@ -94,6 +94,12 @@ pcm_pairwise_mi(d_data, stride_ex, stride_var, num_examples, num_vars, num_cats,
     ccall((:pcm_pairwise_mi, libpcmi355), Cint, (Ptr{UInt8}, Int64, Int64, Int64, Int32, Int32, Float32, Ptr{Float32}, Ptr{Cvoid}), d_data, stride_ex, stride_var, num_examples, num_vars, num_cats, pseudocount, d_mi, stream)
 pcm_chow_liu_tree(mi, num_vars, clt_parent) =
     ccall((:pcm_chow_liu_tree, libpcmi355), Cint, (Ptr{Float32}, Int32, Ptr{Int32}), mi, num_vars, clt_parent)
+pcm_chow_liu_edges_workspace(num_vars) =
+    ccall((:pcm_chow_liu_edges_workspace, libpcmi355), Int64, (Int32,), num_vars)
+pcm_chow_liu_edges(d_mi, num_vars, d_edges, d_workspace, stream) =
+    ccall((:pcm_chow_liu_edges, libpcmi355), Cint, (Ptr{Float32}, Int32, Ptr{Int32}, Ptr{Cvoid}, Ptr{Cvoid}), d_mi, num_vars, d_edges, d_workspace, stream)
+pcm_chow_liu_root(edges, num_vars, clt_parent) =
+    ccall((:pcm_chow_liu_root, libpcmi355), Cint, (Ptr{Int32}, Int32, Ptr{Int32}), edges, num_vars, clt_parent)
 pcm_pairwise_mi_static(d_data, stride_ex, stride_var, num_examples, num_vars, num_cats, pseudocount, d_mi, stream) =
     ccall((:pcm_pairwise_mi_static, libpcmi355), Cint, (Ptr{UInt8}, Int64, Int64, Int64, Int32, Int32, Float32, Ptr{Float32}, Ptr{Cvoid}), d_data, stride_ex, stride_var, num_examples, num_vars, num_cats, pseudocount, d_mi, stream)
 pcm_adam_step(c, d_grad, d_params, d_m, d_v, lr, beta1, beta2, eps, t) =

@@ -20,6 +20,8 @@ H = ctypes.c_void_p  # pcm_circuit*
 lib.pcm_last_error.restype = ctypes.c_char_p
 lib.pcm_version.restype = ctypes.c_int
 lib.pcm_size.restype = c_i64
+lib.pcm_chow_liu_edges_workspace.restype = c_i64
+lib.pcm_chow_liu_edges_workspace.argtypes = [c_i32]
 lib.pcm_size.argtypes = [H, c_i32]
 lib.pcm_sample_noise_size.restype = c_i64
 lib.pcm_sample_noise_size.argtypes = [H]
@@ -69,6 +71,8 @@ _SIGS = {
     "pcm_pairwise_mi": [vp, c_i64, c_i64, c_i64, c_i32, c_i32, c_f32, vp, vp],
     "pcm_pairwise_mi_static": [vp, c_i64, c_i64, c_i64, c_i32, c_i32, c_f32, vp, vp],
     "pcm_chow_liu_tree": [vp, c_i32, vp],
+    "pcm_chow_liu_edges": [vp, c_i32, vp, vp, vp],
+    "pcm_chow_liu_root": [vp, c_i32, vp],
     "pcm_set_timing": [H, c_i32],
     "pcm_get_timing": [H, vp, c_i32],
 }

@@ -23,10 +23,37 @@ def pairwise_MI(data, num_cats=None, pseudocount=0.1):
     return mi
 
 
+# vertices from which on a matrix on the GPU has its tree found there (host / device, ms: 200 0.058 / 0.118, 400 0.151 / 0.133,
+# 784 0.449 / 0.161, 3072 5.03 / 0.40)
+_DEVICE_TREE = 400
+
+
+def _unique_tree_edges(mi):
+    """The edges of a device matrix's maximum spanning tree, or None where it may have several (ties), where the matrix
+    is not symmetric and finite, or where there are too many vertices: the host's rules decide those."""
+    v = mi.shape[0]
+    size = lib.pcm_chow_liu_edges_workspace(v)
+    if size == 0:
+        return None
+    with torch.cuda.device(mi.device):
+        m = mi.detach().to(torch.float32).contiguous()
+        out = torch.empty(2 * v - 1, dtype=torch.int32, device=mi.device)
+        work = torch.empty(size, dtype=torch.uint8, device=mi.device)
+        check(lib.pcm_chow_liu_edges(m.data_ptr(), v, out.data_ptr(), work.data_ptr(), torch.cuda.current_stream().cuda_stream))
+        edges = out.cpu().numpy()
+    return np.ascontiguousarray(edges[1:]) if edges[0] == 1 else None
+
+
 def chow_liu_tree(mi):
     """Maximum spanning tree of a mutual-information matrix, directed away from the centre of
     the tree (what `learn_chow_liu_tree` followed by `clt_edges2graphs(...; shape = :directed)`
     gives src/structures/hclts.jl:17-18), as the parent array `hclt_from_clt` takes."""
+    if isinstance(mi, torch.Tensor) and mi.is_cuda and mi.dim() == 2 and mi.shape[0] == mi.shape[1] >= _DEVICE_TREE:
+        edges = _unique_tree_edges(mi)
+        if edges is not None:
+            parent = np.empty(mi.shape[0], np.int32)
+            check(lib.pcm_chow_liu_root(np_ptr(edges), len(parent), np_ptr(parent)))
+            return parent
     if isinstance(mi, torch.Tensor) and mi.is_cuda:     # by way of pinned memory: a third of the time of a pageable copy
         mi = torch.empty(mi.shape, dtype=torch.float32, pin_memory=True).copy_(mi.detach())
     m = np.ascontiguousarray(mi.detach().cpu().numpy() if isinstance(mi, torch.Tensor) else mi, dtype=np.float32)

@@ -112,6 +112,30 @@ def test_chow_liu_tree_and_single_nans(V):
             assert np.array_equal(P.chow_liu_tree(odd), P.chow_liu_tree(none))
 
 
+def test_tree_from_its_edges():
+    """`pcm_chow_liu_root`: the edges of a tree in any order and direction give the parent array that the matrix gave;
+    what is no tree is refused."""
+    import ctypes
+    import pcmi355 as P
+    from pcmi355._lib import lib, np_ptr
+    rng = np.random.default_rng(3)
+    for V in (1, 2, 3, 17, 200):
+        a = rng.normal(size=(V, V)).astype(np.float32)
+        want = P.chow_liu_tree(a + a.T)
+        kids = rng.permutation(np.flatnonzero(want >= 0))
+        edges = np.stack([kids, want[kids]], 1).astype(np.int32)
+        flip = rng.random(len(edges)) < 0.5
+        edges[flip] = edges[flip][:, ::-1]
+        edges, got = np.ascontiguousarray(edges.reshape(-1)), np.empty(V, np.int32)
+        padded = np.concatenate([edges, np.zeros(2, np.int32)])
+        assert lib.pcm_chow_liu_root(np_ptr(padded), V, np_ptr(got)) == 0
+        assert np.array_equal(got, want)
+    for bad in ([0, 1, 1, 2, 2, 0], [0, 1, 0, 1, 2, 3], [0, 4, 1, 2, 2, 3], [0, -1, 1, 2, 2, 3], [0, 0, 1, 2, 2, 3]):
+        assert lib.pcm_chow_liu_root(np_ptr(np.array(bad, np.int32)), 4, np_ptr(np.empty(4, np.int32))) == -1
+    assert lib.pcm_chow_liu_edges_workspace(1) == 0 and lib.pcm_chow_liu_edges_workspace(8193) == 0
+    assert lib.pcm_chow_liu_edges_workspace(8192) > 0
+
+
 # ---- the HIP path -------------------------------------------------------------------------
 
 @pytest.fixture(scope="module")
@@ -238,6 +262,45 @@ def test_hclt_over_variable_groups_and_for_colored_images(gpu):
     bpc = P.CuBitsProbCircuit(pc, nc * h * w)
     lls = P.mini_batch_em_with_reg(bpc, d, 3, batch_size=200, pseudocount=0.1, param_inertia=0.9, shuffle="none")
     assert lls[-1] > lls[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V", [2, 3, 63, 64, 65, 500, 1030])
+def test_tree_found_on_the_device(gpu, V):
+    """Where the maximum spanning tree is unique the device's edges give the host's tree, bit for bit; two largest edges of a
+    component, asymmetry, NaN and infinities are left to the host, which answers as before."""
+    torch, P = gpu
+    from pcmi355 import structures
+    from pcmi355._lib import lib, check, np_ptr
+    rng = np.random.default_rng(V)
+    for scale in (1e-6, 1.0, -3.0):
+        a = rng.normal(size=(V, V)).astype(np.float32)
+        a = np.maximum(a, a.T) * np.float32(scale)
+        edges = structures._unique_tree_edges(torch.from_numpy(a).cuda())
+        parent = np.empty(V, np.int32)
+        check(lib.pcm_chow_liu_root(np_ptr(edges), V, np_ptr(parent)))
+        assert np.array_equal(parent, P.chow_liu_tree(a))
+        assert np.array_equal(P.chow_liu_tree(torch.from_numpy(a).cuda().double()), parent)
+    if V < 63:
+        return
+    for kind in ("ties", "twin", "zeros", "asymmetric", "nan", "inf", "-inf"):
+        b = a.copy()
+        if kind == "ties":
+            b = np.round(b)
+        elif kind == "twin":                      # two columns of the data alike
+            b[2], b[:, 2] = b[4], b[:, 4]
+        elif kind == "zeros":                     # the two zeros are one weight
+            b[...] = np.where(rng.random(V) < 0.5, np.float32(0.0), np.float32(-0.0))
+        elif kind == "asymmetric":
+            b[5, 7] += 1.0
+        else:
+            b[5, 7] = b[7, 5] = float(kind)
+        m = torch.from_numpy(b).cuda()
+        assert structures._unique_tree_edges(m) is None or kind in ("ties", "twin")   # (ties that no component meets)
+        assert np.array_equal(P.chow_liu_tree(m), P.chow_liu_tree(b))
+    none = np.full((V, V), -np.inf, np.float32)
+    with pytest.raises(P.PcmError):
+        P.chow_liu_tree(torch.from_numpy(none).cuda())
 
 
 @pytest.mark.gpu
