@@ -1757,7 +1757,11 @@ void SparseCircuit::launch_groups(int layer, int what, int Bp, int batch, bool t
   for (const GroupLaunch& L : what == 2 ? group_stat_launches_ : group_launches_) {
     if (what != 2 && L.layer != layer) continue;
     const size_t lds = what == 2 ? group_lds_floats(L.gt * 16, L.ct * 16) * sizeof(float) : 0;
-    const dim3 grid(L.count, what == 2 ? Bp / 64 : Bp / 16), block(what == 2 ? 256 : 64);
+    // (the edge flows of few groups of many sums, a circuit's heads: the sums' tiles over several workgroups; 128 heads over 32
+    // products, 512 examples: 20 us in 8 workgroups, 8 in 32)
+    int split = 1;
+    while (what == 2 && 2 * split <= L.gt && L.gt * L.ct >= 8 * split && (int64_t)L.count * (Bp / 64) * split < 128) split *= 2;
+    const dim3 grid(L.count, what == 2 ? Bp / 64 : Bp / 16, split), block(what == 2 ? 256 : 64);
     const GroupBase base{L.group0, L.pnode0, L.pslot0, L.pw0};
     auto run = [&](auto kernel, auto arg) {
       if (lds > 48 * 1024)

@@ -697,6 +697,7 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
   const int group = d.order[first + blockIdx.x];
   const GroupRec r = d.rec[group];
   constexpr int Gp = GT * 16, Cp = CT * 16;
+  const int gt0 = GT * blockIdx.z / gridDim.z, gt1 = GT * (blockIdx.z + 1) / gridDim.z;   // the workgroup's tiles of sums
   float* E = glds;
   float* R = E + Cp * kGroupPad;
   const int b0 = blockIdx.y * 64;
@@ -719,7 +720,7 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
       for (int q = 0; q < 8; ++q)
         if (cb + 4 * q < Cp) child(cb + 4 * q, x[q] > -INFINITY ? x[q] * d.inv_f : -INFINITY);
     }
-    for (int gb = part; gb < Gp; gb += 32) {   // (eight sums' rows requested before the first is used, as above)
+    for (int gb = 16 * gt0 + part; gb < 16 * gt1; gb += 32) {   // (eight sums' rows requested before the first is used, as above)
       float f[8], v[8], nv[8];
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
@@ -727,7 +728,7 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
         f[q] = 0.f;
         v[q] = 0.f;
         nv[q] = 0.f;
-        if (g < r.G) {
+        if (g < min(r.G, 16 * gt1)) {
           const int64_t n = guni(d.node[r.pnode0 + g]);
           f[q] = d.flows[n * d.Bp + b0 + b];
           v[q] = d.mars[n * d.Bp + b0 + b];
@@ -736,7 +737,7 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
       }
 #pragma unroll
       for (int q = 0; q < 8; ++q)
-        if (gb + 4 * q < Gp) sum(gb + 4 * q, f[q] > 0.f && v[q] > -INFINITY ? f[q] : 0.f, (mb - v[q]) * d.inv_f - nv[q]);
+        if (gb + 4 * q < 16 * gt1) sum(gb + 4 * q, f[q] > 0.f && v[q] > -INFINITY ? f[q] : 0.f, (mb - v[q]) * d.inv_f - nv[q]);
     }
   };
   if (t == 0) any_again = 0;
@@ -756,7 +757,7 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
   __syncthreads();
   uint64_t again = 0;   // a bit per (tile of the wave, i): edges with something to be added in logarithms
   int nth = 0;
-  for (int tile = wave; tile < GT * CT; tile += 4, ++nth) {
+  for (int tile = gt0 * CT + wave; tile < gt1 * CT; tile += 4, ++nth) {
     const int gt = tile / CT, ct = tile % CT;
     g4f acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -787,7 +788,7 @@ __global__ __launch_bounds__(256) void sparse_group_stats_kernel(GroupDev d, int
         });
   __syncthreads();
   nth = 0;
-  for (int tile = wave; tile < GT * CT; tile += 4, ++nth) {
+  for (int tile = gt0 * CT + wave; tile < gt1 * CT; tile += 4, ++nth) {
     const int mine = (int)(again >> (4 * nth)) & 15;
     if (!__any(mine)) continue;
     const int gt = tile / CT, ct = tile % CT, c = ct * 16 + lo;
