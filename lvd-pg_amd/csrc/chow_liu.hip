@@ -16,7 +16,7 @@
 // raises a count from c to c + 1 brings g(c + 1) - g(c) -- so a pair costs ONE pass over its N examples against a C x C
 // table of counters in LDS: an atomic add that returns the old count, and a look-up of its difference; then the table is
 // cleared.  Up to 65535 examples the counters are 16 bits wide and the whole table fits; beyond, they are 32 bits wide
-// and the table is walked in bands of rows.  Many variables go to another kernel, a pair per lane (mi_lanes.hip.hpp).
+// and the table is walked in bands of rows.  Many variables go to another kernel, a pair per two lanes (mi_lanes.hip.hpp).
 #include "common.hpp"
 #include "chow_liu.hpp"
 #include "stage_kernel.hip.hpp"

@@ -181,15 +181,15 @@ def test_pairwise_mi_at_the_edges_of_its_launch_rules(gpu, N, V, C):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("N,V,C", [(1, 450, 256), (17, 461, 255), (300, 1100, 129), (2000, 1030, 130), (2500, 700, 256),
+@pytest.mark.parametrize("N,V,C", [(1, 510, 256), (17, 521, 255), (300, 1100, 129), (2000, 1030, 130), (2500, 700, 256),
                                    (2500, 700, 200), (4096, 640, 256), (4097, 1000, 128), (14000, 1152, 64), (15000, 1100, 33),
                                    (16000, 1024, 256), (3000, 900, 1), (3000, 900, 100)])
-def test_pairwise_mi_with_a_pair_per_lane(gpu, N, V, C):
+def test_pairwise_mi_with_a_pair_per_two_lanes(gpu, N, V, C):
     """Enough variables for the kernel that sorts a variable's examples by category, against the one with a pair per
-    workgroup (`pcm_pairwise_mi_static`, the oracle's tests' kernel): both add the same integers, so the results are the same
+    workgroup (`pcm_pairwise_mi_static`, the kernel of the oracle tests): both add the same integers, so the results are the same
     bits.  Columns whose categories hold 8, 9, 16, 17, 255, 256 and 257 examples (ends of chunks, the last 8-bit count), one
     that is constant, one with nine tenths of its examples in one category (counts past the terms in LDS); variables past a
-    whole block of 64; categories shared out among several waves and not."""
+    whole block of 32; a category of a thousand and more examples whose counts pass 255 and one whose do not; categories shared out among several waves and not."""
     torch, P = gpu
     from pcmi355._lib import lib, check
     rng = np.random.default_rng(N + V + C)
@@ -202,6 +202,8 @@ def test_pairwise_mi_with_a_pair_per_lane(gpu, N, V, C):
         x[:, v] = x[rng.permutation(N), v]
     x[:, 5] = C // 2
     x[rng.random(N) < 0.9, 9] = 0
+    x[:, 10] = np.arange(N) % 3 % C          # counts past 255 (2500 examples) between this column and the next, not with noise
+    x[:, 11] = x[:, 10]
     x[rng.random(N) < 0.9, 70] = C - 1
     d = torch.from_numpy(x).cuda()
     got = P.pairwise_MI(d, C, 0.1)
