@@ -439,7 +439,8 @@ int pcm_chow_liu_root(const int32_t* edges, int32_t num_vars, int32_t* clt_paren
 /*
  * pcm_pairwise_mi without any allocation.  No counterpart in the reference: it is for callers that
  * cannot call hipMalloc (code under HIP graph capture, tight serving loops, harnesses that forbid
- * it).  Same arguments, kernels and results as pcm_pairwise_mi; the staging buffer and the two
+ * it).  Same arguments and results (the same bits) as pcm_pairwise_mi, always on the kernel that
+ * shares a pair's counters in a workgroup; the staging buffer and the two
  * tables the kernels need live in a fixed 16.6 MiB array of the library's code object, held by every
  * GPU the library runs on until the process ends.  Limits (PCM_ERR_UNSUPPORTED beyond them):
  * num_examples <= 65535, num_vars <= 4096, num_vars * ceil64(num_examples) <= 16 MiB (e.g. 4096

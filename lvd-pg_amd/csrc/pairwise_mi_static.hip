@@ -1,6 +1,7 @@
 // pcm_pairwise_mi_static: pairwise mutual information for callers that cannot allocate device
-// memory (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc).  The same
-// kernels as pcm_pairwise_mi (chow_liu.hip); their working memory is a fixed array of this code object.
+// memory (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc).  The
+// workgroup kernels of pcm_pairwise_mi (chow_liu.hip; many variables have others there, with the same bits); their working
+// memory is a fixed array of this code object.
 #include "chow_liu.hpp"
 
 #include <mutex>

@@ -10,8 +10,9 @@ def pairwise_MI(data, num_cats=None, pseudocount=0.1):
     """`pairwise_MI_chunked(data; num_cats, pseudocount)` (src/utils/information.jl:97-141):
     mutual information of every pair of variables of a uint8 device tensor [N, V]; returns a
     float32 device tensor [V, V] (symmetric, diagonal included).  Any number of examples in one
-    call: a pair's table never leaves the workgroup that counts it (16-bit cells up to 65535
-    examples, 32-bit cells walked in bands of rows beyond)."""
+    call: a pair's counters never leave the LDS (many variables: one category of the first at a time,
+    two lanes a pair; few: 16-bit cells shared by a workgroup; beyond 65535 examples 32-bit cells
+    walked in bands of rows)."""
     if not (isinstance(data, torch.Tensor) and data.is_cuda and data.dtype == torch.uint8 and data.dim() == 2):
         raise ValueError("data must be a 2-D uint8 tensor on the GPU (examples x variables)")
     n, v = data.shape
