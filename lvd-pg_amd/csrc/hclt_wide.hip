@@ -499,7 +499,7 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_backw
 // E tile of a slice is read from memory once per workgroup (the four waves' requests meet in L1) and serves
 // K / 16 x K / 16 matrix instructions per wave.  (With a workgroup per row tile, as before, every row tile read
 // all of E again: 0.5 GB of L2 traffic on C2, which bound the kernel at 77 us.)  The splits' shares go to rows
-// of `part` [splits][n_inner * K * K]; sum_parts_kernel adds them in order and weights them.
+// of `part` [splits][n_inner * K * K]; wide_edge_sum (soft evidence: sum_parts_kernel) adds them in order and weights them.
 constexpr int kWideEdgeSplits = 8;
 template <int K>
 __device__ __forceinline__ void wide_edge_block(const HcltDev& d, const float* __restrict__ RS, const float* __restrict__ ES,
@@ -613,11 +613,46 @@ __global__ __launch_bounds__(kWideWaves * 64) void hclt_wide_edge_kernel(HcltDev
   wide_edge_block<K>(d, RS, ES, part, blockIdx.x, blockIdx.y, gridDim.y);
 }
 
+// The splits' sum of hclt_wide_edge_kernel, four elements a thread, added up in sum_parts_kernel's order.
+struct WideEdgeSum {
+  const float* part;
+  const float* logw;
+  float* dst;
+  int64_t n;   // a multiple of 4
+  int n_parts;
+};
+
+__device__ __forceinline__ void wide_edge_sum(const WideEdgeSum& e, float rate, int64_t i) {
+  if (i >= e.n) return;
+  const v4f lw = *reinterpret_cast<const v4f*>(e.logw + i);
+  v4f old = {0.f, 0.f, 0.f, 0.f}, p[kWideEdgeSplits], s[4];
+  if (rate != 0.f) old = *reinterpret_cast<const v4f*>(e.dst + i) * rate;
+#pragma unroll
+  for (int q = 0; q < kWideEdgeSplits; ++q)   // (all requested before the first is added)
+    p[q] = *reinterpret_cast<const v4f*>(e.part + (size_t)min(q, e.n_parts - 1) * e.n + i);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) s[g] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < kWideEdgeSplits; ++q)
+    if (q < e.n_parts) s[q & 3] += p[q];
+  const v4f sum = ((s[0] + s[1]) + s[2]) + s[3];
+  v4f out;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) out[j] = old[j] + __expf(lw[j]) * sum[j];
+  *reinterpret_cast<v4f*>(e.dst + i) = out;
+}
+
+// Histograms, n_hist workgroups of them, and behind those the edge flows' sum: a stream of loads that the compute units
+// with one histogram workgroup (of two that fit) take meanwhile: 48 variables, K = 128, 4096 examples 25 us the histograms and 8
+// the sum in a launch of its own, 24 both.
 __global__ __launch_bounds__(kWideLeafWaves * 64) void hclt_wide_leaf_kernel(HcltDev d, const float* __restrict__ G,
                                                                          const int32_t* __restrict__ state_node, int K,
                                                                          float* __restrict__ leaf_flow, float rate,
-                                                                         int limb, const int* __restrict__ flow_shift) {
-  wide_leaf_block(d, G, state_node, K, leaf_flow, rate, limb, flow_shift, blockIdx.x, blockIdx.y);
+                                                                         int limb, const int* __restrict__ flow_shift,
+                                                                         int n_hist, WideEdgeSum edges) {
+  const int kt = K / 16, i = blockIdx.x;
+  if (i < n_hist) wide_leaf_block(d, G, state_node, K, leaf_flow, rate, limb, flow_shift, i / kt, i % kt);
+  else wide_edge_sum(edges, rate, ((int64_t)(i - n_hist) * (kWideLeafWaves * 64) + threadIdx.x) * 4);
 }
 
 // ---- host --------------------------------------------------------------------------------
@@ -715,20 +750,24 @@ void HcltCircuit::wide_backward_stats(const HcltDev& d, float rate, bool soft) {
     // histograms.  (Edge blocks and histograms as two halves of one launch ran slower than one after the other: 357
     // against 320 us per step on C2.)
     const int splits = std::min(kWideEdgeSplits, d.nslices);
-    const int64_t n_edge = (int64_t)n_inner_ * KK * KK;
-    d_part_.ensure((size_t)splits * n_edge);
+    d_part_.ensure((size_t)splits * n_inner_ * KK * KK);
     hipExtLaunchKernelGGL(hclt_wide_edge_kernel<KK>, dim3(n_inner_, splits), dim3(kWideWaves * 64), 0, stream,
                           t_stat ? ev[4] : nullptr, nullptr, 0, d, d_wide_rs_.p, d_wide_es_.p, d_part_.p);
-    hipExtLaunchKernelGGL(sum_parts_kernel<true>, dim3(ceil_div(n_edge, 64)), dim3(256), 0, stream, nullptr,
-                          t_stat && soft ? ev[5] : nullptr, 0, (const float*)d_part_.p, splits, n_edge,
-                          (const float*)d_logtheta_.p, d_edge_aggr_.p, rate);
   });
+  const int splits = std::min(kWideEdgeSplits, d.nslices);
+  const int64_t n_edge = (int64_t)n_inner_ * K_ * K_;
+  if (soft)
+    hipExtLaunchKernelGGL(sum_parts_kernel<true>, dim3(ceil_div(n_edge, 64)), dim3(256), 0, stream, nullptr,
+                          t_stat ? ev[5] : nullptr, 0, (const float*)d_part_.p, splits, n_edge,
+                          (const float*)d_logtheta_.p, d_edge_aggr_.p, rate);
   const size_t lds = 2 * (size_t)C_ * 17 * sizeof(unsigned);
   if (!soft && soft_reg_ > 0.f) PCM_HIP(hipMemsetAsync(d_leaf_hist_.p, 0, d_leaf_hist_.n * sizeof(float), stream));   // (the kernel adds to rate x what is there)
+  const int n_hist = V_ * (K_ / 16);
+  const WideEdgeSum edges = {d_part_.p, d_logtheta_.p, d_edge_aggr_.p, n_edge, splits};
   if (!soft)
-    hipExtLaunchKernelGGL(hclt_wide_leaf_kernel, dim3(V_, K_ / 16), dim3(kWideLeafWaves * 64), (uint32_t)lds, stream, nullptr,
-                          t_stat ? ev[5] : nullptr, 0, d, d_G_.p, d_wide_state_node_.p, K_, stats_leaf_out(), rate, limb,
-                          d.w ? (const int*)d_flow_shift_.p : (const int*)nullptr);
+    hipExtLaunchKernelGGL(hclt_wide_leaf_kernel, dim3(n_hist + ceil_div(n_edge, kWideLeafWaves * 64 * 4)), dim3(kWideLeafWaves * 64),
+                          (uint32_t)lds, stream, nullptr, t_stat ? ev[5] : nullptr, 0, d, d_G_.p, d_wide_state_node_.p, K_,
+                          stats_leaf_out(), rate, limb, d.w ? (const int*)d_flow_shift_.p : (const int*)nullptr, n_hist, edges);
   check_launch_w("hclt_wide_stats");
   if (!soft) soft_reg_counts(rate);
 }
