@@ -1803,28 +1803,21 @@ void HcltCircuit::em_update(float pseudocount, float inertia) {
     pull_from_general();
     return;
   }
-  // the leaf tables first, the parameter blocks last: what the next forward walk reads most often is then
-  // what the caches saw last (the blocks are read by every workgroup, a leaf table row by sixteen examples)
-  // 32 category groups per workgroup; a thread holds its group's share of the categories (8 of 256)
-  {
-    const int threads = 1024, cats = ceil_div(C_, threads / 32);
-    auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(Vu_, ceil_div(K_, 32)), dim3(threads), 0, stream, d_leaf_.p, d_leaf_flow_.p, C_, K_,
-                         pseudocount, inertia, missing_ ? 1 : 0, (const int32_t*)d_walk_void_.p);
-    };
-    if (cats <= 8) launch(&hclt_leaf_update_kernel<8>);
-    else if (cats <= 16) launch(&hclt_leaf_update_kernel<16>);
-    else launch(&hclt_leaf_update_kernel<32>);
-  }
-  check_launch("leaf_update");
-  leaf_changed();   // (the smoothed table of soft_reg follows the leaf table)
   PCM_DISPATCH_PARAM_K(K_, {
-    constexpr int rows_per_block = 256 / (KK < 64 ? KK : 64);
-    hipLaunchKernelGGL(hclt_theta_update_kernel<KK>, dim3(ceil_div((int64_t)n_inner_ * K_, rows_per_block)), dim3(256), 0,
-                       stream, d_nodes_.p, d_logtheta_.p, d_Wf_.p, d_Wb_.p, d_edge_aggr_.p, n_inner_, pseudocount, inertia,
-                       H_ > 0 ? 1 : 0, (const int32_t*)d_walk_void_.p);
+    // 32 category groups per workgroup; a thread holds its group's share of the categories (8 of 256)
+    const int cats = ceil_div(C_, kUpdateThreads / 32), n_leaf = Vu_ * ceil_div(KK, 32);
+    constexpr int rows = kUpdateThreads / (KK < 64 ? KK : 64);   // sum nodes per workgroup
+    const ThetaUpdate theta = {d_nodes_.p, d_logtheta_.p, d_Wf_.p, d_Wb_.p, d_edge_aggr_.p, n_inner_, H_ > 0 ? 1 : 0};
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(n_leaf + ceil_div((int64_t)n_inner_ * KK, rows)), dim3(kUpdateThreads), 0, stream, d_leaf_.p,
+                         d_leaf_flow_.p, C_, K_, n_leaf, pseudocount, inertia, missing_ ? 1 : 0, theta, (const int32_t*)d_walk_void_.p);
+    };
+    if (cats <= 8) launch(&hclt_update_kernel<8, KK>);
+    else if (cats <= 16) launch(&hclt_update_kernel<16, KK>);
+    else launch(&hclt_update_kernel<32, KK>);
   });
-  check_launch("theta_update");
+  check_launch("update");
+  leaf_changed();   // (the smoothed table of soft_reg follows the leaf table)
   if (H_ > 0) {
     hipLaunchKernelGGL(hclt_heads_update_kernel, dim3(ceil_div(H_, 4), T_), dim3(256), 0, stream, head_logp(), head_aggr(), H_,
                        Hp_, K_, pseudocount, inertia, d_head_wf_.p, d_head_wb_.p, (const int32_t*)d_walk_void_.p);
