@@ -1804,17 +1804,13 @@ void HcltCircuit::em_update(float pseudocount, float inertia) {
     return;
   }
   PCM_DISPATCH_PARAM_K(K_, {
-    // 32 category groups per workgroup; a thread holds its group's share of the categories (8 of 256)
-    const int cats = ceil_div(C_, kUpdateThreads / 32), n_leaf = Vu_ * ceil_div(KK, 32);
+    constexpr int cats = 256 / (kUpdateThreads / 32);   // of a thread: 32 category groups per workgroup share the 256 at most
     constexpr int rows = kUpdateThreads / (KK < 64 ? KK : 64);   // sum nodes per workgroup
+    const int n_leaf = Vu_ * ceil_div(KK, 32);
     const ThetaUpdate theta = {d_nodes_.p, d_logtheta_.p, d_Wf_.p, d_Wb_.p, d_edge_aggr_.p, n_inner_, H_ > 0 ? 1 : 0};
-    auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(n_leaf + ceil_div((int64_t)n_inner_ * KK, rows)), dim3(kUpdateThreads), 0, stream, d_leaf_.p,
-                         d_leaf_flow_.p, C_, K_, n_leaf, pseudocount, inertia, missing_ ? 1 : 0, theta, (const int32_t*)d_walk_void_.p);
-    };
-    if (cats <= 8) launch(&hclt_update_kernel<8, KK>);
-    else if (cats <= 16) launch(&hclt_update_kernel<16, KK>);
-    else launch(&hclt_update_kernel<32, KK>);
+    hipLaunchKernelGGL((hclt_update_kernel<cats, KK>), dim3(n_leaf + ceil_div((int64_t)n_inner_ * KK, rows)), dim3(kUpdateThreads), 0,
+                       stream, d_leaf_.p, d_leaf_flow_.p, C_, K_, n_leaf, pseudocount, inertia, missing_ ? 1 : 0, theta,
+                       (const int32_t*)d_walk_void_.p);
   });
   check_launch("update");
   leaf_changed();   // (the smoothed table of soft_reg follows the leaf table)

@@ -979,7 +979,8 @@ __device__ __forceinline__ void leaf_update_block(float* __restrict__ leaf, cons
 
 // Both updates in one launch: a step of 784 variables, K = 32, 22.7 + 5.9 -> 24.6 us, 48 variables, K = 128, 8.4 + 5.2 -> 9.8.
 // The leaf tables' workgroups first, the parameter blocks' last: what the next forward walk reads most often is then what the
-// caches saw last (the blocks are read by every workgroup, a leaf table row by sixteen examples).  K_ is K and blockDim.x kUpdateThreads: where the leaf tables' half knows their values, it keeps an address
+// caches saw last (the blocks are read by every workgroup, a leaf table row by sixteen examples).
+// K_ is K and blockDim.x kUpdateThreads: where the leaf tables' half knows their values, it keeps an address
 // per category from its loads to its stores (K = 32, eight categories a thread: 74 registers instead of 38, one workgroup a compute
 // unit instead of two, sixteen trees of 192 variables 9.9 -> 10.4 ms an epoch).
 template <int kCats, int K>

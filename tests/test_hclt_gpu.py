@@ -63,6 +63,15 @@ def test_em_step_matches_oracle(gpu, oracle, V, K, C, B):
     _compare_step(gpu, oracle, V, K, C, B, seed=100 + V)
 
 
+@pytest.mark.parametrize("V,K,C,B", [(2, 16, 2, 3), (5, 16, 31, 20), (6, 16, 33, 20), (3, 32, 32, 17), (4, 32, 255, 40),
+                                     (3, 64, 33, 16), (3, 128, 2, 1), (4, 128, 32, 16), (5, 128, 65, 112), (4, 128, 255, 128),
+                                     (6, 128, 33, 129)])
+def test_update_and_edge_sums_at_the_edges_of_their_workgroups(gpu, oracle, V, K, C, B):
+    """Chains, so that V - 1 nodes have parameter blocks: one workgroup of the update's second half filled in part, wholly and by
+    one node too many, categories on either side of a group's 32; K = 128: edge flows in one to eight shares."""
+    _compare_step(gpu, oracle, V, K, C, B, seed=V + K + C, tree=[-1] + list(range(V - 1)))
+
+
 @pytest.mark.parametrize("tree", [[-1, 0, 0, 0, 0, 0, 0],                      # star: six leaf children
                                   [-1, 0, 0, 0, 0, 0, 1, 2, 3, 4, 5],        # five inner children
                                   [-1, 0, 1, 1, 1, 1, 2, 3, 0, 8, 8, 8, 8]])  # mixed, four children twice
