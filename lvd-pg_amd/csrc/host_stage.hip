@@ -23,14 +23,6 @@ std::shared_ptr<HostStage> HostStage::shared() {
 
 HostStage::~HostStage() {
   for (Lane& l : lanes_) l.give_back();
-  for (hipStream_t& s : streams_)
-    if (s) (void)hipStreamDestroy(s);
-}
-
-void HostStage::make(int lanes) {
-  for (int i = 0; i < lanes; ++i) lanes_[i].make();
-  for (hipStream_t& s : streams_)
-    if (!s) PCM_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
 }
 
 void HostStage::Lane::make() {
@@ -56,7 +48,7 @@ int HostStage::lanes_for(size_t bytes) const {
 void HostStage::reserve(size_t bytes) {
   if (bytes < kSmall) return;
   std::lock_guard<std::mutex> lock(mu_);
-  make(lanes_for(bytes));
+  for (int i = 0; i < lanes_for(bytes); ++i) lanes_[i].make();
 }
 
 // lane_work(lane, next): takes chunk numbers from `next` until there are none.
@@ -65,7 +57,7 @@ void HostStage::run(size_t bytes, hipStream_t stream, F&& lane_work) {
   int dev = 0;
   PCM_HIP(hipGetDevice(&dev));
   const int n = lanes_for(bytes);
-  make(n);
+  for (int i = 0; i < n; ++i) lanes_[i].make();
   std::atomic<size_t> next{0};
   std::atomic<int> failed{0};
   auto work = [&](int i) {
@@ -89,7 +81,6 @@ void HostStage::run(size_t bytes, hipStream_t stream, F&& lane_work) {
   work(0);
   for (std::thread& t : others) t.join();
   if (failed) {
-    for (hipStream_t s : streams_) (void)hipStreamSynchronize(s);
     (void)hipStreamSynchronize(stream);   // whatever is under way on the buffers or the caller's memory ends before they are free
     fail(PCM_ERR_HIP, "a staged copy of %zu bytes between host and device failed", bytes);
   }
@@ -106,12 +97,11 @@ void HostStage::to_host(void* dst, const void* d_src, size_t bytes, hipStream_t 
   run(bytes, stream, [&](Lane& l, std::atomic<size_t>& next) {
     size_t at[2] = {bytes, bytes};
     auto request = [&](int b) {
-      const hipStream_t on = streams_[(2 * (&l - lanes_) + b) % kStreams];
       at[b] = std::min(bytes, next.fetch_add(1) * kChunk);
       if (at[b] == bytes) return;
       PCM_HIP(hipMemcpyAsync(l.buf[b], static_cast<const char*>(d_src) + at[b], std::min(kChunk, bytes - at[b]),
-                             hipMemcpyDeviceToHost, on));
-      PCM_HIP(hipEventRecord(l.ev[b], on));
+                             hipMemcpyDeviceToHost, stream));
+      PCM_HIP(hipEventRecord(l.ev[b], stream));
     };
     request(0);
     request(1);

@@ -4,9 +4,7 @@
 // array costs a page fault (and the kernel's zeroing) for every page on top: 111 MB of parameters took 11 ms one way,
 // where the link moves them in 2.  Here a few threads each take chunks through a pair of pinned buffers of their own, so
 // that the link, the copies and the page faults overlap: 10.8 -> 3.1 ms for the 111 MB parameter vector of 3072 variables
-// at K = 32, 1.58 -> 0.84 ms for 28 MB, 0.50 -> 0.41 ms for 8 MB (one thread).  On their way to the host the chunks go through three
-// streams of the stage's own, as one stream leaves the link idle for about 15 us between two chunks: 3.05 -> 2.60 ms, 0.84 -> 0.69 (two
-// streams 2.70 and 0.74; chunks of 1 MB 2.80; the link alone takes 2.1).
+// at K = 32, 1.58 -> 0.84 ms for 28 MB, 0.50 -> 0.41 ms for 8 MB (one thread).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -46,10 +44,7 @@ class HostStage {
   int lanes_for(size_t bytes) const;
   template <typename F>
   void run(size_t bytes, hipStream_t stream, F&& lane_work);
-  static constexpr int kStreams = 3;
-  void make(int lanes);   // the lanes' buffers, and the streams
   std::mutex mu_;
-  hipStream_t streams_[kStreams] = {nullptr, nullptr, nullptr};   // (they wait for no other stream and none for them)
   Lane lanes_[kThreads];
 };
 
