@@ -428,9 +428,14 @@ int pcm_flows_soft(pcm_circuit* c, const float* d_evidence, int64_t stride_ex, i
  * to pcm_chow_liu_tree then).  d_workspace: pcm_chow_liu_edges_workspace(num_vars) bytes, 0 for numbers of variables that it does not
  * take (fewer than 2, more than 8192: PCM_ERR_UNSUPPORTED).  Queued on `stream`; waits for nothing and allocates nothing.
  * pcm_chow_liu_root: host, the tree of those edges directed as pcm_chow_liu_tree directs it.
+ *
+ * pcm_pairwise_mi_plan: how pcm_pairwise_mi takes a call of these sizes on the current device.  plan (host, [3]): lanes of a
+ * pair (2, or 0 where a pair's counters are a workgroup's), shares that a variable's categories are dealt to, and the bytes of
+ * device memory that the call allocates (if that fails with two lanes, it takes the other way, with less).
  */
 int pcm_pairwise_mi(const uint8_t* d_data, int64_t stride_ex, int64_t stride_var, int64_t num_examples,
                     int32_t num_vars, int32_t num_cats, float pseudocount, float* d_mi, void* stream);
+int pcm_pairwise_mi_plan(int64_t num_examples, int32_t num_vars, int32_t num_cats, int64_t* plan);
 int pcm_chow_liu_tree(const float* mi, int32_t num_vars, int32_t* clt_parent);
 int64_t pcm_chow_liu_edges_workspace(int32_t num_vars);
 int pcm_chow_liu_edges(const float* d_mi, int32_t num_vars, int32_t* d_edges, void* d_workspace, void* stream);

@@ -351,6 +351,10 @@ int pcm_pairwise_mi_static(const uint8_t* d_data, int64_t stride_ex, int64_t str
   });
 }
 
+int pcm_pairwise_mi_plan(int64_t num_examples, int32_t num_vars, int32_t num_cats, int64_t* plan) {
+  return guarded([&] { pcm::pairwise_mi_plan(num_examples, num_vars, num_cats, plan); });
+}
+
 int pcm_chow_liu_tree(const float* mi, int32_t num_vars, int32_t* clt_parent) {
   return guarded([&] { pcm::chow_liu_tree(mi, num_vars, clt_parent); });
 }

@@ -306,18 +306,23 @@ __global__ __launch_bounds__(kMiThreads) void mi_pair_wide_kernel(const uint8_t*
   }
 }
 
-MiShape mi_check(const uint8_t* d_data, int64_t n_examples, int num_vars, int num_cats, float pseudocount, const float* d_mi) {
-  if (!d_data || !d_mi) fail(PCM_ERR_ARG, "data or output pointer is null");
+static MiShape mi_check_shape(int64_t n_examples, int num_vars, int num_cats) {
   if (n_examples < 1 || n_examples > 2147483584LL)
     fail(PCM_ERR_ARG, "pairwise MI takes 1..2147483584 examples per call, got %lld", (long long)n_examples);
   if (num_vars < 1) fail(PCM_ERR_SHAPE, "num_vars must be positive, got %d", num_vars);
   if (num_cats < 1 || num_cats > 256) fail(PCM_ERR_SHAPE, "num_cats must be in 1..256 (uint8 data), got %d", num_cats);
-  if (pseudocount < 0.f) fail(PCM_ERR_ARG, "pseudocount must not be negative");
   MiShape s;
   s.N = (int)n_examples;
   s.V = num_vars;
   s.C = num_cats;
   s.Np = (n_examples + 63) / 64 * 64;
+  return s;
+}
+
+MiShape mi_check(const uint8_t* d_data, int64_t n_examples, int num_vars, int num_cats, float pseudocount, const float* d_mi) {
+  if (!d_data || !d_mi) fail(PCM_ERR_ARG, "data or output pointer is null");
+  const MiShape s = mi_check_shape(n_examples, num_vars, num_cats);
+  if (pseudocount < 0.f) fail(PCM_ERR_ARG, "pseudocount must not be negative");
   return s;
 }
 
@@ -395,38 +400,60 @@ void mi_launch(const uint8_t* d_data, int64_t stride_ex, int64_t stride_var, con
 #include "mi_lanes.hip.hpp"
 namespace pcm {
 
+namespace {
+// The device memory of a call, in one allocation: each costs more than a small call's kernels.
+struct MiMemory {
+  size_t xb, stat, terms, xt, order, begin, partial;   // offsets; the last four only where lanes take the pairs
+  size_t bytes = 0;
+  MiMemory(const MiShape& sh, const MiLanesPlan& p) {
+    auto take = [&](size_t n) { const size_t at = bytes; bytes += (n + 255) & ~(size_t)255; return at; };
+    xb = take((size_t)sh.V * sh.Np);
+    stat = take((size_t)2 * sh.V * sizeof(double));
+    terms = take(((size_t)sh.N + 1) * sizeof(long long));
+    xt = order = begin = partial = bytes;
+    if (!p.items) return;
+    xt = take((size_t)p.blocks * sh.N * kMiBlock * sizeof(uint32_t));
+    order = take((size_t)sh.V * p.stride * sizeof(uint32_t));
+    begin = take((size_t)sh.V * (p.parts + 1) * sizeof(int));
+    partial = take(p.parts > 1 ? mi_lanes_cells(sh, p) * sizeof(unsigned long long) : 0);
+  }
+};
+}  // namespace
+
 void pairwise_mi(const uint8_t* d_data, int64_t stride_ex, int64_t stride_var, int64_t n_examples, int num_vars,
                  int num_cats, float pseudocount, float* d_mi, hipStream_t stream) {
   const MiShape sh = mi_check(d_data, n_examples, num_vars, num_cats, pseudocount, d_mi);
   MiLanesPlan p = mi_lanes_plan(sh);
-  DevBuf<uint8_t> scratch;   // one allocation: each costs more than a small call's kernels
-  size_t bytes = 0;
-  auto take = [&](size_t n) { const size_t at = bytes; bytes += (n + 255) & ~(size_t)255; return at; };
-  const size_t xb = take((size_t)sh.V * sh.Np), stat = take((size_t)2 * sh.V * sizeof(double)),
-               terms = take(((size_t)sh.N + 1) * sizeof(long long));
-  const size_t pairs_bytes = bytes;
-  const size_t xt = take((size_t)p.blocks * sh.N * 128), order = take((size_t)sh.V * p.stride * sizeof(uint32_t)),
-               begin = take((size_t)sh.V * (p.parts + 1) * sizeof(int)),
-               partial = take(p.parts > 1 ? (size_t)sh.V * 64 * p.blocks * sizeof(long long) : 0);
+  DevBuf<uint8_t> scratch;
   if (p.items) {
     try {
-      scratch.alloc(bytes);
+      scratch.alloc(MiMemory(sh, p).bytes);
     } catch (const Error&) {   // a device that is nearly full: the pairs go to workgroups, whose lists of examples are the data
       (void)hipGetLastError();
-      p.items = 0;
+      p = MiLanesPlan{};
     }
   }
-  if (!p.items) scratch.alloc(pairs_bytes);
-  const MiScratch w{scratch.p + xb, reinterpret_cast<double*>(scratch.p + stat), reinterpret_cast<long long*>(scratch.p + terms)};
+  const MiMemory m(sh, p);
+  if (!p.items) scratch.alloc(m.bytes);
+  const MiScratch w{scratch.p + m.xb, reinterpret_cast<double*>(scratch.p + m.stat), reinterpret_cast<long long*>(scratch.p + m.terms)};
   if (p.items)
     mi_lanes_launch(d_data, stride_ex, stride_var, sh, p, pseudocount, w,
-                    MiLanesScratch{reinterpret_cast<uint32_t*>(scratch.p + xt), reinterpret_cast<uint32_t*>(scratch.p + order),
-                                   reinterpret_cast<int*>(scratch.p + begin),
-                                   reinterpret_cast<unsigned long long*>(scratch.p + partial)},
+                    MiLanesScratch{reinterpret_cast<uint32_t*>(scratch.p + m.xt), reinterpret_cast<uint32_t*>(scratch.p + m.order),
+                                   reinterpret_cast<int*>(scratch.p + m.begin),
+                                   reinterpret_cast<unsigned long long*>(scratch.p + m.partial)},
                     d_mi, stream);
   else
     mi_launch(d_data, stride_ex, stride_var, sh, pseudocount, w, d_mi, stream);
   PCM_HIP(hipStreamSynchronize(stream));   // the scratch array dies with this call
+}
+
+void pairwise_mi_plan(int64_t n_examples, int num_vars, int num_cats, int64_t* plan) {
+  if (!plan) fail(PCM_ERR_ARG, "plan pointer is null");
+  const MiShape sh = mi_check_shape(n_examples, num_vars, num_cats);
+  const MiLanesPlan p = mi_lanes_plan(sh);
+  plan[0] = p.items ? 2 : 0;
+  plan[1] = p.items ? p.parts : 1;
+  plan[2] = (int64_t)MiMemory(sh, p).bytes;
 }
 
 // One vertex of Prim's algorithm: its row's better links, and the largest of the vertices still outside (those inside

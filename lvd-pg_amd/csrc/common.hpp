@@ -130,6 +130,7 @@ void stream_probe(const void* d_src, void* d_dst, int64_t lanes, int reads, int 
 void pairwise_mi_static(const uint8_t* d_data, int64_t stride_ex, int64_t stride_var, int64_t n_examples, int num_vars,
                         int num_cats, float pseudocount, float* d_mi, hipStream_t stream);
 void chow_liu_tree(const float* mi, int num_vars, int32_t* parent_out);
+void pairwise_mi_plan(int64_t n_examples, int num_vars, int num_cats, int64_t* plan);
 void chow_liu_root(const int32_t* edges, int num_vars, int32_t* parent_out);
 int64_t chow_liu_edges_workspace(int num_vars);
 void chow_liu_edges(const float* d_w, int num_vars, int32_t* d_out, void* d_work, hipStream_t stream);

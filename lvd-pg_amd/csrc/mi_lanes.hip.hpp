@@ -411,10 +411,13 @@ static MiLanesPlan mi_lanes_plan(const MiShape& sh) {
   return q;
 }
 
+// pairs' sums that the shares of a pair add to: whole blocks of variables in every row
+static size_t mi_lanes_cells(const MiShape& sh, const MiLanesPlan& p) { return (size_t)sh.V * kMiBlock * p.blocks; }
+
 static void mi_lanes_launch(const uint8_t* d_data, int64_t stride_ex, int64_t stride_var, const MiShape& sh, const MiLanesPlan& p,
                             float pseudocount, const MiScratch& w, const MiLanesScratch& b, float* d_mi, hipStream_t stream) {
   const int N = sh.N, V = sh.V, C = sh.C;
-  const int64_t cells = (int64_t)V * kMiBlock * p.blocks;
+  const int64_t cells = (int64_t)mi_lanes_cells(sh, p);
   pcm_stage(d_data, stride_ex, stride_var, nullptr, N, sh.Np, V, C, w.xb, stream);
   hipLaunchKernelGGL(mi_single_kernel, dim3(V), dim3(256), 0, stream, w.xb, N, sh.Np, C, pseudocount, w.stat);
   hipLaunchKernelGGL(mi_table_kernel, dim3(ceil_div(N, 256)), dim3(256), 0, stream, N, C, pseudocount, w.g);

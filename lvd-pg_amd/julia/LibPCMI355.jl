@@ -92,6 +92,8 @@ pcm_flows_soft(c, d_evidence, stride_ex, stride_var, stride_cat, d_example_ids, 
     ccall((:pcm_flows_soft, libpcmi355), Cint, (Ptr{Cvoid}, Ptr{Float32}, Int64, Int64, Int64, Ptr{Int32}, Int32, Float32, Ptr{Float32}, Ptr{Float32}), c, d_evidence, stride_ex, stride_var, stride_cat, d_example_ids, batch, rate, d_head_mask, d_ll)
 pcm_pairwise_mi(d_data, stride_ex, stride_var, num_examples, num_vars, num_cats, pseudocount, d_mi, stream) =
     ccall((:pcm_pairwise_mi, libpcmi355), Cint, (Ptr{UInt8}, Int64, Int64, Int64, Int32, Int32, Float32, Ptr{Float32}, Ptr{Cvoid}), d_data, stride_ex, stride_var, num_examples, num_vars, num_cats, pseudocount, d_mi, stream)
+pcm_pairwise_mi_plan(num_examples, num_vars, num_cats, plan) =
+    ccall((:pcm_pairwise_mi_plan, libpcmi355), Cint, (Int64, Int32, Int32, Ptr{Int64}), num_examples, num_vars, num_cats, plan)
 pcm_chow_liu_tree(mi, num_vars, clt_parent) =
     ccall((:pcm_chow_liu_tree, libpcmi355), Cint, (Ptr{Float32}, Int32, Ptr{Int32}), mi, num_vars, clt_parent)
 pcm_chow_liu_edges_workspace(num_vars) =

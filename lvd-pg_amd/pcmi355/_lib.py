@@ -70,6 +70,7 @@ _SIGS = {
     "pcm_flows_soft": [H, vp, c_i64, c_i64, c_i64, vp, c_i32, c_f32, vp, vp],
     "pcm_pairwise_mi": [vp, c_i64, c_i64, c_i64, c_i32, c_i32, c_f32, vp, vp],
     "pcm_pairwise_mi_static": [vp, c_i64, c_i64, c_i64, c_i32, c_i32, c_f32, vp, vp],
+    "pcm_pairwise_mi_plan": [c_i64, c_i32, c_i32, vp],
     "pcm_chow_liu_tree": [vp, c_i32, vp],
     "pcm_chow_liu_edges": [vp, c_i32, vp, vp, vp],
     "pcm_chow_liu_root": [vp, c_i32, vp],

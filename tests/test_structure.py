@@ -217,6 +217,35 @@ def test_pairwise_mi_with_a_pair_per_two_lanes(gpu, N, V, C):
     assert torch.equal(P.pairwise_MI(d.t().contiguous().t(), C, 0.1), got)
 
 
+def _mi_plan(N, V, C):
+    """[lanes of a pair, shares of a variable's categories, bytes of scratch] of `pairwise_MI`"""
+    from pcmi355._lib import lib, check, np_ptr
+    plan = np.zeros(3, np.int64)
+    check(lib.pcm_pairwise_mi_plan(N, V, C, np_ptr(plan)))
+    return plan.tolist()
+
+
+@pytest.mark.gpu
+def test_which_pairs_go_to_lanes(gpu):
+    """The sizes of the tests above and below reach the kernel they name, at one share and at several, and a call's scratch is
+    what its kernels use: staged data, marginals, terms; codes, lists, starts and, with several shares, the pairs' sums."""
+    up = lambda n: (n + 255) // 256 * 256
+    lanes = [(1, 510, 256), (17, 521, 255), (300, 1100, 129), (2000, 1030, 130), (2500, 700, 256), (2500, 700, 200), (4096, 640, 256),
+             (4097, 1000, 128), (14000, 1152, 64), (15000, 1100, 33), (16000, 1024, 256), (3000, 900, 1), (3000, 900, 100),
+             (4000, 545, 200), (3500, 813, 256), (65535, 801, 64), (65535, 801, 256)]
+    shares = set()
+    for N, V, C in lanes + [(1000, 100, 256), (16384, 400, 256), (65536, 3072, 256), (4097, 640, 256)]:
+        two, parts, size = _mi_plan(N, V, C)
+        Np, blocks = (N + 63) // 64 * 64, (V + 31) // 32
+        want = up(V * Np) + up(16 * V) + up(8 * (N + 1))
+        if two:
+            stride = (N + 31 * min(N, C) + 64 + 63) // 64 * 64
+            want += up(blocks * N * 128) + up(4 * V * stride) + up(4 * V * (parts + 1)) + (up(8 * V * 32 * blocks) if parts > 1 else 0)
+            shares.add(parts > 1)
+        assert (two == 2) == ((N, V, C) in lanes) and (two or parts == 1) and size == want, (N, V, C, two, parts, size, want)
+    assert shares == {False, True}
+
+
 @pytest.mark.gpu
 def test_learned_tree_and_hclt(gpu):
     torch, P = gpu
