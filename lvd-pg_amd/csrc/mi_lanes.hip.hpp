@@ -192,6 +192,10 @@ __global__ __launch_bounds__(1024) void mi_lanes_kernel(MiLanesArgs g) {
   // end (`past` of them).  16-bit counters count in steps of 8, so that a count is its term's place.  watch: true if a counter
   // has overflowed (into its neighbour's bits).
   constexpr uint32_t kOne = kBits == 16 ? 8u : 1u;
+  // Only a lane whose sum is stored has a say in that: a variable past the last one counts all of a category in one place, and so
+  // does one before u where u has a copy there.  What such a lane's overflow leaves stays in its own column, its sum is given up.
+  const int v = block * kMiBlock + (lane & 31);
+  const bool stored = v >= u && v < g.V;
   int past = 0;
   auto count = [&](const uint32_t (&d)[kMiHalf], int n, auto watch) {
     uint32_t most = 0u;
@@ -221,7 +225,7 @@ __global__ __launch_bounds__(1024) void mi_lanes_kernel(MiLanesArgs g) {
     else if (n > kMiChunk / 2) places(std::integral_constant<int, kMiHalf>{}, std::false_type{});
     else if (n > kMiChunk / 4) places(std::integral_constant<int, kMiHalf / 2>{}, std::false_type{});
     else places(std::integral_constant<int, kMiHalf / 4>{}, std::false_type{});
-    return decltype(watch)::value && __any(most >= (1u << kBits) - 1u);
+    return decltype(watch)::value && __any(stored && most >= (1u << kBits) - 1u);
   };
   auto wipe = [&](const uint32_t (&d)[kMiHalf]) {   // (the places past the chunk's examples hold another's, whose word is zero)
 #pragma unroll
@@ -330,8 +334,7 @@ __global__ __launch_bounds__(1024) void mi_lanes_kernel(MiLanesArgs g) {
   }
   acc -= (double)past * (double)g.dg[0];
   acc += __shfl_xor(acc, 32);   // both halves' examples
-  const int v = block * kMiBlock + (lane & 31);
-  if (odd || v < u || v >= g.V) return;
+  if (odd || !stored) return;
   const long long total = (long long)acc;
   if (g.parts > 1) {
     atomicAdd(g.partial + (size_t)u * (kMiBlock * g.blocks) + v, (unsigned long long)total);
@@ -399,7 +402,7 @@ static MiLanesPlan mi_lanes_plan(const MiShape& sh) {
   const int64_t slots = (int64_t)cus * q.waves;
   // Two and a half rounds of the device's waves, or one round of few examples; else a category with most of the examples, which
   // stays with one wave, is what the call waits for.  Workgroups -> lanes, ms, smooth images (four fifths black): 784 variables,
-  // 256 categories 3.72 -> 3.36 (16.4 -> 14.5) at 16384 examples, 1.66 -> 1.06 (4.4 -> 3.3) at 4000; 128 categories 2.59 -> 2.28 (14.9 ->
+  // 256 categories 3.72 -> 2.84 (16.4 -> 14.5) at 16384 examples, 1.66 -> 1.06 (4.4 -> 3.3) at 4000; 128 categories 2.59 -> 2.28 (14.9 ->
   // 9.3) at 16384; 64 categories 2.58 -> 2.17 (15.3 -> 9.4); 600 variables, 256 categories 1.03 -> 0.64 (2.7 -> 1.3) at 4000.
   if (2 * rounds < 5 * slots && !(rounds >= slots && sh.N <= 4096)) return p;
   q.parts = (int)std::max<int64_t>(1, std::min<int64_t>({16, 6 * cus / items, sh.N / 1024}));

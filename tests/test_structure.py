@@ -247,6 +247,54 @@ def test_which_pairs_go_to_lanes(gpu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,V,C", [(4000, 545, 200), (3500, 813, 256), (65535, 801, 64), (65535, 801, 256)])
+def test_counts_past_their_bits_in_lanes(gpu, N, V, C):
+    """Few categories of many examples, so that only lanes without a pair count past 255 (the last block's, past the last
+    variable); and as many examples as 16-bit counts hold, with columns of one category (a count of 65535) beside others."""
+    torch, P = gpu
+    from pcmi355._lib import lib, check
+    rng = np.random.default_rng(N + V + C)
+    x = rng.integers(0, 10, size=(N, V)).astype(np.uint8) * np.uint8(C // 10)
+    if N == 65535:
+        for v in (0, 31, 32, 500, V - 1):
+            x[:, v] = C - 1 - v % 2
+        x[:, 7] = x[:, 501] = np.arange(N) < 33000     # counts past 32767
+    assert _mi_plan(N, V, C)[0] == 2
+    d = torch.from_numpy(x).cuda()
+    got = P.pairwise_MI(d, C, 0.1)
+    part = 240 if N == 65535 else V      # (the other kernel's memory of its own holds 16 MB of data)
+    for v0 in sorted({0, V - part} | ({480} if N == 65535 else set())):
+        want = torch.empty((part, part), device="cuda")
+        cols = d[:, v0:v0 + part]
+        check(lib.pcm_pairwise_mi_static(cols.data_ptr(), cols.stride(0), cols.stride(1), N, part, C, 0.1, want.data_ptr(),
+                                         torch.cuda.current_stream().cuda_stream))
+        assert torch.equal(got[v0:v0 + part, v0:v0 + part], want)
+    assert torch.equal(got, got.t())
+
+
+@pytest.mark.gpu
+def test_lanes_without_a_pair_cost_nothing(gpu):
+    """784 variables are 24 blocks of 32 and a half: the lanes past the last variable count every example of a category in one
+    place, more than 255 of them here, but no pair does, so the half block takes no second pass.  4 % more pairs than with 768
+    variables; 1.6 times as long where those lanes were heeded, so 1.3 lies half way and far from either."""
+    import time
+    torch, P = gpu
+    g = torch.Generator(device="cuda").manual_seed(5)
+    d = torch.randint(0, 10, (4000, 784), device="cuda", generator=g, dtype=torch.uint8) * 25
+    assert _mi_plan(4000, 768, 256)[:2] == _mi_plan(4000, 784, 256)[:2] == [2, 1]
+    least = {}
+    for V in 3 * (768, 784):
+        x = d[:, :V].contiguous()
+        for _ in range(8):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            P.pairwise_MI(x, 256, 0.1)
+            torch.cuda.synchronize()
+            least[V] = min(least.get(V, 1.0), time.perf_counter() - t)
+    assert least[784] < 1.3 * least[768]
+
+
+@pytest.mark.gpu
 def test_learned_tree_and_hclt(gpu):
     torch, P = gpu
     x = _data(2000, 30, 8, 11)
