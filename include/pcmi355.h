@@ -184,7 +184,8 @@ int pcm_set_stream(pcm_circuit* c, void* hip_stream);
  * of groups that go inside walk launches: runs of consecutive layers that hold groups of one shape and nothing else take
  * one launch per direction where their groups are few (PCMI355_GROUP_WALK=0 at creation: a launch per layer, the same
  * bits), 19 workgroups that walked a slice of 16 examples in the last likelihood or flow pass on the tree walks (parts of
- * one tree, groups of a forest's trees; of a circuit with walks of groups the most of a walk's launches; 0: no such pass yet), 20 workgroups that walked a row in the last row query on the
+ * one tree, groups of a forest's trees; of a pcm_circuit_create circuit the most of a launch of the pass's walks of groups, up
+ * and down, 1 where none went in parts; 0: no such pass yet), 20 workgroups that walked a row in the last row query on the
  * block kernels (0: none yet). */
 int64_t pcm_size(const pcm_circuit* c, int32_t what);
 

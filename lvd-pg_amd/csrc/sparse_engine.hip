@@ -1721,7 +1721,6 @@ bool SparseCircuit::launch_group_walk(int run, bool forward, int Bp, int batch, 
   const bool small = g.flow_bytes && d_grp_rows_.n * (size_t)Bp * 4 < gib2 && (size_t)n_group_elems_ * 4 < gib2 &&
                      d_grp_copies_.n * sizeof(int4) < gib2;
   const std::vector<GroupStage>* stages = nullptr;
-  walk_parts_ = 1;
   for (int k = 0; k < 3; ++k)
     if (small && slices * kGroupParts[k] <= 256) stages = &(forward ? group_stages_fwd_ : group_stages_bwd_)[run][k];
   if (stages && !stages->empty()) {
@@ -2120,6 +2119,7 @@ void SparseCircuit::run_forward(const BatchRef* b, const SoftRef* s) {
   if (b ? !b->d_data : !s->d_ev) fail(PCM_ERR_ARG, "data pointer is null");
   if (batch < 1) fail(PCM_ERR_ARG, "batch must be positive, got %d", batch);
   ensure_batch(batch);
+  walk_parts_ = 1;
   const int Bp = ceil_div(batch, 64) * 64;
   // the staged categories live in a dedicated buffer
   d_visit_.ensure((size_t)std::max<int64_t>((int64_t)fc_.num_vars, fc_.n_nodes()) * Bp);

@@ -774,6 +774,26 @@ def test_walks_of_groups_in_parts(gpu, oracle, V, K, H, keep, B):
         assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+def test_parts_are_those_of_the_last_pass(gpu, oracle):
+    """The selector of the walks' parts follows each pass: a batch whose walks go in parts, one whose walks are whole, one that
+    is too large for walks (16 groups a layer), and the first again; a flow pass counts its way up and its way down."""
+    torch, P = gpu
+    from helpers import multihead_hclt
+    rng = np.random.default_rng(8)
+    V = 63
+    heads, _ = multihead_hclt(np.array([-1] + [(v - 1) // 2 for v in range(1, V)], np.int32), 16, 3, 5, rng)
+    bpc = _compile(P, heads, V, 3, 5)
+    assert bpc.size("walk_levels") >= 2 and bpc.size("walk_parts") == 0
+    data = torch.from_numpy(rng.integers(0, 3, size=(4200, V)).astype(np.uint8)).cuda()
+    up = []
+    for n in (64, 4200, 64, 1100, 250, 4200):
+        P.loglikelihoods(bpc, data[:n], batch_size=n)
+        up.append(bpc.size("walk_parts"))
+    assert up[0] > 1 and up[2] == up[0] and up[4] > 1 and up[1] == up[3] == up[5] == 1
+    P.probs_flows_circuit(bpc, data[:64], head_mask=torch.ones((64, 5), device="cuda"))
+    assert bpc.size("walk_parts") >= up[0]
+
+
 def test_dense_groups_after_pruning_and_growing(gpu, oracle):
     """prune_pc takes edges out of some of a group's sums (their lists of children differ from then on) and
     grow_heads_by_flows doubles sums and products: what is left of the groups, and the new ones, still compute what
