@@ -774,6 +774,55 @@ def test_walks_of_groups_in_parts(gpu, oracle, V, K, H, keep, B):
         assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+@pytest.mark.parametrize("V,K,H,keep,B,fscale,sharp,tiny", [(60, 32, 9, 0.6, 250, 0.5, 1.0, 0.0), (40, 16, 7, 1.0, 100, 2.5, 1.0, 0.0),
+                                                            (40, 16, 7, 0.5, 64, 1.0, 60.0, 0.0), (60, 32, 9, 0.4, 250, 1.0, 90.0, 0.5),
+                                                            (60, 32, 9, 1.0, 500, 1.0, 100.0, 0.5), (40, 64, 5, 0.5, 70, 2.5, 60.0, 0.3)])
+def test_walks_in_parts_tempered_and_far_below(gpu, oracle, V, K, H, keep, B, fscale, sharp, tiny):
+    """Tempered flows, sums far below their group's maximum (leaves `sharp` apart) and hanging on log-parameters below exp's
+    range (a share of `tiny`), in walks that do go in parts, against a launch per layer: the same bits."""
+    torch, P = gpu
+    import dag_oracle
+    from helpers import multihead_hclt
+    rng = np.random.default_rng(int(V + K + B + sharp))
+    parent = np.array([-1] + [max(0, v - 2) if rng.random() < 0.6 else int(rng.integers(max(0, v - 12), v)) for v in range(1, V)], np.int32)
+    heads, _ = multihead_hclt(parent, K, 5, H, rng)
+    products = {}   # of a sum: those of its group
+    for n in dag_oracle.topo(list(heads)):
+        if n.kind == oracle.INPUT and sharp > 1.0:
+            x = rng.normal(size=5) * sharp
+            n.logps = (x - np.logaddexp.reduce(x)).astype(np.float32)
+        elif n.kind == oracle.SUM and len(n.children) == K and not any(n is h for h in heads):
+            kept = np.sort(rng.permutation(K)[: int(keep * K)])
+            products[id(n)] = n.children
+            n.children = [n.children[i] for i in kept]
+            n.logps = np.asarray(n.logps)[kept] - np.logaddexp.reduce(np.asarray(n.logps)[kept])
+            small = rng.random(len(kept)) < tiny
+            small[rng.integers(len(kept))] = False
+            n.logps[small] = -(88 + 40 * rng.random(int(small.sum()))).astype(np.float32)
+    data = torch.from_numpy(rng.integers(0, 5, size=(B, V)).astype(np.uint8)).cuda()
+    mask = torch.from_numpy((rng.random((B, H)) + 0.05).astype(np.float32)).cuda()
+    got = []
+    for c in (_compile(P, heads, V, 5, H), _without_group_walks(P, heads, V, 5)):
+        c.set_flow_scale(fscale)
+        ll = P.probs_flows_circuit(c, data, head_mask=mask).cpu().numpy()
+        got.append((ll, *c.get_node_values(B), *c.get_aggregates()))
+        assert (c.size("walk_parts") > 1) == (c.size("walk_levels") > 0) == (len(got) == 1)
+    for a, b in zip(*got):
+        assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    if sharp > 1.0:   # there are sums further below their group's maximum than exp reaches
+        x, val, far = data.cpu().numpy(), {}, 0.0
+        for n in dag_oracle.topo(list(heads)):
+            if n.kind == oracle.INPUT:
+                val[id(n)] = np.asarray(n.logps, np.float64)[x[:, n.var]]
+            elif n.kind == oracle.SUM:
+                val[id(n)] = np.logaddexp.reduce([val[id(c)] + w for c, w in zip(n.children, n.logps)])
+                group = [sum(val[id(f)] for f in p.children) for p in products.get(id(n), ()) if all(id(f) in val for f in p.children)]
+                far = max(far, (np.max(group, axis=0) - val[id(n)]).max()) if group else far
+            else:
+                val[id(n)] = sum(val[id(c)] for c in n.children)
+        assert far > 87
+
+
 def test_parts_are_those_of_the_last_pass(gpu, oracle):
     """The selector of the walks' parts follows each pass: a batch whose walks go in parts, one whose walks are whole, one that
     is too large for walks (16 groups a layer), and the first again; a flow pass counts its way up and its way down."""
