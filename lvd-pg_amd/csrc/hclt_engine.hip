@@ -271,7 +271,7 @@ void HcltCircuit::build_schedules() {
   const int tile_bytes = kSlice * K_ * (int)sizeof(float);
   // (the lean walks keep one state word per slot behind the slots)
   // (the packed categories of a small tree's slice have their place behind the slots' states: LeanRows)
-  const int row_bytes = n_inner_ <= kLeanRowNodes ? (n_inner_ + 1) * kSlice * 4 : 0;
+  const int row_bytes = n_inner_ <= lean_row_nodes(K_) ? (n_inner_ + 1) * kSlice * 4 : 0;
   lds_slots_ = std::min((max_lds_ - kLeanFlagWords * 4 - row_bytes) / tile_bytes, (1 << (31 - kSlotShift)) - 2);
   if (lds_slots_ < 3) fail(PCM_ERR_UNSUPPORTED, "device offers %d bytes of LDS, a value tile needs %d", max_lds_, tile_bytes);
   const InnerTree kin = inner_tree();
@@ -1263,7 +1263,7 @@ void HcltCircuit::check_batch(const BatchRef& b) {
 // whether a scoring walk packs its categories itself: a small tree's, where the batch's rows stay in the caches (the line of
 // hclt_gather_x_kernel)
 bool HcltCircuit::packs_in_walk(int batch) const {
-  return n_inner_ <= kLeanRowNodes && (int64_t)batch * Vu_ <= kGatherBytes;
+  return n_inner_ <= lean_row_nodes(K_) && (int64_t)batch * Vu_ <= kGatherBytes;
 }
 
 void HcltCircuit::stage_batch(const BatchRef& b, bool tiles) {

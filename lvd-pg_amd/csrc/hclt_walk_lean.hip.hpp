@@ -254,7 +254,12 @@ struct LeanRows {
   int64_t stride_ex, stride_var;
   const int32_t* idx;
 };
-constexpr int kLeanRowNodes = 256;   // most inner nodes of a tree whose categories a workgroup keeps: 64 bytes each
+// Most inner nodes of a tree whose categories a workgroup packs and keeps, 64 bytes each (0: never).  What packing takes grows with the
+// nodes, a lookup per variable and example; the kernel in front takes 5 us whatever they are.  At K = 16 steps are short and
+// the categories out of LDS shorten them: 64 / 171 / 225 nodes, 200 examples 24.7 -> 19.2 / 77.9 -> 61.1 / 94.1 -> 75.1 us.  At K = 32
+// they do not: 72 / 93 / 115 / 130 / 219 nodes 46.1 -> 45.1 / 59.1 -> 58.1 / 64.8 -> 64.5 / 72.7 -> 73.0 / 116.4 -> 118.2.  (All lookups of a
+// thread requested at once, those of missing children too: 119.3; a lane's lookups are a cache line each.)
+constexpr int lean_row_nodes(int K) { return K == 16 ? 256 : K == 32 ? 112 : 0; }
 
 template <int K, int kKeep, bool kRows>
 __global__ __launch_bounds__(kWalkWaves * 64) void hclt_forward_lean_kernel(

@@ -344,6 +344,19 @@ def test_scores_of_small_trees_pack_their_own_categories(gpu, K, V, B):
     assert torch.equal(P.loglikelihoods(bpc, x, example_ids=ids), want[torch.from_numpy(ids).long().cuda()])
 
 
+@pytest.mark.parametrize("K,V,B", [(32, 112, 20), (32, 113, 100), (32, 114, 33), (32, 220, 200), (16, 220, 200)])
+def test_scores_on_either_side_of_packing_in_the_walk(gpu, K, V, B):
+    """Chains (V - 1 inner nodes): with 32 states a scoring walk packs categories up to 112 nodes only, with 16 up to 256; the same
+    bits as the flow pass on either side of the line."""
+    torch, P = gpu
+    rng = np.random.default_rng(V + B)
+    bpc = P.hclt_from_clt(np.arange(-1, V - 1, dtype=np.int32), 5, K)
+    x = torch.from_numpy(rng.integers(0, 6, size=(B, V)).astype(np.uint8)).cuda()
+    want = P.probs_flows_circuit(bpc, x)
+    assert torch.isfinite(want).all()
+    assert torch.equal(P.loglikelihoods(bpc, x), want) and torch.equal(P.loglikelihoods(bpc, x.t().contiguous().t()), want)
+
+
 @pytest.mark.parametrize("K,V", [(16, 9), (32, 40), (64, 6), (8, 5)])
 def test_scores_do_not_depend_on_the_batch_size(gpu, K, V):
     """A scoring pass on the lean walk keeps no tiles and takes the examples in batches of its own; the other kernels
