@@ -1,5 +1,5 @@
-// Chow-Liu structure learning: pairwise mutual information of categorical data on the device,
-// maximum spanning tree and rooting on the host.
+// Chow-Liu structure learning: pairwise mutual information of categorical data on the device; maximum spanning tree (of a
+// matrix on the device chow_liu_edges.hip finds it where it is the only one) and rooting on the host.
 //
 // Reference: src/utils/information.jl:3-95 (pairwise and single marginals with a pseudocount
 // spread as pc/C per category and pc/C^2 per cell, normalised by Z = N + pc) and :97-141
@@ -8,7 +8,7 @@
 // for: a maximum spanning tree of MI, directed away from the centre of the tree.
 //
 // The reference fills a dense [V][V][C][C] table with float atomics and reduces it on the host.
-// Here a pair never leaves the workgroup.  With c(a,b) the count of a cell, s = pc/C^2,
+// Here a pair's counters never leave the LDS.  With c(a,b) the count of a cell, s = pc/C^2,
 // p(c) = (c + s)/Z, la[u][a] = log P_u[a]:
 //   MI[u,v] = sum over non-empty cells of g(c(cell))  -  M_u - M_v  +  C^2 * xlogx(p(0))  -  p(0) * C * (L_u + L_v)
 //   g(c) = xlogx(p(c)) - xlogx(p(0)),   M_u = (1/Z) sum_e la[u][x_eu],   L_u = sum_a la[u][a]

@@ -243,7 +243,6 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_forwa
     const WideSlot cur = nxt;
     const int n = __builtin_amdgcn_readfirstlane(cur.node);
     nxt = slot_or_idle(t + 1);
-    const int nn = __builtin_amdgcn_readfirstlane(nxt.node);
     // ---- first half
     if (n >= 0) {
       v4f w[NW], z[Q];
@@ -409,7 +408,6 @@ __global__ __launch_bounds__(2 * wide_walk_waves<K>() * 64) void hclt_wide_backw
     const WideSlot cur = nxt;
     const int n = __builtin_amdgcn_readfirstlane(cur.node);
     nxt = slot_or_idle(t + 1);
-    const int nn = __builtin_amdgcn_readfirstlane(nxt.node);
     const size_t tile = ((size_t)max(n, 0) * d.nslices + s) * kSlice * K;
     // ---- first half
     if (n >= 0) {

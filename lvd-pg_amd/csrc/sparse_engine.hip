@@ -1491,6 +1491,9 @@ void SparseCircuit::build_group_runs(const std::vector<int32_t>& group_of) {
   n_walk_levels_ = 0;
   const char* env = std::getenv("PCMI355_GROUP_WALK");
   if (group_launches_.empty() || (env && env[0] == '0')) return;
+  int dev_id = 0;
+  PCM_HIP(hipGetDevice(&dev_id));
+  PCM_HIP(hipDeviceGetAttribute(&n_cus_, hipDeviceAttributeMultiprocessorCount, dev_id));
   std::vector<int2> levels;
   auto collect = [&](const std::vector<int>& layer0, std::vector<GroupRun>& runs) {
     // per layer: the one launch of its groups (-1: none, -2: several shapes)
@@ -1722,7 +1725,7 @@ bool SparseCircuit::launch_group_walk(int run, bool forward, int Bp, int batch, 
                      d_grp_copies_.n * sizeof(int4) < gib2;
   const std::vector<GroupStage>* stages = nullptr;
   for (int k = 0; k < 3; ++k)
-    if (small && slices * kGroupParts[k] <= 256) stages = &(forward ? group_stages_fwd_ : group_stages_bwd_)[run][k];
+    if (small && slices * kGroupParts[k] <= n_cus_) stages = &(forward ? group_stages_fwd_ : group_stages_bwd_)[run][k];
   if (stages && !stages->empty()) {
     for (const GroupStage& st : *stages) {
       walk_parts_ = std::max(walk_parts_, st.parts);

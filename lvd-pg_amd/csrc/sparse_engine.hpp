@@ -135,6 +135,7 @@ class SparseCircuit : public pcm_circuit {
   static constexpr int kGroupParts[3] = {4, 8, 16};   // most parts a plan has
   std::vector<std::array<std::vector<GroupStage>, 3>> group_stages_fwd_, group_stages_bwd_;   // per run, per entry of kGroupParts
   DevBuf<int2> d_grp_items_;
+  int n_cus_ = 0;                             // of the device, where there are runs
   int walk_parts_ = 0;                        // most parts of a launch in the last pass's walks, up and down (1: whole or no walks, 0: no pass yet)
   int64_t n_walk_levels_ = 0;                 // layers of groups inside forward runs
   void build_group_runs(const std::vector<int32_t>& group_of);

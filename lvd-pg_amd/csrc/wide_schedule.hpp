@@ -4,9 +4,9 @@
 // A workgroup of the wide walks has two groups of waves that work half a step apart: while one group runs a
 // node's matrix instructions, the other sums, exponentiates and exchanges the operands of ITS node, and the
 // two swap roles at every barrier.  In units of half a step, the slot (step t, group g) starts at 2t + g; its
-// tile is stored at the end of the slot, and the group waits for its stores at the barrier in the middle of its
-// next slot, so the tile is in memory for the other group at 2t + g + 3.  The tiles a node needs are requested
-// during the second half of the same group's slot before, at 2t + g - 1, so they must be in memory by then --
+// tile is stored at the end of the slot, ahead of the barrier in the middle of the group's next slot, behind which the
+// other group reads it (through the same compute unit's cache): from 2t + g + 3 on.  The tiles a node needs are requested
+// during the second half of the same group's slot before, at 2t + g - 1, so they must be there by then --
 // unless it is the tile of that very slot before, which is still in the group's registers.  Going up the tree (forward) a node needs
 // the tiles of its non-leaf children; going down (backward) the flow tile of its parent.
 #pragma once

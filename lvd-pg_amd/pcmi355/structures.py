@@ -24,8 +24,9 @@ def pairwise_MI(data, num_cats=None, pseudocount=0.1):
     return mi
 
 
-# vertices from which on a matrix on the GPU has its tree found there (host / device, ms: 200 0.058 / 0.118, 400 0.151 / 0.133,
-# 784 0.449 / 0.161, 3072 5.03 / 0.40)
+# vertices from which on a matrix on the GPU has its tree found there (host / device, ms: 200 0.058 / 0.118, 400 0.151 / 0.136,
+# 500 0.200 / 0.139, 600 0.269 / 0.151, 784 0.436 / 0.161, 1500 1.35 / 0.216, 3072 5.1 / 0.34).  Where the device meets a tie (columns
+# of the data alike, constant ones) the host decides behind it: 400 0.285, 500 0.329, 600 0.403, 784 0.578, 1500 1.52, 3072 5.26.
 _DEVICE_TREE = 400
 
 
