@@ -325,7 +325,7 @@ def test_batches_gathered_and_staged_agree(gpu, K):
 @pytest.mark.parametrize("K,V,B", [(16, 2, 1), (16, 64, 100), (32, 64, 15), (32, 65, 17), (16, 257, 33), (32, 257, 16), (32, 258, 20),
                                    (16, 258, 4097)])
 def test_scores_of_small_trees_pack_their_own_categories(gpu, K, V, B):
-    """Up to 256 inner nodes (K = 32: 112) a scoring walk packs its categories itself; the flow pass and larger trees (the last four)
+    """Up to 256 inner nodes (K = 32: 112) a scoring walk packs its categories itself; the flow pass and larger trees (the last three)
     have them packed by a kernel in front.  The same bits for rows of bytes, columns, a window of wider rows and ids, and
     for categories past the last one."""
     torch, P = gpu
